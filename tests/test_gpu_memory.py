@@ -1,0 +1,48 @@
+"""Device memory that is kept between calls (thundergbm_amd/csrc/device_memory.hip)."""
+import os
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import datasets as D  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def test_calls_share_and_return_kept_memory():
+    """Sessions of two threads at once, of different sizes, then again after everything kept went back to the driver:
+    the same models each time."""
+    import thundergbm_amd as T
+    L = T.load()
+    D.warm_up(T)
+    data = []
+    for n, F in ((3000, 5), (777, 40)):
+        X, y = D.config1(n, F, seed=n)
+        data.append(D.dense_to_csr(X) + (y,))
+
+    def train(i):
+        val, rp, col, y = data[i]
+        s = T.Session(val, rp, col, y, depth=5, n_trees=6, learning_rate=0.5)
+        s.boost(6)
+        m = s.model().tobytes()
+        s.close()
+        return m
+
+    alone = [train(0), train(1)]
+    got = {}
+
+    def loop(i):
+        got[i] = [train(i) for _ in range(5)]
+
+    threads = [threading.Thread(target=loop, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    L.tgbm_release_memory()
+    for i in (0, 1):
+        assert all(m == alone[i] for m in got[i])
+        assert train(i) == alone[i]

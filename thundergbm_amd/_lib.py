@@ -48,6 +48,7 @@ SIGNATURES = {
     "tgbm_trainer_export_model": (_P, [_P]),
     "tgbm_predict_raw": (None, [C.c_int, _P, _P, _P, _P, C.c_int, C.c_int, C.c_float, C.c_float, _P]),
     "tgbm_predict_raw_noalloc": (C.c_int, [C.c_int, _P, _P, _P, _P, C.c_int, C.c_int, C.c_float, C.c_float, _P]),
+    "tgbm_release_memory": (None, []),
     "tgbm_cut_points": (C.c_int, [C.c_int, C.c_int, _P, _P, _P, C.c_int, _P, _P, _P, _P]),
 }
 

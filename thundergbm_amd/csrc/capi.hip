@@ -337,12 +337,11 @@ void tgbm_predict_raw(int row_size, const float *val, const int *row_ptr, const 
 int tgbm_cut_points(int row_size, int n_features, const float *val, const int *row_ptr, const int *col_ptr,
                     int max_num_bin, float *cut_val, int *cut_row_ptr, int *cut_fid, int *bin_id) {
     const long nnz = row_ptr[row_size];
-    hipStream_t s;
-    HIP_CHECK(hipStreamCreate(&s));
+    hipStream_t s = stream_acquire();
     float *d_val = nullptr;
     int *d_col = nullptr, *d_bin = nullptr;
-    HIP_CHECK(hipMalloc(&d_val, sizeof(float) * (size_t)std::max(nnz, 1l)));
-    HIP_CHECK(hipMalloc(&d_col, sizeof(int) * (size_t)std::max(nnz, 1l)));
+    device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz, 1l));
+    device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz, 1l));
     if (nnz) {
         HIP_CHECK(hipMemcpyAsync(d_val, val, sizeof(float) * (size_t)nnz, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(d_col, col_ptr, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice, s));
@@ -355,18 +354,18 @@ int tgbm_cut_points(int row_size, int n_features, const float *val, const int *r
         HIP_CHECK(hipMemcpyAsync(cut_fid, c.cut_fid, sizeof(int) * (size_t)c.n_bins, hipMemcpyDeviceToHost, s));
     }
     if (bin_id != nullptr && nnz) {
-        HIP_CHECK(hipMalloc(&d_bin, sizeof(int) * (size_t)nnz));
+        device_alloc_to(d_bin, sizeof(int) * (size_t)nnz);
         launch_bin_csr(s, nnz, d_col, d_val, c.cut_val, c.cut_row_ptr, d_bin);
         HIP_CHECK(hipMemcpyAsync(bin_id, d_bin, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToHost, s));
     }
     HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipFree(d_val));
-    HIP_CHECK(hipFree(d_col));
-    if (d_bin) HIP_CHECK(hipFree(d_bin));
-    HIP_CHECK(hipFree(c.cut_row_ptr));
-    if (c.cut_val) HIP_CHECK(hipFree(c.cut_val));
-    if (c.cut_fid) HIP_CHECK(hipFree(c.cut_fid));
-    HIP_CHECK(hipStreamDestroy(s));
+    device_free(d_val);
+    device_free(d_col);
+    if (d_bin) device_free(d_bin);
+    device_free(c.cut_row_ptr);
+    if (c.cut_val) device_free(c.cut_val);
+    if (c.cut_fid) device_free(c.cut_fid);
+    stream_release(s);
     return c.n_bins;
 }
 

@@ -25,6 +25,18 @@
 
 namespace tgbm {
 
+// Device blocks and streams that are kept for the next call (device_memory.hip). Whoever frees a block or gives a
+// stream back has synchronised the work on it; device_mem_info counts the kept blocks as free memory.
+void *device_alloc(size_t bytes);
+void device_free(void *p);
+template <typename T>
+void device_alloc_to(T *&p, size_t bytes) {
+    p = static_cast<T *>(device_alloc(bytes));
+}
+void device_mem_info(size_t *free_b, size_t *total_b);
+hipStream_t stream_acquire();
+void stream_release(hipStream_t s);
+
 constexpr int kMissingBin = 255;   // dense matrix sentinel: the feature has no stored value in this row
 constexpr int kMissingBin16 = 65535;  // the same for 16-bit bins
 // 16-bit bins: bins of a feature block that leave the LDS room for two histogram workgroups per CU, and the most a

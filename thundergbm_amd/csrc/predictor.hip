@@ -69,8 +69,7 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
         log_debug("predict: %s %.3f s", what, std::chrono::duration<double>(now - t_begin).count());
         t_begin = now;
     };
-    hipStream_t s;
-    HIP_CHECK(hipStreamCreate(&s));
+    hipStream_t s = stream_acquire();
     float *d_val = nullptr, *d_out = nullptr, *d_label = nullptr;
     int *d_col = nullptr, *d_row_ptr = nullptr;
     TreeNode *d_model = nullptr;
@@ -78,12 +77,12 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
     uint2 *d_compact = nullptr;
     int compact_depth = 0;
     const size_t n_out = (size_t)n * nct;
-    HIP_CHECK(hipMalloc(&d_val, sizeof(float) * (size_t)std::max(nnz, 1l)));
-    HIP_CHECK(hipMalloc(&d_col, sizeof(int) * (size_t)std::max(nnz, 1l)));
-    HIP_CHECK(hipMalloc(&d_row_ptr, sizeof(int) * (size_t)(n + 1)));
-    HIP_CHECK(hipMalloc(&d_model, sizeof(TreeNode) * flat.size()));
-    HIP_CHECK(hipMalloc(&d_packed, sizeof(PackedNode) * flat.size()));
-    HIP_CHECK(hipMalloc(&d_out, sizeof(float) * std::max(n_out, (size_t)1)));
+    device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz, 1l));
+    device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz, 1l));
+    device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n + 1));
+    device_alloc_to(d_model, sizeof(TreeNode) * flat.size());
+    device_alloc_to(d_packed, sizeof(PackedNode) * flat.size());
+    device_alloc_to(d_out, sizeof(float) * std::max(n_out, (size_t)1));
     HIP_CHECK(hipMemcpyAsync(d_row_ptr, ds.row_ptr, sizeof(int) * (size_t)(n + 1), hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(d_model, flat.data(), sizeof(TreeNode) * flat.size(), hipMemcpyHostToDevice, s));
     launch_pack_model(s, d_model, (long)flat.size(), n_nodes, d_packed);
@@ -95,14 +94,13 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
     if (!ds.features_counted) F = device_max_int(s, d_col, nnz) + 1;
     compact_depth = compact_records_apply(flat.data(), flat.size(), n_nodes, F);  // (F is known only now)
     if (compact_depth > 0) {
-        HIP_CHECK(hipMalloc(&d_compact, sizeof(uint2) * flat.size()));
+        device_alloc_to(d_compact, sizeof(uint2) * flat.size());
         launch_pack_compact(s, d_model, n_iter, nct, n_nodes, F, d_compact);
     }
     HIP_CHECK(hipStreamSynchronize(s));
     lap("allocation, model and column indices");
     {
-        hipStream_t s_up;
-        HIP_CHECK(hipStreamCreate(&s_up));
+        hipStream_t s_up = stream_acquire();
         const long slice_entries = 64l << 20;  // ~256 MB of values per slice
         int r0 = 0;
         while (r0 < n) {
@@ -120,7 +118,7 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
             r0 = r1;
         }
         HIP_CHECK(hipStreamSynchronize(s));
-        HIP_CHECK(hipStreamDestroy(s_up));
+        stream_release(s_up);
     }
     lap("values and traversal");
     size_t n_ret = n_out;
@@ -133,13 +131,13 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
             const bool ndcg = param.objective == "rank:ndcg";
             RankContext rc(s, ds.y, ds.group, ndcg);
             float *d_m = nullptr;
-            HIP_CHECK(hipMalloc(&d_m, sizeof(float)));
+            device_alloc_to(d_m, sizeof(float));
             rc.metric(ndcg ? RANK_METRIC_NDCG : RANK_METRIC_MAP, d_out, d_m);
             float v = 0;
             HIP_CHECK(hipMemcpyAsync(&v, d_m, sizeof(float), hipMemcpyDeviceToHost, s));
             HIP_CHECK(hipStreamSynchronize(s));
             log_info("%s = %g", ndcg ? "NDCG" : "MAP", v);
-            HIP_CHECK(hipFree(d_m));
+            device_free(d_m);
         }
     } else if (log_metric && (int)ds.y.size() == n && n > 0) {
         int kind = 0;
@@ -148,25 +146,25 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
         static const char *names[] = {"RMSE", "test error", "multi-class accuracy"};
         float *d_y = nullptr, *d_m = nullptr;
         double *d_scratch = nullptr;
-        HIP_CHECK(hipMalloc(&d_y, sizeof(float) * (size_t)n));
-        HIP_CHECK(hipMalloc(&d_m, sizeof(float)));
-        HIP_CHECK(hipMalloc(&d_scratch, sizeof(double) * (size_t)row_blocks(n)));
+        device_alloc_to(d_y, sizeof(float) * (size_t)n);
+        device_alloc_to(d_m, sizeof(float));
+        device_alloc_to(d_scratch, sizeof(double) * (size_t)row_blocks(n));
         HIP_CHECK(hipMemcpyAsync(d_y, ds.y.data(), sizeof(float) * (size_t)n, hipMemcpyHostToDevice, s));
         launch_metric(s, kind, n, nct, d_y, d_out, d_scratch, d_m);
         float v = 0;
         HIP_CHECK(hipMemcpyAsync(&v, d_m, sizeof(float), hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipStreamSynchronize(s));
         log_info("%s = %g", names[kind], v);
-        HIP_CHECK(hipFree(d_y));
-        HIP_CHECK(hipFree(d_m));
-        HIP_CHECK(hipFree(d_scratch));
+        device_free(d_y);
+        device_free(d_m);
+        device_free(d_scratch);
     }
     if (transform) {
         const int kind = transform_kind(param.objective);
         if (kind == 1 || kind == 2) {
             const size_t need = kind == 1 ? 2 : (size_t)std::max(param.num_class, 1);
             TGBM_CHECK(ds.label.size() >= need, "predict: %zu class labels given, %zu needed", ds.label.size(), need);
-            HIP_CHECK(hipMalloc(&d_label, sizeof(float) * ds.label.size()));
+            device_alloc_to(d_label, sizeof(float) * ds.label.size());
             HIP_CHECK(hipMemcpyAsync(d_label, ds.label.data(), sizeof(float) * ds.label.size(), hipMemcpyHostToDevice, s));
         }
         launch_predict_transform(s, kind, n, kind == 2 || kind == 3 ? nct : param.num_class, d_label, d_out);
@@ -177,15 +175,15 @@ static std::vector<float> run_predict(const GBMParam &param, const std::vector<s
     if (n_ret) HIP_CHECK(hipMemcpyAsync(out.data(), d_out, sizeof(float) * n_ret, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     lap("transform and download");
-    HIP_CHECK(hipFree(d_val));
-    HIP_CHECK(hipFree(d_col));
-    HIP_CHECK(hipFree(d_row_ptr));
-    HIP_CHECK(hipFree(d_model));
-    HIP_CHECK(hipFree(d_packed));
-    if (d_compact) HIP_CHECK(hipFree(d_compact));
-    HIP_CHECK(hipFree(d_out));
-    if (d_label) HIP_CHECK(hipFree(d_label));
-    HIP_CHECK(hipStreamDestroy(s));
+    device_free(d_val);
+    device_free(d_col);
+    device_free(d_row_ptr);
+    device_free(d_model);
+    device_free(d_packed);
+    if (d_compact) device_free(d_compact);
+    device_free(d_out);
+    if (d_label) device_free(d_label);
+    stream_release(s);
     lap("release");
     return out;
 }

@@ -231,11 +231,14 @@ void exclusive_scan(hipStream_t s, const void *in, unsigned *out, long n, unsign
     if (sc.levels.size() <= level) sc.levels.resize(level + 1);
     ScanScratch::Level &lv = sc.levels[level];
     if (lv.cap < (size_t)tiles + 1) {
-        if (lv.sums) HIP_CHECK(hipFree(lv.sums));
-        if (lv.scanned) HIP_CHECK(hipFree(lv.scanned));
+        if (lv.cap > 0) {
+            HIP_CHECK(hipStreamSynchronize(s));  // (earlier scans of this stream may still use the smaller arrays)
+            device_free(lv.sums);
+            device_free(lv.scanned);
+        }
         lv.cap = (size_t)tiles + 1;
-        HIP_CHECK(hipMalloc(&lv.sums, sizeof(unsigned) * lv.cap));
-        HIP_CHECK(hipMalloc(&lv.scanned, sizeof(unsigned) * lv.cap));
+        device_alloc_to(lv.sums, sizeof(unsigned) * lv.cap);
+        device_alloc_to(lv.scanned, sizeof(unsigned) * lv.cap);
     }
     unsigned *sums = lv.sums, *sums_scanned = lv.scanned;  // the recursion may move sc.levels
     k_scan_tiles<FROM_KEYS><<<(unsigned)tiles, kBlock, 0, s>>>(in, out, n, sums);
@@ -442,7 +445,7 @@ int grid_for(size_t n, int cap = 8192) {
 // Cut points of the reference's HistCut::get_cut_points_single (src/thundergbm/hist_cut.cu:232-286).
 DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin) {
     DeviceCuts out;
-    HIP_CHECK(hipMalloc(&out.cut_row_ptr, sizeof(int) * (size_t)(F + 1)));
+    device_alloc_to(out.cut_row_ptr, sizeof(int) * (size_t)(F + 1));
     if (nnz == 0) {
         HIP_CHECK(hipMemsetAsync(out.cut_row_ptr, 0, sizeof(int) * (size_t)(F + 1), s));
         HIP_CHECK(hipStreamSynchronize(s));
@@ -451,8 +454,8 @@ DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, 
     }
     ScanScratch scratch;
     unsigned long long *keys[2];
-    HIP_CHECK(hipMalloc(&keys[0], sizeof(unsigned long long) * (size_t)nnz));
-    HIP_CHECK(hipMalloc(&keys[1], sizeof(unsigned long long) * (size_t)nnz));
+    device_alloc_to(keys[0], sizeof(unsigned long long) * (size_t)nnz);
+    device_alloc_to(keys[1], sizeof(unsigned long long) * (size_t)nnz);
     k_make_keys<<<grid_for(nnz), kBlock, 0, s>>>(nnz, d_val, d_col, keys[0]);
 
     int fid_bits = 0;
@@ -461,9 +464,9 @@ DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, 
     const long n_tiles = (nnz + kSortTile - 1) / kSortTile;
     const size_t n_counts = (size_t)256 * n_tiles;
     unsigned *counts = nullptr, *offsets = nullptr, *d_total = nullptr;
-    HIP_CHECK(hipMalloc(&counts, sizeof(unsigned) * n_counts));
-    HIP_CHECK(hipMalloc(&offsets, sizeof(unsigned) * (n_counts + 1)));
-    HIP_CHECK(hipMalloc(&d_total, sizeof(unsigned)));
+    device_alloc_to(counts, sizeof(unsigned) * n_counts);
+    device_alloc_to(offsets, sizeof(unsigned) * (n_counts + 1));
+    device_alloc_to(d_total, sizeof(unsigned));
     const unsigned sort_grid = (unsigned)((n_tiles + kWaves - 1) / kWaves);
     int cur = 0;
     for (int p = 0; p < passes; ++p) {
@@ -476,12 +479,12 @@ DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, 
     }
     const unsigned long long *sorted = keys[cur];
     unsigned *uidx = nullptr;
-    HIP_CHECK(hipMalloc(&uidx, sizeof(unsigned) * (size_t)nnz));
+    device_alloc_to(uidx, sizeof(unsigned) * (size_t)nnz);
     exclusive_scan<true>(s, sorted, uidx, nnz, d_total, scratch);
     long *estart = nullptr;
     unsigned *ustart = nullptr;
-    HIP_CHECK(hipMalloc(&estart, sizeof(long) * (size_t)(F + 1)));
-    HIP_CHECK(hipMalloc(&ustart, sizeof(unsigned) * (size_t)(F + 1)));
+    device_alloc_to(estart, sizeof(long) * (size_t)(F + 1));
+    device_alloc_to(ustart, sizeof(unsigned) * (size_t)(F + 1));
     k_feature_starts<<<grid_for(F + 1), kBlock, 0, s>>>(sorted, nnz, F, estart);
     k_unique_starts<<<grid_for(F + 1), kBlock, 0, s>>>(estart, uidx, nnz, F, d_total, ustart);
     std::vector<unsigned> h_ustart(F + 1);
@@ -499,20 +502,20 @@ DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, 
     }
     out.n_bins = h_crp[F];
     HIP_CHECK(hipMemcpyAsync(out.cut_row_ptr, h_crp.data(), sizeof(int) * (size_t)(F + 1), hipMemcpyHostToDevice, s));
-    HIP_CHECK(hipMalloc(&out.cut_val, sizeof(float) * (size_t)std::max(out.n_bins, 1)));
-    HIP_CHECK(hipMalloc(&out.cut_fid, sizeof(int) * (size_t)std::max(out.n_bins, 1)));
+    device_alloc_to(out.cut_val, sizeof(float) * (size_t)std::max(out.n_bins, 1));
+    device_alloc_to(out.cut_fid, sizeof(int) * (size_t)std::max(out.n_bins, 1));
     k_emit_cuts<<<grid_for(nnz), kBlock, 0, s>>>(sorted, uidx, nnz, ustart, out.cut_row_ptr, max_num_bin, out.cut_val,
                                                out.cut_fid);
     HIP_CHECK(hipStreamSynchronize(s));
     scratch.release();
-    HIP_CHECK(hipFree(keys[0]));
-    HIP_CHECK(hipFree(keys[1]));
-    HIP_CHECK(hipFree(counts));
-    HIP_CHECK(hipFree(offsets));
-    HIP_CHECK(hipFree(d_total));
-    HIP_CHECK(hipFree(uidx));
-    HIP_CHECK(hipFree(estart));
-    HIP_CHECK(hipFree(ustart));
+    device_free(keys[0]);
+    device_free(keys[1]);
+    device_free(counts);
+    device_free(offsets);
+    device_free(d_total);
+    device_free(uidx);
+    device_free(estart);
+    device_free(ustart);
     return out;
 }
 
@@ -539,13 +542,13 @@ __global__ __launch_bounds__(256) void k_min_max_int(const int *__restrict__ v, 
 int device_max_int(hipStream_t s, const int *d_v, long n) {
     if (n <= 0) return 0;
     int *d_out = nullptr;
-    HIP_CHECK(hipMalloc(&d_out, 2 * sizeof(int)));
+    device_alloc_to(d_out, 2 * sizeof(int));
     HIP_CHECK(hipMemsetAsync(d_out, 0, 2 * sizeof(int), s));
     k_min_max_int<<<grid_for((size_t)n, 4096), 256, 0, s>>>(d_v, n, d_out);
     int h[2] = {0, 0};
     HIP_CHECK(hipMemcpyAsync(h, d_out, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipFree(d_out));
+    device_free(d_out);
     TGBM_CHECK(h[1] >= 0, "CSR input: negative column index %d", h[1]);
     TGBM_CHECK(h[0] < 2147483647, "CSR input: column index %d leaves no room for the feature count", h[0]);
     return h[0];
@@ -642,8 +645,8 @@ void launch_cols_from_rows(hipStream_t s, int n, int W, int F, int n_blocks, con
 
 void ScanScratch::release() {
     for (Level &lv : levels) {
-        if (lv.sums) (void)hipFree(lv.sums);
-        if (lv.scanned) (void)hipFree(lv.scanned);
+        if (lv.sums) device_free(lv.sums);
+        if (lv.scanned) device_free(lv.scanned);
     }
     levels.clear();
 }
@@ -659,24 +662,24 @@ void PairSorter::alloc(long n) {
     n_tiles = (n + kSortTile - 1) / kSortTile;
     const size_t n_counts = (size_t)256 * (size_t)std::max(n_tiles, 1l);
     for (int b = 0; b < 2; ++b) {
-        HIP_CHECK(hipMalloc(&keys[b], sizeof(unsigned long long) * m));
-        HIP_CHECK(hipMalloc(&vals[b], sizeof(int) * m));
+        device_alloc_to(keys[b], sizeof(unsigned long long) * m);
+        device_alloc_to(vals[b], sizeof(int) * m);
     }
-    HIP_CHECK(hipMalloc(&counts, sizeof(unsigned) * n_counts));
-    HIP_CHECK(hipMalloc(&offsets, sizeof(unsigned) * (n_counts + 1)));
-    HIP_CHECK(hipMalloc(&d_total, sizeof(unsigned)));
+    device_alloc_to(counts, sizeof(unsigned) * n_counts);
+    device_alloc_to(offsets, sizeof(unsigned) * (n_counts + 1));
+    device_alloc_to(d_total, sizeof(unsigned));
 }
 
 void PairSorter::release() {
     for (int b = 0; b < 2; ++b) {
-        if (keys[b]) (void)hipFree(keys[b]);
-        if (vals[b]) (void)hipFree(vals[b]);
+        if (keys[b]) device_free(keys[b]);
+        if (vals[b]) device_free(vals[b]);
         keys[b] = nullptr;
         vals[b] = nullptr;
     }
-    if (counts) (void)hipFree(counts);
-    if (offsets) (void)hipFree(offsets);
-    if (d_total) (void)hipFree(d_total);
+    if (counts) device_free(counts);
+    if (offsets) device_free(offsets);
+    if (d_total) device_free(d_total);
     counts = offsets = d_total = nullptr;
     scan.release();
     cap = 0;
@@ -726,12 +729,12 @@ void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, 
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col) {
     if (n == 0) return true;
     int *d_flag = nullptr, h = 0;
-    HIP_CHECK(hipMalloc(&d_flag, sizeof(int)));
+    device_alloc_to(d_flag, sizeof(int));
     HIP_CHECK(hipMemsetAsync(d_flag, 0, sizeof(int), s));
     k_rows_ascend<<<grid_for((size_t)n * 16, 1 << 20), kBlock, 0, s>>>(n, row_ptr, col, d_flag);
     HIP_CHECK(hipMemcpyAsync(&h, d_flag, sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipFree(d_flag));
+    device_free(d_flag);
     return h == 0;
 }
 

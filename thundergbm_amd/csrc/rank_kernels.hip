@@ -277,7 +277,7 @@ int bits_for(long count) {
 template <typename T>
 T *RankContext::dalloc(size_t count) {
     void *p = nullptr;
-    HIP_CHECK(hipMalloc(&p, sizeof(T) * std::max<size_t>(count, 1)));
+    device_alloc_to(p, sizeof(T) * std::max<size_t>(count, 1));
     allocs_.push_back(p);
     return static_cast<T *>(p);
 }
@@ -390,7 +390,7 @@ RankContext::RankContext(hipStream_t s, const std::vector<float> &y, const std::
 
 RankContext::~RankContext() {
     sorter_.release();
-    for (void *p : allocs_) (void)hipFree(p);
+    for (void *p : allocs_) device_free(p);
 }
 
 void RankContext::gradient(const float *d_score, GHPair *d_gh, unsigned seed, bool order_is_fresh) {

@@ -17,7 +17,7 @@ template <typename T>
 T *Trainer::dalloc(size_t count) {
     void *p = nullptr;
     if (count == 0) count = 1;
-    HIP_CHECK(hipMalloc(&p, count * sizeof(T)));
+    device_alloc_to(p, count * sizeof(T));
     allocs_.push_back(p);
     return static_cast<T *>(p);
 }
@@ -71,7 +71,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     int n_dev = 0;
     hipError_t e = hipGetDeviceCount(&n_dev);
     TGBM_CHECK(e == hipSuccess && n_dev >= 1, "no HIP device available: this library has no CPU path");
-    HIP_CHECK(hipStreamCreate(&stream_));
+    stream_ = stream_acquire();
     n_ = (int)ds.n_instances();
     F_ = (int)ds.n_features();
     nnz_ = ds.nnz;
@@ -122,9 +122,9 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     // ---- upload CSR, cut points, bin matrix --------------------------------------------------
     float *d_val = nullptr;
     int *d_col = nullptr, *d_row_ptr = nullptr;
-    HIP_CHECK(hipMalloc(&d_val, sizeof(float) * (size_t)std::max(nnz_, 1l)));
-    HIP_CHECK(hipMalloc(&d_col, sizeof(int) * (size_t)std::max(nnz_, 1l)));
-    HIP_CHECK(hipMalloc(&d_row_ptr, sizeof(int) * (size_t)(n_ + 1)));
+    device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz_, 1l));
+    device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
+    device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
     auto t_up = std::chrono::steady_clock::now();
     upload_large(stream_, d_val, ds.val, sizeof(float) * (size_t)nnz_);
     upload_large(stream_, d_col, ds.col_idx, sizeof(int) * (size_t)nnz_);
@@ -157,7 +157,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     // n x F bytes twice). Sparse: CSR rows of global bin ids, for wide data whose rows store few values.
     const double density = (double)nnz_ / ((double)n_ * (double)F_);
     size_t free_b = 0, total_b = 0;
-    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    device_mem_info(&free_b, &total_b);
     const char *force = std::getenv("TGBM_LAYOUT");  // "dense" / "sparse" override the heuristic (tests)
     sparse_ = (F_ > 4096 && density < 0.05) || (size_t)n_ * F_ * 2 > free_b / 2 || n_ >= (1 << 29);
     if (force != nullptr && std::string(force) == "sparse") sparse_ = true;
@@ -225,14 +225,14 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         }
         if (!head_bin.empty()) {
             int *d_slot = nullptr;
-            HIP_CHECK(hipMalloc(&d_slot, sizeof(int) * (size_t)F_));
+            device_alloc_to(d_slot, sizeof(int) * (size_t)F_);
             upload(stream_, d_slot, feat_slot.data(), (size_t)F_);
             int *d_word = dalloc<int>((size_t)std::max(nnz_, 1l));
             int *d_head = dalloc<int>(head_bin.size());
             upload(stream_, d_head, head_bin.data(), head_bin.size());
             launch_bin_csr(stream_, nnz_, d_col, d_val, cuts_.cut_val, cuts_.cut_row_ptr, d_bin, d_slot, d_word);
             HIP_CHECK(hipStreamSynchronize(stream_));
-            HIP_CHECK(hipFree(d_slot));
+            device_free(d_slot);
             csr_.hist_word = d_word;
             csr_.head_bin = d_head;
             csr_.head_bins = (int)head_bin.size();
@@ -258,7 +258,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
                 for (int f = 0; f < F_; ++f)
                     for (int b = h_cut_row_ptr_[f]; b < h_cut_row_ptr_[f + 1]; ++b)
                         sort_key[(size_t)b] = sparse_feature_in_tables(f) ? h_cut_row_ptr_[f] : b;
-                HIP_CHECK(hipMalloc(&d_sort_key, sizeof(int) * (size_t)n_bins_));
+                device_alloc_to(d_sort_key, sizeof(int) * (size_t)n_bins_);
                 upload(stream_, d_sort_key, sort_key.data(), sort_key.size());
                 HIP_CHECK(hipStreamSynchronize(stream_));
             }
@@ -270,7 +270,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             launch_csc_unpack(stream_, nnz_, ps.keys[cur], ps.vals[cur], d_cbin, d_crow);
             HIP_CHECK(hipStreamSynchronize(stream_));
             ps.release();
-            if (d_sort_key != nullptr) HIP_CHECK(hipFree(d_sort_key));
+            if (d_sort_key != nullptr) device_free(d_sort_key);
             csr_.csc_bin = d_cbin;
             csr_.csc_row = d_crow;
             csr_.nnz = nnz_;
@@ -284,7 +284,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
                 if (cuts_.feature_nnz[f] > 0 && cuts_.feature_nnz[f] > kSortedTile) order.push_back(f);
             std::stable_sort(order.begin(), order.end(),
                              [&](int a, int b) { return cuts_.feature_nnz[a] > cuts_.feature_nnz[b]; });
-            HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+            device_mem_info(&free_b, &total_b);
             const size_t col_stride = ((size_t)n_ + 3) / 4 * 4;
             const char *ce2 = std::getenv("TGBM_SPARSE_COLS");  // "0": none (tests of the search path)
             size_t n_cols = std::min(order.size(), free_b / 8 / col_stride);
@@ -309,8 +309,8 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         bins_.W = 4;
         bins_.n_blocks = 1;
         HIP_CHECK(hipStreamSynchronize(stream_));
-        HIP_CHECK(hipFree(d_val));
-        HIP_CHECK(hipFree(d_col));
+        device_free(d_val);
+        device_free(d_col);
     } else {
         // dense column-blocked layout: blocks of W columns, each block n rows x W bins
         // Bundles: a run of consecutive features of which no row stores more than one (the columns of a one-hot
@@ -327,14 +327,14 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         // (rows that store every feature leave nothing to bundle)
         if (bin_bytes == 1 && F_ > 1 && nnz_ < (long)n_ * F_ && !(be != nullptr && std::string(be) == "0")) {
             int *d_next = nullptr;
-            HIP_CHECK(hipMalloc(&d_next, sizeof(int) * ((size_t)F_ + 1)));
+            device_alloc_to(d_next, sizeof(int) * ((size_t)F_ + 1));
             HIP_CHECK(hipMemsetAsync(d_next, 0x7f, sizeof(int) * (size_t)F_, stream_));  // 0x7f7f7f7f: above every column
             HIP_CHECK(hipMemsetAsync(d_next + F_, 0, sizeof(int), stream_));
             launch_min_next_col(stream_, n_, d_row_ptr, d_col, d_next, d_next + F_);
             std::vector<int> next((size_t)F_ + 1);
             HIP_CHECK(hipMemcpyAsync(next.data(), d_next, sizeof(int) * next.size(), hipMemcpyDeviceToHost, stream_));
             HIP_CHECK(hipStreamSynchronize(stream_));
-            HIP_CHECK(hipFree(d_next));
+            device_free(d_next);
             rows_ascend = next[F_] == 0;
             ascend_known = true;
             if (next[F_] == 0) {  // (rows whose columns do not ascend: the argument above does not hold)
@@ -450,9 +450,9 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             }
         }
         HIP_CHECK(hipStreamSynchronize(stream_));
-        HIP_CHECK(hipFree(d_val));
-        HIP_CHECK(hipFree(d_col));
-        HIP_CHECK(hipFree(d_row_ptr));
+        device_free(d_val);
+        device_free(d_col);
+        device_free(d_row_ptr);
     }
 
     // ---- labels, predictions, gradients (Booster::init) --------------------------------------
@@ -523,7 +523,7 @@ void Trainer::alloc_tree_buffers() {
     // buffer - all of the deepest level when that fits, else the largest power of two that does - and deeper levels
     // are served in batches of that many nodes (find_split_sets). TGBM_HIST_ARENA_NODES caps it (tests).
     size_t free_b = 0, total_b = 0;
-    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    device_mem_info(&free_b, &total_b);
     int hist_nodes = max_level_nodes;
     const size_t fixed_bytes = sparse_pass_ ? 0 : (size_t)n_ * 13 + tb.n_end_bound * sizeof(int);
     auto arena_bytes = [&](int nodes) {  // two buffers + the work items' partial histograms (dense layout)
@@ -663,7 +663,7 @@ void Trainer::alloc_tree_buffers() {
         sp_.partial = dalloc<longlong2>(S * (size_t)sp_.n_partial_slots * sp_.partial_stride);
         // per-value gradient pairs in the order of the bin-major copy, when they fit comfortably
         sp_.nnz = nnz_;
-        HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+        device_mem_info(&free_b, &total_b);
         const char *ge = std::getenv("TGBM_SPARSE_GH_COPY");  // "0": gather the pairs per value instead (tests)
         if (S * (size_t)nnz_ * sizeof(GHPair) < free_b / 4 && !(ge != nullptr && std::string(ge) == "0"))
             sp_.csc_gh = dalloc<GHPair>(S * (size_t)nnz_);
@@ -716,8 +716,8 @@ Trainer::~Trainer() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     for (auto &m : marks_) (void)hipEventDestroy(m.ev);
     reorder_sorter_.release();
-    for (void *p : allocs_) (void)hipFree(p);
-    if (stream_) (void)hipStreamDestroy(stream_);
+    for (void *p : allocs_) device_free(p);
+    if (stream_) stream_release(stream_);
 }
 
 void Trainer::sync() { HIP_CHECK(hipStreamSynchronize(stream_)); }
@@ -838,7 +838,7 @@ void Trainer::ensure_hist_arena() {
     if (tb_.hist_q[0] != nullptr) return;
     const size_t cells = (size_t)n_sets_ * tb_.max_level_nodes * n_bins_;
     size_t free_b = 0, total_b = 0;
-    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    device_mem_info(&free_b, &total_b);
     TGBM_CHECK(cells * 2 * sizeof(longlong2) < free_b / 2,
                "per-node histograms for stage-wise inspection need %zu bytes (free %zu); use tgbm_trainer_boost",
                cells * 2 * sizeof(longlong2), free_b);
@@ -860,7 +860,7 @@ bool Trainer::sparse_feature_in_tables(int f) {
         // the sorted pass keeps 40 bytes per stored value of its features for every class tree built together;
         // it is left out when that would take more than a quarter of the free memory
         size_t free_b = 0, total_b = 0;
-        HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+        device_mem_info(&free_b, &total_b);
         if ((size_t)nnz_ * 40 * (size_t)std::max(1, param_.tree_per_rounds) > free_b / 4) sparse_sorted_on_ = false;
     }
     return !sparse_sorted_on_ || cuts_.feature_nnz[f] > kSortedTile || f == sparse_bin0_owner_;
@@ -1374,7 +1374,7 @@ int Trainer::info(const std::string &key) const {
     if (key == "reorders_done") return reorders_done_;
     if (key == "device_free_mb") {
         size_t free_b = 0, total_b = 0;
-        HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+        device_mem_info(&free_b, &total_b);
         return (int)(free_b >> 20);
     }
     if (key == "dense_blocks") return bins_.n_blocks;

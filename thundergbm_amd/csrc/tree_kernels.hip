@@ -2440,23 +2440,23 @@ void launch_root_sum(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_clas
 
 long device_count_bytes(hipStream_t s, const uint8_t *d_v, size_t n, uint8_t value) {
     unsigned long long *d_out = nullptr, h = 0;
-    HIP_CHECK(hipMalloc(&d_out, sizeof(unsigned long long)));
+    device_alloc_to(d_out, sizeof(unsigned long long));
     HIP_CHECK(hipMemsetAsync(d_out, 0, sizeof(unsigned long long), s));
     k_count_bytes<<<grid_for(n, 2048), kBlock, 0, s>>>(d_v, n, value, d_out);
     HIP_CHECK(hipMemcpyAsync(&h, d_out, sizeof(h), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipFree(d_out));
+    device_free(d_out);
     return (long)h;
 }
 
 long device_count_u16(hipStream_t s, const uint16_t *d_v, size_t n, uint16_t value) {
     unsigned long long *d_out = nullptr, h = 0;
-    HIP_CHECK(hipMalloc(&d_out, sizeof(unsigned long long)));
+    device_alloc_to(d_out, sizeof(unsigned long long));
     HIP_CHECK(hipMemsetAsync(d_out, 0, sizeof(unsigned long long), s));
     k_count_u16<<<grid_for(n, 2048), kBlock, 0, s>>>(d_v, n, value, d_out);
     HIP_CHECK(hipMemcpyAsync(&h, d_out, sizeof(h), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipFree(d_out));
+    device_free(d_out);
     return (long)h;
 }
 
