@@ -46,6 +46,17 @@ void sparse_train_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, f
                          float learning_rate, char *obj_type, int *num_class, char *tree_method, tgbm_model **model,
                          int *tree_per_iter, float *group_label, int *group, int num_group);
 
+/* sparse_train_scikit for a dense matrix x: float (x_is_double 0) or double [row_size][columns], row by row, fewer than
+ * 2^32 cells. A zero is a value that is not stored, as for the reference's wrapper, which drops the zeros of dense input
+ * on its way to CSR (thundergbm.py:98-103); doubles are trained on as floats. group_label has row_size slots, n_distinct
+ * receives the number of distinct labels. The other arguments and the model are those of sparse_train_scikit on the same
+ * data. It has no counterpart in the reference. */
+void tgbm_train_dense(int row_size, int columns, const void *x, int x_is_double, const float *label, int depth,
+                      int n_trees, int n_device, float min_child_weight, float lambda, float gamma, int max_num_bin,
+                      int verbose, float column_sampling_rate, int bagging, int n_parallel_trees, float learning_rate,
+                      const char *obj_type, int *num_class, const char *tree_method, tgbm_model **model,
+                      int *tree_per_iter, float *group_label, int *n_distinct, const int *group, int num_group);
+
 /* scikit_tgbm.cpp:83-121. y_pred: row_size floats, or row_size * num_class (class-major) for
  * multi:softprob. As in the reference the base score is not part of this path. group / num_group: query
  * groups of the rows for a ranking objective; they only feed the metric line of the log and may be absent. */

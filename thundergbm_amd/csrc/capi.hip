@@ -3,6 +3,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <thread>
 
 #include "../../include/thundergbm.h"
 #include "model_handle.h"
@@ -40,18 +41,9 @@ tgbm_model *from_nested(const std::vector<std::vector<Tree>> &nested) {
     return m;
 }
 
-}  // namespace
-
-extern "C" {
-
-void set_logger(int verbose) { g_verbose = verbose; }
-
-void sparse_train_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, float *label, int depth, int n_trees,
-                         int n_device, float min_child_weight, float lambda, float gamma, int max_num_bin,
-                         int verbose, float column_sampling_rate, int bagging, int n_parallel_trees,
-                         float learning_rate, char *obj_type, int *num_class, char *tree_method, tgbm_model **model,
-                         int *tree_per_iter, float *group_label, int *group, int num_group) {
-    std::lock_guard<std::mutex> lock(g_call_mutex);
+GBMParam train_param(int depth, int n_trees, int n_device, float min_child_weight, float lambda, float gamma,
+                     int max_num_bin, int verbose, float column_sampling_rate, int bagging, int n_parallel_trees,
+                     float learning_rate, const char *obj_type, int num_class, const char *tree_method) {
     GBMParam p;
     p.depth = depth;
     p.n_trees = n_trees;
@@ -66,22 +58,99 @@ void sparse_train_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, f
     p.n_parallel_trees = n_parallel_trees;
     p.learning_rate = learning_rate;
     p.objective = obj_type;
-    p.num_class = *num_class;
+    p.num_class = num_class;
     p.tree_method = tree_method;
     p.rt_eps = 1e-6f;
     p.tree_per_rounds = 1;
-    set_logger(verbose);
-    DataSet ds;
-    auto t0 = std::chrono::steady_clock::now();
-    ds.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false);
-    log_debug("host-side dataset checks and label grouping: %.3f s",
-              std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+    g_verbose = verbose;
+    return p;
+}
+
+void run_train(GBMParam &p, const DataSet &ds, int *num_class, tgbm_model **model, int *tree_per_iter,
+               float *group_label) {
+    const int n_trees = p.n_trees;
     *num_class = p.num_class;
     std::vector<std::vector<Tree>> boosted = train(p, ds);
     TGBM_CHECK((int)boosted.size() == n_trees, "%d v.s. %zu", n_trees, boosted.size());
     *tree_per_iter = (int)boosted[0].size();
     *model = from_nested(boosted);
     for (size_t i = 0; i < ds.label.size(); ++i) group_label[i] = ds.label[i];
+}
+
+// Distinct values among the labels (NaNs count as one, as do the two zeros): open addressing in a table that grows with
+// what it holds, so that the usual handful of classes stays in the L1.
+int count_distinct(const float *v, int n) {
+    std::vector<unsigned> table(1024, 0u);
+    size_t mask = table.size() - 1, held = 0;
+    bool zero_seen = false;
+    unsigned last = 0;
+    auto slot_of = [&](unsigned key) {
+        size_t at = (size_t)(key * 0x9e3779b97f4a7c15ull >> 24) & mask;
+        while (table[at] != 0 && table[at] != key) at = (at + 1) & mask;
+        return at;
+    };
+    for (int i = 0; i < n; ++i) {
+        unsigned key;
+        std::memcpy(&key, v + i, 4);
+        if (v[i] == 0.f) {  // (the table's mark of a free slot)
+            zero_seen = true;
+            continue;
+        }
+        if (v[i] != v[i]) key = 0x7fc00000u;
+        if (key == last) continue;
+        last = key;
+        size_t at = slot_of(key);
+        if (table[at] == key) continue;
+        table[at] = key;
+        if (++held * 2 > table.size()) {
+            std::vector<unsigned> old(table.size() * 4, 0u);
+            old.swap(table);
+            mask = table.size() - 1;
+            for (unsigned k : old)
+                if (k != 0) table[slot_of(k)] = k;
+        }
+    }
+    return (int)held + (zero_seen ? 1 : 0);
+}
+
+}  // namespace
+
+extern "C" {
+
+void set_logger(int verbose) { g_verbose = verbose; }
+
+void sparse_train_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, float *label, int depth, int n_trees,
+                         int n_device, float min_child_weight, float lambda, float gamma, int max_num_bin,
+                         int verbose, float column_sampling_rate, int bagging, int n_parallel_trees,
+                         float learning_rate, char *obj_type, int *num_class, char *tree_method, tgbm_model **model,
+                         int *tree_per_iter, float *group_label, int *group, int num_group) {
+    std::lock_guard<std::mutex> lock(g_call_mutex);
+    GBMParam p = train_param(depth, n_trees, n_device, min_child_weight, lambda, gamma, max_num_bin, verbose,
+                             column_sampling_rate, bagging, n_parallel_trees, learning_rate, obj_type, *num_class, tree_method);
+    DataSet ds;
+    auto t0 = std::chrono::steady_clock::now();
+    ds.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false);
+    log_debug("host-side dataset checks and label grouping: %.3f s",
+              std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+    run_train(p, ds, num_class, model, tree_per_iter, group_label);
+}
+
+void tgbm_train_dense(int row_size, int columns, const void *x, int x_is_double, const float *label, int depth,
+                      int n_trees, int n_device, float min_child_weight, float lambda, float gamma, int max_num_bin,
+                      int verbose, float column_sampling_rate, int bagging, int n_parallel_trees, float learning_rate,
+                      const char *obj_type, int *num_class, const char *tree_method, tgbm_model **model,
+                      int *tree_per_iter, float *group_label, int *n_distinct, const int *group, int num_group) {
+    std::lock_guard<std::mutex> lock(g_call_mutex);
+    GBMParam p = train_param(depth, n_trees, n_device, min_child_weight, lambda, gamma, max_num_bin, verbose,
+                             column_sampling_rate, bagging, n_parallel_trees, learning_rate, obj_type, *num_class, tree_method);
+    // (counted by a thread of its own: the calling thread mostly waits for the device)
+    std::thread counter;
+    if (row_size > 4096) counter = std::thread([&] { *n_distinct = count_distinct(label, row_size); });
+    else *n_distinct = count_distinct(label, row_size);
+    DataSet ds;
+    ds.load_from_dense(row_size, columns, x, x_is_double != 0, label, group, num_group, p);
+    run_train(p, ds, num_class, model, tree_per_iter, group_label);
+    if (counter.joinable()) counter.join();
 }
 
 void sparse_predict_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, float *y_pred, tgbm_model **model,

@@ -514,9 +514,25 @@ void launch_cols_from_rows(hipStream_t s, int n, int W, int F, int n_blocks, con
 // Largest of n ints in device memory (synchronises; 0 for n == 0); aborts when one of them is negative.
 int device_max_int(hipStream_t s, const int *d_v, long n);
 
-// Host -> device copy of a pageable array on stream s; large ones go through pinned staging buffers and are
-// complete on return, small ones (< 128 MB) are a plain stream-ordered hipMemcpyAsync.
+// Host -> device copy of a pageable array, stream-ordered on s; large ones go through pinned staging pieces. The source
+// has been read when the call returns.
 void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes);
+// The same for doubles that the device takes as floats. Zeros of either sign arrive as +0, other values that are too
+// small for a float as -0.
+void upload_doubles_as_floats(hipStream_t s, float *dst, const double *src, size_t count);
+void release_transfer_memory();  // the pinned pieces that are kept for later copies
+
+// CSR form of a dense row-major matrix [n][columns] on the device: the stored values are those that are not zero
+// (NaN is stored); with minus_zero_is_stored -0 is a stored zero (upload_doubles_as_floats).
+struct DeviceCsr {
+    float *val = nullptr;
+    int *col = nullptr;
+    int *row_ptr = nullptr;
+    long nnz = 0;
+    int n_features = 1;  // largest column with a stored value + 1, at least 1
+};
+// Takes `x` over (it becomes the value array when every cell is stored, and is freed otherwise). Synchronises.
+DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored);
 
 // prediction of the n rows that row_ptr addresses (entry offsets into col / val); out[t * out_stride + i] for
 // class tree t and row i, out_stride = 0 means n (a slice of a larger row set passes the whole set's size)

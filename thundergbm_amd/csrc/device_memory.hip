@@ -186,4 +186,7 @@ void release_device_memory() {
 
 }  // namespace tgbm
 
-extern "C" void tgbm_release_memory(void) { tgbm::release_device_memory(); }
+extern "C" void tgbm_release_memory(void) {
+    tgbm::release_device_memory();
+    tgbm::release_transfer_memory();
+}

@@ -21,6 +21,12 @@ struct DataSet {
     const int *row_ptr = nullptr;
     const int *col_idx = nullptr;
     long nnz = 0;
+    // A dense row-major matrix instead (load_from_dense): zeros are values that are not stored. The device makes the CSR
+    // form of it; row_ptr, val, col_idx and nnz stay empty.
+    const float *dense_f32 = nullptr;
+    const double *dense_f64 = nullptr;
+    int dense_columns = 0;
+    bool is_dense() const { return dense_columns > 0; }
     std::vector<float> y;
     std::vector<float> label;  // distinct class labels, ascending
     std::vector<int> group;
@@ -37,12 +43,19 @@ struct DataSet {
     void load_from_sparse(int n_instances, const float *csr_val, const int *csr_row_ptr, const int *csr_col_idx,
                           const float *y, const int *group, int num_group, GBMParam &param,
                           bool count_features = true);
+    // x: float or double [n_rows][columns]; the caller's buffer, like the CSR arrays
+    void load_from_dense(int n_rows, int columns, const void *x, bool doubles, const float *labels, const int *group,
+                         int num_group, GBMParam &param);
     // src/thundergbm/dataset.cpp:170-320 (LIBSVM text, 1-based feature ids)
     void load_from_file(const std::string &file_name, GBMParam &param);
     // src/thundergbm/dataset.cpp:83-101
     void group_label();
     // src/thundergbm/dataset.cpp:71-81 (sizes of the query groups, one number per token)
     void load_group_file(const std::string &file_name);
+
+   private:
+    void take_labels(int n_rows, const float *labels);
+    void finish_load(bool labelled, const int *grp, int num_group, GBMParam &param);
 };
 
 bool objective_needs_group_label(const std::string &objective);

@@ -62,18 +62,13 @@ bool objective_supported(const std::string &o) {
 void DataSet::load_from_sparse(int n_rows, const float *val, const int *row_ptr, const int *col_idx,
                                const float *labels, const int *grp, int num_group, GBMParam &param,
                                bool count_features) {
-    n_features_ = 0;
-    y.clear();
-    label.clear();
-    group.clear();
     TGBM_CHECK(n_rows >= 0 && row_ptr != nullptr, "CSR input: %d rows", n_rows);
     TGBM_CHECK(row_ptr[0] == 0, "CSR input: row_ptr[0] is %d, expected 0", row_ptr[0]);
     for (int i = 0; i < n_rows; ++i)
         TGBM_CHECK(row_ptr[i + 1] >= row_ptr[i], "CSR input: row_ptr decreases at row %d (%d -> %d)", i, row_ptr[i],
                    row_ptr[i + 1]);
     const int nnz = row_ptr[n_rows];
-    y.assign(n_rows, 0.f);
-    if (labels != nullptr) std::copy(labels, labels + n_rows, y.begin());
+    take_labels(n_rows, labels);
     this->val = val;
     this->row_ptr = row_ptr;
     this->col_idx = col_idx;
@@ -104,7 +99,30 @@ void DataSet::load_from_sparse(int n_rows, const float *val, const int *row_ptr,
         n_features_ = (size_t)max_col + 1;
         log_info("#instances = %zu, #features = %zu", n_instances(), n_features());
     }
-    if (labels != nullptr && objective_needs_group_label(param.objective)) {
+    finish_load(labels != nullptr, grp, num_group, param);
+}
+
+void DataSet::load_from_dense(int n_rows, int columns, const void *x, bool doubles, const float *labels, const int *grp,
+                              int num_group, GBMParam &param) {
+    TGBM_CHECK(n_rows > 0 && columns > 0 && x != nullptr, "dense input of %d x %d", n_rows, columns);
+    take_labels(n_rows, labels);
+    dense_f32 = doubles ? nullptr : static_cast<const float *>(x);
+    dense_f64 = doubles ? static_cast<const double *>(x) : nullptr;
+    dense_columns = columns;
+    features_counted = false;
+    finish_load(labels != nullptr, grp, num_group, param);
+}
+
+void DataSet::take_labels(int n_rows, const float *labels) {
+    n_features_ = 0;
+    label.clear();
+    group.clear();
+    if (labels != nullptr) y.assign(labels, labels + n_rows);
+    else y.assign(n_rows, 0.f);
+}
+
+void DataSet::finish_load(bool labelled, const int *grp, int num_group, GBMParam &param) {
+    if (labelled && objective_needs_group_label(param.objective)) {
         group_label();
         param.num_class = (int)label.size();
     }

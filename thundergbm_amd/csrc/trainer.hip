@@ -5,7 +5,6 @@
 #include "trainer.h"
 
 #include <algorithm>
-#include <thread>
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
@@ -26,45 +25,6 @@ template <typename T>
 static T *upload(hipStream_t s, T *dst, const T *src, size_t count) {
     if (count) HIP_CHECK(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyHostToDevice, s));
     return dst;
-}
-
-// Host -> device copy of a large pageable array: chunks are copied by a few host threads into two pinned
-// staging buffers and sent with asynchronous DMA, so the host copy of one chunk overlaps the transfer of
-// the previous one (a plain hipMemcpy of pageable memory stages through one thread).
-void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
-    constexpr size_t kChunk = (size_t)32 << 20;
-    if (bytes < 4 * kChunk) {
-        if (bytes) HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-        return;
-    }
-    void *pin[2] = {nullptr, nullptr};
-    hipEvent_t done[2];
-    for (int b = 0; b < 2; ++b) {
-        HIP_CHECK(hipHostMalloc(&pin[b], kChunk, hipHostMallocDefault));
-        HIP_CHECK(hipEventCreateWithFlags(&done[b], hipEventDisableTiming));
-    }
-    const int n_thr = (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
-    size_t off = 0;
-    for (int i = 0; off < bytes; ++i, off += kChunk) {
-        const int b = i & 1;
-        const size_t len = std::min(kChunk, bytes - off);
-        if (i >= 2) HIP_CHECK(hipEventSynchronize(done[b]));  // the DMA that last read this buffer
-        std::vector<std::thread> pool;
-        auto part = [&](int t) {
-            const size_t pb = len * t / n_thr, pe = len * (t + 1) / n_thr;
-            std::memcpy(static_cast<char *>(pin[b]) + pb, static_cast<const char *>(src) + off + pb, pe - pb);
-        };
-        for (int t = 1; t < n_thr; ++t) pool.emplace_back(part, t);
-        part(0);
-        for (auto &th : pool) th.join();
-        HIP_CHECK(hipMemcpyAsync(static_cast<char *>(dst) + off, pin[b], len, hipMemcpyHostToDevice, s));
-        HIP_CHECK(hipEventRecord(done[b], s));
-    }
-    HIP_CHECK(hipStreamSynchronize(s));
-    for (int b = 0; b < 2; ++b) {
-        HIP_CHECK(hipEventDestroy(done[b]));
-        HIP_CHECK(hipHostFree(pin[b]));
-    }
 }
 
 Trainer::Trainer(const DataSet &ds, GBMParam &param) {
@@ -122,17 +82,34 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     // ---- upload CSR, cut points, bin matrix --------------------------------------------------
     float *d_val = nullptr;
     int *d_col = nullptr, *d_row_ptr = nullptr;
-    device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz_, 1l));
-    device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
-    device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
     auto t_up = std::chrono::steady_clock::now();
-    upload_large(stream_, d_val, ds.val, sizeof(float) * (size_t)nnz_);
-    upload_large(stream_, d_col, ds.col_idx, sizeof(int) * (size_t)nnz_);
-    upload(stream_, d_row_ptr, ds.row_ptr, (size_t)n_ + 1);
-    HIP_CHECK(hipStreamSynchronize(stream_));
+    bool rows_ascend = true, ascend_known = false;
+    if (ds.is_dense()) {
+        const size_t cells = (size_t)n_ * ds.dense_columns;
+        float *d_x = nullptr;
+        device_alloc_to(d_x, sizeof(float) * cells);
+        if (ds.dense_f64 != nullptr) upload_doubles_as_floats(stream_, d_x, ds.dense_f64, cells);
+        else upload_large(stream_, d_x, ds.dense_f32, sizeof(float) * cells);
+        const DeviceCsr csr = dense_to_csr(stream_, n_, ds.dense_columns, d_x, ds.dense_f64 != nullptr);
+        d_val = csr.val;
+        d_col = csr.col;
+        d_row_ptr = csr.row_ptr;
+        nnz_ = csr.nnz;
+        F_ = csr.n_features;
+        rows_ascend = ascend_known = true;
+        log_info("#instances = %d, #features = %d", n_, F_);
+    } else {
+        device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz_, 1l));
+        device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
+        device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
+        upload_large(stream_, d_val, ds.val, sizeof(float) * (size_t)nnz_);
+        upload_large(stream_, d_col, ds.col_idx, sizeof(int) * (size_t)nnz_);
+        upload(stream_, d_row_ptr, ds.row_ptr, (size_t)n_ + 1);
+        HIP_CHECK(hipStreamSynchronize(stream_));
+    }
     log_debug("upload of %.2f GB: %.3f s", (double)nnz_ * 8e-9,
               std::chrono::duration<double>(std::chrono::steady_clock::now() - t_up).count());
-    if (!ds.features_counted) {  // the number of features = largest column index + 1 (dataset.cpp:40-46)
+    if (!ds.is_dense() && !ds.features_counted) {  // the number of features = largest column index + 1 (dataset.cpp:40-46)
         F_ = device_max_int(stream_, d_col, nnz_) + 1;
         log_info("#instances = %d, #features = %d", n_, F_);
     }
@@ -319,8 +296,6 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         // a row), so the smallest successor of every column decides: one pass over the column indices.
         h_col_bin_begin_ = h_cut_row_ptr_;
         int P = F_;  // columns of the matrix
-        bool rows_ascend = true;
-        bool ascend_known = false;
         std::vector<int> h_feat_col;
         std::vector<uint8_t> h_feat_lo;
         const char *be = std::getenv("TGBM_BUNDLE");  // "0": one column per feature (tests, measurements)

@@ -30,8 +30,24 @@ def _csr(X):
     return X
 
 
+def _dense(X):
+    """X as a C-contiguous float32 or float64 matrix for the entry points that take dense data as it is, or None where
+    the conversion to CSR has to decide (sparse input, other shapes and types). Types that float32 holds as well as the
+    CSR path's own cast go in as float32."""
+    if sp.issparse(X):
+        return None
+    X = np.asarray(X)
+    if X.ndim != 2 or X.size == 0 or X.size >= 1 << 32:
+        return None
+    if X.dtype.kind in "iub" or X.dtype == np.float16:
+        X = X.astype(np.float32)
+    if X.dtype != np.float32 and X.dtype != np.float64:
+        return None
+    return np.ascontiguousarray(X)
+
+
 def _ptr(a):
-    return a.ctypes.data_as(C.c_void_p)
+    return C.c_void_p(a.ctypes.data)
 
 
 def _stored_label_count(model_path):
@@ -72,10 +88,13 @@ class TGBMModel(BaseEstimator):
     def fit(self, X, y, groups=None):
         lib = _lib.load()
         self._release()
-        X = _csr(X)
+        dense = _dense(X)
+        X = _csr(X) if dense is None else dense
         y = np.ascontiguousarray(y, dtype=np.float32)
         if X.shape[0] != len(y):
             raise ValueError("X and y have different numbers of rows")
+        if dense is not None:
+            return self._fit_dense(lib, X, y, groups)
         indptr = np.ascontiguousarray(X.indptr, dtype=np.int32)
         indices = np.ascontiguousarray(X.indices, dtype=np.int32)
         n_labels = len(np.unique(y))
@@ -95,6 +114,27 @@ class TGBMModel(BaseEstimator):
         self.num_class = n_class[0]
         self.tree_per_iter = per_iter[0]
         self.group_label = [group_label[i] for i in range(n_labels)]
+        if not self.model:
+            raise RuntimeError("The model returned is empty!")
+        return self
+
+    def _fit_dense(self, lib, X, y, groups):
+        group_label = np.zeros(len(y), dtype=np.float32)
+        n_labels = C.c_int(0)
+        n_class = C.c_int(self.num_class)
+        per_iter = C.c_int(0)
+        self.model = C.c_void_p(None)
+        grp = None if groups is None else np.ascontiguousarray(groups, dtype=np.int32)
+        lib.tgbm_train_dense(X.shape[0], X.shape[1], _ptr(X), int(X.dtype == np.float64), _ptr(y), self.depth,
+                             self.n_trees, self.n_gpus, self.min_child_weight, self.lambda_tgbm, self.gamma,
+                             self.max_num_bin, self.verbose, self.column_sampling_rate, int(self.bagging),
+                             self.n_parallel_trees, self.learning_rate, self.objective.encode("utf-8"),
+                             C.byref(n_class), self.tree_method.encode("utf-8"), C.byref(self.model),
+                             C.byref(per_iter), _ptr(group_label), C.byref(n_labels),
+                             None if grp is None else _ptr(grp), 0 if grp is None else len(grp))
+        self.num_class = n_class.value
+        self.tree_per_iter = per_iter.value
+        self.group_label = group_label[: n_labels.value].tolist()
         if not self.model:
             raise RuntimeError("The model returned is empty!")
         return self
