@@ -64,6 +64,12 @@ void sparse_predict_scikit(int row_size, float *val, int *row_ptr, int *col_ptr,
                            int n_trees, int trees_per_iter, char *objective, int num_class, float learning_rate,
                            float *group_label, int *group, int num_group, int verbose);
 
+/* sparse_predict_scikit for a dense matrix (x, x_is_double: see tgbm_train_dense). The predictions are those of
+ * sparse_predict_scikit on the same data. It has no counterpart in the reference. */
+void tgbm_predict_dense(int row_size, int columns, const void *x, int x_is_double, float *y_pred, tgbm_model **model,
+                        int n_trees, int trees_per_iter, const char *objective, int num_class, float learning_rate,
+                        const float *group_label, const int *group, int num_group, int verbose);
+
 /* scikit_tgbm.cpp:123-147 / parser.cpp:146-171: raw binary model file. */
 void save(char *model_path, char *objective, float learning_rate, int num_class, int n_trees, int trees_per_iter,
           tgbm_model **model, float *group_label);

@@ -57,3 +57,50 @@ def test_dense_fit_of_classes_and_groups_equals_csr_fit():
             mm.fit(XX, labels, groups=groups)
         assert trees_of(m[0]) == trees_of(m[1]), objective
         assert m[0].group_label == m[1].group_label and m[0].num_class == m[1].num_class
+
+
+@pytest.mark.parametrize("n,F,used,classes,depth,n_iter", [
+    (1, 3, 3, 1, 1, 1), (1, 40, 40, 1, 6, 300), (257, 20, 20, 4, 4, 70), (1025, 50, 50, 1, 8, 11), (3000, 97, 97, 1, 5, 9),
+    (1500, 700, 300, 3, 6, 20)])
+def test_scoring_kernels_agree(n, F, used, classes, depth, n_iter):
+    """Dense rows and their CSR form, a thread per row and a group of lanes per row, and the walk of the 48-byte nodes:
+    the same bits, below and above the 96 features where the sums change from double to float."""
+    import ctypes as C
+    import datasets as D
+    import thundergbm_amd as T
+    L = T.load()
+    rng = np.random.default_rng(n + F)
+    X = rng.standard_normal((4000, F)).astype(np.float32)
+    X[:, used:] *= 1e-3
+    X[rng.random(X.shape) < 0.1] = 0
+    z = X[:, :used] @ rng.standard_normal(used)
+    y = np.digitize(z, np.quantile(z, np.linspace(0, 1, classes + 1)[1:-1])).astype(np.float32) if classes > 1 else z
+    m = (T.TGBMClassifier if classes > 1 else T.TGBMRegressor)(
+        depth=depth, n_trees=n_iter, learning_rate=0.3, verbose=0, objective="multi:softprob" if classes > 1 else "reg:linear")
+    m.fit(X, y)
+    Xt = rng.standard_normal((n, F)).astype(np.float64)
+    Xt[rng.random(Xt.shape) < 0.2] = 0
+    Xt.reshape(-1)[::37] = np.inf
+    Xt.reshape(-1)[1::41] = np.nan
+    Xt.reshape(-1)[2::43] = -1e-70
+    csr = sp.csr_matrix(Xt)
+    want, got = None, {}
+    val, rp, col = csr.data.astype(np.float32), csr.indptr.astype(np.int32), csr.indices.astype(np.int32)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    try:
+        for name, env in (("nodes", {"TGBM_PREDICT_TPS": "0"}), ("rows", {"TGBM_PREDICT_GROUP": "0"}),
+                          ("group", {"TGBM_PREDICT_GROUP": "1"}), ("default", {})):
+            os.environ.update(env)
+            raw = np.zeros(n * m.tree_per_iter, np.float32)
+            L.tgbm_predict_raw(n, p(val), p(rp), p(col), m.model, n_iter, m.tree_per_iter, 0.3, 0.25, p(raw))
+            got[name] = (raw, m.predict(Xt).copy(), m.predict(csr).copy(), m.predict(Xt.astype(np.float32)).copy())
+            for k in env:
+                os.environ.pop(k)
+    finally:
+        for k in ("TGBM_PREDICT_TPS", "TGBM_PREDICT_GROUP"):
+            os.environ.pop(k, None)
+    want = got["nodes"]
+    for name, outs in got.items():
+        for a, b in zip(outs, want):
+            assert np.array_equal(a, b, equal_nan=True), name
+        assert np.array_equal(outs[1], outs[2], equal_nan=True), name

@@ -19,6 +19,8 @@ SIGNATURES = {
                                 C.c_char_p, _P, _P, _P, _P, _P, C.c_int]),
     "sparse_predict_scikit": (None, [C.c_int, _P, _P, _P, _P, _P, C.c_int, C.c_int, C.c_char_p, C.c_int, C.c_float,
                                      _P, _P, C.c_int, C.c_int]),
+    "tgbm_predict_dense": (None, [C.c_int, C.c_int, _P, C.c_int, _P, _P, C.c_int, C.c_int, C.c_char_p, C.c_int, C.c_float,
+                                  _P, _P, C.c_int, C.c_int]),
     "save": (None, [C.c_char_p, C.c_char_p, C.c_float, C.c_int, C.c_int, C.c_int, _P, _P]),
     "load_model": (None, [C.c_char_p, _P, _P, _P, _P, _P]),
     "load_config": (None, [C.c_char_p, _P]),

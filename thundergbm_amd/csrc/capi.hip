@@ -77,6 +77,24 @@ void run_train(GBMParam &p, const DataSet &ds, int *num_class, tgbm_model **mode
     for (size_t i = 0; i < ds.label.size(); ++i) group_label[i] = ds.label[i];
 }
 
+GBMParam predict_param(const char *objective, int num_class, float learning_rate, int verbose) {
+    GBMParam p;  // base_score stays 0 on this path, as in the reference (scikit_tgbm.cpp:87-90)
+    p.objective = objective;
+    p.learning_rate = learning_rate;
+    p.num_class = num_class;
+    g_verbose = verbose;
+    return p;
+}
+
+void run_predict(const GBMParam &p, DataSet &ds, tgbm_model **model, int n_trees, int trees_per_iter, int num_class,
+                 const float *group_label, float *y_pred) {
+    ds.label.clear();
+    if (group_label != nullptr && objective_needs_group_label(p.objective))
+        for (int i = 0; i < num_class; ++i) ds.label.push_back(group_label[i]);
+    TGBM_CHECK(model != nullptr && *model != nullptr, "model is null!");
+    score(p, **model, n_trees, trees_per_iter, ds, true, false, y_pred);
+}
+
 // Distinct values among the labels (NaNs count as one, as do the two zeros): open addressing in a table that grows with
 // what it holds, so that the usual handful of classes stays in the L1.
 int count_distinct(const float *v, int n) {
@@ -157,23 +175,25 @@ void sparse_predict_scikit(int row_size, float *val, int *row_ptr, int *col_ptr,
                            int n_trees, int trees_per_iter, char *objective, int num_class, float learning_rate,
                            float *group_label, int *group, int num_group, int verbose) {
     std::lock_guard<std::mutex> lock(g_call_mutex);
-    GBMParam p;  // base_score stays 0 on this path, as in the reference (scikit_tgbm.cpp:87-90)
-    p.objective = objective;
-    p.learning_rate = learning_rate;
-    p.num_class = num_class;
-    DataSet ds;
+    GBMParam p = predict_param(objective, num_class, learning_rate, verbose);
     GBMParam load_param = p;
-    set_logger(verbose);
+    DataSet ds;
     auto t0 = std::chrono::steady_clock::now();
     ds.load_from_sparse(row_size, val, row_ptr, col_ptr, nullptr, group, num_group, load_param, false);
     log_debug("predict: host-side dataset %.3f s",
               std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
-    ds.label.clear();
-    if (group_label != nullptr && objective_needs_group_label(p.objective))
-        for (int i = 0; i < num_class; ++i) ds.label.push_back(group_label[i]);
-    TGBM_CHECK(model != nullptr && *model != nullptr, "model is null!");
-    std::vector<float> out = predict(p, to_nested(*model, n_trees, trees_per_iter), ds, false);
-    std::memcpy(y_pred, out.data(), out.size() * sizeof(float));
+    run_predict(p, ds, model, n_trees, trees_per_iter, num_class, group_label, y_pred);
+}
+
+void tgbm_predict_dense(int row_size, int columns, const void *x, int x_is_double, float *y_pred, tgbm_model **model,
+                        int n_trees, int trees_per_iter, const char *objective, int num_class, float learning_rate,
+                        const float *group_label, const int *group, int num_group, int verbose) {
+    std::lock_guard<std::mutex> lock(g_call_mutex);
+    GBMParam p = predict_param(objective, num_class, learning_rate, verbose);
+    GBMParam load_param = p;
+    DataSet ds;
+    ds.load_from_dense(row_size, columns, x, x_is_double != 0, nullptr, group, num_group, load_param);
+    run_predict(p, ds, model, n_trees, trees_per_iter, num_class, group_label, y_pred);
 }
 
 void save(char *model_path, char *objective, float learning_rate, int num_class, int n_trees, int trees_per_iter,
@@ -399,8 +419,8 @@ void tgbm_predict_raw(int row_size, const float *val, const int *row_ptr, const 
     g_verbose = 0;
     ds.load_from_sparse(row_size, val, row_ptr, col_ptr, nullptr, nullptr, 0, load_param, false);
     g_verbose = saved;
-    std::vector<float> r = predict_raw(p, to_nested(model, n_trees, trees_per_iter), ds);
-    std::memcpy(out, r.data(), r.size() * sizeof(float));
+    TGBM_CHECK(model != nullptr, "model is null!");
+    score(p, *model, n_trees, trees_per_iter, ds, false, false, out);
 }
 
 int tgbm_cut_points(int row_size, int n_features, const float *val, const int *row_ptr, const int *col_ptr,

@@ -520,6 +520,12 @@ void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes);
 // The same for doubles that the device takes as floats. Zeros of either sign arrive as +0, other values that are too
 // small for a float as -0.
 void upload_doubles_as_floats(hipStream_t s, float *dst, const double *src, size_t count);
+// The conversion alone, for arrays that the device reads from host memory.
+void doubles_to_floats(float *to, const double *from, size_t count);
+// A pinned block of kPinnedBytes that the device can read and write directly; kept for later calls.
+constexpr size_t kPinnedBytes = (size_t)4 << 20;
+void *pinned_acquire();
+void pinned_release(void *p);  // the work that uses it is done
 void release_transfer_memory();  // the pinned pieces that are kept for later copies
 
 // CSR form of a dense row-major matrix [n][columns] on the device: the stored values are those that are not zero
@@ -534,13 +540,13 @@ struct DeviceCsr {
 // Takes `x` over (it becomes the value array when every cell is stored, and is freed otherwise). Synchronises.
 DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored);
 
-// prediction of the n rows that row_ptr addresses (entry offsets into col / val); out[t * out_stride + i] for
-// class tree t and row i, out_stride = 0 means n (a slice of a larger row set passes the whole set's size)
-// `packed` (optional): the same nodes as 16-byte records (launch_pack_model); with them the trees are walked from LDS
+// Prediction of the n rows that row_ptr addresses (entry offsets into col / val); out[t * out_stride + i] for
+// class tree t and row i, out_stride = 0 means n (a slice of a larger row set passes the whole set's size); adds to out.
+// `packed` (optional): the same nodes as 16-byte records (launch_pack_model); with them the trees are walked from LDS.
+// For the models that launch_score's records do not describe, and for the entry point that allocates nothing.
 void launch_predict(hipStream_t s, int n, int F, const int *row_ptr, const int *col, const float *val,
                     const TreeNode *model, int n_iter, int n_class_trees, int n_nodes, float lr, float base_score,
-                    float *out, size_t out_stride = 0, const struct PackedNode *packed = nullptr,
-                    const uint2 *compact = nullptr, int compact_depth = 0);
+                    float *out, size_t out_stride = 0, const struct PackedNode *packed = nullptr);
 // What a traversal reads of a node, in one 16-byte record.
 struct PackedNode {
     float split_value, base_weight;
@@ -548,16 +554,42 @@ struct PackedNode {
     unsigned meta;      // split feature (24 bits, all ones: not a feature of the data) | default_right << 30 | leaf << 31
 };
 void launch_pack_model(hipStream_t s, const TreeNode *model, long n_total, int n_nodes, PackedNode *packed);
-// `compact` of launch_predict: eight-byte records (threshold or leaf weight; left child | address of the split feature's
-// values | flags) for a model and data of F features that compact_records_apply() accepts; `compact_depth`: what it
-// returned. The records depend on F (features the data lacks, rows per workgroup), so they are packed per data set.
-void launch_pack_compact(hipStream_t s, const TreeNode *model, int n_iter, int n_class_trees, int n_nodes, int F,
-                         uint2 *packed);
-// Do the eight-byte records describe this model on data of F features? Every split node keeps its children side by
-// side (right = left + 1) and below itself - then a walk needs one child index and ends after at most `depth` steps,
-// the number returned (0: they do not apply) -, and one tree fits the LDS next to the rows' dense vectors.
-int compact_records_apply(const TreeNode *model, size_t n_total, int n_nodes, int F);
-int compact_rows_per_group(int F);  // rows per workgroup of the kernel that walks the eight-byte records
+
+// A model as the scoring kernels read it. The features that its splits use are numbered 0 .. n_used - 1 (ascending);
+// a row is spread into keys of these slots, whatever the number of columns of the data. Slot n_used is the leaves' (its
+// key is zero), slot n_used + 1 that of features no data can have (always missing).
+// Records of eight bytes for models whose trees keep the two children of a node side by side and below it (every tree
+// the trainer builds, and the reference's: heap order):
+//   x: a split: key(threshold) + (default left ? 1 : 0) - 1, so that "goes right" is `value key + that one > x`;
+//      a leaf: the bits of its weight
+//   y: slot of the split feature (15 bits; a leaf: slot n_used, whose key never exceeds x)
+//      | byte offset of the left child in the tree << 15 (16 bits; a leaf: of the leaf itself)
+//      | default left << 31 (a leaf: 0)
+// A leaf therefore walks to itself, and a walk of `depth` steps needs no test for the end.
+// The model is stored round by round; the records class by class, so that the trees a workgroup stages together
+// (consecutive rounds of one class) are one contiguous run.
+struct ScoreModel {
+    const uint2 *records = nullptr;  // [n_class][n_iter][n_nodes]
+    const int *used = nullptr;       // [n_used] feature of every slot
+    const int *slot_of = nullptr;    // [n_features + 1] slot of a feature, -1: not used
+    int n_used = 0, n_slots = 0, leaf_slot = 0, n_features = 0;
+    int n_iter = 0, n_class = 0, n_nodes = 0, depth = 0;
+};
+struct ScoreRows {
+    int n = 0;
+    const float *x = nullptr;  // dense [n][columns], else the CSR arrays
+    int columns = 0;
+    bool minus_zero_is_stored = false;
+    const int *row_ptr = nullptr, *col = nullptr;
+    const float *val = nullptr;
+};
+// Scores of the rows: out[t * out_stride + i] is set. narrow: the reference's shared-memory path (at most 96 features in
+// the data: double sums, a stored +inf or NaN counts as missing), else its global-memory path (float sums).
+// false: the rows' keys fit no kernel's LDS and nothing was launched.
+bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &model, bool narrow, float lr, float base_score,
+                  float *out, size_t out_stride);
+// Below this many rows k_score_group takes them (see there).
+constexpr int kScoreGroupRows = 65536;
 void launch_predict_transform(hipStream_t s, int kind, int n, int num_class, const float *label, float *y);
 
 }  // namespace tgbm

@@ -76,10 +76,7 @@ class Trainer;  // device trainer, trainer.hip
 // src/thundergbm/trainer.cu:18-57
 std::vector<std::vector<Tree>> train(GBMParam &param, const DataSet &dataset);
 
-// src/thundergbm/predictor.cu:11-30 / :32-189. Returns class-major raw scores (predict_raw) or the
-// transformed predictions (predict).
-std::vector<float> predict_raw(const GBMParam &param, const std::vector<std::vector<Tree>> &model,
-                               const DataSet &dataset);
+// src/thundergbm/predictor.cu:11-30 / :32-189: the objective's predictions (score() in model_handle.h has the raw ones)
 std::vector<float> predict(const GBMParam &param, const std::vector<std::vector<Tree>> &model,
                            const DataSet &dataset, bool log_metric);
 

@@ -1,5 +1,7 @@
 // Tree-traversal prediction (the reference's Predictor::predict_raw, src/thundergbm/predictor.cu:32-189)
 // and the objectives' predict_transform.
+#include <type_traits>
+
 #include "device_api.h"
 
 namespace tgbm {
@@ -191,127 +193,135 @@ __device__ __forceinline__ unsigned order_key(float v) {
 constexpr unsigned kMissingKey = 0xffffffffu;
 __device__ __forceinline__ unsigned value_key(float v) { return v < INFINITY ? order_key(v) : kMissingKey; }
 
-// Eight-byte records for models whose trees keep the two children of a node side by side and below it (every tree the
-// trainer builds, and the reference's: heap order), walked by k_predict_compact:
-//   x: a split: key(threshold) + (default left ? 1 : 0) - 1, so that "goes right" is `value key + that one > x`;
-//      a leaf: the bits of its weight
-//   y: dword offset of the split feature's keys in the workgroup's dense vectors (15 bits; a feature the data does not
-//      have: that of the all-missing feature F; a leaf: that of the all-zero feature F + 1, whose key never exceeds x)
-//      | byte offset of the left child in the tree << 15 (16 bits; a leaf: of the leaf itself)
-//      | default left << 31 (a leaf: 0)
-// A leaf therefore walks to itself, and a walk of `depth` steps needs no test for the end.
-// Half the LDS bytes per node visit of the 16-byte record. B: rows per workgroup of the kernel that reads the records.
-__global__ void k_pack_compact(const TreeNode *__restrict__ model, int n_iter, int n_class_trees, int n_nodes, int F,
-                               int B, uint2 *__restrict__ packed) {
-    const long n_total = (long)n_iter * n_class_trees * n_nodes;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n_total; i += (long)gridDim.x * blockDim.x) {
-        const TreeNode nd = model[i];
-        const bool children_ok = nd.lch_index >= 0 && nd.lch_index < n_nodes && nd.rch_index >= 0 && nd.rch_index < n_nodes;
-        const bool leaf = nd.is_leaf || !children_ok;
-        const unsigned f = (nd.split_feature_id >= 0 && nd.split_feature_id < F) ? (unsigned)nd.split_feature_id : (unsigned)F;
-        const long tree = i / n_nodes;
-        const int self = (int)(i - tree * n_nodes);
-        uint2 p;
-        if (leaf) {
-            p.x = __float_as_uint(nd.base_weight);
-            p.y = (unsigned)(F + 1) * (unsigned)B | (unsigned)self * 8u << 15;
-        } else {
-            const unsigned left = nd.default_right ? 0u : 1u;
-            p.x = order_key(nd.split_value) + left - 1u;
-            p.y = f * (unsigned)B | (unsigned)nd.lch_index * 8u << 15 | left << 31;
-        }
-        // the model is stored round by round; the records class by class, so that the trees a workgroup stages
-        // together (consecutive rounds of one class) are one contiguous run
-        const long it = tree / n_class_trees, t = tree - it * n_class_trees;
-        packed[(t * n_iter + it) * n_nodes + self] = p;
-    }
+// The rows of a call as the scoring kernels read them: CSR entries (row_ptr addresses the slice's first row), or a dense
+// row-major matrix in which a zero is a value that is not stored (minus_zero_is_stored: -0 is a stored zero,
+// upload_doubles_as_floats).
+//
+// Key of a stored value. NARROW: the reference's shared-memory path, where a stored +inf or NaN counts as missing; else
+// its global-memory path (predictor.cu:160-189), where +inf is a value and a NaN, which is not below any threshold, goes
+// right like the largest value.
+template <bool NARROW>
+__device__ __forceinline__ unsigned stored_key(float v) {
+    if (NARROW) return value_key(v);
+    return v != v ? kMissingKey - 1u : order_key(v);
 }
+template <bool NARROW>
+__device__ __forceinline__ unsigned dense_key(float v, bool minus_zero_is_stored) {
+    const bool stored = v != 0.f || (minus_zero_is_stored && __float_as_uint(v) != 0u);
+    return stored ? stored_key<NARROW>(v) : kMissingKey;
+}
+// Sums: double where the reference's shared-memory path is (predictor.cu:85-160), else float with the product and the
+// sum in one rounding, as the compiler contracts k_predict's.
+__device__ __forceinline__ double add_leaf(double sum, float lr, float w) { return sum + lr * w; }
+__device__ __forceinline__ float add_leaf(float sum, float lr, float w) { return fmaf(lr, w, sum); }
 
-// k_predict_lds with the eight-byte records, ILP trees walked at a time by every thread and `depth` steps for every tree:
-// the walks of different trees do not depend on each other, so their LDS round trips (node, feature key, node, ...)
-// overlap; a walk that has reached its leaf stays there until the deepest possible walk is done (straight-line
-// code: eight vector instructions and two LDS reads per step). The leaf weights are added in the order of the
-// trees, as in the other kernels: same bits.
-// Rows of equal length with ascending columns (dense data handed over as CSR) are spread into the LDS vectors by
+// Many rows: a thread per row, the row's keys of the features that the model uses in LDS (feature-major, so the reads of
+// a wavefront never conflict), the trees of a class staged in LDS tps at a time, ILP trees walked at a time by every
+// thread and `depth` steps for every tree: the walks of different trees do not depend on each other, so their LDS round
+// trips (node, feature key, node, ...) overlap; a walk that has reached its leaf stays there until the deepest possible
+// walk is done (straight-line code: nine vector instructions and two LDS reads per step). The leaf weights are added in
+// the order of the trees, as in the other kernels: same bits. 10 M rows x 40 trees of depth 8: 2.0 ms (two trees per
+// stage; 2.1 with four, 2.7 with one), bound by the LDS (busy 62 %) and the vector ALUs (57 %).
+// CSR rows of equal length with ascending columns (dense data handed over as CSR) are spread into the LDS vectors by
 // consecutive lanes reading consecutive entries - whole cache lines per load instruction instead of one 4-byte word from
 // each of 64 lines; anything else takes the row-per-thread loop (whose result for a repeated column, the later entry,
-// does not depend on the order in which lanes write).
-template <int B, int ILP, int kFetch>
-__global__ __launch_bounds__(B) void k_predict_compact(int n, int F, const int *__restrict__ row_ptr,
-                                                       const int *__restrict__ col, const float *__restrict__ val,
-                                                       const uint2 *__restrict__ packed, int n_iter, int n_class_trees,
-                                                       int n_nodes, int depth, float lr, float base_score,
-                                                       float *__restrict__ out, size_t out_stride, int trees_per_stage,
-                                                       int coalesced_fill) {
+// does not depend on the order in which lanes write). A dense matrix is read by the row's thread, used columns only.
+template <int B, int ILP, int kFetch, bool NARROW>
+__global__ __launch_bounds__(B) void k_score_rows(ScoreRows rows_in, ScoreModel m, float lr, float base_score,
+                                                  float *__restrict__ out, size_t out_stride, int trees_per_stage,
+                                                  int coalesced_fill) {
+    using Sum = typename std::conditional<NARROW, double, float>::type;
     extern __shared__ unsigned smem_u[];
-    unsigned *dense = smem_u;                                        // [F + 2][B] keys; feature F: missing, F + 1: zero
-    uint2 *nodes = reinterpret_cast<uint2 *>(smem_u + (F + 2) * B);  // [trees_per_stage][n_nodes]
+    const int n = rows_in.n, slots = m.n_slots, n_nodes = m.n_nodes, n_iter = m.n_iter, n_class_trees = m.n_class;
+    unsigned *dense = smem_u;                                        // [slots][B] keys
+    uint2 *nodes = reinterpret_cast<uint2 *>(smem_u + slots * B);    // [trees_per_stage][n_nodes]
     const int row0 = blockIdx.x * B;
     const int i = row0 + threadIdx.x;
     const bool live = i < n;
-    for (int f = 0; f <= F; ++f) dense[f * B + threadIdx.x] = kMissingKey;
-    dense[(F + 1) * B + threadIdx.x] = 0u;
-    const int rb = live ? row_ptr[i] : 0, re = live ? row_ptr[i + 1] : 0;
-    const int len0 = row_ptr[row0 + 1] - row_ptr[row0];  // (row0 < n: the grid covers no workgroup without rows)
-    bool per_row = true;
-    if (coalesced_fill && __syncthreads_and(!live || re - rb == len0) && len0 > 0) {
-        // (the barrier above also orders the clearing before the writes of other lanes below)
-        const int rows = min(B, n - row0);
-        const int e0 = row_ptr[row0];
-        const int total = rows * len0;
-        int r = threadIdx.x / len0, slot = threadIdx.x - r * len0;
-        const int dr = B / len0, ds = B - dr * len0;
-        bool bad = false;
-        // (four entries per lane in flight: the loop is a chain of memory round trips otherwise)
-        for (int idx0 = threadIdx.x; idx0 < total; idx0 += 4 * B) {
-            int c[4], before[4];
-            float v[4];
+    for (int f = 0; f < slots; ++f) dense[f * B + threadIdx.x] = f == m.leaf_slot ? 0u : kMissingKey;
+    if (rows_in.x != nullptr) {
+        const float *__restrict__ x = rows_in.x + (size_t)min(i, n - 1) * rows_in.columns;
+        for (int f0 = 0; f0 < m.n_used; f0 += 8) {  // (eight loads in flight; the feature list is read by scalar loads)
+            float v[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = min(idx0 + u * B, total - 1);
-                c[u] = col[e0 + idx];
-                v[u] = val[e0 + idx];
-                // ascending inside the row: the entry before this one sits in the lane below (or, for lane 0, in memory)
-                before[u] = (threadIdx.x & 63) == 0 && idx > 0 ? col[e0 + idx - 1] : 0;
+            for (int u = 0; u < 8; ++u) {
+                const int f = m.used[min(f0 + u, m.n_used - 1)];
+                v[u] = x[min(f, rows_in.columns - 1)];
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int below = __shfl_up(c[u], 1);
-                if ((threadIdx.x & 63) != 0) before[u] = below;
-                if (idx0 + u * B < total) {
-                    if (slot > 0 && before[u] >= c[u]) bad = true;
-                    if ((unsigned)c[u] < (unsigned)F) dense[c[u] * B + r] = value_key(v[u]);
-                }
-                r += dr;
-                slot += ds;
-                if (slot >= len0) {
-                    slot -= len0;
-                    ++r;
-                }
-            }
+            for (int u = 0; u < 8; ++u)
+                if (f0 + u < m.n_used && m.used[f0 + u] < rows_in.columns)
+                    dense[(f0 + u) * B + threadIdx.x] = dense_key<NARROW>(v[u], rows_in.minus_zero_is_stored);
         }
-        per_row = __syncthreads_or(bad);
-        if (per_row)
-            for (int f = 0; f < F; ++f) dense[f * B + threadIdx.x] = kMissingKey;
-    }
-    if (per_row) {
-        for (int e = rb; e < re; e += 4) {  // (four entries in flight, written in their order)
-            int c[4];
-            float v[4];
+    } else {
+        const int *__restrict__ row_ptr = rows_in.row_ptr;
+        const int *__restrict__ col = rows_in.col;
+        const float *__restrict__ val = rows_in.val;
+        const int *__restrict__ slot_of = m.slot_of;
+        const int rb = live ? row_ptr[i] : 0, re = live ? row_ptr[i + 1] : 0;
+        const int len0 = row_ptr[row0 + 1] - row_ptr[row0];  // (row0 < n: the grid covers no workgroup without rows)
+        bool per_row = true;
+        if (coalesced_fill && __syncthreads_and(!live || re - rb == len0) && len0 > 0) {
+            // (the barrier above also orders the clearing before the writes of other lanes below)
+            const int rows = min(B, n - row0);
+            const int e0 = row_ptr[row0];
+            const int total = rows * len0;
+            int r = threadIdx.x / len0, slot = threadIdx.x - r * len0;
+            const int dr = B / len0, ds = B - dr * len0;
+            bool bad = false;
+            // (four entries per lane in flight: the loop is a chain of memory round trips otherwise)
+            for (int idx0 = threadIdx.x; idx0 < total; idx0 += 4 * B) {
+                int c[4], before[4], at[4];
+                float v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                c[u] = col[min(e + u, re - 1)];
-                v[u] = val[min(e + u, re - 1)];
+                for (int u = 0; u < 4; ++u) {
+                    const int idx = min(idx0 + u * B, total - 1);
+                    c[u] = col[e0 + idx];
+                    v[u] = val[e0 + idx];
+                    // ascending inside the row: the entry before this one sits in the lane below (or, for lane 0, in memory)
+                    before[u] = (threadIdx.x & 63) == 0 && idx > 0 ? col[e0 + idx - 1] : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) at[u] = slot_of[min((unsigned)c[u], (unsigned)m.n_features)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int below = __shfl_up(c[u], 1);
+                    if ((threadIdx.x & 63) != 0) before[u] = below;
+                    if (idx0 + u * B < total) {
+                        if (slot > 0 && before[u] >= c[u]) bad = true;
+                        if (at[u] >= 0) dense[at[u] * B + r] = stored_key<NARROW>(v[u]);
+                    }
+                    r += dr;
+                    slot += ds;
+                    if (slot >= len0) {
+                        slot -= len0;
+                        ++r;
+                    }
+                }
             }
+            per_row = __syncthreads_or(bad);
+            if (per_row)
+                for (int f = 0; f < m.n_used; ++f) dense[f * B + threadIdx.x] = kMissingKey;
+        }
+        if (per_row) {
+            for (int e = rb; e < re; e += 4) {  // (four entries in flight, written in their order)
+                int at[4];
+                float v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (e + u < re && (unsigned)c[u] < (unsigned)F) dense[c[u] * B + threadIdx.x] = value_key(v[u]);
+                for (int u = 0; u < 4; ++u) {
+                    at[u] = slot_of[min((unsigned)col[min(e + u, re - 1)], (unsigned)m.n_features)];
+                    v[u] = val[min(e + u, re - 1)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (e + u < re && at[u] >= 0) dense[at[u] * B + threadIdx.x] = stored_key<NARROW>(v[u]);
+            }
         }
     }
     // (byte offsets into the workgroup's LDS, so that a step adds record fields to them without further scaling)
     const char *lds = reinterpret_cast<const char *>(smem_u);
-    const unsigned mine = threadIdx.x * 4u;  // this row's key of feature 0
-    const unsigned trees0 = (unsigned)(F + 2) * B * 4u;
+    const unsigned mine = threadIdx.x * 4u;  // this row's key of slot 0
+    const unsigned trees0 = (unsigned)slots * B * 4u;
     // The trees of a stage are fetched into registers while the stage before is walked and go to the LDS between two
     // barriers after it, so that no walk waits for global memory (kFetch records per thread, as many as the stage needs:
     // the loads are unconditional - clamped -, or the compiler waits for them at once; stages of more than 8 records
@@ -320,13 +330,13 @@ __global__ __launch_bounds__(B) void k_predict_compact(int n, int F, const int *
     uint2 fetched[kFetch];
     auto fetch = [&](int t, int it0) {
         const int count = min(trees_per_stage, n_iter - it0) * n_nodes;
-        const uint2 *src = packed + ((size_t)t * n_iter + it0) * n_nodes;
+        const uint2 *src = m.records + ((size_t)t * n_iter + it0) * n_nodes;
 #pragma unroll
         for (int q = 0; q < kFetch; ++q) fetched[q] = src[min((int)threadIdx.x + q * B, count - 1)];
     };
     if (prefetch) fetch(0, 0);
     for (int t = 0; t < n_class_trees; ++t) {
-        double sum = base_score;
+        Sum sum = base_score;
         for (int it0 = 0; it0 < n_iter; it0 += trees_per_stage) {
             const int staged = min(trees_per_stage, n_iter - it0);
             __syncthreads();  // the walks of the previous stage are done (and, the first time, the vectors are filled)
@@ -340,7 +350,7 @@ __global__ __launch_bounds__(B) void k_predict_compact(int n, int F, const int *
                 if (it0 + trees_per_stage < n_iter) fetch(t, it0 + trees_per_stage);
                 else if (t + 1 < n_class_trees) fetch(t + 1, 0);
             } else {
-                const uint2 *src = packed + ((size_t)t * n_iter + it0) * n_nodes;
+                const uint2 *src = m.records + ((size_t)t * n_iter + it0) * n_nodes;
                 for (int idx = threadIdx.x; idx < staged * n_nodes; idx += B) nodes[idx] = src[idx];
             }
             __syncthreads();
@@ -354,11 +364,11 @@ __global__ __launch_bounds__(B) void k_predict_compact(int n, int F, const int *
                     tree[j] = trees0 + (unsigned)(min(k + j, staged - 1) * n_nodes) * 8u;
                     nd[j] = *reinterpret_cast<const uint2 *>(lds + tree[j]);
                 }
-                for (int step = 0; step < depth; ++step) {
+                for (int step = 0; step < m.depth; ++step) {
                     unsigned key[ILP];
 #pragma unroll
                     for (int j = 0; j < ILP; ++j)
-                        key[j] = *reinterpret_cast<const unsigned *>(lds + (mine + ((nd[j].y & 0x7fffu) << 2)));
+                        key[j] = *reinterpret_cast<const unsigned *>(lds + (mine + (nd[j].y & 0x7fffu) * (B * 4u)));
 #pragma unroll
                     for (int j = 0; j < ILP; ++j) {
                         const bool right = key[j] + (nd[j].y >> 31) > nd[j].x;
@@ -367,11 +377,103 @@ __global__ __launch_bounds__(B) void k_predict_compact(int n, int F, const int *
                 }
 #pragma unroll
                 for (int j = 0; j < ILP; ++j)
-                    if (k + j < staged) sum += lr * __uint_as_float(nd[j].x);
+                    if (k + j < staged) sum = add_leaf(sum, lr, __uint_as_float(nd[j].x));
             }
         }
-        if (live) out[(size_t)t * out_stride + i] += (float)sum;
+        if (live) out[(size_t)t * out_stride + i] = 0.f + (float)sum;
     }
+}
+
+// Few rows, or rows over more features than k_score_rows' vectors hold: G lanes per row (a wavefront, or the whole
+// workgroup), a tree per lane. The row's keys of the used features are spread into LDS once; the node records come
+// through the caches - the top of a tree is one line that stays in the L1, the lower levels come from the L2 - and the
+// leaf weights meet in LDS, where one lane per class adds them in the order of the trees: same bits as k_score_rows.
+// One row of 100 trees is two dependent walks of `depth` L2 round trips instead of a hundred LDS walks by one thread.
+constexpr int kScoreGroupTrees = 256;  // leaf weights of a row that meet in LDS at a time
+
+template <int G, bool NARROW>
+__global__ __launch_bounds__(256) void k_score_group(ScoreRows rows_in, ScoreModel m, float lr, float base_score,
+                                                     float *__restrict__ out, size_t out_stride) {
+    using Sum = typename std::conditional<NARROW, double, float>::type;
+    constexpr int R = 256 / G;  // rows of a workgroup
+    extern __shared__ unsigned smem_u[];
+    const int g = threadIdx.x / G, lane = threadIdx.x % G;
+    const int n_class = m.n_class, n_iter = m.n_iter, slots = m.n_slots;
+    Sum *sums = reinterpret_cast<Sum *>(smem_u) + g * n_class;  // [R][n_class]
+    float *weights = reinterpret_cast<float *>(reinterpret_cast<Sum *>(smem_u) + R * n_class) + g * kScoreGroupTrees;
+    unsigned *keys = reinterpret_cast<unsigned *>(reinterpret_cast<float *>(reinterpret_cast<Sum *>(smem_u) + R * n_class) +
+                                                  R * kScoreGroupTrees) + g * slots;
+    const int row = blockIdx.x * R + g;
+    const int i = min(row, rows_in.n - 1);  // (every wavefront meets every barrier)
+    if (rows_in.x != nullptr) {
+        const float *__restrict__ x = rows_in.x + (size_t)i * rows_in.columns;
+        for (int f = lane; f < slots; f += G) {
+            unsigned key = f == m.leaf_slot ? 0u : kMissingKey;
+            if (f < m.n_used && m.used[f] < rows_in.columns) key = dense_key<NARROW>(x[m.used[f]], rows_in.minus_zero_is_stored);
+            keys[f] = key;
+        }
+    } else {
+        for (int f = lane; f < slots; f += G) keys[f] = f == m.leaf_slot ? 0u : kMissingKey;
+        const int rb = rows_in.row_ptr[i], re = rows_in.row_ptr[i + 1];
+        const int *__restrict__ col = rows_in.col;
+        bool descends = false;
+        __syncthreads();
+        for (int e = rb + lane; e < re; e += G) {
+            const int c = col[e], next = e + 1 < re ? col[e + 1] : 0x7fffffff;
+            descends |= next < c;
+            const int at = m.slot_of[min((unsigned)c, (unsigned)m.n_features)];
+            if (at >= 0 && next != c) keys[at] = stored_key<NARROW>(rows_in.val[e]);  // (of equal columns the later entry)
+        }
+        if (__syncthreads_or(descends)) {
+            // a row whose columns do not ascend may repeat one with others in between: entry by entry, the later one counts
+            if (lane == 0)
+                for (int e = rb; e < re; ++e) {
+                    const int at = m.slot_of[min((unsigned)col[e], (unsigned)m.n_features)];
+                    if (at >= 0) keys[at] = stored_key<NARROW>(rows_in.val[e]);
+                }
+        }
+    }
+    for (int c = lane; c < n_class; c += G) sums[c] = base_score;
+    const int n_trees = n_iter * n_class;
+    const char *records = reinterpret_cast<const char *>(m.records);
+    for (int k0 = 0; k0 < n_trees; k0 += kScoreGroupTrees) {
+        const int k1 = min(k0 + kScoreGroupTrees, n_trees);
+        __syncthreads();  // the keys are filled; the previous weights are added
+        constexpr int ILP = G == 64 ? 2 : 1;
+        for (int k = k0 + lane; k < k1; k += ILP * G) {
+            const char *tree[ILP];
+            uint2 nd[ILP];
+#pragma unroll
+            for (int j = 0; j < ILP; ++j) {
+                tree[j] = records + (size_t)min(k + j * G, k1 - 1) * m.n_nodes * 8u;
+                nd[j] = *reinterpret_cast<const uint2 *>(tree[j]);
+            }
+            for (int step = 0; step < m.depth; ++step) {
+                unsigned key[ILP];
+#pragma unroll
+                for (int j = 0; j < ILP; ++j) key[j] = keys[nd[j].y & 0x7fffu];
+#pragma unroll
+                for (int j = 0; j < ILP; ++j) {
+                    const bool right = key[j] + (nd[j].y >> 31) > nd[j].x;
+                    nd[j] = *reinterpret_cast<const uint2 *>(tree[j] + ((nd[j].y >> 15) & 0xffffu) + (right ? 8u : 0u));
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < ILP; ++j)
+                if (k + j * G < k1) weights[k + j * G - k0] = __uint_as_float(nd[j].x);
+        }
+        __syncthreads();
+        const int c0 = k0 / n_iter, c1 = (k1 - 1) / n_iter;
+        for (int c = c0 + lane; c <= c1; c += G) {
+            Sum sum = sums[c];
+            const int e = min(k1, (c + 1) * n_iter) - k0;
+            for (int k = max(k0, c * n_iter) - k0; k < e; ++k) sum = add_leaf(sum, lr, weights[k]);
+            sums[c] = sum;
+        }
+    }
+    __syncthreads();
+    if (row < rows_in.n)
+        for (int c = lane; c < n_class; c += G) out[(size_t)c * out_stride + row] = 0.f + (float)sums[c];
 }
 
 // kind 1: binary label lookup, 2: arg-max label lookup, 3: softmax probabilities in place,
@@ -412,50 +514,16 @@ __global__ void k_predict_transform(int kind, int n, int K, const float *__restr
 
 void launch_predict(hipStream_t s, int n, int F, const int *row_ptr, const int *col, const float *val,
                     const TreeNode *model, int n_iter, int n_class_trees, int n_nodes, float lr, float base_score,
-                    float *out, size_t out_stride, const PackedNode *packed, const uint2 *compact, int compact_depth) {
+                    float *out, size_t out_stride, const PackedNode *packed) {
     if (n == 0) return;
     if (out_stride == 0) out_stride = (size_t)n;
     if (n_class_trees > 1) base_score = 0;  // predictor.cu:81-83
     const bool dense_path = (size_t)F * 128 * sizeof(float) <= 48 * 1024;
     int grid = (n + kBlock - 1) / kBlock;
-    // (TGBM_PREDICT_TPS: trees staged at a time, 0 = walk the 48-byte nodes in global memory; measurements)
-    // (both switches are read at every call, so a test can compare the kernels within one process)
+    // (TGBM_PREDICT_TPS: trees staged at a time, 0 = walk the 48-byte nodes in global memory; read at every call, so a test
+    // can compare the kernels within one process)
     const int tps_given = std::getenv("TGBM_PREDICT_TPS") ? atoi(std::getenv("TGBM_PREDICT_TPS")) : -1;
-    int tps_env = tps_given < 0 ? 2 : tps_given;
-    // (TGBM_PREDICT_COMPACT=0: the 16-byte records also where the 8-byte ones apply; =2: those without the coalesced
-    // spreading of equal-length rows; measurements and tests)
-    const int compact_env = std::getenv("TGBM_PREDICT_COMPACT") ? atoi(std::getenv("TGBM_PREDICT_COMPACT")) : 1;
-    if (compact != nullptr && compact_env > 0 && tps_env > 0) {
-        const int B = compact_rows_per_group(F);
-        const size_t dense_bytes = (size_t)(F + 2) * B * sizeof(float), tree_bytes = (size_t)n_nodes * sizeof(uint2);
-        const size_t fit = (64 * 1024 - dense_bytes) / tree_bytes;  // (>= 1: compact_records_apply)
-        // two trees per stage and thread (more were not faster: 10 M rows x 40 trees of depth 8 take 2.0 ms with two,
-        // 2.1 ms with four, 2.7 ms with one)
-        const int tps = (int)std::max<size_t>(1, std::min<size_t>(std::min(tps_env, 2), fit));
-        const size_t lds = dense_bytes + (size_t)tps * tree_bytes;
-        const int fill = compact_env == 2 ? 0 : 1;
-        const int g = (n + B - 1) / B;
-        const int per_thread = (tps * n_nodes + B - 1) / B;  // records of a stage
-#define TGBM_PREDICT_COMPACT_LAUNCH(BLK, ILP, FETCH)                                                                  \
-    k_predict_compact<BLK, ILP, FETCH><<<g, BLK, lds, s>>>(n, F, row_ptr, col, val, compact, n_iter, n_class_trees,  \
-                                                           n_nodes, compact_depth, lr, base_score, out, out_stride, \
-                                                           tps, fill)
-#define TGBM_PREDICT_COMPACT_FETCH(BLK, ILP)                               \
-    if (per_thread <= 2) TGBM_PREDICT_COMPACT_LAUNCH(BLK, ILP, 2);         \
-    else if (per_thread <= 4) TGBM_PREDICT_COMPACT_LAUNCH(BLK, ILP, 4);    \
-    else TGBM_PREDICT_COMPACT_LAUNCH(BLK, ILP, 8)
-        if (B == 256) {
-            if (tps >= 2) { TGBM_PREDICT_COMPACT_FETCH(256, 2); }
-            else { TGBM_PREDICT_COMPACT_FETCH(256, 1); }
-        } else {
-            if (tps >= 2) { TGBM_PREDICT_COMPACT_FETCH(128, 2); }
-            else { TGBM_PREDICT_COMPACT_FETCH(128, 1); }
-        }
-#undef TGBM_PREDICT_COMPACT_FETCH
-#undef TGBM_PREDICT_COMPACT_LAUNCH
-        return;
-    }
-    tps_env = tps_given < 0 ? 4 : tps_given;
+    const int tps_env = tps_given < 0 ? 4 : tps_given;
     if (dense_path && packed != nullptr && tps_env > 0 && n_nodes <= 0xffff) {  // (16-bit child indices)
         // trees in LDS: 256 rows per workgroup while their dense vectors take at most 48 KB, else 128; trees are staged
         // one at a time unless several fit next to the vectors in 40 KB (four workgroups per CU: measured on 10 M rows
@@ -488,14 +556,75 @@ void launch_pack_model(hipStream_t s, const TreeNode *model, long n_total, int n
     k_pack_model<<<(int)std::min<long>((n_total + 255) / 256, 4096), 256, 0, s>>>(model, n_total, n_nodes, packed);
 }
 
-int compact_rows_per_group(int F) { return (size_t)(F + 2) * 256 * sizeof(float) <= 50 * 1024 ? 256 : 128; }
-
-void launch_pack_compact(hipStream_t s, const TreeNode *model, int n_iter, int n_class_trees, int n_nodes, int F,
-                         uint2 *packed) {
-    const long n_total = (long)n_iter * n_class_trees * n_nodes;
-    if (n_total <= 0) return;
-    k_pack_compact<<<(int)std::min<long>((n_total + 255) / 256, 4096), 256, 0, s>>>(model, n_iter, n_class_trees, n_nodes,
-                                                                                    F, compact_rows_per_group(F), packed);
+bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, bool narrow, float lr, float base_score,
+                  float *out, size_t out_stride) {
+    if (rows.n == 0) return true;
+    if (m.n_class > 1) base_score = 0;  // predictor.cu:81-83
+    // (TGBM_PREDICT_COMPACT=2: without the coalesced spreading of equal-length rows; TGBM_PREDICT_TPS: that many trees per
+    // stage of k_score_rows, which then takes every row count; tests and measurements)
+    const char *ce = std::getenv("TGBM_PREDICT_COMPACT"), *te = std::getenv("TGBM_PREDICT_TPS");
+    const char *ge = std::getenv("TGBM_PREDICT_GROUP");  // 1 / 0: k_score_group always / never where the other serves
+    const int fill = ce != nullptr && atoi(ce) == 2 ? 0 : 1;
+    // k_score_rows: 256 rows per workgroup while their vectors take at most 50 KB, else 128
+    const int B = (size_t)m.n_slots * 256 * sizeof(float) <= 50 * 1024 ? 256 : 128;
+    const size_t dense_bytes = (size_t)m.n_slots * B * sizeof(float), tree_bytes = (size_t)m.n_nodes * sizeof(uint2);
+    const bool rows_fit = dense_bytes <= 50 * 1024 && dense_bytes + tree_bytes <= 64 * 1024;
+    // k_score_group
+    const size_t sum_bytes = narrow ? sizeof(double) : sizeof(float);
+    auto group_bytes = [&](int G) {
+        return (size_t)(256 / G) * ((size_t)m.n_class * sum_bytes + kScoreGroupTrees * sizeof(float) + (size_t)m.n_slots * 4);
+    };
+    // A wavefront per row while four rows leave the LDS room for four workgroups per CU; the whole workgroup for rows too
+    // few to fill the chip otherwise, and for wider ones.
+    const int G = rows.n > 1024 && group_bytes(64) <= 40 * 1024 ? 64 : 256;
+    const bool group_fits = group_bytes(G) <= 150 * 1024;
+    bool group = rows.n < kScoreGroupRows;
+    if (te != nullptr && atoi(te) > 0) group = false;
+    if (ge != nullptr) group = atoi(ge) != 0;
+    if (group_fits && (group || !rows_fit)) {
+        const int grid = (rows.n + 256 / G - 1) / (256 / G);
+        const size_t lds = group_bytes(G);
+#define TGBM_SCORE_GROUP(GG, NN) k_score_group<GG, NN><<<grid, 256, lds, s>>>(rows, m, lr, base_score, out, out_stride)
+        if (G == 64) {
+            if (narrow) TGBM_SCORE_GROUP(64, true);
+            else TGBM_SCORE_GROUP(64, false);
+        } else {
+            if (lds > 64 * 1024)  // (what a kernel may ask for without saying so)
+                HIP_CHECK(hipFuncSetAttribute(narrow ? reinterpret_cast<const void *>(&k_score_group<256, true>)
+                                                     : reinterpret_cast<const void *>(&k_score_group<256, false>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            if (narrow) TGBM_SCORE_GROUP(256, true);
+            else TGBM_SCORE_GROUP(256, false);
+        }
+#undef TGBM_SCORE_GROUP
+        return true;
+    }
+    if (!rows_fit) return false;
+    const size_t fit = (64 * 1024 - dense_bytes) / tree_bytes;  // (>= 1)
+    const int tps = (int)std::max<size_t>(1, std::min<size_t>(te != nullptr && atoi(te) == 1 ? 1 : 2, fit));
+    const size_t lds = dense_bytes + (size_t)tps * tree_bytes;
+    const int g = (rows.n + B - 1) / B;
+    const int per_thread = (tps * m.n_nodes + B - 1) / B;  // records of a stage
+#define TGBM_SCORE_ROWS(BLK, ILP, FETCH, NN) \
+    k_score_rows<BLK, ILP, FETCH, NN><<<g, BLK, lds, s>>>(rows, m, lr, base_score, out, out_stride, tps, fill)
+#define TGBM_SCORE_FETCH(BLK, ILP, NN)                          \
+    if (per_thread <= 2) TGBM_SCORE_ROWS(BLK, ILP, 2, NN);      \
+    else if (per_thread <= 4) TGBM_SCORE_ROWS(BLK, ILP, 4, NN); \
+    else TGBM_SCORE_ROWS(BLK, ILP, 8, NN)
+#define TGBM_SCORE_ILP(BLK, NN)                  \
+    if (tps >= 2) { TGBM_SCORE_FETCH(BLK, 2, NN); } \
+    else { TGBM_SCORE_FETCH(BLK, 1, NN); }
+    if (B == 256) {
+        if (narrow) { TGBM_SCORE_ILP(256, true) }
+        else { TGBM_SCORE_ILP(256, false) }
+    } else {
+        if (narrow) { TGBM_SCORE_ILP(128, true) }
+        else { TGBM_SCORE_ILP(128, false) }
+    }
+#undef TGBM_SCORE_ILP
+#undef TGBM_SCORE_FETCH
+#undef TGBM_SCORE_ROWS
+    return true;
 }
 
 void launch_predict_transform(hipStream_t s, int kind, int n, int num_class, const float *label, float *y) {

@@ -20,7 +20,7 @@
 namespace tgbm {
 namespace {
 
-constexpr size_t kPiece = (size_t)4 << 20;
+constexpr size_t kPiece = kPinnedBytes;
 constexpr size_t kStagedBytes = (size_t)12 << 20;
 constexpr size_t kKeepPieces = 16;
 
@@ -34,6 +34,7 @@ struct PieceStore {
     std::mutex mutex;
     std::vector<Piece> pieces;
     std::map<int, std::array<hipStream_t, 2>> streams;  // per device
+    std::map<char *, Piece> lent;                       // by pinned_acquire
 };
 
 PieceStore &piece_store() {
@@ -138,23 +139,46 @@ void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
                 [&](char *to, size_t off, size_t len) { std::memcpy(to, static_cast<const char *>(src) + off, len); });
 }
 
+void doubles_to_floats(float *to, const double *from, size_t count) {
+    unsigned *out = reinterpret_cast<unsigned *>(to);
+    for (size_t i = 0; i < count; ++i) {
+        const double d = from[i];
+        const float f = (float)d;
+        unsigned bits;
+        std::memcpy(&bits, &f, 4);
+        // zero: +0; a value that is only zero as a float: -0 (see dense_to_csr)
+        out[i] = (bits & 0x7fffffffu) != 0 ? bits : (d == 0.0 ? 0u : 0x80000000u);
+    }
+}
+
 // The conversion happens while the pieces are filled, so the doubles cross PCIe as floats.
 void upload_doubles_as_floats(hipStream_t s, float *dst, const double *src, size_t count) {
     send_staged(s, dst, count * sizeof(float), 8, [&](char *to, size_t off, size_t len) {
-        const double *from = src + off / sizeof(float);
-        unsigned *out = reinterpret_cast<unsigned *>(to);
-        const size_t m = len / sizeof(float);
-        for (size_t i = 0; i < m; ++i) {
-            const double d = from[i];
-            const float f = (float)d;
-            unsigned bits;
-            std::memcpy(&bits, &f, 4);
-            const unsigned magnitude = bits & 0x7fffffffu;
-            // zero: +0; a value that is only zero as a float: -0 (see dense_to_csr)
-            bits = magnitude != 0 ? bits : (d == 0.0 ? 0u : 0x80000000u);
-            out[i] = bits;
-        }
+        doubles_to_floats(reinterpret_cast<float *>(to), src + off / sizeof(float), len / sizeof(float));
     });
+}
+
+void *pinned_acquire() {
+    const Piece p = take_piece();
+    if (p.in_flight) HIP_CHECK(hipEventSynchronize(p.sent));
+    PieceStore &store = piece_store();
+    std::lock_guard<std::mutex> lock(store.mutex);
+    store.lent[p.host] = p;
+    return p.host;
+}
+
+void pinned_release(void *host) {
+    PieceStore &store = piece_store();
+    Piece p;
+    {
+        std::lock_guard<std::mutex> lock(store.mutex);
+        auto it = store.lent.find(static_cast<char *>(host));
+        TGBM_CHECK(it != store.lent.end(), "pinned_release: not a block of pinned_acquire");
+        p = it->second;
+        store.lent.erase(it);
+    }
+    p.in_flight = false;
+    give_piece(p);
 }
 
 void release_transfer_memory() {

@@ -143,18 +143,33 @@ class TGBMModel(BaseEstimator):
         if not self.model:
             raise ValueError("Please train the model first or load model from file!")
         lib = _lib.load()
-        X = _csr(X)
-        indptr = np.ascontiguousarray(X.indptr, dtype=np.int32)
-        indices = np.ascontiguousarray(X.indices, dtype=np.int32)
+        dense = _dense(X)
+        X = _csr(X) if dense is None else dense
         n = X.shape[0]
         n_out = n * self.num_class if self.objective == "multi:softprob" else n
         out = np.zeros(max(n_out, n * max(self.tree_per_iter, 1)), dtype=np.float32)
-        labels = np.asarray(self.group_label if self.group_label else [0.0], dtype=np.float32)
+        labels = np.asarray(self._class_labels(), dtype=np.float32)
         grp = None if groups is None else np.ascontiguousarray(groups, dtype=np.int32)
+        if dense is not None:
+            lib.tgbm_predict_dense(n, X.shape[1], _ptr(X), int(X.dtype == np.float64), _ptr(out), C.byref(self.model),
+                                   self.n_trees, self.tree_per_iter, self.objective.encode("utf-8"), self.num_class,
+                                   self.learning_rate, _ptr(labels), None if grp is None else _ptr(grp),
+                                   0 if grp is None else len(grp), self.verbose)
+            return self._predictions(out, n, n_out)
+        indptr = np.ascontiguousarray(X.indptr, dtype=np.int32)
+        indices = np.ascontiguousarray(X.indices, dtype=np.int32)
         lib.sparse_predict_scikit(n, _ptr(X.data), _ptr(indptr), _ptr(indices), _ptr(out),
                                   C.cast(C.byref(self.model), C.c_void_p), self.n_trees, self.tree_per_iter,
                                   self.objective.encode("utf-8"), self.num_class, self.learning_rate, _ptr(labels),
                                   None if grp is None else _ptr(grp), 0 if grp is None else len(grp), self.verbose)
+        return self._predictions(out, n, n_out)
+
+    def _class_labels(self):
+        """The labels a prediction maps to: the library reads num_class of them (a regressor's list has an entry per
+        distinct target, none of which is read)."""
+        return (self.group_label or [0.0])[: max(self.num_class, 2)]
+
+    def _predictions(self, out, n, n_out):
         if self.objective == "multi:softprob":
             # the library returns class-major probabilities; the reference wrapper reshapes them as
             # [-1, num_class] without transposing (thundergbm.py:169-171) and so does this one
