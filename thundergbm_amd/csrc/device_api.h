@@ -451,7 +451,7 @@ void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, 
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col);
 // min_next[c] (pre-filled with INT_MAX) = smallest column index that follows column c in a row (equal neighbours, a
 // column stored twice, do not count); *descending is set when a row's columns do not ascend
-void launch_min_next_col(hipStream_t s, int n, const int *row_ptr, const int *col, int *min_next, int *descending);
+void launch_min_next_col(hipStream_t s, int n, int F, const int *row_ptr, const int *col, int *min_next, int *descending);
 // feat_slot (may be nullptr): first head slot of a feature or -1; then hist_word is written as well
 void launch_bin_csr(hipStream_t s, long nnz, const int *col, const float *val, const float *cut_val,
                     const int *cut_row_ptr, int *bin_id, const int *feat_slot = nullptr, int *hist_word = nullptr);
@@ -520,6 +520,9 @@ void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes);
 // The same for doubles that the device takes as floats. Zeros of either sign arrive as +0, other values that are too
 // small for a float as -0.
 void upload_doubles_as_floats(hipStream_t s, float *dst, const double *src, size_t count);
+// Column indices, which cross PCIe as bytes or 16-bit words where they all fit; anything else (negative ones too)
+// arrives as it is.
+void upload_columns(hipStream_t s, int *dst, const int *src, size_t count);
 // The conversion alone, for arrays that the device reads from host memory.
 void doubles_to_floats(float *to, const double *from, size_t count);
 // A pinned block of kPinnedBytes that the device can read and write directly; kept for later calls.

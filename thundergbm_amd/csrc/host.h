@@ -1,12 +1,33 @@
 // Host-side pieces that mirror the reference's DataSet, Parser, TreeTrainer and Predictor.
 #pragma once
 #include <memory>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "common.h"
 
 namespace tgbm {
+
+// A vector of plain values that does not clear what resize() adds.
+template <typename T>
+struct NoClear : std::allocator<T> {
+    template <typename U>
+    struct rebind {
+        using other = NoClear<U>;
+    };
+    NoClear() = default;
+    template <typename U>
+    NoClear(const NoClear<U> &) {}
+    template <typename U>
+    void construct(U *) noexcept {}
+    template <typename U, typename... A>
+    void construct(U *p, A &&...a) {
+        ::new (static_cast<void *>(p)) U(std::forward<A>(a)...);
+    }
+};
+using LabelVector = std::vector<float, NoClear<float>>;
 
 // Host CSR dataset (the reference's DataSet, include/thundergbm/dataset.h).
 struct DataSet {
@@ -27,7 +48,7 @@ struct DataSet {
     const double *dense_f64 = nullptr;
     int dense_columns = 0;
     bool is_dense() const { return dense_columns > 0; }
-    std::vector<float> y;
+    LabelVector y;
     std::vector<float> label;  // distinct class labels, ascending
     std::vector<int> group;
     size_t n_features_ = 0;

@@ -344,7 +344,7 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz, 1l));
         device_alloc_to(d_row_ptr, sizeof(int) * ((size_t)n + 1));
         upload_large(s_up, d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n + 1));
-        if (nnz) upload_large(s_up, d_col, ds.col_idx, sizeof(int) * (size_t)nnz);
+        if (nnz) upload_columns(s_up, d_col, ds.col_idx, (size_t)nnz);
         if (!ds.features_counted) F = device_max_int(s_up, d_col, nnz) + 1;
         narrow = F <= kNarrowFeatures;
         done = usable;

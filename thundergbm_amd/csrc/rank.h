@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "device_api.h"
+#include "host.h"
 
 namespace tgbm {
 
@@ -30,7 +31,7 @@ struct RankRun {
 class RankContext {
    public:
     // y: labels of all rows; group: sizes of the query groups (consecutive rows), their sum must be y.size()
-    RankContext(hipStream_t s, const std::vector<float> &y, const std::vector<int> &group, bool ndcg);
+    RankContext(hipStream_t s, const LabelVector &y, const std::vector<int> &group, bool ndcg);
     ~RankContext();
     RankContext(const RankContext &) = delete;
     RankContext &operator=(const RankContext &) = delete;

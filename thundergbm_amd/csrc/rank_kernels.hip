@@ -282,7 +282,7 @@ T *RankContext::dalloc(size_t count) {
     return static_cast<T *>(p);
 }
 
-RankContext::RankContext(hipStream_t s, const std::vector<float> &y, const std::vector<int> &group, bool ndcg)
+RankContext::RankContext(hipStream_t s, const LabelVector &y, const std::vector<int> &group, bool ndcg)
     : stream_(s), ndcg_(ndcg) {
     n_ = (int)y.size();
     n_groups_ = (int)group.size();

@@ -103,9 +103,8 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
         device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
         upload_large(stream_, d_val, ds.val, sizeof(float) * (size_t)nnz_);
-        upload_large(stream_, d_col, ds.col_idx, sizeof(int) * (size_t)nnz_);
-        upload(stream_, d_row_ptr, ds.row_ptr, (size_t)n_ + 1);
-        HIP_CHECK(hipStreamSynchronize(stream_));
+        upload_columns(stream_, d_col, ds.col_idx, (size_t)nnz_);
+        upload_large(stream_, d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n_ + 1));
     }
     log_debug("upload of %.2f GB: %.3f s", (double)nnz_ * 8e-9,
               std::chrono::duration<double>(std::chrono::steady_clock::now() - t_up).count());
@@ -305,7 +304,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             device_alloc_to(d_next, sizeof(int) * ((size_t)F_ + 1));
             HIP_CHECK(hipMemsetAsync(d_next, 0x7f, sizeof(int) * (size_t)F_, stream_));  // 0x7f7f7f7f: above every column
             HIP_CHECK(hipMemsetAsync(d_next + F_, 0, sizeof(int), stream_));
-            launch_min_next_col(stream_, n_, d_row_ptr, d_col, d_next, d_next + F_);
+            launch_min_next_col(stream_, n_, F_, d_row_ptr, d_col, d_next, d_next + F_);
             std::vector<int> next((size_t)F_ + 1);
             HIP_CHECK(hipMemcpyAsync(next.data(), d_next, sizeof(int) * next.size(), hipMemcpyDeviceToHost, stream_));
             HIP_CHECK(hipStreamSynchronize(stream_));
@@ -432,7 +431,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
 
     // ---- labels, predictions, gradients (Booster::init) --------------------------------------
     d_y_ = dalloc<float>(n_);
-    upload(stream_, d_y_, ds.y.data(), (size_t)n_);
+    upload_large(stream_, d_y_, ds.y.data(), sizeof(float) * (size_t)n_);
     log_debug("bin matrix: %.3f s", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_bin).count());
     auto t_rest = std::chrono::steady_clock::now();
     n_yp_ = (long)param_.num_class * n_;
