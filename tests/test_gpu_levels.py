@@ -1,0 +1,55 @@
+"""The level kernels of the dense layout (thundergbm_amd/csrc/level_kernels.hip): what boost() runs in fewer launches
+against the stages one by one, at the edges of the work items and of the nodes a workgroup looks at together."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import datasets as D  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def one_by_one(s, rounds, depth, K):
+    for _ in range(rounds):
+        s.gradient()
+        for k in range(K):
+            s.tree_init(k)
+            for level in range(depth):
+                s.find_split(level)
+                s.partition(level)
+            s.finish_tree(k)
+
+
+@pytest.mark.parametrize("n,F,depth,bins,objective", [
+    (1, 1, 1, 255, "reg:linear"), (2047, 3, 2, 255, "reg:linear"), (2048, 5, 4, 16, "binary:logistic"),
+    (2049, 130, 5, 255, "reg:linear"), (20_480, 9, 8, 255, "binary:logistic"), (20_481, 4, 11, 64, "reg:linear"),
+    (5000, 12, 6, 1000, "reg:linear"), (4500, 8, 5, 255, "multi:softmax"), (300_000, 6, 9, 255, "reg:logistic")])
+def test_boost_equals_the_stages(n, F, depth, bins, objective):
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n + F)
+    X = rng.standard_normal((n, F)).astype(np.float32)
+    X[rng.random((n, F)) < 0.1] = 0
+    X[0, 0] = 1.0
+    z = X[:, 0] + np.abs(X[:, F // 2]) + 0.3 * rng.standard_normal(n)
+    K = 3 if objective.startswith("multi") else 1
+    y = z if objective == "reg:linear" else (np.digitize(z, [0, 1]) if K > 1 else z > 0.5)
+    y = np.asarray(y, np.float32)
+    val, rp, col = D.dense_to_csr(X)
+    models, maps, preds = [], [], []
+    for stages in (False, True):
+        s = T.Session(val, rp, col, y, depth=depth, n_trees=3, learning_rate=0.5, max_num_bin=bins, objective=objective,
+                      min_child_weight=0.5)
+        if stages:
+            one_by_one(s, 3, depth, K)
+        else:
+            s.boost(3)
+        models.append(s.model().tobytes())
+        maps.append(s.nid())
+        preds.append(s.y_pred())
+        s.close()
+    assert models[0] == models[1]
+    assert np.array_equal(maps[0], maps[1])
+    assert np.array_equal(preds[0], preds[1])

@@ -102,7 +102,7 @@ struct SplitCand {
     int index;    // global bin index
     GHPair miss;
     GHPair left;  // sum of the bins strictly below the candidate, within its feature
-    int pad[2];
+    int feature, bin;  // dense layout: its feature, its bin within the feature
 };
 
 // Dense column-blocked bin matrix: block b holds features [b*W, (b+1)*W) as n rows of W bytes.
@@ -264,6 +264,7 @@ struct TreeBuffers {
     float *leaf_value = nullptr;   // [n_nodes] prediction increment of a row that ended in the node (after pruning)
     int *end_bound = nullptr;      // [(row_blocks(n) + 1) x (2^depth - 1)] list positions of the row block boundaries
     int *hpair_begin = nullptr;    // [max_pairs + 1] first histogram item of every sibling pair
+    int4 *hpair_plan = nullptr;    // [max_pairs] dense layout: (hpair_built, its row-list segment), see plan_hist_item
     int *hpair_built = nullptr;    // [max_pairs] heap id of the node built from rows, -1 = inactive pair
     int *pitem_begin = nullptr;    // [2][max_level_nodes + 1] first partition item of every node of a level, by level parity
     int *pitem_nleft = nullptr;    // [max_pitems]
@@ -276,8 +277,9 @@ struct TreeBuffers {
     int n_grad_blocks = 0;
     // split finder packing: wavefront w scans global bins [pack_begin[w], pack_begin[w+1]) (whole features)
     const int *pack_begin = nullptr;
-    // per bin: distance to the last bin of its feature (low byte) and whether it is the feature's first bin (bit 8)
-    const unsigned short *bin_meta = nullptr;  // [n_bins]
+    // per bin: distance to the last bin of its feature (low byte), distance from the first one (next byte), and in the
+    // dense layout, whose feature ids fit 16 bits, the feature (high half)
+    const unsigned *bin_meta = nullptr;  // [n_bins]
     int n_packs = 0;
     const uint8_t *ignored = nullptr;  // [F] columns whose candidates score 0 this round (nullptr: none)
     // Features with more than 255 cut points (max_num_bin up to 65 535; CSR layout, per-node path): the node's split
@@ -352,6 +354,7 @@ struct TreeBuffers {
         t.leaf_value += K * n_nodes;
         t.end_bound += K * n_end_bound;
         t.hpair_begin += K * (max_level_nodes + 1);
+        t.hpair_plan += K * max_level_nodes;
         t.hpair_built += K * max_level_nodes;
         t.pitem_begin += K * 2 * (max_level_nodes + 1);
         t.pitem_nleft += K * ((size_t)max_pitems + 1);
@@ -400,7 +403,10 @@ void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mc
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
                             bool store_sibling = true);
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class = 1);
-void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, int n_class = 1);
+// Dense layout: the rows of a level's split nodes move into the children's lists. update: the nodes' best candidates have
+// not been applied to the tree yet (launch_best_update); it happens here.
+void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
+                            float rt_eps, float lambda, int n_class = 1);
 // Sparse level pass (tb.nid16 set): split search of a level (candidates into tb.cand, one slot per task / big
 // feature; launch_best_update follows) and the row -> node update. dump_hist: also store the (node, bin) tables
 // into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q). last_level: the tree's deepest level (the

@@ -1,0 +1,353 @@
+// The rows of a level move on to its nodes' children (dense layout): two launches per level. The first picks every node's
+// best candidate, applies it to the tree and decides left or right for every row; the second compacts the row lists and
+// leaves the next level's sibling pairs. What used to be launches of their own in between - the update of the tree, the
+// scan of the items' counts, the plan of the next level - is done again by every workgroup from a few hundred bytes
+// that it finds in the L2: a launch costs 4 to 8 us whatever it does, the repeated work well below one.
+// 500 k x 28, depth 8: five launches and 23 us a level (update 4.8, count 5.7, plan 5.5, scatter 4.9, gaps) -> two.
+#include <algorithm>
+
+#include "device_api.h"
+#include "kernel_common.h"
+#include "tree_common.h"
+
+namespace tgbm {
+namespace {
+
+// A partition work item: kPartChunk rows of one node. The nodes of a level own ceil(rows / kPartChunk) items each, at
+// least one (a node without rows still has a split record to fill), numbered node by node.
+struct NodeItem {
+    int x_in;   // node within the level, -1: there is no such item
+    int first;  // first item of the node
+    int count;  // items of the node
+    int2 seg;
+};
+
+// lds: kWaves ints, s: 5 ints; every thread of the workgroup calls
+__device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level, int item, int *lds, int *s) {
+    const int nl = 1 << level, off = nl - 1;
+    NodeItem out;
+    if (level == 0) {
+        out.count = max(1, (tb.n + kPartChunk - 1) / kPartChunk);
+        out.x_in = item < out.count ? 0 : -1;
+        out.first = 0;
+        out.seg = make_int2(0, tb.n);
+        return out;
+    }
+    if (threadIdx.x == 0) s[0] = -1;
+    int carry = 0;
+    for (int base = 0; base < nl && carry <= item; base += kBlock) {  // (carry is the same in every thread)
+        const int x_in = base + threadIdx.x;
+        int2 sg = make_int2(0, 0);
+        int cnt = 0;
+        if (x_in < nl) {
+            sg = tb.seg[off + x_in];
+            cnt = max(1, (sg.y - sg.x + kPartChunk - 1) / kPartChunk);
+        }
+        int tot;
+        const int ex = carry + block_excl_scan(cnt, lds, &tot);
+        if (item >= ex && item < ex + cnt) {
+            s[0] = x_in;
+            s[1] = ex;
+            s[2] = cnt;
+            s[3] = sg.x;
+            s[4] = sg.y;
+        }
+        carry += tot;
+    }
+    __syncthreads();
+    out.x_in = s[0];
+    out.first = s[1];
+    out.count = s[2];
+    out.seg = make_int2(s[3], s[4]);
+    return out;
+}
+
+// UPDATE: the nodes' candidates are fresh from the split search; else the tree has been updated already.
+// A row goes right if its bin is not below the split bin, or if it has no value of the feature and the default says so
+// (hist_tree_builder_single.cu:986-1011).
+template <bool DIRECT, typename BinT, bool UPDATE>
+__global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, DenseBins bins, int level, float rt_eps,
+                                                       float lambda) {
+    __shared__ int lds[kWaves];
+    __shared__ int s_item[5];
+    __shared__ SplitCand s_cand;
+    __shared__ float s_abs[kWaves];
+    __shared__ int s_idx[kWaves];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int *__restrict__ ridx = tb.list(level);
+    const int item = blockIdx.x;
+    const NodeItem it = locate_item(tb, level, item, lds, s_item);
+    if (it.x_in < 0) return;
+    const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
+    const int2 sg = it.seg;
+    const int pb = sg.x + (item - it.first) * kPartChunk;
+    const int pe = min(sg.y, pb + kPartChunk);
+    // All row ids first, then all bins, then the decisions, then the stores. Every load is unconditional (positions
+    // past the item's end are clamped to its last row), so each phase's loads are issued back to back and a thread's
+    // eight gathers are in flight together; a conditional load would make the compiler wait for everything
+    // outstanding, the previous store included, before the next one.
+    constexpr int R = kPartChunk / kBlock;
+    int row[R], b[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int pos = max(min(pb + k * kBlock + (int)threadIdx.x, pe - 1), 0);
+        row[k] = DIRECT ? pos : ridx[pos];
+    }
+    const TreeNode node = tb.nodes[x];
+    bool splits, found = false, dr = false;
+    int f = 0, sbid = 0;
+    if (UPDATE) {
+        const bool valid = node.is_valid;
+        float a_best = -1.f;
+        int i_best = 0x7fffffff;
+        SplitCand best;
+        best.score = 0.f;
+        best.index = 0x7fffffff;
+        best.miss = best.left = GHPair{0, 0};
+        best.feature = best.bin = 0;
+        if (valid)
+            for (int p = threadIdx.x; p < tb.n_packs; p += kBlock) {
+                const SplitCand c = tb.cand[(size_t)x_in * tb.n_packs + p];
+                const float a = fabsf(c.score);
+                // (index 0x7fffffff: a wavefront whose features have no bins)
+                const bool better = c.index != 0x7fffffff && (a > a_best || (a == a_best && c.index < i_best));
+                a_best = better ? a : a_best;
+                i_best = better ? c.index : i_best;
+                best.score = better ? c.score : best.score;
+                best.miss.g = better ? c.miss.g : best.miss.g;
+                best.miss.h = better ? c.miss.h : best.miss.h;
+                best.left.g = better ? c.left.g : best.left.g;
+                best.left.h = better ? c.left.h : best.left.h;
+                best.feature = better ? c.feature : best.feature;
+                best.bin = better ? c.bin : best.bin;
+            }
+        // larger |score|, then the smaller bin index; bin indices are distinct
+        float win = a_best;
+        int win_idx = i_best;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            const float oa = __shfl_xor(win, d);
+            const int oi = __shfl_xor(win_idx, d);
+            if (oa > win || (oa == win && oi < win_idx)) {
+                win = oa;
+                win_idx = oi;
+            }
+        }
+        if (lane_id() == 0) {
+            s_abs[wave_id()] = win;
+            s_idx[wave_id()] = win_idx;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i)
+            if (s_abs[i] > win || (s_abs[i] == win && s_idx[i] < win_idx)) {
+                win = s_abs[i];
+                win_idx = s_idx[i];
+            }
+        found = win_idx != 0x7fffffff;
+        if (found && a_best == win && i_best == win_idx) {
+            best.index = i_best;
+            s_cand = best;
+        }
+        __syncthreads();
+        splits = found && fabsf(s_cand.score) > rt_eps;
+        if (splits) {
+            f = s_cand.feature;
+            // (the byte that the model keeps, unless the features have more than 255 bins)
+            sbid = tb.split_bin != nullptr ? s_cand.bin : (int)(unsigned char)s_cand.bin;
+            dr = s_cand.score < 0;
+        }
+    } else {
+        splits = node_splits(node);
+        if (splits) {
+            f = node.split_feature_id;
+            sbid = tb.split_bin != nullptr ? tb.split_bin[x] : (int)node.split_bid;
+            dr = node.default_right;
+        }
+    }
+    // (the tree's own stores come last: nothing of this workgroup waits for them)
+    auto update = [&] {
+        if (!UPDATE || item != it.first || threadIdx.x != 0) return;
+        if (!node.is_valid) {
+            SplitPoint z{};
+            z.nid = -1;
+            z.split_fea_id = -1;
+            tb.sp[x_in] = z;
+        } else if (!found) {
+            no_split(tb, x, x_in);
+        } else {
+            const SplitCand c = s_cand;
+            apply_split(tb, x, x_in, node, c, c.feature, c.bin, tb.cut_val[c.index - (c.bin != 0 ? 1 : 0)], rt_eps, lambda);
+        }
+    };
+    if (!splits) {
+        if (threadIdx.x == 0) tb.pitem_nleft[item] = 0;
+        update();
+        return;
+    }
+    // A stored bin outside [lo, lo + span) means that the row has no value of the feature: the missing sentinel, or
+    // (a feature that shares its column with others, DenseBins::feat_col) a bin of another feature of the bundle.
+    int c = f, lo = 0, span = sizeof(BinT) == 2 ? kMissingBin16 : kMissingBin;
+    if (sizeof(BinT) == 1 && bins.feat_col != nullptr) {
+        c = bins.feat_col[f];
+        lo = bins.feat_lo[f];
+        span = tb.cut_row_ptr[f + 1] - tb.cut_row_ptr[f];
+    }
+    const BinT *column = reinterpret_cast<const BinT *>(bins.col) + (size_t)c * bins.col_stride;
+    int nleft = 0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) b[k] = column[row[k]];
+    unsigned rights = 0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int t = b[k] - lo;
+        const bool right = ((unsigned)t >= (unsigned)span) ? dr : (t >= sbid);
+        rights |= (right ? 1u : 0u) << k;
+        if (pb + k * kBlock + (int)threadIdx.x < pe) nleft += right ? 0 : 1;
+    }
+    // the decisions of a thread's eight rows as one byte (k_split_scatter gives the same rows to the same thread)
+    static_assert(R <= 8, "a byte per thread holds the decisions of its rows");
+    tb.goes_right[(size_t)item * kBlock + threadIdx.x] = (uint8_t)rights;
+    const int tot = block_sum(nleft, lds);
+    if (threadIdx.x == 0) tb.pitem_nleft[item] = tot;
+    update();
+}
+
+// Stable two-way compaction of a work item's rows into the children's segments with wavefront ballots and popcounts;
+// where the item's rows go follows from the counts of its node's items, which the workgroup adds up itself (a node of
+// 10 M rows has 4 883 of them: 20 KB from the L2). Every node's first item also leaves the children's segments and the
+// pair of the next level: the child with fewer rows is built from them (ties: the left one, as
+// hist_tree_builder_single.cu:466-467), the other one comes from subtraction. (Moving the gradient pairs along with the
+// row ids was measured: it makes the histogram's gradient reads sequential but costs more here than it saves there.)
+template <bool DIRECT>
+__global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, int level) {
+    __shared__ int lds[kWaves];
+    __shared__ int s_item[5];
+    __shared__ int s_sum[2][kWaves];
+    __shared__ int s_cnt[kPartChunk / kBlock][2][kWaves];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int *__restrict__ ridx_cur = tb.list(level);
+    int *__restrict__ ridx_next = tb.list(level + 1);
+    const int item = blockIdx.x;
+    const NodeItem it = locate_item(tb, level, item, lds, s_item);
+    if (it.x_in < 0) return;
+    const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
+    const int2 sg = it.seg;
+    const int mine = item - it.first;  // of the node's items
+    const int pb = sg.x + mine * kPartChunk;
+    const int pe = min(sg.y, pb + kPartChunk);
+    const int lane = lane_id(), w = wave_id();
+    const TreeNode &nd = tb.nodes[x];
+    const bool splits = node_splits(nd);
+    const int lch = nd.lch_index, rch = nd.rch_index;
+    // all loads of the item first (unconditional, clamped positions), then one barrier for the sums of the node's counts
+    // and the wavefront counts of all eight steps, then all stores
+    constexpr int R = kPartChunk / kBlock;
+    int row[R];
+    const unsigned rights = tb.goes_right[(size_t)item * kBlock + threadIdx.x];  // bit k: the thread's k-th row goes right
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int pos = max(min(pb + k * kBlock + (int)threadIdx.x, pe - 1), 0);
+        row[k] = DIRECT ? pos : ridx_cur[pos];
+    }
+    int before = 0, total = 0;
+    for (int t = threadIdx.x; t < it.count; t += kBlock) {
+        const int c = tb.pitem_nleft[it.first + t];
+        total += c;
+        before += t < mine ? c : 0;
+    }
+    before = wave_sum_i(before);
+    total = wave_sum_i(total);
+    if (lane == 0) {
+        s_sum[0][w] = before;
+        s_sum[1][w] = total;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const bool valid = pb + k * kBlock + (int)threadIdx.x < pe;
+        const bool right = (rights >> k) & 1u;
+        const unsigned long long mL = __ballot(valid && !right), mR = __ballot(valid && right);
+        if (lane == 0) {
+            s_cnt[k][0][w] = __popcll(mL);
+            s_cnt[k][1][w] = __popcll(mR);
+        }
+    }
+    __syncthreads();
+    before = total = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+        before += s_sum[0][i];
+        total += s_sum[1][i];
+    }
+    if (mine == 0 && threadIdx.x == 0) {
+        const bool singles = tb.singles(level + 1);
+        const int nleft = splits ? total : 0, nright = (sg.y - sg.x) - nleft;
+        const int2 left = splits ? make_int2(sg.x, sg.x + nleft) : make_int2(0, 0);
+        const int2 right = splits ? make_int2(sg.x + nleft, sg.y) : make_int2(0, 0);
+        tb.node_nleft[x_in] = nleft;
+        tb.seg[lch] = left;
+        tb.seg[rch] = right;
+        if (singles) {
+            // no parent histograms below this level (the arena is smaller than the level): every child of a split node is
+            // built from its own rows, and the "pairs" of the next level are its single nodes
+            tb.hpair_built[2 * x_in] = splits ? lch : -1;
+            tb.hpair_built[2 * x_in + 1] = splits ? rch : -1;
+            tb.hpair_plan[2 * x_in] = make_int4(splits ? lch : -1, left.x, left.y, 0);
+            tb.hpair_plan[2 * x_in + 1] = make_int4(splits ? rch : -1, right.x, right.y, 0);
+        } else {
+            const bool build_left = nleft <= nright;
+            const int built = splits ? (build_left ? lch : rch) : -1;
+            const int2 bs = build_left ? left : right;
+            tb.hpair_built[x_in] = built;
+            tb.hpair_plan[x_in] = make_int4(built, bs.x, bs.y, 0);
+        }
+    }
+    if (!splits) return;
+    int left_base = sg.x + before;
+    int right_base = sg.x + total + ((pb - sg.x) - before);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const bool valid = pb + k * kBlock + (int)threadIdx.x < pe;
+        const bool right = (rights >> k) & 1u;
+        const unsigned long long mL = __ballot(valid && !right), mR = __ballot(valid && right);
+        int bL = 0, bR = 0, tL = 0, tR = 0;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+            const int cl = s_cnt[k][0][i], cr = s_cnt[k][1][i];
+            if (i < w) {
+                bL += cl;
+                bR += cr;
+            }
+            tL += cl;
+            tR += cr;
+        }
+        if (valid) {
+            const int dest = right ? right_base + bR + lanes_below(mR) : left_base + bL + lanes_below(mL);
+            ridx_next[dest] = row[k];
+        }
+        left_base += tL;
+        right_base += tR;
+    }
+}
+
+}  // namespace
+
+void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
+                            float rt_eps, float lambda, int n_class) {
+    if (level == tb.depth - 1) return;  // the last level's children never get row lists (see k_tree_end)
+    const int most = level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
+    const dim3 items(most, 1, n_class);
+#define TGBM_SPLIT_COUNT(D, T, U) k_split_count<D, T, U><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
+    if (bins.bin_bytes == 2) {
+        if (level == 0) { if (update) TGBM_SPLIT_COUNT(true, uint16_t, true); else TGBM_SPLIT_COUNT(true, uint16_t, false); }
+        else { if (update) TGBM_SPLIT_COUNT(false, uint16_t, true); else TGBM_SPLIT_COUNT(false, uint16_t, false); }
+    } else {
+        if (level == 0) { if (update) TGBM_SPLIT_COUNT(true, uint8_t, true); else TGBM_SPLIT_COUNT(true, uint8_t, false); }
+        else { if (update) TGBM_SPLIT_COUNT(false, uint8_t, true); else TGBM_SPLIT_COUNT(false, uint8_t, false); }
+    }
+#undef TGBM_SPLIT_COUNT
+    if (level == 0) k_split_scatter<true><<<items, kBlock, 0, s>>>(tb, level);
+    else k_split_scatter<false><<<items, kBlock, 0, s>>>(tb, level);
+}
+
+}  // namespace tgbm

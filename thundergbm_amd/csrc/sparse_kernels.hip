@@ -203,7 +203,7 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
             c.index = idx;
             c.miss = r.miss;
             c.left = r.left;
-            c.pad[0] = c.pad[1] = 0;
+            c.feature = c.bin = 0;
             tb.cand[(size_t)node * tb.n_packs + cand_slot] = c;
         }
     }
@@ -826,7 +826,7 @@ __global__ __launch_bounds__(kSortedBlock) void k_sparse_sorted(TreeBuffers tb_a
         const GHPair S = s_S[x];
         SplitCand o;
         o.miss = GHPair{S.g - tot[j].g, S.h - tot[j].h};
-        o.pad[0] = o.pad[1] = 0;
+        o.feature = o.bin = 0;
         if (win_head) {
             o.score = sc_head[j];
             o.index = fbegin;

@@ -79,6 +79,7 @@ class Trainer {
     TreeBuffers set_of(int k) const;
     void find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class);
     void partition_sets(const TreeBuffers &tb, int level, int n_class);
+    bool update_with_partition(int level) const;
     void build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class);
     void build_round_together();
     void log_plan(const TreeBuffers &tb);

@@ -581,6 +581,7 @@ void Trainer::alloc_tree_buffers() {
     tb.hpair_begin = dalloc<int>(S * ((size_t)max_level_nodes + 1));
     tb.leaf_value = dalloc<float>(S * tb.n_nodes);
     tb.end_bound = dalloc<int>(S * tb.n_end_bound);
+    tb.hpair_plan = dalloc<int4>(S * max_level_nodes);
     tb.hpair_built = dalloc<int>(S * max_level_nodes);
     tb.pitem_begin = dalloc<int>(S * 2 * ((size_t)max_level_nodes + 1));
     tb.pitem_nleft = dalloc<int>(S * ((size_t)tb.max_pitems + 1));
@@ -645,11 +646,12 @@ void Trainer::alloc_tree_buffers() {
     int *d_pack = dalloc<int>(pack_begin.size());
     upload(stream_, d_pack, pack_begin.data(), pack_begin.size());
     tb.pack_begin = d_pack;
-    std::vector<unsigned short> bin_meta((size_t)n_bins_);
+    std::vector<unsigned> bin_meta((size_t)n_bins_);
     for (int f = 0; f < F_; ++f)
         for (int b = h_cut_row_ptr_[f]; b < h_cut_row_ptr_[f + 1]; ++b)
-            bin_meta[(size_t)b] = (unsigned short)((h_cut_row_ptr_[f + 1] - 1 - b) | (b == h_cut_row_ptr_[f] ? 0x100 : 0));
-    unsigned short *d_meta = dalloc<unsigned short>(bin_meta.size());
+            bin_meta[(size_t)b] = ((unsigned)(h_cut_row_ptr_[f + 1] - 1 - b) & 0xffu) |
+                                  ((unsigned)(b - h_cut_row_ptr_[f]) & 0xffu) << 8 | (unsigned)f << 16;
+    unsigned *d_meta = dalloc<unsigned>(bin_meta.size());
     upload(stream_, d_meta, bin_meta.data(), bin_meta.size());
     tb.bin_meta = d_meta;
     tb.cand = dalloc<SplitCand>(S * max_level_nodes * tb.n_packs);
@@ -994,10 +996,17 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                               !(in_boost_ && level == param_.depth - 1));
     }
-    launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
+    if (!update_with_partition(level)) launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
     mark(PH_SPLIT, level);
     lookup_level_ = level;  // until partition(level) moves the rows into the children's lists
     HIP_CHECK_LAUNCHES("find_split");
+}
+
+// Inside boost() nobody looks at a level's split records between its split search and its partition, so the dense
+// layout's partition picks the nodes' best candidates itself (a launch less per level). The last level is not
+// partitioned, and a level served in batches needs its updates batch by batch.
+bool Trainer::update_with_partition(int level) const {
+    return in_boost_ && !sparse_ && level < param_.depth - 1 && (hist_cap_level_ < 0 || level < hist_cap_level_);
 }
 
 void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class) {
@@ -1028,7 +1037,7 @@ void Trainer::partition_sets(const TreeBuffers &tb, int level, int n_class) {
     } else if (sparse_)
         launch_partition_csr(stream_, tb, csr_, level, n_class);
     else
-        launch_partition_dense(stream_, tb, bins_, level, n_class);
+        launch_partition_dense(stream_, tb, bins_, level, update_with_partition(level), param_.rt_eps, param_.lambda, n_class);
     mark(PH_PARTITION, level);
     HIP_CHECK_LAUNCHES("partition");
 }

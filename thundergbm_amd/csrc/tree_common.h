@@ -1,0 +1,194 @@
+// What the tree-building kernel sources share: workgroup scans and sums, the record of a node's split, the plan of a
+// level's histogram work items.
+#pragma once
+#include "device_api.h"
+#include "kernel_common.h"
+
+namespace tgbm {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / 64;
+constexpr int kHistMinChunk = 1024;
+constexpr int kHistBlock = 1024;      // threads per histogram workgroup (they share one LDS histogram)
+
+// Exclusive scan of one int per thread over a 256-thread block; lds needs kWaves ints.
+__device__ int block_excl_scan(int v, int *lds, int *total) {
+    int lane = lane_id(), w = wave_id();
+    int inc = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        int t = __shfl_up(inc, d);
+        if (lane >= d) inc += t;
+    }
+    if (lane == 63) lds[w] = inc;
+    __syncthreads();
+    int base = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+        int c = lds[i];
+        if (i < w) base += c;
+        tot += c;
+    }
+    *total = tot;
+    __syncthreads();
+    return base + inc - v;
+}
+
+__device__ int block_sum(int v, int *lds) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    if (lane_id() == 0) lds[wave_id()] = v;
+    __syncthreads();
+    int tot = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) tot += lds[i];
+    __syncthreads();
+    return tot;
+}
+
+__device__ __forceinline__ float wave_sum_f(float v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+
+// Node x (x_in within its level) stays a leaf: none of its candidates can split it, or it has none.
+__device__ __forceinline__ void no_split(const TreeBuffers &tb, int x, int x_in) {
+    SplitPoint z{};
+    z.nid = x;
+    z.split_fea_id = -1;
+    TreeNode &node = tb.nodes[x];
+    const int lch = node.lch_index, rch = node.rch_index;
+    tb.sp[x_in] = z;
+    node.is_leaf = true;
+    tb.nodes[lch].is_valid = false;
+    tb.nodes[rch].is_valid = false;
+}
+
+// The split record of node x from its best candidate c (the split feature and the candidate's bin within it), applied to
+// the tree: hist_tree_builder_single.cu:365-389 and update_tree, :860-899. `node` is a copy that was loaded before: a
+// load that follows a store waits for the store to reach memory, so everything is read first and written last.
+// fval: cut_val[c.index - 1], or cut_val[c.index] for the first bin of a feature
+__device__ __forceinline__ void apply_split(const TreeBuffers &tb, int x, int x_in, TreeNode node, const SplitCand &c,
+                                            int f, int bin, float fval, float rt_eps, float lambda) {
+    SplitPoint s{};
+    s.split_fea_id = f;
+    s.nid = x;
+    s.gain = fabsf(c.score);
+    s.split_bid = (int)(unsigned char)bin;
+    s.fea_missing_gh = c.miss;
+    s.default_right = c.score < 0;
+    s.best_index = c.index;
+    if (bin != 0) {
+        s.lch_sum_gh = c.left;
+        s.fval = fval;
+    } else {
+        s.lch_sum_gh = GHPair{0, 0};
+        s.fval = (float)((double)(fval - fabsf(fval)) - 1e-5);
+    }
+    TreeNode &out = tb.nodes[x];
+    TreeNode &l = tb.nodes[node.lch_index];
+    TreeNode &r = tb.nodes[node.rch_index];
+    if (s.gain > rt_eps) {
+        GHPair ls = s.lch_sum_gh;
+        if (!s.default_right) {
+            ls.g += s.fea_missing_gh.g;
+            ls.h += s.fea_missing_gh.h;
+        }
+        GHPair rs{node.sum_gh_pair.g - ls.g, node.sum_gh_pair.h - ls.h};
+        const float lw = -ls.g / (ls.h + lambda), rw = -rs.g / (rs.h + lambda);
+        out.gain = s.gain;
+        out.split_feature_id = f;
+        out.split_value = s.fval;
+        out.split_bid = (unsigned char)s.split_bid;
+        out.default_right = s.default_right != 0;
+        if (tb.split_bin != nullptr) tb.split_bin[x] = bin;
+        l.is_valid = true;
+        r.is_valid = true;
+        l.sum_gh_pair = ls;
+        r.sum_gh_pair = rs;
+        l.base_weight = lw;
+        r.base_weight = rw;
+    } else {
+        out.is_leaf = true;
+        l.is_valid = false;
+        r.is_valid = false;
+    }
+    tb.sp[x_in] = s;
+}
+
+__device__ __forceinline__ int wave_sum_i(int v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+
+// Histogram work items of a level, planned by whoever needs them from the level's pairs (hpair_plan) instead of by a
+// launch of its own: every wavefront of the asking workgroup does the same few steps, so nothing waits at a barrier.
+// Every built node adds up to one partly filled item: the items are sized so that their number stays within
+// target_hitems (= the workgroups the chip holds at once; one more would run as a second round).
+struct HistPlan {
+    int pair = -1;  // the pair that `item` belongs to, -1: there is no such item
+    int built = 0, chunk = 0, first_item = 0;
+    int item0 = 0;  // first item of the pairs that the launch serves (TreeBuffers::hpair_lo)
+    int2 seg = make_int2(0, 0);
+};
+// publish (wave-uniform): also store the level's plan - hpair_begin and ctl[level] -, for k_hist_merge and the profile
+__device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_pairs, int item, bool publish, int level) {
+    const int lane = lane_id();
+    int4 mine = make_int4(-1, 0, 0, 0);
+    if (lane < n_pairs) mine = tb.hpair_plan[lane];
+    int total = 0, n_built = 0;
+    for (int p0 = 0; p0 < n_pairs; p0 += 64) {
+        const int4 q = p0 == 0 ? mine : (p0 + lane < n_pairs ? tb.hpair_plan[p0 + lane] : make_int4(-1, 0, 0, 0));
+        total += q.x >= 0 ? q.z - q.y : 0;
+        n_built += q.x >= 0 ? 1 : 0;
+    }
+    total = wave_sum_i(total);
+    n_built = wave_sum_i(n_built);
+    const int room = max(tb.target_hitems / 4, tb.target_hitems - n_built);
+    int chunk = (total + room - 1) / room;
+    chunk = max(kHistMinChunk, (chunk + 255) / 256 * 256);
+    HistPlan out;
+    out.chunk = chunk;
+    int carry = 0;
+    for (int p0 = 0; p0 < n_pairs; p0 += 64) {
+        const int4 q = p0 == 0 ? mine : (p0 + lane < n_pairs ? tb.hpair_plan[p0 + lane] : make_int4(-1, 0, 0, 0));
+        const int cnt = q.x >= 0 ? (q.z - q.y + chunk - 1) / chunk : 0;
+        int inc = cnt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int t = __shfl_up(inc, d);
+            if (lane >= d) inc += t;
+        }
+        const int ex = carry + inc - cnt;
+        const int lo = tb.hpair_lo(level);
+        if (lo >= p0 && lo < p0 + 64) out.item0 = __shfl(ex, lo - p0);
+        if (publish && p0 + lane < n_pairs) tb.hpair_begin[p0 + lane] = ex;
+        const unsigned long long owner = __ballot(item >= ex && item < ex + cnt);
+        if (owner != 0ull) {
+            const int l = __ffsll((long long)owner) - 1;
+            out.pair = p0 + l;
+            out.built = __shfl(q.x, l);
+            out.seg = make_int2(__shfl(q.y, l), __shfl(q.z, l));
+            out.first_item = __shfl(ex, l);
+        }
+        carry += __shfl(inc, 63);
+    }
+    if (publish && lane == 0) {
+        tb.hpair_begin[n_pairs] = carry;
+        tb.ctl[level] = LevelCtl{chunk, carry, 0, total};
+    }
+    // (the same in every lane: scalar registers from here on)
+    out.pair = __builtin_amdgcn_readfirstlane(out.pair);
+    out.built = __builtin_amdgcn_readfirstlane(out.built);
+    out.chunk = __builtin_amdgcn_readfirstlane(out.chunk);
+    out.first_item = __builtin_amdgcn_readfirstlane(out.first_item);
+    out.item0 = __builtin_amdgcn_readfirstlane(out.item0);
+    out.seg = make_int2(__builtin_amdgcn_readfirstlane(out.seg.x), __builtin_amdgcn_readfirstlane(out.seg.y));
+    return out;
+}
+
+}  // namespace
+}  // namespace tgbm

@@ -6,55 +6,10 @@
 
 #include "device_api.h"
 #include "kernel_common.h"
+#include "tree_common.h"
 
 namespace tgbm {
 namespace {
-
-constexpr int kBlock = 256;
-constexpr int kWaves = kBlock / 64;
-constexpr int kHistMinChunk = 1024;
-constexpr int kHistBlock = 1024;      // threads per histogram workgroup (they share one LDS histogram)
-
-// Exclusive scan of one int per thread over a 256-thread block; lds needs kWaves ints.
-__device__ int block_excl_scan(int v, int *lds, int *total) {
-    int lane = lane_id(), w = wave_id();
-    int inc = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int t = __shfl_up(inc, d);
-        if (lane >= d) inc += t;
-    }
-    if (lane == 63) lds[w] = inc;
-    __syncthreads();
-    int base = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-        int c = lds[i];
-        if (i < w) base += c;
-        tot += c;
-    }
-    *total = tot;
-    __syncthreads();
-    return base + inc - v;
-}
-
-__device__ int block_sum(int v, int *lds) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-    if (lane_id() == 0) lds[wave_id()] = v;
-    __syncthreads();
-    int tot = 0;
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) tot += lds[i];
-    __syncthreads();
-    return tot;
-}
-
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-    return v;
-}
 
 // Largest p in [0, n) with begin[p] <= item (begin is non-decreasing, begin[0] <= item < begin[n]).
 __device__ int find_owner(const int *begin, int n, int item) {
@@ -431,21 +386,38 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
     const int *__restrict__ ridx = tb.list(level);
-    const int2 *__restrict__ seg = tb.seg;
-    const int *__restrict__ hpair_begin = tb.hpair_begin;
-    const int *__restrict__ hpair_built = tb.hpair_built;
     const QuantCtl *__restrict__ quant = tb.quant;
     const int *__restrict__ blk_bin_begin = tb.blk_bin_begin;
     const int *__restrict__ feat_lds_off = tb.feat_lds_off;
     longlong2 *__restrict__ partial = tb.partial;
     const int n_bins = tb.n_bins;
-    const LevelCtl c = tb.ctl[level];
     // (the feature blocks of an item are neighbours in the launch order: the item's row list and gradient pairs, which
     // every block reads again, are then fetched while they still sit in an L2 - with the items of a block as
     // neighbours, every block of 500 k x 2000 data fetched them from HBM again: 2.72 -> 2.29 ms per tree)
     const int item = blockIdx.y;
-    if (item >= c.n_hitems) return;
     const int fb = blockIdx.x;
+    // The item's node and rows: the same few look-ups in every lane (uniform addresses: scalar loads) or in every
+    // wavefront, so that the first row loads can be issued before the barrier that publishes the LDS histogram's clearing.
+    int node, hchunk;
+    int2 sg;
+    int first_item;  // of the node
+    int item0 = 0;
+    if constexpr (!DIRECT) {
+        const HistPlan plan = plan_hist_item(tb, n_pairs, item, fb == 0 && item == 0 && threadIdx.x < 64, level);
+        if (plan.pair < 0) return;
+        node = plan.built;
+        sg = plan.seg;
+        hchunk = plan.chunk;
+        first_item = plan.first_item;
+        item0 = plan.item0;
+    } else {
+        const LevelCtl c = tb.ctl[level];
+        if (item >= c.n_hitems) return;
+        node = 0;
+        sg = make_int2(0, tb.n);
+        hchunk = c.hchunk;
+        first_item = 0;
+    }
     const int bin0 = blk_bin_begin[fb];
     const int nb = blk_bin_begin[fb + 1] - bin0;
     if (nb == 0) return;
@@ -453,13 +425,8 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     const int flush_rows = quant->flush_rows;
     const int gh_objective = bins.gh_objective;
     const bool word_lane = bins.gh_lane >= 0 && (int)(threadIdx.x % LPR) == bins.gh_lane;
-    // The item's node and rows: the same few look-ups in every lane (uniform addresses: scalar loads), so that the
-    // first row loads can be issued before the barrier that publishes the LDS histogram's clearing.
-    const int p = find_owner(hpair_begin, n_pairs, item);
-    const int node = hpair_built[p];
-    const int2 sg = seg[node];
-    const int begin = __builtin_amdgcn_readfirstlane(sg.x + (item - hpair_begin[p]) * c.hchunk);
-    const int end = __builtin_amdgcn_readfirstlane(min(sg.y, begin + c.hchunk));
+    const int begin = __builtin_amdgcn_readfirstlane(sg.x + (item - first_item) * hchunk);
+    const int end = __builtin_amdgcn_readfirstlane(min(sg.y, begin + hchunk));
     const int x_in = node - ((1 << level) - 1);
     if (x_in < tb.lvl_x0 || x_in >= tb.lvl_x1) return;  // not in the batch of nodes this launch serves
     if (threadIdx.x == 0) {
@@ -472,8 +439,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
         s_shift[1] = shift.y;
         if (fb == 0) tb.hitem_shift[item] = shift;
     }
-    // (slots of `partial` count from the first item of the served batch of nodes: item 0 unless the arena is capped)
-    const int item0 = hpair_begin[tb.hpair_lo(level)];
+    // (slots of `partial` count from item0, the first item of the served batch of nodes: 0 unless the arena is capped)
     const unsigned long long h_mask = (1ull << h_bits) - 1ull;  // h_bits <= 32
     constexpr int RPS = BLK / LPR;  // rows per step of the whole block
     // rows per thread and stage: what the registers left over by the drain accumulators hold without spills (64
@@ -593,7 +559,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
         }
     }
     __syncthreads();
-    if (c.hchunk <= flush_rows) {
+    if (hchunk <= flush_rows) {
         // an item this short was never drained: its packed LDS words are the complete sums and go out as
         // they are (8 bytes per bin instead of 16; k_hist_merge unpacks them)
         unsigned long long *out = reinterpret_cast<unsigned long long *>(partial) + (size_t)(item - item0) * n_bins + bin0;
@@ -1074,6 +1040,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
     long long incg[4], inch[4];
     int lastb[4];  // pack-relative index of the last bin of the element's feature
     bool valid[4], head[4], last[4], ign[4];
+    unsigned meta[4] = {0, 0, 0, 0};
     long long rung = 0, runh = 0;
     bool any_head = false;
 #pragma unroll
@@ -1088,10 +1055,10 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
         if (valid[j]) {
             const longlong2 v = s_v[w][lane * 4 + j];
             // one word per bin instead of the chain bin -> feature -> feature's bin range
-            const unsigned meta = tb.bin_meta[b];  // low byte: bins up to the feature's last one, bit 8: first bin
+            meta[j] = tb.bin_meta[b];
             ign[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[b]] != 0;
-            const int to_last = (int)(meta & 0xffu);
-            head[j] = (meta & 0x100u) != 0;
+            const int to_last = (int)(meta[j] & 0xffu);
+            head[j] = (meta[j] & 0xff00u) == 0;
             last[j] = to_last == 0;
             lastb[j] = b + to_last - b_begin;
             if (head[j]) {
@@ -1150,6 +1117,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
     float best = -1.f;  // |score| of the lane's best candidate
     float best_score = 0.f;
     int best_idx = 0x7fffffff;
+    unsigned best_meta = 0;
     GHPair best_miss{0, 0}, best_left{0, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1166,6 +1134,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
                 best = a;
                 best_score = score;
                 best_idx = b_begin + lane * 4 + j;
+                best_meta = meta[j];
                 best_miss = m;
                 best_left = l;
             }
@@ -1192,7 +1161,8 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
         c.index = best_idx;
         c.miss = best_miss;
         c.left = best_left;
-        c.pad[0] = c.pad[1] = 0;
+        c.feature = (int)(best_meta >> 16);
+        c.bin = (int)(best_meta >> 8 & 0xffu);
         tb.cand[(size_t)x_in * tb.n_packs + pack] = c;
     }
 }
@@ -1343,7 +1313,8 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
         c.index = best_idx;
         c.miss = m;
         c.left = best_left;
-        c.pad[0] = c.pad[1] = 0;
+        c.feature = f;
+        c.bin = best_idx - cb;
         *out = c;
     }
 }
@@ -1419,135 +1390,21 @@ __global__ __launch_bounds__(kBlock) void k_best_update(TreeBuffers tb_all, int 
         }
     }
     if (best_pack < 0) {  // no candidate at all (a node none of whose rows stores a value): a leaf
-        SplitPoint z{};
-        z.nid = x;
-        z.split_fea_id = -1;
-        sp = z;
-        node.is_leaf = true;
-        tb.nodes[node.lch_index].is_valid = false;
-        tb.nodes[node.rch_index].is_valid = false;
+        no_split(tb, x, x_in);
         return;
     }
     const SplitCand c = tb.cand[(size_t)x_in * tb.n_packs + best_pack];
     const int f = tb.cut_fid[c.index];
-    const int fbegin = tb.cut_row_ptr[f];
-    SplitPoint s{};
-    s.split_fea_id = f;
-    s.nid = x;
-    s.gain = fabsf(c.score);
-    s.split_bid = (int)(unsigned char)(c.index - fbegin);
-    s.fea_missing_gh = c.miss;
-    s.default_right = c.score < 0;
-    s.best_index = c.index;
-    if (c.index != fbegin) {
-        s.lch_sum_gh = c.left;
-        s.fval = tb.cut_val[c.index - 1];
-    } else {
-        s.lch_sum_gh = GHPair{0, 0};
-        float c0 = tb.cut_val[fbegin];
-        s.fval = (float)((double)(c0 - fabsf(c0)) - 1e-5);
-    }
-    sp = s;
-    if (s.gain > rt_eps) {
-        node.gain = s.gain;
-        TreeNode &l = tb.nodes[node.lch_index];
-        TreeNode &r = tb.nodes[node.rch_index];
-        l.is_valid = true;
-        r.is_valid = true;
-        node.split_feature_id = f;
-        node.split_value = s.fval;
-        node.split_bid = (unsigned char)s.split_bid;
-        if (tb.split_bin != nullptr) tb.split_bin[x] = c.index - fbegin;
-        GHPair ls = s.lch_sum_gh;
-        if (!s.default_right) {
-            ls.g += s.fea_missing_gh.g;
-            ls.h += s.fea_missing_gh.h;
-            node.default_right = false;
-        } else {
-            node.default_right = true;
-        }
-        GHPair rs{node.sum_gh_pair.g - ls.g, node.sum_gh_pair.h - ls.h};
-        l.sum_gh_pair = ls;
-        r.sum_gh_pair = rs;
-        l.base_weight = -ls.g / (ls.h + lambda);
-        r.base_weight = -rs.g / (rs.h + lambda);
-    } else {
-        node.is_leaf = true;
-        tb.nodes[node.lch_index].is_valid = false;
-        tb.nodes[node.rch_index].is_valid = false;
-    }
+    const int bin = c.index - tb.cut_row_ptr[f];
+    apply_split(tb, x, x_in, node, c, f, bin, tb.cut_val[c.index - (bin != 0 ? 1 : 0)], rt_eps, lambda);
 }
 
 // ------------------------------------------------------------------------------ partition
 
-// Partition work items: every node of a level that holds rows owns ceil(rows / kPartChunk) items, planned one level
-// ahead (k_tree_init for the root, k_part_scan_plan for the children it creates) so that no planning step sits
-// between the split search and the partition; the items of a node that did not split return at once.
-// Decide left/right for every row of a work item from the split feature's column of the bin matrix
-// (missing -> default direction, else right iff bin >= split bin; the reference's rule at
-// hist_tree_builder_single.cu:986-1011) and count the rows that go left.
-template <bool DIRECT, typename BinT>
-__global__ __launch_bounds__(kBlock) void k_part_count_dense(TreeBuffers tb_all, DenseBins bins, int level) {
-    __shared__ int lds[kWaves];
-    __shared__ int s_x;
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    const int *__restrict__ ridx = tb.list(level);
-    const int item = blockIdx.x;
-    if (item >= tb.ctl[level].n_pitems) return;
-    const int nl = 1 << level, off = nl - 1;
-    if (threadIdx.x == 0) s_x = find_owner(tb.pbegin(level), nl, item);
-    __syncthreads();
-    const int x_in = s_x;
-    const TreeNode &nd = tb.nodes[off + x_in];
-    if (!node_splits(nd)) {
-        if (threadIdx.x == 0) tb.pitem_nleft[item] = 0;
-        return;
-    }
-    const int2 sg = tb.seg[off + x_in];
-    const int pb = sg.x + (item - tb.pbegin(level)[x_in]) * kPartChunk;
-    const int pe = min(sg.y, pb + kPartChunk);
-    const int f = nd.split_feature_id;
-    // (features of more than 255 bins keep their split bin in a side array: TreeNode::split_bid is a byte)
-    const int sbid = tb.split_bin != nullptr ? tb.split_bin[off + x_in] : (int)nd.split_bid;
-    const bool dr = nd.default_right;
-    // A stored bin outside [lo, lo + span) means that the row has no value of the feature: the missing sentinel, or
-    // (a feature that shares its column with others, DenseBins::feat_col) a bin of another feature of the bundle.
-    int c = f, lo = 0, span = sizeof(BinT) == 2 ? kMissingBin16 : kMissingBin;
-    if (sizeof(BinT) == 1 && bins.feat_col != nullptr) {
-        c = bins.feat_col[f];
-        lo = bins.feat_lo[f];
-        span = tb.cut_row_ptr[f + 1] - tb.cut_row_ptr[f];
-    }
-    const BinT *column = reinterpret_cast<const BinT *>(bins.col) + (size_t)c * bins.col_stride;
-    int nleft = 0;
-    // All row ids first, then all bins, then the decisions, then the stores. Every load is unconditional (positions
-    // past the item's end are clamped to its last row), so each phase's loads are issued back to back and a thread's
-    // eight gathers are in flight together; a conditional load would make the compiler wait for everything
-    // outstanding, the previous store included, before the next one.
-    constexpr int R = kPartChunk / kBlock;
-    int row[R], b[R];
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int pos = min(pb + k * kBlock + (int)threadIdx.x, pe - 1);
-        row[k] = DIRECT ? pos : ridx[pos];
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) b[k] = column[row[k]];
-    unsigned rights = 0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int t = b[k] - lo;
-        const bool right = ((unsigned)t >= (unsigned)span) ? dr : (t >= sbid);
-        rights |= (right ? 1u : 0u) << k;
-        if (pb + k * kBlock + (int)threadIdx.x < pe) nleft += right ? 0 : 1;
-    }
-    // the decisions of a thread's eight rows as one byte (k_part_scatter gives the same rows to the same thread)
-    static_assert(R <= 8, "a byte per thread holds the decisions of its rows");
-    tb.goes_right[(size_t)item * kBlock + threadIdx.x] = (uint8_t)rights;
-    int tot = block_sum(nleft, lds);
-    if (threadIdx.x == 0) tb.pitem_nleft[item] = tot;
-}
-
+// Row lists of the CSR layout. Partition work items: every node of a level that holds rows owns ceil(rows / kPartChunk)
+// items, planned one level ahead (k_tree_init for the root, k_part_scan_plan for the children it creates) so that no
+// planning step sits between the split search and the partition; the items of a node that did not split return at once.
+// (The dense layout's partition plans its items itself: level_kernels.hip.)
 // Scan the per-item left counts, publish the children's row segments and plan the histogram work
 // of the next level: per sibling pair the child with fewer rows is built (ties: the left one, as
 // hist_tree_builder_single.cu:466-467), the other one comes from subtraction. One workgroup.
@@ -2335,7 +2192,11 @@ template <int LPR, int SLOTS, bool BIN16>
 static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh,
                               int level, int n_class) {
     const int n_pairs = tb.n_hpairs(level);
-    dim3 grid(bins.n_blocks, tb.max_hitems, n_class);
+    // (an upper bound on the work items: whole chunks of the rows that can be built - half of them below the root, unless
+    // single nodes are built - and one partly filled item per built node; see plan_hist_item)
+    const long rows = level == 0 || tb.singles(level) ? tb.n : tb.n / 2;
+    const long by_rows = rows / kHistMinChunk + n_pairs, by_target = std::max(tb.target_hitems, tb.target_hitems / 4 + n_pairs) + 1;
+    dim3 grid(bins.n_blocks, (unsigned)std::max(1l, std::min({by_rows, by_target, (long)tb.max_hitems})), n_class);
     size_t lds = (size_t)tb.max_block_bins * sizeof(unsigned long long);
     if (lds > 64 * 1024) {
         // more than the default dynamic LDS window: opt in once per kernel instance and size
@@ -2508,23 +2369,6 @@ void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, flo
 
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class) {
     k_best_update<<<dim3(tb.nodes_served(level), 1, n_class), kBlock, 0, s>>>(tb, level, rt_eps, lambda);
-}
-
-void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, int n_class) {
-    if (level == tb.depth - 1) return;  // the last level's children never get row lists (see k_tree_end)
-    const dim3 one(1, 1, n_class), items(tb.max_pitems, 1, n_class);
-    const bool b16 = bins.bin_bytes == 2;
-    if (level == 0) {
-        if (b16) k_part_count_dense<true, uint16_t><<<items, kBlock, 0, s>>>(tb, bins, level);
-        else k_part_count_dense<true, uint8_t><<<items, kBlock, 0, s>>>(tb, bins, level);
-        k_part_scan_plan<<<one, kBlock, 0, s>>>(tb, level);
-        k_part_scatter<true><<<items, kBlock, 0, s>>>(tb, level);
-    } else {
-        if (b16) k_part_count_dense<false, uint16_t><<<items, kBlock, 0, s>>>(tb, bins, level);
-        else k_part_count_dense<false, uint8_t><<<items, kBlock, 0, s>>>(tb, bins, level);
-        k_part_scan_plan<<<one, kBlock, 0, s>>>(tb, level);
-        k_part_scatter<false><<<items, kBlock, 0, s>>>(tb, level);
-    }
 }
 
 void launch_partition_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class) {
