@@ -505,6 +505,9 @@ int sort_pairs(hipStream_t s, PairSorter &ps, long n, int key_bits);
 // (the bin itself stays in the key's high half and is what csc_bin receives).
 void launch_csc_keys(hipStream_t s, int n_rows, const int *row_ptr, const int *bin, const int *sort_key,
                      unsigned long long *keys, int *vals);
+void launch_bin_sort_keys(hipStream_t s, int n_bins, const int *cut_fid, const int *cut_row_ptr, const uint8_t *in_tables,
+                          int *sort_key);
+void launch_bin_meta(hipStream_t s, int n_bins, const int *cut_fid, const int *cut_row_ptr, unsigned *meta);
 void launch_csc_unpack(hipStream_t s, long nnz, const unsigned long long *keys, const int *vals, int *csc_bin,
                        int *csc_row);
 

@@ -17,6 +17,8 @@ enum RankMetric { RANK_METRIC_MAP = 3, RANK_METRIC_NDCG = 4 };
 constexpr int kRankCountSortMax = 2048;
 constexpr int kRankCountSortMean = 384;  // ... and only while sum(len^2) / rows stays below this
 
+constexpr int kRankSetupRows = 1 << 14;  // the groups of fewer rows are ordered by one thread (about 0.5 ms)
+
 // One run of equal labels inside a query group, in the group's label-descending order. The run owns the
 // positions [begin, end) of that order; [first_l, end) are the positions that draw a partner (the reference's
 // loop over a group skips the first position of a run that follows a processed run,

@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <string>
+#include <thread>
 
 #include "rank.h"
 
@@ -299,48 +300,72 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const std::vector<
     for (float v : y) labels_ok = labels_ok && v >= 0.f && v < 31.f;
     TGBM_CHECK(!ndcg || labels_ok, "rank:ndcg needs labels in 0..30");
 
+    // The groups are independent: the threads take contiguous ranges of about equally many rows (one thread: 6.8 ms for
+    // 200 k rows in groups of 120). Runs are numbered inside a range first, then moved behind the earlier ranges' runs.
     std::vector<int> static_row(n_), run_of(n_), run_of_row(n_), group_of(n_), hits(n_groups_, 0);
-    std::vector<RankRun> runs;
     std::vector<float> idcg(n_groups_, 0.f);
-    int ndcg_one = 0;  // groups whose NDCG is 1 by definition (IDCG == 0)
-    for (int g = 0; g < n_groups_; ++g) {
-        const int b = gptr[g], e = gptr[g + 1];
-        for (int i = b; i < e; ++i) {
-            static_row[i] = i;
-            group_of[i] = g;
-            if (y[i] != 0.f) ++hits[g];
-        }
-        std::stable_sort(static_row.begin() + b, static_row.begin() + e,
-                         [&](int a, int c) { return y[a] > y[c]; });
-        if (labels_ok) {  // NDCG::get_IDCG (rank_metric.cpp:106-123): float sum in descending label order
-            float z = 0.f;
-            for (int i = b; i < e; ++i)
-                z += (float)((1 << (int)y[static_row[i]]) - 1) / log2f((float)(i - b + 2));
-            idcg[g] = z;
-        }
-        if (idcg[g] == 0.f) ++ndcg_one;
-        if (hits[g] == 0) ++zero_hit_groups_;
-        bool skip_first = false;
-        for (int i = b; i < e;) {
-            int j = i + 1;
-            while (j < e && y[static_row[j]] == y[static_row[i]]) ++j;
-            RankRun r;
-            r.group_begin = b;
-            r.group_end = e;
-            r.end = j;
-            r.first_l = std::min(j, i + (skip_first ? 1 : 0));
-            r.group = g;
-            r.begin = i;
-            skip_first = r.first_l < j;  // a processed run makes the loop step over the next run's first position
-            for (int k = i; k < j; ++k) {
-                run_of[k] = (int)runs.size();
-                run_of_row[static_row[k]] = (int)runs.size();
-            }
-            runs.push_back(r);
-            i = j;
-        }
+    struct Range {
+        int g0 = 0, g1 = 0;
+        int ndcg_one = 0;  // groups whose NDCG is 1 by definition (IDCG == 0)
+        int zero_hit = 0;
+        std::vector<RankRun> runs;
+    };
+    const int n_ranges = n_ < kRankSetupRows ? 1 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+    std::vector<Range> ranges((size_t)n_ranges);
+    for (int t = 0; t < n_ranges; ++t) {
+        const long first_row = (long)n_ * (t + 1) / n_ranges;  // of the next range
+        ranges[t].g0 = t == 0 ? 0 : ranges[t - 1].g1;
+        ranges[t].g1 = t + 1 == n_ranges ? n_groups_
+                                         : (int)(std::lower_bound(gptr.begin(), gptr.end() - 1, (int)first_row) - gptr.begin());
     }
-    ndcg_one_groups_ = ndcg_one;
+    auto order_range = [&](Range &range) {
+        for (int g = range.g0; g < range.g1; ++g) {
+            const int b = gptr[g], e = gptr[g + 1];
+            for (int i = b; i < e; ++i) {
+                static_row[i] = i;
+                group_of[i] = g;
+                if (y[i] != 0.f) ++hits[g];
+            }
+            std::stable_sort(static_row.begin() + b, static_row.begin() + e, [&](int a, int c) { return y[a] > y[c]; });
+            if (labels_ok) {  // NDCG::get_IDCG (rank_metric.cpp:106-123): float sum in descending label order
+                float z = 0.f;
+                for (int i = b; i < e; ++i) z += (float)((1 << (int)y[static_row[i]]) - 1) / log2f((float)(i - b + 2));
+                idcg[g] = z;
+            }
+            if (idcg[g] == 0.f) ++range.ndcg_one;
+            if (hits[g] == 0) ++range.zero_hit;
+            bool skip_first = false;
+            for (int i = b; i < e;) {
+                int j = i + 1;
+                while (j < e && y[static_row[j]] == y[static_row[i]]) ++j;
+                RankRun r;
+                r.group_begin = b;
+                r.group_end = e;
+                r.end = j;
+                r.first_l = std::min(j, i + (skip_first ? 1 : 0));
+                r.group = g;
+                r.begin = i;
+                skip_first = r.first_l < j;  // a processed run makes the loop step over the next run's first position
+                for (int k = i; k < j; ++k) run_of[k] = (int)range.runs.size();
+                range.runs.push_back(r);
+                i = j;
+            }
+        }
+    };
+    auto number_range = [&](const Range &range, int before) {
+        for (int i = gptr[range.g0]; i < gptr[range.g1]; ++i) run_of_row[static_row[i]] = run_of[i] += before;
+    };
+    std::vector<std::thread> pool;
+    for (int t = 1; t < n_ranges; ++t) pool.emplace_back(order_range, std::ref(ranges[t]));
+    order_range(ranges[0]);
+    for (auto &th : pool) th.join();
+    std::vector<RankRun> runs;
+    for (const Range &range : ranges) {
+        number_range(range, (int)runs.size());
+        runs.insert(runs.end(), range.runs.begin(), range.runs.end());
+        ndcg_one_groups_ += range.ndcg_one;
+        zero_hit_groups_ += range.zero_hit;
+    }
     idcg_valid_ = labels_ok;
     n_runs_ = (int)runs.size();
     // ordering by counting costs sum(len^2) steps (measured: 50 us for a million rows in groups of 120, where the radix

@@ -180,7 +180,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         // Head of the histogram: the most frequent features whose bins fit the LDS slots. Worth it when
         // they carry a real share of the stored values (skewed, e.g. Zipf-distributed, feature usage).
         std::vector<int> feat_slot(F_, -1), head_bin;
-        {
+        if (!sparse_pass_) {  // (the level pass has no head)
             std::vector<int> order(F_);
             for (int f = 0; f < F_; ++f) order[f] = f;
             std::stable_sort(order.begin(), order.end(),
@@ -195,7 +195,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
                 head_nnz += cuts_.feature_nnz[f];
             }
             const char *he = std::getenv("TGBM_CSR_HEAD");  // "0" disables the head (tests of both kernels)
-            if (head_nnz * 10 < nnz_ || (he != nullptr && std::string(he) == "0") || sparse_pass_) head_bin.clear();
+            if (head_nnz * 10 < nnz_ || (he != nullptr && std::string(he) == "0")) head_bin.clear();
             log_info("sparse histogram head: %zu bins in LDS carry %.1f%% of the stored values", head_bin.size(),
                      nnz_ > 0 ? 100.0 * (double)head_nnz / (double)nnz_ : 0.0);
         }
@@ -230,13 +230,15 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             // addresses, and neighbouring lanes add to different table cells.
             int *d_sort_key = nullptr;
             if (sparse_pass_) {
-                std::vector<int> sort_key((size_t)n_bins_);
-                for (int f = 0; f < F_; ++f)
-                    for (int b = h_cut_row_ptr_[f]; b < h_cut_row_ptr_[f + 1]; ++b)
-                        sort_key[(size_t)b] = sparse_feature_in_tables(f) ? h_cut_row_ptr_[f] : b;
+                std::vector<uint8_t> in_tables((size_t)F_);
+                for (int f = 0; f < F_; ++f) in_tables[(size_t)f] = sparse_feature_in_tables(f) ? 1 : 0;
+                uint8_t *d_in_tables = nullptr;
+                device_alloc_to(d_in_tables, (size_t)F_);
+                upload(stream_, d_in_tables, in_tables.data(), in_tables.size());
                 device_alloc_to(d_sort_key, sizeof(int) * (size_t)n_bins_);
-                upload(stream_, d_sort_key, sort_key.data(), sort_key.size());
+                launch_bin_sort_keys(stream_, n_bins_, cuts_.cut_fid, cuts_.cut_row_ptr, d_in_tables, d_sort_key);
                 HIP_CHECK(hipStreamSynchronize(stream_));
+                device_free(d_in_tables);
             }
             launch_csc_keys(stream_, n_, d_row_ptr, d_bin, d_sort_key, ps.keys[0], ps.vals[0]);
             int bits = 1;
@@ -646,13 +648,8 @@ void Trainer::alloc_tree_buffers() {
     int *d_pack = dalloc<int>(pack_begin.size());
     upload(stream_, d_pack, pack_begin.data(), pack_begin.size());
     tb.pack_begin = d_pack;
-    std::vector<unsigned> bin_meta((size_t)n_bins_);
-    for (int f = 0; f < F_; ++f)
-        for (int b = h_cut_row_ptr_[f]; b < h_cut_row_ptr_[f + 1]; ++b)
-            bin_meta[(size_t)b] = ((unsigned)(h_cut_row_ptr_[f + 1] - 1 - b) & 0xffu) |
-                                  ((unsigned)(b - h_cut_row_ptr_[f]) & 0xffu) << 8 | (unsigned)f << 16;
-    unsigned *d_meta = dalloc<unsigned>(bin_meta.size());
-    upload(stream_, d_meta, bin_meta.data(), bin_meta.size());
+    unsigned *d_meta = dalloc<unsigned>((size_t)n_bins_);
+    launch_bin_meta(stream_, n_bins_, cuts_.cut_fid, cuts_.cut_row_ptr, d_meta);
     tb.bin_meta = d_meta;
     tb.cand = dalloc<SplitCand>(S * max_level_nodes * tb.n_packs);
 
@@ -832,17 +829,12 @@ bool Trainer::sparse_feature_in_tables(int f) {
         for (int q = 0; q < F_ && sparse_bin0_owner_ < 0; ++q)
             if (h_cut_row_ptr_[q + 1] > h_cut_row_ptr_[q]) sparse_bin0_owner_ = q;
         const char *se = std::getenv("TGBM_SPARSE_SORTED");  // "0": every feature through the tables (tests)
-        sparse_sorted_on_ = !(se != nullptr && std::string(se) == "0");
-        // the sorted pass keeps 40 bytes per stored value of its features for every class tree built together;
-        // it is left out when that would take more than a quarter of the free memory
-        size_t free_b = 0, total_b = 0;
-        device_mem_info(&free_b, &total_b);
-        if ((size_t)nnz_ * 40 * (size_t)std::max(1, param_.tree_per_rounds) > free_b / 4) sparse_sorted_on_ = false;
+        sparse_rare_on_ = !(se != nullptr && std::string(se) == "0");
     }
-    return !sparse_sorted_on_ || cuts_.feature_nnz[f] > kSortedTile || f == sparse_bin0_owner_;
+    return !sparse_rare_on_ || cuts_.feature_nnz[f] > kRareTile || f == sparse_bin0_owner_;
 }
 
-// Work lists of the sparse level pass. Features with at most kSortedTile stored values go to the sorted pass (tasks:
+// Work lists of the sparse level pass. Features with at most kRareTile stored values go to k_sparse_rare_filter (tasks:
 // runs of such features whose values fit one tile); the others to table tasks: runs of consecutive such features
 // with about kSparseTaskValues values, a feature with more values than that cut into chunks (tasks of their own)
 // whose tables k_sparse_big adds up. The feature that owns global bin 0 is always a table feature (its table is
