@@ -1,0 +1,68 @@
+"""Rare features of the sparse layout: the filtered search (k_sparse_rare) against the complete (bin, node) tables
+(TGBM_SPARSE_SORTED=0), byte for byte, at the edges of its tiles."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def T():
+    import thundergbm_amd
+    thundergbm_amd.load()
+    return thundergbm_amd
+
+
+def _by_feature(counts, n, seed):
+    """CSR of features with the given numbers of stored values, in random rows."""
+    rng = np.random.default_rng(seed)
+    rows = np.concatenate([rng.choice(n, k, replace=False) for k in counts])
+    cols = np.repeat(np.arange(len(counts), dtype=np.int32), counts)
+    order = np.lexsort((cols, rows))
+    rp = np.zeros(n + 1, np.int64)
+    np.cumsum(np.bincount(rows, minlength=n), out=rp[1:])
+    val = np.exp(rng.standard_normal(len(rows))).astype(np.float32)
+    z = np.zeros(n)
+    w = rng.standard_normal(len(counts)) * (rng.random(len(counts)) < 0.3)
+    np.add.at(z, rows[order], w[cols[order]] * val)
+    return val, rp.astype(np.int32), cols[order], z + 0.3 * rng.standard_normal(n)
+
+
+SHAPES = {
+    "single_values": ([1] * 5000 + [2] * 3000, 9000),              # more features than a tile takes
+    "tile_edges": ([4096, 4097, 4095, 1, 4096, 2048, 2048, 1, 4097], 5000),
+    "two_tiles_a_group": ([20000] * 3 + [4000, 3000] + [190] * 11500, 60000),
+    "everything_rare": ([300] * 60, 2000),                         # the tables publish next to nothing
+}
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("objective,kw", [
+    ("reg:linear", {}), ("binary:logistic", {"min_child_weight": 5.0}), ("multi:softmax", {"num_class": 3}),
+    ("reg:linear", {"lambda_": 0.0, "min_child_weight": 0.0, "sampled": True})])
+def test_rare_features_equal_tables(T, shape, objective, kw):
+    counts, n = SHAPES[shape]
+    val, rp, col, z = _by_feature(counts, n, 5)
+    kw = dict(kw)
+    sampled = kw.pop("sampled", False)
+    y = (z if objective == "reg:linear" else np.digitize(z, [-0.5, 0.5][: 2 if "multi" in objective else 1])).astype(np.float32)
+    runs = []
+    os.environ["TGBM_LAYOUT"] = "sparse"
+    try:
+        for rare in ("1", "0"):
+            os.environ["TGBM_SPARSE_SORTED"] = rare
+            ctypes.CDLL(None).srand(7)
+            s = T.Session(val, rp, col, y, objective=objective, depth=7, n_trees=3, max_num_bin=63, learning_rate=0.5, **kw)
+            assert s.info("sparse_pass") == 1
+            if sampled:
+                s.set_option("bagging", 1)
+                s.set_option("column_sampling_rate", 0.5)
+            s.boost(3)
+            runs.append((s.model().tobytes(), s.y_pred().tobytes()))
+            s.close()
+    finally:
+        del os.environ["TGBM_SPARSE_SORTED"], os.environ["TGBM_LAYOUT"]
+    assert runs[0] == runs[1]

@@ -174,23 +174,22 @@ struct SparseTask {
     int cand_slot;       // candidate slot the task fills, -1: a chunk (its feature's slot is filled by k_sparse_big)
     int partial_slot;    // chunk: where its table goes in SparsePass::partial, else -1
 };
-// Features with at most kSortedTile stored values are not searched through tables: their values are kept sorted by
-// (feature, node, bin) from level to level - a stable two-way partition of every (feature, node) run when the node
-// splits - and the split search is a segmented scan of that order, so the work follows the stored values and not
-// the (bin, node) cells. A task is a run of whole features whose values fit one workgroup tile.
-constexpr int kSortedBlock = 512;                        // threads of a sorted-pass workgroup
-constexpr int kSortedPerThread = 8;                      // consecutive values a thread owns
-constexpr int kSortedTile = kSortedBlock * kSortedPerThread;  // values per task at most
-constexpr int kSortedLevels = 12;                        // levels the pass serves (depth <= 11, one spare)
-struct SortedTask {
-    int v_begin;     // first position of the task's tile in the sorted-pass arrays
-    int count;       // stored values of its features (= live values at the root)
-    int meta_begin;  // first entry of its features in SparsePass::sorted_meta / sorted_fid
+// Features with at most kRareTile stored values are not searched through tables: k_sparse_rare_filter looks for the (feature, node)
+// runs of their values that could win at all and searches only those. A task is a run of whole features whose values
+// fit one tile; a workgroup of the search takes every n_rare_groups-th task.
+constexpr int kRareBlock = 512;
+constexpr int kRareTile = 4096;       // values per task at most
+constexpr int kRareFeatures = 2048;   // features per task at most
+constexpr int kRareGroupTiles = 16;   // tasks of a search workgroup at most
+constexpr int kRareGroups = 512;      // search workgroups that are resident together (two per CU)
+struct RareTask {
+    int v_begin;     // first position of the task's values in SparsePass::rare_row / rare_key
+    int count;       // stored values of its features
+    int meta_begin;  // first entry of its features in SparsePass::rare_meta / rare_fid
     int n_feat;      // features of the task
-    int cand_slot;   // candidate slot the task fills
 };
-// Key of a stored value in the sorted pass: feature (index inside its task) << 20 | node of the level << 8 | local bin
-constexpr int kSortedNodeShift = 8, kSortedFeatShift = 20;
+// key of a stored value: feature (index inside its task) << 20 | sixty-fourth of the feature's values << 8 | local bin
+constexpr int kRareFeatShift = 20;
 struct SparseBig {
     int feature;
     int slot_begin, slot_end;  // partial slots of its chunks
@@ -201,20 +200,17 @@ struct SparsePass {
     int n_tasks = 0;
     const SparseBig *big = nullptr;
     int n_big = 0;
-    // sorted pass (features of at most kSortedTile values)
-    const SortedTask *sorted_tasks = nullptr;
-    int n_sorted_tasks = 0;
-    const int2 *sorted_meta = nullptr;    // per feature of a task: (first global bin, number of bins)
-    const int *sorted_fid = nullptr;      // its feature id
-    const int *sorted_row0 = nullptr;     // [n_sorted] rows and keys in the static order (feature, bin, row): the
-    const unsigned *sorted_key0 = nullptr;  // root level's input
-    const unsigned short *sorted_start0 = nullptr;  // [n_sorted] tile position where the value's feature starts
-    long n_sorted = 0;
-    // per set: the order of the previous and of the current level, ping-pong by level parity
-    int *sorted_row[2] = {nullptr, nullptr};
-    unsigned *sorted_key[2] = {nullptr, nullptr};
-    GHPair *sorted_gh[2] = {nullptr, nullptr};
-    int *sorted_live = nullptr;           // [n_sets][kSortedLevels][n_sorted_tasks] live values of a tile after a level
+    // rare features (at most kRareTile values)
+    const RareTask *rare_tasks = nullptr;
+    int n_rare_tasks = 0, n_rare_groups = 0;
+    int rare_slot = 0;                  // candidate slot of the first group
+    const int2 *rare_meta = nullptr;    // per feature of a task: (first global bin, number of bins)
+    const int *rare_fid = nullptr;      // its feature id
+    const int *rare_row = nullptr;      // [values of the rare features] rows and keys in the order (feature, bin, row)
+    const unsigned *rare_key = nullptr;
+    long n_rare = 0;
+    unsigned long long *rare_item = nullptr;  // [n_sets][n_rare] values of a level that may matter, tile by tile
+    int *rare_passed = nullptr;               // [n_sets][n_rare_tasks] how many of a tile
     const int *feat_val_begin = nullptr;  // [F + 1] first position of every feature in the bin-major copy
     // [n_sets][nnz] the gradient pair of every stored value's row, in the order of the bin-major copy, refreshed once
     // per tree: the level passes then stream it instead of fetching a cache line per value (nullptr: no room, gather)
@@ -224,11 +220,6 @@ struct SparsePass {
     size_t partial_stride = 0;            // cells per slot: most bins of a big feature x kSparseMaxLevelNodes at most
     int n_partial_slots = 0;
     int n_cand_slots = 0;
-
-    // the sorted pass's order of a level (selected without indexing an array member dynamically)
-    __host__ __device__ int *srow(int level) const { return (level & 1) ? sorted_row[1] : sorted_row[0]; }
-    __host__ __device__ unsigned *skey(int level) const { return (level & 1) ? sorted_key[1] : sorted_key[0]; }
-    __host__ __device__ GHPair *sgh(int level) const { return (level & 1) ? sorted_gh[1] : sorted_gh[0]; }
 };
 
 struct TreeBuffers {
@@ -249,11 +240,9 @@ struct TreeBuffers {
     // sparse level pass only (else nullptr): node every row has reached (heap id) and rows per node
     unsigned short *nid16 = nullptr;  // [n + 2]
     int *node_rows = nullptr;         // [n_nodes]
-    // what the last row -> node update did with every row: bit 0 = the row moved to a child (its node split), bit 1 =
-    // to the right child. A byte per row instead of the 16-bit node: the sorted pass, which knows a value's previous
-    // node from its key, looks its rows up here with one-byte loads, eight of them in flight per thread (the whole
-    // map stays in every L2).
-    uint8_t *row_move = nullptr;      // [n rounded up to 64]
+    // sparse level pass: the row's node of the level and what bounds its part in a candidate, see k_sparse_rare_filter
+    // (nullptr: no rare features)
+    unsigned *row_word = nullptr;     // [n]
     // sparse level pass: best candidate key of every node of the level over all tasks, and the candidate slot of
     // the task that searches a feature (k_best_update reads the winner's record from that slot)
     unsigned long long *best_key = nullptr;  // [max_level_nodes]
@@ -348,7 +337,7 @@ struct TreeBuffers {
         if (nid16 != nullptr) {
             t.nid16 += K * (((size_t)n + 2) / 2 * 2);
             t.node_rows += K * n_nodes;
-            t.row_move += K * (((size_t)n + 63) / 64 * 64);
+            if (row_word != nullptr) t.row_word += K * n;
             t.best_key += K * max_level_nodes;
         }
         t.leaf_value += K * n_nodes;
@@ -409,18 +398,18 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
                             float rt_eps, float lambda, int n_class = 1);
 // Sparse level pass (tb.nid16 set): split search of a level (candidates into tb.cand, one slot per task / big
 // feature; launch_best_update follows) and the row -> node update. dump_hist: also store the (node, bin) tables
-// into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q). last_level: the tree's deepest level (the
-// sorted pass then keeps its new order to itself: no level reads it).
+// into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q).
 void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
-                         const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class = 1,
-                         bool last_level = false);
+                         const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class = 1);
 void launch_sparse_partition(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class = 1);
 // Byte columns of the frequent features (CsrBins::colbin, pre-filled with kMissingBin) from the bin-major copy.
 void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *csc_row, const int *cut_fid,
                         const int *cut_row_ptr, const int *col_of_feature, uint8_t *colbin, size_t col_stride);
-// Fills the static order of the sorted pass (row0 / key0, sp.n_sorted entries) from the bin-major copy.
-void launch_sorted_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row0,
-                         unsigned *key0, unsigned short *start0);
+// Fills row / key (SparsePass::rare_row / rare_key, sp.n_rare entries) from the bin-major copy.
+void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row,
+                       unsigned *key);
+// The rows' words of a tree (TreeBuffers::row_word).
+void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class);
 // csc_gh[e] = gh[csc_row[e]] for the values of the table tasks, n_class gradient planes (once per tree)
 void launch_sparse_gh_refresh(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
                               const GHPair *gh, int n_class = 1);

@@ -284,9 +284,12 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int e = min(e0 + u * kSpBlock, v1 - 1);
-                    gb[u] = bins.csc_bin[e];
-                    row[u] = bins.csc_row[e];
-                    if (csc_gh != nullptr) s[u] = csc_gh[e];
+                    gb[u] = __builtin_nontemporal_load(bins.csc_bin + e);
+                    row[u] = __builtin_nontemporal_load(bins.csc_row + e);
+                    if (csc_gh != nullptr) {
+                        const unsigned long long w = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(csc_gh + e));
+                        s[u] = GHPair{__uint_as_float((unsigned)w), __uint_as_float((unsigned)(w >> 32))};
+                    }
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) x[u] = (int)nid16[row[u]] - off - n0;
@@ -362,135 +365,176 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_big(TreeBuffers tb_all, Spa
     sp_publish(tb, sh, level);
 }
 
-// ------------------------------------------------------------------------------------ sorted pass
-// Features with at most kSortedTile stored values. A task (one workgroup) owns a run of whole features and a tile of
-// the sorted-pass arrays; the tile holds the features' values in the order (feature, node of the level, bin), rows
-// in arrival order inside a bin. A level reads the previous level's order, looks up the node every value's row has
-// moved to, and partitions every (feature, node) run stably into the values of the left and of the right child;
-// the runs of nodes that did not split drop out (all rows of a node split or none, so a run is all live or all
-// dead). The new order goes back to HBM for the next level and is scanned right away: a forward and a backward
-// segmented sum per (feature, node) run give every position the run's sum up to it and after it, hence the left
-// sum and the feature's total in the node (missing = node sum - total). Candidates exist only where the left sum
-// changes: the feature's first bin (left side empty) and the bin after every bin that holds a value - the bins in
-// between repeat the previous candidate's gain and lose the tie on the smaller index - so the result is what the
-// scan of a complete (bin, node) table gives. The root level reads the static order and fetches the gradient pairs.
-constexpr int kSoV = kSortedPerThread;
-constexpr int kSoWaves = kSortedBlock / 64;
-constexpr unsigned kSoNodeMask = 0xfffu << kSortedNodeShift;
-// LDS position of tile position i: one element of padding after every 32, so that neither the lanes of a wavefront
-// that each own eight consecutive positions nor lanes at consecutive positions collide in a bank
-constexpr int kSoLds = kSortedTile + kSortedTile / 32;
-__device__ __forceinline__ int so_phys(int i) { return i + (i >> 5); }
+// ------------------------------------------------------------------------------------ rare features
+// Features with at most kRareTile stored values: nearly none of their candidates can win a node (1 M rows x 100 k
+// features: fewer than 20 of 23 M a level pass a reciprocal estimate of their gain), so the pass first finds the few
+// (feature, node) runs that could and searches only those.
+//
+// The filter. A candidate of a run splits off a subset A of the run's values - a prefix in the order of their bins when
+// the missing rows go right, a suffix when they go left. One word per row holds its node and g and h in ten-bit units of
+// the tree's largest. The values of a feature are cut into groups of neighbours in bin order (as many as the cells
+// allow: 64 at the root, one where the level has more (feature, node) runs than that), and every (feature, node, group)
+// has a cell in LDS that adds up its positive and its negative g, its h and its values. A prefix that ends inside a
+// group is the sum of the groups before it and some of that group's values, which bounds A.g from both sides and A.h
+// from both sides, hence the gain. A run all of whose bounds stay below the best gain its node has seen so far - the table
+// tasks of the level have published theirs - loses whatever its order is. The margins cover the float roundings of the
+// missing-value arithmetic, a few ulps of the node's sums. (Bounds without groups or signs leave most runs of the later
+// trees, whose best gains are small.)
+//
+// What is left is collected over the tiles of a group (k_sparse_rare_search), sorted by (feature, node, bin) and searched by one segmented scan:
+// candidates exist only where the left sum changes - the feature's first bin (left side empty) and the bin after every bin
+// that holds a value; the bins in between repeat the previous candidate's gain and lose the tie on the smaller index - so
+// the result is what the scan of a complete (bin, node) table gives.
+//
+// Bound by the row -> word look-ups of every stored value (4 bytes each, the words of 1 M rows fill an L2). The tiles of a
+// group are strided over the features, whose frequencies often fall with their index.
+constexpr int kRareV = kRareTile / kRareBlock;
+constexpr int kRareWaves = kRareBlock / 64;
+constexpr int kRareCells = 3072;  // (with them two workgroups fit a CU)
+constexpr int kRareMaxGroups = 64;
+// LDS position of position i: one element of padding after every 32, so that the lanes of a wavefront that each own
+// eight consecutive positions do not meet in a bank
+constexpr int kRareLds = kRareTile + kRareTile / 32;
+__device__ __forceinline__ int rare_phys(int i) { return i + (i >> 5); }
 
-struct SoCount {
-    int seg;    // since the run began: values << 16 | values that go left
-    int plain;  // over the whole tile: dead values
+// row word: node of the level (11 bits, all ones: the row has come to rest above), sign of g, |g| (10 bits, rounded up), h
+// (10 bits, rounded down)
+constexpr unsigned kRareNodeMask = 0x7ffu;
+constexpr float kRareSteps = 1022.f;
+__device__ __forceinline__ unsigned rare_row_word(unsigned node, GHPair s, const QuantCtl &q) {
+    // (of the integers that the sums are made of)
+    const float g = fabsf((float)round_to_ll(s.g * q.scale_g)), h = (float)round_to_ll(s.h * q.scale_h);
+    const unsigned cg = g > 0.f ? min(1023u, (unsigned)ceilf(g * (kRareSteps / q.gq_max))) : 0u;
+    const unsigned ch = h > 0.f ? min(1023u, (unsigned)(h * (kRareSteps / q.hq_max))) : 0u;
+    return node | (s.g < 0.f ? 1u << 11 : 0u) | cg << 12 | ch << 22;
+}
+struct RareCell {
+    unsigned long long g;  // sums of the positive g (22 bits) and of the negative g (22), values (13)
+    unsigned h;            // sum of h
+    __device__ int plus() const { return (int)((unsigned)g & 0x3fffffu); }
+    __device__ int minus() const { return (int)((unsigned)(g >> 22) & 0x3fffffu); }
+    __device__ int values() const { return (int)(g >> 44); }
 };
-struct SoSum {
+__device__ __forceinline__ RareCell operator+(RareCell a, RareCell b) { return {a.g + b.g, a.h + b.h}; }
+__device__ __forceinline__ RareCell operator-(RareCell a, RareCell b) { return {a.g - b.g, a.h - b.h}; }
+__device__ __forceinline__ unsigned long long rare_addend(unsigned word) {
+    const unsigned long long g = (word >> 12) & 0x3ffu;
+    return 1ull << 44 | ((word >> 11 & 1u) ? g << 22 : g);
+}
+static_assert(kRareTile * 1023 < 1 << 22 && kRareTile < 1 << 13, "fields of a cell");
+
+struct RareBound {
+    float g, h, mcw, lambda;  // one step of g and of h
+};
+
+// No candidate that splits off all of `whole` and some of the values of `part` reaches the gain `floor`.
+__device__ __forceinline__ bool rare_hopeless(RareCell whole, RareCell part, GHPair S, float P, float floor, RareBound u) {
+    constexpr float up = 1.f + 0x1p-12f, down = 1.f - 0x1p-12f;  // (roundings of the codes)
+    const float base = (float)(whole.plus() - whole.minus()), slack = 1.01f * (float)whole.values();
+    const float hi = (base + slack + (float)part.plus()) * u.g * up, lo = (base - slack - (float)part.minus()) * u.g * up;
+    const float eg = (fabsf(S.g) + fabsf(hi) + fabsf(lo)) * 0x1p-21f, eh = S.h * 0x1p-21f;
+    const float h_min = (float)whole.h * u.h * down - eh;
+    const float h_max = (float)((int)(whole.h + part.h) + whole.values() + part.values()) * u.h * up + eh;
+    if (h_max < u.mcw || S.h - h_min + eh < u.mcw) return true;  // one of the sides weighs too little
+    const float a = fmaxf(fabsf(hi), fabsf(lo)) + eg, b = fmaxf(fabsf(S.g - hi), fabsf(S.g - lo)) + eg;
+    const float t = a * a * __builtin_amdgcn_rcpf(fmaxf(u.mcw, h_min) + u.lambda) +
+                    b * b * __builtin_amdgcn_rcpf(fmaxf(u.mcw, S.h - h_max) + u.lambda);
+    return (t - P) + (t + fabsf(P)) * 0x1p-18f < floor;
+}
+
+// The runs of a tile with at least two groups per (feature, node): a thread takes four cells that follow each other, a run
+// is a part of a thread's cells or the cells of up to sixteen neighbouring lanes. open(): the run may hold a winner.
+template <typename MayWin, typename Open>
+__device__ __forceinline__ void rare_check_cells(const unsigned long long *cell_g, const unsigned *cell_h, int cells,
+                                                 int log_groups, const MayWin &may_win, const Open &open) {
+    constexpr int V = 4;
+    const int groups = 1 << log_groups, lanes = groups / V;  // lanes of a run (0: several runs per thread)
+#pragma unroll 1
+    for (int i0 = (int)threadIdx.x * V; __any(i0 < cells); i0 += kRareBlock * V) {
+        RareCell upto[V], carry{0, 0}, run{0, 0};
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const RareCell c = i0 + j < cells ? RareCell{cell_g[i0 + j], cell_h[i0 + j]} : RareCell{0, 0};
+            run = (j & (groups - 1)) == 0 ? c : run + c;
+            upto[j] = run;
+        }
+        RareCell total = run;
+        if (lanes > 1) {
+            for (int d = 1; d < lanes; d <<= 1) {
+                const RareCell o{(unsigned long long)shfl_up_ll((long long)total.g, d), (unsigned)__shfl_up((int)total.h, d)};
+                if ((lane_id() & (lanes - 1)) >= d) total = total + o;
+            }
+            carry = total - run;
+            const int last = lane_id() | (lanes - 1);
+            total.g = (unsigned long long)(unsigned)__shfl((int)(unsigned)total.g, last) |
+                      (unsigned long long)(unsigned)__shfl((int)(total.g >> 32), last) << 32;
+            total.h = (unsigned)__shfl((int)total.h, last);
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            if (groups == 2) total = upto[j | 1];
+            const RareCell before = (j & (groups - 1)) == 0 ? carry : carry + upto[j > 0 ? j - 1 : 0];
+            const RareCell own = carry + upto[j] - before;
+            if (own.g != 0 && may_win((i0 + j) >> log_groups, before, own, total - before - own)) open((i0 + j) >> log_groups);
+        }
+    }
+}
+
+struct RareSum {
     long long g, h;
+    int n;
 };
-__device__ __forceinline__ void so_zero_seg(SoCount &a) { a.seg = 0; }
-__device__ __forceinline__ void so_add_seg(SoCount &a, const SoCount &b) { a.seg += b.seg; }
-__device__ __forceinline__ void so_add_plain(SoCount &a, const SoCount &b) { a.plain += b.plain; }
-__device__ __forceinline__ void so_zero_seg(SoSum &a) { a.g = a.h = 0; }
-__device__ __forceinline__ void so_add_seg(SoSum &a, const SoSum &b) {
-    a.g += b.g;
-    a.h += b.h;
-}
-__device__ __forceinline__ void so_add_plain(SoSum &, const SoSum &) {}
+__device__ __forceinline__ RareSum operator+(RareSum a, RareSum b) { return {a.g + b.g, a.h + b.h, a.n + b.n}; }
 
-template <bool FWD>
-__device__ __forceinline__ int so_shfl(int v, int d) {
-    return FWD ? __shfl_up(v, d) : __shfl_down(v, d);
-}
-template <bool FWD>
-__device__ __forceinline__ long long so_shfl(long long v, int d) {
-    const int lo = so_shfl<FWD>((int)(unsigned)(unsigned long long)v, d);
-    const int hi = so_shfl<FWD>((int)((unsigned long long)v >> 32), d);
-    return (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-template <bool FWD>
-__device__ __forceinline__ SoCount so_shfl(SoCount v, int d) {
-    return SoCount{so_shfl<FWD>(v.seg, d), so_shfl<FWD>(v.plain, d)};
-}
-template <bool FWD>
-__device__ __forceinline__ SoSum so_shfl(SoSum v, int d) {
-    return SoSum{so_shfl<FWD>(v.g, d), so_shfl<FWD>(v.h, d)};
-}
-
-// Inclusive segmented scan over the tile (thread t owns positions t * kSoV ..). FWD: v[j] becomes the sum from the
-// start of its run (brk = a run starts here) up to j; !FWD: from j to the end of its run (brk = a run ends here).
-// The `plain` part of T ignores the breaks. Two barriers; s_agg / s_flag are free again afterwards.
-template <typename T, bool FWD>
-__device__ void so_block_scan(T (&v)[kSoV], const bool (&brk)[kSoV], T *s_agg, int *s_flag) {
+// Inclusive segmented scan (thread t owns positions t * kRareV ..): v[j] becomes the sum from the start of its run
+// (head = a run starts here) up to j. Two barriers.
+__device__ void rare_block_scan(RareSum (&v)[kRareV], const bool (&head)[kRareV], RareSum *s_agg, int *s_flag) {
     const int lane = lane_id(), w = wave_id();
-    T run{};
+    RareSum run{0, 0, 0};
     bool any = false;
 #pragma unroll
-    for (int jj = 0; jj < kSoV; ++jj) {
-        const int j = FWD ? jj : kSoV - 1 - jj;
-        if (brk[j]) {
-            so_zero_seg(run);
-            any = true;
-        }
-        so_add_seg(run, v[j]);
-        so_add_plain(run, v[j]);
+    for (int j = 0; j < kRareV; ++j) {
+        run = head[j] ? v[j] : run + v[j];
+        any = any || head[j];
         v[j] = run;
     }
-    T agg = run;
+    RareSum agg = run;
     int flag = any ? 1 : 0;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const T o = so_shfl<FWD>(agg, d);
-        const int of = so_shfl<FWD>(flag, d);
-        const bool has = FWD ? lane >= d : lane + d < 64;
-        if (has) {
-            if (!flag) so_add_seg(agg, o);
-            so_add_plain(agg, o);
+        const RareSum o{shfl_up_ll(agg.g, d), shfl_up_ll(agg.h, d), __shfl_up(agg.n, d)};
+        const int of = __shfl_up(flag, d);
+        if (lane >= d) {
+            if (!flag) agg = o + agg;
             flag |= of;
         }
     }
-    T carry = so_shfl<FWD>(agg, 1);
-    int cflag = so_shfl<FWD>(flag, 1);
-    if (FWD ? lane == 0 : lane == 63) {
-        carry = T{};
+    RareSum carry{shfl_up_ll(agg.g, 1), shfl_up_ll(agg.h, 1), __shfl_up(agg.n, 1)};
+    int cflag = __shfl_up(flag, 1);
+    if (lane == 0) {
+        carry = RareSum{0, 0, 0};
         cflag = 0;
     }
-    if (FWD ? lane == 63 : lane == 0) {
+    if (lane == 63) {
         s_agg[w] = agg;
         s_flag[w] = flag;
     }
     __syncthreads();
-    T wc{};
-    if (FWD) {
-        for (int u = 0; u < w; ++u) {
-            if (s_flag[u]) so_zero_seg(wc);
-            so_add_seg(wc, s_agg[u]);
-            so_add_plain(wc, s_agg[u]);
-        }
-    } else {
-        for (int u = kSoWaves - 1; u > w; --u) {
-            if (s_flag[u]) so_zero_seg(wc);
-            so_add_seg(wc, s_agg[u]);
-            so_add_plain(wc, s_agg[u]);
-        }
-    }
-    if (!cflag) so_add_seg(carry, wc);
-    so_add_plain(carry, wc);
+    RareSum before{0, 0, 0};
+    for (int u = 0; u < w; ++u) before = s_flag[u] ? s_agg[u] : before + s_agg[u];
+    if (!cflag) carry = before + carry;
     bool open = true;
 #pragma unroll
-    for (int jj = 0; jj < kSoV; ++jj) {
-        const int j = FWD ? jj : kSoV - 1 - jj;
-        if (brk[j]) open = false;
-        if (open) so_add_seg(v[j], carry);
-        so_add_plain(v[j], carry);
+    for (int j = 0; j < kRareV; ++j) {
+        open = open && !head[j];
+        if (open) v[j] = carry + v[j];
     }
     __syncthreads();
 }
 
 // split_gain with the node's own term (f.g^2 / (f.h + lambda), the same for every candidate of the node) taken from
 // a table: the same operations in the same order, hence the same bits
-__device__ __forceinline__ float so_gain(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
+__device__ __forceinline__ float rare_gain(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
 #pragma clang fp contract(off)
     const GHPair r{f.g - l.g, f.h - l.h};
     float gain = 0.f;
@@ -498,334 +542,184 @@ __device__ __forceinline__ float so_gain(GHPair f, float fterm, GHPair l, float 
     return fmaxf(0.f, gain);
 }
 
-// Upper estimate of so_gain from the hardware reciprocal (1 ulp) instead of divisions; -1: the weight gate closes
-__device__ __forceinline__ float so_gain_estimate(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
+// Upper estimate of rare_gain from the hardware reciprocal (1 ulp) instead of divisions; -1: the weight gate closes
+__device__ __forceinline__ float rare_gain_estimate(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
     const GHPair r{f.g - l.g, f.h - l.h};
     if (!(l.h >= mcw && r.h >= mcw)) return -1.f;
     const float a = l.g * l.g * __builtin_amdgcn_rcpf(l.h + lambda), b = r.g * r.g * __builtin_amdgcn_rcpf(r.h + lambda);
-    return (a + b - fterm) + (a + b + fabsf(fterm)) * 3.8146973e-6f;  // + 2^-18 of the terms: far above the roundings
+    return (a + b - fterm) + (a + b + fabsf(fterm)) * 0x1p-18f;  // + 2^-18 of the terms: far above the roundings
 }
 
 // Signed score of a candidate (> 0: missing values go left), hist_tree_builder_single.cu:300-323. `floor`: the
 // largest |score| the candidate's node has seen so far; a candidate whose estimate stays below it cannot become the
 // node's best and is not evaluated (0 = no candidate).
-__device__ __forceinline__ float so_score(GHPair S, float fterm, GHPair m, GHPair l, bool ignored, float mcw,
-                                          float lambda, float floor) {
+__device__ __forceinline__ float rare_score(GHPair S, float fterm, GHPair m, GHPair l, float mcw, float lambda, float floor) {
 #pragma clang fp contract(off)
     const GHPair l2{l.g + m.g, l.h + m.h};
-    const float er = so_gain_estimate(S, fterm, l, mcw, lambda), el = so_gain_estimate(S, fterm, l2, mcw, lambda);
-    if (fmaxf(er, el) < floor || ignored) return 0.f;  // (column sampling: hist_tree_builder_single.cu:304 / :663)
-    const float gr = so_gain(S, fterm, l, mcw, lambda);
-    const float gl = so_gain(S, fterm, l2, mcw, lambda);
+    const float er = rare_gain_estimate(S, fterm, l, mcw, lambda), el = rare_gain_estimate(S, fterm, l2, mcw, lambda);
+    if (fmaxf(er, el) < floor) return 0.f;
+    const float gr = rare_gain(S, fterm, l, mcw, lambda);
+    const float gl = rare_gain(S, fterm, l2, mcw, lambda);
     return (gl > gr) ? gl : -gr;
 }
 
-template <bool LEVEL0>
-__global__ __launch_bounds__(kSortedBlock) void k_sparse_sorted(TreeBuffers tb_all, SparsePass sp,
-                                                               const GHPair *__restrict__ gh, int level, float mcw,
-                                                               float lambda, int dump_hist, int last_level) {
-#pragma clang fp contract(off)
-    extern __shared__ unsigned char so_dyn[];  // per node of the level: best key (8 bytes), sums (8), own gain term (4)
-    __shared__ int s_row[kSoLds];
-    __shared__ unsigned s_key[kSoLds];
-    __shared__ GHPair s_gh[kSoLds];
-    __shared__ unsigned short s_aux[kSoLds];  // first the left counts of the old runs, then the start of every value's run
-    __shared__ SoSum s_agg_sum[kSoWaves];
-    __shared__ SoCount s_agg_cnt[kSoWaves];
-    __shared__ int s_flag[kSoWaves];
-    __shared__ int s_dead;
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    const SortedTask task = sp.sorted_tasks[blockIdx.x];
-    const int nl = 1 << level, off = nl - 1;
-    unsigned long long *s_best = reinterpret_cast<unsigned long long *>(so_dyn);
-    GHPair *s_S = reinterpret_cast<GHPair *>(s_best + nl);
-    float *s_P = reinterpret_cast<float *>(s_S + nl);
-    const size_t base = (size_t)blockIdx.z * (size_t)sp.n_sorted + (size_t)task.v_begin;
-    int *live = sp.sorted_live + ((size_t)blockIdx.z * kSortedLevels + level) * sp.n_sorted_tasks;
-    const int M = LEVEL0 ? task.count : live[(long)blockIdx.x - sp.n_sorted_tasks];
-    gh += (size_t)blockIdx.z * tb.n;
-    const int *__restrict__ in_row = LEVEL0 ? sp.sorted_row0 + task.v_begin : sp.srow(level - 1) + base;
-    const unsigned *__restrict__ in_key = LEVEL0 ? sp.sorted_key0 + task.v_begin : sp.skey(level - 1) + base;
-    const GHPair *__restrict__ in_gh = LEVEL0 ? nullptr : sp.sgh(level - 1) + base;
-    int *__restrict__ out_row = sp.srow(level) + base;
-    unsigned *__restrict__ out_key = sp.skey(level) + base;
-    GHPair *__restrict__ out_gh = sp.sgh(level) + base;
-    if (M == 0) {
-        if (threadIdx.x == 0) live[blockIdx.x] = 0;
-        return;
-    }
-    for (int x = threadIdx.x; x < nl; x += kSortedBlock) {
-        const GHPair S = tb.nodes[off + x].sum_gh_pair;
-        // what the other tasks have published so far: a candidate below it need not be looked at
-        s_best[x] = __hip_atomic_load(&tb.best_key[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_S[x] = S;
-        s_P[x] = (S.g * S.g) / (S.h + lambda);
-    }
-    // ---- the previous order into LDS with coalesced loads (position q = k * block + thread), every load of the
-    // thread in flight before the first one is used; the root level also fetches the gradient pair of every value's
-    // row here and takes the run starts (= feature starts) from the static arrays
-    {
-        int lrow[kSoV];
-        unsigned lkey[kSoV];
-        GHPair lgh[kSoV];
-        unsigned short lst[kSoV];
-#pragma unroll
-        for (int k = 0; k < kSoV; ++k) {
-            const int q = k * kSortedBlock + threadIdx.x;
-            lrow[k] = q < M ? in_row[q] : 0;
-            lkey[k] = q < M ? in_key[q] : 0u;
-            if (!LEVEL0) lgh[k] = q < M ? in_gh[q] : GHPair{0, 0};
-            if (LEVEL0) lst[k] = q < M ? sp.sorted_start0[task.v_begin + q] : (unsigned short)0;
-        }
-        if (LEVEL0) {
-#pragma unroll
-            for (int k = 0; k < kSoV; ++k) lgh[k] = gh[lrow[k]];  // (row 0 for the positions past the end)
-        }
-#pragma unroll
-        for (int k = 0; k < kSoV; ++k) {
-            const int q = k * kSortedBlock + threadIdx.x;
-            if (q < M) {
-                s_row[so_phys(q)] = lrow[k];
-                s_key[so_phys(q)] = lkey[k];
-                s_gh[so_phys(q)] = lgh[k];
-                if (LEVEL0) s_aux[so_phys(q)] = lst[k];
-            }
-        }
-    }
+// A value that passed the filter: tile of the group (4 bits), feature in the tile (11), node (10), bin (8), row (31)
+__device__ __forceinline__ unsigned long long rare_item(int tile, unsigned key, unsigned node, int row) {
+    const unsigned long long feature = (unsigned)tile << 11 | key >> kRareFeatShift;
+    return ((feature << 10 | node) << 8 | (key & 0xffu)) << 31 | (unsigned)row;
+}
+__device__ __forceinline__ unsigned rare_run(unsigned long long item) { return (unsigned)(item >> 39); }  // feature and node
+__device__ __forceinline__ int rare_node(unsigned long long item) { return (int)(item >> 39) & 0x3ff; }
+__device__ __forceinline__ int rare_bin(unsigned long long item) { return (int)(item >> 31) & 0xff; }
+
+struct RareFilter {
+    unsigned long long g[kRareCells];
+    unsigned h[kRareCells];
+    unsigned open[kRareCells / 32];  // runs of the tile that may hold a winner
+    int passed;
+};
+struct RareShared {
+    unsigned long long item[kRareLds];
+    GHPair gh[kRareLds];
+    RareSum agg[kRareWaves];
+    int flag[kRareWaves];
+    int meta[kRareGroupTiles];  // first entry of the tiles' features in rare_meta
+};
+
+// Sorts the n <= kRareTile collected items. A compare-exchange over at most 64 positions stays inside the 128 items
+// that a wavefront owns, so only the wider ones need a barrier.
+__device__ void rare_sort(unsigned long long *item, int n) {
+    int size = 128;
+    while (size < n) size *= 2;
+    for (int i = n + threadIdx.x; i < size; i += kRareBlock) item[rare_phys(i)] = ~0ull;
     __syncthreads();
-    const int i0 = threadIdx.x * kSoV;
-    static_assert(32 % kSoV == 0, "a thread's positions must not straddle a padding element");
-    const int pb = so_phys(i0);  // so_phys(i0 + j) = pb + j: a thread's positions share one padding count
-    int Mn = M;  // values of the new order
-    if (!LEVEL0) {
-        const uint8_t *__restrict__ row_move = tb.row_move;
-        int row[kSoV];
-        unsigned key[kSoV];
-        GHPair pair[kSoV];
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            const int i = i0 + j;
-            row[j] = i < M ? s_row[pb + j] : -1;
-            key[j] = i < M ? s_key[pb + j] : 0xffffffffu;
-            pair[j] = i < M ? s_gh[pb + j] : GHPair{0, 0};
-        }
-        const unsigned prevk = (i0 > 0 && i0 - 1 < M) ? s_key[so_phys(i0 - 1)] : 0xffffffffu;
-        const unsigned nextk = (i0 + kSoV < M) ? s_key[so_phys(i0 + kSoV)] : 0xffffffffu;
-        // the value's node of the level above is in its key; the row -> node update left two bits per row: did the
-        // node split, and did the row go right (all of a thread's look-ups are issued before the first is used)
-        unsigned mv[kSoV];
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) mv[j] = row_move[max(row[j], 0)];
-        int xn[kSoV];
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            xn[j] = -1;  // the node is a leaf, or the run left the pass at the level above (mark in the key)
-            if (row[j] >= 0 && (key[j] & kSoNodeMask) != kSoNodeMask && (mv[j] & 1u))
-                xn[j] = 2 * (int)((key[j] >> kSortedNodeShift) & 0xfffu) + (int)(mv[j] >> 1);
-        }
-        SoCount fw[kSoV];
-        bool head[kSoV], tail[kSoV];
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            const int i = i0 + j;
-            const bool valid = i < M;
-            const unsigned pk = j == 0 ? prevk : key[j > 0 ? j - 1 : 0];
-            const unsigned nk = j == kSoV - 1 ? nextk : key[j < kSoV - 1 ? j + 1 : 0];
-            head[j] = valid && (i == 0 || (pk >> kSortedNodeShift) != (key[j] >> kSortedNodeShift));
-            tail[j] = valid && (i == M - 1 || (nk >> kSortedNodeShift) != (key[j] >> kSortedNodeShift));
-            const bool alive = valid && xn[j] >= 0;
-            fw[j].seg = alive ? ((1 << 16) | ((xn[j] & 1) ? 0 : 1)) : 0;
-            fw[j].plain = (valid && !alive) ? 1 : 0;
-        }
-        // (the scan's barriers also make sure that every thread has taken its values out of the LDS arrays before
-        // the new order is written over them)
-        so_block_scan<SoCount, true>(fw, head, s_agg_cnt, s_flag);
-        if (threadIdx.x == kSortedBlock - 1) s_dead = fw[kSoV - 1].plain;  // (positions past the end add nothing)
-        // the last value of a run knows how many of the run go left: it leaves the count at the run's start
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j)
-            if (tail[j] && xn[j] >= 0)
-                s_aux[so_phys(i0 + j - ((fw[j].seg >> 16) - 1))] = (unsigned short)(fw[j].seg & 0xffff);
-        __syncthreads();
-        Mn = M - s_dead;
-        int pos[kSoV], start[kSoV];
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            pos[j] = -1;
-            const int i = i0 + j;
-            if (i < M && xn[j] >= 0) {
-                const int cnt = fw[j].seg >> 16, lefts = fw[j].seg & 0xffff;  // inclusive
-                const int nleft = s_aux[so_phys(i - (cnt - 1))];               // of the whole run
-                const int s_new = i - (cnt - 1) - fw[j].plain;                 // the run's start once the dead are gone
-                const bool l = !(xn[j] & 1);
-                start[j] = l ? s_new : s_new + nleft;
-                pos[j] = l ? s_new + lefts - 1 : s_new + nleft + (cnt - 1) - lefts;
+    for (int k = 2; k <= size; k *= 2) {
+        for (int j = k / 2; j > 0; j /= 2) {
+            for (int i = threadIdx.x; i < size / 2; i += kRareBlock) {
+                const int a = ((i & ~(j - 1)) << 1) | (i & (j - 1));
+                const int pa = rare_phys(a), pb = rare_phys(a | j);
+                const unsigned long long x = item[pa], y = item[pb];
+                if ((x > y) == ((a & k) == 0)) {
+                    item[pa] = y;
+                    item[pb] = x;
+                }
             }
-        }
-        __syncthreads();  // every left count has been read: s_aux takes the run starts of the new order
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            if (pos[j] >= 0) {
-                const int pp = so_phys(pos[j]);
-                s_row[pp] = row[j];
-                s_key[pp] = (key[j] & ~kSoNodeMask) | ((unsigned)xn[j] << kSortedNodeShift);
-                s_gh[pp] = pair[j];
-                s_aux[pp] = (unsigned short)start[j];
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) live[blockIdx.x] = Mn;
-    if (Mn == 0) return;
-    // ---- rows and gradient pairs of the new order back to HBM (coalesced); the keys follow once the runs that leave
-    // the pass are marked
-    // (no level reads the order of the tree's last level)
-    if (!last_level) {
-        for (int q = threadIdx.x; q < Mn; q += kSortedBlock) {
-            out_row[q] = s_row[so_phys(q)];
-            out_gh[q] = s_gh[so_phys(q)];
+            if (j > 64 || (j == 1 && k >= 128)) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     }
-    unsigned key[kSoV];
-    SoSum fs[kSoV];
-    bool head[kSoV], tail[kSoV], last_of_bin[kSoV];
+}
+
+// What the search needs of a node: per node of the level its best key (8 bytes), its sums (8) and its own gain term (4).
+struct RareNodes {
+    unsigned long long *best;
+    GHPair *S;
+    float *P;
+    __device__ RareNodes(unsigned char *lds, int nl)
+        : best(reinterpret_cast<unsigned long long *>(lds)), S(reinterpret_cast<GHPair *>(best + nl)),
+          P(reinterpret_cast<float *>(S + nl)) {}
+    __device__ void load(const TreeBuffers &tb, int nl, float lambda) {
+#pragma clang fp contract(off)
+        for (int x = threadIdx.x; x < nl; x += kRareBlock) {
+            const GHPair s = tb.nodes[nl - 1 + x].sum_gh_pair;
+            best[x] = __hip_atomic_load(&tb.best_key[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            S[x] = s;
+            P[x] = (s.g * s.g) / (s.h + lambda);
+        }
+    }
+    __device__ float floor(int x) const { return __uint_as_float((unsigned)(best[x] >> 32)); }
+};
+
+// Searches the n collected values and clears the way for the next ones.
+__device__ void rare_search(const TreeBuffers &tb, const SparsePass &sp, RareShared &sh, const RareNodes &node,
+                            const GHPair *__restrict__ gh, int n, int slot, float mcw, float lambda) {
+#pragma clang fp contract(off)
+    rare_sort(sh.item, n);
+    for (int p = threadIdx.x; p < n; p += kRareBlock)
+        sh.gh[rare_phys(p)] = gh[(int)((unsigned)sh.item[rare_phys(p)] & 0x7fffffffu)];
+    __syncthreads();
     const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
+    const int i0 = threadIdx.x * kRareV;
+    static_assert(32 % kRareV == 0, "a thread's positions must not straddle a padding element");
+    const int pb = rare_phys(i0);  // rare_phys(i0 + j) = pb + j: a thread's positions share one padding count
+    unsigned long long it[kRareV];
+    RareSum fs[kRareV];
+    bool head[kRareV], tail[kRareV], last_of_bin[kRareV];
+    const unsigned long long before = (i0 > 0 && i0 - 1 < n) ? sh.item[rare_phys(i0 - 1)] : ~0ull;
+    const unsigned long long after = i0 + kRareV < n ? sh.item[rare_phys(i0 + kRareV)] : ~0ull;
 #pragma unroll
-    for (int j = 0; j < kSoV; ++j) {
-        const int p = i0 + j;
-        const bool in = p < Mn;
-        key[j] = in ? s_key[pb + j] : 0xffffffffu;
-        fs[j] = SoSum{0, 0};
+    for (int j = 0; j < kRareV; ++j) {
+        const bool in = i0 + j < n;
+        it[j] = in ? sh.item[pb + j] : ~0ull;
+        fs[j] = RareSum{0, 0, 0};
         if (in) {
-            const GHPair s = s_gh[pb + j];
-            fs[j].g = round_to_ll(s.g * scale_g);
-            fs[j].h = round_to_ll(s.h * scale_h);
+            const GHPair s = sh.gh[pb + j];
+            fs[j] = RareSum{round_to_ll(s.g * scale_g), round_to_ll(s.h * scale_h), 1};
         }
     }
-    {
-        const unsigned prevk = (i0 > 0 && i0 - 1 < Mn) ? s_key[so_phys(i0 - 1)] : 0xffffffffu;
-        const unsigned nextk = (i0 + kSoV < Mn) ? s_key[so_phys(i0 + kSoV)] : 0xffffffffu;
 #pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            const int p = i0 + j;
-            const bool in = p < Mn;
-            const unsigned pk = j == 0 ? prevk : key[j > 0 ? j - 1 : 0];
-            const unsigned nk = j == kSoV - 1 ? nextk : key[j < kSoV - 1 ? j + 1 : 0];
-            head[j] = in && (p == 0 || (pk >> kSortedNodeShift) != (key[j] >> kSortedNodeShift));
-            tail[j] = in && (p + 1 == Mn || (nk >> kSortedNodeShift) != (key[j] >> kSortedNodeShift));
-            last_of_bin[j] = in && (p + 1 == Mn || nk != key[j]);
-        }
-    }
-    if (dump_hist) {
-        // stage-wise inspection: the per-node histograms of the level (zeroed before the launch) get the values
-        unsigned long long *hist = reinterpret_cast<unsigned long long *>(tb.hist(level));
-#pragma unroll
-        for (int j = 0; j < kSoV; ++j) {
-            if (i0 + j < Mn) {
-                const int x = (int)((key[j] >> kSortedNodeShift) & 0xfffu), lb = (int)(key[j] & 0xffu);
-                const int fbegin = sp.sorted_meta[task.meta_begin + (int)(key[j] >> kSortedFeatShift)].x;
-                unsigned long long *cell = hist + 2 * ((size_t)x * tb.n_bins + fbegin + lb);
-                atomicAdd(cell, (unsigned long long)fs[j].g);
-                atomicAdd(cell + 1, (unsigned long long)fs[j].h);
-            }
-        }
-    }
-    // (the scan's barriers: the stores above have read s_gh, which now takes the run totals)
-    so_block_scan<SoSum, true>(fs, head, s_agg_sum, s_flag);
-    // the last value of a run holds the run's sums = the feature's total in the node: as floats to the run's start.
-    // It also decides whether the run can matter at this level at all. Every candidate of the run splits a subset A
-    // of the run's values off the node (a prefix when the missing rows go right, a suffix when they go left), with
-    // A.h >= min_child_weight, |A.g| <= (values of the run) x (largest |g| of the tree) =: ga and A.h <= the run's
-    // hessian sum th, so its gain is at most
-    //   ga^2 / (mcw + lambda) + (|S.g| + ga)^2 / (max(mcw, S.h - th) + lambda) - S.g^2 / (S.h + lambda).
-    // A run whose bound (plus 2^-18 of its terms, far above the float roundings of the bound and of the gains it
-    // stands for) stays below the best gain the node has seen so far has no candidate worth evaluating: it is
-    // marked in the sign of the hessian total (which is never negative). On 2 M x 100 k data that is 85 % of the
-    // values at every level.
-    int start[kSoV];
-    const float g_max = tb.quant->gq_max * tb.quant->inv_g;
-#pragma unroll
-    for (int j = 0; j < kSoV; ++j) {
-        start[j] = (i0 + j < Mn) ? (int)s_aux[pb + j] : 0;
-        if (tail[j]) {
-            const float tg = (float)((double)fs[j].g * inv_g), th = (float)((double)fs[j].h * inv_h);
-            const int x = (int)((key[j] >> kSortedNodeShift) & 0xfffu);
-            const GHPair S = s_S[x];
-            const float P = s_P[x];
-            const float floor = __uint_as_float((unsigned)(s_best[x] >> 32));
-            const float ga = g_max * (float)(i0 + j - start[j] + 1);
-            const float sa = fabsf(S.g) + ga;
-            const float t1 = ga * ga / (mcw + lambda), t2 = sa * sa / (fmaxf(mcw, S.h - th) + lambda);
-            const bool hopeless = (t1 + t2 - P) + (t1 + t2 + fabsf(P)) * 3.8146973e-6f < floor;
-            s_gh[so_phys(start[j])] = GHPair{tg, hopeless ? -th : th};
-        }
-    }
-    __syncthreads();
-    // ---- A (feature, node) run whose hessians add up to less than min_child_weight cannot yield a split, here or
-    // in any node below (hessians are not negative, so every left or right side taken from the run's values, and
-    // every run of a child node, weighs less still; the margin covers the float roundings of the missing-value
-    // arithmetic, a few ulps of the node's hessian sum). Such runs leave the pass: their keys get the node field's
-    // all-ones mark, which the next level reads as "dead". Not when the per-node histograms are being recorded.
-    GHPair tot[kSoV];
-    bool drop[kSoV], hopeless[kSoV];
-#pragma unroll
-    for (int j = 0; j < kSoV; ++j) {
-        drop[j] = hopeless[j] = false;
-        tot[j] = GHPair{0, 0};
+    for (int j = 0; j < kRareV; ++j) {
         const int p = i0 + j;
-        if (p < Mn) {
-            tot[j] = s_gh[so_phys(start[j])];
-            hopeless[j] = (__float_as_uint(tot[j].h) >> 31) != 0u;
-            tot[j].h = fabsf(tot[j].h);
-            const float Sh = s_S[(key[j] >> kSortedNodeShift) & 0xfffu].h;
-            drop[j] = !dump_hist && tot[j].h + Sh * 4.76837158e-7f < mcw;  // 2^-21
-            if (drop[j]) s_key[pb + j] = key[j] | kSoNodeMask;
-        }
+        const bool in = p < n;
+        const unsigned long long prev = j == 0 ? before : it[j > 0 ? j - 1 : 0];
+        const unsigned long long next = j == kRareV - 1 ? after : it[j < kRareV - 1 ? j + 1 : 0];
+        head[j] = in && (p == 0 || rare_run(prev) != rare_run(it[j]));
+        tail[j] = in && (p + 1 == n || rare_run(next) != rare_run(it[j]));
+        last_of_bin[j] = in && (p + 1 == n || (next >> 31) != (it[j] >> 31));
+    }
+    // (the scan's barriers: every thread has read its pairs, their place takes the run totals)
+    rare_block_scan(fs, head, sh.agg, sh.flag);
+    // the last value of a run holds the run's sums = the feature's total in the node: as floats to the run's start
+    GHPair left[kRareV];
+    int start[kRareV];
+#pragma unroll
+    for (int j = 0; j < kRareV; ++j) {
+        left[j] = GHPair{(float)((double)fs[j].g * inv_g), (float)((double)fs[j].h * inv_h)};
+        start[j] = rare_phys(max(0, i0 + j - fs[j].n + 1));
+        if (tail[j]) sh.gh[start[j]] = left[j];
     }
     __syncthreads();
-    if (!last_level)
-        for (int q = threadIdx.x; q < Mn; q += kSortedBlock) out_key[q] = s_key[so_phys(q)];
-    // ---- candidates: raise the node's key in LDS, then the winners publish. A candidate without gain never
-    // competes: the node's candidate at global bin 0 (a table feature's) has at least its key.
-    float sc_head[kSoV], sc_bin[kSoV];
+    // candidates raise the node's key in LDS, then the winners publish. A candidate without gain never competes: the
+    // node's candidate at global bin 0 (a table feature's) has at least its key.
+    float sc_head[kRareV], sc_bin[kRareV];
 #pragma unroll
-    for (int j = 0; j < kSoV; ++j) {
+    for (int j = 0; j < kRareV; ++j) {
         sc_head[j] = sc_bin[j] = 0.f;
-        if (!(head[j] || last_of_bin[j]) || drop[j] || hopeless[j]) continue;
-        const int x = (int)((key[j] >> kSortedNodeShift) & 0xfffu), lb = (int)(key[j] & 0xffu);
-        const int fi = task.meta_begin + (int)(key[j] >> kSortedFeatShift);
-        const int2 meta = sp.sorted_meta[fi];
-        const bool ign = tb.ignored != nullptr && tb.ignored[sp.sorted_fid[fi]] != 0;
-        const GHPair S = s_S[x];
-        const float P = s_P[x];
-        const GHPair mm{S.g - tot[j].g, S.h - tot[j].h};
-        const float floor = __uint_as_float((unsigned)(s_best[x] >> 32));
+        if (!(head[j] || last_of_bin[j])) continue;
+        const unsigned long long item = sh.item[pb + j];
+        const int x = rare_node(item), lb = rare_bin(item);
+        const int2 meta = sp.rare_meta[sh.meta[(int)(item >> 60)] + ((int)(item >> 49) & 0x7ff)];
+        const GHPair tot = sh.gh[start[j]];
+        const GHPair S = node.S[x];
+        const float P = node.P[x];
+        const GHPair mm{S.g - tot.g, S.h - tot.h};
+        const float floor = node.floor(x);
         if (head[j]) {
-            sc_head[j] = so_score(S, P, mm, GHPair{0, 0}, ign, mcw, lambda, floor);
-            if (sc_head[j] != 0.f) atomicMax(&s_best[x], cand_key(fabsf(sc_head[j]), meta.x));
+            sc_head[j] = rare_score(S, P, mm, GHPair{0, 0}, mcw, lambda, floor);
+            if (sc_head[j] != 0.f) atomicMax(&node.best[x], cand_key(fabsf(sc_head[j]), meta.x));
         }
         if (last_of_bin[j] && lb < meta.y - 1) {
-            const GHPair l{(float)((double)fs[j].g * inv_g), (float)((double)fs[j].h * inv_h)};
-            sc_bin[j] = so_score(S, P, mm, l, ign, mcw, lambda, floor);
-            if (sc_bin[j] != 0.f) atomicMax(&s_best[x], cand_key(fabsf(sc_bin[j]), meta.x + lb + 1));
+            sc_bin[j] = rare_score(S, P, mm, left[j], mcw, lambda, floor);
+            if (sc_bin[j] != 0.f) atomicMax(&node.best[x], cand_key(fabsf(sc_bin[j]), meta.x + lb + 1));
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kSoV; ++j) {
+    for (int j = 0; j < kRareV; ++j) {
         if (sc_head[j] == 0.f && sc_bin[j] == 0.f) continue;
-        const int x = (int)((key[j] >> kSortedNodeShift) & 0xfffu), lb = (int)(key[j] & 0xffu);
-        const int fbegin = sp.sorted_meta[task.meta_begin + (int)(key[j] >> kSortedFeatShift)].x;
-        const unsigned long long best = s_best[x];
+        const unsigned long long item = sh.item[pb + j];
+        const int x = rare_node(item), lb = rare_bin(item);
+        const int fbegin = sp.rare_meta[sh.meta[(int)(item >> 60)] + ((int)(item >> 49) & 0x7ff)].x;
+        const unsigned long long best = node.best[x];
         const bool win_head = sc_head[j] != 0.f && best == cand_key(fabsf(sc_head[j]), fbegin);
         const bool win_bin = sc_bin[j] != 0.f && best == cand_key(fabsf(sc_bin[j]), fbegin + lb + 1);
         if (!(win_head || win_bin)) continue;
-        // the tile's best of the node: worth publishing only if it beats what other tasks have published so far
+        // the group's best of the node: worth publishing only if it beats what other groups have published so far
         if (best <= __hip_atomic_load(&tb.best_key[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) continue;
-        const GHPair S = s_S[x];
+        const GHPair S = node.S[x], tot = sh.gh[start[j]];
         SplitCand o;
-        o.miss = GHPair{S.g - tot[j].g, S.h - tot[j].h};
+        o.miss = GHPair{S.g - tot.g, S.h - tot.h};
         o.feature = o.bin = 0;
         if (win_head) {
             o.score = sc_head[j];
@@ -834,10 +728,153 @@ __global__ __launch_bounds__(kSortedBlock) void k_sparse_sorted(TreeBuffers tb_a
         } else {
             o.score = sc_bin[j];
             o.index = fbegin + lb + 1;
-            o.left = GHPair{(float)((double)fs[j].g * inv_g), (float)((double)fs[j].h * inv_h)};
+            o.left = left[j];
         }
-        tb.cand[(size_t)x * tb.n_packs + task.cand_slot] = o;
+        tb.cand[(size_t)x * tb.n_packs + slot] = o;
         atomicMax(&tb.best_key[x], best);
+    }
+    __syncthreads();
+}
+
+// One workgroup per tile: the values of the runs that may hold a winner go to the tile's part of rare_item.
+template <bool DUMP>
+__global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffers tb_all, SparsePass sp,
+                                                                     const GHPair *__restrict__ gh, int level, float mcw,
+                                                                     float lambda) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char rare_dyn[];
+    __shared__ RareFilter sh;
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    gh += (size_t)blockIdx.z * tb.n;
+    const int nl = 1 << level;
+    const RareTask task = sp.rare_tasks[blockIdx.x];
+    const unsigned *__restrict__ keys = sp.rare_key + task.v_begin;
+    const int *__restrict__ rows = sp.rare_row + task.v_begin;
+    const unsigned *__restrict__ words = tb.row_word;
+    unsigned key[kRareV], word[kRareV];
+    int row[kRareV];
+    // (positions past the end repeat the last value, so that all loads are issued at once)
+#pragma unroll
+    for (int k = 0; k < kRareV; ++k) {
+        const int q = min(k * kRareBlock + (int)threadIdx.x, task.count - 1);
+        // (streamed past the caches: the words stay in the L2s)
+        row[k] = __builtin_nontemporal_load(rows + q);
+        key[k] = __builtin_nontemporal_load(keys + q);
+    }
+#pragma unroll
+    for (int k = 0; k < kRareV; ++k) word[k] = words[row[k]];
+    int log_groups = 0;
+    while (2 << log_groups <= kRareMaxGroups && task.n_feat * nl << (log_groups + 1) <= kRareCells) ++log_groups;
+    const int cells = min(kRareCells, task.n_feat * nl << log_groups);
+    for (int c = threadIdx.x; c < cells; c += kRareBlock) {
+        sh.g[c] = 0ull;
+        sh.h[c] = 0u;
+    }
+    for (int c = threadIdx.x; c < kRareCells / 32; c += kRareBlock) sh.open[c] = 0u;
+    if (threadIdx.x == 0) sh.passed = 0;
+    RareNodes node(rare_dyn, nl);
+    node.load(tb, nl, lambda);
+    const RareBound unit{tb.quant->gq_max * tb.quant->inv_g / kRareSteps, tb.quant->hq_max * tb.quant->inv_h / kRareSteps, mcw,
+                         lambda};
+    __syncthreads();
+    int cell[kRareV];  // -1: the value takes no part
+#pragma unroll
+    for (int k = 0; k < kRareV; ++k) {
+        const unsigned x = word[k] & kRareNodeMask;
+        const int feature = (int)(key[k] >> kRareFeatShift);
+        const bool on = k * kRareBlock + (int)threadIdx.x < task.count && x != kRareNodeMask;
+        // (more runs than cells: two runs that meet in one only loosen the bound)
+        const unsigned group = (key[k] >> 8 & 0x3fu) >> (6 - log_groups);
+        cell[k] = on ? (int)((((unsigned)(feature * nl) + x) << log_groups | group) % kRareCells) : -1;
+        if (tb.ignored != nullptr && on && tb.ignored[sp.rare_fid[task.meta_begin + feature]] != 0)
+            cell[k] = -1;  // column sampling: all scores are 0 (hist_tree_builder_single.cu:304 / :663)
+        if (cell[k] >= 0) {
+            atomicAdd(&sh.g[cell[k]], rare_addend(word[k]));
+            atomicAdd(&sh.h[cell[k]], word[k] >> 22);
+        }
+        if (DUMP && on) {
+            // stage-wise inspection: the per-node histograms of the level (zeroed before the launch) get the values
+            const GHPair s = gh[row[k]];
+            const size_t b = (size_t)x * tb.n_bins + sp.rare_meta[task.meta_begin + feature].x + (key[k] & 0xffu);
+            unsigned long long *out = reinterpret_cast<unsigned long long *>(tb.hist(level) + b);
+            atomicAdd(out, (unsigned long long)round_to_ll(s.g * tb.quant->scale_g));
+            atomicAdd(out + 1, (unsigned long long)round_to_ll(s.h * tb.quant->scale_h));
+        }
+    }
+    __syncthreads();
+    if (log_groups > 0) {
+        rare_check_cells(
+            sh.g, sh.h, cells, log_groups,
+            [&](int run, RareCell before, RareCell own, RareCell after) {
+                const int x = run & (nl - 1);
+                const GHPair S = node.S[x];
+                const float P = node.P[x], floor = node.floor(x);
+                return !rare_hopeless(before, own, S, P, floor, unit) || !rare_hopeless(after, own, S, P, floor, unit);
+            },
+            [&](int run) { atomicOr(&sh.open[run >> 5], 1u << (run & 31)); });
+        __syncthreads();
+    }
+    unsigned pass = 0;
+#pragma unroll
+    for (int k = 0; k < kRareV; ++k) {
+        if (cell[k] < 0) continue;
+        const int x = (int)(word[k] & kRareNodeMask);
+        bool on;
+        if (log_groups > 0) {
+            const int run = cell[k] >> log_groups;
+            on = (sh.open[run >> 5] >> (run & 31) & 1u) != 0;
+        } else {
+            on = !rare_hopeless(RareCell{0, 0}, RareCell{sh.g[cell[k]], sh.h[cell[k]]}, node.S[x], node.P[x], node.floor(x), unit);
+        }
+        if (on) pass |= 1u << k;
+    }
+    if (__any(pass != 0)) {
+        // (few values pass: they are read again)
+        int at = pass != 0 ? atomicAdd(&sh.passed, __popc(pass)) : 0;
+        unsigned long long *out = sp.rare_item + (size_t)blockIdx.z * sp.n_rare + task.v_begin;
+        for (unsigned left = pass; left != 0; left &= left - 1) {
+            const int q = (__ffs(left) - 1) * kRareBlock + (int)threadIdx.x;
+            out[at++] = rare_item((int)(blockIdx.x / (unsigned)sp.n_rare_groups), keys[q], words[rows[q]] & kRareNodeMask, rows[q]);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) sp.rare_passed[(size_t)blockIdx.z * sp.n_rare_tasks + blockIdx.x] = sh.passed;
+}
+
+// One workgroup = the tiles blockIdx.x, blockIdx.x + gridDim.x, ... (at most kRareGroupTiles).
+__global__ __launch_bounds__(kRareBlock, 4) void k_sparse_rare_search(TreeBuffers tb_all, SparsePass sp,
+                                                                     const GHPair *__restrict__ gh, int level, float mcw,
+                                                                     float lambda) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char rare_dyn[];
+    __shared__ RareShared sh;
+    __shared__ int s_passed[kRareGroupTiles];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    gh += (size_t)blockIdx.z * tb.n;
+    if (threadIdx.x < kRareGroupTiles) {
+        const int tile = (int)blockIdx.x + (int)threadIdx.x * (int)gridDim.x;
+        const bool in = tile < sp.n_rare_tasks;
+        s_passed[threadIdx.x] = in ? sp.rare_passed[(size_t)blockIdx.z * sp.n_rare_tasks + tile] : 0;
+        sh.meta[threadIdx.x] = in ? sp.rare_tasks[tile].meta_begin : 0;
+    }
+    __syncthreads();
+    int all = 0;
+    for (int j = 0; j < kRareGroupTiles; ++j) all += s_passed[j];
+    if (all == 0) return;
+    RareNodes node(rare_dyn, 1 << level);
+    node.load(tb, 1 << level, lambda);
+    const int slot = sp.rare_slot + (int)blockIdx.x;
+    int filled = 0;
+    for (int j = 0; j <= kRareGroupTiles; ++j) {
+        const int passed = j < kRareGroupTiles ? s_passed[j] : 0;
+        if (filled > 0 && (j == kRareGroupTiles || filled + passed > kRareTile)) {
+            rare_search(tb, sp, sh, node, gh, filled, slot, mcw, lambda);
+            filled = 0;
+        }
+        if (passed == 0) continue;
+        const unsigned long long *__restrict__ in =
+            sp.rare_item + (size_t)blockIdx.z * sp.n_rare + sp.rare_tasks[(int)blockIdx.x + j * (int)gridDim.x].v_begin;
+        for (int q = threadIdx.x; q < passed; q += kRareBlock) sh.item[rare_phys(filled + q)] = in[q];
+        filled += passed;
+        __syncthreads();
     }
 }
 
@@ -850,15 +887,14 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_partition(TreeBuffers tb_al
     const int nl = 1 << level, off = nl - 1;
     for (int i = threadIdx.x; i < 2 * nl; i += kSpBlock) cnt[i] = 0;
     __syncthreads();
-    const int n64 = (tb.n + 63) & ~63;
-    for (int r = blockIdx.x * kSpBlock + threadIdx.x; r < n64; r += gridDim.x * kSpBlock) {
-        bool moved = false, right = false;
-        if (r < tb.n) {
+    for (int r = blockIdx.x * kSpBlock + threadIdx.x; r < tb.n; r += gridDim.x * kSpBlock) {
+        int child = (int)kRareNodeMask;  // of the next level; all ones: the row stays
+        {
             const int node = tb.nid16[r];
             if (node >= off) {  // (else the row stays in a leaf of an earlier level)
                 const TreeNode &nd = tb.nodes[node];
                 if (node_splits(nd)) {
-                    moved = true;
+                    bool right;
                     const int col = bins.col_of_feature != nullptr ? bins.col_of_feature[nd.split_feature_id] : -1;
                     if (col >= 0) {
                         // a frequent feature: the row's local bin id is one byte away (same rule: missing -> default
@@ -870,18 +906,27 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_partition(TreeBuffers tb_al
                         right = csr_goes_right(bins, r, cb, ce, cb + nd.split_bid, nd.default_right);
                     }
                     tb.nid16[r] = (unsigned short)(right ? nd.rch_index : nd.lch_index);
-                    atomicAdd(&cnt[2 * (node - off) + (right ? 1 : 0)], 1);
+                    child = 2 * (node - off) + (right ? 1 : 0);
+                    atomicAdd(&cnt[child], 1);
                 }
             }
         }
-        tb.row_move[r] = (uint8_t)((moved ? 1 : 0) | (moved && right ? 2 : 0));  // (r < n rounded up to 64: allocated)
+        if (tb.row_word != nullptr) tb.row_word[r] = (tb.row_word[r] & ~kRareNodeMask) | (unsigned)child;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * nl; i += kSpBlock)
         if (cnt[i] != 0) atomicAdd(&tb.node_rows[2 * off + 1 + i], cnt[i]);  // children of level node x: 2 (off + x) + 1, + 2
 }
 
-// csc_gh[e] = gh[csc_row[e]] for the stored values of the table tasks (the sorted pass fetches its pairs itself)
+// The rows' words of a tree, every row in the root.
+__global__ __launch_bounds__(256) void k_sparse_row_words(TreeBuffers tb_all, const GHPair *__restrict__ gh) {
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    gh += (size_t)blockIdx.z * tb.n;
+    const QuantCtl q = *tb.quant;
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < tb.n; r += gridDim.x * 256) tb.row_word[r] = rare_row_word(0u, gh[r], q);
+}
+
+// csc_gh[e] = gh[csc_row[e]] for the stored values of the table tasks
 __global__ __launch_bounds__(256) void k_sparse_gh_refresh(int n, SparsePass sp, const int *__restrict__ csc_row,
                                                           const GHPair *__restrict__ gh) {
     gh += (size_t)blockIdx.z * n;
@@ -903,20 +948,19 @@ __global__ __launch_bounds__(256) void k_sparse_cols(long nnz, const int *__rest
     }
 }
 
-// Static order of a sorted task's tile: its features one after the other, each in the order of the bin-major copy.
-__global__ __launch_bounds__(256) void k_sorted_setup(SparsePass sp, CsrBins bins, const int *__restrict__ cut_row_ptr,
-                                                     int *__restrict__ row0, unsigned *__restrict__ key0,
-                                                     unsigned short *__restrict__ start0) {
-    const SortedTask task = sp.sorted_tasks[blockIdx.x];
+// Values of a tile of rare features: its features one after the other, each in the order of the bin-major copy.
+__global__ __launch_bounds__(256) void k_rare_setup(SparsePass sp, CsrBins bins, const int *__restrict__ cut_row_ptr,
+                                                   int *__restrict__ row, unsigned *__restrict__ key) {
+    const RareTask task = sp.rare_tasks[blockIdx.x];
     int dst = task.v_begin;
     for (int fi = 0; fi < task.n_feat; ++fi) {
-        const int f = sp.sorted_fid[task.meta_begin + fi];
+        const int f = sp.rare_fid[task.meta_begin + fi];
         const int v0 = sp.feat_val_begin[f], m = sp.feat_val_begin[f + 1] - v0;
         const int fbegin = cut_row_ptr[f];
         for (int a = threadIdx.x; a < m; a += 256) {
-            row0[dst + a] = bins.csc_row[v0 + a];
-            key0[dst + a] = ((unsigned)fi << kSortedFeatShift) | (unsigned)(bins.csc_bin[v0 + a] - fbegin);
-            start0[dst + a] = (unsigned short)(dst - task.v_begin);
+            row[dst + a] = bins.csc_row[v0 + a];
+            key[dst + a] = ((unsigned)fi << kRareFeatShift) | (unsigned)(a * kRareMaxGroups / m) << 8 |
+                           (unsigned)(bins.csc_bin[v0 + a] - fbegin);
         }
         dst += m;
     }
@@ -931,10 +975,15 @@ void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *
     k_sparse_cols<<<grid, 256, 0, s>>>(nnz, csc_bin, csc_row, cut_fid, cut_row_ptr, col_of_feature, colbin, col_stride);
 }
 
-void launch_sorted_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row0,
-                         unsigned *key0, unsigned short *start0) {
-    if (sp.n_sorted_tasks == 0) return;
-    k_sorted_setup<<<sp.n_sorted_tasks, 256, 0, s>>>(sp, bins, tb.cut_row_ptr, row0, key0, start0);
+void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row,
+                       unsigned *key) {
+    if (sp.n_rare_tasks == 0) return;
+    k_rare_setup<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, tb.cut_row_ptr, row, key);
+}
+
+void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class) {
+    if (tb.row_word == nullptr) return;
+    k_sparse_row_words<<<dim3(std::max(1, std::min(1024, (tb.n + 255) / 256)), 1, n_class), 256, 0, s>>>(tb, gh);
 }
 
 void launch_sparse_gh_refresh(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
@@ -944,15 +993,14 @@ void launch_sparse_gh_refresh(hipStream_t s, const TreeBuffers &tb, const CsrBin
 }
 
 void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
-                         const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class,
-                         bool last_level) {
+                         const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class) {
     // LDS table of a table task: room for one feature of 255 bins with every node of the level, at least 2048 and at
     // most kSparseCells cells (shallow levels: small tables, two workgroups per CU; deep levels: node ranges)
     int n_cells = 2048;
     while (n_cells < kSparseCells && n_cells < 256 * (1 << level)) n_cells *= 2;
     const size_t lds = sizeof(longlong2) * (size_t)n_cells;
     if (dump_hist) {
-        // the table kernels store the cells of their features, the sorted pass adds its values: start from zero
+        // the table kernels store the cells of their features, the rare features' values are added: start from zero
         for (int k = 0; k < n_class; ++k)
             launch_fill_f32(s, reinterpret_cast<float *>(tb.for_class(k).hist(level)), 0.f,
                             (size_t)(1 << level) * tb.n_bins * 4);
@@ -972,15 +1020,12 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
     if (sp.n_big > 0)
         k_sparse_big<<<dim3(sp.n_big, std::min(1 << level, 16), n_class), kSpBlock, lds, s>>>(
             tb, sp, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
-    if (sp.n_sorted_tasks > 0) {
-        const int dh = dump_hist ? 1 : 0;
-        const size_t so_lds = (size_t)(1 << level) * 20;
-        if (level == 0)
-            k_sparse_sorted<true><<<dim3(sp.n_sorted_tasks, 1, n_class), kSortedBlock, so_lds, s>>>(
-                tb, sp, gh, level, mcw, lambda, dh, last_level ? 1 : 0);
-        else
-            k_sparse_sorted<false><<<dim3(sp.n_sorted_tasks, 1, n_class), kSortedBlock, so_lds, s>>>(
-                tb, sp, gh, level, mcw, lambda, dh, last_level ? 1 : 0);
+    if (sp.n_rare_tasks > 0) {
+        const size_t nodes_lds = (size_t)(1 << level) * 20;
+        const dim3 tiles(sp.n_rare_tasks, 1, n_class);
+        if (dump_hist) k_sparse_rare_filter<true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        else k_sparse_rare_filter<false><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        k_sparse_rare_search<<<dim3(sp.n_rare_groups, 1, n_class), kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
     }
 }
 

@@ -129,7 +129,7 @@ class Trainer {
     bool wide_eval_ = false;        // split search with one workgroup per (feature, node)
     int hist_cap_level_ = -1;       // first level with more nodes than the histogram arena holds (-1: none)
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
-    bool sparse_sorted_on_ = true;
+    bool sparse_rare_on_ = true;
     bool sparse_feature_in_tables(int f);
     SparsePass sp_;
     void build_sparse_tasks();

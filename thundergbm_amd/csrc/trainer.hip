@@ -259,7 +259,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             // row's bin ids. As many of the table features, most frequent first, as fit an eighth of the free memory.
             std::vector<int> order;
             for (int f = 0; f < F_; ++f)
-                if (cuts_.feature_nnz[f] > 0 && cuts_.feature_nnz[f] > kSortedTile) order.push_back(f);
+                if (cuts_.feature_nnz[f] > 0 && cuts_.feature_nnz[f] > kRareTile) order.push_back(f);
             std::stable_sort(order.begin(), order.end(),
                              [&](int a, int b) { return cuts_.feature_nnz[a] > cuts_.feature_nnz[b]; });
             device_mem_info(&free_b, &total_b);
@@ -532,7 +532,7 @@ void Trainer::alloc_tree_buffers() {
     const size_t set_bytes =
         sparse_pass_ ? (size_t)n_ * 15 + (size_t)sp_.n_partial_slots * sp_.partial_stride * sizeof(longlong2) +
                            (size_t)max_level_nodes * sp_.n_cand_slots * sizeof(SplitCand) +
-                           (size_t)sp_.n_sorted * 32 + (size_t)nnz_ * sizeof(GHPair)
+                           (size_t)sp_.n_rare * 8 + (size_t)nnz_ * sizeof(GHPair)
                      : fixed_bytes + arena_bytes(hist_nodes);
     const char *be = std::getenv("TGBM_BATCH_CLASSES");  // "0": build the trees of a round one after the other
     n_sets_ = (K > 1 && set_bytes * K < free_b / 2 && !(be != nullptr && std::string(be) == "0")) ? K : 1;
@@ -550,7 +550,7 @@ void Trainer::alloc_tree_buffers() {
     } else {
         tb.nid16 = dalloc<unsigned short>(S * (((size_t)n_ + 2) / 2 * 2));
         tb.node_rows = dalloc<int>(S * tb.n_nodes);
-        tb.row_move = dalloc<uint8_t>(S * (((size_t)n_ + 63) / 64 * 64));
+        if (sp_.n_rare_tasks > 0) tb.row_word = dalloc<unsigned>(S * (size_t)n_);
     }
     tb.partial = dalloc<longlong2>(S * tb.n_partial);
     tb.quant = dalloc<QuantCtl>(S);
@@ -619,23 +619,14 @@ void Trainer::alloc_tree_buffers() {
     if (sparse_pass_) {
         tb.best_key = dalloc<unsigned long long>(S * (size_t)max_level_nodes);
         HIP_CHECK(hipMemsetAsync(tb.best_key, 0, sizeof(unsigned long long) * S * (size_t)max_level_nodes, stream_));
-        if (sp_.n_sorted_tasks > 0) {
-            // static order of the sorted pass, then per set the two level orders and the live counts
-            int *row0 = dalloc<int>((size_t)sp_.n_sorted);
-            unsigned *key0 = dalloc<unsigned>((size_t)sp_.n_sorted);
-            unsigned short *start0 = dalloc<unsigned short>((size_t)sp_.n_sorted);
-            launch_sorted_setup(stream_, tb, csr_, sp_, row0, key0, start0);
-            sp_.sorted_row0 = row0;
-            sp_.sorted_key0 = key0;
-            sp_.sorted_start0 = start0;
-            for (int b = 0; b < 2; ++b) {
-                sp_.sorted_row[b] = dalloc<int>(S * (size_t)sp_.n_sorted);
-                sp_.sorted_key[b] = dalloc<unsigned>(S * (size_t)sp_.n_sorted);
-                sp_.sorted_gh[b] = dalloc<GHPair>(S * (size_t)sp_.n_sorted);
-            }
-            sp_.sorted_live = dalloc<int>(S * (size_t)kSortedLevels * sp_.n_sorted_tasks);
-            HIP_CHECK(hipMemsetAsync(sp_.sorted_live, 0, sizeof(int) * S * (size_t)kSortedLevels * sp_.n_sorted_tasks,
-                                     stream_));
+        if (sp_.n_rare_tasks > 0) {
+            int *row = dalloc<int>((size_t)sp_.n_rare);
+            unsigned *key = dalloc<unsigned>((size_t)sp_.n_rare);
+            launch_rare_setup(stream_, tb, csr_, sp_, row, key);
+            sp_.rare_row = row;
+            sp_.rare_key = key;
+            sp_.rare_item = dalloc<unsigned long long>(S * (size_t)sp_.n_rare);
+            sp_.rare_passed = dalloc<int>(S * (size_t)sp_.n_rare_tasks);
         }
         sp_.partial = dalloc<longlong2>(S * (size_t)sp_.n_partial_slots * sp_.partial_stride);
         // per-value gradient pairs in the order of the bin-major copy, when they fit comfortably
@@ -820,8 +811,8 @@ void Trainer::ensure_hist_arena() {
     tb_.hist_nodes = tb_.max_level_nodes;
 }
 
-// Which features the sparse level pass serves through (bin, node) tables: those with more values than a sorted-pass
-// tile holds, and the feature that owns global bin 0 (its table is searched for every node even without values: the
+// Which features the sparse level pass serves through (bin, node) tables: those with more values than a tile of rare
+// features holds, and the feature that owns global bin 0 (its table is searched for every node even without values: the
 // arg-max of a node without any positive gain ends there).
 bool Trainer::sparse_feature_in_tables(int f) {
     if (sparse_bin0_owner_ == -2) {
@@ -845,9 +836,9 @@ void Trainer::build_sparse_tasks() {
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
     std::vector<SparseTask> tasks;
     std::vector<SparseBig> big;
-    std::vector<SortedTask> sorted_tasks;
-    std::vector<int> sorted_fid;
-    std::vector<int2> sorted_meta;
+    std::vector<RareTask> rare_tasks;
+    std::vector<int> rare_fid;
+    std::vector<int2> rare_meta;
     std::vector<int> feat_slot(F_, -1);
     int n_small = 0, n_partial = 0, max_big_bins = 0;
     int f = 0;
@@ -855,8 +846,8 @@ void Trainer::build_sparse_tasks() {
         const long m = cuts_.feature_nnz[f];
         if (!is_table(f)) {
             if (m > 0) {
-                sorted_fid.push_back(f);
-                sorted_meta.push_back(make_int2(h_cut_row_ptr_[f], h_cut_row_ptr_[f + 1] - h_cut_row_ptr_[f]));
+                rare_fid.push_back(f);
+                rare_meta.push_back(make_int2(h_cut_row_ptr_[f], h_cut_row_ptr_[f + 1] - h_cut_row_ptr_[f]));
             }
             ++f;
             continue;
@@ -893,59 +884,66 @@ void Trainer::build_sparse_tasks() {
         feat_slot[big[i].feature] = big[i].cand_slot;
     }
     int next_slot = n_small + (int)big.size();
-    long n_sorted = 0;
-    for (size_t i = 0; i < sorted_fid.size();) {
+    long n_rare = 0;
+    for (size_t i = 0; i < rare_fid.size();) {
         size_t e = i;
         long vals = 0;
-        while (e < sorted_fid.size() && e - i < ((size_t)1 << (32 - kSortedFeatShift)) &&
-               vals + cuts_.feature_nnz[sorted_fid[e]] <= kSortedTile)
-            vals += cuts_.feature_nnz[sorted_fid[e++]];
-        for (size_t q = i; q < e; ++q) feat_slot[sorted_fid[q]] = next_slot;
-        sorted_tasks.push_back(SortedTask{(int)n_sorted, (int)vals, (int)i, (int)(e - i), next_slot++});
-        n_sorted += vals;
+        while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && vals + cuts_.feature_nnz[rare_fid[e]] <= kRareTile)
+            vals += cuts_.feature_nnz[rare_fid[e++]];
+        rare_tasks.push_back(RareTask{(int)n_rare, (int)vals, (int)i, (int)(e - i)});
+        n_rare += vals;
         i = e;
     }
+    // as few rounds of resident workgroups as the tasks per workgroup allow
+    const int n_rt = (int)rare_tasks.size(), per_round = kRareGroups * kRareGroupTiles;
+    const int n_groups = std::min(n_rt, kRareGroups * ((n_rt + per_round - 1) / per_round));
+    sp_.rare_slot = next_slot;
+    for (int t = 0; t < n_rt; ++t)
+        for (int q = 0; q < rare_tasks[t].n_feat; ++q) feat_slot[rare_fid[rare_tasks[t].meta_begin + q]] = next_slot + t % n_groups;
+    next_slot += n_groups;
     // the biggest tasks first: they decide when the level is done
     std::stable_sort(tasks.begin(), tasks.end(),
                      [](const SparseTask &a, const SparseTask &b) { return a.v_end - a.v_begin > b.v_end - b.v_begin; });
     sp_.n_tasks = (int)tasks.size();
     sp_.n_big = (int)big.size();
-    sp_.n_sorted_tasks = (int)sorted_tasks.size();
-    sp_.n_sorted = n_sorted;
+    sp_.n_rare_tasks = n_rt;
+    sp_.n_rare_groups = n_groups;
+    sp_.n_rare = n_rare;
     sp_.n_cand_slots = std::max(1, next_slot);
     sp_.n_partial_slots = n_partial;
     sp_.partial_stride = (size_t)max_big_bins * (size_t)tb_.max_level_nodes;
     SparseTask *d_tasks = dalloc<SparseTask>(tasks.size());
     SparseBig *d_big = dalloc<SparseBig>(big.size());
-    SortedTask *d_sorted = dalloc<SortedTask>(sorted_tasks.size());
-    int *d_sorted_fid = dalloc<int>(sorted_fid.size());
-    int2 *d_sorted_meta = dalloc<int2>(sorted_meta.size());
+    RareTask *d_rare = dalloc<RareTask>(rare_tasks.size());
+    int *d_rare_fid = dalloc<int>(rare_fid.size());
+    int2 *d_rare_meta = dalloc<int2>(rare_meta.size());
     int *d_feat_slot = dalloc<int>(feat_slot.size());
     int *d_fvb = dalloc<int>(fvb.size());
     upload(stream_, d_tasks, tasks.data(), tasks.size());
     upload(stream_, d_big, big.data(), big.size());
-    upload(stream_, d_sorted, sorted_tasks.data(), sorted_tasks.size());
-    upload(stream_, d_sorted_fid, sorted_fid.data(), sorted_fid.size());
-    upload(stream_, d_sorted_meta, sorted_meta.data(), sorted_meta.size());
+    upload(stream_, d_rare, rare_tasks.data(), rare_tasks.size());
+    upload(stream_, d_rare_fid, rare_fid.data(), rare_fid.size());
+    upload(stream_, d_rare_meta, rare_meta.data(), rare_meta.size());
     upload(stream_, d_feat_slot, feat_slot.data(), feat_slot.size());
     upload(stream_, d_fvb, fvb.data(), fvb.size());
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
     sp_.tasks = d_tasks;
     sp_.big = d_big;
-    sp_.sorted_tasks = d_sorted;
-    sp_.sorted_fid = d_sorted_fid;
-    sp_.sorted_meta = d_sorted_meta;
+    sp_.rare_tasks = d_rare;
+    sp_.rare_fid = d_rare_fid;
+    sp_.rare_meta = d_rare_meta;
     sp_.feat_val_begin = d_fvb;
     tb_.feat_slot = d_feat_slot;
     log_info("sparse level pass: %d table tasks, %d features in chunks (%d chunks), %zu features (%ld values) in %d "
-             "sorted tasks, %d candidate slots per node", sp_.n_tasks, sp_.n_big, n_partial, sorted_fid.size(), n_sorted,
-             sp_.n_sorted_tasks, sp_.n_cand_slots);
+             "rare tasks, %d candidate slots per node", sp_.n_tasks, sp_.n_big, n_partial, rare_fid.size(), n_rare,
+             sp_.n_rare_tasks, sp_.n_cand_slots);
 }
 
 void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class) {
     if (sparse_pass_ && level == 0) {
         launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         launch_sparse_gh_refresh(stream_, tb, csr_, sp_, gh, n_class);
+        launch_sparse_row_words(stream_, tb, gh, n_class);
     }
     if (hist_cap_level_ >= 0 && level >= hist_cap_level_) {
         // the level has more nodes than the histogram arena: batches of hist_nodes nodes, each through the whole
@@ -1005,7 +1003,7 @@ void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *g
     if (sparse_pass_) {
         // histogram and split search of the level in one pass; stage-wise driving also gets the per-node histograms
         launch_sparse_level(stream_, tb, csr_, sp_, gh, level, param_.min_child_weight, param_.lambda,
-                            !in_boost_ && tb_.hist_q[0] != nullptr, n_class, level == param_.depth - 1);
+                            !in_boost_ && tb_.hist_q[0] != nullptr, n_class);
     } else if (sparse_)
         launch_hist_csr(stream_, tb, csr_, gh, level, n_class);
     else {
