@@ -370,8 +370,15 @@ void launch_bagging(hipStream_t s, int N, unsigned seed, int *count, GHPair *gh,
 // Tree-building launchers: `tb` is the first buffer set, `n_class` consecutive sets (the class trees of one
 // round) are served by one launch; gradient / prediction pointers address the first of those classes.
 // stats_ready: tb.root_partial already holds the block statistics of gh_class (fused round end)
+struct TreeLeftovers {  // of the tree before: see k_tree_init
+    TreeNode *model = nullptr;  // where its nodes go (nullptr: they are there)
+    float *metric_out = nullptr;  // where its round's metric goes (nullptr: it is there), and what to add up
+    const double *metric_partial = nullptr;
+    int metric_kind = 0, metric_blocks = 0;
+};
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda,
-                      bool stats_ready = false, int n_class = 1);
+                      bool stats_ready = false, int n_class = 1, const TreeLeftovers &left = TreeLeftovers());
+void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left);
 void launch_hist_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
                        int n_class = 1);
 void launch_hist_merge(hipStream_t s, const TreeBuffers &tb, int level, int n_class = 1);
@@ -385,9 +392,9 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
                      int n_class = 1);
 void launch_partition_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class = 1);
 // store_sibling (sparse layout only): keep the derived sibling histograms; nobody reads those of a tree's
-// last level
+// last level. root: level 0 of the dense layout with a complete feature, in place of launch_root_sum
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
-                       bool store_sibling = true);
+                       bool store_sibling = true, bool root = false);
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
                             bool store_sibling = true);
@@ -421,18 +428,17 @@ void launch_nid_rebuild(hipStream_t s, const TreeBuffers &tb, const DenseBins *d
 void launch_predict_in_training(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbins, const CsrBins *cbins,
                                 int lookup_level, float *yp_class, float lr, int n_class = 1,
                                 const float *prune_gamma = nullptr);
-// prediction update + metric + next gradients + their block statistics (tb.root_partial); metric_scratch
+// prediction update + metric partials + next gradients + their block statistics (tb.root_partial); metric_scratch
 // holds row_blocks(n) doubles
 void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbins, const CsrBins *cbins,
                       int lookup_level, int objective, int metric_kind, const float *y, float *yp, float lr,
-                      GHPair *gh, double *metric_scratch, float *metric_out, const float *prune_gamma = nullptr,
-                      unsigned *gh_words = nullptr);
+                      GHPair *gh, double *metric_scratch, const float *prune_gamma = nullptr, unsigned *gh_words = nullptr);
 // words[i] = the gradient word of row i (the pair of a squared or 0/1-label logistic loss in 32 bits, which the
 // histogram kernels decode to the very pair launch_gradient computes; see DenseBins::gh_lane)
 void launch_gh_words(hipStream_t s, int objective, int n, const float *y, const float *yp, unsigned *words);
-// scratch: row_blocks(n) doubles
+// scratch: row_blocks(n) doubles, which launch_metric_final adds up
 void launch_metric(hipStream_t s, int objective_metric, int n, int num_class, const float *y, const float *yp,
-                   double *scratch, float *out);
+                   double *scratch);
 void launch_fill_f32(hipStream_t s, float *p, float v, size_t n);
 void launch_fill_u8(hipStream_t s, uint8_t *p, uint8_t v, size_t n);
 

@@ -182,7 +182,13 @@ void log_the_metric(hipStream_t s, const GBMParam &param, const DataSet &ds, int
         device_alloc_to(d_m, sizeof(float));
         device_alloc_to(d_scratch, sizeof(double) * (size_t)row_blocks(n));
         HIP_CHECK(hipMemcpyAsync(d_y, ds.y.data(), sizeof(float) * (size_t)n, hipMemcpyHostToDevice, s));
-        launch_metric(s, kind, n, n_class, d_y, d_out, d_scratch, d_m);
+        launch_metric(s, kind, n, n_class, d_y, d_out, d_scratch);
+        TreeLeftovers sum;
+        sum.metric_out = d_m;
+        sum.metric_partial = d_scratch;
+        sum.metric_kind = kind;
+        sum.metric_blocks = row_blocks(n);
+        launch_metric_final(s, n, sum);
         float v = 0;
         HIP_CHECK(hipMemcpyAsync(&v, d_m, sizeof(float), hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipStreamSynchronize(s));

@@ -86,7 +86,8 @@ class Trainer {
     bool reorder_allowed() const;
     void reorder_rows();                 // physical re-ordering of the rows by the leaves of the tree just built
     const std::vector<int> &host_perm();  // original row of every physical position (empty: identity)
-    void run_metric(float *slot);
+    void run_metric(float *slot);  // (leaves the last step of the point-wise metrics in left_)
+    void settle();                 // what the last tree has left to do, where no next tree takes it along
     void alloc_tree_buffers();
     template <typename T>
     T *dalloc(size_t count);
@@ -141,6 +142,9 @@ class Trainer {
     int trees_built_ = 0, rounds_done_ = 0, model_cap_trees_ = 0;
     float *d_metric_ = nullptr;
     double *d_metric_scratch_ = nullptr;
+    TreeLeftovers left_;
+    const TreeNode *left_nodes_ = nullptr;  // where left_.model's trees are, and how many
+    size_t left_trees_ = 0;
     std::vector<uint8_t> h_ignored_;
     uint8_t *d_ignored_ = nullptr;
     int cur_class_ = 0;

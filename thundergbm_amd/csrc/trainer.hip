@@ -778,7 +778,8 @@ void Trainer::tree_init(int k) {
     if (!in_boost_) ensure_gh_array();
     cur_class_ = k;
     HIP_CHECK_LAUNCHES("the stages before tree_init");  // gradients, bagging, column sampling, metric, re-ordering
-    launch_tree_init(stream_, set_of(k), d_gh_ + (size_t)k * n_, param_.lambda, next_round_ready_);
+    launch_tree_init(stream_, set_of(k), d_gh_ + (size_t)k * n_, param_.lambda, next_round_ready_, 1, left_);
+    left_ = TreeLeftovers();
     next_round_ready_ = false;
     lookup_level_ = -1;
     nid_materialized_ = false;
@@ -975,7 +976,9 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     mark(PH_HIST, level);
     if (!sparse_pass_) {
         if (!sparse_) launch_hist_merge(stream_, tb, level, n_class);
-        if (level == 0) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
+        // (inside boost() the split search adds up the root itself where a feature is stored in every row)
+        const bool root = level == 0 && in_boost_ && tb.complete_feature >= 0 && !wide_eval_ && !sparse_;
+        if (level == 0 && !root) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         mark(PH_MERGE, level);
         // inside boost() nobody looks at the last level's derived histograms (the stage-wise API keeps them); the
         // last level that fits a capped arena keeps them for the batches of the next one
@@ -984,7 +987,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
                                    !(in_boost_ && level == param_.depth - 1));
         else
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                              !(in_boost_ && level == param_.depth - 1));
+                              !(in_boost_ && level == param_.depth - 1), root);
     }
     if (!update_with_partition(level)) launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
     mark(PH_SPLIT, level);
@@ -1062,8 +1065,11 @@ void Trainer::finish_tree(int k, bool fuse_round_end) {
         // (see gh_array_stale_: inside boost() the next tree may need the words only)
         const bool words_only = in_boost_ && d_gh_words_ != nullptr && tb.complete_feature >= 0;
         launch_round_end(stream_, tb, &bins_, &csr_, lookup_level_, objective_, metric_kind_, d_y_, d_yp_,
-                         param_.learning_rate, words_only ? nullptr : d_gh_, d_metric_scratch_, d_metric_ + rounds_done_,
-                         &param_.gamma, d_gh_words_);
+                         param_.learning_rate, words_only ? nullptr : d_gh_, d_metric_scratch_, &param_.gamma, d_gh_words_);
+        left_.metric_out = d_metric_ + rounds_done_;
+        left_.metric_partial = d_metric_scratch_;
+        left_.metric_kind = metric_kind_;
+        left_.metric_blocks = row_blocks(n_);
         gh_array_stale_ = words_only;
         gh_words_fresh_ = d_gh_words_ != nullptr;
         gh_records_fresh_ = false;  // (the records still hold the finished tree's words)
@@ -1073,8 +1079,10 @@ void Trainer::finish_tree(int k, bool fuse_round_end) {
                                    param_.learning_rate, 1, &param_.gamma);
     }
     TGBM_CHECK(trees_built_ < model_cap_trees_, "more trees built than n_trees * tree_per_rounds");
-    HIP_CHECK(hipMemcpyAsync(d_model_ + (size_t)trees_built_ * tb.n_nodes, tb.nodes,
-                             sizeof(TreeNode) * (size_t)tb.n_nodes, hipMemcpyDeviceToDevice, stream_));
+    left_.model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
+    left_nodes_ = tb.nodes;
+    left_trees_ = 1;
+    if (!in_boost_) settle();
     mark(PH_TREE_END);
     if (profiling_) log_plan(tb);
     ++trees_built_;
@@ -1088,7 +1096,8 @@ void Trainer::build_round_together() {
     TreeBuffers tb = tb_;
     // the K classes share the chip: size every class's histogram items for its share of the workgroup slots
     tb.target_hitems = std::max(4, tb_.target_hitems / K);
-    launch_tree_init(stream_, tb, d_gh_, param_.lambda, false, K);
+    launch_tree_init(stream_, tb, d_gh_, param_.lambda, false, K, left_);
+    left_ = TreeLeftovers();
     lookup_level_ = -1;
     nid_materialized_ = false;
     for (int level = 0; level < param_.depth; ++level) {
@@ -1097,8 +1106,9 @@ void Trainer::build_round_together() {
     }
     launch_predict_in_training(stream_, tb, &bins_, &csr_, lookup_level_, d_yp_, param_.learning_rate, K, &param_.gamma);
     TGBM_CHECK(trees_built_ + K <= model_cap_trees_, "more trees built than n_trees * tree_per_rounds");
-    HIP_CHECK(hipMemcpyAsync(d_model_ + (size_t)trees_built_ * tb.n_nodes, tb.nodes,
-                             sizeof(TreeNode) * (size_t)tb.n_nodes * K, hipMemcpyDeviceToDevice, stream_));
+    left_.model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
+    left_nodes_ = tb.nodes;
+    left_trees_ = (size_t)K;
     mark(PH_TREE_END);
     if (profiling_)
         for (int k = 0; k < K; ++k) log_plan(tb.for_class(k));
@@ -1111,13 +1121,27 @@ void Trainer::run_metric(float *slot) {
     if (objective_ == OBJ_RANK) {
         rank_->metric(metric_kind_, d_yp_, slot);
         rank_order_fresh_ = true;
-    } else
-        launch_metric(stream_, metric_kind_, n_, param_.num_class, d_y_, d_yp_, d_metric_scratch_, slot);
+    } else {
+        launch_metric(stream_, metric_kind_, n_, param_.num_class, d_y_, d_yp_, d_metric_scratch_);
+        left_.metric_out = slot;
+        left_.metric_partial = d_metric_scratch_;
+        left_.metric_kind = metric_kind_;
+        left_.metric_blocks = row_blocks(n_);
+    }
+}
+
+void Trainer::settle() {
+    if (left_.model != nullptr)
+        HIP_CHECK(hipMemcpyAsync(left_.model, left_nodes_, sizeof(TreeNode) * (size_t)tb_.n_nodes * left_trees_,
+                                 hipMemcpyDeviceToDevice, stream_));
+    if (left_.metric_out != nullptr) launch_metric_final(stream_, n_, left_);
+    left_ = TreeLeftovers();
 }
 
 float Trainer::metric() {
     float *slot = d_metric_ + std::min(rounds_done_, std::max(1, param_.n_trees) - 1);
     run_metric(slot);
+    settle();
     float v = 0;
     HIP_CHECK(hipMemcpyAsync(&v, slot, sizeof(float), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipStreamSynchronize(stream_));
@@ -1160,6 +1184,7 @@ void Trainer::boost(int rounds) {
             mark(PH_METRIC);
         }
         if (g_verbose >= 1) {
+            settle();
             float v = 0;
             HIP_CHECK(hipMemcpyAsync(&v, slot, sizeof(float), hipMemcpyDeviceToHost, stream_));
             HIP_CHECK(hipStreamSynchronize(stream_));
@@ -1180,6 +1205,7 @@ void Trainer::boost(int rounds) {
         }
         HIP_CHECK_LAUNCHES("boost");
     }
+    settle();
     in_boost_ = false;
 }
 

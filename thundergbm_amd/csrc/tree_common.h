@@ -12,7 +12,8 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kHistMinChunk = 1024;
 constexpr int kHistBlock = 1024;      // threads per histogram workgroup (they share one LDS histogram)
 
-// Exclusive scan of one int per thread over a 256-thread block; lds needs kWaves ints.
+// Exclusive scan of one int per thread over a block of NW wavefronts; lds needs NW ints.
+template <int NW = kWaves>
 __device__ int block_excl_scan(int v, int *lds, int *total) {
     int lane = lane_id(), w = wave_id();
     int inc = v;
@@ -25,7 +26,7 @@ __device__ int block_excl_scan(int v, int *lds, int *total) {
     __syncthreads();
     int base = 0, tot = 0;
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
+    for (int i = 0; i < NW; ++i) {
         int c = lds[i];
         if (i < w) base += c;
         tot += c;

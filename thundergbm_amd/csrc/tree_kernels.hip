@@ -147,9 +147,8 @@ __global__ void k_bagging_apply(int N, int *__restrict__ count, GHPair *__restri
 }
 
 // Row-blocked reductions: workgroup b owns rows [b * kRowBlock, (b + 1) * kRowBlock), thread t adds its
-// rows t, t + kBlock, ... in that order, then lanes, then wavefronts. Every kernel that produces
-// gradient statistics or metric partials follows this order, so fused and separate passes give the
-// same bits.
+// rows t, t + threads, ... in that order, then lanes, then wavefronts. The kernels that produce metric partials follow
+// this order with as many threads (end_wide), so fused and separate passes give the same bits.
 struct RowStats {
     float g = 0, h = 0, gm = 0, hm = 0, hf = 0;
     __device__ __forceinline__ void add(GHPair v) {
@@ -161,11 +160,10 @@ struct RowStats {
     }
 };
 
-constexpr int kStatsLds = 5 * kWaves;  // floats of LDS that store_block_stats needs
-
-// lds: kStatsLds floats; every thread of the block must call
+// lds: 5 NW floats (NW wavefronts per workgroup); every thread of the block must call
+template <int NW>
 __device__ void store_block_stats(RowStats r, float *lds, GradStats *out) {
-    float *sg = lds, *sh = lds + kWaves, *mg = lds + 2 * kWaves, *mh = lds + 3 * kWaves, *fh = lds + 4 * kWaves;
+    float *sg = lds, *sh = lds + NW, *mg = lds + 2 * NW, *mh = lds + 3 * NW, *fh = lds + 4 * NW;
     float g = wave_sum_f(r.g), h = wave_sum_f(r.h), gm = r.gm, hm = r.hm, hf = r.hf;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -183,7 +181,7 @@ __device__ void store_block_stats(RowStats r, float *lds, GradStats *out) {
     __syncthreads();
     if (threadIdx.x == 0) {
         GradStats o{0, 0, 0, 0, 0};
-        for (int i = 0; i < kWaves; ++i) {
+        for (int i = 0; i < NW; ++i) {
             o.g += sg[i];
             o.h += sh[i];
             o.gmax = fmaxf(o.gmax, mg[i]);
@@ -194,7 +192,8 @@ __device__ void store_block_stats(RowStats r, float *lds, GradStats *out) {
     }
 }
 
-// lds: kWaves doubles
+// lds: NW doubles
+template <int NW>
 __device__ void store_block_sum_d(double acc, double *lds, double *out) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d);
@@ -202,7 +201,7 @@ __device__ void store_block_sum_d(double acc, double *lds, double *out) {
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0;
-        for (int i = 0; i < kWaves; ++i) t += lds[i];
+        for (int i = 0; i < NW; ++i) t += lds[i];
         *out = t;
     }
 }
@@ -210,13 +209,13 @@ __device__ void store_block_sum_d(double acc, double *lds, double *out) {
 // Block sums of (g,h) and block maxima of |g|, h for one tree.
 // Class trees of a round: blockIdx.z selects the class (gradients and outputs are class-major).
 __global__ __launch_bounds__(kBlock) void k_sum_gh(int n, const GHPair *__restrict__ gh, GradStats *__restrict__ out) {
-    __shared__ float lds[kStatsLds];
+    __shared__ float lds[5 * kWaves];
     gh += (size_t)blockIdx.z * n;
     out += (size_t)blockIdx.z * gridDim.x;
     const int r0 = blockIdx.x * kRowBlock, r1 = min(n, r0 + kRowBlock);
     RowStats st;
     for (int i = r0 + threadIdx.x; i < r1; i += kBlock) st.add(gh[i]);
-    store_block_stats(st, lds, out + blockIdx.x);
+    store_block_stats<kWaves>(st, lds, out + blockIdx.x);
 }
 
 // Largest power of two s with rows * (vmax * s + 0.5) < limit; 1 when vmax is 0 or not finite.
@@ -232,7 +231,14 @@ __device__ float pow2_scale(float vmax, int rows, float limit) {
 // ------------------------------------------------------------------------------- tree init
 // Node array initialisation of the reference's Tree::init2 (src/thundergbm/tree.cu:8-39), root sum
 // from the block partials, root segment and the histogram plan of level 0. One workgroup.
-__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda) {
+// What the previous tree has left to do rides along: its finished nodes go into the model before they are reset, and a
+// second workgroup adds up the round's metric (two launches of 4 to 5 us per tree otherwise).
+__device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out);
+__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda, TreeLeftovers left) {
+    if (blockIdx.x == 1) {
+        if (blockIdx.z == 0) metric_final(left.metric_kind, tb_all.n, left.metric_blocks, left.metric_partial, left.metric_out);
+        return;
+    }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const GradStats *__restrict__ block_sums = tb.root_partial;
@@ -262,6 +268,14 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
         // zero the padding bytes too: nodes are written raw into model files
         unsigned *raw = reinterpret_cast<unsigned *>(&nd);
         raw[9] &= 0x000000ffu;  // bytes 37..39 are padding (byte 36 = is_pruned)
+        if (left.model != nullptr) {
+            const int4 *from = reinterpret_cast<const int4 *>(tb.nodes + i);
+            int4 *to = reinterpret_cast<int4 *>(left.model + (size_t)blockIdx.z * nn + i);
+            const int4 v0 = from[0], v1 = from[1], v2 = from[2];
+            to[0] = v0;
+            to[1] = v1;
+            to[2] = v2;
+        }
         tb.nodes[i] = nd;
         tb.seg[i] = make_int2(0, 0);
         if (tb.node_rows != nullptr) tb.node_rows[i] = i == 0 ? tb.n : 0;
@@ -651,8 +665,10 @@ __global__ __launch_bounds__(kBlock) void k_hist_merge(TreeBuffers tb_all, int l
 // order of the rows; every later quantity of a tree (child sums, weights, gains, predictions, the next gradients)
 // derives from it. These kernels replace it by the exact fixed-point total - the same integers in any order - so
 // that a tree does not depend on the row order at all.
-__device__ void set_root_sums(const TreeBuffers &tb, long long G, long long H, float lambda) {
-    GHPair s{(float)((double)G * (double)tb.quant->inv_g), (float)((double)H * (double)tb.quant->inv_h)};
+__device__ __forceinline__ GHPair root_sums(const TreeBuffers &tb, long long G, long long H) {
+    return {(float)((double)G * (double)tb.quant->inv_g), (float)((double)H * (double)tb.quant->inv_h)};
+}
+__device__ __forceinline__ void set_root_sums(const TreeBuffers &tb, GHPair s, float lambda) {
     TreeNode &root = tb.nodes[0];
     root.sum_gh_pair = s;
     root.base_weight = -s.g / (s.h + lambda);
@@ -682,7 +698,7 @@ __global__ __launch_bounds__(kBlock) void k_root_sum_bins(TreeBuffers tb_all, fl
             g += s_g[i];
             hh += s_h[i];
         }
-        set_root_sums(tb, g, hh, lambda);
+        set_root_sums(tb, root_sums(tb, g, hh), lambda);
     }
 }
 
@@ -738,7 +754,7 @@ __global__ __launch_bounds__(kBlock) void k_root_sum_final(TreeBuffers tb_all, i
         g += s_g[i];
         hh += s_h[i];
     }
-    set_root_sums(tb, g, hh, lambda);
+    set_root_sums(tb, root_sums(tb, g, hh), lambda);
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_bytes(const uint8_t *__restrict__ v, size_t n, uint8_t value,
@@ -987,7 +1003,9 @@ __global__ __launch_bounds__(kBlock) void k_part_count_csr(TreeBuffers tb_all, C
 // SUB (sparse layout, whose histograms are not merged from work-item partials): the node of a pair that
 // was not built from rows is derived here as parent - built while it is scanned, and stored for the next
 // level, instead of by a separate pass over the (very long) histograms.
-template <bool SUB>
+// ROOT (level 0, a feature stored in every row): the node's sums are that feature's bins added up, by every wavefront
+// for itself.
+template <bool SUB, bool ROOT = false>
 __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int level, float mcw, float lambda,
                                                       bool store_sibling) {
 #pragma clang fp contract(off)
@@ -1005,9 +1023,22 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
         b_begin = tb.pack_begin[pack];
         b_end = tb.pack_begin[pack + 1];
     }
-    const GHPair S = nd.sum_gh_pair;
+    GHPair S = nd.sum_gh_pair;
     longlong2 *h = hist_q + (size_t)x_in * tb.n_bins;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
+    if constexpr (ROOT) {
+        long long g = 0, hh = 0;
+        const int b0 = tb.cut_row_ptr[tb.complete_feature], b1 = tb.cut_row_ptr[tb.complete_feature + 1];
+        for (int b = b0 + lane; b < b1; b += 64) {
+            const longlong2 v = h[b];
+            g += v.x;
+            hh += v.y;
+        }
+        g = wave_sum_ll(g);
+        hh = wave_sum_ll(hh);
+        S = root_sums(tb, g, hh);
+        if (pack == 0 && lane == 0) set_root_sums(tb, S, lambda);
+    }
     // SUB: is this node the sibling of the pair's built node?
     const longlong2 *h_par = nullptr, *h_built = nullptr;
     if (SUB && level > 0 && active && !tb.singles(level)) {
@@ -1798,6 +1829,11 @@ struct TreeEndArgs {
     unsigned *gh_words;  // MODE 2: where the rows' gradient words go (word_from_row; nullptr: nowhere)
 };
 
+// Threads per row block. While the workgroups fit the chip at once, four rows per thread make every step of the chain list
+// position -> row -> bin -> leaf -> prediction one round of loads (500 k rows: 28 us with 256 threads, 14 with 1024);
+// beyond that the registers of the 1024 cost residency (10 M rows: 74 and 128 us).
+constexpr int kEndWide = 1024;
+bool end_wide(int n) { return row_blocks(n) <= 512; }
 constexpr int kEndInline = 8;                        // shorter sub-ranges are handled by the finding thread
 constexpr int kEndListCap = kRowBlock / kEndInline;  // so at most this many longer ones exist per block
 
@@ -1897,19 +1933,19 @@ __global__ __launch_bounds__(kBlock) void k_end_bounds(TreeBuffers tb_all, int l
 }
 
 // The row-ordered part of the end of a tree: s_leaf holds the node of every row of the block.
-template <int MODE>
+template <int MODE, int BLK>
 __device__ __forceinline__ void tree_end_rows(const TreeBuffers &tb, const TreeEndArgs &a, const short *s_leaf, int r0, int r1) {
-    __shared__ float s_f[kStatsLds];
-    __shared__ double s_d[kWaves];
+    __shared__ float s_f[5 * BLK / 64];
+    __shared__ double s_d[BLK / 64];
     constexpr int U = 4;
     if (MODE == 0) {
-        for (int i = r0 + threadIdx.x; i < r1; i += kBlock) {
+        for (int i = r0 + threadIdx.x; i < r1; i += BLK) {
             const int x = s_leaf[i - r0];
             if (x >= 0) tb.nid[i] = x;
         }
         return;
     }
-    // rows in order; thread t takes rows t, t + kBlock, ... (the order every row-blocked reduction uses)
+    // rows in order; thread t takes rows t, t + BLK, ... (the order every row-blocked reduction uses)
     const float *__restrict__ y = a.y;
     float *__restrict__ yp = a.yp;
     GHPair *__restrict__ gh = a.gh;
@@ -1917,12 +1953,12 @@ __device__ __forceinline__ void tree_end_rows(const TreeBuffers &tb, const TreeE
     RowStats st;
     double acc = 0;
     float accf = 0;
-    for (int i0 = r0 + threadIdx.x; i0 < r1; i0 += kBlock * U) {
+    for (int i0 = r0 + threadIdx.x; i0 < r1; i0 += BLK * U) {
         float p[U], w[U], yi[U];
         bool ok[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int i = i0 + u * kBlock;
+            const int i = i0 + u * BLK;
             ok[u] = i < r1;
             const int x = ok[u] ? s_leaf[i - r0] : -1;
             p[u] = ok[u] ? yp[i] : 0.f;
@@ -1934,7 +1970,7 @@ __device__ __forceinline__ void tree_end_rows(const TreeBuffers &tb, const TreeE
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (!ok[u]) continue;
-            const int i = i0 + u * kBlock;
+            const int i = i0 + u * BLK;
             yp[i] = p[u];
             if (MODE == 2) {
                 metric_row(a.metric_kind, tb.n, 1, i, yi[u], yp, p[u], acc, accf);
@@ -1946,35 +1982,35 @@ __device__ __forceinline__ void tree_end_rows(const TreeBuffers &tb, const TreeE
         }
     }
     if (MODE == 2) {
-        store_block_stats(st, s_f, a.stats + blockIdx.x);
+        store_block_stats<BLK / 64>(st, s_f, a.stats + blockIdx.x);
         acc += (double)accf;
-        store_block_sum_d(acc, s_d, a.metric_partial + blockIdx.x);
+        store_block_sum_d<BLK / 64>(acc, s_d, a.metric_partial + blockIdx.x);
     }
 }
 
 
-template <int MODE, bool SPARSE>
-__global__ __launch_bounds__(kBlock) void k_tree_end(TreeBuffers tb_all, DenseBins dbins, CsrBins cbins, TreeEndArgs a) {
+template <int MODE, bool SPARSE, int BLK>
+__global__ __launch_bounds__(BLK) void k_tree_end(TreeBuffers tb_all, DenseBins dbins, CsrBins cbins, TreeEndArgs a) {
     __shared__ short s_leaf[kRowBlock];  // node of every row of the block (depth <= 14: ids below 2^15), -1: none
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     if (MODE == 1) a.yp += (size_t)blockIdx.z * tb.n;  // class-major predictions
     __shared__ int s_list[kEndListCap][3];  // node, first and one-past-last list position
     __shared__ int s_split[kEndListCap];    // -1: the rows stay in the node; else feature | bin << 16 | default_right << 24
     __shared__ int s_off[kEndListCap];
-    __shared__ int s_scan[kWaves];
+    __shared__ int s_scan[BLK / 64];
     __shared__ int s_n;
     const int r0 = blockIdx.x * kRowBlock, r1 = min(tb.n, r0 + kRowBlock);
     constexpr int U = 4;
     if (tb.nid16 != nullptr) {
         // sparse level pass: the row -> node map is kept per row, nothing to look up
-        for (int i = threadIdx.x; i < kRowBlock; i += kBlock) s_leaf[i] = r0 + i < r1 ? (short)tb.nid16[r0 + i] : (short)-1;
+        for (int i = threadIdx.x; i < kRowBlock; i += BLK) s_leaf[i] = r0 + i < r1 ? (short)tb.nid16[r0 + i] : (short)-1;
     } else {
-    for (int i = threadIdx.x; i < kRowBlock; i += kBlock) s_leaf[i] = -1;
+    for (int i = threadIdx.x; i < kRowBlock; i += BLK) s_leaf[i] = -1;
     if (threadIdx.x == 0) s_n = 0;
     __syncthreads();
     const int n_holders = (1 << tb.depth) - 1;  // nodes of the levels that own row lists
     const int *b_lo = tb.end_bound + (size_t)blockIdx.x * n_holders, *b_hi = b_lo + n_holders;
-    for (int x = threadIdx.x; x < n_holders; x += kBlock) {
+    for (int x = threadIdx.x; x < n_holders; x += BLK) {
         const int pa = b_lo[x], pb = b_hi[x];
         if (pb <= pa) continue;
         const TreeNode &nd = tb.nodes[x];
@@ -2001,22 +2037,22 @@ __global__ __launch_bounds__(kBlock) void k_tree_end(TreeBuffers tb_all, DenseBi
     // loads in flight instead of one dependent chain per sub-range): s_off = exclusive scan of the lengths.
     const int n_list = s_n;
     int total = 0;
-    for (int base = 0; base < n_list; base += kBlock) {
+    for (int base = 0; base < n_list; base += BLK) {
         const int e = base + threadIdx.x;
         const int len = e < n_list ? s_list[e][2] - s_list[e][1] : 0;
         int tot;
-        const int ex = block_excl_scan(len, s_scan, &tot);
+        const int ex = block_excl_scan<BLK / 64>(len, s_scan, &tot);
         if (e < n_list) s_off[e] = total + ex;
         total += tot;
     }
     __syncthreads();
-    for (int j0 = threadIdx.x; j0 < total; j0 += kBlock * U) {
+    for (int j0 = threadIdx.x; j0 < total; j0 += BLK * U) {
         // (every load is unconditional - entries past the end repeat the last one and are skipped when the results
         // are stored -, so a thread's four list entries, then its four bins, are in flight together)
         int node[U], row[U], split[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = min(j0 + u * kBlock, total - 1);
+            const int j = min(j0 + u * BLK, total - 1);
             int lo = 0, hi = n_list;  // last entry with s_off <= j
             while (hi - lo > 1) {
                 const int mid = (lo + hi) / 2;
@@ -2032,7 +2068,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_end(TreeBuffers tb_all, DenseBi
         if (SPARSE || dbins.bin_bytes == 2 || dbins.feat_col != nullptr) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (j0 + u * kBlock >= total) continue;
+                if (j0 + u * BLK >= total) continue;
                 s_leaf[row[u] - r0] =
                     split[u] >= 0 ? end_child_of<SPARSE>(tb, dbins, cbins, tb.nodes[node[u]], row[u]) : node[u];
             }
@@ -2043,7 +2079,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_end(TreeBuffers tb_all, DenseBi
                 bin[u] = dbins.col[(size_t)(split[u] >= 0 ? split[u] & 0xffff : 0) * dbins.col_stride + row[u]];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (j0 + u * kBlock >= total) continue;
+                if (j0 + u * BLK >= total) continue;
                 int leaf = node[u];
                 if (split[u] >= 0) {
                     const bool right = bin[u] == kMissingBin ? (split[u] >> 24) != 0 : bin[u] >= ((split[u] >> 16) & 0xff);
@@ -2055,7 +2091,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_end(TreeBuffers tb_all, DenseBi
     }
     }  // row lists
     __syncthreads();
-    tree_end_rows<MODE>(tb, a, s_leaf, r0, r1);
+    tree_end_rows<MODE, BLK>(tb, a, s_leaf, r0, r1);
 }
 
 // ---------------------------------------------------------------------------------- metric
@@ -2084,15 +2120,16 @@ __device__ __forceinline__ void metric_row(int kind, int n, int K, int i, float 
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_metric_partial(int kind, int n, int K, const float *__restrict__ y,
+template <int BLK>
+__global__ __launch_bounds__(BLK) void k_metric_partial(int kind, int n, int K, const float *__restrict__ y,
                                                           const float *__restrict__ yp, double *__restrict__ out) {
-    __shared__ double sd[kWaves];
+    __shared__ double sd[BLK / 64];
     double acc = 0;
     float accf = 0;
     const int r0 = blockIdx.x * kRowBlock, r1 = min(n, r0 + kRowBlock);
-    for (int i = r0 + threadIdx.x; i < r1; i += kBlock) metric_row(kind, n, K, i, y[i], yp, yp[i], acc, accf);
+    for (int i = r0 + threadIdx.x; i < r1; i += BLK) metric_row(kind, n, K, i, y[i], yp, yp[i], acc, accf);
     acc += (double)accf;
-    store_block_sum_d(acc, sd, out + blockIdx.x);
+    store_block_sum_d<BLK / 64>(acc, sd, out + blockIdx.x);
 }
 
 // The counting metrics (kind 1 and 2) do not depend on the order of their additions, so their partials come from
@@ -2117,8 +2154,7 @@ __global__ __launch_bounds__(kCountBlock) void k_metric_count(int kind, int n, i
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_metric_final(int kind, int n, int n_blocks, const double *__restrict__ in,
-                                                        float *__restrict__ out) {
+__device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out) {
     __shared__ double sd[kWaves];
     double acc = 0;
     for (int i = threadIdx.x; i < n_blocks; i += kBlock) acc += in[i];
@@ -2136,6 +2172,11 @@ __global__ __launch_bounds__(kBlock) void k_metric_final(int kind, int n, int n_
             out[0] = kind == 1 ? 1.f - a : a;
         }
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_metric_final(int kind, int n, int n_blocks, const double *__restrict__ in,
+                                                        float *__restrict__ out) {
+    metric_final(kind, n, n_blocks, in, out);
 }
 
 int grid_for(size_t n, int cap = 4096) {
@@ -2177,10 +2218,10 @@ void launch_bagging(hipStream_t s, int N, unsigned seed, int *count, GHPair *gh,
 // are served by the same launch through blockIdx.z; gradient and prediction pointers address the
 // first of those classes.
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda, bool stats_ready,
-                      int n_class) {
+                      int n_class, const TreeLeftovers &left) {
     if (!stats_ready)  // n_grad_blocks == row_blocks(n)
         k_sum_gh<<<dim3(tb.n_grad_blocks, 1, n_class), kBlock, 0, s>>>(tb.n, gh_class, tb.root_partial);
-    k_tree_init<<<dim3(1, 1, n_class), kBlock, 0, s>>>(tb, lambda);
+    k_tree_init<<<dim3(left.metric_out != nullptr ? 2 : 1, 1, n_class), kBlock, 0, s>>>(tb, lambda, left);
     if (tb.nid16 != nullptr) {
         // sparse level pass: every row starts in the root (the n_class maps lie back to back)
         const size_t words = ((size_t)tb.n + 2) / 2 * (size_t)n_class;
@@ -2355,9 +2396,10 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
 }
 
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
-                       bool store_sibling) {
+                       bool store_sibling, bool root) {
     dim3 grid((tb.n_packs + kWaves - 1) / kWaves, tb.nodes_served(level), n_class);
-    if (tb.sparse) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
+    if (root) k_eval_split<false, true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
+    else if (tb.sparse) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
 }
 
@@ -2389,9 +2431,12 @@ template <bool SPARSE>
 static void tree_end_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &d, const CsrBins &c, int mode,
                             const TreeEndArgs &a, int n_class) {
     const dim3 grid(row_blocks(tb.n), 1, n_class);
-    if (mode == 0) k_tree_end<0, SPARSE><<<grid, kBlock, 0, s>>>(tb, d, c, a);
-    else if (mode == 1) k_tree_end<1, SPARSE><<<grid, kBlock, 0, s>>>(tb, d, c, a);
-    else k_tree_end<2, SPARSE><<<grid, kBlock, 0, s>>>(tb, d, c, a);
+    // (mode 0 has nothing per row to wait for)
+    if (mode == 0) k_tree_end<0, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
+    else if (mode == 1 && end_wide(tb.n)) k_tree_end<1, SPARSE, kEndWide><<<grid, kEndWide, 0, s>>>(tb, d, c, a);
+    else if (mode == 1) k_tree_end<1, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
+    else if (end_wide(tb.n)) k_tree_end<2, SPARSE, kEndWide><<<grid, kEndWide, 0, s>>>(tb, d, c, a);
+    else k_tree_end<2, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
 }
 
 static void tree_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbins, const CsrBins *cbins, int mode,
@@ -2427,8 +2472,7 @@ void launch_predict_in_training(hipStream_t s, const TreeBuffers &tb, const Dens
 
 void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbins, const CsrBins *cbins,
                       int lookup_level, int objective, int metric_kind, const float *y, float *yp, float lr,
-                      GHPair *gh, double *metric_scratch, float *metric_out, const float *prune_gamma,
-                      unsigned *gh_words) {
+                      GHPair *gh, double *metric_scratch, const float *prune_gamma, unsigned *gh_words) {
     TreeEndArgs a{};
     a.gh_words = gh_words;
     a.with_prune = prune_gamma != nullptr;
@@ -2443,7 +2487,10 @@ void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbi
     a.stats = tb.root_partial;
     a.metric_partial = metric_scratch;
     tree_end(s, tb, dbins, cbins, 2, a);
-    k_metric_final<<<1, kBlock, 0, s>>>(metric_kind, tb.n, row_blocks(tb.n), metric_scratch, metric_out);
+}
+
+void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left) {
+    k_metric_final<<<1, kBlock, 0, s>>>(left.metric_kind, n, left.metric_blocks, left.metric_partial, left.metric_out);
 }
 
 void launch_gh_words(hipStream_t s, int objective, int n, const float *y, const float *yp, unsigned *words) {
@@ -2451,14 +2498,13 @@ void launch_gh_words(hipStream_t s, int objective, int n, const float *y, const 
     k_gh_words<<<std::min(4096, (n + kBlock - 1) / kBlock), kBlock, 0, s>>>(objective, n, y, yp, words);
 }
 
-void launch_metric(hipStream_t s, int kind, int n, int num_class, const float *y, const float *yp, double *scratch,
-                   float *out) {
+void launch_metric(hipStream_t s, int kind, int n, int num_class, const float *y, const float *yp, double *scratch) {
     int blocks = row_blocks(n);  // scratch: one double per block
     if (kind == 0)
-        k_metric_partial<<<blocks, kBlock, 0, s>>>(kind, n, num_class, y, yp, scratch);
+        end_wide(n) ? k_metric_partial<kEndWide><<<blocks, kEndWide, 0, s>>>(kind, n, num_class, y, yp, scratch)
+                    : k_metric_partial<kBlock><<<blocks, kBlock, 0, s>>>(kind, n, num_class, y, yp, scratch);
     else
         k_metric_count<<<blocks, kCountBlock, 0, s>>>(kind, n, num_class, y, yp, scratch);
-    k_metric_final<<<1, kBlock, 0, s>>>(kind, n, blocks, scratch, out);
 }
 
 }  // namespace tgbm
