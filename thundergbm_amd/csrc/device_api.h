@@ -54,6 +54,10 @@ constexpr int kCsrHeadBins = 4864;  // head slots of the sparse histogram: 2 x 8
 // 500 k x 2000 regression builds a tree in 1.90 instead of 2.00 ms.
 constexpr int kHistFlushRows = 8192;
 constexpr int kHistFlushRowsInt = 32768;
+// Data of so few rows is trained on by the launches of launch_small_level, trees of so many levels at most.
+constexpr int kSmallRows = 16384;
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallDepth = 10;
 constexpr int kRowBlock = 4096;    // rows owned by one workgroup of the row-ordered passes and reductions
 inline int row_blocks(int n) { return n <= 0 ? 1 : (n + kRowBlock - 1) / kRowBlock; }
 
@@ -375,6 +379,7 @@ struct TreeLeftovers {  // of the tree before: see k_tree_init
     float *metric_out = nullptr;  // where its round's metric goes (nullptr: it is there), and what to add up
     const double *metric_partial = nullptr;
     int metric_kind = 0, metric_blocks = 0;
+    bool small = false;  // (of the tree that begins) the rows' nodes are kept in tb.nid
 };
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda,
                       bool stats_ready = false, int n_class = 1, const TreeLeftovers &left = TreeLeftovers());
@@ -392,17 +397,27 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
                      int n_class = 1);
 void launch_partition_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class = 1);
 // store_sibling (sparse layout only): keep the derived sibling histograms; nobody reads those of a tree's
-// last level. root: level 0 of the dense layout with a complete feature, in place of launch_root_sum
+// last level. derive: the nodes that were not built are parent - built (always so in the sparse layout). root: level 0 of the dense layout with a complete feature, in place of launch_root_sum
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
-                       bool store_sibling = true, bool root = false);
+                       bool store_sibling = true, bool root = false, bool derive = false);
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
-                            bool store_sibling = true);
+                            bool store_sibling = true, bool derive = false);
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class = 1);
 // Dense layout: the rows of a level's split nodes move into the children's lists. update: the nodes' best candidates have
 // not been applied to the tree yet (launch_best_update); it happens here.
 void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
                             float rt_eps, float lambda, int n_class = 1);
+// Dense layout, few rows: the level's splits, the children's lists and the histograms of the next level's built nodes in one
+// launch. The split search of the next level then derives the siblings (launch_eval_split with derive).
+bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins);
+void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
+                        float lambda, int n_class = 1);
+// The end of a tree whose rows' nodes are in tb.nid: prunes the tree into `model` (n_class trees back to back; tb.nodes
+// stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics.
+void launch_small_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, TreeNode *model, float gamma, float *yp,
+                      float lr, int n_class = 1, const float *y = nullptr, int objective = 0, int metric_kind = 0,
+                      GHPair *gh = nullptr, double *metric_scratch = nullptr, unsigned *gh_words = nullptr);
 // Sparse level pass (tb.nid16 set): split search of a level (candidates into tb.cand, one slot per task / big
 // feature; launch_best_update follows) and the row -> node update. dump_hist: also store the (node, bin) tables
 // into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q).

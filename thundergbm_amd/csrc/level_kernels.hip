@@ -62,6 +62,80 @@ __device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level
     return out;
 }
 
+// The node's best candidate into *s_cand (larger |score|, then the smaller bin index), false: it has none. s_abs, s_idx: NW
+// entries; every thread of the workgroup calls.
+template <int NW>
+__device__ __forceinline__ bool pick_candidate(const TreeBuffers &tb, int x_in, bool valid, float *s_abs, int *s_idx,
+                                               SplitCand *s_cand) {
+            float a_best = -1.f;
+            int i_best = 0x7fffffff;
+            SplitCand best;
+            best.score = 0.f;
+            best.index = 0x7fffffff;
+            best.miss = best.left = GHPair{0, 0};
+            best.feature = best.bin = 0;
+            if (valid)
+                for (int p = threadIdx.x; p < tb.n_packs; p += NW * 64) {
+                    const SplitCand c = tb.cand[(size_t)x_in * tb.n_packs + p];
+                    const float a = fabsf(c.score);
+                    // (index 0x7fffffff: a wavefront whose features have no bins)
+                    const bool better = c.index != 0x7fffffff && (a > a_best || (a == a_best && c.index < i_best));
+                    a_best = better ? a : a_best;
+                    i_best = better ? c.index : i_best;
+                    best.score = better ? c.score : best.score;
+                    best.miss.g = better ? c.miss.g : best.miss.g;
+                    best.miss.h = better ? c.miss.h : best.miss.h;
+                    best.left.g = better ? c.left.g : best.left.g;
+                    best.left.h = better ? c.left.h : best.left.h;
+                    best.feature = better ? c.feature : best.feature;
+                    best.bin = better ? c.bin : best.bin;
+                }
+            // larger |score|, then the smaller bin index; bin indices are distinct
+            float win = a_best;
+            int win_idx = i_best;
+    #pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+                const float oa = __shfl_xor(win, d);
+                const int oi = __shfl_xor(win_idx, d);
+                if (oa > win || (oa == win && oi < win_idx)) {
+                    win = oa;
+                    win_idx = oi;
+                }
+            }
+            if (lane_id() == 0) {
+                s_abs[wave_id()] = win;
+                s_idx[wave_id()] = win_idx;
+            }
+            __syncthreads();
+    #pragma unroll
+            for (int i = 0; i < NW; ++i)
+                if (s_abs[i] > win || (s_abs[i] == win && s_idx[i] < win_idx)) {
+                    win = s_abs[i];
+                    win_idx = s_idx[i];
+                }
+            const bool found = win_idx != 0x7fffffff;
+            if (found && a_best == win && i_best == win_idx) {
+                best.index = i_best;
+                *s_cand = best;
+            }
+            __syncthreads();
+    return found;
+}
+
+__device__ __forceinline__ void apply_candidate(const TreeBuffers &tb, int x, int x_in, const TreeNode &node, bool found,
+                                                const SplitCand &c, float rt_eps, float lambda) {
+    if (!node.is_valid) {
+        SplitPoint z{};
+        z.nid = -1;
+        z.split_fea_id = -1;
+        tb.sp[x_in] = z;
+    } else if (!found) {
+        no_split(tb, x, x_in);
+    } else {
+        apply_split(tb, x, x_in, node, c, c.feature, c.bin, tb.cut_val[c.index - (c.bin != 0 ? 1 : 0)], rt_eps, lambda);
+    }
+}
+
 // UPDATE: the nodes' candidates are fresh from the split search; else the tree has been updated already.
 // A row goes right if its bin is not below the split bin, or if it has no value of the feature and the default says so
 // (hist_tree_builder_single.cu:986-1011).
@@ -98,58 +172,7 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     int f = 0, sbid = 0;
     if (UPDATE) {
         const bool valid = node.is_valid;
-        float a_best = -1.f;
-        int i_best = 0x7fffffff;
-        SplitCand best;
-        best.score = 0.f;
-        best.index = 0x7fffffff;
-        best.miss = best.left = GHPair{0, 0};
-        best.feature = best.bin = 0;
-        if (valid)
-            for (int p = threadIdx.x; p < tb.n_packs; p += kBlock) {
-                const SplitCand c = tb.cand[(size_t)x_in * tb.n_packs + p];
-                const float a = fabsf(c.score);
-                // (index 0x7fffffff: a wavefront whose features have no bins)
-                const bool better = c.index != 0x7fffffff && (a > a_best || (a == a_best && c.index < i_best));
-                a_best = better ? a : a_best;
-                i_best = better ? c.index : i_best;
-                best.score = better ? c.score : best.score;
-                best.miss.g = better ? c.miss.g : best.miss.g;
-                best.miss.h = better ? c.miss.h : best.miss.h;
-                best.left.g = better ? c.left.g : best.left.g;
-                best.left.h = better ? c.left.h : best.left.h;
-                best.feature = better ? c.feature : best.feature;
-                best.bin = better ? c.bin : best.bin;
-            }
-        // larger |score|, then the smaller bin index; bin indices are distinct
-        float win = a_best;
-        int win_idx = i_best;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const float oa = __shfl_xor(win, d);
-            const int oi = __shfl_xor(win_idx, d);
-            if (oa > win || (oa == win && oi < win_idx)) {
-                win = oa;
-                win_idx = oi;
-            }
-        }
-        if (lane_id() == 0) {
-            s_abs[wave_id()] = win;
-            s_idx[wave_id()] = win_idx;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kWaves; ++i)
-            if (s_abs[i] > win || (s_abs[i] == win && s_idx[i] < win_idx)) {
-                win = s_abs[i];
-                win_idx = s_idx[i];
-            }
-        found = win_idx != 0x7fffffff;
-        if (found && a_best == win && i_best == win_idx) {
-            best.index = i_best;
-            s_cand = best;
-        }
-        __syncthreads();
+        found = pick_candidate<kWaves>(tb, x_in, valid, s_abs, s_idx, &s_cand);
         splits = found && fabsf(s_cand.score) > rt_eps;
         if (splits) {
             f = s_cand.feature;
@@ -167,18 +190,7 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     }
     // (the tree's own stores come last: nothing of this workgroup waits for them)
     auto update = [&] {
-        if (!UPDATE || item != it.first || threadIdx.x != 0) return;
-        if (!node.is_valid) {
-            SplitPoint z{};
-            z.nid = -1;
-            z.split_fea_id = -1;
-            tb.sp[x_in] = z;
-        } else if (!found) {
-            no_split(tb, x, x_in);
-        } else {
-            const SplitCand c = s_cand;
-            apply_split(tb, x, x_in, node, c, c.feature, c.bin, tb.cut_val[c.index - (c.bin != 0 ? 1 : 0)], rt_eps, lambda);
-        }
+        if (UPDATE && item == it.first && threadIdx.x == 0) apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
     };
     if (!splits) {
         if (threadIdx.x == 0) tb.pitem_nleft[item] = 0;
@@ -330,6 +342,184 @@ __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, in
     }
 }
 
+// Few rows (kSmallRows): a level in one launch instead of count, scatter, histogram and merge, which take 5 to 7 us each with
+// nothing to do. A workgroup owns a node and a feature block: it picks the node's split, decides for every row, lays the
+// children's lists down and adds up the histogram of the child with fewer rows, whose list it has in LDS, right at the
+// tree's scales; the split search derives the sibling (k_eval_split<true>). Every block of a node repeats the split, the
+// first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
+// (k_small_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
+// A level of 10 k x 8: 28 -> 14 us with its split search.
+// The sums are those of k_hist_dense, whose work items count at a scale that hangs on the node's rows only.
+constexpr int kSmallWaves = kSmallBlock / 64;
+constexpr int kSmallSteps = kSmallRows / kSmallBlock;
+static_assert(kSmallRows / 2 <= kHistFlushRows, "the built child's packed sums are never drained");
+static_assert(kSmallRows <= 1 << 16 && kSmallSteps * kSmallWaves == 256, "16-bit row ids, four step counts per lane");
+
+template <int LPR, bool BIN16>
+__global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
+                                                            int level, float rt_eps, float lambda) {
+    extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
+    __shared__ SplitCand s_cand;
+    __shared__ float s_abs[kSmallWaves];
+    __shared__ int s_idx[kSmallWaves];
+    __shared__ int s_left[kSmallSteps * kSmallWaves + 1];  // rows that go left: per step and wavefront, then before them
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    gh += (size_t)blockIdx.z * tb.n;
+    unsigned short *s_rows = reinterpret_cast<unsigned short *>(lds + tb.max_block_bins);
+    const int fb = blockIdx.x, x_in = blockIdx.y, x = (1 << level) - 1 + x_in;
+    const int lane = lane_id(), w = wave_id();
+    const TreeNode node = tb.nodes[x];
+    const int2 sg = level == 0 ? make_int2(0, tb.n) : tb.seg[x];
+    const int len = sg.y - sg.x, steps = (len + kSmallBlock - 1) / kSmallBlock;
+    const int *__restrict__ ridx = tb.list(level);
+    int row[kSmallSteps];
+#pragma unroll
+    for (int k = 0; k < kSmallSteps; ++k) {
+        row[k] = 0;
+        if (k < steps) {
+            const int pos = min(sg.x + k * kSmallBlock + (int)threadIdx.x, sg.y - 1);
+            row[k] = level == 0 ? pos : ridx[pos];
+        }
+    }
+    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
+    for (int i = threadIdx.x; i < nb; i += kSmallBlock) lds[i] = 0ull;
+    const bool found = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_abs, s_idx, &s_cand);
+    const bool splits = found && fabsf(s_cand.score) > rt_eps;
+    const bool first = fb == 0 && threadIdx.x == 0;
+    if (!splits) {
+        if (first) {
+            tb.node_nleft[x_in] = 0;
+            if (node.lch_index >= 0) tb.seg[node.lch_index] = tb.seg[node.rch_index] = make_int2(0, 0);
+            tb.hpair_built[x_in] = -1;
+            apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
+        }
+        return;
+    }
+    const int f = s_cand.feature;
+    const int sbid = tb.split_bin != nullptr ? s_cand.bin : (int)(unsigned char)s_cand.bin;
+    const bool dr = s_cand.score < 0;
+    int c = f, lo = 0, span = BIN16 ? kMissingBin16 : kMissingBin;
+    if (!BIN16 && bins.feat_col != nullptr) {  // (see k_split_count)
+        c = bins.feat_col[f];
+        lo = bins.feat_lo[f];
+        span = tb.cut_row_ptr[f + 1] - tb.cut_row_ptr[f];
+    }
+    const uint8_t *column = bins.col + (size_t)c * bins.col_stride * (BIN16 ? 2 : 1);
+    int b[kSmallSteps];
+#pragma unroll
+    for (int k = 0; k < kSmallSteps; ++k)
+        if (k < steps) b[k] = BIN16 ? (int)reinterpret_cast<const uint16_t *>(column)[row[k]] : (int)column[row[k]];
+    unsigned long long left_mask[kSmallSteps];  // (wave-uniform)
+#pragma unroll
+    for (int k = 0; k < kSmallSteps; ++k) {
+        left_mask[k] = 0;
+        if (k < steps) {
+            const int t = b[k] - lo;
+            const bool right = ((unsigned)t >= (unsigned)span) ? dr : (t >= sbid);
+            left_mask[k] = __ballot(!right && k * kSmallBlock + (int)threadIdx.x < len);
+        }
+        if (lane == 0) s_left[k * kSmallWaves + w] = __popcll(left_mask[k]);
+    }
+    __syncthreads();
+    if (w == 0) {
+        int v[4], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v[q] = s_left[lane * 4 + q];
+            sum += v[q];
+        }
+        int upto = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(upto, d);
+            if (lane >= d) upto += o;
+        }
+        int before = upto - sum;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            s_left[lane * 4 + q] = before;
+            before += v[q];
+        }
+        if (lane == 63) s_left[kSmallSteps * kSmallWaves] = before;
+    }
+    __syncthreads();
+    const int nleft = s_left[kSmallSteps * kSmallWaves], nright = len - nleft;
+    // the child with fewer rows is built from them (ties: the left one, as hist_tree_builder_single.cu:466-467)
+    const bool build_left = nleft <= nright;
+    const int m = build_left ? nleft : nright;
+    int *__restrict__ ridx_next = tb.list(level + 1);
+#pragma unroll
+    for (int k = 0; k < kSmallSteps; ++k) {
+        const int i = k * kSmallBlock + (int)threadIdx.x;
+        if (k < steps && i < len) {
+            const int lefts = s_left[k * kSmallWaves + w] + lanes_below(left_mask[k]);
+            const bool left = (left_mask[k] >> lane & 1ull) != 0;
+            const int at = left ? lefts : i - lefts;  // in the child's list
+            if (left == build_left) s_rows[at] = (unsigned short)row[k];
+            if (fb == 0) {
+                ridx_next[sg.x + (left ? at : nleft + at)] = row[k];
+                tb.nid[row[k]] = left ? node.lch_index : node.rch_index;
+            }
+        }
+    }
+    __syncthreads();
+    const QuantCtl quant = *tb.quant;
+    const int h_bits = quant.h_bits;
+    const int rows = max(1, min(m, quant.flush_rows));
+    const int shift_g = item_shift(quant.gq_max, rows, 63 - h_bits), shift_h = quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits);
+    const float scale_g = ldexpf(quant.scale_g, -shift_g), scale_h = ldexpf(quant.scale_h, -shift_h);
+    constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, U = 8;
+    const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
+    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
+    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
+    const bool word_lane = bins.gh_lane >= 0 && q == bins.gh_lane;
+    const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
+    for (int base = rsub; base < m; base += RPS * U) {
+        unsigned pk[U];
+        GHPair s[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned r = s_rows[min(base + u * RPS, m - 1)];
+            pk[u] = *reinterpret_cast<const unsigned *>(blk + (r * (unsigned)(LPR * 4) + (unsigned)q * 4));
+            s[u] = gh[r];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned v = base + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
+            const long long gq = round_to_ll(s[u].g * scale_g), hq = round_to_ll(fmaxf(s[u].h, 0.f) * scale_h);
+            const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
+            if (BIN16) {
+                const unsigned b0 = v & 0xffff, b1 = v >> 16;
+                if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
+                if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
+            } else {
+                const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
+                if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
+                if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
+                if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
+                if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
+            }
+        }
+    }
+    __syncthreads();
+    const int built = build_left ? node.lch_index : node.rch_index;
+    const unsigned long long h_mask = (1ull << h_bits) - 1ull;
+    longlong2 *out = tb.hist(level + 1) + (size_t)(built - ((2 << level) - 1)) * tb.n_bins + bin0;
+    for (int i = threadIdx.x; i < nb; i += kSmallBlock) {
+        const unsigned long long t = lds[i], low = t & h_mask;
+        out[i] = make_longlong2(((long long)(t - low) >> h_bits) << shift_g, (long long)low << shift_h);
+    }
+    if (first) {
+        tb.node_nleft[x_in] = nleft;
+        tb.seg[node.lch_index] = make_int2(sg.x, sg.x + nleft);
+        tb.seg[node.rch_index] = make_int2(sg.x + nleft, sg.y);
+        tb.hpair_built[x_in] = built;
+        atomicAdd(&tb.ctl[level + 1].n_hitems, 1);
+        atomicAdd(&tb.ctl[level + 1].rows_built, m);
+        apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
+    }
+}
+
 }  // namespace
 
 void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
@@ -348,6 +538,48 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
 #undef TGBM_SPLIT_COUNT
     if (level == 0) k_split_scatter<true><<<items, kBlock, 0, s>>>(tb, level);
     else k_split_scatter<false><<<items, kBlock, 0, s>>>(tb, level);
+}
+
+static size_t small_lds(const TreeBuffers &tb) {
+    return (size_t)tb.max_block_bins * 8 + ((size_t)(tb.n / 2 + 1) * 2 + 7) / 8 * 8;
+}
+
+// One workgroup adds up to half of the rows to one feature block's histogram (about five bins per clock): beyond 8192 rows x
+// 32 columns that takes longer at the first levels than the launches that are saved.
+bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins) {
+    return tb.n <= kSmallRows && tb.depth <= kSmallDepth && (long)(tb.n / 2) * std::min(bins.W, bins.n_cols) <= 1l << 18 &&
+           small_lds(tb) + 4096 <= 160 * 1024;
+}
+
+template <int LPR, bool BIN16>
+static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
+                               float rt_eps, float lambda, int n_class) {
+    const size_t lds = small_lds(tb);
+    static size_t opted = 0;
+    if (lds > 48 * 1024 && lds > opted) {  // (with the kernel's own tables more than the default window)
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_level<LPR, BIN16>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        opted = lds;
+    }
+    k_small_level<LPR, BIN16><<<dim3(bins.n_blocks, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda);
+}
+
+void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
+                        float lambda, int n_class) {
+    if (level == tb.depth - 1) return;
+#define TGBM_SMALL_LEVEL(LPR)                                                                               \
+    if (bins.bin_bytes == 2) small_level_launch<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, n_class); \
+    else small_level_launch<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, n_class);                    \
+    break
+    switch (bins.W * bins.bin_bytes) {  // bytes per row of a block
+        case 4: TGBM_SMALL_LEVEL(1);
+        case 8: TGBM_SMALL_LEVEL(2);
+        case 16: TGBM_SMALL_LEVEL(4);
+        case 32: TGBM_SMALL_LEVEL(8);
+        case 64: TGBM_SMALL_LEVEL(16);
+        default: fatal("unsupported dense block width %d x %d bytes", bins.W, bins.bin_bytes);
+    }
+#undef TGBM_SMALL_LEVEL
 }
 
 }  // namespace tgbm

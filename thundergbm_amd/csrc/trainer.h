@@ -78,7 +78,7 @@ class Trainer {
    private:
     TreeBuffers set_of(int k) const;
     void find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class);
-    void partition_sets(const TreeBuffers &tb, int level, int n_class);
+    void partition_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class);
     bool update_with_partition(int level) const;
     void build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class);
     void build_round_together();
@@ -87,6 +87,13 @@ class Trainer {
     void reorder_rows();                 // physical re-ordering of the rows by the leaves of the tree just built
     const std::vector<int> &host_perm();  // original row of every physical position (empty: identity)
     void run_metric(float *slot);  // (leaves the last step of the point-wise metrics in left_)
+    void leave_metric();
+    void leave_model(const TreeNode *nodes, int trees);
+    TreeLeftovers leftovers() const {
+        TreeLeftovers l = left_;
+        l.small = small();
+        return l;
+    }
     void settle();                 // what the last tree has left to do, where no next tree takes it along
     void alloc_tree_buffers();
     template <typename T>
@@ -164,6 +171,8 @@ class Trainer {
     int *d_bag_count_ = nullptr;         // bagging: draws per gradient entry (zero between rounds)
     bool rank_order_fresh_ = false;      // d_yp_ unchanged since the last ranking metric pass
     bool in_boost_ = false;
+    bool small_ok_ = false;          // inside boost() the levels go through launch_small_level
+    bool small() const { return in_boost_ && small_ok_; }
     int lookup_level_ = -1;          // level whose split nodes have not been partitioned into row lists yet
     bool next_round_ready_ = false;  // d_gh_ and the root statistics already belong to the next round
     // profiling

@@ -669,6 +669,8 @@ void Trainer::alloc_tree_buffers() {
     tb.feat_lds_off = d_off;
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors above go out of scope
 
+    const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
+    small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb, bins_) && !(small_env != nullptr && std::string(small_env) == "0");
     model_cap_trees_ = std::max(1, param_.n_trees) * param_.tree_per_rounds;
     d_model_ = dalloc<TreeNode>((size_t)model_cap_trees_ * tb.n_nodes);
     d_metric_ = dalloc<float>((size_t)std::max(1, param_.n_trees));
@@ -778,7 +780,7 @@ void Trainer::tree_init(int k) {
     if (!in_boost_) ensure_gh_array();
     cur_class_ = k;
     HIP_CHECK_LAUNCHES("the stages before tree_init");  // gradients, bagging, column sampling, metric, re-ordering
-    launch_tree_init(stream_, set_of(k), d_gh_ + (size_t)k * n_, param_.lambda, next_round_ready_, 1, left_);
+    launch_tree_init(stream_, set_of(k), d_gh_ + (size_t)k * n_, param_.lambda, next_round_ready_, 1, leftovers());
     left_ = TreeLeftovers();
     next_round_ready_ = false;
     lookup_level_ = -1;
@@ -972,10 +974,11 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
         return;
     }
     mark(level == 0 ? PH_GRADIENT : PH_PARTITION, level);  // closes what ran before this level's histogram
-    build_level_hist(tb, level, gh, n_class);
+    const bool derive = small() && level > 0;  // the level before has built its histograms
+    if (!derive) build_level_hist(tb, level, gh, n_class);
     mark(PH_HIST, level);
     if (!sparse_pass_) {
-        if (!sparse_) launch_hist_merge(stream_, tb, level, n_class);
+        if (!sparse_ && !derive) launch_hist_merge(stream_, tb, level, n_class);
         // (inside boost() the split search adds up the root itself where a feature is stored in every row)
         const bool root = level == 0 && in_boost_ && tb.complete_feature >= 0 && !wide_eval_ && !sparse_;
         if (level == 0 && !root) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
@@ -984,10 +987,10 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
         // last level that fits a capped arena keeps them for the batches of the next one
         if (wide_eval_)
             launch_eval_split_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                                   !(in_boost_ && level == param_.depth - 1));
+                                   !(in_boost_ && level == param_.depth - 1), derive);
         else
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                              !(in_boost_ && level == param_.depth - 1), root);
+                              !(in_boost_ && level == param_.depth - 1), root, derive);
     }
     if (!update_with_partition(level)) launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
     mark(PH_SPLIT, level);
@@ -1019,9 +1022,9 @@ void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *g
     }
 }
 
-void Trainer::partition(int level) { partition_sets(set_of(cur_class_), level, 1); }
+void Trainer::partition(int level) { partition_sets(set_of(cur_class_), d_gh_ + (size_t)cur_class_ * n_, level, 1); }
 
-void Trainer::partition_sets(const TreeBuffers &tb, int level, int n_class) {
+void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class) {
     // the last level is not partitioned: its split nodes keep their rows until the tree's final pass
     if (level < param_.depth - 1) lookup_level_ = -1;
     if (sparse_pass_) {
@@ -1029,6 +1032,8 @@ void Trainer::partition_sets(const TreeBuffers &tb, int level, int n_class) {
         lookup_level_ = -1;
     } else if (sparse_)
         launch_partition_csr(stream_, tb, csr_, level, n_class);
+    else if (small())
+        launch_small_level(stream_, tb, bins_, gh, level, param_.rt_eps, param_.lambda, n_class);
     else
         launch_partition_dense(stream_, tb, bins_, level, update_with_partition(level), param_.rt_eps, param_.lambda, n_class);
     mark(PH_PARTITION, level);
@@ -1060,16 +1065,25 @@ void Trainer::finish_tree(int k, bool fuse_round_end) {
     const TreeBuffers tb = set_of(k);
     rank_order_fresh_ = false;  // the scores change below
     // (the tree is pruned by a workgroup of the same launches)
-    if (fuse_round_end) {
+    if (small()) {
+        TreeNode *model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
+        if (fuse_round_end) {
+            launch_small_end(stream_, tb, bins_, model, param_.gamma, d_yp_, param_.learning_rate, 1, d_y_, objective_,
+                             metric_kind_, d_gh_, d_metric_scratch_, d_gh_words_);
+            gh_words_fresh_ = d_gh_words_ != nullptr;
+            gh_records_fresh_ = false;
+            next_round_ready_ = true;
+            leave_metric();
+        } else {
+            launch_small_end(stream_, tb, bins_, model, param_.gamma, d_yp_ + (size_t)k * n_, param_.learning_rate);
+        }
+    } else if (fuse_round_end) {
         // one tree per round: prediction update + metric + next gradients + their statistics in one pass
         // (see gh_array_stale_: inside boost() the next tree may need the words only)
         const bool words_only = in_boost_ && d_gh_words_ != nullptr && tb.complete_feature >= 0;
         launch_round_end(stream_, tb, &bins_, &csr_, lookup_level_, objective_, metric_kind_, d_y_, d_yp_,
                          param_.learning_rate, words_only ? nullptr : d_gh_, d_metric_scratch_, &param_.gamma, d_gh_words_);
-        left_.metric_out = d_metric_ + rounds_done_;
-        left_.metric_partial = d_metric_scratch_;
-        left_.metric_kind = metric_kind_;
-        left_.metric_blocks = row_blocks(n_);
+        leave_metric();
         gh_array_stale_ = words_only;
         gh_words_fresh_ = d_gh_words_ != nullptr;
         gh_records_fresh_ = false;  // (the records still hold the finished tree's words)
@@ -1079,9 +1093,7 @@ void Trainer::finish_tree(int k, bool fuse_round_end) {
                                    param_.learning_rate, 1, &param_.gamma);
     }
     TGBM_CHECK(trees_built_ < model_cap_trees_, "more trees built than n_trees * tree_per_rounds");
-    left_.model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
-    left_nodes_ = tb.nodes;
-    left_trees_ = 1;
+    leave_model(tb.nodes, 1);
     if (!in_boost_) settle();
     mark(PH_TREE_END);
     if (profiling_) log_plan(tb);
@@ -1096,19 +1108,20 @@ void Trainer::build_round_together() {
     TreeBuffers tb = tb_;
     // the K classes share the chip: size every class's histogram items for its share of the workgroup slots
     tb.target_hitems = std::max(4, tb_.target_hitems / K);
-    launch_tree_init(stream_, tb, d_gh_, param_.lambda, false, K, left_);
+    launch_tree_init(stream_, tb, d_gh_, param_.lambda, false, K, leftovers());
     left_ = TreeLeftovers();
     lookup_level_ = -1;
     nid_materialized_ = false;
     for (int level = 0; level < param_.depth; ++level) {
         find_split_sets(tb, d_gh_, level, K);
-        partition_sets(tb, level, K);
+        partition_sets(tb, d_gh_, level, K);
     }
-    launch_predict_in_training(stream_, tb, &bins_, &csr_, lookup_level_, d_yp_, param_.learning_rate, K, &param_.gamma);
+    if (small())
+        launch_small_end(stream_, tb, bins_, d_model_ + (size_t)trees_built_ * tb.n_nodes, param_.gamma, d_yp_, param_.learning_rate, K);
+    else
+        launch_predict_in_training(stream_, tb, &bins_, &csr_, lookup_level_, d_yp_, param_.learning_rate, K, &param_.gamma);
     TGBM_CHECK(trees_built_ + K <= model_cap_trees_, "more trees built than n_trees * tree_per_rounds");
-    left_.model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
-    left_nodes_ = tb.nodes;
-    left_trees_ = (size_t)K;
+    leave_model(tb.nodes, K);
     mark(PH_TREE_END);
     if (profiling_)
         for (int k = 0; k < K; ++k) log_plan(tb.for_class(k));
@@ -1123,11 +1136,23 @@ void Trainer::run_metric(float *slot) {
         rank_order_fresh_ = true;
     } else {
         launch_metric(stream_, metric_kind_, n_, param_.num_class, d_y_, d_yp_, d_metric_scratch_);
+        leave_metric();
         left_.metric_out = slot;
-        left_.metric_partial = d_metric_scratch_;
-        left_.metric_kind = metric_kind_;
-        left_.metric_blocks = row_blocks(n_);
     }
+}
+
+// (the small-data path has put them there and leaves the buffers' own nodes unpruned)
+void Trainer::leave_model(const TreeNode *nodes, int trees) {
+    if (!small()) left_.model = d_model_ + (size_t)trees_built_ * tb_.n_nodes;
+    left_nodes_ = nodes;
+    left_trees_ = (size_t)trees;
+}
+
+void Trainer::leave_metric() {
+    left_.metric_out = d_metric_ + rounds_done_;
+    left_.metric_partial = d_metric_scratch_;
+    left_.metric_kind = metric_kind_;
+    left_.metric_blocks = row_blocks(n_);
 }
 
 void Trainer::settle() {
@@ -1206,6 +1231,9 @@ void Trainer::boost(int rounds) {
         HIP_CHECK_LAUNCHES("boost");
     }
     settle();
+    if (small() && trees_built_ > 0)  // (for the getters)
+        HIP_CHECK(hipMemcpyAsync(const_cast<TreeNode *>(left_nodes_), d_model_ + (size_t)(trees_built_ - (int)left_trees_) * tb_.n_nodes,
+                                 sizeof(TreeNode) * (size_t)tb_.n_nodes * left_trees_, hipMemcpyDeviceToDevice, stream_));
     in_boost_ = false;
 }
 

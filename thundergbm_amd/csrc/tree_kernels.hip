@@ -241,6 +241,10 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
     }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    if (left.small) {  // every row starts in the root; k_small_level counts the levels' rows
+        for (int i = threadIdx.x; i < tb.n; i += kBlock) tb.nid[i] = 0;
+        for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{0, 0, 0, 0};
+    }
     const GradStats *__restrict__ block_sums = tb.root_partial;
     const int nn = tb.n_nodes;
     for (int i = threadIdx.x; i < nn; i += kBlock) {
@@ -1211,7 +1215,7 @@ __device__ __forceinline__ longlong2 wide_bin(const longlong2 *h, const longlong
 }
 
 __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, int level, float mcw, float lambda,
-                                                           bool store_sibling) {
+                                                           bool store_sibling, bool derive) {
 #pragma clang fp contract(off)
     __shared__ long long s_g[kWaves], s_h[kWaves];
     __shared__ float s_abs[kWaves];
@@ -1231,7 +1235,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
     const int lane = lane_id(), w = wave_id();
     longlong2 *h = tb.hist(level) + (size_t)x_in * tb.n_bins;
     const longlong2 *h_par = nullptr, *h_built = nullptr;
-    if (tb.sparse && level > 0 && !tb.singles(level)) {  // (the dense layout's k_hist_merge has derived the siblings)
+    if (derive && level > 0 && !tb.singles(level)) {  // (the dense layout's k_hist_merge has derived the siblings)
         const int built = tb.hpair_built[x_in >> 1];
         if (built >= 0 && built != x) {
             h_par = tb.hist(level + 1) + (size_t)(x_in >> 1) * tb.n_bins;
@@ -2094,6 +2098,89 @@ __global__ __launch_bounds__(BLK) void k_tree_end(TreeBuffers tb_all, DenseBins 
     tree_end_rows<MODE, BLK>(tb, a, s_leaf, r0, r1);
 }
 
+// The end of a tree of the small-data path (k_small_level): the rows' nodes are in tb.nid, and the tree is small enough for
+// every workgroup to prune it in LDS by itself; the first one writes the finished nodes into the model (in place they would
+// change under the other workgroups' eyes). One launch instead of k_end_bounds, k_tree_end and the copy: 31 -> 10 us at 10 k
+// rows.
+template <int MODE>
+__global__ __launch_bounds__(kEndWide) void k_small_end(TreeBuffers tb_all, DenseBins bins, TreeEndArgs a, TreeNode *model) {
+    constexpr int kNodes = (2 << kSmallDepth) - 1;
+    __shared__ short s_leaf[kRowBlock];
+    __shared__ float s_value[kNodes];     // what a row adds that ended in the node
+    __shared__ unsigned char s_flag[kNodes];
+    __shared__ int s_scan[kEndWide / 64];
+    enum { VALID = 1, LEAF = 2, BELOW = 4, PRUNED = 8 };
+    TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    if (MODE == 1) a.yp += (size_t)blockIdx.z * tb.n;
+    const int r0 = blockIdx.x * kRowBlock, r1 = min(tb.n, r0 + kRowBlock);
+    constexpr int V = kRowBlock / kEndWide;
+    int at[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) at[v] = tb.nid[min(r0 + v * kEndWide + (int)threadIdx.x, tb.n - 1)];
+    for (int i = threadIdx.x; i < tb.n_nodes; i += kEndWide) {
+        const TreeNode nd = tb.nodes[i];
+        s_flag[i] = (unsigned char)((nd.is_valid ? VALID : 0) | (nd.is_leaf ? LEAF : 0) | (nd.gain < a.gamma ? BELOW : 0));
+        s_value[i] = nd.base_weight;
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = v * kEndWide + (int)threadIdx.x;
+        if (r0 + i >= r1) continue;
+        // (the last level's split nodes still hold their rows)
+        const TreeNode &nd = tb.nodes[at[v]];
+        s_leaf[i] = (short)(nd.split_feature_id >= 0 && at[v] >= tb.n_nodes / 4
+                                ? end_child_of<false>(tb, bins, CsrBins{}, nd, r0 + i) : at[v]);
+    }
+    __syncthreads();
+    // (prune_tree in LDS)
+    for (int level = tb.depth - 1; level >= 0; --level) {
+        const int x = (1 << level) - 1 + (int)threadIdx.x;
+        static_assert(1 << (kSmallDepth - 1) <= kEndWide, "one node of a level per thread");
+        if ((int)threadIdx.x < 1 << level && (s_flag[x] & (VALID | LEAF | BELOW)) == (VALID | BELOW)) {
+            constexpr int both = VALID | LEAF;
+            if ((s_flag[2 * x + 1] & both) == both && (s_flag[2 * x + 2] & both) == both) {
+                s_flag[2 * x + 1] |= PRUNED;
+                s_flag[2 * x + 2] |= PRUNED;
+                s_flag[x] |= LEAF;
+            }
+        }
+        __syncthreads();
+    }
+    if (blockIdx.x == 0) {
+        model += (size_t)blockIdx.z * tb.n_nodes;
+        int carry = 0;
+        for (int base = 0; base < tb.n_nodes; base += kEndWide) {
+            const int i = base + threadIdx.x;
+            const bool in = i < tb.n_nodes;
+            const bool keep = in && (s_flag[i] & (VALID | PRUNED)) == VALID;
+            int tot;
+            const int ex = block_excl_scan<kEndWide / 64>(keep ? 1 : 0, s_scan, &tot);
+            if (in) {
+                static_assert(offsetof(TreeNode, final_id) == 0 && offsetof(TreeNode, is_leaf) == 34 && offsetof(TreeNode, is_pruned) == 36,
+                              "TreeNode layout");
+                const int4 *from = reinterpret_cast<const int4 *>(tb.nodes + i);
+                int4 v0 = from[0], v2 = from[2];
+                if (keep) v0.x = carry + ex;
+                v2.x = (v2.x & ~0x00ff0000) | ((s_flag[i] & LEAF) ? 1 << 16 : 0);
+                v2.y = (v2.y & ~0x000000ff) | ((s_flag[i] & PRUNED) ? 1 : 0);
+                int4 *to = reinterpret_cast<int4 *>(model + i);
+                to[0] = v0;
+                to[1] = from[1];
+                to[2] = v2;
+            }
+            carry += tot;
+        }
+    }
+    // the weight of the first ancestor that was not pruned (tree_builder.cu:62-74), top-down
+    for (int level = 1; level <= tb.depth; ++level) {
+        for (int x = (1 << level) - 1 + (int)threadIdx.x; x < (2 << level) - 1; x += kEndWide)
+            if (s_flag[x] & PRUNED) s_value[x] = s_value[(x - 1) / 2];
+        __syncthreads();
+    }
+    tb.leaf_value = s_value;
+    tree_end_rows<MODE, kEndWide>(tb, a, s_leaf, r0, r1);
+}
+
 // ---------------------------------------------------------------------------------- metric
 // kind 0: sum of squared errors; 1: correct binary decisions (sigmoid > 0.5 in double, like
 // multiclass_metric.cu:40); 2: correct arg-max decisions (first maximum wins, :17-29).
@@ -2396,17 +2483,17 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
 }
 
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
-                       bool store_sibling, bool root) {
+                       bool store_sibling, bool root, bool derive) {
     dim3 grid((tb.n_packs + kWaves - 1) / kWaves, tb.nodes_served(level), n_class);
     if (root) k_eval_split<false, true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
-    else if (tb.sparse) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
+    else if (tb.sparse || derive) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
 }
 
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
-                            bool store_sibling) {
+                            bool store_sibling, bool derive) {
     dim3 grid(tb.F, tb.nodes_served(level), n_class);
-    k_eval_split_wide<<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
+    k_eval_split_wide<<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling, derive || tb.sparse);
 }
 
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class) {
@@ -2487,6 +2574,25 @@ void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbi
     a.stats = tb.root_partial;
     a.metric_partial = metric_scratch;
     tree_end(s, tb, dbins, cbins, 2, a);
+}
+
+void launch_small_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, TreeNode *model, float gamma, float *yp,
+                      float lr, int n_class, const float *y, int objective, int metric_kind, GHPair *gh,
+                      double *metric_scratch, unsigned *gh_words) {
+    TreeEndArgs a{};
+    a.gamma = gamma;
+    a.yp = yp;
+    a.lr = lr;
+    a.y = y;
+    a.objective = objective;
+    a.metric_kind = metric_kind;
+    a.gh = gh;
+    a.stats = tb.root_partial;
+    a.metric_partial = metric_scratch;
+    a.gh_words = gh_words;
+    const dim3 grid(row_blocks(tb.n), 1, n_class);
+    if (y != nullptr) k_small_end<2><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+    else k_small_end<1><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
 }
 
 void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left) {
