@@ -978,14 +978,19 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     if (!derive) build_level_hist(tb, level, gh, n_class);
     mark(PH_HIST, level);
     if (!sparse_pass_) {
-        if (!sparse_ && !derive) launch_hist_merge(stream_, tb, level, n_class);
+        // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
+        const bool fused = !sparse_ && !derive && level > 0 && !wide_eval_ && hist_cap_level_ < 0;
+        if (!sparse_ && !derive && !fused) launch_hist_merge(stream_, tb, level, n_class);
         // (inside boost() the split search adds up the root itself where a feature is stored in every row)
         const bool root = level == 0 && in_boost_ && tb.complete_feature >= 0 && !wide_eval_ && !sparse_;
         if (level == 0 && !root) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         mark(PH_MERGE, level);
         // inside boost() nobody looks at the last level's derived histograms (the stage-wise API keeps them); the
         // last level that fits a capped arena keeps them for the batches of the next one
-        if (wide_eval_)
+        if (fused)
+            launch_merge_eval(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
+                              !(in_boost_ && level == param_.depth - 1));
+        else if (wide_eval_)
             launch_eval_split_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                                    !(in_boost_ && level == param_.depth - 1), derive);
         else

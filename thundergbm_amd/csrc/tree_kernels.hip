@@ -1004,6 +1004,149 @@ __global__ __launch_bounds__(kBlock) void k_part_count_csr(TreeBuffers tb_all, C
 // left = sum of the feature's bins below it, missing = node sum - feature total, gain with missing
 // values sent right and left (hist_tree_builder_single.cu:257-325 / :614-681 of the reference);
 // the wavefront keeps its best candidate: largest |gain|, ties to the smaller bin index (:330-335).
+// What a wavefront has stored in LDS is there for its other lanes (the accesses of a wavefront stay in order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The search of one pack of one node, by one wavefront: s_v holds the pack's bins, s_miss takes its features' missing sums
+// (kEvalPackBins entries each).
+__device__ __forceinline__ void search_pack(const TreeBuffers &tb, const longlong2 *s_v, GHPair *s_miss, int x_in, int pack,
+                                            bool active, int b_begin, int b_end, GHPair S, double inv_g, double inv_h, float mcw,
+                                            float lambda) {
+#pragma clang fp contract(off)
+    const int lane = lane_id();
+    long long incg[4], inch[4];
+    int lastb[4];  // pack-relative index of the last bin of the element's feature
+    bool valid[4], head[4], last[4], ign[4];
+    unsigned meta[4] = {0, 0, 0, 0};
+    long long rung = 0, runh = 0;
+    bool any_head = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        int b = b_begin + lane * 4 + j;
+        valid[j] = b < b_end;
+        lastb[j] = 0;
+        head[j] = false;
+        last[j] = false;
+        ign[j] = false;
+        incg[j] = inch[j] = 0;
+        if (valid[j]) {
+            const longlong2 v = s_v[lane * 4 + j];
+            // one word per bin instead of the chain bin -> feature -> feature's bin range
+            meta[j] = tb.bin_meta[b];
+            ign[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[b]] != 0;
+            const int to_last = (int)(meta[j] & 0xffu);
+            head[j] = (meta[j] & 0xff00u) == 0;
+            last[j] = to_last == 0;
+            lastb[j] = b + to_last - b_begin;
+            if (head[j]) {
+                rung = v.x;
+                runh = v.y;
+                any_head = true;
+            } else {
+                rung += v.x;
+                runh += v.y;
+            }
+            incg[j] = rung;
+            inch[j] = runh;
+        }
+    }
+    // wavefront segmented inclusive scan of the lane aggregates
+    long long aggg = rung, aggh = runh;
+    int flag = any_head ? 1 : 0;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        long long pg = shfl_up_ll(aggg, d);
+        long long ph = shfl_up_ll(aggh, d);
+        int pf = __shfl_up(flag, d);
+        if (lane >= d) {
+            if (!flag) {
+                aggg += pg;
+                aggh += ph;
+            }
+            flag |= pf;
+        }
+    }
+    long long carryg = shfl_up_ll(aggg, 1), carryh = shfl_up_ll(aggh, 1);
+    if (lane == 0) carryg = carryh = 0;
+    bool seen = false;
+    long long exg[4], exh[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (valid[j]) {
+            if (head[j]) seen = true;
+            if (!seen) {
+                incg[j] += carryg;
+                inch[j] += carryh;
+            }
+        }
+        if (head[j]) {
+            exg[j] = exh[j] = 0;
+        } else {
+            exg[j] = (j == 0) ? carryg : incg[j > 0 ? j - 1 : 0];
+            exh[j] = (j == 0) ? carryh : inch[j > 0 ? j - 1 : 0];
+        }
+        if (valid[j] && last[j]) {
+            const float tg = (float)((double)incg[j] * inv_g), th = (float)((double)inch[j] * inv_h);
+            s_miss[lastb[j]] = GHPair{S.g - tg, S.h - th};
+        }
+    }
+    wave_lds_sync();
+    float best = -1.f;  // |score| of the lane's best candidate
+    float best_score = 0.f;
+    int best_idx = 0x7fffffff;
+    unsigned best_meta = 0;
+    GHPair best_miss{0, 0}, best_left{0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (valid[j]) {
+            const GHPair m = s_miss[lastb[j]];
+            const GHPair l{(float)((double)exg[j] * inv_g), (float)((double)exh[j] * inv_h)};
+            float gr = split_gain(S, l, mcw, lambda);
+            GHPair l2{l.g + m.g, l.h + m.h};
+            float gl = split_gain(S, l2, mcw, lambda);
+            float score = (gl > gr) ? gl : -gr;
+            if (ign[j]) score = 0.f;  // column sampling: hist_tree_builder_single.cu:304 / :663
+            float a = fabsf(score);
+            if (a > best) {
+                best = a;
+                best_score = score;
+                best_idx = b_begin + lane * 4 + j;
+                best_meta = meta[j];
+                best_miss = m;
+                best_left = l;
+            }
+        }
+    }
+    // wavefront arg-max: larger |score| wins, ties go to the smaller bin index. Only the key travels through the
+    // butterfly; the lane that holds the winner writes its candidate itself.
+    float win = best;
+    int win_idx = best_idx;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const float oa = __shfl_xor(win, d);
+        const int oi = __shfl_xor(win_idx, d);
+        if (oa > win || (oa == win && oi < win_idx)) {
+            win = oa;
+            win_idx = oi;
+        }
+    }
+    // (without any candidate every lane still holds the initial key and the first one writes the empty record)
+    const unsigned long long owners = __ballot(best == win && best_idx == win_idx);
+    if (active && lane == __ffsll((long long)owners) - 1) {
+        SplitCand c;
+        c.score = best_score;
+        c.index = best_idx;
+        c.miss = best_miss;
+        c.left = best_left;
+        c.feature = (int)(best_meta >> 16);
+        c.bin = (int)(best_meta >> 8 & 0xffu);
+        tb.cand[(size_t)x_in * tb.n_packs + pack] = c;
+    }
+}
+
 // SUB (sparse layout, whose histograms are not merged from work-item partials): the node of a pair that
 // was not built from rows is derived here as parent - built while it is scanned, and stored for the next
 // level, instead of by a separate pass over the (very long) histograms.
@@ -1071,135 +1214,94 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
             s_v[w][j * 64 + lane] = v;
         }
     }
+    wave_lds_sync();
+    search_pack(tb, s_v[w], s_miss[w], x_in, pack, active, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
+}
+
+// k_hist_merge and k_eval_split of a level below the root in one launch: a workgroup owns a pack of a sibling pair. Its
+// wavefronts share out the pair's work items, the sums meet in LDS, parent - built gives the sibling, one wavefront searches
+// the built node and one its sibling. The histograms are stored for the next level only (not at a tree's last one, which holds
+// half of a tree's nodes) and not read back. NW follows from the items per pair (launch_merge_eval).
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int level, float mcw, float lambda, bool store) {
+    __shared__ longlong2 s_sum[NW][kEvalPackBins];
+    __shared__ GHPair s_miss[2][kEvalPackBins];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int p = blockIdx.y, pack = blockIdx.x;
+    const int built = tb.hpair_built[p];
+    if (built < 0) return;  // (nobody reads the candidates of nodes that do not exist)
+    const int lane = lane_id(), w = wave_id();
+    const int off = (1 << level) - 1, n_bins = tb.n_bins;
+    const int b_begin = tb.pack_begin[pack], b_end = tb.pack_begin[pack + 1], nb = b_end - b_begin;
+    const int ib = tb.hpair_begin[p], ie = tb.hpair_begin[p + 1];
+    // (every thread below kEvalPackBins carries one bin of the pack from here to the search)
+    const bool carrier = threadIdx.x < kEvalPackBins && (int)threadIdx.x < nb;
+    longlong2 parent = make_longlong2(0, 0);
+    if (carrier) parent = tb.hist(level + 1)[(size_t)p * n_bins + b_begin + threadIdx.x];
+    const int sibling = (built & 1) ? built + 1 : built - 1;
+    const GHPair S = tb.nodes[w == 0 ? built : sibling].sum_gh_pair;
+    const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
+    long long g[4] = {0, 0, 0, 0}, h[4] = {0, 0, 0, 0};
+    int at[4];  // (bins past the pack's end repeat its last one: all loads of an item are issued at once)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) at[j] = b_begin + min(j * 64 + lane, nb - 1);
+    // every item counted at its own scale (item_shift): shift its sums to the tree's
+    const int2 *__restrict__ shift = tb.hitem_shift;
+    if (tb.ctl[level].hchunk <= tb.quant->flush_rows) {  // packed 8-byte partials (see k_hist_dense)
+        const unsigned long long *__restrict__ packed = reinterpret_cast<const unsigned long long *>(tb.partial);
+        const int h_bits = tb.quant->h_bits;
+        const unsigned long long h_mask = (1ull << h_bits) - 1ull;
+#pragma unroll 2
+        for (int it = ib + w; it < ie; it += NW) {
+            unsigned long long t[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[j] = packed[(size_t)it * n_bins + at[j]];
+            const int2 sh = shift[it];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const unsigned long long lo = t[j] & h_mask;
+                g[j] += ((long long)(t[j] - lo) >> h_bits) << sh.x;
+                h[j] += (long long)lo << sh.y;
+            }
+        }
+    } else {
+        for (int it = ib + w; it < ie; it += NW) {
+            longlong2 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = tb.partial[(size_t)it * n_bins + at[j]];
+            const int2 sh = shift[it];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                g[j] += v[j].x << sh.x;
+                h[j] += v[j].y << sh.y;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s_sum[w][j * 64 + lane] = make_longlong2(g[j], h[j]);
     __syncthreads();
-    long long incg[4], inch[4];
-    int lastb[4];  // pack-relative index of the last bin of the element's feature
-    bool valid[4], head[4], last[4], ign[4];
-    unsigned meta[4] = {0, 0, 0, 0};
-    long long rung = 0, runh = 0;
-    bool any_head = false;
+    longlong2 sum = make_longlong2(0, 0);
+    if (carrier) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        int b = b_begin + lane * 4 + j;
-        valid[j] = b < b_end;
-        lastb[j] = 0;
-        head[j] = false;
-        last[j] = false;
-        ign[j] = false;
-        incg[j] = inch[j] = 0;
-        if (valid[j]) {
-            const longlong2 v = s_v[w][lane * 4 + j];
-            // one word per bin instead of the chain bin -> feature -> feature's bin range
-            meta[j] = tb.bin_meta[b];
-            ign[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[b]] != 0;
-            const int to_last = (int)(meta[j] & 0xffu);
-            head[j] = (meta[j] & 0xff00u) == 0;
-            last[j] = to_last == 0;
-            lastb[j] = b + to_last - b_begin;
-            if (head[j]) {
-                rung = v.x;
-                runh = v.y;
-                any_head = true;
-            } else {
-                rung += v.x;
-                runh += v.y;
-            }
-            incg[j] = rung;
-            inch[j] = runh;
-        }
-    }
-    // wavefront segmented inclusive scan of the lane aggregates
-    long long aggg = rung, aggh = runh;
-    int flag = any_head ? 1 : 0;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        long long pg = shfl_up_ll(aggg, d);
-        long long ph = shfl_up_ll(aggh, d);
-        int pf = __shfl_up(flag, d);
-        if (lane >= d) {
-            if (!flag) {
-                aggg += pg;
-                aggh += ph;
-            }
-            flag |= pf;
-        }
-    }
-    long long carryg = shfl_up_ll(aggg, 1), carryh = shfl_up_ll(aggh, 1);
-    if (lane == 0) carryg = carryh = 0;
-    bool seen = false;
-    long long exg[4], exh[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (valid[j]) {
-            if (head[j]) seen = true;
-            if (!seen) {
-                incg[j] += carryg;
-                inch[j] += carryh;
-            }
-        }
-        if (head[j]) {
-            exg[j] = exh[j] = 0;
-        } else {
-            exg[j] = (j == 0) ? carryg : incg[j > 0 ? j - 1 : 0];
-            exh[j] = (j == 0) ? carryh : inch[j > 0 ? j - 1 : 0];
-        }
-        if (valid[j] && last[j]) {
-            const float tg = (float)((double)incg[j] * inv_g), th = (float)((double)inch[j] * inv_h);
-            s_miss[w][lastb[j]] = GHPair{S.g - tg, S.h - th};
+        for (int i = 0; i < NW; ++i) {
+            const longlong2 v = s_sum[i][threadIdx.x];
+            sum.x += v.x;
+            sum.y += v.y;
         }
     }
     __syncthreads();
-    float best = -1.f;  // |score| of the lane's best candidate
-    float best_score = 0.f;
-    int best_idx = 0x7fffffff;
-    unsigned best_meta = 0;
-    GHPair best_miss{0, 0}, best_left{0, 0};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (valid[j]) {
-            const GHPair m = s_miss[w][lastb[j]];
-            const GHPair l{(float)((double)exg[j] * inv_g), (float)((double)exh[j] * inv_h)};
-            float gr = split_gain(S, l, mcw, lambda);
-            GHPair l2{l.g + m.g, l.h + m.h};
-            float gl = split_gain(S, l2, mcw, lambda);
-            float score = (gl > gr) ? gl : -gr;
-            if (ign[j]) score = 0.f;  // column sampling: hist_tree_builder_single.cu:304 / :663
-            float a = fabsf(score);
-            if (a > best) {
-                best = a;
-                best_score = score;
-                best_idx = b_begin + lane * 4 + j;
-                best_meta = meta[j];
-                best_miss = m;
-                best_left = l;
-            }
+    if (carrier) {
+        const longlong2 other = make_longlong2(parent.x - sum.x, parent.y - sum.y);
+        s_sum[0][threadIdx.x] = sum;
+        s_sum[1][threadIdx.x] = other;
+        if (store) {
+            tb.hist(level)[(size_t)(built - off) * n_bins + b_begin + threadIdx.x] = sum;
+            tb.hist(level)[(size_t)(sibling - off) * n_bins + b_begin + threadIdx.x] = other;
         }
     }
-    // wavefront arg-max: larger |score| wins, ties go to the smaller bin index. Only the key travels through the
-    // butterfly; the lane that holds the winner writes its candidate itself.
-    float win = best;
-    int win_idx = best_idx;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const float oa = __shfl_xor(win, d);
-        const int oi = __shfl_xor(win_idx, d);
-        if (oa > win || (oa == win && oi < win_idx)) {
-            win = oa;
-            win_idx = oi;
-        }
-    }
-    // (without any candidate every lane still holds the initial key and the first one writes the empty record)
-    const unsigned long long owners = __ballot(best == win && best_idx == win_idx);
-    if (active && lane == __ffsll((long long)owners) - 1) {
-        SplitCand c;
-        c.score = best_score;
-        c.index = best_idx;
-        c.miss = best_miss;
-        c.left = best_left;
-        c.feature = (int)(best_meta >> 16);
-        c.bin = (int)(best_meta >> 8 & 0xffu);
-        tb.cand[(size_t)x_in * tb.n_packs + pack] = c;
-    }
+    __syncthreads();
+    if (w < 2)
+        search_pack(tb, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
 // Split search for features of any number of bins (max_num_bin above 255): one workgroup per (feature, node) walks the
@@ -2488,6 +2590,16 @@ void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mc
     if (root) k_eval_split<false, true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
     else if (tb.sparse || derive) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
+}
+
+void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store) {
+    const int n_pairs = tb.n_hpairs(level);
+    const dim3 grid(tb.n_packs, n_pairs, n_class);
+    // (as many items as the level can have, see hist_dense_launch)
+    const int items = std::min(tb.target_hitems, tb.n / 2 / kHistMinChunk + n_pairs), per_pair = items / n_pairs;
+    if (per_pair > 32) k_merge_eval<16><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+    else if (per_pair > 8) k_merge_eval<8><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
+    else k_merge_eval<4><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
 }
 
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
