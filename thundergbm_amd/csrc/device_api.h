@@ -397,11 +397,11 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
                      int n_class = 1);
 void launch_partition_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class = 1);
 // store_sibling (sparse layout only): keep the derived sibling histograms; nobody reads those of a tree's
-// last level. derive: the nodes that were not built are parent - built (always so in the sparse layout). root: level 0 of the dense layout with a complete feature, in place of launch_root_sum
+// last level. derive: the nodes that were not built are parent - built (always so in the sparse layout).
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
-                       bool store_sibling = true, bool root = false, bool derive = false);
-// Dense layout below the root, all nodes of the level at once: launch_hist_merge and launch_eval_split in one launch. store:
-// the histograms are kept (nobody reads those of a tree's last level).
+                       bool store_sibling = true, bool derive = false);
+// Dense layout, all nodes of the level at once: launch_hist_merge and launch_eval_split in one launch (level 0: and
+// launch_root_sum, needs a complete feature). store: the histograms are kept (nobody reads those of a tree's last level).
 void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store);
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,

@@ -979,11 +979,9 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     mark(PH_HIST, level);
     if (!sparse_pass_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
-        const bool fused = !sparse_ && !derive && level > 0 && !wide_eval_ && hist_cap_level_ < 0;
+        const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0 && (level > 0 || tb.complete_feature >= 0);
         if (!sparse_ && !derive && !fused) launch_hist_merge(stream_, tb, level, n_class);
-        // (inside boost() the split search adds up the root itself where a feature is stored in every row)
-        const bool root = level == 0 && in_boost_ && tb.complete_feature >= 0 && !wide_eval_ && !sparse_;
-        if (level == 0 && !root) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
+        if (level == 0 && !fused) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         mark(PH_MERGE, level);
         // inside boost() nobody looks at the last level's derived histograms (the stage-wise API keeps them); the
         // last level that fits a capped arena keeps them for the batches of the next one
@@ -995,7 +993,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
                                    !(in_boost_ && level == param_.depth - 1), derive);
         else
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                              !(in_boost_ && level == param_.depth - 1), root, derive);
+                              !(in_boost_ && level == param_.depth - 1), derive);
     }
     if (!update_with_partition(level)) launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
     mark(PH_SPLIT, level);

@@ -1218,14 +1218,16 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
     search_pack(tb, s_v[w], s_miss[w], x_in, pack, active, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
-// k_hist_merge and k_eval_split of a level below the root in one launch: a workgroup owns a pack of a sibling pair. Its
-// wavefronts share out the pair's work items, the sums meet in LDS, parent - built gives the sibling, one wavefront searches
-// the built node and one its sibling. The histograms are stored for the next level only (not at a tree's last one, which holds
-// half of a tree's nodes) and not read back. NW follows from the items per pair (launch_merge_eval).
-template <int NW>
+// k_hist_merge and k_eval_split of a level in one launch: a workgroup owns a pack of a sibling pair. Its wavefronts share
+// out the pair's work items, the sums meet in LDS, parent - built gives the sibling, one wavefront searches the built node
+// and one its sibling. The histograms are stored for the next level only (not at a tree's last one, which holds half of a
+// tree's nodes) and not read back. NW follows from the items per pair (launch_merge_eval). ROOT: level 0, with a feature
+// stored in every row, whose bins every workgroup adds up as well: they are the node's sums.
+template <int NW, bool ROOT>
 __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int level, float mcw, float lambda, bool store) {
     __shared__ longlong2 s_sum[NW][kEvalPackBins];
     __shared__ GHPair s_miss[2][kEvalPackBins];
+    __shared__ longlong2 s_root[NW];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int p = blockIdx.y, pack = blockIdx.x;
     const int built = tb.hpair_built[p];
@@ -1234,74 +1236,121 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
     const int off = (1 << level) - 1, n_bins = tb.n_bins;
     const int b_begin = tb.pack_begin[pack], b_end = tb.pack_begin[pack + 1], nb = b_end - b_begin;
     const int ib = tb.hpair_begin[p], ie = tb.hpair_begin[p + 1];
-    // (every thread below kEvalPackBins carries one bin of the pack from here to the search)
-    const bool carrier = threadIdx.x < kEvalPackBins && (int)threadIdx.x < nb;
-    longlong2 parent = make_longlong2(0, 0);
-    if (carrier) parent = tb.hist(level + 1)[(size_t)p * n_bins + b_begin + threadIdx.x];
-    const int sibling = (built & 1) ? built + 1 : built - 1;
-    const GHPair S = tb.nodes[w == 0 ? built : sibling].sum_gh_pair;
-    const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
-    long long g[4] = {0, 0, 0, 0}, h[4] = {0, 0, 0, 0};
-    int at[4];  // (bins past the pack's end repeat its last one: all loads of an item are issued at once)
+    // (the first threads carry one bin of the pack each - with two wavefronts two bins - from here to the search)
+    constexpr int C = NW * 64 < kEvalPackBins ? kEvalPackBins / (NW * 64) : 1;
+    longlong2 parent[C];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) at[j] = b_begin + min(j * 64 + lane, nb - 1);
+    for (int c = 0; c < C; ++c) {
+        const int b = c * NW * 64 + (int)threadIdx.x;
+        parent[c] = make_longlong2(0, 0);
+        if (!ROOT && b < nb) parent[c] = tb.hist(level + 1)[(size_t)p * n_bins + b_begin + b];
+    }
+    const int sibling = (built & 1) ? built + 1 : built - 1;
+    GHPair S{0, 0};
+    if (!ROOT) S = tb.nodes[w == 0 ? built : sibling].sum_gh_pair;
+    const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
     // every item counted at its own scale (item_shift): shift its sums to the tree's
     const int2 *__restrict__ shift = tb.hitem_shift;
-    if (tb.ctl[level].hchunk <= tb.quant->flush_rows) {  // packed 8-byte partials (see k_hist_dense)
-        const unsigned long long *__restrict__ packed = reinterpret_cast<const unsigned long long *>(tb.partial);
-        const int h_bits = tb.quant->h_bits;
-        const unsigned long long h_mask = (1ull << h_bits) - 1ull;
+    const bool packed = tb.ctl[level].hchunk <= tb.quant->flush_rows;  // 8-byte partials (see k_hist_dense)
+    const int h_bits = tb.quant->h_bits;
+    const unsigned long long h_mask = (1ull << h_bits) - 1ull;
+    // the bins [first, first + count) of all items that are this wavefront's turn, four per lane (past the end: the last
+    // one again, so that all loads of an item are issued at once)
+    auto add_items = [&](int first, int count, long long(&g)[4], long long(&h)[4]) {
+        int at[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            at[j] = first + min(j * 64 + lane, count - 1);
+            g[j] = h[j] = 0;
+        }
+        if (packed) {
+            const unsigned long long *__restrict__ from = reinterpret_cast<const unsigned long long *>(tb.partial);
 #pragma unroll 2
-        for (int it = ib + w; it < ie; it += NW) {
-            unsigned long long t[4];
+            for (int it = ib + w; it < ie; it += NW) {
+                unsigned long long t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) t[j] = packed[(size_t)it * n_bins + at[j]];
-            const int2 sh = shift[it];
+                for (int j = 0; j < 4; ++j) t[j] = from[(size_t)it * n_bins + at[j]];
+                const int2 sh = shift[it];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const unsigned long long lo = t[j] & h_mask;
-                g[j] += ((long long)(t[j] - lo) >> h_bits) << sh.x;
-                h[j] += (long long)lo << sh.y;
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned long long lo = t[j] & h_mask;
+                    g[j] += ((long long)(t[j] - lo) >> h_bits) << sh.x;
+                    h[j] += (long long)lo << sh.y;
+                }
+            }
+        } else {
+            for (int it = ib + w; it < ie; it += NW) {
+                longlong2 v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = tb.partial[(size_t)it * n_bins + at[j]];
+                const int2 sh = shift[it];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    g[j] += v[j].x << sh.x;
+                    h[j] += v[j].y << sh.y;
+                }
             }
         }
-    } else {
-        for (int it = ib + w; it < ie; it += NW) {
-            longlong2 v[4];
+    };
+    if constexpr (ROOT) {
+        const int b0 = tb.cut_row_ptr[tb.complete_feature], kf = tb.cut_row_ptr[tb.complete_feature + 1] - b0;
+        long long g[4], h[4], G = 0, H = 0;
+        add_items(b0, kf, g, h);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = tb.partial[(size_t)it * n_bins + at[j]];
-            const int2 sh = shift[it];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                g[j] += v[j].x << sh.x;
-                h[j] += v[j].y << sh.y;
-            }
+        for (int j = 0; j < 4; ++j) {
+            G += j * 64 + lane < kf ? g[j] : 0;
+            H += j * 64 + lane < kf ? h[j] : 0;
         }
+        G = wave_sum_ll(G);
+        H = wave_sum_ll(H);
+        if (lane == 0) s_root[w] = make_longlong2(G, H);
     }
+    {
+        long long g[4], h[4];
+        add_items(b_begin, nb, g, h);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s_sum[w][j * 64 + lane] = make_longlong2(g[j], h[j]);
+        for (int j = 0; j < 4; ++j) s_sum[w][j * 64 + lane] = make_longlong2(g[j], h[j]);
+    }
     __syncthreads();
-    longlong2 sum = make_longlong2(0, 0);
-    if (carrier) {
+    longlong2 sum[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int b = c * NW * 64 + (int)threadIdx.x;
+        sum[c] = make_longlong2(0, 0);
+        if (b >= nb) continue;
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
-            const longlong2 v = s_sum[i][threadIdx.x];
-            sum.x += v.x;
-            sum.y += v.y;
+            const longlong2 v = s_sum[i][b];
+            sum[c].x += v.x;
+            sum[c].y += v.y;
         }
     }
     __syncthreads();
-    if (carrier) {
-        const longlong2 other = make_longlong2(parent.x - sum.x, parent.y - sum.y);
-        s_sum[0][threadIdx.x] = sum;
-        s_sum[1][threadIdx.x] = other;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int b = c * NW * 64 + (int)threadIdx.x;
+        if (b >= nb) continue;
+        const longlong2 other = make_longlong2(parent[c].x - sum[c].x, parent[c].y - sum[c].y);
+        s_sum[0][b] = sum[c];
+        if (!ROOT) s_sum[1][b] = other;
         if (store) {
-            tb.hist(level)[(size_t)(built - off) * n_bins + b_begin + threadIdx.x] = sum;
-            tb.hist(level)[(size_t)(sibling - off) * n_bins + b_begin + threadIdx.x] = other;
+            tb.hist(level)[(size_t)(built - off) * n_bins + b_begin + b] = sum[c];
+            if (!ROOT) tb.hist(level)[(size_t)(sibling - off) * n_bins + b_begin + b] = other;
         }
     }
     __syncthreads();
-    if (w < 2)
-        search_pack(tb, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
+    if (w >= (ROOT ? 1 : 2)) return;
+    if constexpr (ROOT) {
+        long long G = 0, H = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            G += s_root[i].x;
+            H += s_root[i].y;
+        }
+        S = root_sums(tb, G, H);
+        if (pack == 0 && lane == 0) set_root_sums(tb, S, lambda);
+    }
+    search_pack(tb, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
 // Split search for features of any number of bins (max_num_bin above 255): one workgroup per (feature, node) walks the
@@ -1939,7 +1988,7 @@ struct TreeEndArgs {
 // position -> row -> bin -> leaf -> prediction one round of loads (500 k rows: 28 us with 256 threads, 14 with 1024);
 // beyond that the registers of the 1024 cost residency (10 M rows: 74 and 128 us).
 constexpr int kEndWide = 1024;
-bool end_wide(int n) { return row_blocks(n) <= 512; }
+bool end_wide(int n, int n_class = 1) { return (long)row_blocks(n) * n_class <= 512; }
 constexpr int kEndInline = 8;                        // shorter sub-ranges are handled by the finding thread
 constexpr int kEndListCap = kRowBlock / kEndInline;  // so at most this many longer ones exist per block
 
@@ -2585,10 +2634,9 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
 }
 
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
-                       bool store_sibling, bool root, bool derive) {
+                       bool store_sibling, bool derive) {
     dim3 grid((tb.n_packs + kWaves - 1) / kWaves, tb.nodes_served(level), n_class);
-    if (root) k_eval_split<false, true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
-    else if (tb.sparse || derive) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
+    if (tb.sparse || derive) k_eval_split<true><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling);
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
 }
 
@@ -2596,10 +2644,25 @@ void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mc
     const int n_pairs = tb.n_hpairs(level);
     const dim3 grid(tb.n_packs, n_pairs, n_class);
     // (as many items as the level can have, see hist_dense_launch)
-    const int items = std::min(tb.target_hitems, tb.n / 2 / kHistMinChunk + n_pairs), per_pair = items / n_pairs;
-    if (per_pair > 32) k_merge_eval<16><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
-    else if (per_pair > 8) k_merge_eval<8><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
-    else k_merge_eval<4><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+    const int items = std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
+    if (level == 0) {
+        // One workgroup per pack: with hundreds of items two launches that spread them over the chip are faster (512 items of
+        // 28 packs: 12 + 9 instead of 43 us; 23 items of 700 packs: 18 instead of 16 + 15).
+        if (items > 64) {
+            launch_hist_merge(s, tb, level, n_class);
+            k_eval_split<false, true><<<dim3((tb.n_packs + kWaves - 1) / kWaves, 1, n_class), kBlock, 0, s>>>(tb, level, mcw, lambda, true);
+        } else if (items > 8) {
+            k_merge_eval<16, true><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+        } else {
+            k_merge_eval<4, true><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+        }
+        return;
+    }
+    const int per_pair = items / n_pairs;
+    if (per_pair > 32) k_merge_eval<16, false><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+    else if (per_pair > 8) k_merge_eval<8, false><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
+    else if (per_pair > 2) k_merge_eval<4, false><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+    else k_merge_eval<2, false><<<grid, 128, 0, s>>>(tb, level, mcw, lambda, store);
 }
 
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
@@ -2632,7 +2695,7 @@ static void tree_end_launch(hipStream_t s, const TreeBuffers &tb, const DenseBin
     const dim3 grid(row_blocks(tb.n), 1, n_class);
     // (mode 0 has nothing per row to wait for)
     if (mode == 0) k_tree_end<0, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
-    else if (mode == 1 && end_wide(tb.n)) k_tree_end<1, SPARSE, kEndWide><<<grid, kEndWide, 0, s>>>(tb, d, c, a);
+    else if (mode == 1 && end_wide(tb.n, n_class)) k_tree_end<1, SPARSE, kEndWide><<<grid, kEndWide, 0, s>>>(tb, d, c, a);
     else if (mode == 1) k_tree_end<1, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
     else if (end_wide(tb.n)) k_tree_end<2, SPARSE, kEndWide><<<grid, kEndWide, 0, s>>>(tb, d, c, a);
     else k_tree_end<2, SPARSE, kBlock><<<grid, kBlock, 0, s>>>(tb, d, c, a);
