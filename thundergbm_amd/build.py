@@ -9,7 +9,7 @@ LIB = os.path.join(HERE, "libthundergbm.so")
 CALIBRATION_LIB = os.path.join(HERE, "libtgbm_calibration.so")
 BIN_DIR = os.path.join(HERE, "bin")
 
-HIP_SOURCES = ["tree_kernels.hip", "level_kernels.hip", "sparse_kernels.hip", "prep_kernels.hip", "predict_kernels.hip", "rank_kernels.hip", "trainer.hip",
+HIP_SOURCES = ["tree_kernels.hip", "level_kernels.hip", "sparse_kernels.hip", "prep_kernels.hip", "cut_kernels.hip", "predict_kernels.hip", "rank_kernels.hip", "trainer.hip",
                "predictor.hip", "capi.hip", "predict_noalloc.hip", "device_memory.hip", "transfer.hip"]
 CPP_SOURCES = ["host_io.cpp"]
 

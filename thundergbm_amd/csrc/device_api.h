@@ -464,8 +464,8 @@ void launch_fill_u8(hipStream_t s, uint8_t *p, uint8_t v, size_t n);
 // F: columns of the matrix; feat_col / feat_lo: DenseBins' bundle tables or nullptr
 void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, const float *val, const float *cut_val,
                       const int *cut_row_ptr, uint8_t *binmat, int W, size_t block_stride, uint8_t *colmat,
-                      size_t col_stride, int bin_bytes, int F, const int *feat_col = nullptr,
-                      const uint8_t *feat_lo = nullptr, bool rows_ascend = true);
+                      size_t col_stride, int bin_bytes, int F, const int *feat_col,
+                      const uint8_t *feat_lo, bool rows_ascend, int n_features, int n_bins);
 // false when some row holds a column index below its predecessor's
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col);
 // min_next[c] (pre-filled with INT_MAX) = smallest column index that follows column c in a row (equal neighbours, a
@@ -482,7 +482,12 @@ struct DeviceCuts {
     int n_bins = 0;
     std::vector<long> feature_nnz;  // host: stored values per feature
 };
-DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin);
+// full_rows: every row stores every column, in order (d_val is a row-major matrix)
+DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin,
+                            bool full_rows = false);
+// (at most 256 features, or full rows)
+DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, bool full_rows,
+                                       int max_num_bin);
 
 // Tile sums of the device-wide exclusive scan, one pair of arrays per recursion level (grown on demand).
 struct ScanScratch {

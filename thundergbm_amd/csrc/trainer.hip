@@ -114,7 +114,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     }
     log_info("Fast getting cut points...");
     auto t_cut = std::chrono::steady_clock::now();
-    cuts_ = build_cut_points(stream_, F_, nnz_, d_val, d_col, param_.max_num_bin);
+    cuts_ = build_cut_points(stream_, F_, nnz_, d_val, d_col, param_.max_num_bin, ds.is_dense() && nnz_ == (long)n_ * ds.dense_columns);
     log_debug("cut points: %.3f s", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_cut).count());
     auto t_bin = std::chrono::steady_clock::now();
     n_bins_ = cuts_.n_bins;
@@ -408,7 +408,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         if (!ascend_known && nnz_ != (long)n_ * F_) rows_ascend = device_rows_ascend(stream_, n_, d_row_ptr, d_col);
         if (!rows_ascend) log_info("rows with descending column indices: the dense bins are filled row by row");
         launch_bin_dense(stream_, n_, d_row_ptr, d_col, d_val, cuts_.cut_val, cuts_.cut_row_ptr, d_binmat_, W,
-                         bins_.block_stride, d_colmat, col_stride, bin_bytes, P, bins_.feat_col, bins_.feat_lo, rows_ascend);
+                         bins_.block_stride, d_colmat, col_stride, bin_bytes, P, bins_.feat_col, bins_.feat_lo, rows_ascend, F_, n_bins_);
         bins_.col = d_colmat;
         bins_.col_stride = col_stride;
         bins_.data = d_binmat_;
