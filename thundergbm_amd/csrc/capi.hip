@@ -74,6 +74,7 @@ void run_train(GBMParam &p, const DataSet &ds, int *num_class, tgbm_model **mode
     TGBM_CHECK((int)boosted.size() == n_trees, "%d v.s. %zu", n_trees, boosted.size());
     *tree_per_iter = (int)boosted[0].size();
     *model = from_nested(boosted);
+    if (objective_needs_group_label(p.objective)) *num_class = (int)ds.label.size();  // (the labels may come with the training)
     for (size_t i = 0; i < ds.label.size(); ++i) group_label[i] = ds.label[i];
 }
 
@@ -147,7 +148,7 @@ void sparse_train_scikit(int row_size, float *val, int *row_ptr, int *col_ptr, f
                              column_sampling_rate, bagging, n_parallel_trees, learning_rate, obj_type, *num_class, tree_method);
     DataSet ds;
     auto t0 = std::chrono::steady_clock::now();
-    ds.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false);
+    ds.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false, true);
     log_debug("host-side dataset checks and label grouping: %.3f s",
               std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
     run_train(p, ds, num_class, model, tree_per_iter, group_label);
@@ -166,7 +167,7 @@ void tgbm_train_dense(int row_size, int columns, const void *x, int x_is_double,
     if (row_size > 4096) counter = std::thread([&] { *n_distinct = count_distinct(label, row_size); });
     else *n_distinct = count_distinct(label, row_size);
     DataSet ds;
-    ds.load_from_dense(row_size, columns, x, x_is_double != 0, label, group, num_group, p);
+    ds.load_from_dense(row_size, columns, x, x_is_double != 0, label, group, num_group, p, true);
     run_train(p, ds, num_class, model, tree_per_iter, group_label);
     if (counter.joinable()) counter.join();
 }
@@ -348,7 +349,7 @@ tgbm_trainer *tgbm_trainer_create_grouped(int row_size, const float *val, const 
     p.num_class = num_class;
     p.verbose = verbose;
     p.tree_method = "hist";
-    t->dataset.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false);
+    t->dataset.load_from_sparse(row_size, val, row_ptr, col_ptr, label, group, num_group, p, false, true);
     t->impl.reset(new Trainer(t->dataset, p));
     t->dataset.val = nullptr;  // the caller's buffers are not referenced after this call
     t->dataset.col_idx = nullptr;

@@ -3,6 +3,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <functional>
+#include <memory>
 #include <vector>
 
 #include "common.h"
@@ -547,9 +550,40 @@ void upload_large(hipStream_t s, void *dst, const void *src, size_t bytes);
 // The same for doubles that the device takes as floats. Zeros of either sign arrive as +0, other values that are too
 // small for a float as -0.
 void upload_doubles_as_floats(hipStream_t s, float *dst, const double *src, size_t count);
-// Column indices, which cross PCIe as bytes or 16-bit words where they all fit; anything else (negative ones too)
-// arrives as it is.
-void upload_columns(hipStream_t s, int *dst, const int *src, size_t count);
+// Several arrays at once: the threads convert and copy one while another crosses PCIe.
+class UploadSet {
+   public:
+    void add(void *dst, const void *src, size_t bytes);
+    void add_doubles(float *dst, const double *src, size_t count);
+    // Column indices, which cross PCIe as bytes or 16-bit words where they all fit; anything else (negative ones too)
+    // arrives as it is.
+    void add_columns(int *dst, const int *src, size_t count);
+    // an array that another thread is still making: source() waits for it; it is sent last
+    void add_late(void *dst, size_t bytes, std::function<const void *()> source);
+    void send(hipStream_t s);  // once
+
+   private:
+    struct Job {
+        void *dst;
+        size_t bytes;
+        std::function<const void *()> source;                              // the bytes as they are, or:
+        std::function<void(char *to, size_t offset, size_t length)> fill;  // writes bytes [offset, offset + length) of them
+        bool late;
+    };
+    friend void send_jobs(hipStream_t s, const std::vector<Job> &jobs, int threads);
+    struct Columns {
+        int *dst;
+        const int *src;
+        size_t count;
+        int width;  // bytes of the narrow form
+        void *narrow;
+        std::shared_ptr<std::atomic<bool>> fits;
+    };
+    template <typename Narrow>
+    bool add_narrow(int *dst, const int *src, size_t count);
+    std::vector<Job> jobs_;
+    std::vector<Columns> columns_;
+};
 // The conversion alone, for arrays that the device reads from host memory.
 void doubles_to_floats(float *to, const double *from, size_t count);
 // A pinned block of kPinnedBytes that the device can read and write directly; kept for later calls.

@@ -1,5 +1,6 @@
 // Host-side pieces that mirror the reference's DataSet, Parser, TreeTrainer and Predictor.
 #pragma once
+#include <future>
 #include <memory>
 #include <new>
 #include <string>
@@ -63,10 +64,14 @@ struct DataSet {
     // where the scan of a few hundred million indices costs a fraction of a millisecond instead of tens
     void load_from_sparse(int n_instances, const float *csr_val, const int *csr_row_ptr, const int *csr_col_idx,
                           const float *y, const int *group, int num_group, GBMParam &param,
-                          bool count_features = true);
+                          bool count_features = true, bool labels_later = false);
     // x: float or double [n_rows][columns]; the caller's buffer, like the CSR arrays
     void load_from_dense(int n_rows, int columns, const void *x, bool doubles, const float *labels, const int *group,
-                         int num_group, GBMParam &param);
+                         int num_group, GBMParam &param, bool labels_later = false);
+    // labels_later: for many rows a thread checks row_ptr, copies the labels and groups them while the caller uploads the
+    // matrix; y, label and param.num_class count after labels_ready().
+    void labels_ready(GBMParam &param) const;
+    const float *labels_when_ready() const;  // (for any thread)
     // src/thundergbm/dataset.cpp:170-320 (LIBSVM text, 1-based feature ids)
     void load_from_file(const std::string &file_name, GBMParam &param);
     // src/thundergbm/dataset.cpp:83-101
@@ -75,7 +80,8 @@ struct DataSet {
     void load_group_file(const std::string &file_name);
 
    private:
-    void take_labels(int n_rows, const float *labels);
+    std::shared_future<void> label_job_;
+    void make_labels(int n_rows, const int *row_ptr, const float *labels, const GBMParam &param, bool later);
     void finish_load(bool labelled, const int *grp, int num_group, GBMParam &param);
 };
 

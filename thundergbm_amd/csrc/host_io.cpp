@@ -88,17 +88,11 @@ bool descends(const int *v, size_t n) {
 
 void DataSet::load_from_sparse(int n_rows, const float *val, const int *row_ptr, const int *col_idx,
                                const float *labels, const int *grp, int num_group, GBMParam &param,
-                               bool count_features) {
+                               bool count_features, bool labels_later) {
     TGBM_CHECK(n_rows >= 0 && row_ptr != nullptr, "CSR input: %d rows", n_rows);
     TGBM_CHECK(row_ptr[0] == 0, "CSR input: row_ptr[0] is %d, expected 0", row_ptr[0]);
-    on_threads((size_t)n_rows, [&](int, size_t b, size_t e) {
-        if (!descends(row_ptr + b, e - b)) return;
-        for (size_t i = b; i < e; ++i)
-            TGBM_CHECK(row_ptr[i + 1] >= row_ptr[i], "CSR input: row_ptr decreases at row %zu (%d -> %d)", i, row_ptr[i],
-                       row_ptr[i + 1]);
-    });
     const int nnz = row_ptr[n_rows];
-    take_labels(n_rows, labels);
+    make_labels(n_rows, row_ptr, labels, param, labels_later && nnz >= 0);
     this->val = val;
     this->row_ptr = row_ptr;
     this->col_idx = col_idx;
@@ -133,9 +127,9 @@ void DataSet::load_from_sparse(int n_rows, const float *val, const int *row_ptr,
 }
 
 void DataSet::load_from_dense(int n_rows, int columns, const void *x, bool doubles, const float *labels, const int *grp,
-                              int num_group, GBMParam &param) {
+                              int num_group, GBMParam &param, bool labels_later) {
     TGBM_CHECK(n_rows > 0 && columns > 0 && x != nullptr, "dense input of %d x %d", n_rows, columns);
-    take_labels(n_rows, labels);
+    make_labels(n_rows, nullptr, labels, param, labels_later);
     dense_f32 = doubles ? nullptr : static_cast<const float *>(x);
     dense_f64 = doubles ? static_cast<const double *>(x) : nullptr;
     dense_columns = columns;
@@ -143,24 +137,46 @@ void DataSet::load_from_dense(int n_rows, int columns, const void *x, bool doubl
     finish_load(labels != nullptr, grp, num_group, param);
 }
 
-void DataSet::take_labels(int n_rows, const float *labels) {
+void DataSet::make_labels(int n_rows, const int *row_ptr, const float *labels, const GBMParam &param, bool later) {
     n_features_ = 0;
     label.clear();
     group.clear();
+    label_job_ = {};
     y.clear();
-    if (labels == nullptr) {
-        y.assign(n_rows, 0.f);
-        return;
-    }
     y.resize((size_t)n_rows);  // (not filled: the threads touch the pages)
-    on_threads((size_t)n_rows, [&](int, size_t b, size_t e) { std::memcpy(y.data() + b, labels + b, (e - b) * sizeof(float)); });
+    const bool grouped = labels != nullptr && objective_needs_group_label(param.objective);
+    auto job = [this, n_rows, row_ptr, labels, grouped] {
+        if (row_ptr != nullptr)
+            on_threads((size_t)n_rows, [&](int, size_t b, size_t e) {
+                if (!descends(row_ptr + b, e - b)) return;
+                for (size_t i = b; i < e; ++i)
+                    TGBM_CHECK(row_ptr[i + 1] >= row_ptr[i], "CSR input: row_ptr decreases at row %zu (%d -> %d)", i, row_ptr[i],
+                               row_ptr[i + 1]);
+            });
+        if (labels == nullptr) {
+            std::fill(y.begin(), y.end(), 0.f);
+            return;
+        }
+        on_threads((size_t)n_rows, [&](int, size_t b, size_t e) { std::memcpy(y.data() + b, labels + b, (e - b) * sizeof(float)); });
+        if (grouped) group_label();
+    };
+    if (later && host_threads((size_t)n_rows) > 1) label_job_ = std::async(std::launch::async, job).share();
+    else job();
+}
+
+void DataSet::labels_ready(GBMParam &param) const {
+    if (!label_job_.valid()) return;
+    label_job_.wait();
+    if (objective_needs_group_label(param.objective)) param.num_class = (int)label.size();
+}
+
+const float *DataSet::labels_when_ready() const {
+    if (label_job_.valid()) label_job_.wait();
+    return y.data();
 }
 
 void DataSet::finish_load(bool labelled, const int *grp, int num_group, GBMParam &param) {
-    if (labelled && objective_needs_group_label(param.objective)) {
-        group_label();
-        param.num_class = (int)label.size();
-    }
+    if (!label_job_.valid() && labelled && objective_needs_group_label(param.objective)) param.num_class = (int)label.size();
     // query group sizes of the ranking objectives (dataset.cpp:64-68)
     if (objective_needs_groups(param.objective)) {
         for (int i = 0; i < num_group; ++i) group.push_back(grp[i]);

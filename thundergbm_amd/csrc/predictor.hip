@@ -349,8 +349,10 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz, 1l));
         device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz, 1l));
         device_alloc_to(d_row_ptr, sizeof(int) * ((size_t)n + 1));
-        upload_large(s_up, d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n + 1));
-        if (nnz) upload_columns(s_up, d_col, ds.col_idx, (size_t)nnz);
+        UploadSet first;
+        first.add(d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n + 1));
+        if (nnz) first.add_columns(d_col, ds.col_idx, (size_t)nnz);
+        first.send(s_up);
         if (!ds.features_counted) F = device_max_int(s_up, d_col, nnz) + 1;
         narrow = F <= kNarrowFeatures;
         done = usable;
@@ -358,8 +360,8 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         for (int r0 = 0; r0 < n;) {
             const long e0 = ds.row_ptr[r0];
             // last row whose entries still fit the slice (at least one row)
-            const int *first = ds.row_ptr + r0 + 1, *last = ds.row_ptr + n + 1;
-            int r1 = (int)(std::upper_bound(first, last, (int)std::min<long>(e0 + slice_entries, nnz)) - ds.row_ptr) - 1;
+            const int *from = ds.row_ptr + r0 + 1, *last = ds.row_ptr + n + 1;
+            int r1 = (int)(std::upper_bound(from, last, (int)std::min<long>(e0 + slice_entries, nnz)) - ds.row_ptr) - 1;
             r1 = std::max(r1, r0 + 1);
             const long e1 = ds.row_ptr[r1];
             if (e1 > e0) upload_large(s_up, d_val + e0, ds.val + e0, sizeof(float) * (size_t)(e1 - e0));

@@ -41,6 +41,39 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
                "max_num_bin %d out of the supported range 2..65535", param.max_num_bin);
     TGBM_CHECK(objective_supported(param.objective), "undefined objective %s", param.objective.c_str());
     TGBM_CHECK(param.column_sampling_rate > 0.f, "column_sampling_rate must be positive");
+    // ---- upload CSR, cut points, bin matrix --------------------------------------------------
+    float *d_val = nullptr;
+    int *d_col = nullptr, *d_row_ptr = nullptr;
+    auto t_up = std::chrono::steady_clock::now();
+    bool rows_ascend = true, ascend_known = false;
+    UploadSet up;  // the labels last: the host threads that group them start with the upload
+    d_y_ = dalloc<float>(n_);
+    up.add_late(d_y_, sizeof(float) * (size_t)n_, [&ds] { return ds.labels_when_ready(); });
+    if (ds.is_dense()) {
+        const size_t cells = (size_t)n_ * ds.dense_columns;
+        float *d_x = nullptr;
+        device_alloc_to(d_x, sizeof(float) * cells);
+        if (ds.dense_f64 != nullptr) up.add_doubles(d_x, ds.dense_f64, cells);
+        else up.add(d_x, ds.dense_f32, sizeof(float) * cells);
+        up.send(stream_);
+        const DeviceCsr csr = dense_to_csr(stream_, n_, ds.dense_columns, d_x, ds.dense_f64 != nullptr);
+        d_val = csr.val;
+        d_col = csr.col;
+        d_row_ptr = csr.row_ptr;
+        nnz_ = csr.nnz;
+        F_ = csr.n_features;
+        rows_ascend = ascend_known = true;
+        log_info("#instances = %d, #features = %d", n_, F_);
+    } else {
+        device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz_, 1l));
+        device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
+        device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
+        up.add(d_val, ds.val, sizeof(float) * (size_t)nnz_);
+        up.add_columns(d_col, ds.col_idx, (size_t)nnz_);
+        up.add(d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n_ + 1));
+        up.send(stream_);
+    }
+    ds.labels_ready(param);
     // class bookkeeping of TreeTrainer::train (src/thundergbm/trainer.cu:24-37)
     if (param.objective.find("multi:") != std::string::npos || param.objective.find("binary:") != std::string::npos) {
         int nc = (int)ds.label.size();
@@ -79,33 +112,6 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     }
     param_ = param;
 
-    // ---- upload CSR, cut points, bin matrix --------------------------------------------------
-    float *d_val = nullptr;
-    int *d_col = nullptr, *d_row_ptr = nullptr;
-    auto t_up = std::chrono::steady_clock::now();
-    bool rows_ascend = true, ascend_known = false;
-    if (ds.is_dense()) {
-        const size_t cells = (size_t)n_ * ds.dense_columns;
-        float *d_x = nullptr;
-        device_alloc_to(d_x, sizeof(float) * cells);
-        if (ds.dense_f64 != nullptr) upload_doubles_as_floats(stream_, d_x, ds.dense_f64, cells);
-        else upload_large(stream_, d_x, ds.dense_f32, sizeof(float) * cells);
-        const DeviceCsr csr = dense_to_csr(stream_, n_, ds.dense_columns, d_x, ds.dense_f64 != nullptr);
-        d_val = csr.val;
-        d_col = csr.col;
-        d_row_ptr = csr.row_ptr;
-        nnz_ = csr.nnz;
-        F_ = csr.n_features;
-        rows_ascend = ascend_known = true;
-        log_info("#instances = %d, #features = %d", n_, F_);
-    } else {
-        device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz_, 1l));
-        device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz_, 1l));
-        device_alloc_to(d_row_ptr, sizeof(int) * (size_t)(n_ + 1));
-        upload_large(stream_, d_val, ds.val, sizeof(float) * (size_t)nnz_);
-        upload_columns(stream_, d_col, ds.col_idx, (size_t)nnz_);
-        upload_large(stream_, d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n_ + 1));
-    }
     log_debug("upload of %.2f GB: %.3f s", (double)nnz_ * 8e-9,
               std::chrono::duration<double>(std::chrono::steady_clock::now() - t_up).count());
     if (!ds.is_dense() && !ds.features_counted) {  // the number of features = largest column index + 1 (dataset.cpp:40-46)
@@ -432,8 +438,6 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     }
 
     // ---- labels, predictions, gradients (Booster::init) --------------------------------------
-    d_y_ = dalloc<float>(n_);
-    upload_large(stream_, d_y_, ds.y.data(), sizeof(float) * (size_t)n_);
     log_debug("bin matrix: %.3f s", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_bin).count());
     auto t_rest = std::chrono::steady_clock::now();
     n_yp_ = (long)param_.num_class * n_;
