@@ -991,7 +991,7 @@ __global__ __launch_bounds__(kBlock) void k_part_count_csr(TreeBuffers tb_all, C
             nleft += right ? 0 : 1;
         }
     }
-    tb.goes_right[(size_t)item * kBlock + threadIdx.x] = (uint8_t)rights;  // (see k_part_count_dense)
+    tb.goes_right[(size_t)item * kBlock + threadIdx.x] = (uint8_t)rights;  // (bit k: the thread's k-th row)
     int tot = block_sum(nleft, lds);
     if (threadIdx.x == 0) tb.pitem_nleft[item] = tot;
 }
