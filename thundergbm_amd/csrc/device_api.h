@@ -186,6 +186,7 @@ struct SparseTask {
 // fit one tile; a workgroup of the search takes every n_rare_groups-th task.
 constexpr int kRareBlock = 512;
 constexpr int kRareTile = 4096;       // values per task at most
+constexpr int kRareTileLeast = 512;   // a value per thread: smaller tasks leave threads without one
 constexpr int kRareFeatures = 2048;   // features per task at most
 constexpr int kRareGroupTiles = 16;   // tasks of a search workgroup at most
 constexpr int kRareGroups = 512;      // search workgroups that are resident together (two per CU)

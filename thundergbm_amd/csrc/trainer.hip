@@ -891,11 +891,16 @@ void Trainer::build_sparse_tasks() {
         feat_slot[big[i].feature] = big[i].cand_slot;
     }
     int next_slot = n_small + (int)big.size();
+    // Full tiles where there are enough of them for every search workgroup that the chip holds; smaller data is dealt out
+    // over as many workgroups, because a level takes as long as its fullest tile: sorting and searching it is one chain.
     long n_rare = 0;
+    for (int f : rare_fid) n_rare += cuts_.feature_nnz[f];
+    const long tile_values = std::min<long>(kRareTile, std::max<long>(kRareTileLeast, n_rare / kRareGroups));
+    n_rare = 0;
     for (size_t i = 0; i < rare_fid.size();) {
         size_t e = i;
         long vals = 0;
-        while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && vals + cuts_.feature_nnz[rare_fid[e]] <= kRareTile)
+        while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && (e == i || vals + cuts_.feature_nnz[rare_fid[e]] <= tile_values))
             vals += cuts_.feature_nnz[rare_fid[e++]];
         rare_tasks.push_back(RareTask{(int)n_rare, (int)vals, (int)i, (int)(e - i)});
         n_rare += vals;
