@@ -1,0 +1,29 @@
+"""Host-side parts of the library compiled with g++ against a runtime that the test itself stands in for: no GPU, no
+HIP runtime."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture
+def run_native(tmp_path):
+    def run(source, *more):
+        exe = str(tmp_path / source.rsplit(".", 1)[0])
+        subprocess.check_call(["g++", "-std=c++17", "-O1", "-w", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                               "-x", "c++", os.path.join(HERE, "native", source)] + list(more) + ["-o", exe])
+        out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+        assert out.returncode == 0, out.stdout + out.stderr
+        return out.stdout
+    return run
+
+
+def test_lds_limit_of_a_kernel_is_set_once_and_to_the_most(run_native):
+    """A limit that follows the launches' sizes can be lowered by one thread between another's call and its launch."""
+    run_native("lds_opt_in.cpp")
+    csrc = os.path.join(os.path.dirname(HERE), "thundergbm_amd", "csrc")
+    setters = [f for f in sorted(os.listdir(csrc)) if os.path.isfile(os.path.join(csrc, f)) and
+               "hipFuncSetAttribute" in open(os.path.join(csrc, f)).read()]
+    assert setters == ["device_api.h"]

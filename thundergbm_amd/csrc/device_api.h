@@ -5,7 +5,9 @@
 
 #include <atomic>
 #include <functional>
+#include <initializer_list>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.h"
@@ -37,6 +39,30 @@ void device_alloc_to(T *&p, size_t bytes) {
     p = static_cast<T *>(device_alloc(bytes));
 }
 void device_mem_info(size_t *free_b, size_t *total_b);
+
+// More dynamic LDS than the default window, for kernels of one launcher: a static object of the launcher, called before
+// each launch. The limit belongs to the kernel, not to a launch, so it is set once per device and to the most that the
+// kernel can take: set to a launch's own size, it could fall below that of another thread between its call and its launch.
+constexpr int kLdsBytes = 160 * 1024;
+class LdsOptIn {
+  public:
+    void operator()(std::initializer_list<const void *> kernels) {
+        int dev = 0;
+        HIP_CHECK(hipGetDevice(&dev));
+        TGBM_CHECK(dev < kDevices, "device %d: more than %d devices", dev, kDevices);
+        std::call_once(once_[dev], [&] {
+            for (const void *k : kernels) {
+                hipFuncAttributes a;
+                HIP_CHECK(hipFuncGetAttributes(&a, k));
+                HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes - (int)a.sharedSizeBytes));
+            }
+        });
+    }
+
+  private:
+    static constexpr int kDevices = 64;
+    std::once_flag once_[kDevices];
+};
 hipStream_t stream_acquire();
 void stream_release(hipStream_t s);
 

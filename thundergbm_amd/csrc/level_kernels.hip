@@ -548,19 +548,16 @@ static size_t small_lds(const TreeBuffers &tb) {
 // 32 columns that takes longer at the first levels than the launches that are saved.
 bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins) {
     return tb.n <= kSmallRows && tb.depth <= kSmallDepth && (long)(tb.n / 2) * std::min(bins.W, bins.n_cols) <= 1l << 18 &&
-           small_lds(tb) + 4096 <= 160 * 1024;
+           small_lds(tb) + 4096 <= kLdsBytes;
 }
 
 template <int LPR, bool BIN16>
 static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
                                float rt_eps, float lambda, int n_class) {
     const size_t lds = small_lds(tb);
-    static size_t opted = 0;
-    if (lds > 48 * 1024 && lds > opted) {  // (with the kernel's own tables more than the default window)
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_level<LPR, BIN16>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        opted = lds;
-    }
+    static LdsOptIn opt_in;
+    if (lds > 48 * 1024)  // (with the kernel's own tables more than the default window)
+        opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16>)});
     k_small_level<LPR, BIN16><<<dim3(bins.n_blocks, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda);
 }
 

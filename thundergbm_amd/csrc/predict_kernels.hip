@@ -589,10 +589,10 @@ bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, boo
             if (narrow) TGBM_SCORE_GROUP(64, true);
             else TGBM_SCORE_GROUP(64, false);
         } else {
+            static LdsOptIn opt_in;
             if (lds > 64 * 1024)  // (what a kernel may ask for without saying so)
-                HIP_CHECK(hipFuncSetAttribute(narrow ? reinterpret_cast<const void *>(&k_score_group<256, true>)
-                                                     : reinterpret_cast<const void *>(&k_score_group<256, false>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                opt_in({reinterpret_cast<const void *>(&k_score_group<256, true>),
+                        reinterpret_cast<const void *>(&k_score_group<256, false>)});
             if (narrow) TGBM_SCORE_GROUP(256, true);
             else TGBM_SCORE_GROUP(256, false);
         }

@@ -1005,15 +1005,8 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
             launch_fill_f32(s, reinterpret_cast<float *>(tb.for_class(k).hist(level)), 0.f,
                             (size_t)(1 << level) * tb.n_bins * 4);
     }
-    static bool opted = false;
-    if (!opted) {  // more than the default dynamic LDS window: opt in once
-        const size_t lds_max = sizeof(longlong2) * (size_t)kSparseCells;
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_sparse_level),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_sparse_big),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
-        opted = true;
-    }
+    static LdsOptIn opt_in;
+    opt_in({reinterpret_cast<const void *>(&k_sparse_level), reinterpret_cast<const void *>(&k_sparse_big)});
     if (sp.n_tasks > 0)
         k_sparse_level<<<dim3(sp.n_tasks, 1, n_class), kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda,
                                                                           dump_hist ? 1 : 0, n_cells);

@@ -2478,31 +2478,16 @@ static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseB
     dim3 grid(bins.n_blocks, (unsigned)std::max(1l, std::min({by_rows, by_target, (long)tb.max_hitems})), n_class);
     size_t lds = (size_t)tb.max_block_bins * sizeof(unsigned long long);
     if (lds > 64 * 1024) {
-        // more than the default dynamic LDS window: opt in once per kernel instance and size
-        static size_t opted = 0;
-        if (lds > opted) {
-            HIP_CHECK(hipFuncSetAttribute(
-                reinterpret_cast<const void *>(&k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            HIP_CHECK(hipFuncSetAttribute(
-                reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            opted = lds;
-        }
+        static LdsOptIn opt_in;
+        opt_in({reinterpret_cast<const void *>(&k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16>),
+                reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16>)});
     }
     if constexpr (!BIN16 && LPR >= 4) {
         if (bins.gh_lane >= 0 && bins.gh_fresh) {
             if (lds > 64 * 1024) {
-                static size_t opted_w = 0;
-                if (lds > opted_w) {
-                    HIP_CHECK(hipFuncSetAttribute(
-                        reinterpret_cast<const void *>(&k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                    HIP_CHECK(hipFuncSetAttribute(
-                        reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                    opted_w = lds;
-                }
+                static LdsOptIn opt_in_words;
+                opt_in_words({reinterpret_cast<const void *>(&k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true>),
+                              reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true>)});
             }
             if (level == 0)
                 k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs);
@@ -2607,14 +2592,8 @@ void launch_hist_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, 
     k_hist_zero_built<<<dim3(zgrid, tb.hpair_hi(level) - tb.hpair_lo(level), n_class), kBlock, 0, s>>>(tb, level);
     const size_t lds = (size_t)bins.head_bins * 2 * sizeof(unsigned long long);
     if (bins.hist_word != nullptr && lds > 64 * 1024) {
-        static size_t opted = 0;  // more than the default dynamic LDS window: opt in once
-        if (lds > opted) {
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_hist_csr_head<true>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_hist_csr_head<false>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            opted = lds;
-        }
+        static LdsOptIn opt_in;
+        opt_in({reinterpret_cast<const void *>(&k_hist_csr_head<true>), reinterpret_cast<const void *>(&k_hist_csr_head<false>)});
     }
     if (level == 0 && bins.csc_row != nullptr) {
         const long tiles = (bins.nnz + 63) / 64;
