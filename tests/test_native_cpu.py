@@ -27,3 +27,9 @@ def test_lds_limit_of_a_kernel_is_set_once_and_to_the_most(run_native):
     setters = [f for f in sorted(os.listdir(csrc)) if os.path.isfile(os.path.join(csrc, f)) and
                "hipFuncSetAttribute" in open(os.path.join(csrc, f)).read()]
     assert setters == ["device_api.h"]
+
+
+def test_sums_lie_in_the_range_of_their_codes(run_native):
+    """The filter of the rare features may exclude a run only by a true bound on its candidates' sums: an end that is
+    scaled up moves inwards where the whole range is on one side of zero."""
+    run_native("rare_range.cpp")

@@ -15,6 +15,7 @@
 
 #include "device_api.h"
 #include "kernel_common.h"
+#include "rare_bound.h"
 
 namespace tgbm {
 namespace {
@@ -397,46 +398,21 @@ constexpr int kRareMaxGroups = 64;
 constexpr int kRareLds = kRareTile + kRareTile / 32;
 __device__ __forceinline__ int rare_phys(int i) { return i + (i >> 5); }
 
-// row word: node of the level (11 bits, all ones: the row has come to rest above), sign of g, |g| (10 bits, rounded up), h
-// (10 bits, rounded down)
-constexpr unsigned kRareNodeMask = 0x7ffu;
-constexpr float kRareSteps = 1022.f;
+// (the tree's largest as an integer too: rounded, a small one can exceed its product with the scale)
 __device__ __forceinline__ unsigned rare_row_word(unsigned node, GHPair s, const QuantCtl &q) {
-    // (of the integers that the sums are made of)
-    const float g = fabsf((float)round_to_ll(s.g * q.scale_g)), h = (float)round_to_ll(s.h * q.scale_h);
-    const unsigned cg = g > 0.f ? min(1023u, (unsigned)ceilf(g * (kRareSteps / q.gq_max))) : 0u;
-    const unsigned ch = h > 0.f ? min(1023u, (unsigned)(h * (kRareSteps / q.hq_max))) : 0u;
-    return node | (s.g < 0.f ? 1u << 11 : 0u) | cg << 12 | ch << 22;
-}
-struct RareCell {
-    unsigned long long g;  // sums of the positive g (22 bits) and of the negative g (22), values (13)
-    unsigned h;            // sum of h
-    __device__ int plus() const { return (int)((unsigned)g & 0x3fffffu); }
-    __device__ int minus() const { return (int)((unsigned)(g >> 22) & 0x3fffffu); }
-    __device__ int values() const { return (int)(g >> 44); }
-};
-__device__ __forceinline__ RareCell operator+(RareCell a, RareCell b) { return {a.g + b.g, a.h + b.h}; }
-__device__ __forceinline__ RareCell operator-(RareCell a, RareCell b) { return {a.g - b.g, a.h - b.h}; }
-__device__ __forceinline__ unsigned long long rare_addend(unsigned word) {
-    const unsigned long long g = (word >> 12) & 0x3ffu;
-    return 1ull << 44 | ((word >> 11 & 1u) ? g << 22 : g);
+    return rare_word(node, (float)round_to_ll(s.g * q.scale_g), (float)round_to_ll(s.h * q.scale_h),
+                     (float)round_to_ll(q.gq_max), (float)round_to_ll(q.hq_max));
 }
 static_assert(kRareTile * 1023 < 1 << 22 && kRareTile < 1 << 13, "fields of a cell");
 
-struct RareBound {
-    float g, h, mcw, lambda;  // one step of g and of h
-};
-
 // No candidate that splits off all of `whole` and some of the values of `part` reaches the gain `floor`.
 __device__ __forceinline__ bool rare_hopeless(RareCell whole, RareCell part, GHPair S, float P, float floor, RareBound u) {
-    constexpr float up = 1.f + 0x1p-12f, down = 1.f - 0x1p-12f;  // (roundings of the codes)
-    const float base = (float)(whole.plus() - whole.minus()), slack = 1.01f * (float)whole.values();
-    const float hi = (base + slack + (float)part.plus()) * u.g * up, lo = (base - slack - (float)part.minus()) * u.g * up;
-    const float eg = (fabsf(S.g) + fabsf(hi) + fabsf(lo)) * 0x1p-21f, eh = S.h * 0x1p-21f;
-    const float h_min = (float)whole.h * u.h * down - eh;
-    const float h_max = (float)((int)(whole.h + part.h) + whole.values() + part.values()) * u.h * up + eh;
+    const RareRange r = rare_range(whole, part, u);
+    // (the candidates' sums are differences of floats)
+    const float eg = (fabsf(S.g) + fabsf(r.g_max) + fabsf(r.g_min)) * 0x1p-21f, eh = S.h * 0x1p-21f;
+    const float h_min = r.h_min - eh, h_max = r.h_max + eh;
     if (h_max < u.mcw || S.h - h_min + eh < u.mcw) return true;  // one of the sides weighs too little
-    const float a = fmaxf(fabsf(hi), fabsf(lo)) + eg, b = fmaxf(fabsf(S.g - hi), fabsf(S.g - lo)) + eg;
+    const float a = fmaxf(fabsf(r.g_max), fabsf(r.g_min)) + eg, b = fmaxf(fabsf(S.g - r.g_max), fabsf(S.g - r.g_min)) + eg;
     const float t = a * a * __builtin_amdgcn_rcpf(fmaxf(u.mcw, h_min) + u.lambda) +
                     b * b * __builtin_amdgcn_rcpf(fmaxf(u.mcw, S.h - h_max) + u.lambda);
     return (t - P) + (t + fabsf(P)) * 0x1p-18f < floor;
@@ -773,8 +749,8 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
     if (threadIdx.x == 0) sh.passed = 0;
     RareNodes node(rare_dyn, nl);
     node.load(tb, nl, lambda);
-    const RareBound unit{tb.quant->gq_max * tb.quant->inv_g / kRareSteps, tb.quant->hq_max * tb.quant->inv_h / kRareSteps, mcw,
-                         lambda};
+    const RareBound unit{(float)round_to_ll(tb.quant->gq_max) * tb.quant->inv_g / kRareSteps,
+                         (float)round_to_ll(tb.quant->hq_max) * tb.quant->inv_h / kRareSteps, mcw, lambda};
     __syncthreads();
     int cell[kRareV];  // -1: the value takes no part
 #pragma unroll
