@@ -39,13 +39,36 @@ SHAPES = {
 }
 
 
-@pytest.mark.parametrize("shape", sorted(SHAPES))
-@pytest.mark.parametrize("objective,kw", [
+# The most frequent features go to tables whatever they hold (kRareExempt, kRareLeast): shapes around that rule, and around a
+# search with a value per thread.
+FREQUENT = {
+    "full_tiles": ([4500] * 128 + [4096, 4097, 4095, 1, 4096, 2048, 2048, 1], 5000),
+    "few_rows": ([257] * 60 + [256, 255, 1, 256, 256, 128, 128, 257, 2] * 8, 300),
+    "tiles_around_512": ([900] * 128 + [700, 512, 513, 1, 511] * 6, 1000),
+    "one_feature_more": ([400] * 129 + [400, 300], 600),
+    "few_values": ([3] * 20, 50),
+}
+OPTIONS = pytest.mark.parametrize("objective,kw", [
     ("reg:linear", {}), ("binary:logistic", {"min_child_weight": 5.0}), ("multi:softmax", {"num_class": 3}),
     ("reg:linear", {"lambda_": 0.0, "min_child_weight": 0.0, "sampled": True})])
+
+
+@pytest.mark.parametrize("shape", sorted(FREQUENT))
+@OPTIONS
+def test_features_at_the_edge_of_rare_equal_tables(T, shape, objective, kw):
+    val, rp, col, z = _by_feature(*FREQUENT[shape], 5)
+    compare(T, val, rp, col, (z - np.median(z)) / z.std(), objective, kw)
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@OPTIONS
 def test_rare_features_equal_tables(T, shape, objective, kw):
     counts, n = SHAPES[shape]
     val, rp, col, z = _by_feature(counts, n, 5)
+    compare(T, val, rp, col, z, objective, kw)
+
+
+def compare(T, val, rp, col, z, objective, kw):
     kw = dict(kw)
     sampled = kw.pop("sampled", False)
     y = (z if objective == "reg:linear" else np.digitize(z, [-0.5, 0.5][: 2 if "multi" in objective else 1])).astype(np.float32)

@@ -200,20 +200,24 @@ struct CsrBins {
 constexpr int kSparseCells = 8192;      // (node, bin) cells of 16 bytes an LDS table holds
 constexpr int kSparseMaxLevelNodes = 1024;  // deepest level the pass serves (depth <= 11)
 constexpr int kSparseBatchFeatures = 2047;  // features whose tables share one LDS batch at most
-constexpr int kSparseTaskValues = 32768;    // stored values per task (and per chunk of a big feature)
+constexpr int kSparseTaskValues = 32768;    // stored values per task at most (and per chunk of a big feature)
+constexpr int kSparseTasks = 1024;          // smaller tasks where there would be fewer than that
 struct SparseTask {
     int f_begin, f_end;  // features [f_begin, f_end) (a chunk task: one feature)
     int v_begin, v_end;  // positions of the bin-major copy
     int cand_slot;       // candidate slot the task fills, -1: a chunk (its feature's slot is filled by k_sparse_big)
     int partial_slot;    // chunk: where its table goes in SparsePass::partial, else -1
 };
-// Features with at most kRareTile stored values are not searched through tables: k_sparse_rare_filter looks for the (feature, node)
+// Features with few stored values (Trainer::sparse_feature_in_tables) are not searched through tables: k_sparse_rare_filter looks for the (feature, node)
 // runs of their values that could win at all and searches only those. A task is a run of whole features whose values
 // fit one tile; a workgroup of the search takes every n_rare_groups-th task.
 constexpr int kRareBlock = 512;
 constexpr int kRareTile = 4096;       // values per task at most
 constexpr int kRareTileLeast = 512;   // a value per thread: smaller tasks leave threads without one
 constexpr int kRareFeatures = 2048;   // features per task at most
+// Features with more than kRareLeast values (at most this many, the most frequent ones) are served through tables too.
+constexpr int kRareExempt = 128;
+constexpr int kRareLeast = 256;
 constexpr int kRareGroupTiles = 16;   // tasks of a search workgroup at most
 constexpr int kRareGroups = 512;      // search workgroups that are resident together (two per CU)
 struct RareTask {
@@ -234,7 +238,7 @@ struct SparsePass {
     int n_tasks = 0;
     const SparseBig *big = nullptr;
     int n_big = 0;
-    // rare features (at most kRareTile values)
+    // rare features
     const RareTask *rare_tasks = nullptr;
     int n_rare_tasks = 0, n_rare_groups = 0;
     int rare_slot = 0;                  // candidate slot of the first group

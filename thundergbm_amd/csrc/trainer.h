@@ -137,7 +137,7 @@ class Trainer {
     bool wide_eval_ = false;        // split search with one workgroup per (feature, node)
     int hist_cap_level_ = -1;       // first level with more nodes than the histogram arena holds (-1: none)
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
-    bool sparse_rare_on_ = true;
+    long sparse_rare_most_ = 0;  // a feature with more stored values is served through tables
     bool sparse_feature_in_tables(int f);
     SparsePass sp_;
     void build_sparse_tasks();

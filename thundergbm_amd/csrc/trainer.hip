@@ -262,10 +262,11 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         if (sparse_pass_) {
             // One byte per row (local bin id, 255 = no stored value) for the frequent features - the ones that win
             // most splits: the row -> node update then takes a row's side from one byte instead of searching the
-            // row's bin ids. As many of the table features, most frequent first, as fit an eighth of the free memory.
+            // row's bin ids. As many of the features with more than kRareTile values, most frequent first, as fit an
+            // eighth of the free memory.
             std::vector<int> order;
             for (int f = 0; f < F_; ++f)
-                if (cuts_.feature_nnz[f] > 0 && cuts_.feature_nnz[f] > kRareTile) order.push_back(f);
+                if (cuts_.feature_nnz[f] > kRareTile) order.push_back(f);
             std::stable_sort(order.begin(), order.end(),
                              [&](int a, int b) { return cuts_.feature_nnz[a] > cuts_.feature_nnz[b]; });
             device_mem_info(&free_b, &total_b);
@@ -819,28 +820,42 @@ void Trainer::ensure_hist_arena() {
 }
 
 // Which features the sparse level pass serves through (bin, node) tables: those with more values than a tile of rare
-// features holds, and the feature that owns global bin 0 (its table is searched for every node even without values: the
-// arg-max of a node without any positive gain ends there).
+// features holds, the most frequent ones of the others, and the feature that owns global bin 0 (its table is searched
+// for every node even without values: the arg-max of a node without any positive gain ends there).
+// The most frequent ones: on few rows a feature of a tile's size is no rare one. Its runs pass the filter, and sorting
+// and searching them is one chain that the whole level waits for, while a table of its own costs a workgroup on a CU that
+// is idle. 20 k x 100 k, depth 8: 0.93 ms a tree without the exemption, 0.51 with 64 to 512 features; 60 k rows, depth
+// 11: 1.98 without, 1.77 with 128, 2.80 with 256 (tables of deep levels fill the LDS: beyond a workgroup per CU a
+// second round begins). From 1 M rows on more features than that have over kRareTile values, and nothing changes.
 bool Trainer::sparse_feature_in_tables(int f) {
     if (sparse_bin0_owner_ == -2) {
         sparse_bin0_owner_ = -1;
         for (int q = 0; q < F_ && sparse_bin0_owner_ < 0; ++q)
             if (h_cut_row_ptr_[q + 1] > h_cut_row_ptr_[q]) sparse_bin0_owner_ = q;
         const char *se = std::getenv("TGBM_SPARSE_SORTED");  // "0": every feature through the tables (tests)
-        sparse_rare_on_ = !(se != nullptr && std::string(se) == "0");
+        std::vector<long> count(cuts_.feature_nnz);
+        count.resize(std::max<size_t>(count.size(), kRareExempt + 1), 0);
+        std::nth_element(count.begin(), count.begin() + kRareExempt, count.end(), std::greater<long>());
+        sparse_rare_most_ = se != nullptr && std::string(se) == "0"
+                                ? -1 : std::min<long>(kRareTile, std::max<long>(kRareLeast, count[kRareExempt]));
     }
-    return !sparse_rare_on_ || cuts_.feature_nnz[f] > kRareTile || f == sparse_bin0_owner_;
+    return cuts_.feature_nnz[f] > sparse_rare_most_ || f == sparse_bin0_owner_;
 }
 
-// Work lists of the sparse level pass. Features with at most kRareTile stored values go to k_sparse_rare_filter (tasks:
-// runs of such features whose values fit one tile); the others to table tasks: runs of consecutive such features
-// with about kSparseTaskValues values, a feature with more values than that cut into chunks (tasks of their own)
-// whose tables k_sparse_big adds up. The feature that owns global bin 0 is always a table feature (its table is
-// searched for every node even without values: the arg-max of a node without any positive gain ends there).
+// Work lists of the sparse level pass. Features with few stored values go to k_sparse_rare_filter (tasks: runs of such
+// features whose values fit one tile); the others to table tasks: runs of consecutive such features with about
+// task_values values, a feature with more than kSparseTaskValues cut into chunks (tasks of their own) whose tables
+// k_sparse_big adds up.
 void Trainer::build_sparse_tasks() {
     std::vector<int> fvb(F_ + 1, 0);
     for (int f = 0; f < F_; ++f) fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
+    // A task serves its features one after the other, about 12 us each at 128 nodes: where all tasks together do not fill the
+    // chip they are smaller (200 k x 100 k, depth 8, 67 tasks of 32768 values: 1.48 ms a tree, a thousandth of the values
+    // each: 1.05; 1 M rows: 2.63 -> 2.43).
+    long table_values = 0;
+    for (int f = 0; f < F_; ++f) table_values += is_table(f) ? cuts_.feature_nnz[f] : 0;
+    const long task_values = std::min<long>(kSparseTaskValues, std::max<long>(kRareLeast, table_values / kSparseTasks));
     std::vector<SparseTask> tasks;
     std::vector<SparseBig> big;
     std::vector<RareTask> rare_tasks;
@@ -877,7 +892,7 @@ void Trainer::build_sparse_tasks() {
         int fe = f;
         long vals = 0;
         while (fe < F_ && is_table(fe) && cuts_.feature_nnz[fe] <= kSparseTaskValues &&
-               vals + cuts_.feature_nnz[fe] <= kSparseTaskValues) {
+               (fe == f || vals + cuts_.feature_nnz[fe] <= task_values)) {
             vals += cuts_.feature_nnz[fe];
             ++fe;
         }
