@@ -73,6 +73,8 @@ constexpr int kMissingBin16 = 65535;  // the same for 16-bit bins
 constexpr int kDense16BlockBins = 8192;
 constexpr int kDense16MaxBlockBins = 20480;
 constexpr int kPartChunk = 2048;   // rows per partition work item (256 threads x 8 rounds)
+// Dense layout: up to so many pairs (nodes, where single nodes are built) in a level every workgroup plans for itself.
+constexpr int kUnplannedPairs = 256;
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
 constexpr int kCsrHeadBins = 4864;  // head slots of the sparse histogram: 2 x 8 bytes each, two workgroups per CU
 // Rows a packed LDS bin may absorb before it is drained (QuantCtl::flush_rows). With float hessians (32 + 32-bit
@@ -290,7 +292,7 @@ struct TreeBuffers {
     int max_hitems = 0, target_hitems = 0, max_pitems = 0;
     float *leaf_value = nullptr;   // [n_nodes] prediction increment of a row that ended in the node (after pruning)
     int *end_bound = nullptr;      // [(row_blocks(n) + 1) x (2^depth - 1)] list positions of the row block boundaries
-    int *hpair_begin = nullptr;    // [max_pairs + 1] first histogram item of every sibling pair
+    int *hpair_begin = nullptr;    // [max_level_nodes + 1] first histogram item of every sibling pair
     int4 *hpair_plan = nullptr;    // [max_pairs] dense layout: (hpair_built, its row-list segment), see plan_hist_item
     int *hpair_built = nullptr;    // [max_pairs] heap id of the node built from rows, -1 = inactive pair
     int *pitem_begin = nullptr;    // [2][max_level_nodes + 1] first partition item of every node of a level, by level parity
@@ -337,6 +339,7 @@ struct TreeBuffers {
     __host__ __device__ int n_hpairs(int level) const {
         return level == 0 ? 1 : (singles(level) ? (1 << level) : (1 << (level - 1)));
     }
+    __host__ __device__ bool planned(int level) const { return n_hpairs(level) > kUnplannedPairs; }
     __host__ __device__ int hpair_lo(int level) const { return singles(level) ? lvl_x0 : (lvl_x0 >> 1); }
     __host__ __device__ int hpair_hi(int level) const {  // end of the pairs of the served nodes
         const int n = n_hpairs(level);

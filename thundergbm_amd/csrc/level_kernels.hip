@@ -4,6 +4,8 @@
 // scan of the items' counts, the plan of the next level - is done again by every workgroup from a few hundred bytes
 // that it finds in the L2: a launch costs 4 to 8 us whatever it does, the repeated work well below one.
 // 500 k x 28, depth 8: five launches and 23 us a level (update 4.8, count 5.7, plan 5.5, scatter 4.9, gaps) -> two.
+// That holds up to 512 nodes. Deeper levels have 16 to 130 KB of plan and more items to repeat it for; they are planned by a
+// third launch (TreeBuffers::planned).
 #include <algorithm>
 
 #include "device_api.h"
@@ -31,6 +33,16 @@ __device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level
         out.x_in = item < out.count ? 0 : -1;
         out.first = 0;
         out.seg = make_int2(0, tb.n);
+        return out;
+    }
+    if (tb.planned(level)) {
+        const int *__restrict__ begin = tb.pbegin(level);
+        out.x_in = -1;
+        if (item >= begin[nl]) return out;
+        out.x_in = find_owner_wave(begin, nl, item);
+        out.first = begin[out.x_in];
+        out.count = begin[out.x_in + 1] - out.first;
+        out.seg = tb.seg[off + out.x_in];
         return out;
     }
     if (threadIdx.x == 0) s[0] = -1;
@@ -342,6 +354,61 @@ __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, in
     }
 }
 
+// The plan of a level of many nodes: its histogram work items (hpair_begin, ctl) and its nodes' partition items (pbegin), by
+// one workgroup. A thread has consecutive nodes, so that one scan serves them all.
+// 500 k x 28, depth 14: planned by every wavefront instead, the histogram launches of 512, 1024, 2048 and 4096 pairs took 25,
+// 55, 148 and 478 us and the partition of as many nodes twice 7, 12, 19 and 31.
+constexpr int kPlanBlock = 1024;
+__global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, int level, int n_pairs) {
+    constexpr int NW = kPlanBlock / 64;
+    __shared__ int lds[NW];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int nl = 1 << level, off = nl - 1;
+    const int pairs_each = (n_pairs + kPlanBlock - 1) / kPlanBlock, p0 = min(n_pairs, (int)threadIdx.x * pairs_each);
+    const int p1 = min(n_pairs, p0 + pairs_each);
+    int rows = 0, built = 0;
+    for (int p = p0; p < p1; ++p) {
+        const int4 q = tb.hpair_plan[p];
+        rows += q.x >= 0 ? q.z - q.y : 0;
+        built += q.x >= 0 ? 1 : 0;
+    }
+    int total, n_built, n_items;
+    block_excl_scan<NW>(rows, lds, &total);
+    block_excl_scan<NW>(built, lds, &n_built);
+    const int chunk = hist_chunk(tb, total, n_built);
+    auto hist_items = [&](int p) {
+        const int4 q = tb.hpair_plan[p];
+        return q.x >= 0 ? (q.z - q.y + chunk - 1) / chunk : 0;
+    };
+    int items = 0;
+    for (int p = p0; p < p1; ++p) items += hist_items(p);
+    int at = block_excl_scan<NW>(items, lds, &n_items);
+    for (int p = p0; p < p1; ++p) {
+        tb.hpair_begin[p] = at;
+        at += hist_items(p);
+    }
+    const int nodes_each = (nl + kPlanBlock - 1) / kPlanBlock, x0 = min(nl, (int)threadIdx.x * nodes_each);
+    const int x1 = min(nl, x0 + nodes_each);
+    auto part_items = [&](int x) {
+        const int2 sg = tb.seg[off + x];
+        return max(1, (sg.y - sg.x + kPartChunk - 1) / kPartChunk);
+    };
+    int n_part;
+    items = 0;
+    for (int x = x0; x < x1; ++x) items += part_items(x);
+    at = block_excl_scan<NW>(items, lds, &n_part);
+    int *__restrict__ pbegin = tb.pbegin(level);
+    for (int x = x0; x < x1; ++x) {
+        pbegin[x] = at;
+        at += part_items(x);
+    }
+    if (threadIdx.x == 0) {
+        tb.hpair_begin[n_pairs] = n_items;
+        pbegin[nl] = n_part;
+        tb.ctl[level] = LevelCtl{chunk, n_items, n_part, total};
+    }
+}
+
 // Few rows (kSmallRows): a level in one launch instead of count, scatter, histogram and merge, which take 5 to 7 us each with
 // nothing to do. A workgroup owns a node and a feature block: it picks the node's split, decides for every row, lays the
 // children's lists down and adds up the histogram of the child with fewer rows, whose list it has in LDS, right at the
@@ -538,6 +605,7 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
 #undef TGBM_SPLIT_COUNT
     if (level == 0) k_split_scatter<true><<<items, kBlock, 0, s>>>(tb, level);
     else k_split_scatter<false><<<items, kBlock, 0, s>>>(tb, level);
+    if (tb.planned(level + 1)) k_plan_level<<<dim3(1, 1, n_class), kPlanBlock, 0, s>>>(tb, level + 1, tb.n_hpairs(level + 1));
 }
 
 static size_t small_lds(const TreeBuffers &tb) {

@@ -125,19 +125,58 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
-// Histogram work items of a level, planned by whoever needs them from the level's pairs (hpair_plan) instead of by a
-// launch of its own: every wavefront of the asking workgroup does the same few steps, so nothing waits at a barrier.
-// Every built node adds up to one partly filled item: the items are sized so that their number stays within
-// target_hitems (= the workgroups the chip holds at once; one more would run as a second round).
+// Rows per histogram work item of a level that builds n_built nodes of `total` rows. Every built node adds up to one
+// partly filled item: the items are sized so that their number stays within target_hitems (= the workgroups the chip
+// holds at once; one more would run as a second round).
+__device__ __forceinline__ int hist_chunk(const TreeBuffers &tb, int total, int n_built) {
+    const int room = max(tb.target_hitems / 4, tb.target_hitems - n_built);
+    const int chunk = (total + room - 1) / room;
+    return max(kHistMinChunk, (chunk + 255) / 256 * 256);
+}
+
+// The owner of `item` among n >= 1 owners whose items begin at begin[0] = 0, ..., begin[n] (item < begin[n]; owners may be
+// empty), found by a wavefront in steps of 64. The same in every lane.
+__device__ __forceinline__ int find_owner_wave(const int *__restrict__ begin, int n, int item) {
+    const int lane = lane_id();
+    int lo = 0;
+    while (n > 1) {
+        const int step = (n + 63) >> 6;
+        const bool upto = lane * step < n && begin[lo + lane * step] <= item;
+        const int at = (__popcll(__ballot(upto)) - 1) * step;
+        lo += at;
+        n = min(step, n - at);
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// Histogram work items of a level, planned from its pairs (hpair_plan) by whoever needs them: every wavefront of the asking
+// workgroup does the same few steps, so nothing waits at a barrier and no launch is needed. The steps grow with the
+// pairs, for each of the items that grow with them too; levels of more than kUnplannedPairs pairs are planned by one
+// launch (k_plan_level) and looked up here.
 struct HistPlan {
     int pair = -1;  // the pair that `item` belongs to, -1: there is no such item
     int built = 0, chunk = 0, first_item = 0;
     int item0 = 0;  // first item of the pairs that the launch serves (TreeBuffers::hpair_lo)
     int2 seg = make_int2(0, 0);
 };
-// publish (wave-uniform): also store the level's plan - hpair_begin and ctl[level] -, for k_hist_merge and the profile
+// publish (wave-uniform): also store the plan of a level that nobody has planned - hpair_begin and ctl[level] -, for
+// k_hist_merge and the profile
 __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_pairs, int item, bool publish, int level) {
     const int lane = lane_id();
+    if (tb.planned(level)) {
+        HistPlan out;
+        const LevelCtl ctl = tb.ctl[level];
+        if (item >= ctl.n_hitems) return out;
+        const int pair = find_owner_wave(tb.hpair_begin, n_pairs, item);
+        const int4 q = tb.hpair_plan[pair];
+        out.pair = pair;
+        out.built = q.x;
+        out.seg = make_int2(q.y, q.z);
+        out.chunk = ctl.hchunk;
+        out.first_item = tb.hpair_begin[pair];
+        out.item0 = tb.hpair_begin[tb.hpair_lo(level)];
+        return out;
+    }
     int4 mine = make_int4(-1, 0, 0, 0);
     if (lane < n_pairs) mine = tb.hpair_plan[lane];
     int total = 0, n_built = 0;
@@ -148,9 +187,7 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
     }
     total = wave_sum_i(total);
     n_built = wave_sum_i(n_built);
-    const int room = max(tb.target_hitems / 4, tb.target_hitems - n_built);
-    int chunk = (total + room - 1) / room;
-    chunk = max(kHistMinChunk, (chunk + 255) / 256 * 256);
+    const int chunk = hist_chunk(tb, total, n_built);
     HistPlan out;
     out.chunk = chunk;
     int carry = 0;
