@@ -230,24 +230,27 @@ __device__ float pow2_scale(float vmax, int rows, float limit) {
 
 // ------------------------------------------------------------------------------- tree init
 // Node array initialisation of the reference's Tree::init2 (src/thundergbm/tree.cu:8-39), root sum
-// from the block partials, root segment and the histogram plan of level 0. One workgroup.
-// What the previous tree has left to do rides along: its finished nodes go into the model before they are reset, and a
-// second workgroup adds up the round's metric (two launches of 4 to 5 us per tree otherwise).
+// from the block partials, root segment and the histogram plan of level 0.
+// What the previous tree has left to do rides along: its finished nodes go into the model before they are reset, and the
+// last workgroup adds up the round's metric (two launches of 4 to 5 us per tree otherwise).
+// The first workgroup does all but the metric; trees of more than kInitNodes nodes are shared out over `parts` of them (with
+// one, the nodes of depth 14 took 85 us).
+constexpr int kInitNodes = 1024;
 __device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out);
-__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda, TreeLeftovers left) {
-    if (blockIdx.x == 1) {
+__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda, TreeLeftovers left, int parts) {
+    if ((int)blockIdx.x == parts) {
         if (blockIdx.z == 0) metric_final(left.metric_kind, tb_all.n, left.metric_blocks, left.metric_partial, left.metric_out);
         return;
     }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    if (left.small) {  // every row starts in the root; k_small_level counts the levels' rows
+    if (left.small && blockIdx.x == 0) {  // every row starts in the root; k_small_level counts the levels' rows
         for (int i = threadIdx.x; i < tb.n; i += kBlock) tb.nid[i] = 0;
         for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{0, 0, 0, 0};
     }
     const GradStats *__restrict__ block_sums = tb.root_partial;
     const int nn = tb.n_nodes;
-    for (int i = threadIdx.x; i < nn; i += kBlock) {
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < nn; i += parts * kBlock) {
         TreeNode nd;
         nd.final_id = i;
         nd.parent_index = i == 0 ? -1 : (i - 1) / 2;
@@ -284,6 +287,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
         tb.seg[i] = make_int2(0, 0);
         if (tb.node_rows != nullptr) tb.node_rows[i] = i == 0 ? tb.n : 0;
     }
+    if (blockIdx.x != 0) return;
     float g = 0, h = 0, gm = 0, hm = 0, hf = 0;
     for (int i = threadIdx.x; i < tb.n_grad_blocks; i += kBlock) {
         g += block_sums[i].g;
@@ -2459,7 +2463,8 @@ void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_cla
                       int n_class, const TreeLeftovers &left) {
     if (!stats_ready)  // n_grad_blocks == row_blocks(n)
         k_sum_gh<<<dim3(tb.n_grad_blocks, 1, n_class), kBlock, 0, s>>>(tb.n, gh_class, tb.root_partial);
-    k_tree_init<<<dim3(left.metric_out != nullptr ? 2 : 1, 1, n_class), kBlock, 0, s>>>(tb, lambda, left);
+    const int parts = (tb.n_nodes + kInitNodes - 1) / kInitNodes;
+    k_tree_init<<<dim3(parts + (left.metric_out != nullptr ? 1 : 0), 1, n_class), kBlock, 0, s>>>(tb, lambda, left, parts);
     if (tb.nid16 != nullptr) {
         // sparse level pass: every row starts in the root (the n_class maps lie back to back)
         const size_t words = ((size_t)tb.n + 2) / 2 * (size_t)n_class;
