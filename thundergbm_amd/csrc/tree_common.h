@@ -163,19 +163,28 @@ struct HistPlan {
 // k_hist_merge and the profile
 __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_pairs, int item, bool publish, int level) {
     const int lane = lane_id();
+    HistPlan out;
+    // (the same in every lane: scalar registers from here on)
+    auto scalars = [&] {
+        out.pair = __builtin_amdgcn_readfirstlane(out.pair);
+        out.built = __builtin_amdgcn_readfirstlane(out.built);
+        out.chunk = __builtin_amdgcn_readfirstlane(out.chunk);
+        out.first_item = __builtin_amdgcn_readfirstlane(out.first_item);
+        out.item0 = __builtin_amdgcn_readfirstlane(out.item0);
+        out.seg = make_int2(__builtin_amdgcn_readfirstlane(out.seg.x), __builtin_amdgcn_readfirstlane(out.seg.y));
+        return out;
+    };
     if (tb.planned(level)) {
-        HistPlan out;
         const LevelCtl ctl = tb.ctl[level];
-        if (item >= ctl.n_hitems) return out;
-        const int pair = find_owner_wave(tb.hpair_begin, n_pairs, item);
-        const int4 q = tb.hpair_plan[pair];
-        out.pair = pair;
+        if (item >= ctl.n_hitems) return scalars();
+        out.pair = find_owner_wave(tb.hpair_begin, n_pairs, item);
+        const int4 q = tb.hpair_plan[out.pair];
         out.built = q.x;
         out.seg = make_int2(q.y, q.z);
         out.chunk = ctl.hchunk;
-        out.first_item = tb.hpair_begin[pair];
+        out.first_item = tb.hpair_begin[out.pair];
         out.item0 = tb.hpair_begin[tb.hpair_lo(level)];
-        return out;
+        return scalars();
     }
     int4 mine = make_int4(-1, 0, 0, 0);
     if (lane < n_pairs) mine = tb.hpair_plan[lane];
@@ -188,7 +197,6 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
     total = wave_sum_i(total);
     n_built = wave_sum_i(n_built);
     const int chunk = hist_chunk(tb, total, n_built);
-    HistPlan out;
     out.chunk = chunk;
     int carry = 0;
     for (int p0 = 0; p0 < n_pairs; p0 += 64) {
@@ -218,14 +226,7 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
         tb.hpair_begin[n_pairs] = carry;
         tb.ctl[level] = LevelCtl{chunk, carry, 0, total};
     }
-    // (the same in every lane: scalar registers from here on)
-    out.pair = __builtin_amdgcn_readfirstlane(out.pair);
-    out.built = __builtin_amdgcn_readfirstlane(out.built);
-    out.chunk = __builtin_amdgcn_readfirstlane(out.chunk);
-    out.first_item = __builtin_amdgcn_readfirstlane(out.first_item);
-    out.item0 = __builtin_amdgcn_readfirstlane(out.item0);
-    out.seg = make_int2(__builtin_amdgcn_readfirstlane(out.seg.x), __builtin_amdgcn_readfirstlane(out.seg.y));
-    return out;
+    return scalars();
 }
 
 }  // namespace
