@@ -53,3 +53,28 @@ def test_boost_equals_the_stages(n, F, depth, bins, objective):
     assert models[0] == models[1]
     assert np.array_equal(maps[0], maps[1])
     assert np.array_equal(preds[0], preds[1])
+
+
+@pytest.mark.parametrize("n", [256 * 2048 + 1, 1_300_001, (1 << 24) - 1, 1 << 24])
+def test_rows_of_nodes_of_many_items(n):
+    """Nodes of more work items than a workgroup has threads, below and above the rows from which on their counts are added up
+    by groups: every node holds the rows that its path leads there (squared loss: the hessians count them, exactly up to
+    2^24)."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    X = rng.integers(1, 1000, (n, 2)).astype(np.float32)
+    y = (np.floor(X[:, 0] / 100) + (X[:, 1] > 700) * (X[:, 0] > 300) + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    s = T.Session(X.reshape(-1), np.arange(0, 2 * n + 1, 2, dtype=np.int32), np.tile(np.arange(2, dtype=np.int32), n), y,
+                  depth=5, n_trees=2, learning_rate=0.5, gamma=0.0)
+    s.boost(2)
+    for tree in s.model().reshape(2, -1):
+        node = np.zeros(n, np.int64)
+        for _ in range(6):
+            rows = np.bincount(node, minlength=len(tree))
+            at = np.unique(node)
+            assert np.array_equal(tree["sum_h"][at], rows[at])
+            inner = ~tree["is_leaf"][node].astype(bool)
+            left = X[np.arange(n), np.maximum(tree["split_fid"][node], 0)] < tree["split_value"][node]
+            node = np.where(inner, np.where(left, tree["lch"][node], tree["rch"][node]), node)
+    assert np.array_equal(s.nid(), node)
+    s.close()

@@ -73,6 +73,10 @@ constexpr int kMissingBin16 = 65535;  // the same for 16-bit bins
 constexpr int kDense16BlockBins = 8192;
 constexpr int kDense16MaxBlockBins = 20480;
 constexpr int kPartChunk = 2048;   // rows per partition work item (256 threads x 8 rounds)
+// From so many rows on the partition's launches are shared out as far as they go: what every work item would do for itself
+// grows with the rows a second time. Items whose counts then also come as one sum:
+constexpr int kPartGroupRows = 1 << 24;
+constexpr int kPartGroup = 64;
 // Dense layout: up to so many pairs (nodes, where single nodes are built) in a level every workgroup plans for itself.
 constexpr int kUnplannedPairs = 256;
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
@@ -297,6 +301,8 @@ struct TreeBuffers {
     int *hpair_built = nullptr;    // [max_pairs] heap id of the node built from rows, -1 = inactive pair
     int *pitem_begin = nullptr;    // [2][max_level_nodes + 1] first partition item of every node of a level, by level parity
     int *pitem_nleft = nullptr;    // [max_pitems]
+    int *pgroup_nleft = nullptr;   // [n_pgroups] dense layout, many rows: sums of kPartGroup items each (else nullptr)
+    int n_pgroups = 0;
     int *pitem_loff = nullptr;     // [max_pitems]
     int *node_nleft = nullptr;     // [max_level_nodes]
     LevelCtl *ctl = nullptr;       // [depth + 1]
@@ -388,6 +394,7 @@ struct TreeBuffers {
         t.hpair_built += K * max_level_nodes;
         t.pitem_begin += K * 2 * (max_level_nodes + 1);
         t.pitem_nleft += K * ((size_t)max_pitems + 1);
+        if (pgroup_nleft != nullptr) t.pgroup_nleft += K * n_pgroups;
         t.pitem_loff += K * ((size_t)max_pitems + 1);
         t.node_nleft += K * max_level_nodes;
         t.ctl += K * (depth + 2);

@@ -593,6 +593,10 @@ void Trainer::alloc_tree_buffers() {
     tb.pitem_begin = dalloc<int>(S * 2 * ((size_t)max_level_nodes + 1));
     tb.pitem_nleft = dalloc<int>(S * ((size_t)tb.max_pitems + 1));
     tb.pitem_loff = dalloc<int>(S * ((size_t)tb.max_pitems + 1));
+    if (!sparse_ && n_ >= kPartGroupRows) {
+        tb.n_pgroups = tb.max_pitems / kPartGroup + 1;
+        tb.pgroup_nleft = dalloc<int>(S * (size_t)tb.n_pgroups);
+    }
     tb.node_nleft = dalloc<int>(S * max_level_nodes);
     tb.ctl = dalloc<LevelCtl>(S * ((size_t)depth + 2));
     tb.sp = dalloc<SplitPoint>(S * max_level_nodes);
@@ -1027,9 +1031,11 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
 
 // Inside boost() nobody looks at a level's split records between its split search and its partition, so the dense
 // layout's partition picks the nodes' best candidates itself (a launch less per level). The last level is not
-// partitioned, and a level served in batches needs its updates batch by batch.
+// partitioned, a level served in batches needs its updates batch by batch, and on many rows the launch costs less than
+// the picking of every work item (100 M x 6, depth 8: 9.69 against 9.83 ms a tree; 30 M x 8: 3.28 against 3.30).
 bool Trainer::update_with_partition(int level) const {
-    return in_boost_ && !sparse_ && level < param_.depth - 1 && (hist_cap_level_ < 0 || level < hist_cap_level_);
+    return in_boost_ && !sparse_ && n_ < kPartGroupRows && level < param_.depth - 1 &&
+           (hist_cap_level_ < 0 || level < hist_cap_level_);
 }
 
 void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class) {
