@@ -33,3 +33,9 @@ def test_sums_lie_in_the_range_of_their_codes(run_native):
     """The filter of the rare features may exclude a run only by a true bound on its candidates' sums: an end that is
     scaled up moves inwards where the whole range is on one side of zero."""
     run_native("rare_range.cpp")
+
+
+def test_kept_device_blocks(run_native):
+    """Reuse, the limit, the order in which blocks go, an allocation that fails, and who pays: requests that follow a
+    training call free nothing that it has left, and no thread waits for another one's driver call."""
+    run_native("device_pool.cpp")
