@@ -211,7 +211,7 @@ int tgbm_predict_raw_noalloc(int row_size, const float *val, const int *row_ptr,
                              tgbm_model *model, int n_trees, int trees_per_iter, float learning_rate,
                              float base_score, float *out);
 
-/* Device memory that calls have given back is kept for later ones, at most an eighth of each GPU's memory; this returns
+/* Device memory that calls have given back is kept for later ones, at most a 32nd of each GPU's memory; this returns
  * all of it to the driver. It has no counterpart in the reference. */
 void tgbm_release_memory(void);
 

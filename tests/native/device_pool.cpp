@@ -69,7 +69,7 @@ void release_transfer_memory() {}
 
 int main() {
     using namespace tgbm;
-    const size_t limit = kTotal / kKeepPart;
+    const size_t limit = kTotal / 32;  // (of 16 GB)
     // the second call of a size takes the first one's block
     void *a = device_alloc(10 * kMB);
     device_free(a);

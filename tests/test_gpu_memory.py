@@ -46,3 +46,32 @@ def test_calls_share_and_return_kept_memory():
     for i in (0, 1):
         assert all(m == alone[i] for m in got[i])
         assert train(i) == alone[i]
+
+
+def test_an_idle_process_holds_little_and_can_give_it_back():
+    import ctypes as C
+    import thundergbm_amd as T
+    D.warm_up(T)
+    hip = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+    def memory():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value, total.value
+
+    X, y = D.config1(400_000, 20, seed=1)
+    val, rp, col = D.dense_to_csr(X)
+
+    def train():
+        s = T.Session(val, rp, col, y, depth=6, n_trees=2)
+        s.boost(2)
+        s.close()
+
+    train()
+    T.release_memory()
+    free, total = memory()
+    train()
+    kept = free - memory()[0]
+    assert 0 < kept <= total // 32
+    T.release_memory()
+    assert free - memory()[0] < kept // 4

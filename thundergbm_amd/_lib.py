@@ -73,3 +73,9 @@ def load():
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def release_memory():
+    """Returns the device and pinned host memory that the library keeps for later calls (tgbm_release_memory). Any thread, any
+    time: what calls and sessions are using stays theirs."""
+    load().tgbm_release_memory()
