@@ -661,8 +661,8 @@ def test_sparse_root_histogram_from_either_copy(T, objective, kind, head):
 
 @pytest.mark.parametrize("mcw,gamma", [(1.0, 0.0), (40.0, 0.0), (1.0, 30.0)])
 def test_sparse_sorted_pass_equals_table_pass_on_deep_uneven_trees(T, mcw, gamma):
-    """Sparse level pass: features of a few thousand values are searched through their values kept sorted by
-    (feature, node, bin) from level to level, the frequent ones through (bin, node) tables; TGBM_SPARSE_SORTED=0
+    """Sparse level pass: features of few values are searched through those of their values that a bound does not
+    exclude, the frequent ones through (bin, node) tables; TGBM_SPARSE_SORTED=0
     sends every feature through the tables. Same integers either way: identical models, predictions and row -> node
     maps, on trees whose nodes stop at different levels (min_child_weight) and with frequent and rare features
     mixed (a few columns in nearly every row, many in a handful of rows)."""
@@ -1169,7 +1169,7 @@ def test_bundle_of_a_complete_feature_and_an_empty_one(T):
 
 def test_sparse_level_pass_at_its_deepest_level(T):
     """Depth 11 (1024 nodes on the last level: the sparse level pass's limit, 12-bit node field of the sorted keys,
-    20 KB of per-node LDS state): sorted pass against tables, byte for byte."""
+    20 KB of per-node LDS state): filtered search against tables, byte for byte."""
     os.environ["TGBM_LAYOUT"] = "sparse"
     n, F = 60000, 400
     val, rp, col = _ragged(n, F, 51, 10)

@@ -1006,7 +1006,7 @@ def test_full_size_properties_config4_sparse(T):
 def test_full_size_oracle_config4_sparse(T):
     """2 M x 100k CSR, depth 8, 63 bins against the oracle at the full shape (6.3 M cut points: the oracle keeps the
     reference's histogram of all of them per node): the first tree of the level pass - 981 frequent features through
-    tables and byte columns, 99 k rare ones through the sorted pass."""
+    tables and byte columns, 99 k rare ones through the filtered search."""
     val, rp, col, y = _full_data("c4")
     kw = dict(objective="binary:logistic", depth=8, max_num_bin=63, learning_rate=0.3, n_trees=1)
     s = T.Session(val, rp, col, y, **kw)

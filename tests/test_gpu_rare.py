@@ -1,5 +1,5 @@
-"""Rare features of the sparse layout: the filtered search (k_sparse_rare) against the complete (bin, node) tables
-(TGBM_SPARSE_SORTED=0), byte for byte, at the edges of its tiles."""
+"""Rare features of the sparse layout: the filtered search (k_sparse_rare_filter, k_sparse_rare_search) against the complete
+(bin, node) tables (TGBM_SPARSE_SORTED=0: every feature through them), byte for byte, at the edges of its tiles."""
 import ctypes
 import os
 
@@ -47,6 +47,11 @@ FREQUENT = {
     "tiles_around_512": ([900] * 128 + [700, 512, 513, 1, 511] * 6, 1000),
     "one_feature_more": ([400] * 129 + [400, 300], 600),
     "few_values": ([3] * 20, 50),
+    "only_rare": ([250] * 70, 2000),                               # the tables publish next to nothing
+}
+RARE_VALUES = {  # (feature 0 owns bin 0 and goes to a table whatever it holds)
+    "full_tiles": 4096 + 4095 + 1 + 4096 + 2048 + 2048 + 1, "few_rows": (256 + 255 + 1 + 256 + 256 + 128 + 128 + 2) * 8,
+    "tiles_around_512": (700 + 512 + 513 + 1 + 511) * 6, "one_feature_more": 129 * 400 + 300, "few_values": 19 * 3, "only_rare": 69 * 250,
 }
 OPTIONS = pytest.mark.parametrize("objective,kw", [
     ("reg:linear", {}), ("binary:logistic", {"min_child_weight": 5.0}), ("multi:softmax", {"num_class": 3}),
@@ -57,7 +62,7 @@ OPTIONS = pytest.mark.parametrize("objective,kw", [
 @OPTIONS
 def test_features_at_the_edge_of_rare_equal_tables(T, shape, objective, kw):
     val, rp, col, z = _by_feature(*FREQUENT[shape], 5)
-    compare(T, val, rp, col, (z - np.median(z)) / z.std(), objective, kw)
+    compare(T, val, rp, col, (z - np.median(z)) / z.std(), objective, kw, RARE_VALUES[shape])
 
 
 @pytest.mark.parametrize("shape", sorted(SHAPES))
@@ -68,7 +73,7 @@ def test_rare_features_equal_tables(T, shape, objective, kw):
     compare(T, val, rp, col, z, objective, kw)
 
 
-def compare(T, val, rp, col, z, objective, kw):
+def compare(T, val, rp, col, z, objective, kw, rare_values=None):
     kw = dict(kw)
     sampled = kw.pop("sampled", False)
     y = (z if objective == "reg:linear" else np.digitize(z, [-0.5, 0.5][: 2 if "multi" in objective else 1])).astype(np.float32)
@@ -80,6 +85,8 @@ def compare(T, val, rp, col, z, objective, kw):
             ctypes.CDLL(None).srand(7)
             s = T.Session(val, rp, col, y, objective=objective, depth=7, n_trees=3, max_num_bin=63, learning_rate=0.5, **kw)
             assert s.info("sparse_pass") == 1
+            assert rare == "1" or s.info("sparse_rare_values") == 0
+            assert rare == "0" or rare_values is None or s.info("sparse_rare_values") == rare_values
             if sampled:
                 s.set_option("bagging", 1)
                 s.set_option("column_sampling_rate", 0.5)

@@ -279,8 +279,6 @@ struct TreeBuffers {
     longlong2 *partial = nullptr;  // [max_hitems * n_bins] per-item fixed-point sums (g, h)
     QuantCtl *quant = nullptr;     // scales of the current tree
     int2 *hitem_shift = nullptr;   // [max_hitems] powers of two by which a dense work item (its node) coarsened (g, h)
-    // Root sums as exact integers at the tree's scales (what a row order cannot change), from the gradients when no
-    // feature is stored in every row: [2 i], [2 i + 1] the sums of workgroup i of k_root_sum_rows (up to 256)
     // sparse level pass only (else nullptr): node every row has reached (heap id) and rows per node
     unsigned short *nid16 = nullptr;  // [n + 2]
     int *node_rows = nullptr;         // [n_nodes]
@@ -291,6 +289,8 @@ struct TreeBuffers {
     // the task that searches a feature (k_best_update reads the winner's record from that slot)
     unsigned long long *best_key = nullptr;  // [max_level_nodes]
     const int *feat_slot = nullptr;          // [F]
+    // Root sums as exact integers at the tree's scales (what a row order cannot change), from the gradients when no
+    // feature is stored in every row: [2 i], [2 i + 1] the sums of workgroup i of k_root_sum_rows (up to 256)
     long long *root_total = nullptr;
     int complete_feature = -1;     // dense layout: a feature stored in every row (its bins add up to the root), or -1
     int max_hitems = 0, target_hitems = 0, max_pitems = 0;

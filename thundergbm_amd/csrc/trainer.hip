@@ -1424,6 +1424,7 @@ int Trainer::info(const std::string &key) const {
     if (key == "n_sets") return n_sets_;
     if (key == "sparse") return sparse_ ? 1 : 0;
     if (key == "sparse_pass") return sparse_pass_ ? 1 : 0;
+    if (key == "sparse_rare_values") return (int)sp_.n_rare;
     if (key == "wide_bins") return wide_bins_ ? 1 : 0;
     if (key == "wide_eval") return wide_eval_ ? 1 : 0;
     if (key == "row_lists") return sparse_pass_ ? 0 : 1;  // the sparse level pass keeps a row -> node map only
