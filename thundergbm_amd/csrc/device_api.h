@@ -301,9 +301,9 @@ struct TreeBuffers {
     int *hpair_built = nullptr;    // [max_pairs] heap id of the node built from rows, -1 = inactive pair
     int *pitem_begin = nullptr;    // [2][max_level_nodes + 1] first partition item of every node of a level, by level parity
     int *pitem_nleft = nullptr;    // [max_pitems]
-    int *pgroup_nleft = nullptr;   // [n_pgroups] dense layout, many rows: sums of kPartGroup items each (else nullptr)
-    int n_pgroups = 0;
-    int *pitem_loff = nullptr;     // [max_pitems]
+    // [max_pitems] per-node path of the sparse layout: pitem_nleft added up; dense layout of many rows: its sums over
+    // kPartGroup items each (not a pointer of its own: every launch takes these as arguments)
+    int *pitem_loff = nullptr;
     int *node_nleft = nullptr;     // [max_level_nodes]
     LevelCtl *ctl = nullptr;       // [depth + 1]
     SplitPoint *sp = nullptr;      // [max_level_nodes]
@@ -394,7 +394,6 @@ struct TreeBuffers {
         t.hpair_built += K * max_level_nodes;
         t.pitem_begin += K * 2 * (max_level_nodes + 1);
         t.pitem_nleft += K * ((size_t)max_pitems + 1);
-        if (pgroup_nleft != nullptr) t.pgroup_nleft += K * n_pgroups;
         t.pitem_loff += K * ((size_t)max_pitems + 1);
         t.node_nleft += K * max_level_nodes;
         t.ctl += K * (depth + 2);

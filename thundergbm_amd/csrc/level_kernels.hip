@@ -244,9 +244,9 @@ __global__ __launch_bounds__(kBlock) void k_split_groups(TreeBuffers tb_all, int
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int g = blockIdx.x * kWaves + wave_id(), item = g * kPartGroup + lane_id();
     static_assert(kPartGroup == 64, "a lane per item");
-    if (g >= tb.n_pgroups) return;
+    if (g * kPartGroup >= items) return;
     const int sum = wave_sum_i(item < items ? tb.pitem_nleft[item] : 0);
-    if (lane_id() == 0) tb.pgroup_nleft[g] = sum;
+    if (lane_id() == 0) tb.pitem_loff[g] = sum;
 }
 
 // Stable two-way compaction of a work item's rows into the children's segments with wavefront ballots and popcounts;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, in
             total = part < 2 ? c : 0;
             before = from + t < item ? c : 0;
         }
-        const int *__restrict__ groups = tb.pgroup_nleft;
+        const int *__restrict__ groups = tb.pitem_loff;
         for (int g = g0 + threadIdx.x; g < g1; g += kBlock) {
             const int c = groups[g];
             total += c;
@@ -636,10 +636,10 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
         else { if (update) TGBM_SPLIT_COUNT(false, uint8_t, true); else TGBM_SPLIT_COUNT(false, uint8_t, false); }
     }
 #undef TGBM_SPLIT_COUNT
-    if (tb.pgroup_nleft != nullptr)
-        k_split_groups<<<dim3((tb.n_pgroups + kWaves - 1) / kWaves, 1, n_class), kBlock, 0, s>>>(tb, most);
+    const bool groups = tb.n >= kPartGroupRows;
+    if (groups) k_split_groups<<<dim3((most + kPartGroup * kWaves - 1) / (kPartGroup * kWaves), 1, n_class), kBlock, 0, s>>>(tb, most);
 #define TGBM_SPLIT_SCATTER(D, G) k_split_scatter<D, G><<<items, kBlock, 0, s>>>(tb, level)
-    if (tb.pgroup_nleft != nullptr) { if (level == 0) TGBM_SPLIT_SCATTER(true, true); else TGBM_SPLIT_SCATTER(false, true); }
+    if (groups) { if (level == 0) TGBM_SPLIT_SCATTER(true, true); else TGBM_SPLIT_SCATTER(false, true); }
     else { if (level == 0) TGBM_SPLIT_SCATTER(true, false); else TGBM_SPLIT_SCATTER(false, false); }
 #undef TGBM_SPLIT_SCATTER
     if (tb.planned(level + 1)) k_plan_level<<<dim3(1, 1, n_class), kPlanBlock, 0, s>>>(tb, level + 1, tb.n_hpairs(level + 1));

@@ -593,10 +593,6 @@ void Trainer::alloc_tree_buffers() {
     tb.pitem_begin = dalloc<int>(S * 2 * ((size_t)max_level_nodes + 1));
     tb.pitem_nleft = dalloc<int>(S * ((size_t)tb.max_pitems + 1));
     tb.pitem_loff = dalloc<int>(S * ((size_t)tb.max_pitems + 1));
-    if (!sparse_ && n_ >= kPartGroupRows) {
-        tb.n_pgroups = tb.max_pitems / kPartGroup + 1;
-        tb.pgroup_nleft = dalloc<int>(S * (size_t)tb.n_pgroups);
-    }
     tb.node_nleft = dalloc<int>(S * max_level_nodes);
     tb.ctl = dalloc<LevelCtl>(S * ((size_t)depth + 2));
     tb.sp = dalloc<SplitPoint>(S * max_level_nodes);
