@@ -24,18 +24,20 @@ struct NodeItem {
     int2 seg;
 };
 
-// lds: kWaves ints, s: 5 ints; every thread of the workgroup calls
+// lds: kWaves ints, s: 5 ints; every thread of the workgroup calls. PLANNED: TreeBuffers::planned(level), by the launcher (as a
+// branch in here it cost the count launches of the other levels 0.4 us each)
+template <bool PLANNED>
 __device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level, int item, int *lds, int *s) {
     const int nl = 1 << level, off = nl - 1;
     NodeItem out;
-    if (level == 0) {
+    if (!PLANNED && level == 0) {
         out.count = max(1, (tb.n + kPartChunk - 1) / kPartChunk);
         out.x_in = item < out.count ? 0 : -1;
         out.first = 0;
         out.seg = make_int2(0, tb.n);
         return out;
     }
-    if (tb.planned(level)) {
+    if (PLANNED) {
         const int *__restrict__ begin = tb.pbegin(level);
         out.x_in = -1;
         if (item >= begin[nl]) return out;
@@ -151,7 +153,7 @@ __device__ __forceinline__ void apply_candidate(const TreeBuffers &tb, int x, in
 // UPDATE: the nodes' candidates are fresh from the split search; else the tree has been updated already.
 // A row goes right if its bin is not below the split bin, or if it has no value of the feature and the default says so
 // (hist_tree_builder_single.cu:986-1011).
-template <bool DIRECT, typename BinT, bool UPDATE>
+template <bool DIRECT, typename BinT, bool UPDATE, bool PLANNED>
 __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, DenseBins bins, int level, float rt_eps,
                                                        float lambda) {
     __shared__ int lds[kWaves];
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int *__restrict__ ridx = tb.list(level);
     const int item = blockIdx.x;
-    const NodeItem it = locate_item(tb, level, item, lds, s_item);
+    const NodeItem it = locate_item<PLANNED>(tb, level, item, lds, s_item);
     if (it.x_in < 0) return;
     const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
     const int2 sg = it.seg;
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void k_split_groups(TreeBuffers tb_all, int
 // pair of the next level: the child with fewer rows is built from them (ties: the left one, as
 // hist_tree_builder_single.cu:466-467), the other one comes from subtraction. (Moving the gradient pairs along with the
 // row ids was measured: it makes the histogram's gradient reads sequential but costs more here than it saves there.)
-template <bool DIRECT, bool GROUPS>
+template <bool DIRECT, bool GROUPS, bool PLANNED>
 __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, int level) {
     __shared__ int lds[kWaves];
     __shared__ int s_item[5];
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, in
     const int *__restrict__ ridx_cur = tb.list(level);
     int *__restrict__ ridx_next = tb.list(level + 1);
     const int item = blockIdx.x;
-    const NodeItem it = locate_item(tb, level, item, lds, s_item);
+    const NodeItem it = locate_item<PLANNED>(tb, level, item, lds, s_item);
     if (it.x_in < 0) return;
     const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
     const int2 sg = it.seg;
@@ -627,20 +629,29 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
     if (level == tb.depth - 1) return;  // the last level's children never get row lists (see k_tree_end)
     const int most = level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
     const dim3 items(most, 1, n_class);
-#define TGBM_SPLIT_COUNT(D, T, U) k_split_count<D, T, U><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
+    const bool planned = tb.planned(level);
+#define TGBM_SPLIT_COUNT(D, T, U, P) k_split_count<D, T, U, P><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
+#define TGBM_SPLIT_COUNT_LEVEL(T, U)                           \
+    if (level == 0) TGBM_SPLIT_COUNT(true, T, U, false);       \
+    else if (planned) TGBM_SPLIT_COUNT(false, T, U, true);     \
+    else TGBM_SPLIT_COUNT(false, T, U, false)
     if (bins.bin_bytes == 2) {
-        if (level == 0) { if (update) TGBM_SPLIT_COUNT(true, uint16_t, true); else TGBM_SPLIT_COUNT(true, uint16_t, false); }
-        else { if (update) TGBM_SPLIT_COUNT(false, uint16_t, true); else TGBM_SPLIT_COUNT(false, uint16_t, false); }
+        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint16_t, true); }
+        else { TGBM_SPLIT_COUNT_LEVEL(uint16_t, false); }
     } else {
-        if (level == 0) { if (update) TGBM_SPLIT_COUNT(true, uint8_t, true); else TGBM_SPLIT_COUNT(true, uint8_t, false); }
-        else { if (update) TGBM_SPLIT_COUNT(false, uint8_t, true); else TGBM_SPLIT_COUNT(false, uint8_t, false); }
+        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint8_t, true); }
+        else { TGBM_SPLIT_COUNT_LEVEL(uint8_t, false); }
     }
+#undef TGBM_SPLIT_COUNT_LEVEL
 #undef TGBM_SPLIT_COUNT
     const bool groups = tb.n >= kPartGroupRows;
     if (groups) k_split_groups<<<dim3((most + kPartGroup * kWaves - 1) / (kPartGroup * kWaves), 1, n_class), kBlock, 0, s>>>(tb, most);
-#define TGBM_SPLIT_SCATTER(D, G) k_split_scatter<D, G><<<items, kBlock, 0, s>>>(tb, level)
-    if (groups) { if (level == 0) TGBM_SPLIT_SCATTER(true, true); else TGBM_SPLIT_SCATTER(false, true); }
-    else { if (level == 0) TGBM_SPLIT_SCATTER(true, false); else TGBM_SPLIT_SCATTER(false, false); }
+#define TGBM_SPLIT_SCATTER(G)                                                      \
+    if (level == 0) k_split_scatter<true, G, false><<<items, kBlock, 0, s>>>(tb, level);   \
+    else if (planned) k_split_scatter<false, G, true><<<items, kBlock, 0, s>>>(tb, level); \
+    else k_split_scatter<false, G, false><<<items, kBlock, 0, s>>>(tb, level)
+    if (groups) { TGBM_SPLIT_SCATTER(true); }
+    else { TGBM_SPLIT_SCATTER(false); }
 #undef TGBM_SPLIT_SCATTER
     if (tb.planned(level + 1)) k_plan_level<<<dim3(1, 1, n_class), kPlanBlock, 0, s>>>(tb, level + 1, tb.n_hpairs(level + 1));
 }
