@@ -24,10 +24,11 @@ struct NodeItem {
     int2 seg;
 };
 
-// lds: kWaves ints, s: 5 ints; every thread of the workgroup calls. PLANNED: TreeBuffers::planned(level), by the launcher (as a
-// branch in here it cost the count launches of the other levels 0.4 us each)
+// Every wavefront of the workgroup finds the item for itself, without a barrier; the result is the same in all of its lanes.
+// PLANNED: TreeBuffers::planned(level), by the launcher (as a branch in here it cost the count launches of the other
+// levels 0.4 us each)
 template <bool PLANNED>
-__device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level, int item, int *lds, int *s) {
+__device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level, int item) {
     const int nl = 1 << level, off = nl - 1;
     NodeItem out;
     if (!PLANNED && level == 0) {
@@ -37,103 +38,128 @@ __device__ __forceinline__ NodeItem locate_item(const TreeBuffers &tb, int level
         out.seg = make_int2(0, tb.n);
         return out;
     }
+    out.x_in = -1;
     if (PLANNED) {
         const int *__restrict__ begin = tb.pbegin(level);
-        out.x_in = -1;
-        if (item >= begin[nl]) return out;
+        if (item >= __builtin_amdgcn_readfirstlane(begin[nl])) return out;
         out.x_in = find_owner_wave(begin, nl, item);
-        out.first = begin[out.x_in];
-        out.count = begin[out.x_in + 1] - out.first;
-        out.seg = tb.seg[off + out.x_in];
+        out.first = __builtin_amdgcn_readfirstlane(begin[out.x_in]);
+        out.count = __builtin_amdgcn_readfirstlane(begin[out.x_in + 1]) - out.first;
+        const int2 sg = tb.seg[off + out.x_in];
+        out.seg = make_int2(__builtin_amdgcn_readfirstlane(sg.x), __builtin_amdgcn_readfirstlane(sg.y));
         return out;
     }
-    if (threadIdx.x == 0) s[0] = -1;
+    constexpr int A = 4;  // 64 nodes each, loaded together
+    const int2 *__restrict__ segs = tb.seg + off;
     int carry = 0;
-    for (int base = 0; base < nl && carry <= item; base += kBlock) {  // (carry is the same in every thread)
-        const int x_in = base + threadIdx.x;
-        int2 sg = make_int2(0, 0);
-        int cnt = 0;
-        if (x_in < nl) {
-            sg = tb.seg[off + x_in];
-            cnt = max(1, (sg.y - sg.x + kPartChunk - 1) / kPartChunk);
+    for (int base = 0; base < nl; base += A * 64) {
+        int2 sg[A];
+#pragma unroll
+        for (int a = 0; a < A; ++a) sg[a] = segs[min(base + a * 64 + lane_id(), nl - 1)];
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            if (base + a * 64 >= nl) break;
+            const int cnt = base + a * 64 + lane_id() < nl ? max(1, (sg[a].y - sg[a].x + kPartChunk - 1) / kPartChunk) : 0;
+            const int inc = wave_scan_i(cnt), ex = carry + inc - cnt;
+            const unsigned long long owner = __ballot(item >= ex && item < ex + cnt);
+            if (owner != 0ull) {
+                const int l = __ffsll((long long)owner) - 1;
+                out.x_in = base + a * 64 + l;
+                out.first = read_lane(ex, l);
+                out.count = read_lane(cnt, l);
+                out.seg = make_int2(read_lane(sg[a].x, l), read_lane(sg[a].y, l));
+                return out;
+            }
+            carry += read_lane(inc, 63);
         }
-        int tot;
-        const int ex = carry + block_excl_scan(cnt, lds, &tot);
-        if (item >= ex && item < ex + cnt) {
-            s[0] = x_in;
-            s[1] = ex;
-            s[2] = cnt;
-            s[3] = sg.x;
-            s[4] = sg.y;
-        }
-        carry += tot;
     }
-    __syncthreads();
-    out.x_in = s[0];
-    out.first = s[1];
-    out.count = s[2];
-    out.seg = make_int2(s[3], s[4]);
     return out;
 }
 
-// The node's best candidate into *s_cand (larger |score|, then the smaller bin index), false: it has none. s_abs, s_idx: NW
-// entries; every thread of the workgroup calls.
+// What the workgroups of a node need of its best candidate (larger |score|, then the smaller bin index).
+struct Picked {
+    bool found;  // false: the node has no candidate
+    SplitCand c;
+};
+// Up to so many packs - one for every lane - each wavefront looks at all of them: no barrier, no LDS (500 k x 28: the
+// candidates' part of a count launch 1.7 -> 0.95 us). Beyond, the workgroup shares them out.
+constexpr int kWavePacks = 64;
+struct PickShared {
+    SplitCand cand;
+    float abs[16];
+    int idx[16];
+};
+// NW: wavefronts of the workgroup, all of whose threads call
 template <int NW>
-__device__ __forceinline__ bool pick_candidate(const TreeBuffers &tb, int x_in, bool valid, float *s_abs, int *s_idx,
-                                               SplitCand *s_cand) {
-            float a_best = -1.f;
-            int i_best = 0x7fffffff;
-            SplitCand best;
-            best.score = 0.f;
-            best.index = 0x7fffffff;
-            best.miss = best.left = GHPair{0, 0};
-            best.feature = best.bin = 0;
-            if (valid)
-                for (int p = threadIdx.x; p < tb.n_packs; p += NW * 64) {
-                    const SplitCand c = tb.cand[(size_t)x_in * tb.n_packs + p];
-                    const float a = fabsf(c.score);
-                    // (index 0x7fffffff: a wavefront whose features have no bins)
-                    const bool better = c.index != 0x7fffffff && (a > a_best || (a == a_best && c.index < i_best));
-                    a_best = better ? a : a_best;
-                    i_best = better ? c.index : i_best;
-                    best.score = better ? c.score : best.score;
-                    best.miss.g = better ? c.miss.g : best.miss.g;
-                    best.miss.h = better ? c.miss.h : best.miss.h;
-                    best.left.g = better ? c.left.g : best.left.g;
-                    best.left.h = better ? c.left.h : best.left.h;
-                    best.feature = better ? c.feature : best.feature;
-                    best.bin = better ? c.bin : best.bin;
-                }
-            // larger |score|, then the smaller bin index; bin indices are distinct
-            float win = a_best;
-            int win_idx = i_best;
-    #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) {
-                const float oa = __shfl_xor(win, d);
-                const int oi = __shfl_xor(win_idx, d);
-                if (oa > win || (oa == win && oi < win_idx)) {
-                    win = oa;
-                    win_idx = oi;
-                }
+__device__ __forceinline__ Picked pick_candidate(const TreeBuffers &tb, int x_in, bool valid, PickShared &sh) {
+    const bool alone = tb.n_packs <= kWavePacks;
+    float a_best = -1.f;
+    int i_best = 0x7fffffff;
+    SplitCand best;
+    best.score = 0.f;
+    best.index = 0x7fffffff;
+    best.miss = best.left = GHPair{0, 0};
+    best.feature = best.bin = 0;
+    const SplitCand *__restrict__ cand = tb.cand + (size_t)x_in * tb.n_packs;
+    auto look = [&](const SplitCand &c, bool in) {
+        const float a = fabsf(c.score);
+        // (index 0x7fffffff: a wavefront whose features have no bins)
+        const bool better = in && c.index != 0x7fffffff && (a > a_best || (a == a_best && c.index < i_best));
+        a_best = better ? a : a_best;
+        i_best = better ? c.index : i_best;
+        best.score = better ? c.score : best.score;
+        best.miss.g = better ? c.miss.g : best.miss.g;
+        best.miss.h = better ? c.miss.h : best.miss.h;
+        best.left.g = better ? c.left.g : best.left.g;
+        best.left.h = better ? c.left.h : best.left.h;
+        best.feature = better ? c.feature : best.feature;
+        best.bin = better ? c.bin : best.bin;
+    };
+    if (alone) {
+        look(cand[min(lane_id(), tb.n_packs - 1)], valid && lane_id() < tb.n_packs);
+    } else {
+        constexpr int U = 3;  // candidates per thread whose loads are issued together
+        for (int p0 = threadIdx.x; p0 - (int)threadIdx.x < tb.n_packs; p0 += U * NW * 64) {
+            SplitCand c[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) c[u] = cand[min(p0 + u * NW * 64, tb.n_packs - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u) look(c[u], valid && p0 + u * NW * 64 < tb.n_packs);
+        }
+    }
+    best.index = i_best;
+    float win;
+    int win_idx;
+    const int owner = wave_best(a_best, i_best, &win, &win_idx);
+    if (!alone) {
+        if (lane_id() == 0) {
+            sh.abs[wave_id()] = win;
+            sh.idx[wave_id()] = win_idx;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NW; ++i)
+            if (sh.abs[i] > win || (sh.abs[i] == win && sh.idx[i] < win_idx)) {
+                win = sh.abs[i];
+                win_idx = sh.idx[i];
             }
-            if (lane_id() == 0) {
-                s_abs[wave_id()] = win;
-                s_idx[wave_id()] = win_idx;
-            }
-            __syncthreads();
-    #pragma unroll
-            for (int i = 0; i < NW; ++i)
-                if (s_abs[i] > win || (s_abs[i] == win && s_idx[i] < win_idx)) {
-                    win = s_abs[i];
-                    win_idx = s_idx[i];
-                }
-            const bool found = win_idx != 0x7fffffff;
-            if (found && a_best == win && i_best == win_idx) {
-                best.index = i_best;
-                *s_cand = best;
-            }
-            __syncthreads();
-    return found;
+        if (win_idx != 0x7fffffff && a_best == win && i_best == win_idx) sh.cand = best;
+        __syncthreads();
+        best = sh.cand;
+        if (win_idx == 0x7fffffff) best.index = win_idx;
+    }
+    const int from = alone ? owner : 0;
+    Picked out;
+    out.found = win_idx != 0x7fffffff;
+    out.c.score = read_lane(best.score, from);
+    out.c.index = read_lane(best.index, from);
+    out.c.miss.g = read_lane(best.miss.g, from);
+    out.c.miss.h = read_lane(best.miss.h, from);
+    out.c.left.g = read_lane(best.left.g, from);
+    out.c.left.h = read_lane(best.left.h, from);
+    out.c.feature = read_lane(best.feature, from);
+    out.c.bin = read_lane(best.bin, from);
+    return out;
 }
 
 __device__ __forceinline__ void apply_candidate(const TreeBuffers &tb, int x, int x_in, const TreeNode &node, bool found,
@@ -157,14 +183,11 @@ template <bool DIRECT, typename BinT, bool UPDATE, bool PLANNED>
 __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, DenseBins bins, int level, float rt_eps,
                                                        float lambda) {
     __shared__ int lds[kWaves];
-    __shared__ int s_item[5];
-    __shared__ SplitCand s_cand;
-    __shared__ float s_abs[kWaves];
-    __shared__ int s_idx[kWaves];
+    __shared__ PickShared s_pick;
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int *__restrict__ ridx = tb.list(level);
     const int item = blockIdx.x;
-    const NodeItem it = locate_item<PLANNED>(tb, level, item, lds, s_item);
+    const NodeItem it = locate_item<PLANNED>(tb, level, item);
     if (it.x_in < 0) return;
     const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
     const int2 sg = it.seg;
@@ -182,17 +205,17 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
         row[k] = DIRECT ? pos : ridx[pos];
     }
     const TreeNode node = tb.nodes[x];
-    bool splits, found = false, dr = false;
+    Picked best{};
+    bool splits, dr = false;
     int f = 0, sbid = 0;
     if (UPDATE) {
-        const bool valid = node.is_valid;
-        found = pick_candidate<kWaves>(tb, x_in, valid, s_abs, s_idx, &s_cand);
-        splits = found && fabsf(s_cand.score) > rt_eps;
+        best = pick_candidate<kWaves>(tb, x_in, node.is_valid, s_pick);
+        splits = best.found && fabsf(best.c.score) > rt_eps;
         if (splits) {
-            f = s_cand.feature;
+            f = best.c.feature;
             // (the byte that the model keeps, unless the features have more than 255 bins)
-            sbid = tb.split_bin != nullptr ? s_cand.bin : (int)(unsigned char)s_cand.bin;
-            dr = s_cand.score < 0;
+            sbid = tb.split_bin != nullptr ? best.c.bin : (int)(unsigned char)best.c.bin;
+            dr = best.c.score < 0;
         }
     } else {
         splits = node_splits(node);
@@ -204,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     }
     // (the tree's own stores come last: nothing of this workgroup waits for them)
     auto update = [&] {
-        if (UPDATE && item == it.first && threadIdx.x == 0) apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
+        if (UPDATE && item == it.first && threadIdx.x == 0) apply_candidate(tb, x, x_in, node, best.found, best.c, rt_eps, lambda);
     };
     if (!splits) {
         if (threadIdx.x == 0) tb.pitem_nleft[item] = 0;
@@ -260,15 +283,13 @@ __global__ __launch_bounds__(kBlock) void k_split_groups(TreeBuffers tb_all, int
 // row ids was measured: it makes the histogram's gradient reads sequential but costs more here than it saves there.)
 template <bool DIRECT, bool GROUPS, bool PLANNED>
 __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, int level) {
-    __shared__ int lds[kWaves];
-    __shared__ int s_item[5];
     __shared__ int s_sum[2][kWaves];
     __shared__ int s_cnt[kPartChunk / kBlock][2][kWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int *__restrict__ ridx_cur = tb.list(level);
     int *__restrict__ ridx_next = tb.list(level + 1);
     const int item = blockIdx.x;
-    const NodeItem it = locate_item<PLANNED>(tb, level, item, lds, s_item);
+    const NodeItem it = locate_item<PLANNED>(tb, level, item);
     if (it.x_in < 0) return;
     const int x_in = it.x_in, x = (1 << level) - 1 + x_in;
     const int2 sg = it.seg;
@@ -461,9 +482,7 @@ template <int LPR, bool BIN16>
 __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
                                                             int level, float rt_eps, float lambda) {
     extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
-    __shared__ SplitCand s_cand;
-    __shared__ float s_abs[kSmallWaves];
-    __shared__ int s_idx[kSmallWaves];
+    __shared__ PickShared s_pick;
     __shared__ int s_left[kSmallSteps * kSmallWaves + 1];  // rows that go left: per step and wavefront, then before them
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
@@ -485,21 +504,21 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     }
     const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
     for (int i = threadIdx.x; i < nb; i += kSmallBlock) lds[i] = 0ull;
-    const bool found = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_abs, s_idx, &s_cand);
-    const bool splits = found && fabsf(s_cand.score) > rt_eps;
+    const Picked best = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_pick);
+    const bool splits = best.found && fabsf(best.c.score) > rt_eps;
     const bool first = fb == 0 && threadIdx.x == 0;
     if (!splits) {
         if (first) {
             tb.node_nleft[x_in] = 0;
             if (node.lch_index >= 0) tb.seg[node.lch_index] = tb.seg[node.rch_index] = make_int2(0, 0);
             tb.hpair_built[x_in] = -1;
-            apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
+            apply_candidate(tb, x, x_in, node, best.found, best.c, rt_eps, lambda);
         }
         return;
     }
-    const int f = s_cand.feature;
-    const int sbid = tb.split_bin != nullptr ? s_cand.bin : (int)(unsigned char)s_cand.bin;
-    const bool dr = s_cand.score < 0;
+    const int f = best.c.feature;
+    const int sbid = tb.split_bin != nullptr ? best.c.bin : (int)(unsigned char)best.c.bin;
+    const bool dr = best.c.score < 0;
     int c = f, lo = 0, span = BIN16 ? kMissingBin16 : kMissingBin;
     if (!BIN16 && bins.feat_col != nullptr) {  // (see k_split_count)
         c = bins.feat_col[f];
@@ -530,13 +549,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
             v[q] = s_left[lane * 4 + q];
             sum += v[q];
         }
-        int upto = sum;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(upto, d);
-            if (lane >= d) upto += o;
-        }
-        int before = upto - sum;
+        int before = wave_scan_i(sum) - sum;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             s_left[lane * 4 + q] = before;
@@ -618,7 +631,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
         tb.hpair_built[x_in] = built;
         atomicAdd(&tb.ctl[level + 1].n_hitems, 1);
         atomicAdd(&tb.ctl[level + 1].rows_built, m);
-        apply_candidate(tb, x, x_in, node, found, s_cand, rt_eps, lambda);
+        apply_candidate(tb, x, x_in, node, best.found, best.c, rt_eps, lambda);
     }
 }
 

@@ -55,20 +55,8 @@ __device__ SegResult eval_segment(const longlong2 *cells, int stride, int kf, in
         incg[j] = rung;
         inch[j] = runh;
     }
-    long long aggg = rung, aggh = runh;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const long long pg = shfl_up_ll(aggg, d), ph = shfl_up_ll(aggh, d);
-        if (lane >= d) {
-            aggg += pg;
-            aggh += ph;
-        }
-    }
-    // totals: the last lane's inclusive sum
-    const long long totg = (long long)(((unsigned long long)(unsigned)__shfl((int)((unsigned long long)aggg >> 32), 63) << 32) |
-                                       (unsigned)__shfl((int)(unsigned)(unsigned long long)aggg, 63));
-    const long long toth = (long long)(((unsigned long long)(unsigned)__shfl((int)((unsigned long long)aggh >> 32), 63) << 32) |
-                                       (unsigned)__shfl((int)(unsigned)(unsigned long long)aggh, 63));
+    const long long aggg = wave_scan_ll(rung), aggh = wave_scan_ll(runh);
+    const long long totg = read_lane_ll(aggg, 63), toth = read_lane_ll(aggh, 63);  // the last lane's inclusive sum
     SegResult r;
     r.win = -1.f;
     r.win_idx = 0x7fffffff;
@@ -103,20 +91,12 @@ __device__ SegResult eval_segment(const longlong2 *cells, int stride, int kf, in
             }
         }
     }
-    float win = best;
-    int win_idx = best_idx;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const float oa = __shfl_xor(win, d);
-        const int oi = __shfl_xor(win_idx, d);
-        if (oa > win || (oa == win && oi < win_idx)) {
-            win = oa;
-            win_idx = oi;
-        }
-    }
+    // (lanes hold ascending bins: among equal gains the first lane's is the smallest)
+    const float win = wave_max_f(best);
+    const int first = __ffsll((long long)__ballot(best == win)) - 1;
     r.win = win;
-    r.win_idx = win_idx;
-    r.owner = best == win && best_idx == win_idx && best >= 0.f;
+    r.win_idx = read_lane(best_idx, first);
+    r.owner = lane == first && best >= 0.f;
     r.score = best_score;
     r.miss = m;
     r.left = best_left;
@@ -462,6 +442,18 @@ struct RareSum {
 };
 __device__ __forceinline__ RareSum operator+(RareSum a, RareSum b) { return {a.g + b.g, a.h + b.h, a.n + b.n}; }
 
+struct RareScan {
+    RareSum sum;
+    int flag;  // a run starts in one of the lanes summed up
+    template <int CTRL, int ROWS>
+    __device__ __forceinline__ void at() {
+        const RareSum o{dpp_ll<CTRL, ROWS>(sum.g), dpp_ll<CTRL, ROWS>(sum.h), dpp_i<CTRL, ROWS>(0, sum.n)};
+        const int of = dpp_i<CTRL, ROWS>(0, flag);
+        if (!flag) sum = o + sum;
+        flag |= of;
+    }
+};
+
 // Inclusive segmented scan (thread t owns positions t * V ..): v[j] becomes the sum from the start of its run
 // (head = a run starts here) up to j. Two barriers.
 template <int V>
@@ -475,26 +467,13 @@ __device__ void rare_block_scan(RareSum (&v)[V], const bool (&head)[V], RareSum 
         any = any || head[j];
         v[j] = run;
     }
-    RareSum agg = run;
-    int flag = any ? 1 : 0;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const RareSum o{shfl_up_ll(agg.g, d), shfl_up_ll(agg.h, d), __shfl_up(agg.n, d)};
-        const int of = __shfl_up(flag, d);
-        if (lane >= d) {
-            if (!flag) agg = o + agg;
-            flag |= of;
-        }
-    }
-    RareSum carry{shfl_up_ll(agg.g, 1), shfl_up_ll(agg.h, 1), __shfl_up(agg.n, 1)};
-    int cflag = __shfl_up(flag, 1);
-    if (lane == 0) {
-        carry = RareSum{0, 0, 0};
-        cflag = 0;
-    }
+    RareScan scan{run, any ? 1 : 0};
+    wave_scan_steps(scan);
+    RareSum carry{dpp_ll<kDppWaveShr1>(scan.sum.g), dpp_ll<kDppWaveShr1>(scan.sum.h), dpp_i<kDppWaveShr1>(0, scan.sum.n)};
+    const int cflag = dpp_i<kDppWaveShr1>(0, scan.flag);  // (nothing in lane 0)
     if (lane == 63) {
-        s_agg[w] = agg;
-        s_flag[w] = flag;
+        s_agg[w] = scan.sum;
+        s_flag[w] = scan.flag;
     }
     __syncthreads();
     RareSum before{0, 0, 0};

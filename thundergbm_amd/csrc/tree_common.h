@@ -16,12 +16,7 @@ constexpr int kHistBlock = 1024;      // threads per histogram workgroup (they s
 template <int NW = kWaves>
 __device__ int block_excl_scan(int v, int *lds, int *total) {
     int lane = lane_id(), w = wave_id();
-    int inc = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int t = __shfl_up(inc, d);
-        if (lane >= d) inc += t;
-    }
+    const int inc = wave_scan_i(v);
     if (lane == 63) lds[w] = inc;
     __syncthreads();
     int base = 0, tot = 0;
@@ -37,8 +32,7 @@ __device__ int block_excl_scan(int v, int *lds, int *total) {
 }
 
 __device__ int block_sum(int v, int *lds) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    v = wave_sum_i(v);
     if (lane_id() == 0) lds[wave_id()] = v;
     __syncthreads();
     int tot = 0;
@@ -119,12 +113,6 @@ __device__ __forceinline__ void apply_split(const TreeBuffers &tb, int x, int x_
     tb.sp[x_in] = s;
 }
 
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-    return v;
-}
-
 // Rows per histogram work item of a level that builds n_built nodes of `total` rows. Every built node adds up to one
 // partly filled item: the items are sized so that their number stays within target_hitems (= the workgroups the chip
 // holds at once; one more would run as a second round).
@@ -163,28 +151,18 @@ struct HistPlan {
 // k_hist_merge and the profile
 __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_pairs, int item, bool publish, int level) {
     const int lane = lane_id();
-    HistPlan out;
-    // (the same in every lane: scalar registers from here on)
-    auto scalars = [&] {
-        out.pair = __builtin_amdgcn_readfirstlane(out.pair);
-        out.built = __builtin_amdgcn_readfirstlane(out.built);
-        out.chunk = __builtin_amdgcn_readfirstlane(out.chunk);
-        out.first_item = __builtin_amdgcn_readfirstlane(out.first_item);
-        out.item0 = __builtin_amdgcn_readfirstlane(out.item0);
-        out.seg = make_int2(__builtin_amdgcn_readfirstlane(out.seg.x), __builtin_amdgcn_readfirstlane(out.seg.y));
-        return out;
-    };
+    HistPlan out;  // (the same in every lane: scalar registers)
     if (tb.planned(level)) {
         const LevelCtl ctl = tb.ctl[level];
-        if (item >= ctl.n_hitems) return scalars();
+        if (item >= __builtin_amdgcn_readfirstlane(ctl.n_hitems)) return out;
         out.pair = find_owner_wave(tb.hpair_begin, n_pairs, item);
         const int4 q = tb.hpair_plan[out.pair];
-        out.built = q.x;
-        out.seg = make_int2(q.y, q.z);
-        out.chunk = ctl.hchunk;
-        out.first_item = tb.hpair_begin[out.pair];
-        out.item0 = tb.hpair_begin[tb.hpair_lo(level)];
-        return scalars();
+        out.built = __builtin_amdgcn_readfirstlane(q.x);
+        out.seg = make_int2(__builtin_amdgcn_readfirstlane(q.y), __builtin_amdgcn_readfirstlane(q.z));
+        out.chunk = __builtin_amdgcn_readfirstlane(ctl.hchunk);
+        out.first_item = __builtin_amdgcn_readfirstlane(tb.hpair_begin[out.pair]);
+        out.item0 = __builtin_amdgcn_readfirstlane(tb.hpair_begin[tb.hpair_lo(level)]);
+        return out;
     }
     int4 mine = make_int4(-1, 0, 0, 0);
     if (lane < n_pairs) mine = tb.hpair_plan[lane];
@@ -202,31 +180,26 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
     for (int p0 = 0; p0 < n_pairs; p0 += 64) {
         const int4 q = p0 == 0 ? mine : (p0 + lane < n_pairs ? tb.hpair_plan[p0 + lane] : make_int4(-1, 0, 0, 0));
         const int cnt = q.x >= 0 ? (q.z - q.y + chunk - 1) / chunk : 0;
-        int inc = cnt;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(inc, d);
-            if (lane >= d) inc += t;
-        }
+        const int inc = wave_scan_i(cnt);
         const int ex = carry + inc - cnt;
         const int lo = tb.hpair_lo(level);
-        if (lo >= p0 && lo < p0 + 64) out.item0 = __shfl(ex, lo - p0);
+        if (lo >= p0 && lo < p0 + 64) out.item0 = read_lane(ex, lo - p0);
         if (publish && p0 + lane < n_pairs) tb.hpair_begin[p0 + lane] = ex;
         const unsigned long long owner = __ballot(item >= ex && item < ex + cnt);
         if (owner != 0ull) {
             const int l = __ffsll((long long)owner) - 1;
             out.pair = p0 + l;
-            out.built = __shfl(q.x, l);
-            out.seg = make_int2(__shfl(q.y, l), __shfl(q.z, l));
-            out.first_item = __shfl(ex, l);
+            out.built = read_lane(q.x, l);
+            out.seg = make_int2(read_lane(q.y, l), read_lane(q.z, l));
+            out.first_item = read_lane(ex, l);
         }
-        carry += __shfl(inc, 63);
+        carry += read_lane(inc, 63);
     }
     if (publish && lane == 0) {
         tb.hpair_begin[n_pairs] = carry;
         tb.ctl[level] = LevelCtl{chunk, carry, 0, total};
     }
-    return scalars();
+    return out;
 }
 
 }  // namespace

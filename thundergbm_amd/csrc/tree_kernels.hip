@@ -1014,17 +1014,43 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// What search_pack needs of a lane's four bins, loaded early so that nothing waits for it there.
+struct PackMeta {
+    unsigned meta[4];  // TreeBuffers::bin_meta: one word per bin instead of the chain bin -> feature -> feature's bin range
+    bool ignored[4];
+    __device__ __forceinline__ void load(const TreeBuffers &tb, int b_begin, int b_end) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) meta[j] = tb.bin_meta[max(0, min(b_begin + lane_id() * 4 + j, b_end - 1))];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            ignored[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[max(0, min(b_begin + lane_id() * 4 + j, b_end - 1))]] != 0;
+    }
+};
+
+// One step of the segmented scan of a wavefront: the sums since the last lane in which a feature begins.
+struct PackScan {
+    long long g, h;
+    int flag;  // a feature begins in one of the lanes summed up
+    template <int CTRL, int ROWS>
+    __device__ __forceinline__ void at() {
+        const long long pg = dpp_ll<CTRL, ROWS>(g), ph = dpp_ll<CTRL, ROWS>(h);
+        const int pf = dpp_i<CTRL, ROWS>(0, flag);
+        g += flag ? 0 : pg;
+        h += flag ? 0 : ph;
+        flag |= pf;
+    }
+};
+
 // The search of one pack of one node, by one wavefront: s_v holds the pack's bins, s_miss takes its features' missing sums
 // (kEvalPackBins entries each).
-__device__ __forceinline__ void search_pack(const TreeBuffers &tb, const longlong2 *s_v, GHPair *s_miss, int x_in, int pack,
-                                            bool active, int b_begin, int b_end, GHPair S, double inv_g, double inv_h, float mcw,
-                                            float lambda) {
+__device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMeta &pm, const longlong2 *s_v, GHPair *s_miss,
+                                            int x_in, int pack, bool active, int b_begin, int b_end, GHPair S, double inv_g,
+                                            double inv_h, float mcw, float lambda) {
 #pragma clang fp contract(off)
     const int lane = lane_id();
     long long incg[4], inch[4];
     int lastb[4];  // pack-relative index of the last bin of the element's feature
-    bool valid[4], head[4], last[4], ign[4];
-    unsigned meta[4] = {0, 0, 0, 0};
+    bool valid[4], head[4], last[4];
     long long rung = 0, runh = 0;
     bool any_head = false;
 #pragma unroll
@@ -1034,15 +1060,11 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const longlon
         lastb[j] = 0;
         head[j] = false;
         last[j] = false;
-        ign[j] = false;
         incg[j] = inch[j] = 0;
         if (valid[j]) {
             const longlong2 v = s_v[lane * 4 + j];
-            // one word per bin instead of the chain bin -> feature -> feature's bin range
-            meta[j] = tb.bin_meta[b];
-            ign[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[b]] != 0;
-            const int to_last = (int)(meta[j] & 0xffu);
-            head[j] = (meta[j] & 0xff00u) == 0;
+            const int to_last = (int)(pm.meta[j] & 0xffu);
+            head[j] = (pm.meta[j] & 0xff00u) == 0;
             last[j] = to_last == 0;
             lastb[j] = b + to_last - b_begin;
             if (head[j]) {
@@ -1058,23 +1080,9 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const longlon
         }
     }
     // wavefront segmented inclusive scan of the lane aggregates
-    long long aggg = rung, aggh = runh;
-    int flag = any_head ? 1 : 0;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        long long pg = shfl_up_ll(aggg, d);
-        long long ph = shfl_up_ll(aggh, d);
-        int pf = __shfl_up(flag, d);
-        if (lane >= d) {
-            if (!flag) {
-                aggg += pg;
-                aggh += ph;
-            }
-            flag |= pf;
-        }
-    }
-    long long carryg = shfl_up_ll(aggg, 1), carryh = shfl_up_ll(aggh, 1);
-    if (lane == 0) carryg = carryh = 0;
+    PackScan scan{rung, runh, any_head ? 1 : 0};
+    wave_scan_steps(scan);
+    const long long carryg = dpp_ll<kDppWaveShr1>(scan.g), carryh = dpp_ll<kDppWaveShr1>(scan.h);  // (0 in lane 0)
     bool seen = false;
     long long exg[4], exh[4];
 #pragma unroll
@@ -1112,33 +1120,22 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const longlon
             GHPair l2{l.g + m.g, l.h + m.h};
             float gl = split_gain(S, l2, mcw, lambda);
             float score = (gl > gr) ? gl : -gr;
-            if (ign[j]) score = 0.f;  // column sampling: hist_tree_builder_single.cu:304 / :663
+            if (pm.ignored[j]) score = 0.f;  // column sampling: hist_tree_builder_single.cu:304 / :663
             float a = fabsf(score);
             if (a > best) {
                 best = a;
                 best_score = score;
                 best_idx = b_begin + lane * 4 + j;
-                best_meta = meta[j];
+                best_meta = pm.meta[j];
                 best_miss = m;
                 best_left = l;
             }
         }
     }
-    // wavefront arg-max: larger |score| wins, ties go to the smaller bin index. Only the key travels through the
-    // butterfly; the lane that holds the winner writes its candidate itself.
-    float win = best;
-    int win_idx = best_idx;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const float oa = __shfl_xor(win, d);
-        const int oi = __shfl_xor(win_idx, d);
-        if (oa > win || (oa == win && oi < win_idx)) {
-            win = oa;
-            win_idx = oi;
-        }
-    }
-    // (without any candidate every lane still holds the initial key and the first one writes the empty record)
-    const unsigned long long owners = __ballot(best == win && best_idx == win_idx);
+    // wavefront arg-max: larger |score| wins, ties go to the smaller bin index, which is the first lane's: lanes hold ascending
+    // bins. The lane that holds the winner writes its candidate itself (without any candidate every lane holds the initial
+    // one and the first lane writes the empty record).
+    const unsigned long long owners = __ballot(best == wave_max_f(best));
     if (active && lane == __ffsll((long long)owners) - 1) {
         SplitCand c;
         c.score = best_score;
@@ -1174,6 +1171,8 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
         b_begin = tb.pack_begin[pack];
         b_end = tb.pack_begin[pack + 1];
     }
+    PackMeta pm;
+    pm.load(tb, b_begin, b_end);
     GHPair S = nd.sum_gh_pair;
     longlong2 *h = hist_q + (size_t)x_in * tb.n_bins;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
@@ -1219,7 +1218,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
         }
     }
     wave_lds_sync();
-    search_pack(tb, s_v[w], s_miss[w], x_in, pack, active, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
+    search_pack(tb, pm, s_v[w], s_miss[w], x_in, pack, active, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
 // k_hist_merge and k_eval_split of a level in one launch: a workgroup owns a pack of a sibling pair. Its wavefronts share
@@ -1249,6 +1248,8 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
         parent[c] = make_longlong2(0, 0);
         if (!ROOT && b < nb) parent[c] = tb.hist(level + 1)[(size_t)p * n_bins + b_begin + b];
     }
+    PackMeta pm;
+    if (w < (ROOT ? 1 : 2)) pm.load(tb, b_begin, b_end);
     const int sibling = (built & 1) ? built + 1 : built - 1;
     GHPair S{0, 0};
     if (!ROOT) S = tb.nodes[w == 0 ? built : sibling].sum_gh_pair;
@@ -1354,7 +1355,7 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
         S = root_sums(tb, G, H);
         if (pack == 0 && lane == 0) set_root_sums(tb, S, lambda);
     }
-    search_pack(tb, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
+    search_pack(tb, pm, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
 // Split search for features of any number of bins (max_num_bin above 255): one workgroup per (feature, node) walks the
@@ -1431,15 +1432,7 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
         const int b = base + threadIdx.x;
         longlong2 v = make_longlong2(0, 0);
         if (b < ce) v = (h_par != nullptr && !store_sibling) ? wide_bin(h, h_par, h_built, b) : h[b];
-        long long ig = v.x, ih = v.y;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const long long pg = shfl_up_ll(ig, d), ph = shfl_up_ll(ih, d);
-            if (lane >= d) {
-                ig += pg;
-                ih += ph;
-            }
-        }
+        const long long ig = wave_scan_ll(v.x), ih = wave_scan_ll(v.y);
         if (lane == 63) {
             s_g[w] = ig;
             s_h[w] = ih;
@@ -1475,17 +1468,9 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
         carry_h += ch;
     }
     // workgroup arg-max: larger |score| wins, ties go to the smaller bin index (hist_tree_builder_single.cu:330-335)
-    float win = best;
-    int win_idx = best_idx;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const float oa = __shfl_xor(win, d);
-        const int oi = __shfl_xor(win_idx, d);
-        if (oa > win || (oa == win && oi < win_idx)) {
-            win = oa;
-            win_idx = oi;
-        }
-    }
+    float win;
+    int win_idx;
+    wave_best(best, best_idx, &win, &win_idx);
     if (lane == 0) {
         s_abs[w] = win;
         s_idx[w] = win_idx;
@@ -1554,16 +1539,13 @@ __global__ __launch_bounds__(kBlock) void k_best_update(TreeBuffers tb_all, int 
             best_pack = p;
         }
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        float oa = __shfl_xor(best, d);
-        int oi = __shfl_xor(best_idx, d);
-        int op = __shfl_xor(best_pack, d);
-        if (oa > best || (oa == best && oi < best_idx)) {
-            best = oa;
-            best_idx = oi;
-            best_pack = op;
-        }
+    {
+        float win;
+        int win_idx;
+        const int owner = wave_best(best, best_idx, &win, &win_idx);
+        best_pack = read_lane(best_pack, owner);
+        best = win;
+        best_idx = win_idx;
     }
     if (lane_id() == 0) {
         s_abs[wave_id()] = best;
