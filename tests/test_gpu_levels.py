@@ -78,3 +78,29 @@ def test_rows_of_nodes_of_many_items(n):
             node = np.where(inner, np.where(left, tree["lch"][node], tree["rch"][node]), node)
     assert np.array_equal(s.nid(), node)
     s.close()
+
+
+@pytest.mark.parametrize("n,F,depth,bins,objective,missing", [
+    (16_385, 4, 8, 255, "binary:logistic", 0.0), (30_000, 3, 10, 16, "reg:linear", 0.3), (20_480, 30, 5, 63, "binary:logistic", 0.1),
+    (70_001, 9, 8, 1000, "reg:linear", 0.1), (100_000, 21, 7, 255, "multi:softmax", 0.1), (240_000, 28, 8, 255, "reg:logistic", 0.0),
+    (500_001, 28, 8, 255, "binary:logistic", 0.05), (50_000, 260, 6, 255, "reg:linear", 0.0), (1_048_575, 16, 7, 255, "reg:linear", 0.0)])
+def test_lists_and_histograms_in_one_launch(n, F, depth, bins, objective, missing, monkeypatch):
+    """k_split_hist against the scatter and histogram launches: 1, 2 and 4 partition items a workgroup, records with and
+    without gradient words, 16-bit bins, several blocks, class trees, sorted rows (all rows of a child in one workgroup)."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, F)).astype(np.float32)
+    X = X[np.argsort(X[:, 0])]
+    X[rng.random((n, F)) < missing] = 0
+    z = X[:, 0] + np.abs(X[:, F // 2]) + 0.3 * rng.standard_normal(n)
+    y = z if objective == "reg:linear" else (np.digitize(z, [0, 1]) if objective.startswith("multi") else z > 0.5)
+    val, rp, col = D.dense_to_csr(X)
+    out = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("TGBM_SPLIT_HIST", switch)
+        s = T.Session(val, rp, col, np.asarray(y, np.float32), depth=depth, n_trees=3, learning_rate=0.5, max_num_bin=bins,
+                      objective=objective)
+        s.boost(3)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), s.metric_log().tobytes()))
+        s.close()
+    assert out[0] == out[1]

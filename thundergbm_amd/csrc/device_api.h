@@ -77,6 +77,16 @@ constexpr int kPartChunk = 2048;   // rows per partition work item (256 threads 
 // grows with the rows a second time. Items whose counts then also come as one sum:
 constexpr int kPartGroupRows = 1 << 24;
 constexpr int kPartGroup = 64;
+// Dense layout, below so many rows (from there on the rows are re-ordered by leaves: those of a child follow each other, and
+// one workgroup has them all): a level's row lists and the next level's histograms in one launch (launch_partition_hist), by
+// workgroups of 1, 2 or 4 partition items, as few as keep the histograms that they store below kSplitHistBytes. Beyond, storing
+// and reading them back takes longer than more workgroups save, and where four items are not enough the launches for many
+// rows are as fast. ms a tree with 1, 2, 4 items and with launch_hist_dense: 100 k x 28 (3 MB with 1): 0.216, 0.232, 0.269, 0.236;
+// 500 k x 28 (14 MB): 0.270, 0.265, 0.296, 0.281; 900 k x 28 (25 MB): 0.318, 0.298, 0.311, 0.329; 50 k x 700 (36 MB): 0.295, 0.290,
+// 0.275, 0.294; 500 k x 54, 8 classes (41 MB): 0.631, 0.534, 0.515, 0.543; 400 k x 60, 6 classes (144 MB): 0.71, 0.62, 0.556, 0.529.
+constexpr int kSplitHistRows = 1 << 20;
+constexpr int kSplitHistMost = 4;
+constexpr size_t kSplitHistBytes = 13 << 20;
 // Dense layout: up to so many pairs (nodes, where single nodes are built) in a level every workgroup plans for itself.
 constexpr int kUnplannedPairs = 256;
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
@@ -423,6 +433,7 @@ struct TreeLeftovers {  // of the tree before: see k_tree_init
     const double *metric_partial = nullptr;
     int metric_kind = 0, metric_blocks = 0;
     bool small = false;  // (of the tree that begins) the rows' nodes are kept in tb.nid
+    int run = 0;         // (of the tree that begins) the levels' histograms are launch_partition_hist's, see there
 };
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda,
                       bool stats_ready = false, int n_class = 1, const TreeLeftovers &left = TreeLeftovers());
@@ -445,7 +456,8 @@ void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mc
                        bool store_sibling = true, bool derive = false);
 // Dense layout, all nodes of the level at once: launch_hist_merge and launch_eval_split in one launch (level 0: and
 // launch_root_sum, needs a complete feature). store: the histograms are kept (nobody reads those of a tree's last level).
-void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store);
+// run: the histograms' work items are launch_partition_hist's, of so many rows of the parents (0: launch_hist_dense's).
+void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run = 0);
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
                             bool store_sibling = true, bool derive = false);
@@ -454,6 +466,13 @@ void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float r
 // not been applied to the tree yet (launch_best_update); it happens here.
 void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
                             float rt_eps, float lambda, int n_class = 1);
+// Dense layout, moderately many rows: launch_partition_dense and the histograms of the next level's built nodes in two
+// launches instead of three (k_split_hist). split_hist_run: rows of a level's node that a workgroup of the second one serves,
+// 0: such data goes through launch_partition_dense and launch_hist_dense. Inside boost() only (level tb.depth - 1 is not
+// partitioned; the level's candidates are fresh).
+int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class);
+void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
+                           float rt_eps, float lambda, int n_class = 1);
 // Dense layout, few rows: the level's splits, the children's lists and the histograms of the next level's built nodes in one
 // launch. The split search of the next level then derives the siblings (launch_eval_split with derive).
 bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins);

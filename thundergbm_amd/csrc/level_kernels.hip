@@ -635,12 +635,227 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     }
 }
 
+// A run of a node's rows: run / kPartChunk consecutive partition items of it, at least one run for every node.
+struct NodeRun {
+    int x_in;        // node within the level, -1: there is no such run
+    int first, count;  // runs of the node, numbered node by node
+    int pitem, pitems;  // its partition items
+    int2 seg;
+};
+__device__ __forceinline__ NodeRun locate_run(const TreeBuffers &tb, int level, int item, int run) {
+    const int nl = 1 << level;
+    const int2 *__restrict__ segs = tb.seg + (nl - 1);
+    NodeRun out;
+    out.x_in = -1;
+    if (level == 0) {
+        out.first = out.pitem = 0;
+        out.count = max(1, (tb.n + run - 1) / run);
+        out.pitems = max(1, (tb.n + kPartChunk - 1) / kPartChunk);
+        out.seg = make_int2(0, tb.n);
+        if (item < out.count) out.x_in = 0;
+        return out;
+    }
+    constexpr int A = 4;  // 64 nodes each, loaded together
+    int carry = 0, pcarry = 0;
+    for (int base = 0; base < nl; base += A * 64) {
+        int2 sg[A];
+#pragma unroll
+        for (int a = 0; a < A; ++a) sg[a] = segs[min(base + a * 64 + lane_id(), nl - 1)];
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            if (base + a * 64 >= nl) break;
+            const bool in = base + a * 64 + lane_id() < nl;
+            const int rows = sg[a].y - sg[a].x;
+            const int cnt = in ? max(1, (rows + run - 1) / run) : 0, pcnt = in ? max(1, (rows + kPartChunk - 1) / kPartChunk) : 0;
+            const int inc = wave_scan_i(cnt), ex = carry + inc - cnt, pinc = wave_scan_i(pcnt);
+            const unsigned long long owner = __ballot(item >= ex && item < ex + cnt);
+            if (owner != 0ull) {
+                const int l = __ffsll((long long)owner) - 1;
+                out.x_in = base + a * 64 + l;
+                out.first = read_lane(ex, l);
+                out.count = read_lane(cnt, l);
+                out.pitem = pcarry + read_lane(pinc - pcnt, l);
+                out.pitems = read_lane(pcnt, l);
+                out.seg = make_int2(read_lane(sg[a].x, l), read_lane(sg[a].y, l));
+                return out;
+            }
+            carry += read_lane(inc, 63);
+            pcarry += read_lane(pinc, 63);
+        }
+    }
+    return out;
+}
+
+// Moderately many rows (split_hist_run): k_split_scatter and the next level's k_hist_dense in one launch. A workgroup owns a
+// run of S partition items of a node and a feature block. The counts of the node's items tell it where the run's rows go and
+// which child has fewer rows; those of them that go there meet in LDS, and their histogram is a work item of the next level,
+// stored packed at the child's own scale (item_shift), so its sums are k_hist_dense's whatever the items. The first block
+// stores the lists. Bound by its chain of dependent steps - segments, decisions with rows and counts, lists, records - and by
+// the LDS, which adds about 8 pairs a nanosecond and CU to random bins: 1000 rows x 28 in 3.5 us.
+// 500 k x 28: 9.5 us with 1 item, where scatter, gap and histogram (which looks for its pair and fetches the row ids again) took
+// 13.3; a tree of depth 8 0.281 -> 0.266 ms.
+// Measured and not kept: every row's addend rounded once, by a thread of its own, and passed on through LDS (the LDS is what it
+// waits for: 4.6 -> 6.1 us in that part); the decisions taken here as well, the runs of a node telling each other their counts
+// through agent-scope atomics (a launch less, but 245 workgroups that look at 245 words each: a tree 0.32 instead of 0.27 ms).
+constexpr int kRunWaves = kHistBlock / 64;
+constexpr int kRunHalves = kPartChunk / kHistBlock;  // rows of a partition item per thread
+static_assert(kSplitHistMost * kPartChunk <= kHistFlushRows, "a run's packed sums are never drained");
+static_assert(kRunHalves == 2 && kBlock * 8 == kPartChunk, "the mapping of k_split_count's decision bytes");
+template <int LPR, bool BIN16, bool GHW, int S>
+__global__ __launch_bounds__(kHistBlock) __attribute__((amdgpu_waves_per_eu(8)))
+void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level) {
+    constexpr int R = S * kRunHalves;  // rows per thread
+    constexpr int E = R * kRunWaves;   // counts of the run: one per round and wavefront
+    extern __shared__ unsigned long long lds[];  // the block's histogram, then the rows to add up
+    __shared__ int s_cnt[E < 64 ? 64 : E];
+    __shared__ int s_sum[2][kRunWaves];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    gh += (size_t)blockIdx.z * tb.n;
+    int *s_rows = reinterpret_cast<int *>(lds + tb.max_block_bins);
+    const int fb = blockIdx.x, item = blockIdx.y;
+    const NodeRun it = locate_run(tb, level, item, S * kPartChunk);
+    if (it.x_in < 0) return;
+    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
+    const int nl = 1 << level, x_in = it.x_in, x = nl - 1 + x_in;
+    const int2 sg = it.seg;
+    const int mine = item - it.first;  // of the node's runs
+    const int pb = sg.x + mine * (S * kPartChunk);
+    const int pe = min(sg.y, pb + S * kPartChunk);
+    const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
+    const int *__restrict__ ridx = tb.list(level);
+    const TreeNode &nd = tb.nodes[x];
+    const bool splits = node_splits(nd);
+    const int lch = nd.lch_index, rch = nd.rch_index;
+    int row[R];
+    unsigned rights[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+        rights[k] = tb.goes_right[(size_t)(it.pitem + min(mine * S + k, it.pitems - 1)) * kBlock + threadIdx.x % kBlock];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int pos = max(min(pb + k * kHistBlock + (int)threadIdx.x, pe - 1), 0);
+        row[k] = level == 0 ? pos : ridx[pos];
+    }
+    static_assert(kSplitHistRows / kPartChunk <= kHistBlock, "a partition item of the node per thread");
+    int total = tb.pitem_nleft[it.pitem + min((int)threadIdx.x, it.pitems - 1)];
+    if ((int)threadIdx.x >= it.pitems) total = 0;
+    int before = (int)threadIdx.x < mine * S ? total : 0;
+    const QuantCtl quant = *tb.quant;
+    for (int i = threadIdx.x; i < nb; i += kHistBlock) lds[i] = 0ull;
+    before = wave_sum_i(before);
+    total = wave_sum_i(total);
+    if (lane == 0) {
+        s_sum[0][w] = before;
+        s_sum[1][w] = total;
+    }
+    unsigned long long left_mask[R];  // (wave-uniform)
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const bool valid = pb + k * kHistBlock + (int)threadIdx.x < pe;
+        // (k_split_count's thread t decides for the rows t, t + 256, ... of a partition item, bit by bit)
+        const bool right = rights[k / kRunHalves] >> (k % kRunHalves * (8 / kRunHalves) + threadIdx.x / kBlock) & 1u;
+        left_mask[k] = __ballot(valid && !right);
+        if (lane == 0) s_cnt[k * kRunWaves + w] = __popcll(left_mask[k]);
+    }
+    __syncthreads();
+    before = wave_sum_i(lane < kRunWaves ? s_sum[0][lane % kRunWaves] : 0);
+    total = wave_sum_i(lane < kRunWaves ? s_sum[1][lane % kRunWaves] : 0);
+    const int nleft = splits ? total : 0, nright = (sg.y - sg.x) - nleft;
+    // the child with fewer rows is built from them (ties: the left one, as hist_tree_builder_single.cu:466-467)
+    const bool build_left = nleft <= nright;
+    const int built = splits ? (build_left ? lch : rch) : -1;
+    if (fb == 0 && mine == 0 && threadIdx.x == 0) {
+        tb.node_nleft[x_in] = nleft;
+        tb.seg[lch] = splits ? make_int2(sg.x, sg.x + nleft) : make_int2(0, 0);
+        tb.seg[rch] = splits ? make_int2(sg.x + nleft, sg.y) : make_int2(0, 0);
+        tb.hpair_built[x_in] = built;
+        tb.hpair_begin[x_in] = it.first;
+        if (x_in == nl - 1) tb.hpair_begin[nl] = it.first + it.count;
+        if (splits) {
+            atomicAdd(&tb.ctl[level + 1].n_hitems, it.count);
+            atomicAdd(&tb.ctl[level + 1].rows_built, min(nleft, nright));
+        }
+    }
+    if (!splits) return;
+    // lefts of the run before every (round, wavefront)
+    int sum[E > 64 ? E / 64 : 1], upto[E > 64 ? E / 64 : 1], lefts = 0;
+#pragma unroll
+    for (int q = 0; q < (E > 64 ? E / 64 : 1); ++q) {
+        sum[q] = q * 64 + lane < E ? s_cnt[q * 64 + lane] : 0;
+        const int inc = wave_scan_i(sum[q]);
+        upto[q] = lefts + inc - sum[q];
+        lefts += read_lane(inc, 63);
+    }
+    const int m = build_left ? lefts : pe - pb - lefts;  // rows of the run to add up
+    int *__restrict__ ridx_next = tb.list(level + 1);
+    const int left_base = sg.x + before, right_base = sg.x + total + ((pb - sg.x) - before);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = k * kHistBlock + (int)threadIdx.x;
+        const int e = k * kRunWaves;
+        const int l = read_lane(upto[e / 64], e % 64 + w) + lanes_below(left_mask[k]);  // lefts before row i
+        const bool left = (left_mask[k] >> lane & 1ull) != 0;
+        if (pb + i < pe) {
+            const int at = left ? l : i - l;
+            if (left == build_left) s_rows[at] = row[k];
+            if (fb == 0) ridx_next[left ? left_base + at : right_base + at] = row[k];
+        }
+    }
+    __syncthreads();
+    // The rows in batches: a batch's loads are issued together, the first ones before the scales are worked out.
+    constexpr int RPS = kHistBlock / LPR, FPL = BIN16 ? 2 : 4, U = LPR >= 16 ? 8 : 4;
+    const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
+    const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
+    unsigned pk[U];
+    GHPair s[U];
+    auto load_rows = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned r = (unsigned)s_rows[min(base + rsub + u * RPS, m - 1)];
+            pk[u] = *reinterpret_cast<const unsigned *>(blk + (r * (unsigned)(LPR * 4) + (unsigned)q * 4));
+            if (!GHW) s[u] = *reinterpret_cast<const GHPair *>(reinterpret_cast<const char *>(gh) + r * 8u);
+        }
+    };
+    if (m > 0) load_rows(0);
+    const int h_bits = quant.h_bits;
+    const int rows = max(1, min(min(nleft, nright), quant.flush_rows));
+    const int shift_g = item_shift(quant.gq_max, rows, 63 - h_bits), shift_h = quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits);
+    if (fb == 0 && threadIdx.x == 0) tb.hitem_shift[item] = make_int2(shift_g, shift_h);
+    const float scale_g = ldexpf(quant.scale_g, -shift_g), scale_h = ldexpf(quant.scale_h, -shift_h);
+    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
+    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
+    const bool word_lane = bins.gh_lane >= 0 && q == bins.gh_lane;
+    for (int base = 0; base < m; base += RPS * U) {
+        if (base > 0) load_rows(base);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (base + u * RPS >= m) break;  // (uniform)
+            const GHPair sv = GHW ? pair_from_word(bins.gh_objective, last_lane_of_row<LPR>(pk[u])) : s[u];
+            const unsigned v = base + rsub + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
+            const long long gq = round_to_ll(sv.g * scale_g), hq = round_to_ll(fmaxf(sv.h, 0.f) * scale_h);
+            const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
+            if (BIN16) {
+                const unsigned b0 = v & 0xffff, b1 = v >> 16;
+                if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
+                if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
+            } else {
+                const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
+                if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
+                if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
+                if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
+                if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
+            }
+        }
+    }
+    __syncthreads();
+    unsigned long long *out = reinterpret_cast<unsigned long long *>(tb.partial) + (size_t)item * tb.n_bins + bin0;
+    for (int i = threadIdx.x; i < nb; i += kHistBlock) out[i] = lds[i];
+}
+
 }  // namespace
 
-void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
-                            float rt_eps, float lambda, int n_class) {
-    if (level == tb.depth - 1) return;  // the last level's children never get row lists (see k_tree_end)
-    const int most = level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
+static void split_count_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update, float rt_eps,
+                               float lambda, int n_class, int most) {
     const dim3 items(most, 1, n_class);
     const bool planned = tb.planned(level);
 #define TGBM_SPLIT_COUNT(D, T, U, P) k_split_count<D, T, U, P><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
@@ -657,6 +872,69 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
     }
 #undef TGBM_SPLIT_COUNT_LEVEL
 #undef TGBM_SPLIT_COUNT
+}
+
+static int most_partition_items(const TreeBuffers &tb, int level) {
+    return level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
+}
+
+static size_t split_hist_lds(const TreeBuffers &tb, int run) { return (size_t)tb.max_block_bins * 8 + (size_t)run * 4; }
+
+int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class) {
+    if (tb.n >= kSplitHistRows || tb.planned(tb.depth - 1)) return 0;
+    for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2) {
+        const size_t stored = (size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class;
+        if (stored <= kSplitHistBytes && split_hist_lds(tb, run) + 4096 <= kLdsBytes) return run;
+    }
+    return 0;
+}
+
+template <int LPR, bool BIN16, bool GHW, int S>
+static void split_hist_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int n_class) {
+    constexpr int run = S * kPartChunk;
+    const size_t lds = split_hist_lds(tb, run);
+    static LdsOptIn opt_in;
+    if (lds > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_split_hist<LPR, BIN16, GHW, S>)});
+    const dim3 grid(bins.n_blocks, level == 0 ? (tb.n + run - 1) / run : tb.n / run + (1 << level), n_class);
+    k_split_hist<LPR, BIN16, GHW, S><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level);
+}
+
+template <int LPR, bool BIN16, bool GHW>
+static void split_hist_run_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run, int n_class) {
+    if (run == kPartChunk) split_hist_launch<LPR, BIN16, GHW, 1>(s, tb, bins, gh, level, n_class);
+    else if (run == 2 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 2>(s, tb, bins, gh, level, n_class);
+    else if (run == 4 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 4>(s, tb, bins, gh, level, n_class);
+    else fatal("runs of %d rows", run);
+}
+
+void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
+                           float rt_eps, float lambda, int n_class) {
+    if (level == tb.depth - 1) return;
+    split_count_launch(s, tb, bins, level, true, rt_eps, lambda, n_class, most_partition_items(tb, level));
+    const bool words = bins.gh_lane >= 0 && bins.gh_fresh;
+#define TGBM_SPLIT_HIST(LPR)                                                                                        \
+    if (bins.bin_bytes == 2) split_hist_run_launch<LPR, true, false>(s, tb, bins, gh, level, run, n_class);          \
+    else if (LPR >= 4 && words) split_hist_run_launch<LPR, false, (LPR >= 4)>(s, tb, bins, gh, level, run, n_class); \
+    else split_hist_run_launch<LPR, false, false>(s, tb, bins, gh, level, run, n_class);                             \
+    break
+    switch (bins.W * bins.bin_bytes) {  // bytes per row of a block
+        case 4: TGBM_SPLIT_HIST(1);
+        case 8: TGBM_SPLIT_HIST(2);
+        case 16: TGBM_SPLIT_HIST(4);
+        case 32: TGBM_SPLIT_HIST(8);
+        case 64: TGBM_SPLIT_HIST(16);
+        default: fatal("unsupported dense block width %d x %d bytes", bins.W, bins.bin_bytes);
+    }
+#undef TGBM_SPLIT_HIST
+}
+
+void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
+                            float rt_eps, float lambda, int n_class) {
+    if (level == tb.depth - 1) return;  // the last level's children never get row lists (see k_tree_end)
+    const int most = most_partition_items(tb, level);
+    const dim3 items(most, 1, n_class);
+    const bool planned = tb.planned(level);
+    split_count_launch(s, tb, bins, level, update, rt_eps, lambda, n_class, most);
     const bool groups = tb.n >= kPartGroupRows;
     if (groups) k_split_groups<<<dim3((most + kPartGroup * kWaves - 1) / (kPartGroup * kWaves), 1, n_class), kBlock, 0, s>>>(tb, most);
 #define TGBM_SPLIT_SCATTER(G)                                                      \

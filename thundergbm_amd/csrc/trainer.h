@@ -92,6 +92,7 @@ class Trainer {
     TreeLeftovers leftovers() const {
         TreeLeftovers l = left_;
         l.small = small();
+        l.run = run();
         return l;
     }
     void settle();                 // what the last tree has left to do, where no next tree takes it along
@@ -173,6 +174,8 @@ class Trainer {
     bool in_boost_ = false;
     bool small_ok_ = false;          // inside boost() the levels go through launch_small_level
     bool small() const { return in_boost_ && small_ok_; }
+    int run_rows_ = 0;               // inside boost() the levels go through launch_partition_hist, runs of so many rows
+    int run() const { return in_boost_ && !small_ok_ ? run_rows_ : 0; }
     int lookup_level_ = -1;          // level whose split nodes have not been partitioned into row lists yet
     bool next_round_ready_ = false;  // d_gh_ and the root statistics already belong to the next round
     // profiling

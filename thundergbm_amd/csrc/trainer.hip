@@ -490,8 +490,11 @@ void Trainer::alloc_tree_buffers() {
     tb.max_level_nodes = max_level_nodes;
     tb.target_hitems = std::min(512, std::max(4, 512 / bins_.n_blocks));  // ~2 resident workgroups per CU
     tb.max_hitems = tb.target_hitems + max_pairs + 1;
+    // The runs of split_hist_run: what they store, packed, in histograms of `partial`'s size.
+    const int max_runs = n_ < kSplitHistRows ? n_ / kPartChunk + max_level_nodes / 2 + 2 : 0;
+    const size_t run_slots = max_runs == 0 ? 0 : kSplitHistBytes / sizeof(longlong2) / (size_t)n_bins_ + (size_t)max_level_nodes / 4 + 2;
     tb.max_pitems = n_ / kPartChunk + max_level_nodes + 1;
-    tb.n_partial = sparse_ ? 1 : (size_t)tb.max_hitems * n_bins_;
+    tb.n_partial = sparse_ ? 1 : std::max((size_t)tb.max_hitems, run_slots) * n_bins_;
     tb.n_end_bound = ((size_t)row_blocks(n_) + 1) * (((size_t)1 << depth) - 1);
     tb.n_grad_blocks = row_blocks(n_);
     // One set of buffers per class tree of a round when that fits comfortably: the trees of a round are
@@ -508,7 +511,7 @@ void Trainer::alloc_tree_buffers() {
     int hist_nodes = max_level_nodes;
     const size_t fixed_bytes = sparse_pass_ ? 0 : (size_t)n_ * 13 + tb.n_end_bound * sizeof(int);
     auto arena_bytes = [&](int nodes) {  // two buffers + the work items' partial histograms (dense layout)
-        const size_t items = sparse_ ? 0 : (size_t)tb.target_hitems + (nodes < max_level_nodes ? nodes : max_pairs) + 2;
+        const size_t items = sparse_ ? 0 : std::max((size_t)tb.target_hitems + (nodes < max_level_nodes ? nodes : max_pairs) + 2, run_slots);
         return ((size_t)2 * nodes + items) * (size_t)n_bins_ * sizeof(longlong2);
     };
     if (!sparse_pass_) {
@@ -559,6 +562,7 @@ void Trainer::alloc_tree_buffers() {
     }
     tb.partial = dalloc<longlong2>(S * tb.n_partial);
     tb.quant = dalloc<QuantCtl>(S);
+    tb.max_hitems = std::max(tb.max_hitems, max_runs);
     tb.hitem_shift = dalloc<int2>(S * (size_t)tb.max_hitems);
     tb.root_total = dalloc<long long>(S * 512);
     // a feature that is stored in every row (checked on the bin matrix itself: a row with a repeated column index
@@ -676,6 +680,13 @@ void Trainer::alloc_tree_buffers() {
 
     const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
     small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb, bins_) && !(small_env != nullptr && std::string(small_env) == "0");
+    const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
+    if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
+        run_rows_ = split_hist_run(tb, bins_, n_sets_);
+    // What target_hitems then plans is the root: a workgroup per CU, each stores a histogram and the atomics of a CU take as long
+    // for two (500 k x 28: histogram 15.6 -> 14.6 us, sums of the items 12.6 -> 8.1; 128 items: 19 and 5.8), unless their
+    // packed sums would have to be drained.
+    if (run_rows_ > 0 && (long)n_ * n_sets_ <= 256l * kHistFlushRows) tb.target_hitems = std::max(4, tb.target_hitems / 2);
     model_cap_trees_ = std::max(1, param_.n_trees) * param_.tree_per_rounds;
     d_model_ = dalloc<TreeNode>((size_t)model_cap_trees_ * tb.n_nodes);
     d_metric_ = dalloc<float>((size_t)std::max(1, param_.n_trees));
@@ -999,7 +1010,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     }
     mark(level == 0 ? PH_GRADIENT : PH_PARTITION, level);  // closes what ran before this level's histogram
     const bool derive = small() && level > 0;  // the level before has built its histograms
-    if (!derive) build_level_hist(tb, level, gh, n_class);
+    if (!derive && !(run() > 0 && level > 0)) build_level_hist(tb, level, gh, n_class);
     mark(PH_HIST, level);
     if (!sparse_pass_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
@@ -1011,7 +1022,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
         // last level that fits a capped arena keeps them for the batches of the next one
         if (fused)
             launch_merge_eval(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                              !(in_boost_ && level == param_.depth - 1));
+                              !(in_boost_ && level == param_.depth - 1), run());
         else if (wide_eval_)
             launch_eval_split_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                                    !(in_boost_ && level == param_.depth - 1), derive);
@@ -1063,7 +1074,12 @@ void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level,
         launch_partition_csr(stream_, tb, csr_, level, n_class);
     else if (small())
         launch_small_level(stream_, tb, bins_, gh, level, param_.rt_eps, param_.lambda, n_class);
-    else
+    else if (run() > 0) {
+        DenseBins b = bins_;
+        b.gh_fresh = gh_records_fresh_ && n_class == 1 && gh == d_gh_;
+        b.gh_objective = objective_;
+        launch_partition_hist(stream_, tb, b, gh, level, run(), param_.rt_eps, param_.lambda, n_class);
+    } else
         launch_partition_dense(stream_, tb, bins_, level, update_with_partition(level), param_.rt_eps, param_.lambda, n_class);
     mark(PH_PARTITION, level);
     HIP_CHECK_LAUNCHES("partition");

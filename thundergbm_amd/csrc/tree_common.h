@@ -202,5 +202,31 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
     return out;
 }
 
+// A row's gradient pair from the word that travels in its record (word_from_row).
+__device__ __forceinline__ GHPair pair_from_word(int objective, unsigned w) {
+    GHPair o;
+    if (objective == OBJ_SQUARE) {
+        o.g = __uint_as_float(w);
+        o.h = 1.f;
+    } else {
+        const float s = __uint_as_float(w & 0x7fffffffu);
+        const float yi = (w >> 31) ? 1.f : 0.f;
+        o.g = s - yi;
+        o.h = fmaxf(s * (1.f - s), 1e-16f);
+    }
+    return o;
+}
+
+// The value that the last of the LPR lanes of a row holds, in every lane of the row (LPR = 4, 8 or 16 consecutive
+// lanes): a DPP broadcast inside the 16-lane row of the wavefront, no trip through the LDS crossbar.
+template <int LPR>
+__device__ __forceinline__ unsigned last_lane_of_row(unsigned v) {
+    if (LPR == 4) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xff, 0xf, 0xf, false);  // quad_perm:[3,3,3,3]
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x15f, 0xf, 0xf, false);  // row_newbcast:15
+    if (LPR == 16) return hi;
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x157, 0xf, 0xf, false);  // row_newbcast:7
+    return (threadIdx.x & 8u) ? hi : lo;
+}
+
 }  // namespace
 }  // namespace tgbm

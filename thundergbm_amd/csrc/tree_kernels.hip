@@ -59,25 +59,12 @@ __global__ void k_gradient_pointwise(int objective, int n, const float *__restri
 // (launch_gh_words, k_tree_end); the root level's histogram launch, which streams every record anyway, reads them
 // there and writes the records back with the word in place - whole records, so that memory sees full-sector writes
 // (4 bytes of every 32 written by themselves cost a read-modify-write per sector: 90 us per tree on 10 M rows). Squared loss: the gradient itself (the hessian is 1). Logistic loss with 0/1 labels: the
-// sigmoid s (never negative) with the label in the sign bit; pair_from_word repeats pointwise_gradient's operations on
+// sigmoid s (never negative) with the label in the sign bit; pair_from_word (tree_common.h) repeats pointwise_gradient's operations on
 // s, so both give the same bits.
 __device__ __forceinline__ unsigned word_from_row(int objective, float yi, float p) {
     if (objective == OBJ_SQUARE) return __float_as_uint(p - yi);
     const float s = 1.f / (1.f + expf(-p));
     return __float_as_uint(s) | (yi != 0.f ? 0x80000000u : 0u);
-}
-__device__ __forceinline__ GHPair pair_from_word(int objective, unsigned w) {
-    GHPair o;
-    if (objective == OBJ_SQUARE) {
-        o.g = __uint_as_float(w);
-        o.h = 1.f;
-    } else {
-        const float s = __uint_as_float(w & 0x7fffffffu);
-        const float yi = (w >> 31) ? 1.f : 0.f;
-        o.g = s - yi;
-        o.h = fmaxf(s * (1.f - s), 1e-16f);
-    }
-    return o;
 }
 
 __global__ void k_gh_words(int objective, int n, const float *__restrict__ y, const float *__restrict__ yp,
@@ -244,10 +231,11 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
     }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    if (left.small && blockIdx.x == 0) {  // every row starts in the root; k_small_level counts the levels' rows
+    if (left.small && blockIdx.x == 0) {  // every row starts in the root
         for (int i = threadIdx.x; i < tb.n; i += kBlock) tb.nid[i] = 0;
-        for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{0, 0, 0, 0};
     }
+    if ((left.small || left.run > 0) && blockIdx.x == 0)
+        for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{left.run, 0, 0, 0};
     const GradStats *__restrict__ block_sums = tb.root_partial;
     const int nn = tb.n_nodes;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < nn; i += parts * kBlock) {
@@ -386,17 +374,6 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
 // (Packing each row's gradient pair next to its bins so that a gathered row costs one 128-byte line
 // instead of two was measured: it halves the fetched bytes below the root, but the per-tree refresh of
 // the pairs costs what the gathers save.)
-// The value that the last of the LPR lanes of a row holds, in every lane of the row (LPR = 4, 8 or 16 consecutive
-// lanes): a DPP broadcast inside the 16-lane row of the wavefront, no trip through the LDS crossbar.
-template <int LPR>
-__device__ __forceinline__ unsigned last_lane_of_row(unsigned v) {
-    if (LPR == 4) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xff, 0xf, 0xf, false);  // quad_perm:[3,3,3,3]
-    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x15f, 0xf, 0xf, false);  // row_newbcast:15
-    if (LPR == 16) return hi;
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x157, 0xf, 0xf, false);  // row_newbcast:7
-    return (threadIdx.x & 8u) ? hi : lo;
-}
-
 // GHW: the rows' gradient pairs come from 32-bit words (word_from_row). Below the root the word sits in the last
 // dword of the row's record, which the row's last lane has loaded with the bins anyway: no second gather per row. The
 // root launch (DIRECT) reads the words from their own array and puts them there, storing every record back.
@@ -2606,11 +2583,12 @@ void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mc
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
 }
 
-void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store) {
+void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run) {
     const int n_pairs = tb.n_hpairs(level);
     const dim3 grid(tb.n_packs, n_pairs, n_class);
     // (as many items as the level can have, see hist_dense_launch)
-    const int items = std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
+    const int items = run > 0 && level > 0 ? tb.n / run + n_pairs
+                                           : std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
     if (level == 0) {
         // One workgroup per pack: with hundreds of items two launches that spread them over the chip are faster (512 items of
         // 28 packs: 12 + 9 instead of 43 us; 23 items of 700 packs: 18 instead of 16 + 15).
