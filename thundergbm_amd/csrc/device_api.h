@@ -91,6 +91,7 @@ constexpr size_t kSplitHistBytes = 13 << 20;
 constexpr int kUnplannedPairs = 256;
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
 constexpr int kCsrHeadBins = 4864;  // head slots of the sparse histogram: 2 x 8 bytes each, two workgroups per CU
+constexpr int kRootParts = 512;     // parts of the rows whose sums add up to the root's (the root's work items at most)
 // Rows a packed LDS bin may absorb before it is drained (QuantCtl::flush_rows). With float hessians (32 + 32-bit
 // fields) 8192: a row of a large node is then counted at 2^-17 of the tree's largest |g|, and even rows that all
 // round the same way (the first logistic tree has two gradient values) stay within 4e-6 of the sum of |g|; 32768
@@ -300,7 +301,7 @@ struct TreeBuffers {
     unsigned long long *best_key = nullptr;  // [max_level_nodes]
     const int *feat_slot = nullptr;          // [F]
     // Root sums as exact integers at the tree's scales (what a row order cannot change), from the gradients when no
-    // feature is stored in every row: [2 i], [2 i + 1] the sums of workgroup i of k_root_sum_rows (up to 256)
+    // feature is stored in every row: [2 i], [2 i + 1] the sums of part i of the rows (kRootParts at most)
     long long *root_total = nullptr;
     int complete_feature = -1;     // dense layout: a feature stored in every row (its bins add up to the root), or -1
     int max_hitems = 0, target_hitems = 0, max_pitems = 0;
@@ -390,7 +391,7 @@ struct TreeBuffers {
         t.partial += K * n_partial;
         t.quant += K;
         t.hitem_shift += K * max_hitems;
-        t.root_total += K * 512;
+        t.root_total += K * 2 * kRootParts;
         if (nid16 != nullptr) {
             t.nid16 += K * (((size_t)n + 2) / 2 * 2);
             t.node_rows += K * n_nodes;
@@ -438,8 +439,9 @@ struct TreeLeftovers {  // of the tree before: see k_tree_init
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda,
                       bool stats_ready = false, int n_class = 1, const TreeLeftovers &left = TreeLeftovers());
 void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left);
+// sum_rows (level 0): also the sums of the items' rows into tb.root_total, for a split search with root_of_rows.
 void launch_hist_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                       int n_class = 1);
+                       int n_class = 1, bool sum_rows = false);
 void launch_hist_merge(hipStream_t s, const TreeBuffers &tb, int level, int n_class = 1);
 // After the root histogram exists: replaces the root's float sums (whose last bits depend on the order of the rows)
 // by the exact fixed-point totals, from the bins of tb.complete_feature or, without one, from the gradients.
@@ -455,12 +457,13 @@ void launch_partition_csr(hipStream_t s, const TreeBuffers &tb, const CsrBins &b
 void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
                        bool store_sibling = true, bool derive = false);
 // Dense layout, all nodes of the level at once: launch_hist_merge and launch_eval_split in one launch (level 0: and
-// launch_root_sum, needs a complete feature). store: the histograms are kept (nobody reads those of a tree's last level).
+// launch_root_sum, from the bins of a complete feature or from what launch_hist_dense has summed up of the rows). store: the
+// histograms are kept (nobody reads those of a tree's last level).
 // run: the histograms' work items are launch_partition_hist's, of so many rows of the parents (0: launch_hist_dense's).
 void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run = 0);
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
-                            bool store_sibling = true, bool derive = false);
+                            bool store_sibling = true, bool derive = false, bool root_of_rows = false);
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class = 1);
 // Dense layout: the rows of a level's split nodes move into the children's lists. update: the nodes' best candidates have
 // not been applied to the tree yet (launch_best_update); it happens here.

@@ -81,17 +81,22 @@ struct Picked {
     bool found;  // false: the node has no candidate
     SplitCand c;
 };
-// Up to so many packs - one for every lane - each wavefront looks at all of them: no barrier, no LDS (500 k x 28: the
-// candidates' part of a count launch 1.7 -> 0.95 us). Beyond, the workgroup shares them out.
-constexpr int kWavePacks = 64;
+// Up to so many packs each wavefront looks at all of them: no barrier, no LDS (500 k x 28: the candidates' part of a count
+// launch 1.7 -> 0.95 us; of a small level's sixteen wavefronts 2.9 -> 0.4 with 10 packs, TODO with 100). Beyond, the workgroup
+// shares them out.
+constexpr int kWavePacks = 256;
 struct PickShared {
     SplitCand cand;
     float abs[16];
     int idx[16];
 };
+// A lane's candidate where every wavefront looks at all of them, so that its load can be issued ahead of what comes before.
+__device__ __forceinline__ SplitCand early_candidate(const TreeBuffers &tb, int x_in) {
+    return tb.cand[(size_t)x_in * tb.n_packs + min(lane_id(), tb.n_packs - 1)];
+}
 // NW: wavefronts of the workgroup, all of whose threads call
 template <int NW>
-__device__ __forceinline__ Picked pick_candidate(const TreeBuffers &tb, int x_in, bool valid, PickShared &sh) {
+__device__ __forceinline__ Picked pick_candidate(const TreeBuffers &tb, int x_in, bool valid, PickShared &sh, const SplitCand &early) {
     const bool alone = tb.n_packs <= kWavePacks;
     float a_best = -1.f;
     int i_best = 0x7fffffff;
@@ -116,7 +121,15 @@ __device__ __forceinline__ Picked pick_candidate(const TreeBuffers &tb, int x_in
         best.bin = better ? c.bin : best.bin;
     };
     if (alone) {
-        look(cand[min(lane_id(), tb.n_packs - 1)], valid && lane_id() < tb.n_packs);
+        constexpr int U = kWavePacks / 64;
+        SplitCand c[U];
+        c[0] = early;
+#pragma unroll
+        for (int u = 1; u < U; ++u)
+            if (u * 64 < tb.n_packs) c[u] = cand[min(u * 64 + lane_id(), tb.n_packs - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u * 64 < tb.n_packs) look(c[u], valid && u * 64 + lane_id() < tb.n_packs);
     } else {
         constexpr int U = 3;  // candidates per thread whose loads are issued together
         for (int p0 = threadIdx.x; p0 - (int)threadIdx.x < tb.n_packs; p0 += U * NW * 64) {
@@ -209,7 +222,7 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     bool splits, dr = false;
     int f = 0, sbid = 0;
     if (UPDATE) {
-        best = pick_candidate<kWaves>(tb, x_in, node.is_valid, s_pick);
+        best = pick_candidate<kWaves>(tb, x_in, node.is_valid, s_pick, early_candidate(tb, x_in));
         splits = best.found && fabsf(best.c.score) > rt_eps;
         if (splits) {
             f = best.c.feature;
@@ -476,21 +489,29 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 constexpr int kSmallWaves = kSmallBlock / 64;
 constexpr int kSmallSteps = kSmallRows / kSmallBlock;
 static_assert(kSmallRows / 2 <= kHistFlushRows, "the built child's packed sums are never drained");
-static_assert(kSmallRows <= 1 << 16 && kSmallSteps * kSmallWaves == 256, "16-bit row ids, four step counts per lane");
+static_assert(kSmallRows <= 1 << 16 && kSmallWaves == 16 && kSmallSteps % 4 == 0, "16-bit row ids, the counts of four steps per wavefront");
 
 template <int LPR, bool BIN16>
 __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
                                                             int level, float rt_eps, float lambda) {
     extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
     __shared__ PickShared s_pick;
-    __shared__ int s_left[kSmallSteps * kSmallWaves + 1];  // rows that go left: per step and wavefront, then before them
+    __shared__ int s_left[kSmallSteps * kSmallWaves];  // rows that go left, per step and wavefront
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
     unsigned short *s_rows = reinterpret_cast<unsigned short *>(lds + tb.max_block_bins);
     const int fb = blockIdx.x, x_in = blockIdx.y, x = (1 << level) - 1 + x_in;
-    const int lane = lane_id(), w = wave_id();
-    const TreeNode node = tb.nodes[x];
+    const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
+    // (all that follows from the node alone is requested at once)
+    const SplitCand early = early_candidate(tb, x_in);
     const int2 sg = level == 0 ? make_int2(0, tb.n) : tb.seg[x];
+    const TreeNode node = tb.nodes[x];
+    const QuantCtl quant = *tb.quant;
+    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
+    constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, U = 8;
+    const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
+    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
+    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
     const int len = sg.y - sg.x, steps = (len + kSmallBlock - 1) / kSmallBlock;
     const int *__restrict__ ridx = tb.list(level);
     int row[kSmallSteps];
@@ -502,9 +523,8 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
             row[k] = level == 0 ? pos : ridx[pos];
         }
     }
-    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
     for (int i = threadIdx.x; i < nb; i += kSmallBlock) lds[i] = 0ull;
-    const Picked best = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_pick);
+    const Picked best = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_pick, early);
     const bool splits = best.found && fabsf(best.c.score) > rt_eps;
     const bool first = fb == 0 && threadIdx.x == 0;
     if (!splits) {
@@ -542,23 +562,19 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
         if (lane == 0) s_left[k * kSmallWaves + w] = __popcll(left_mask[k]);
     }
     __syncthreads();
-    if (w == 0) {
-        int v[4], sum = 0;
+    // lefts before every (step, wavefront), and of all: by every wavefront for itself, four steps at a time
+    int upto[kSmallSteps / 4], nleft = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v[q] = s_left[lane * 4 + q];
-            sum += v[q];
+    for (int k = 0; k < kSmallSteps / 4; ++k) {
+        upto[k] = 0;
+        if (k * 4 < steps) {
+            const int own = s_left[k * 64 + lane];
+            const int inc = wave_scan_i(own);
+            upto[k] = nleft + inc - own;
+            nleft += read_lane(inc, 63);
         }
-        int before = wave_scan_i(sum) - sum;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            s_left[lane * 4 + q] = before;
-            before += v[q];
-        }
-        if (lane == 63) s_left[kSmallSteps * kSmallWaves] = before;
     }
-    __syncthreads();
-    const int nleft = s_left[kSmallSteps * kSmallWaves], nright = len - nleft;
+    const int nright = len - nleft;
     // the child with fewer rows is built from them (ties: the left one, as hist_tree_builder_single.cu:466-467)
     const bool build_left = nleft <= nright;
     const int m = build_left ? nleft : nright;
@@ -567,7 +583,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     for (int k = 0; k < kSmallSteps; ++k) {
         const int i = k * kSmallBlock + (int)threadIdx.x;
         if (k < steps && i < len) {
-            const int lefts = s_left[k * kSmallWaves + w] + lanes_below(left_mask[k]);
+            const int lefts = read_lane(upto[k / 4], k % 4 * kSmallWaves + w) + lanes_below(left_mask[k]);
             const bool left = (left_mask[k] >> lane & 1ull) != 0;
             const int at = left ? lefts : i - lefts;  // in the child's list
             if (left == build_left) s_rows[at] = (unsigned short)row[k];
@@ -578,29 +594,25 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
         }
     }
     __syncthreads();
-    const QuantCtl quant = *tb.quant;
     const int h_bits = quant.h_bits;
     const int rows = max(1, min(m, quant.flush_rows));
     const int shift_g = item_shift(quant.gq_max, rows, 63 - h_bits), shift_h = quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits);
     const float scale_g = ldexpf(quant.scale_g, -shift_g), scale_h = ldexpf(quant.scale_h, -shift_h);
-    constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, U = 8;
-    const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
-    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
-    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
     const bool word_lane = bins.gh_lane >= 0 && q == bins.gh_lane;
     const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
-    for (int base = rsub; base < m; base += RPS * U) {
+    for (int base = 0; base < m; base += RPS * U) {
         unsigned pk[U];
         GHPair s[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const unsigned r = s_rows[min(base + u * RPS, m - 1)];
+            const unsigned r = s_rows[min(base + rsub + u * RPS, m - 1)];
             pk[u] = *reinterpret_cast<const unsigned *>(blk + (r * (unsigned)(LPR * 4) + (unsigned)q * 4));
             s[u] = gh[r];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const unsigned v = base + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
+            if (base + u * RPS >= m) break;  // (uniform)
+            const unsigned v = base + rsub + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
             const long long gq = round_to_ll(s[u].g * scale_g), hq = round_to_ll(fmaxf(s[u].h, 0.f) * scale_h);
             const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
             if (BIN16) {

@@ -80,7 +80,7 @@ class Trainer {
     void find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class);
     void partition_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class);
     bool update_with_partition(int level) const;
-    void build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class);
+    void build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class, bool sum_rows = false);
     void build_round_together();
     void log_plan(const TreeBuffers &tb);
     bool reorder_allowed() const;

@@ -564,7 +564,7 @@ void Trainer::alloc_tree_buffers() {
     tb.quant = dalloc<QuantCtl>(S);
     tb.max_hitems = std::max(tb.max_hitems, max_runs);
     tb.hitem_shift = dalloc<int2>(S * (size_t)tb.max_hitems);
-    tb.root_total = dalloc<long long>(S * 512);
+    tb.root_total = dalloc<long long>(S * 2 * kRootParts);
     // a feature that is stored in every row (checked on the bin matrix itself: a row with a repeated column index
     // would make the stored-value count lie): its bins add up to the root's sums
     tb.complete_feature = -1;
@@ -1010,13 +1010,15 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     }
     mark(level == 0 ? PH_GRADIENT : PH_PARTITION, level);  // closes what ran before this level's histogram
     const bool derive = small() && level > 0;  // the level before has built its histograms
-    if (!derive && !(run() > 0 && level > 0)) build_level_hist(tb, level, gh, n_class);
+    // the root's sums ride in the launches of its histograms and of its split search (all nodes of the level at once)
+    const bool sum_rows = !sparse_ && level == 0 && hist_cap_level_ != 0 && tb.complete_feature < 0;
+    if (!derive && !(run() > 0 && level > 0)) build_level_hist(tb, level, gh, n_class, sum_rows);
     mark(PH_HIST, level);
     if (!sparse_pass_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
-        const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0 && (level > 0 || tb.complete_feature >= 0);
+        const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0;
         if (!sparse_ && !derive && !fused) launch_hist_merge(stream_, tb, level, n_class);
-        if (level == 0 && !fused) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
+        if (level == 0 && !fused && !(wide_eval_ && sum_rows)) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         mark(PH_MERGE, level);
         // inside boost() nobody looks at the last level's derived histograms (the stage-wise API keeps them); the
         // last level that fits a capped arena keeps them for the batches of the next one
@@ -1025,7 +1027,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
                               !(in_boost_ && level == param_.depth - 1), run());
         else if (wide_eval_)
             launch_eval_split_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
-                                   !(in_boost_ && level == param_.depth - 1), derive);
+                                   !(in_boost_ && level == param_.depth - 1), derive, sum_rows);
         else
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                               !(in_boost_ && level == param_.depth - 1), derive);
@@ -1045,7 +1047,7 @@ bool Trainer::update_with_partition(int level) const {
            (hist_cap_level_ < 0 || level < hist_cap_level_);
 }
 
-void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class) {
+void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class, bool sum_rows) {
     if (sparse_pass_) {
         // histogram and split search of the level in one pass; stage-wise driving also gets the per-node histograms
         launch_sparse_level(stream_, tb, csr_, sp_, gh, level, param_.min_child_weight, param_.lambda,
@@ -1058,7 +1060,7 @@ void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *g
         if (level == 0) gh_records_fresh_ = gh_words_fresh_ && n_class == 1 && gh == d_gh_ && tb.lvl_x0 == 0;
         b.gh_fresh = gh_records_fresh_ && n_class == 1 && gh == d_gh_;
         b.gh_objective = objective_;
-        launch_hist_dense(stream_, tb, b, gh, level, n_class);
+        launch_hist_dense(stream_, tb, b, gh, level, n_class, sum_rows);
     }
 }
 

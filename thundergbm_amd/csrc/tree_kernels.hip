@@ -360,6 +360,106 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
     }
 }
 
+// ------------------------------------------------------------------------------ exact root sums
+// k_tree_init sets the root's sums from a float reduction over the rows, whose last bits depend on the physical
+// order of the rows; every later quantity of a tree (child sums, weights, gains, predictions, the next gradients)
+// derives from it. These kernels replace it by the exact fixed-point total - the same integers in any order - so
+// that a tree does not depend on the row order at all.
+__device__ __forceinline__ GHPair root_sums(const TreeBuffers &tb, long long G, long long H) {
+    return {(float)((double)G * (double)tb.quant->inv_g), (float)((double)H * (double)tb.quant->inv_h)};
+}
+__device__ __forceinline__ void set_root_sums(const TreeBuffers &tb, GHPair s, float lambda) {
+    TreeNode &root = tb.nodes[0];
+    root.sum_gh_pair = s;
+    root.base_weight = -s.g / (s.h + lambda);
+}
+
+// From the root histogram: the bins of a feature that is stored in every row add up to the root. One workgroup.
+__global__ __launch_bounds__(kBlock) void k_root_sum_bins(TreeBuffers tb_all, float lambda) {
+    __shared__ long long s_g[kWaves], s_h[kWaves];
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const longlong2 *__restrict__ h = tb.hist(0);
+    const int b0 = tb.cut_row_ptr[tb.complete_feature], b1 = tb.cut_row_ptr[tb.complete_feature + 1];
+    long long g = 0, hh = 0;
+    for (int b = b0 + threadIdx.x; b < b1; b += kBlock) {
+        const longlong2 v = h[b];
+        g += v.x;
+        hh += v.y;
+    }
+    g = wave_sum_ll(g);
+    hh = wave_sum_ll(hh);
+    if (lane_id() == 0) {
+        s_g[wave_id()] = g;
+        s_h[wave_id()] = hh;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kWaves; ++i) {
+            g += s_g[i];
+            hh += s_h[i];
+        }
+        set_root_sums(tb, root_sums(tb, g, hh), lambda);
+    }
+}
+
+// From the gradients (no feature is stored in every row): every row's pair rounded at the tree's scales, a pair of 64-bit sums
+// per part of the rows into root_total[2 part], [2 part + 1], which whoever needs the root's sums adds up: in the dense layout
+// by the root level's histogram launch and by every workgroup of its split search (two launches of 4 to 9 us a tree less:
+// 500 k x 54 with 8 classes 0.515 -> TODO ms a round). (A ticket that lets the last workgroup finish the job needs a device-scope
+// fence, which writes a whole L2 back on this chip: 288 us per round of 8 class trees.)
+template <int BLK>
+__device__ __forceinline__ void root_sum_rows(const TreeBuffers &tb, const GHPair *__restrict__ gh, int begin, int end, int part) {
+    __shared__ long long s_g[BLK / 64], s_h[BLK / 64];
+    const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
+    long long g = 0, hh = 0;
+    for (int i = begin + (int)threadIdx.x; i < end; i += BLK) {
+        const GHPair v = gh[i];
+        g += __float2ll_rn(v.g * scale_g);
+        hh += __float2ll_rn(fmaxf(v.h, 0.f) * scale_h);
+    }
+    g = wave_sum_ll(g);
+    hh = wave_sum_ll(hh);
+    if (lane_id() == 0) {
+        s_g[wave_id()] = g;
+        s_h[wave_id()] = hh;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int i = 1; i < BLK / 64; ++i) {
+        g += s_g[i];
+        hh += s_h[i];
+    }
+    tb.root_total[2 * part] = g;
+    tb.root_total[2 * part + 1] = hh;
+}
+
+// By one wavefront, the same in all of its lanes.
+__device__ __forceinline__ GHPair root_sums_of_rows(const TreeBuffers &tb, int parts) {
+    const longlong2 *__restrict__ from = reinterpret_cast<const longlong2 *>(tb.root_total);
+    longlong2 v[kRootParts / 64];
+#pragma unroll
+    for (int k = 0; k < kRootParts / 64; ++k) v[k] = from[min(k * 64 + lane_id(), parts - 1)];
+    long long g = 0, h = 0;
+#pragma unroll
+    for (int k = 0; k < kRootParts / 64; ++k) {
+        g += k * 64 + lane_id() < parts ? v[k].x : 0;
+        h += k * 64 + lane_id() < parts ? v[k].y : 0;
+    }
+    return root_sums(tb, wave_sum_ll(g), wave_sum_ll(h));
+}
+
+__global__ __launch_bounds__(kBlock) void k_root_sum_rows(TreeBuffers tb_all, const GHPair *__restrict__ gh) {
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int per = (tb.n + (int)gridDim.x - 1) / (int)gridDim.x, begin = min(tb.n, (int)blockIdx.x * per);
+    root_sum_rows<kBlock>(tb, gh + (size_t)blockIdx.z * tb.n, begin, min(tb.n, begin + per), blockIdx.x);
+}
+
+__global__ __launch_bounds__(64) void k_root_sum_final(TreeBuffers tb_all, int parts, float lambda) {
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const GHPair s = root_sums_of_rows(tb, parts);
+    if (threadIdx.x == 0) set_root_sums(tb, s, lambda);
+}
+
 // ------------------------------------------------------------------------- dense histogram
 // One workgroup = one work item (a run of rows of one node) x one feature block. The block's
 // histogram lives in LDS as one 64-bit integer per bin holding the fixed-point gradient sum in the
@@ -379,7 +479,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
 // root launch (DIRECT) reads the words from their own array and puts them there, storing every record back.
 template <int LPR, bool DIRECT, int BLK, int SLOTS, bool BIN16, bool GHW = false>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(SLOTS <= 8 ? 8 : 4)))  // two 1024-thread groups per CU
-void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level, int n_pairs) {
+void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level, int n_pairs, bool sum_rows) {
     extern __shared__ unsigned long long lds[];
     __shared__ int s_shift[2];  // the item's scale shifts (gradient, hessian)
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
@@ -557,6 +657,8 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
             if (!GHW || DIRECT) s[u] = s_next[u];
         }
     }
+    if constexpr (DIRECT)
+        if (sum_rows && fb == 0) root_sum_rows<BLK>(tb, gh, begin, end, item);
     __syncthreads();
     if (hchunk <= flush_rows) {
         // an item this short was never drained: its packed LDS words are the complete sums and go out as
@@ -643,103 +745,6 @@ __global__ __launch_bounds__(kBlock) void k_hist_merge(TreeBuffers tb_all, int l
         const longlong2 par = prev_q[(size_t)p * n_bins + j];
         cur_q[(size_t)(sib - off) * n_bins + j] = make_longlong2(par.x - sg, par.y - sh);
     }
-}
-
-// ------------------------------------------------------------------------------ exact root sums
-// k_tree_init sets the root's sums from a float reduction over the rows, whose last bits depend on the physical
-// order of the rows; every later quantity of a tree (child sums, weights, gains, predictions, the next gradients)
-// derives from it. These kernels replace it by the exact fixed-point total - the same integers in any order - so
-// that a tree does not depend on the row order at all.
-__device__ __forceinline__ GHPair root_sums(const TreeBuffers &tb, long long G, long long H) {
-    return {(float)((double)G * (double)tb.quant->inv_g), (float)((double)H * (double)tb.quant->inv_h)};
-}
-__device__ __forceinline__ void set_root_sums(const TreeBuffers &tb, GHPair s, float lambda) {
-    TreeNode &root = tb.nodes[0];
-    root.sum_gh_pair = s;
-    root.base_weight = -s.g / (s.h + lambda);
-}
-
-// From the root histogram: the bins of a feature that is stored in every row add up to the root. One workgroup.
-__global__ __launch_bounds__(kBlock) void k_root_sum_bins(TreeBuffers tb_all, float lambda) {
-    __shared__ long long s_g[kWaves], s_h[kWaves];
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    const longlong2 *__restrict__ h = tb.hist(0);
-    const int b0 = tb.cut_row_ptr[tb.complete_feature], b1 = tb.cut_row_ptr[tb.complete_feature + 1];
-    long long g = 0, hh = 0;
-    for (int b = b0 + threadIdx.x; b < b1; b += kBlock) {
-        const longlong2 v = h[b];
-        g += v.x;
-        hh += v.y;
-    }
-    g = wave_sum_ll(g);
-    hh = wave_sum_ll(hh);
-    if (lane_id() == 0) {
-        s_g[wave_id()] = g;
-        s_h[wave_id()] = hh;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < kWaves; ++i) {
-            g += s_g[i];
-            hh += s_h[i];
-        }
-        set_root_sums(tb, root_sums(tb, g, hh), lambda);
-    }
-}
-
-// From the gradients (no feature is stored in every row): every row's pair rounded at the tree's scales, one pair of
-// 64-bit block sums per workgroup into root_total[2 i], [2 i + 1]; k_root_sum_final (one workgroup) adds them up.
-// (A ticket that lets the last workgroup finish the job needs a device-scope fence, which writes a whole L2 back on
-// this chip: 288 us per round of 8 class trees against 2 x 5 us for two launches.)
-constexpr int kRootSumBlocks = 256;
-__global__ __launch_bounds__(kBlock) void k_root_sum_rows(TreeBuffers tb_all, const GHPair *__restrict__ gh) {
-    __shared__ long long s_g[kWaves], s_h[kWaves];
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    gh += (size_t)blockIdx.z * tb.n;
-    const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
-    long long g = 0, hh = 0;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < tb.n; i += gridDim.x * kBlock) {
-        const GHPair v = gh[i];
-        g += __float2ll_rn(v.g * scale_g);
-        hh += __float2ll_rn(fmaxf(v.h, 0.f) * scale_h);
-    }
-    g = wave_sum_ll(g);
-    hh = wave_sum_ll(hh);
-    if (lane_id() == 0) {
-        s_g[wave_id()] = g;
-        s_h[wave_id()] = hh;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int i = 1; i < kWaves; ++i) {
-        g += s_g[i];
-        hh += s_h[i];
-    }
-    tb.root_total[2 * blockIdx.x] = g;
-    tb.root_total[2 * blockIdx.x + 1] = hh;
-}
-
-__global__ __launch_bounds__(kBlock) void k_root_sum_final(TreeBuffers tb_all, int n_blocks, float lambda) {
-    __shared__ long long s_g[kWaves], s_h[kWaves];
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    long long g = 0, hh = 0;
-    for (int i = threadIdx.x; i < n_blocks; i += kBlock) {
-        g += tb.root_total[2 * i];
-        hh += tb.root_total[2 * i + 1];
-    }
-    g = wave_sum_ll(g);
-    hh = wave_sum_ll(hh);
-    if (lane_id() == 0) {
-        s_g[wave_id()] = g;
-        s_h[wave_id()] = hh;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int i = 1; i < kWaves; ++i) {
-        g += s_g[i];
-        hh += s_h[i];
-    }
-    set_root_sums(tb, root_sums(tb, g, hh), lambda);
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_bytes(const uint8_t *__restrict__ v, size_t n, uint8_t value,
@@ -1018,6 +1023,10 @@ struct PackScan {
     }
 };
 
+// Where the split search of level 0 takes the node's sums from: a feature stored in every row, whose bins add up to them, or
+// what the histogram launch has added up of the rows.
+enum RootSums { kNoRoot = 0, kRootOfBins, kRootOfRows };
+
 // The search of one pack of one node, by one wavefront: s_v holds the pack's bins, s_miss takes its features' missing sums
 // (kEvalPackBins entries each).
 __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMeta &pm, const longlong2 *s_v, GHPair *s_miss,
@@ -1128,9 +1137,8 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
 // SUB (sparse layout, whose histograms are not merged from work-item partials): the node of a pair that
 // was not built from rows is derived here as parent - built while it is scanned, and stored for the next
 // level, instead of by a separate pass over the (very long) histograms.
-// ROOT (level 0, a feature stored in every row): the node's sums are that feature's bins added up, by every wavefront
-// for itself.
-template <bool SUB, bool ROOT = false>
+// ROOT, the node's sums by every wavefront for itself (RootSums).
+template <bool SUB, int ROOT = kNoRoot>
 __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int level, float mcw, float lambda,
                                                       bool store_sibling) {
 #pragma clang fp contract(off)
@@ -1153,7 +1161,11 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
     GHPair S = nd.sum_gh_pair;
     longlong2 *h = hist_q + (size_t)x_in * tb.n_bins;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
-    if constexpr (ROOT) {
+    if constexpr (ROOT == kRootOfRows) {
+        S = root_sums_of_rows(tb, tb.ctl[0].n_hitems);
+        if (pack == 0 && lane == 0) set_root_sums(tb, S, lambda);
+    }
+    if constexpr (ROOT == kRootOfBins) {
         long long g = 0, hh = 0;
         const int b0 = tb.cut_row_ptr[tb.complete_feature], b1 = tb.cut_row_ptr[tb.complete_feature + 1];
         for (int b = b0 + lane; b < b1; b += 64) {
@@ -1201,9 +1213,9 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
 // k_hist_merge and k_eval_split of a level in one launch: a workgroup owns a pack of a sibling pair. Its wavefronts share
 // out the pair's work items, the sums meet in LDS, parent - built gives the sibling, one wavefront searches the built node
 // and one its sibling. The histograms are stored for the next level only (not at a tree's last one, which holds half of a
-// tree's nodes) and not read back. NW follows from the items per pair (launch_merge_eval). ROOT: level 0, with a feature
-// stored in every row, whose bins every workgroup adds up as well: they are the node's sums.
-template <int NW, bool ROOT>
+// tree's nodes) and not read back. NW follows from the items per pair (launch_merge_eval). ROOT: level 0, where every
+// workgroup adds up the node's sums as well (RootSums).
+template <int NW, int ROOT>
 __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int level, float mcw, float lambda, bool store) {
     __shared__ longlong2 s_sum[NW][kEvalPackBins];
     __shared__ GHPair s_miss[2][kEvalPackBins];
@@ -1274,7 +1286,7 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
             }
         }
     };
-    if constexpr (ROOT) {
+    if constexpr (ROOT == kRootOfBins) {
         const int b0 = tb.cut_row_ptr[tb.complete_feature], kf = tb.cut_row_ptr[tb.complete_feature + 1] - b0;
         long long g[4], h[4], G = 0, H = 0;
         add_items(b0, kf, g, h);
@@ -1323,13 +1335,17 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
     __syncthreads();
     if (w >= (ROOT ? 1 : 2)) return;
     if constexpr (ROOT) {
-        long long G = 0, H = 0;
+        if constexpr (ROOT == kRootOfBins) {
+            long long G = 0, H = 0;
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            G += s_root[i].x;
-            H += s_root[i].y;
+            for (int i = 0; i < NW; ++i) {
+                G += s_root[i].x;
+                H += s_root[i].y;
+            }
+            S = root_sums(tb, G, H);
+        } else {
+            S = root_sums_of_rows(tb, tb.ctl[0].n_hitems);
         }
-        S = root_sums(tb, G, H);
         if (pack == 0 && lane == 0) set_root_sums(tb, S, lambda);
     }
     search_pack(tb, pm, s_sum[w], s_miss[w], (w == 0 ? built : sibling) - off, pack, true, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
@@ -1348,7 +1364,7 @@ __device__ __forceinline__ longlong2 wide_bin(const longlong2 *h, const longlong
 }
 
 __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, int level, float mcw, float lambda,
-                                                           bool store_sibling, bool derive) {
+                                                           bool store_sibling, bool derive, bool root_of_rows) {
 #pragma clang fp contract(off)
     __shared__ long long s_g[kWaves], s_h[kWaves];
     __shared__ float s_abs[kWaves];
@@ -1359,6 +1375,11 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
     const int x = (1 << level) - 1 + x_in;
     const TreeNode nd = tb.nodes[x];
     if (!nd.is_valid) return;  // (nobody reads the candidates of an invalid node)
+    GHPair S = nd.sum_gh_pair;
+    if (root_of_rows) {
+        S = root_sums_of_rows(tb, tb.ctl[0].n_hitems);
+        if (f == 0 && threadIdx.x == 0) set_root_sums(tb, S, lambda);
+    }
     const int cb = tb.cut_row_ptr[f], ce = tb.cut_row_ptr[f + 1];
     SplitCand *out = &tb.cand[(size_t)x_in * tb.n_packs + f];
     if (cb == ce) {
@@ -1375,7 +1396,6 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
             h_built = tb.hist(level) + (size_t)(built - ((1 << level) - 1)) * tb.n_bins;
         }
     }
-    const GHPair S = nd.sum_gh_pair;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
     const bool ign = tb.ignored != nullptr && tb.ignored[f] != 0;
     // ---- the feature's total (missing = node sum - total), the derived sibling stored on the way
@@ -2433,7 +2453,7 @@ void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_cla
 
 template <int LPR, int SLOTS, bool BIN16>
 static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh,
-                              int level, int n_class) {
+                              int level, int n_class, bool sum_rows) {
     const int n_pairs = tb.n_hpairs(level);
     // (an upper bound on the work items: whole chunks of the rows that can be built - half of them below the root, unless
     // single nodes are built - and one partly filled item per built node; see plan_hist_item)
@@ -2454,49 +2474,49 @@ static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseB
                               reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true>)});
             }
             if (level == 0)
-                k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs);
+                k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, sum_rows);
             else
-                k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs);
+                k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, false);
             return;
         }
     }
     if (level == 0)
-        k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs);
+        k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, sum_rows);
     else
-        k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs);
+        k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, false);
 }
 
 template <int LPR>
 static void hist_dense_dispatch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh,
-                                int level, int n_class) {
+                                int level, int n_class, bool sum_rows) {
     const int slots = (tb.max_block_bins + kHistBlock - 1) / kHistBlock;  // bins drained per thread
     if (bins.bin_bytes == 2) {  // (fewer variants: the blocks of 16-bit bins are sized to fill the LDS)
-        if (slots <= 4) hist_dense_launch<LPR, 4, true>(s, tb, bins, gh, level, n_class);
-        else if (slots <= 8) hist_dense_launch<LPR, 8, true>(s, tb, bins, gh, level, n_class);
-        else if (slots <= 20) hist_dense_launch<LPR, 20, true>(s, tb, bins, gh, level, n_class);
+        if (slots <= 4) hist_dense_launch<LPR, 4, true>(s, tb, bins, gh, level, n_class, sum_rows);
+        else if (slots <= 8) hist_dense_launch<LPR, 8, true>(s, tb, bins, gh, level, n_class, sum_rows);
+        else if (slots <= 20) hist_dense_launch<LPR, 20, true>(s, tb, bins, gh, level, n_class, sum_rows);
         else fatal("feature block with %d bins does not fit the histogram kernel", tb.max_block_bins);
         return;
     }
-    if (slots <= 1) hist_dense_launch<LPR, 1, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 2) hist_dense_launch<LPR, 2, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 3) hist_dense_launch<LPR, 3, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 4) hist_dense_launch<LPR, 4, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 6) hist_dense_launch<LPR, 6, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 7) hist_dense_launch<LPR, 7, false>(s, tb, bins, gh, level, n_class);  // fewer accumulator registers
-    else if (slots <= 8) hist_dense_launch<LPR, 8, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 16) hist_dense_launch<LPR, 16, false>(s, tb, bins, gh, level, n_class);
-    else if (slots <= 20) hist_dense_launch<LPR, 20, false>(s, tb, bins, gh, level, n_class);
+    if (slots <= 1) hist_dense_launch<LPR, 1, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 2) hist_dense_launch<LPR, 2, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 3) hist_dense_launch<LPR, 3, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 4) hist_dense_launch<LPR, 4, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 6) hist_dense_launch<LPR, 6, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 7) hist_dense_launch<LPR, 7, false>(s, tb, bins, gh, level, n_class, sum_rows);  // fewer accumulator registers
+    else if (slots <= 8) hist_dense_launch<LPR, 8, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 16) hist_dense_launch<LPR, 16, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    else if (slots <= 20) hist_dense_launch<LPR, 20, false>(s, tb, bins, gh, level, n_class, sum_rows);
     else fatal("feature block with %d bins does not fit the histogram kernel", tb.max_block_bins);
 }
 
 void launch_hist_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                       int n_class) {
+                       int n_class, bool sum_rows) {
     switch (bins.W * bins.bin_bytes) {  // bytes per row of a block = 4 x lanes per row
-        case 4: hist_dense_dispatch<1>(s, tb, bins, gh, level, n_class); break;
-        case 8: hist_dense_dispatch<2>(s, tb, bins, gh, level, n_class); break;
-        case 16: hist_dense_dispatch<4>(s, tb, bins, gh, level, n_class); break;
-        case 32: hist_dense_dispatch<8>(s, tb, bins, gh, level, n_class); break;
-        case 64: hist_dense_dispatch<16>(s, tb, bins, gh, level, n_class); break;
+        case 4: hist_dense_dispatch<1>(s, tb, bins, gh, level, n_class, sum_rows); break;
+        case 8: hist_dense_dispatch<2>(s, tb, bins, gh, level, n_class, sum_rows); break;
+        case 16: hist_dense_dispatch<4>(s, tb, bins, gh, level, n_class, sum_rows); break;
+        case 32: hist_dense_dispatch<8>(s, tb, bins, gh, level, n_class, sum_rows); break;
+        case 64: hist_dense_dispatch<16>(s, tb, bins, gh, level, n_class, sum_rows); break;
         default: fatal("unsupported dense block width %d x %d bytes", bins.W, bins.bin_bytes);
     }
 }
@@ -2521,9 +2541,9 @@ void launch_root_sum(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_clas
     if (tb.complete_feature >= 0) {
         k_root_sum_bins<<<dim3(1, 1, n_class), kBlock, 0, s>>>(tb, lambda);
     } else {
-        const int blocks = std::max(1, std::min(kRootSumBlocks, (tb.n + kBlock - 1) / kBlock));
+        const int blocks = std::max(1, std::min(256, (tb.n + kBlock - 1) / kBlock));
         k_root_sum_rows<<<dim3(blocks, 1, n_class), kBlock, 0, s>>>(tb, gh_class);
-        k_root_sum_final<<<dim3(1, 1, n_class), kBlock, 0, s>>>(tb, blocks, lambda);
+        k_root_sum_final<<<dim3(1, 1, n_class), 64, 0, s>>>(tb, blocks, lambda);
     }
 }
 
@@ -2591,28 +2611,33 @@ void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mc
                                            : std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
     if (level == 0) {
         // One workgroup per pack: with hundreds of items two launches that spread them over the chip are faster (512 items of
-        // 28 packs: 12 + 9 instead of 43 us; 23 items of 700 packs: 18 instead of 16 + 15).
+        // 28 packs: 12 + 9 instead of 43 us; 245: 8 + 8 and 24; 23 items of 700 packs: 18 instead of 16 + 15).
+        if (items > 64) launch_hist_merge(s, tb, level, n_class);
+        const dim3 packs((tb.n_packs + kWaves - 1) / kWaves, 1, n_class);
+        const bool bins = tb.complete_feature >= 0;
         if (items > 64) {
-            launch_hist_merge(s, tb, level, n_class);
-            k_eval_split<false, true><<<dim3((tb.n_packs + kWaves - 1) / kWaves, 1, n_class), kBlock, 0, s>>>(tb, level, mcw, lambda, true);
+            if (bins) k_eval_split<false, kRootOfBins><<<packs, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
+            else k_eval_split<false, kRootOfRows><<<packs, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
         } else if (items > 8) {
-            k_merge_eval<16, true><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+            if (bins) k_merge_eval<16, kRootOfBins><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+            else k_merge_eval<16, kRootOfRows><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
         } else {
-            k_merge_eval<4, true><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+            if (bins) k_merge_eval<4, kRootOfBins><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+            else k_merge_eval<4, kRootOfRows><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
         }
         return;
     }
     const int per_pair = items / n_pairs;
-    if (per_pair > 32) k_merge_eval<16, false><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
-    else if (per_pair > 8) k_merge_eval<8, false><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
-    else if (per_pair > 2) k_merge_eval<4, false><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
-    else k_merge_eval<2, false><<<grid, 128, 0, s>>>(tb, level, mcw, lambda, store);
+    if (per_pair > 32) k_merge_eval<16, kNoRoot><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+    else if (per_pair > 8) k_merge_eval<8, kNoRoot><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
+    else if (per_pair > 2) k_merge_eval<4, kNoRoot><<<grid, 256, 0, s>>>(tb, level, mcw, lambda, store);
+    else k_merge_eval<2, kNoRoot><<<grid, 128, 0, s>>>(tb, level, mcw, lambda, store);
 }
 
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class,
-                            bool store_sibling, bool derive) {
+                            bool store_sibling, bool derive, bool root_of_rows) {
     dim3 grid(tb.F, tb.nodes_served(level), n_class);
-    k_eval_split_wide<<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling, derive || tb.sparse);
+    k_eval_split_wide<<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling, derive || tb.sparse, root_of_rows);
 }
 
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class) {
