@@ -491,12 +491,12 @@ constexpr int kSmallSteps = kSmallRows / kSmallBlock;
 static_assert(kSmallRows / 2 <= kHistFlushRows, "the built child's packed sums are never drained");
 static_assert(kSmallRows <= 1 << 16 && kSmallWaves == 16 && kSmallSteps % 4 == 0, "16-bit row ids, the counts of four steps per wavefront");
 
-template <int LPR, bool BIN16>
+template <int LPR, bool BIN16, int STEPS>
 __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
                                                             int level, float rt_eps, float lambda) {
     extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
     __shared__ PickShared s_pick;
-    __shared__ int s_left[kSmallSteps * kSmallWaves];  // rows that go left, per step and wavefront
+    __shared__ int s_left[STEPS * kSmallWaves];  // rows that go left, per step and wavefront
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
     unsigned short *s_rows = reinterpret_cast<unsigned short *>(lds + tb.max_block_bins);
@@ -514,9 +514,9 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
     const int len = sg.y - sg.x, steps = (len + kSmallBlock - 1) / kSmallBlock;
     const int *__restrict__ ridx = tb.list(level);
-    int row[kSmallSteps];
+    int row[STEPS];
 #pragma unroll
-    for (int k = 0; k < kSmallSteps; ++k) {
+    for (int k = 0; k < STEPS; ++k) {
         row[k] = 0;
         if (k < steps) {
             const int pos = min(sg.x + k * kSmallBlock + (int)threadIdx.x, sg.y - 1);
@@ -546,13 +546,13 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
         span = tb.cut_row_ptr[f + 1] - tb.cut_row_ptr[f];
     }
     const uint8_t *column = bins.col + (size_t)c * bins.col_stride * (BIN16 ? 2 : 1);
-    int b[kSmallSteps];
+    int b[STEPS];
 #pragma unroll
-    for (int k = 0; k < kSmallSteps; ++k)
+    for (int k = 0; k < STEPS; ++k)
         if (k < steps) b[k] = BIN16 ? (int)reinterpret_cast<const uint16_t *>(column)[row[k]] : (int)column[row[k]];
-    unsigned long long left_mask[kSmallSteps];  // (wave-uniform)
+    unsigned long long left_mask[STEPS];  // (wave-uniform)
 #pragma unroll
-    for (int k = 0; k < kSmallSteps; ++k) {
+    for (int k = 0; k < STEPS; ++k) {
         left_mask[k] = 0;
         if (k < steps) {
             const int t = b[k] - lo;
@@ -563,12 +563,12 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     }
     __syncthreads();
     // lefts before every (step, wavefront), and of all: by every wavefront for itself, four steps at a time
-    int upto[kSmallSteps / 4], nleft = 0;
+    int upto[(STEPS + 3) / 4], nleft = 0;
 #pragma unroll
-    for (int k = 0; k < kSmallSteps / 4; ++k) {
+    for (int k = 0; k < (STEPS + 3) / 4; ++k) {
         upto[k] = 0;
         if (k * 4 < steps) {
-            const int own = s_left[k * 64 + lane];
+            const int own = k * 64 + lane < STEPS * kSmallWaves ? s_left[k * 64 + lane] : 0;
             const int inc = wave_scan_i(own);
             upto[k] = nleft + inc - own;
             nleft += read_lane(inc, 63);
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     const int m = build_left ? nleft : nright;
     int *__restrict__ ridx_next = tb.list(level + 1);
 #pragma unroll
-    for (int k = 0; k < kSmallSteps; ++k) {
+    for (int k = 0; k < STEPS; ++k) {
         const int i = k * kSmallBlock + (int)threadIdx.x;
         if (k < steps && i < len) {
             const int lefts = read_lane(upto[k / 4], k % 4 * kSmallWaves + w) + lanes_below(left_mask[k]);
@@ -970,22 +970,33 @@ bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins) {
            small_lds(tb) + 4096 <= kLdsBytes;
 }
 
-template <int LPR, bool BIN16>
+template <int LPR, bool BIN16, int STEPS>
 static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
                                float rt_eps, float lambda, int n_class) {
     const size_t lds = small_lds(tb);
     static LdsOptIn opt_in;
     if (lds > 48 * 1024)  // (with the kernel's own tables more than the default window)
-        opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16>)});
-    k_small_level<LPR, BIN16><<<dim3(bins.n_blocks, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda);
+        opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16, STEPS>)});
+    k_small_level<LPR, BIN16, STEPS><<<dim3(bins.n_blocks, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda);
+}
+
+// (the code of steps that no node of the data can have is not only skipped but left out, see k_small_level)
+template <int LPR, bool BIN16>
+static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
+                              float rt_eps, float lambda, int n_class) {
+    const int steps = (tb.n + kSmallBlock - 1) / kSmallBlock;
+    if (steps <= 2) small_level_launch<LPR, BIN16, 2>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
+    else if (steps <= 4) small_level_launch<LPR, BIN16, 4>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
+    else if (steps <= 8) small_level_launch<LPR, BIN16, 8>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
+    else small_level_launch<LPR, BIN16, kSmallSteps>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
 }
 
 void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
                         float lambda, int n_class) {
     if (level == tb.depth - 1) return;
 #define TGBM_SMALL_LEVEL(LPR)                                                                               \
-    if (bins.bin_bytes == 2) small_level_launch<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, n_class); \
-    else small_level_launch<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, n_class);                    \
+    if (bins.bin_bytes == 2) small_level_steps<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, n_class); \
+    else small_level_steps<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, n_class);                    \
     break
     switch (bins.W * bins.bin_bytes) {  // bytes per row of a block
         case 4: TGBM_SMALL_LEVEL(1);
