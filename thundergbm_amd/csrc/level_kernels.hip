@@ -705,7 +705,7 @@ __device__ __forceinline__ NodeRun locate_run(const TreeBuffers &tb, int level, 
 // stores the lists. Bound by its chain of dependent steps - segments, decisions with rows and counts, lists, records - and by
 // the LDS, which adds about 8 pairs a nanosecond and CU to random bins: 1000 rows x 28 in 3.5 us.
 // 500 k x 28: 9.5 us with 1 item, where scatter, gap and histogram (which looks for its pair and fetches the row ids again) took
-// 13.3; a tree of depth 8 0.281 -> 0.266 ms.
+// 13.3; a tree of depth 8 0.281 -> 0.266 ms (0.263 and 0.261 without and with the write-through; 900 k x 28 0.296 and 0.290).
 // Measured and not kept: every row's addend rounded once, by a thread of its own, and passed on through LDS (the LDS is what it
 // waits for: 4.6 -> 6.1 us in that part); the decisions taken here as well, the runs of a node telling each other their counts
 // through agent-scope atomics (a launch less, but 245 workgroups that look at 245 words each: a tree 0.32 instead of 0.27 ms).
@@ -861,7 +861,8 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     }
     __syncthreads();
     unsigned long long *out = reinterpret_cast<unsigned long long *>(tb.partial) + (size_t)item * tb.n_bins + bin0;
-    for (int i = threadIdx.x; i < nb; i += kHistBlock) out[i] = lds[i];
+    // (written through: what the launch leaves in the L2s is written back when it ends, and everything waits for that)
+    for (int i = threadIdx.x; i < nb; i += kHistBlock) __hip_atomic_store(&out[i], lds[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace
