@@ -1,4 +1,4 @@
-"""Small data: the levels in one launch each (k_small_level, k_small_end) against the launches of larger data (TGBM_SMALL=0), byte
+"""Small data: the levels in one launch each (k_small_level, k_map_end) against the launches of larger data (TGBM_SMALL=0), byte
 for byte, at the edges of their range."""
 import ctypes
 import os

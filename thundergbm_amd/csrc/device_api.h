@@ -471,8 +471,8 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
                             float rt_eps, float lambda, int n_class = 1);
 // Dense layout, moderately many rows: launch_partition_dense and the histograms of the next level's built nodes in two
 // launches instead of three (k_split_hist). split_hist_run: rows of a level's node that a workgroup of the second one serves,
-// 0: such data goes through launch_partition_dense and launch_hist_dense. Inside boost() only (level tb.depth - 1 is not
-// partitioned; the level's candidates are fresh).
+// 0: such data goes through launch_partition_dense and launch_hist_dense. Inside boost() only: the level's candidates are fresh,
+// and every row leaves the node where it ends in tb.nid (launch_map_end), at level tb.depth - 1 the last of them.
 int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class);
 void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
                            float rt_eps, float lambda, int n_class = 1);
@@ -481,9 +481,10 @@ void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins
 bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins);
 void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
                         float lambda, int n_class = 1);
-// The end of a tree whose rows' nodes are in tb.nid: prunes the tree into `model` (n_class trees back to back; tb.nodes
+// The end of a tree whose rows' nodes are in tb.nid (lookup_level >= 0: split nodes of that level still hold the rows of their
+// children): prunes the tree into `model` (n_class trees back to back; tb.nodes
 // stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics.
-void launch_small_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, TreeNode *model, float gamma, float *yp,
+void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int lookup_level, TreeNode *model, float gamma, float *yp,
                       float lr, int n_class = 1, const float *y = nullptr, int objective = 0, int metric_kind = 0,
                       GHPair *gh = nullptr, double *metric_scratch = nullptr, unsigned *gh_words = nullptr);
 // Sparse level pass (tb.nid16 set): split search of a level (candidates into tb.cand, one slot per task / big

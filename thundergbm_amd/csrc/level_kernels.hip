@@ -192,7 +192,9 @@ __device__ __forceinline__ void apply_candidate(const TreeBuffers &tb, int x, in
 // UPDATE: the nodes' candidates are fresh from the split search; else the tree has been updated already.
 // A row goes right if its bin is not below the split bin, or if it has no value of the feature and the default says so
 // (hist_tree_builder_single.cu:986-1011).
-template <bool DIRECT, typename BinT, bool UPDATE, bool PLANNED>
+// MAP: the rows that end here leave their node in tb.nid for k_map_end. 1: those of nodes that do not split. 2 (the last level,
+// whose children get no lists): all rows.
+template <bool DIRECT, typename BinT, bool UPDATE, bool PLANNED, int MAP = 0>
 __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, DenseBins bins, int level, float rt_eps,
                                                        float lambda) {
     __shared__ int lds[kWaves];
@@ -243,7 +245,11 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
         if (UPDATE && item == it.first && threadIdx.x == 0) apply_candidate(tb, x, x_in, node, best.found, best.c, rt_eps, lambda);
     };
     if (!splits) {
-        if (threadIdx.x == 0) tb.pitem_nleft[item] = 0;
+        if (MAP != 2 && threadIdx.x == 0) tb.pitem_nleft[item] = 0;
+        if (MAP != 0)
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                if (pb + k * kBlock + (int)threadIdx.x < pe) tb.nid[row[k]] = x;
         update();
         return;
     }
@@ -264,8 +270,16 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
     for (int k = 0; k < R; ++k) {
         const int t = b[k] - lo;
         const bool right = ((unsigned)t >= (unsigned)span) ? dr : (t >= sbid);
+        if (MAP == 2) {
+            if (pb + k * kBlock + (int)threadIdx.x < pe) tb.nid[row[k]] = 2 * x + (right ? 2 : 1);
+            continue;
+        }
         rights |= (right ? 1u : 0u) << k;
         if (pb + k * kBlock + (int)threadIdx.x < pe) nleft += right ? 0 : 1;
+    }
+    if (MAP == 2) {
+        update();
+        return;
     }
     // the decisions of a thread's eight rows as one byte (k_split_scatter gives the same rows to the same thread)
     static_assert(R <= 8, "a byte per thread holds the decisions of its rows");
@@ -483,7 +497,7 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 // children's lists down and adds up the histogram of the child with fewer rows, whose list it has in LDS, right at the
 // tree's scales; the split search derives the sibling (k_eval_split<true>). Every block of a node repeats the split, the
 // first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
-// (k_small_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
+// (k_map_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
 // A level of 10 k x 8: 28 -> 14 us with its split search.
 // The sums are those of k_hist_dense, whose work items count at a scale that hangs on the node's rows only.
 constexpr int kSmallWaves = kSmallBlock / 64;
@@ -867,26 +881,6 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
 
 }  // namespace
 
-static void split_count_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update, float rt_eps,
-                               float lambda, int n_class, int most) {
-    const dim3 items(most, 1, n_class);
-    const bool planned = tb.planned(level);
-#define TGBM_SPLIT_COUNT(D, T, U, P) k_split_count<D, T, U, P><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
-#define TGBM_SPLIT_COUNT_LEVEL(T, U)                           \
-    if (level == 0) TGBM_SPLIT_COUNT(true, T, U, false);       \
-    else if (planned) TGBM_SPLIT_COUNT(false, T, U, true);     \
-    else TGBM_SPLIT_COUNT(false, T, U, false)
-    if (bins.bin_bytes == 2) {
-        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint16_t, true); }
-        else { TGBM_SPLIT_COUNT_LEVEL(uint16_t, false); }
-    } else {
-        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint8_t, true); }
-        else { TGBM_SPLIT_COUNT_LEVEL(uint8_t, false); }
-    }
-#undef TGBM_SPLIT_COUNT_LEVEL
-#undef TGBM_SPLIT_COUNT
-}
-
 static int most_partition_items(const TreeBuffers &tb, int level) {
     return level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
 }
@@ -894,7 +888,7 @@ static int most_partition_items(const TreeBuffers &tb, int level) {
 static size_t split_hist_lds(const TreeBuffers &tb, int run) { return (size_t)tb.max_block_bins * 8 + (size_t)run * 4; }
 
 int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class) {
-    if (tb.n >= kSplitHistRows || tb.planned(tb.depth - 1)) return 0;
+    if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return 0;
     for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2) {
         const size_t stored = (size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class;
         if (stored <= kSplitHistBytes && split_hist_lds(tb, run) + 4096 <= kLdsBytes) return run;
@@ -922,8 +916,17 @@ static void split_hist_run_launch(hipStream_t s, const TreeBuffers &tb, const De
 
 void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
                            float rt_eps, float lambda, int n_class) {
-    if (level == tb.depth - 1) return;
-    split_count_launch(s, tb, bins, level, true, rt_eps, lambda, n_class, most_partition_items(tb, level));
+    const dim3 items(most_partition_items(tb, level), 1, n_class);
+    const bool last = level == tb.depth - 1;
+#define TGBM_SPLIT_MAP(T)                                                                                                          \
+    if (last && level == 0) k_split_count<true, T, true, false, 2><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);       \
+    else if (last) k_split_count<false, T, true, false, 2><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);               \
+    else if (level == 0) k_split_count<true, T, true, false, 1><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);          \
+    else k_split_count<false, T, true, false, 1><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
+    if (bins.bin_bytes == 2) { TGBM_SPLIT_MAP(uint16_t); }
+    else { TGBM_SPLIT_MAP(uint8_t); }
+#undef TGBM_SPLIT_MAP
+    if (last) return;
     const bool words = bins.gh_lane >= 0 && bins.gh_fresh;
 #define TGBM_SPLIT_HIST(LPR)                                                                                        \
     if (bins.bin_bytes == 2) split_hist_run_launch<LPR, true, false>(s, tb, bins, gh, level, run, n_class);          \
@@ -947,7 +950,20 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
     const int most = most_partition_items(tb, level);
     const dim3 items(most, 1, n_class);
     const bool planned = tb.planned(level);
-    split_count_launch(s, tb, bins, level, update, rt_eps, lambda, n_class, most);
+#define TGBM_SPLIT_COUNT(D, T, U, P) k_split_count<D, T, U, P><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
+#define TGBM_SPLIT_COUNT_LEVEL(T, U)                           \
+    if (level == 0) TGBM_SPLIT_COUNT(true, T, U, false);       \
+    else if (planned) TGBM_SPLIT_COUNT(false, T, U, true);     \
+    else TGBM_SPLIT_COUNT(false, T, U, false)
+    if (bins.bin_bytes == 2) {
+        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint16_t, true); }
+        else { TGBM_SPLIT_COUNT_LEVEL(uint16_t, false); }
+    } else {
+        if (update) { TGBM_SPLIT_COUNT_LEVEL(uint8_t, true); }
+        else { TGBM_SPLIT_COUNT_LEVEL(uint8_t, false); }
+    }
+#undef TGBM_SPLIT_COUNT_LEVEL
+#undef TGBM_SPLIT_COUNT
     const bool groups = tb.n >= kPartGroupRows;
     if (groups) k_split_groups<<<dim3((most + kPartGroup * kWaves - 1) / (kPartGroup * kWaves), 1, n_class), kBlock, 0, s>>>(tb, most);
 #define TGBM_SPLIT_SCATTER(G)                                                      \

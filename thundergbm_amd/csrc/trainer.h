@@ -176,6 +176,7 @@ class Trainer {
     bool small() const { return in_boost_ && small_ok_; }
     int run_rows_ = 0;               // inside boost() the levels go through launch_partition_hist, runs of so many rows
     int run() const { return in_boost_ && !small_ok_ ? run_rows_ : 0; }
+    bool maps_rows() const { return small() || run() > 0; }  // a tree's rows end in tb.nid: launch_map_end
     int lookup_level_ = -1;          // level whose split nodes have not been partitioned into row lists yet
     bool next_round_ready_ = false;  // d_gh_ and the root statistics already belong to the next round
     // profiling

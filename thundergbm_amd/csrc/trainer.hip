@@ -1043,6 +1043,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
 // partitioned, a level served in batches needs its updates batch by batch, and on many rows the launch costs less than
 // the picking of every work item (100 M x 6, depth 8: 9.69 against 9.83 ms a tree; 30 M x 8: 3.28 against 3.30).
 bool Trainer::update_with_partition(int level) const {
+    if (run() > 0) return true;
     return in_boost_ && !sparse_ && n_ < kPartGroupRows && level < param_.depth - 1 &&
            (hist_cap_level_ < 0 || level < hist_cap_level_);
 }
@@ -1112,22 +1113,23 @@ void Trainer::finish_tree(int k, bool fuse_round_end) {
     const TreeBuffers tb = set_of(k);
     rank_order_fresh_ = false;  // the scores change below
     // (the tree is pruned by a workgroup of the same launches)
-    if (small()) {
+    // (see gh_array_stale_: inside boost() the next tree may need the words only; k_small_level reads the pairs)
+    const bool words_only = in_boost_ && !small() && d_gh_words_ != nullptr && tb.complete_feature >= 0;
+    if (maps_rows()) {
         TreeNode *model = d_model_ + (size_t)trees_built_ * tb.n_nodes;
         if (fuse_round_end) {
-            launch_small_end(stream_, tb, bins_, model, param_.gamma, d_yp_, param_.learning_rate, 1, d_y_, objective_,
-                             metric_kind_, d_gh_, d_metric_scratch_, d_gh_words_);
+            launch_map_end(stream_, tb, bins_, small() ? param_.depth - 1 : -1, model, param_.gamma, d_yp_, param_.learning_rate, 1, d_y_, objective_,
+                           metric_kind_, words_only ? nullptr : d_gh_, d_metric_scratch_, d_gh_words_);
+            gh_array_stale_ = words_only;
             gh_words_fresh_ = d_gh_words_ != nullptr;
             gh_records_fresh_ = false;
             next_round_ready_ = true;
             leave_metric();
         } else {
-            launch_small_end(stream_, tb, bins_, model, param_.gamma, d_yp_ + (size_t)k * n_, param_.learning_rate);
+            launch_map_end(stream_, tb, bins_, small() ? param_.depth - 1 : -1, model, param_.gamma, d_yp_ + (size_t)k * n_, param_.learning_rate);
         }
     } else if (fuse_round_end) {
         // one tree per round: prediction update + metric + next gradients + their statistics in one pass
-        // (see gh_array_stale_: inside boost() the next tree may need the words only)
-        const bool words_only = in_boost_ && d_gh_words_ != nullptr && tb.complete_feature >= 0;
         launch_round_end(stream_, tb, &bins_, &csr_, lookup_level_, objective_, metric_kind_, d_y_, d_yp_,
                          param_.learning_rate, words_only ? nullptr : d_gh_, d_metric_scratch_, &param_.gamma, d_gh_words_);
         leave_metric();
@@ -1163,8 +1165,8 @@ void Trainer::build_round_together() {
         find_split_sets(tb, d_gh_, level, K);
         partition_sets(tb, d_gh_, level, K);
     }
-    if (small())
-        launch_small_end(stream_, tb, bins_, d_model_ + (size_t)trees_built_ * tb.n_nodes, param_.gamma, d_yp_, param_.learning_rate, K);
+    if (maps_rows())
+        launch_map_end(stream_, tb, bins_, small() ? param_.depth - 1 : -1, d_model_ + (size_t)trees_built_ * tb.n_nodes, param_.gamma, d_yp_, param_.learning_rate, K);
     else
         launch_predict_in_training(stream_, tb, &bins_, &csr_, lookup_level_, d_yp_, param_.learning_rate, K, &param_.gamma);
     TGBM_CHECK(trees_built_ + K <= model_cap_trees_, "more trees built than n_trees * tree_per_rounds");
@@ -1188,9 +1190,9 @@ void Trainer::run_metric(float *slot) {
     }
 }
 
-// (the small-data path has put them there and leaves the buffers' own nodes unpruned)
+// (launch_map_end has put them there and leaves the buffers' own nodes unpruned)
 void Trainer::leave_model(const TreeNode *nodes, int trees) {
-    if (!small()) left_.model = d_model_ + (size_t)trees_built_ * tb_.n_nodes;
+    if (!maps_rows()) left_.model = d_model_ + (size_t)trees_built_ * tb_.n_nodes;
     left_nodes_ = nodes;
     left_trees_ = (size_t)trees;
 }
@@ -1278,7 +1280,7 @@ void Trainer::boost(int rounds) {
         HIP_CHECK_LAUNCHES("boost");
     }
     settle();
-    if (small() && trees_built_ > 0)  // (for the getters)
+    if (maps_rows() && trees_built_ > 0)  // (for the getters)
         HIP_CHECK(hipMemcpyAsync(const_cast<TreeNode *>(left_nodes_), d_model_ + (size_t)(trees_built_ - (int)left_trees_) * tb_.n_nodes,
                                  sizeof(TreeNode) * (size_t)tb_.n_nodes * left_trees_, hipMemcpyDeviceToDevice, stream_));
     in_boost_ = false;

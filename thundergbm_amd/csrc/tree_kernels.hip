@@ -2232,12 +2232,14 @@ __global__ __launch_bounds__(BLK) void k_tree_end(TreeBuffers tb_all, DenseBins 
     tree_end_rows<MODE, BLK>(tb, a, s_leaf, r0, r1);
 }
 
-// The end of a tree of the small-data path (k_small_level): the rows' nodes are in tb.nid, and the tree is small enough for
-// every workgroup to prune it in LDS by itself; the first one writes the finished nodes into the model (in place they would
-// change under the other workgroups' eyes). One launch instead of k_end_bounds, k_tree_end and the copy: 31 -> 10 us at 10 k
-// rows.
+// The end of a tree whose rows' nodes are in tb.nid (k_small_level, and k_split_count where launch_partition_hist serves the
+// levels), and which is small enough for every workgroup to prune it in LDS by itself; the first one writes the finished nodes
+// into the model (in place they would change under the other workgroups' eyes). One launch instead of k_end_bounds, k_tree_end
+// and the copy: 31 -> 10 us at 10 k rows. At 500 k x 28 the last level's count launch updates the tree and maps the rows (11 us) and
+// the end takes 13.5, where k_best_update, k_end_bounds and k_tree_end took 4.4, 9.7 and 14.7: a tree 0.260 -> 0.255 ms; 100 k rows
+// 0.213 -> 0.204, 300 k x 28 of depth 4 0.131 -> 0.125.
 template <int MODE>
-__global__ __launch_bounds__(kEndWide) void k_small_end(TreeBuffers tb_all, DenseBins bins, TreeEndArgs a, TreeNode *model) {
+__global__ __launch_bounds__(kEndWide) void k_map_end(TreeBuffers tb_all, DenseBins bins, TreeEndArgs a, TreeNode *model) {
     constexpr int kNodes = (2 << kSmallDepth) - 1;
     __shared__ short s_leaf[kRowBlock];
     __shared__ float s_value[kNodes];     // what a row adds that ended in the node
@@ -2260,10 +2262,12 @@ __global__ __launch_bounds__(kEndWide) void k_small_end(TreeBuffers tb_all, Dens
     for (int v = 0; v < V; ++v) {
         const int i = v * kEndWide + (int)threadIdx.x;
         if (r0 + i >= r1) continue;
-        // (the last level's split nodes still hold their rows)
-        const TreeNode &nd = tb.nodes[at[v]];
-        s_leaf[i] = (short)(nd.split_feature_id >= 0 && at[v] >= tb.n_nodes / 4
-                                ? end_child_of<false>(tb, bins, CsrBins{}, nd, r0 + i) : at[v]);
+        int leaf = at[v];
+        if (a.lookup_level >= 0) {  // (that level's split nodes still hold their rows)
+            const TreeNode &nd = tb.nodes[leaf];
+            if (nd.split_feature_id >= 0 && leaf >= (1 << a.lookup_level) - 1) leaf = end_child_of<false>(tb, bins, CsrBins{}, nd, r0 + i);
+        }
+        s_leaf[i] = (short)leaf;
     }
     __syncthreads();
     // (prune_tree in LDS)
@@ -2720,10 +2724,11 @@ void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbi
     tree_end(s, tb, dbins, cbins, 2, a);
 }
 
-void launch_small_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, TreeNode *model, float gamma, float *yp,
+void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int lookup_level, TreeNode *model, float gamma, float *yp,
                       float lr, int n_class, const float *y, int objective, int metric_kind, GHPair *gh,
                       double *metric_scratch, unsigned *gh_words) {
     TreeEndArgs a{};
+    a.lookup_level = lookup_level;
     a.gamma = gamma;
     a.yp = yp;
     a.lr = lr;
@@ -2735,8 +2740,8 @@ void launch_small_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bin
     a.metric_partial = metric_scratch;
     a.gh_words = gh_words;
     const dim3 grid(row_blocks(tb.n), 1, n_class);
-    if (y != nullptr) k_small_end<2><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
-    else k_small_end<1><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+    if (y != nullptr) k_map_end<2><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+    else k_map_end<1><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
 }
 
 void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left) {
