@@ -438,10 +438,12 @@ struct TreeLeftovers {  // of the tree before: see k_tree_init
 };
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda,
                       bool stats_ready = false, int n_class = 1, const TreeLeftovers &left = TreeLeftovers());
+void launch_root_stats(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, int n_class);
 void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left);
-// sum_rows (level 0): also the sums of the items' rows into tb.root_total, for a split search with root_of_rows.
+// sum_rows (level 0): also the sums of the items' rows into tb.root_total, for a split search with root_of_rows. init (level 0):
+// also what launch_tree_init does; tb.root_partial is ready (launch_root_stats).
 void launch_hist_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                       int n_class = 1, bool sum_rows = false);
+                       int n_class = 1, bool sum_rows = false, const TreeLeftovers *init = nullptr, float lambda = 0);
 void launch_hist_merge(hipStream_t s, const TreeBuffers &tb, int level, int n_class = 1);
 // After the root histogram exists: replaces the root's float sums (whose last bits depend on the order of the rows)
 // by the exact fixed-point totals, from the bins of tb.complete_feature or, without one, from the gradients.

@@ -82,7 +82,7 @@ struct Picked {
     SplitCand c;
 };
 // Up to so many packs each wavefront looks at all of them: no barrier, no LDS (500 k x 28: the candidates' part of a count
-// launch 1.7 -> 0.95 us; of a small level's sixteen wavefronts 2.9 -> 0.4 with 10 packs, TODO with 100). Beyond, the workgroup
+// launch 1.7 -> 0.95 us; of a small level's sixteen wavefronts 2.9 -> 0.65 with 100 packs). Beyond, the workgroup
 // shares them out.
 constexpr int kWavePacks = 256;
 struct PickShared {

@@ -89,6 +89,9 @@ class Trainer {
     void run_metric(float *slot);  // (leaves the last step of the point-wise metrics in left_)
     void leave_metric();
     void leave_model(const TreeNode *nodes, int trees);
+    // Inside boost() the dense layout sets a tree up in its first histogram launch; until then its sets' left_ and that are kept.
+    bool init_pending_ = false;
+    void begin_tree(const TreeBuffers &tb, const GHPair *gh, bool stats_ready, int n_class);
     TreeLeftovers leftovers() const {
         TreeLeftovers l = left_;
         l.small = small();

@@ -796,11 +796,20 @@ void Trainer::tree_init(int k) {
     if (!in_boost_) ensure_gh_array();
     cur_class_ = k;
     HIP_CHECK_LAUNCHES("the stages before tree_init");  // gradients, bagging, column sampling, metric, re-ordering
-    launch_tree_init(stream_, set_of(k), d_gh_ + (size_t)k * n_, param_.lambda, next_round_ready_, 1, leftovers());
-    left_ = TreeLeftovers();
+    begin_tree(set_of(k), d_gh_ + (size_t)k * n_, next_round_ready_, 1);
     next_round_ready_ = false;
     lookup_level_ = -1;
     nid_materialized_ = false;
+}
+
+void Trainer::begin_tree(const TreeBuffers &tb, const GHPair *gh, bool stats_ready, int n_class) {
+    init_pending_ = in_boost_ && !sparse_;
+    if (init_pending_) {
+        if (!stats_ready) launch_root_stats(stream_, tb, gh, n_class);
+        return;
+    }
+    launch_tree_init(stream_, tb, gh, param_.lambda, stats_ready, n_class, leftovers());
+    left_ = TreeLeftovers();
 }
 
 void Trainer::ensure_gh_array() {
@@ -1061,7 +1070,10 @@ void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *g
         if (level == 0) gh_records_fresh_ = gh_words_fresh_ && n_class == 1 && gh == d_gh_ && tb.lvl_x0 == 0;
         b.gh_fresh = gh_records_fresh_ && n_class == 1 && gh == d_gh_;
         b.gh_objective = objective_;
-        launch_hist_dense(stream_, tb, b, gh, level, n_class, sum_rows);
+        const TreeLeftovers left = leftovers();
+        launch_hist_dense(stream_, tb, b, gh, level, n_class, sum_rows, init_pending_ ? &left : nullptr, param_.lambda);
+        if (init_pending_) left_ = TreeLeftovers();
+        init_pending_ = false;
     }
 }
 
@@ -1157,8 +1169,7 @@ void Trainer::build_round_together() {
     TreeBuffers tb = tb_;
     // the K classes share the chip: size every class's histogram items for its share of the workgroup slots
     tb.target_hitems = std::max(4, tb_.target_hitems / K);
-    launch_tree_init(stream_, tb, d_gh_, param_.lambda, false, K, leftovers());
-    left_ = TreeLeftovers();
+    begin_tree(tb, d_gh_, false, K);
     lookup_level_ = -1;
     nid_materialized_ = false;
     for (int level = 0; level < param_.depth; ++level) {

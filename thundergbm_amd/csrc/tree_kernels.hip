@@ -3,6 +3,7 @@
 // in-training prediction update. Every stage of a level is one launch over all nodes of the level;
 // work lists are planned on the device so the host never waits inside a tree.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_api.h"
 #include "kernel_common.h"
@@ -216,29 +217,65 @@ __device__ float pow2_scale(float vmax, int rows, float limit) {
 }
 
 // ------------------------------------------------------------------------------- tree init
+// The tree's scales, from the largest |g| and h of its rows and whether every h is an integer (GradStats): they keep the 64-bit
+// sums over all n rows below 2^62; a dense work item coarsens them by its own power of two so that its packed LDS fields hold
+// the rows between two drains (item_shift).
+__device__ __forceinline__ QuantCtl plan_quant(const TreeBuffers &tb, float gm, float hm, float hf) {
+    QuantCtl q;
+    // (the sparse layout's kernels round with round_to_ll, good below 2^51: its scales are those of at least
+    // 4096 rows, which keeps every row's integers below 2^50)
+    const int scale_rows = tb.sparse ? max(tb.n, 4096) : tb.n;
+    q.scale_g = pow2_scale(gm, scale_rows, 4.6e18f);
+    q.scale_h = pow2_scale(hm, scale_rows, 4.6e18f);
+    q.h_bits = 32;
+    q.h_integer = 0;
+    // every hessian a non-negative integer (squared loss; bagging multiplies by draw counts): the hessian field
+    // takes the bits that kHistFlushRowsInt such rows need, the gradient field the rest
+    q.flush_rows = kHistFlushRows;
+    const float hrows = hm * (float)kHistFlushRowsInt;
+    if (!tb.sparse && hf == 0.f && hm >= 1.f && hrows < 4.0e9f) {
+        q.h_integer = 1;
+        q.h_bits = ilogbf(hrows) + 1;
+        q.scale_h = 1.f;
+        q.flush_rows = kHistFlushRowsInt;
+    }
+    q.inv_g = 1.f / q.scale_g;
+    q.inv_h = 1.f / q.scale_h;
+    q.gq_max = gm * q.scale_g;
+    q.hq_max = hm * q.scale_h;
+    return q;
+}
+
+// Rows per histogram work item of the root.
+__device__ __forceinline__ int root_chunk(const TreeBuffers &tb) {
+    const int chunk = (tb.n + tb.target_hitems - 1) / tb.target_hitems;
+    return max(kHistMinChunk, (chunk + 255) / 256 * 256);
+}
+
 // Node array initialisation of the reference's Tree::init2 (src/thundergbm/tree.cu:8-39), root sum
 // from the block partials, root segment and the histogram plan of level 0.
-// What the previous tree has left to do rides along: its finished nodes go into the model before they are reset, and the
-// last workgroup adds up the round's metric (two launches of 4 to 5 us per tree otherwise).
-// The first workgroup does all but the metric; trees of more than kInitNodes nodes are shared out over `parts` of them (with
-// one, the nodes of depth 14 took 85 us).
+// What the previous tree has left to do rides along: its finished nodes go into the model before they are reset, and one more
+// workgroup adds up the round's metric (two launches of 4 to 5 us per tree otherwise).
+// The first workgroup (part 0) does all but the metric; trees of more than kInitNodes nodes are shared out over `parts` of them
+// (with one, the nodes of depth 14 took 85 us). In the dense layout the root level's histogram launch has these workgroups
+// (k_hist_dense): a launch of 4.7 us less, 10 k x 8 0.126 -> 0.122 ms a tree, 500 k x 28 0.256 -> 0.252.
 constexpr int kInitNodes = 1024;
+int init_parts(const TreeBuffers &tb) { return (tb.n_nodes + kInitNodes - 1) / kInitNodes; }
 __device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out);
-__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda, TreeLeftovers left, int parts) {
-    if ((int)blockIdx.x == parts) {
-        if (blockIdx.z == 0) metric_final(left.metric_kind, tb_all.n, left.metric_blocks, left.metric_partial, left.metric_out);
+__device__ void tree_init_part(const TreeBuffers &tb, float lambda, const TreeLeftovers &left, int part, int parts) {  // kBlock threads
+    if (part == parts) {
+        if (blockIdx.z == 0) metric_final(left.metric_kind, tb.n, left.metric_blocks, left.metric_partial, left.metric_out);
         return;
     }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
-    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
-    if (left.small && blockIdx.x == 0) {  // every row starts in the root
+    if (left.small && part == 0) {  // every row starts in the root
         for (int i = threadIdx.x; i < tb.n; i += kBlock) tb.nid[i] = 0;
     }
-    if ((left.small || left.run > 0) && blockIdx.x == 0)
+    if ((left.small || left.run > 0) && part == 0)
         for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{left.run, 0, 0, 0};
     const GradStats *__restrict__ block_sums = tb.root_partial;
     const int nn = tb.n_nodes;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < nn; i += parts * kBlock) {
+    for (int i = part * kBlock + threadIdx.x; i < nn; i += parts * kBlock) {
         TreeNode nd;
         nd.final_id = i;
         nd.parent_index = i == 0 ? -1 : (i - 1) / 2;
@@ -275,7 +312,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
         tb.seg[i] = make_int2(0, 0);
         if (tb.node_rows != nullptr) tb.node_rows[i] = i == 0 ? tb.n : 0;
     }
-    if (blockIdx.x != 0) return;
+    if (part != 0) return;
     float g = 0, h = 0, gm = 0, hm = 0, hf = 0;
     for (int i = threadIdx.x; i < tb.n_grad_blocks; i += kBlock) {
         g += block_sums[i].g;
@@ -317,9 +354,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
         root.is_valid = true;
         root.base_weight = -s.g / (s.h + lambda);
         tb.seg[0] = make_int2(0, tb.n);
-        int chunk = (tb.n + tb.target_hitems - 1) / tb.target_hitems;
-        chunk = max(kHistMinChunk, (chunk + 255) / 256 * 256);
-        int items = (tb.n + chunk - 1) / chunk;
+        const int chunk = root_chunk(tb), items = (tb.n + chunk - 1) / chunk;
         tb.hpair_begin[0] = 0;
         tb.hpair_begin[1] = items;
         tb.hpair_built[0] = 0;
@@ -332,32 +367,36 @@ __global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float 
         tb.pbegin(0)[0] = 0;
         tb.pbegin(0)[1] = c.n_pitems;
         tb.ctl[tb.depth] = LevelCtl{0, 0, 0, 0};  // the last level plans no further one
-        // The tree's scales keep the 64-bit sums over all n rows below 2^62; a dense work item coarsens them by its
-        // own power of two so that its packed LDS fields hold the rows between two drains (item_shifts).
-        QuantCtl q;
-        // (the sparse layout's kernels round with round_to_ll, good below 2^51: its scales are those of at least
-        // 4096 rows, which keeps every row's integers below 2^50)
-        const int scale_rows = tb.sparse ? max(tb.n, 4096) : tb.n;
-        q.scale_g = pow2_scale(gm, scale_rows, 4.6e18f);
-        q.scale_h = pow2_scale(hm, scale_rows, 4.6e18f);
-        q.h_bits = 32;
-        q.h_integer = 0;
-        // every hessian a non-negative integer (squared loss; bagging multiplies by draw counts): the hessian field
-        // takes the bits that kHistFlushRowsInt such rows need, the gradient field the rest
-        q.flush_rows = kHistFlushRows;
-        const float hrows = hm * (float)kHistFlushRowsInt;
-        if (!tb.sparse && hf == 0.f && hm >= 1.f && hrows < 4.0e9f) {
-            q.h_integer = 1;
-            q.h_bits = ilogbf(hrows) + 1;
-            q.scale_h = 1.f;
-            q.flush_rows = kHistFlushRowsInt;
-        }
-        q.inv_g = 1.f / q.scale_g;
-        q.inv_h = 1.f / q.scale_h;
-        q.gq_max = gm * q.scale_g;
-        q.hq_max = hm * q.scale_h;
-        *tb.quant = q;
+        *tb.quant = plan_quant(tb, gm, hm, hf);
     }
+}
+__global__ __launch_bounds__(kBlock) void k_tree_init(TreeBuffers tb_all, float lambda, TreeLeftovers left, int parts) {
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    tree_init_part(tb, lambda, left, blockIdx.x, parts);
+}
+
+// The tree's scales by every thread of a BLK-wide workgroup for itself; lds: 3 floats per wavefront. One barrier.
+template <int BLK>
+__device__ __forceinline__ QuantCtl quant_of_stats(const TreeBuffers &tb, float *lds) {
+    constexpr int NW = BLK / 64;
+    const GradStats *__restrict__ stats = tb.root_partial;
+    float gm = 0, hm = 0, hf = 0;
+    for (int i = threadIdx.x; i < tb.n_grad_blocks; i += BLK) {
+        gm = fmaxf(gm, stats[i].gmax);
+        hm = fmaxf(hm, stats[i].hmax);
+        hf = fmaxf(hf, stats[i].hfrac);
+    }
+    gm = wave_max_f(gm);
+    hm = wave_max_f(hm);
+    hf = wave_max_f(hf);
+    if (lane_id() == 0) {
+        lds[wave_id()] = gm;
+        lds[NW + wave_id()] = hm;
+        lds[2 * NW + wave_id()] = hf;
+    }
+    __syncthreads();
+    const int w = lane_id() % NW;
+    return plan_quant(tb, wave_max_f(lds[w]), wave_max_f(lds[NW + w]), wave_max_f(lds[2 * NW + w]));
 }
 
 // ------------------------------------------------------------------------------ exact root sums
@@ -405,12 +444,13 @@ __global__ __launch_bounds__(kBlock) void k_root_sum_bins(TreeBuffers tb_all, fl
 // From the gradients (no feature is stored in every row): every row's pair rounded at the tree's scales, a pair of 64-bit sums
 // per part of the rows into root_total[2 part], [2 part + 1], which whoever needs the root's sums adds up: in the dense layout
 // by the root level's histogram launch and by every workgroup of its split search (two launches of 4 to 9 us a tree less:
-// 500 k x 54 with 8 classes 0.515 -> TODO ms a round). (A ticket that lets the last workgroup finish the job needs a device-scope
+// 500 k x 54 with 8 classes 0.515 -> 0.503 ms a round). (A ticket that lets the last workgroup finish the job needs a device-scope
 // fence, which writes a whole L2 back on this chip: 288 us per round of 8 class trees.)
 template <int BLK>
-__device__ __forceinline__ void root_sum_rows(const TreeBuffers &tb, const GHPair *__restrict__ gh, int begin, int end, int part) {
+__device__ __forceinline__ void root_sum_rows(const TreeBuffers &tb, const QuantCtl &quant, const GHPair *__restrict__ gh, int begin, int end,
+                                              int part) {
     __shared__ long long s_g[BLK / 64], s_h[BLK / 64];
-    const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
+    const float scale_g = quant.scale_g, scale_h = quant.scale_h;
     long long g = 0, hh = 0;
     for (int i = begin + (int)threadIdx.x; i < end; i += BLK) {
         const GHPair v = gh[i];
@@ -451,7 +491,7 @@ __device__ __forceinline__ GHPair root_sums_of_rows(const TreeBuffers &tb, int p
 __global__ __launch_bounds__(kBlock) void k_root_sum_rows(TreeBuffers tb_all, const GHPair *__restrict__ gh) {
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int per = (tb.n + (int)gridDim.x - 1) / (int)gridDim.x, begin = min(tb.n, (int)blockIdx.x * per);
-    root_sum_rows<kBlock>(tb, gh + (size_t)blockIdx.z * tb.n, begin, min(tb.n, begin + per), blockIdx.x);
+    root_sum_rows<kBlock>(tb, *tb.quant, gh + (size_t)blockIdx.z * tb.n, begin, min(tb.n, begin + per), blockIdx.x);
 }
 
 __global__ __launch_bounds__(64) void k_root_sum_final(TreeBuffers tb_all, int parts, float lambda) {
@@ -477,15 +517,21 @@ __global__ __launch_bounds__(64) void k_root_sum_final(TreeBuffers tb_all, int p
 // GHW: the rows' gradient pairs come from 32-bit words (word_from_row). Below the root the word sits in the last
 // dword of the row's record, which the row's last lane has loaded with the bins anyway: no second gather per row. The
 // root launch (DIRECT) reads the words from their own array and puts them there, storing every record back.
+struct HistRoot {  // DIRECT: what the root level's launch does besides
+    int init_groups = 0, init_parts = 0;  // the tree's set-up by so many workgroups more (tree_init_part)
+    bool sum_rows = false;                // the sums of the items' rows into root_total
+    float lambda = 0;
+    TreeLeftovers left;
+};
 template <int LPR, bool DIRECT, int BLK, int SLOTS, bool BIN16, bool GHW = false>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(SLOTS <= 8 ? 8 : 4)))  // two 1024-thread groups per CU
-void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level, int n_pairs, bool sum_rows) {
+void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level, int n_pairs,
+                  std::conditional_t<DIRECT, HistRoot, int> root) {
     extern __shared__ unsigned long long lds[];
     __shared__ int s_shift[2];  // the item's scale shifts (gradient, hessian)
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
     const int *__restrict__ ridx = tb.list(level);
-    const QuantCtl *__restrict__ quant = tb.quant;
     const int *__restrict__ blk_bin_begin = tb.blk_bin_begin;
     const int *__restrict__ feat_lds_off = tb.feat_lds_off;
     longlong2 *__restrict__ partial = tb.partial;
@@ -493,8 +539,16 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     // (the feature blocks of an item are neighbours in the launch order: the item's row list and gradient pairs, which
     // every block reads again, are then fetched while they still sit in an L2 - with the items of a block as
     // neighbours, every block of 500 k x 2000 data fetched them from HBM again: 2.72 -> 2.29 ms per tree)
-    const int item = blockIdx.y;
+    int item = blockIdx.y;
     const int fb = blockIdx.x;
+    QuantCtl quant;
+    if constexpr (DIRECT) {
+        if (item < root.init_groups) {  // the tree's set-up, by the first block's workgroups (of kBlock threads)
+            if (fb == 0 && threadIdx.x < kBlock) tree_init_part(tb, root.lambda, root.left, item, root.init_parts);
+            return;
+        }
+        item -= root.init_groups;
+    }
     // The item's node and rows: the same few look-ups in every lane (uniform addresses: scalar loads) or in every
     // wavefront, so that the first row loads can be issued before the barrier that publishes the LDS histogram's clearing.
     int node, hchunk;
@@ -510,18 +564,24 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
         first_item = plan.first_item;
         item0 = plan.item0;
     } else {
-        const LevelCtl c = tb.ctl[level];
-        if (item >= c.n_hitems) return;
         node = 0;
         sg = make_int2(0, tb.n);
-        hchunk = c.hchunk;
+        hchunk = root_chunk(tb);
         first_item = 0;
+        if (item * hchunk >= tb.n) return;
+        if (root.init_groups > 0) {
+            __shared__ float s_stats[3 * BLK / 64];
+            quant = quant_of_stats<BLK>(tb, s_stats);
+        } else {
+            quant = *tb.quant;
+        }
     }
     const int bin0 = blk_bin_begin[fb];
     const int nb = blk_bin_begin[fb + 1] - bin0;
     if (nb == 0) return;
-    const int h_bits = quant->h_bits;
-    const int flush_rows = quant->flush_rows;
+    if constexpr (!DIRECT) quant = *tb.quant;
+    const int h_bits = quant.h_bits;
+    const int flush_rows = quant.flush_rows;
     const int gh_objective = bins.gh_objective;
     const bool word_lane = bins.gh_lane >= 0 && (int)(threadIdx.x % LPR) == bins.gh_lane;
     const int begin = __builtin_amdgcn_readfirstlane(sg.x + (item - first_item) * hchunk);
@@ -531,9 +591,9 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     if (threadIdx.x == 0) {
         // (the node's rows, not the item's: what a row adds must not depend on the item it falls into, or the sums
         // would change with the order of the rows)
-        const int rows = max(1, min(sg.y - sg.x, quant->flush_rows));
-        const int2 shift = make_int2(item_shift(quant->gq_max, rows, 63 - h_bits),
-                                     quant->h_integer ? 0 : item_shift(quant->hq_max, rows, h_bits));
+        const int rows = max(1, min(sg.y - sg.x, quant.flush_rows));
+        const int2 shift = make_int2(item_shift(quant.gq_max, rows, 63 - h_bits),
+                                     quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits));
         s_shift[0] = shift.x;
         s_shift[1] = shift.y;
         if (fb == 0) tb.hitem_shift[item] = shift;
@@ -592,8 +652,8 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     for (int i = threadIdx.x; i < nb; i += BLK) lds[i] = 0ull;
     __syncthreads();
     // the item's scales: powers of two well inside the float range, so the products below are exact
-    const float scale_g = ldexpf(quant->scale_g, -__builtin_amdgcn_readfirstlane(s_shift[0]));
-    const float scale_h = ldexpf(quant->scale_h, -__builtin_amdgcn_readfirstlane(s_shift[1]));
+    const float scale_g = ldexpf(quant.scale_g, -__builtin_amdgcn_readfirstlane(s_shift[0]));
+    const float scale_h = ldexpf(quant.scale_h, -__builtin_amdgcn_readfirstlane(s_shift[1]));
     for (int base = begin; base < end; base += STEP) {
         // the next step's rows are requested before this step's atomics (and before a drain's
         // barriers), so the memory pipeline stays busy
@@ -658,7 +718,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
         }
     }
     if constexpr (DIRECT)
-        if (sum_rows && fb == 0) root_sum_rows<BLK>(tb, gh, begin, end, item);
+        if (root.sum_rows && fb == 0) root_sum_rows<BLK>(tb, quant, gh, begin, end, item);
     __syncthreads();
     if (hchunk <= flush_rows) {
         // an item this short was never drained: its packed LDS words are the complete sums and go out as
@@ -2442,11 +2502,15 @@ void launch_bagging(hipStream_t s, int N, unsigned seed, int *count, GHPair *gh,
 // Launchers: `tb` is the first buffer set to use, `n_class` consecutive sets (class trees of one round)
 // are served by the same launch through blockIdx.z; gradient and prediction pointers address the
 // first of those classes.
+void launch_root_stats(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, int n_class) {
+    // n_grad_blocks == row_blocks(n)
+    k_sum_gh<<<dim3(tb.n_grad_blocks, 1, n_class), kBlock, 0, s>>>(tb.n, gh_class, tb.root_partial);
+}
+
 void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_class, float lambda, bool stats_ready,
                       int n_class, const TreeLeftovers &left) {
-    if (!stats_ready)  // n_grad_blocks == row_blocks(n)
-        k_sum_gh<<<dim3(tb.n_grad_blocks, 1, n_class), kBlock, 0, s>>>(tb.n, gh_class, tb.root_partial);
-    const int parts = (tb.n_nodes + kInitNodes - 1) / kInitNodes;
+    if (!stats_ready) launch_root_stats(s, tb, gh_class, n_class);
+    const int parts = init_parts(tb);
     k_tree_init<<<dim3(parts + (left.metric_out != nullptr ? 1 : 0), 1, n_class), kBlock, 0, s>>>(tb, lambda, left, parts);
     if (tb.nid16 != nullptr) {
         // sparse level pass: every row starts in the root (the n_class maps lie back to back)
@@ -2457,13 +2521,13 @@ void launch_tree_init(hipStream_t s, const TreeBuffers &tb, const GHPair *gh_cla
 
 template <int LPR, int SLOTS, bool BIN16>
 static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh,
-                              int level, int n_class, bool sum_rows) {
+                              int level, int n_class, const HistRoot &root) {
     const int n_pairs = tb.n_hpairs(level);
     // (an upper bound on the work items: whole chunks of the rows that can be built - half of them below the root, unless
     // single nodes are built - and one partly filled item per built node; see plan_hist_item)
     const long rows = level == 0 || tb.singles(level) ? tb.n : tb.n / 2;
     const long by_rows = rows / kHistMinChunk + n_pairs, by_target = std::max(tb.target_hitems, tb.target_hitems / 4 + n_pairs) + 1;
-    dim3 grid(bins.n_blocks, (unsigned)std::max(1l, std::min({by_rows, by_target, (long)tb.max_hitems})), n_class);
+    dim3 grid(bins.n_blocks, (unsigned)std::max(1l, std::min({by_rows, by_target, (long)tb.max_hitems})) + root.init_groups, n_class);
     size_t lds = (size_t)tb.max_block_bins * sizeof(unsigned long long);
     if (lds > 64 * 1024) {
         static LdsOptIn opt_in;
@@ -2478,49 +2542,57 @@ static void hist_dense_launch(hipStream_t s, const TreeBuffers &tb, const DenseB
                               reinterpret_cast<const void *>(&k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true>)});
             }
             if (level == 0)
-                k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, sum_rows);
+                k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, root);
             else
-                k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, false);
+                k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16, true><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, 0);
             return;
         }
     }
     if (level == 0)
-        k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, sum_rows);
+        k_hist_dense<LPR, true, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, root);
     else
-        k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, false);
+        k_hist_dense<LPR, false, kHistBlock, SLOTS, BIN16><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, n_pairs, 0);
 }
 
 template <int LPR>
 static void hist_dense_dispatch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh,
-                                int level, int n_class, bool sum_rows) {
+                                int level, int n_class, const HistRoot &root) {
     const int slots = (tb.max_block_bins + kHistBlock - 1) / kHistBlock;  // bins drained per thread
     if (bins.bin_bytes == 2) {  // (fewer variants: the blocks of 16-bit bins are sized to fill the LDS)
-        if (slots <= 4) hist_dense_launch<LPR, 4, true>(s, tb, bins, gh, level, n_class, sum_rows);
-        else if (slots <= 8) hist_dense_launch<LPR, 8, true>(s, tb, bins, gh, level, n_class, sum_rows);
-        else if (slots <= 20) hist_dense_launch<LPR, 20, true>(s, tb, bins, gh, level, n_class, sum_rows);
+        if (slots <= 4) hist_dense_launch<LPR, 4, true>(s, tb, bins, gh, level, n_class, root);
+        else if (slots <= 8) hist_dense_launch<LPR, 8, true>(s, tb, bins, gh, level, n_class, root);
+        else if (slots <= 20) hist_dense_launch<LPR, 20, true>(s, tb, bins, gh, level, n_class, root);
         else fatal("feature block with %d bins does not fit the histogram kernel", tb.max_block_bins);
         return;
     }
-    if (slots <= 1) hist_dense_launch<LPR, 1, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 2) hist_dense_launch<LPR, 2, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 3) hist_dense_launch<LPR, 3, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 4) hist_dense_launch<LPR, 4, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 6) hist_dense_launch<LPR, 6, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 7) hist_dense_launch<LPR, 7, false>(s, tb, bins, gh, level, n_class, sum_rows);  // fewer accumulator registers
-    else if (slots <= 8) hist_dense_launch<LPR, 8, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 16) hist_dense_launch<LPR, 16, false>(s, tb, bins, gh, level, n_class, sum_rows);
-    else if (slots <= 20) hist_dense_launch<LPR, 20, false>(s, tb, bins, gh, level, n_class, sum_rows);
+    if (slots <= 1) hist_dense_launch<LPR, 1, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 2) hist_dense_launch<LPR, 2, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 3) hist_dense_launch<LPR, 3, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 4) hist_dense_launch<LPR, 4, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 6) hist_dense_launch<LPR, 6, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 7) hist_dense_launch<LPR, 7, false>(s, tb, bins, gh, level, n_class, root);  // fewer accumulator registers
+    else if (slots <= 8) hist_dense_launch<LPR, 8, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 16) hist_dense_launch<LPR, 16, false>(s, tb, bins, gh, level, n_class, root);
+    else if (slots <= 20) hist_dense_launch<LPR, 20, false>(s, tb, bins, gh, level, n_class, root);
     else fatal("feature block with %d bins does not fit the histogram kernel", tb.max_block_bins);
 }
 
 void launch_hist_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                       int n_class, bool sum_rows) {
+                       int n_class, bool sum_rows, const TreeLeftovers *init, float lambda) {
+    HistRoot root;
+    root.sum_rows = sum_rows;
+    if (init != nullptr) {
+        root.init_parts = init_parts(tb);
+        root.init_groups = root.init_parts + (init->metric_out != nullptr ? 1 : 0);
+        root.lambda = lambda;
+        root.left = *init;
+    }
     switch (bins.W * bins.bin_bytes) {  // bytes per row of a block = 4 x lanes per row
-        case 4: hist_dense_dispatch<1>(s, tb, bins, gh, level, n_class, sum_rows); break;
-        case 8: hist_dense_dispatch<2>(s, tb, bins, gh, level, n_class, sum_rows); break;
-        case 16: hist_dense_dispatch<4>(s, tb, bins, gh, level, n_class, sum_rows); break;
-        case 32: hist_dense_dispatch<8>(s, tb, bins, gh, level, n_class, sum_rows); break;
-        case 64: hist_dense_dispatch<16>(s, tb, bins, gh, level, n_class, sum_rows); break;
+        case 4: hist_dense_dispatch<1>(s, tb, bins, gh, level, n_class, root); break;
+        case 8: hist_dense_dispatch<2>(s, tb, bins, gh, level, n_class, root); break;
+        case 16: hist_dense_dispatch<4>(s, tb, bins, gh, level, n_class, root); break;
+        case 32: hist_dense_dispatch<8>(s, tb, bins, gh, level, n_class, root); break;
+        case 64: hist_dense_dispatch<16>(s, tb, bins, gh, level, n_class, root); break;
         default: fatal("unsupported dense block width %d x %d bytes", bins.W, bins.bin_bytes);
     }
 }
