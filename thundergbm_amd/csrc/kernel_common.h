@@ -75,6 +75,30 @@ __device__ __forceinline__ long long read_lane_ll(long long v, int lane) {
     return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
+// Inclusive sums of two 64-bit integers over a wavefront: four instructions a step, the lane move part of the additions. (A
+// register that a vector instruction has just written may be read through DPP two instructions later: between the four they
+// are, before the first step there is an s_nop.)
+__device__ __forceinline__ void wave_scan_pair(long long &a, long long &b) {
+    unsigned al = (unsigned)(unsigned long long)a, ah = (unsigned)((unsigned long long)a >> 32);
+    unsigned bl = (unsigned)(unsigned long long)b, bh = (unsigned)((unsigned long long)b >> 32);
+#define TGBM_SCAN_STEP(MOVE)                           \
+    "v_add_co_u32_dpp %0, vcc, %0, %0 " MOVE "\n"      \
+    "v_addc_co_u32_dpp %1, vcc, %1, %1, vcc " MOVE "\n" \
+    "v_add_co_u32_dpp %2, vcc, %2, %2 " MOVE "\n"      \
+    "v_addc_co_u32_dpp %3, vcc, %3, %3, vcc " MOVE "\n"
+    asm("s_nop 1\n"
+        TGBM_SCAN_STEP("row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0")
+        TGBM_SCAN_STEP("row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0")
+        TGBM_SCAN_STEP("row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0")
+        TGBM_SCAN_STEP("row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0")
+        TGBM_SCAN_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf")
+        TGBM_SCAN_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+        : "+v"(al), "+v"(ah), "+v"(bl), "+v"(bh) : : "vcc");
+#undef TGBM_SCAN_STEP
+    a = (long long)((unsigned long long)ah << 32 | al);
+    b = (long long)((unsigned long long)bh << 32 | bl);
+}
+
 struct WaveSumI {
     int v;
     template <int CTRL, int ROWS>
@@ -164,6 +188,19 @@ __device__ __forceinline__ int item_shift(float qmax, int rows, int bits) {
 }
 
 // ------------------------------------------------------------------------ split finding
+// (float)((double)v * inv), inv a power of two: the integer's halves are scaled exactly and added with one rounding.
+__device__ __forceinline__ float scaled_float(long long v, double inv) {
+    const double hi = (double)(int)(v >> 32), lo = (double)(unsigned)(unsigned long long)v;
+    return (float)__fma_rn(hi, inv * 4294967296.0, lo * inv);
+}
+
+// split_gain without a branch; fterm: (f.g * f.g) / (f.h + lambda)
+__device__ __forceinline__ float split_gain_select(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
+#pragma clang fp contract(off)
+    const GHPair r{f.g - l.g, f.h - l.h};
+    const float gain = (l.g * l.g) / (l.h + lambda) + (r.g * r.g) / (r.h + lambda) - fterm;
+    return fmaxf(0.f, ((l.h >= mcw) & (r.h >= mcw)) ? gain : 0.f);
+}
 __device__ __forceinline__ float split_gain(GHPair f, GHPair l, float mcw, float lambda) {
 #pragma clang fp contract(off)
     GHPair r{f.g - l.g, f.h - l.h};
