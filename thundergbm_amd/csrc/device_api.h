@@ -87,6 +87,10 @@ constexpr int kPartGroup = 64;
 constexpr int kSplitHistRows = 1 << 20;
 constexpr int kSplitHistMost = 4;
 constexpr size_t kSplitHistBytes = 13 << 20;
+// A workgroup's LDS adds about 8 pairs a nanosecond, so up to a workgroup per CU a block's columns are shared out as well
+// (each part lays the lists out again): 20 k x 28 0.128 -> 0.111 ms a tree, 100 k x 28 0.198 -> 0.187, 500 k x 28 0.251 -> 0.246; with two per
+// CU 0.111, 0.200 and 0.279.
+constexpr int kSplitHistGroups = 256;
 // Dense layout: up to so many pairs (nodes, where single nodes are built) in a level every workgroup plans for itself.
 constexpr int kUnplannedPairs = 256;
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
@@ -472,17 +476,23 @@ void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float r
 void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int level, bool update,
                             float rt_eps, float lambda, int n_class = 1);
 // Dense layout, moderately many rows: launch_partition_dense and the histograms of the next level's built nodes in two
-// launches instead of three (k_split_hist). split_hist_run: rows of a level's node that a workgroup of the second one serves,
-// 0: such data goes through launch_partition_dense and launch_hist_dense. Inside boost() only: the level's candidates are fresh,
+// launches instead of three (k_split_hist). split_hist_plan: rows of a level's node that a workgroup of the second one serves,
+// run 0: such data goes through launch_partition_dense and launch_hist_dense. Inside boost() only: the level's candidates are fresh,
 // and every row leaves the node where it ends in tb.nid (launch_map_end), at level tb.depth - 1 the last of them.
-int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class);
-void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
+// Feature blocks are shared out over 1 << log_split workgroups where there would be few. part_bins[k]: most bins of a part of
+// a block in 1 << k parts.
+struct SplitHistPlan {
+    int run = 0, log_split = 0;
+    int lds_bins = 0;  // part_bins[log_split]
+};
+SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, const int *part_bins, int n_class);
+void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, const SplitHistPlan &plan,
                            float rt_eps, float lambda, int n_class = 1);
 // Dense layout, few rows: the level's splits, the children's lists and the histograms of the next level's built nodes in one
 // launch. The split search of the next level then derives the siblings (launch_eval_split with derive).
 bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins);
 void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
-                        float lambda, int n_class = 1);
+                        float lambda, const int *part_bins, int n_class = 1);
 // The end of a tree whose rows' nodes are in tb.nid (lookup_level >= 0: split nodes of that level still hold the rows of their
 // children): prunes the tree into `model` (n_class trees back to back; tb.nodes
 // stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics.

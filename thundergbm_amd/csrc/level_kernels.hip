@@ -495,8 +495,9 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 // Few rows (kSmallRows): a level in one launch instead of count, scatter, histogram and merge, which take 5 to 7 us each with
 // nothing to do. A workgroup owns a node and a feature block: it picks the node's split, decides for every row, lays the
 // children's lists down and adds up the histogram of the child with fewer rows, whose list it has in LDS, right at the
-// tree's scales; the split search derives the sibling (k_eval_split<true>). Every block of a node repeats the split, the
-// first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
+// tree's scales; the split search derives the sibling (k_eval_split<true>). Up to kSplitHistGroups workgroups share a block's
+// columns (1605 x 60, depth 6: 0.105 -> 0.101 ms a tree; 16 k x 30, depth 8: 0.214 -> 0.178). Every workgroup of a node repeats
+// the split, the first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
 // (k_map_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
 // A level of 10 k x 8: 28 -> 14 us with its split search.
 // The sums are those of k_hist_dense, whose work items count at a scale that hangs on the node's rows only.
@@ -507,25 +508,29 @@ static_assert(kSmallRows <= 1 << 16 && kSmallWaves == 16 && kSmallSteps % 4 == 0
 
 template <int LPR, bool BIN16, int STEPS>
 __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
-                                                            int level, float rt_eps, float lambda) {
+                                                            int level, float rt_eps, float lambda, int log_split, int lds_bins) {
     extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
     __shared__ PickShared s_pick;
     __shared__ int s_left[STEPS * kSmallWaves];  // rows that go left, per step and wavefront
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
-    unsigned short *s_rows = reinterpret_cast<unsigned short *>(lds + tb.max_block_bins);
-    const int fb = blockIdx.x, x_in = blockIdx.y, x = (1 << level) - 1 + x_in;
+    unsigned short *s_rows = reinterpret_cast<unsigned short *>(lds + lds_bins);
+    const int fb = blockIdx.x >> log_split, part = blockIdx.x & ((1 << log_split) - 1), x_in = blockIdx.y, x = (1 << level) - 1 + x_in;
     const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     // (all that follows from the node alone is requested at once)
     const SplitCand early = early_candidate(tb, x_in);
     const int2 sg = level == 0 ? make_int2(0, tb.n) : tb.seg[x];
     const TreeNode node = tb.nodes[x];
     const QuantCtl quant = *tb.quant;
-    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
-    constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, U = 8;
+    constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, COLS = LPR * FPL, U = 8;
     const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
-    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
-    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
+    // the part's columns and bins
+    const int *__restrict__ col_off = tb.feat_lds_off + ((fb << log_split) + part) * COLS;
+    const int blk0 = tb.blk_bin_begin[fb], off0 = col_off[0];
+    const int bin0 = blk0 + off0, nb = (part + 1 == 1 << log_split ? tb.blk_bin_begin[fb + 1] - blk0 : col_off[COLS]) - off0;
+    const int o0 = col_off[q * FPL] - off0, o1 = col_off[q * FPL + 1] - off0;
+    const int o2 = BIN16 ? 0 : col_off[q * FPL + 2] - off0, o3 = BIN16 ? 0 : col_off[q * FPL + 3] - off0;
+    const int row_shift = log_split + (LPR == 1 ? 2 : LPR == 2 ? 3 : LPR == 4 ? 4 : LPR == 8 ? 5 : 6);
     const int len = sg.y - sg.x, steps = (len + kSmallBlock - 1) / kSmallBlock;
     const int *__restrict__ ridx = tb.list(level);
     int row[STEPS];
@@ -540,7 +545,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     for (int i = threadIdx.x; i < nb; i += kSmallBlock) lds[i] = 0ull;
     const Picked best = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_pick, early);
     const bool splits = best.found && fabsf(best.c.score) > rt_eps;
-    const bool first = fb == 0 && threadIdx.x == 0;
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
     if (!splits) {
         if (first) {
             tb.node_nleft[x_in] = 0;
@@ -601,7 +606,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
             const bool left = (left_mask[k] >> lane & 1ull) != 0;
             const int at = left ? lefts : i - lefts;  // in the child's list
             if (left == build_left) s_rows[at] = (unsigned short)row[k];
-            if (fb == 0) {
+            if (blockIdx.x == 0) {
                 ridx_next[sg.x + (left ? at : nleft + at)] = row[k];
                 tb.nid[row[k]] = left ? node.lch_index : node.rch_index;
             }
@@ -612,7 +617,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     const int rows = max(1, min(m, quant.flush_rows));
     const int shift_g = item_shift(quant.gq_max, rows, 63 - h_bits), shift_h = quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits);
     const float scale_g = ldexpf(quant.scale_g, -shift_g), scale_h = ldexpf(quant.scale_h, -shift_h);
-    const bool word_lane = bins.gh_lane >= 0 && q == bins.gh_lane;
+    const bool word_lane = bins.gh_lane >= 0 && part * LPR + q == bins.gh_lane;
     const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
     for (int base = 0; base < m; base += RPS * U) {
         unsigned pk[U];
@@ -620,7 +625,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const unsigned r = s_rows[min(base + rsub + u * RPS, m - 1)];
-            pk[u] = *reinterpret_cast<const unsigned *>(blk + (r * (unsigned)(LPR * 4) + (unsigned)q * 4));
+            pk[u] = *reinterpret_cast<const unsigned *>(blk + ((r << row_shift) + (unsigned)(part * LPR + q) * 4));
             s[u] = gh[r];
         }
 #pragma unroll
@@ -712,7 +717,7 @@ __device__ __forceinline__ NodeRun locate_run(const TreeBuffers &tb, int level, 
     return out;
 }
 
-// Moderately many rows (split_hist_run): k_split_scatter and the next level's k_hist_dense in one launch. A workgroup owns a
+// Moderately many rows (split_hist_plan): k_split_scatter and the next level's k_hist_dense in one launch. A workgroup owns a
 // run of S partition items of a node and a feature block. The counts of the node's items tell it where the run's rows go and
 // which child has fewer rows; those of them that go there meet in LDS, and their histogram is a work item of the next level,
 // stored packed at the child's own scale (item_shift), so its sums are k_hist_dense's whatever the items. The first block
@@ -729,19 +734,23 @@ static_assert(kSplitHistMost * kPartChunk <= kHistFlushRows, "a run's packed sum
 static_assert(kRunHalves == 2 && kBlock * 8 == kPartChunk, "the mapping of k_split_count's decision bytes");
 template <int LPR, bool BIN16, bool GHW, int S>
 __global__ __launch_bounds__(kHistBlock) __attribute__((amdgpu_waves_per_eu(8)))
-void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level) {
+void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh, int level, int log_split, int lds_bins) {
     constexpr int R = S * kRunHalves;  // rows per thread
     constexpr int E = R * kRunWaves;   // counts of the run: one per round and wavefront
-    extern __shared__ unsigned long long lds[];  // the block's histogram, then the rows to add up
+    extern __shared__ unsigned long long lds[];  // the histogram, then the rows to add up
     __shared__ int s_cnt[E < 64 ? 64 : E];
     __shared__ int s_sum[2][kRunWaves];
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     gh += (size_t)blockIdx.z * tb.n;
-    int *s_rows = reinterpret_cast<int *>(lds + tb.max_block_bins);
-    const int fb = blockIdx.x, item = blockIdx.y;
+    int *s_rows = reinterpret_cast<int *>(lds + lds_bins);
+    const int fb = blockIdx.x >> log_split, part = blockIdx.x & ((1 << log_split) - 1), item = blockIdx.y;
     const NodeRun it = locate_run(tb, level, item, S * kPartChunk);
     if (it.x_in < 0) return;
-    const int bin0 = tb.blk_bin_begin[fb], nb = tb.blk_bin_begin[fb + 1] - bin0;
+    // the part's columns and bins
+    constexpr int FPL = BIN16 ? 2 : 4, COLS = LPR * FPL;
+    const int *__restrict__ col_off = tb.feat_lds_off + ((fb << log_split) + part) * COLS;
+    const int blk0 = tb.blk_bin_begin[fb], off0 = col_off[0];
+    const int bin0 = blk0 + off0, nb = (part + 1 == 1 << log_split ? tb.blk_bin_begin[fb + 1] - blk0 : col_off[COLS]) - off0;
     const int nl = 1 << level, x_in = it.x_in, x = nl - 1 + x_in;
     const int2 sg = it.seg;
     const int mine = item - it.first;  // of the node's runs
@@ -790,7 +799,7 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     // the child with fewer rows is built from them (ties: the left one, as hist_tree_builder_single.cu:466-467)
     const bool build_left = nleft <= nright;
     const int built = splits ? (build_left ? lch : rch) : -1;
-    if (fb == 0 && mine == 0 && threadIdx.x == 0) {
+    if (blockIdx.x == 0 && mine == 0 && threadIdx.x == 0) {
         tb.node_nleft[x_in] = nleft;
         tb.seg[lch] = splits ? make_int2(sg.x, sg.x + nleft) : make_int2(0, 0);
         tb.seg[rch] = splits ? make_int2(sg.x + nleft, sg.y) : make_int2(0, 0);
@@ -824,39 +833,43 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
         if (pb + i < pe) {
             const int at = left ? l : i - l;
             if (left == build_left) s_rows[at] = row[k];
-            if (fb == 0) ridx_next[left ? left_base + at : right_base + at] = row[k];
+            if (blockIdx.x == 0) ridx_next[left ? left_base + at : right_base + at] = row[k];
         }
     }
     __syncthreads();
     // The rows in batches: a batch's loads are issued together, the first ones before the scales are worked out.
-    constexpr int RPS = kHistBlock / LPR, FPL = BIN16 ? 2 : 4, U = LPR >= 16 ? 8 : 4;
+    constexpr int RPS = kHistBlock / LPR, U = LPR >= 16 ? 8 : 4;
     const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
+    const int row_shift = log_split + (LPR == 1 ? 2 : LPR == 2 ? 3 : LPR == 4 ? 4 : LPR == 8 ? 5 : 6);
     const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
     unsigned pk[U];
-    GHPair s[U];
+    GHPair s[U];  // (GHW: the word, in the first slot)
     auto load_rows = [&](int base) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            if (base + u * RPS >= m) break;  // (uniform)
             const unsigned r = (unsigned)s_rows[min(base + rsub + u * RPS, m - 1)];
-            pk[u] = *reinterpret_cast<const unsigned *>(blk + (r * (unsigned)(LPR * 4) + (unsigned)q * 4));
-            if (!GHW) s[u] = *reinterpret_cast<const GHPair *>(reinterpret_cast<const char *>(gh) + r * 8u);
+            const uint8_t *record = blk + (r << row_shift);
+            pk[u] = *reinterpret_cast<const unsigned *>(record + (unsigned)(part * LPR + q) * 4);
+            if (GHW) s[u].g = __uint_as_float(*reinterpret_cast<const unsigned *>(record + (unsigned)bins.gh_lane * 4));
+            else s[u] = *reinterpret_cast<const GHPair *>(reinterpret_cast<const char *>(gh) + r * 8u);
         }
     };
     if (m > 0) load_rows(0);
     const int h_bits = quant.h_bits;
     const int rows = max(1, min(min(nleft, nright), quant.flush_rows));
     const int shift_g = item_shift(quant.gq_max, rows, 63 - h_bits), shift_h = quant.h_integer ? 0 : item_shift(quant.hq_max, rows, h_bits);
-    if (fb == 0 && threadIdx.x == 0) tb.hitem_shift[item] = make_int2(shift_g, shift_h);
+    if (blockIdx.x == 0 && threadIdx.x == 0) tb.hitem_shift[item] = make_int2(shift_g, shift_h);
     const float scale_g = ldexpf(quant.scale_g, -shift_g), scale_h = ldexpf(quant.scale_h, -shift_h);
-    const int *fo = tb.feat_lds_off + fb * (LPR * FPL) + q * FPL;
-    const int o0 = fo[0], o1 = fo[1], o2 = BIN16 ? 0 : fo[2], o3 = BIN16 ? 0 : fo[3];
-    const bool word_lane = bins.gh_lane >= 0 && q == bins.gh_lane;
+    const int o0 = col_off[q * FPL] - off0, o1 = col_off[q * FPL + 1] - off0;
+    const int o2 = BIN16 ? 0 : col_off[q * FPL + 2] - off0, o3 = BIN16 ? 0 : col_off[q * FPL + 3] - off0;
+    const bool word_lane = bins.gh_lane >= 0 && part * LPR + q == bins.gh_lane;
     for (int base = 0; base < m; base += RPS * U) {
         if (base > 0) load_rows(base);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (base + u * RPS >= m) break;  // (uniform)
-            const GHPair sv = GHW ? pair_from_word(bins.gh_objective, last_lane_of_row<LPR>(pk[u])) : s[u];
+            const GHPair sv = GHW ? pair_from_word(bins.gh_objective, __float_as_uint(s[u].g)) : s[u];
             const unsigned v = base + rsub + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
             const long long gq = round_to_ll(sv.g * scale_g), hq = round_to_ll(fmaxf(sv.h, 0.f) * scale_h);
             const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
@@ -885,36 +898,46 @@ static int most_partition_items(const TreeBuffers &tb, int level) {
     return level == 0 ? std::max(1, (tb.n + kPartChunk - 1) / kPartChunk) : tb.n / kPartChunk + (1 << level);
 }
 
-static size_t split_hist_lds(const TreeBuffers &tb, int run) { return (size_t)tb.max_block_bins * 8 + (size_t)run * 4; }
+static size_t split_hist_lds(int lds_bins, int run) { return (size_t)lds_bins * 8 + (size_t)run * 4; }
 
-int split_hist_run(const TreeBuffers &tb, const DenseBins &bins, int n_class) {
-    if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return 0;
+SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, const int *part_bins, int n_class) {
+    SplitHistPlan plan;
+    if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return plan;
     for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2) {
-        const size_t stored = (size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class;
-        if (stored <= kSplitHistBytes && split_hist_lds(tb, run) + 4096 <= kLdsBytes) return run;
+        const long runs = (tb.n + run - 1) / run;
+        if ((size_t)runs * tb.n_bins * 8 * n_class > kSplitHistBytes) continue;
+        int parts = 0;  // (log2)
+        while (4 << (parts + 1) <= bins.W * bins.bin_bytes && (runs * bins.n_blocks * n_class << (parts + 1)) <= kSplitHistGroups) ++parts;
+        if (split_hist_lds(part_bins[parts], run) + 4096 > kLdsBytes) continue;
+        plan.run = run;
+        plan.log_split = parts;
+        plan.lds_bins = part_bins[parts];
+        return plan;
     }
-    return 0;
+    return plan;
 }
 
 template <int LPR, bool BIN16, bool GHW, int S>
-static void split_hist_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int n_class) {
+static void split_hist_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, const SplitHistPlan &plan,
+                              int n_class) {
     constexpr int run = S * kPartChunk;
-    const size_t lds = split_hist_lds(tb, run);
+    const size_t lds = split_hist_lds(plan.lds_bins, run);
     static LdsOptIn opt_in;
     if (lds > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_split_hist<LPR, BIN16, GHW, S>)});
-    const dim3 grid(bins.n_blocks, level == 0 ? (tb.n + run - 1) / run : tb.n / run + (1 << level), n_class);
-    k_split_hist<LPR, BIN16, GHW, S><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level);
+    const dim3 grid(bins.n_blocks << plan.log_split, level == 0 ? (tb.n + run - 1) / run : tb.n / run + (1 << level), n_class);
+    k_split_hist<LPR, BIN16, GHW, S><<<grid, kHistBlock, lds, s>>>(tb, bins, gh, level, plan.log_split, plan.lds_bins);
 }
 
 template <int LPR, bool BIN16, bool GHW>
-static void split_hist_run_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run, int n_class) {
-    if (run == kPartChunk) split_hist_launch<LPR, BIN16, GHW, 1>(s, tb, bins, gh, level, n_class);
-    else if (run == 2 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 2>(s, tb, bins, gh, level, n_class);
-    else if (run == 4 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 4>(s, tb, bins, gh, level, n_class);
-    else fatal("runs of %d rows", run);
+static void split_hist_run_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
+                                  const SplitHistPlan &plan, int n_class) {
+    if (plan.run == kPartChunk) split_hist_launch<LPR, BIN16, GHW, 1>(s, tb, bins, gh, level, plan, n_class);
+    else if (plan.run == 2 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 2>(s, tb, bins, gh, level, plan, n_class);
+    else if (plan.run == 4 * kPartChunk) split_hist_launch<LPR, BIN16, GHW, 4>(s, tb, bins, gh, level, plan, n_class);
+    else fatal("runs of %d rows", plan.run);
 }
 
-void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, int run,
+void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, const SplitHistPlan &plan,
                            float rt_eps, float lambda, int n_class) {
     const dim3 items(most_partition_items(tb, level), 1, n_class);
     const bool last = level == tb.depth - 1;
@@ -929,11 +952,11 @@ void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins
     if (last) return;
     const bool words = bins.gh_lane >= 0 && bins.gh_fresh;
 #define TGBM_SPLIT_HIST(LPR)                                                                                        \
-    if (bins.bin_bytes == 2) split_hist_run_launch<LPR, true, false>(s, tb, bins, gh, level, run, n_class);          \
-    else if (LPR >= 4 && words) split_hist_run_launch<LPR, false, (LPR >= 4)>(s, tb, bins, gh, level, run, n_class); \
-    else split_hist_run_launch<LPR, false, false>(s, tb, bins, gh, level, run, n_class);                             \
+    if (bins.bin_bytes == 2) split_hist_run_launch<LPR, true, false>(s, tb, bins, gh, level, plan, n_class);          \
+    else if (words) split_hist_run_launch<LPR, false, true>(s, tb, bins, gh, level, plan, n_class);                  \
+    else split_hist_run_launch<LPR, false, false>(s, tb, bins, gh, level, plan, n_class);                             \
     break
-    switch (bins.W * bins.bin_bytes) {  // bytes per row of a block
+    switch (bins.W * bins.bin_bytes >> plan.log_split) {  // bytes per row of a part
         case 4: TGBM_SPLIT_HIST(1);
         case 8: TGBM_SPLIT_HIST(2);
         case 16: TGBM_SPLIT_HIST(4);
@@ -976,46 +999,51 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
     if (tb.planned(level + 1)) k_plan_level<<<dim3(1, 1, n_class), kPlanBlock, 0, s>>>(tb, level + 1, tb.n_hpairs(level + 1));
 }
 
-static size_t small_lds(const TreeBuffers &tb) {
-    return (size_t)tb.max_block_bins * 8 + ((size_t)(tb.n / 2 + 1) * 2 + 7) / 8 * 8;
+static size_t small_lds(const TreeBuffers &tb, int lds_bins) {
+    return (size_t)lds_bins * 8 + ((size_t)(tb.n / 2 + 1) * 2 + 7) / 8 * 8;
 }
 
 // One workgroup adds up to half of the rows to one feature block's histogram (about five bins per clock): beyond 8192 rows x
 // 32 columns that takes longer at the first levels than the launches that are saved.
 bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins) {
     return tb.n <= kSmallRows && tb.depth <= kSmallDepth && (long)(tb.n / 2) * std::min(bins.W, bins.n_cols) <= 1l << 18 &&
-           small_lds(tb) + 4096 <= kLdsBytes;
+           small_lds(tb, tb.max_block_bins) + 4096 <= kLdsBytes;
 }
 
 template <int LPR, bool BIN16, int STEPS>
 static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                               float rt_eps, float lambda, int n_class) {
-    const size_t lds = small_lds(tb);
+                               float rt_eps, float lambda, int log_split, int lds_bins, int n_class) {
+    const size_t lds = small_lds(tb, lds_bins);
     static LdsOptIn opt_in;
     if (lds > 48 * 1024)  // (with the kernel's own tables more than the default window)
         opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16, STEPS>)});
-    k_small_level<LPR, BIN16, STEPS><<<dim3(bins.n_blocks, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda);
+    k_small_level<LPR, BIN16, STEPS><<<dim3(bins.n_blocks << log_split, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda,
+                                                                                                                          log_split, lds_bins);
 }
 
 // (the code of steps that no node of the data can have is not only skipped but left out, see k_small_level)
 template <int LPR, bool BIN16>
 static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                              float rt_eps, float lambda, int n_class) {
+                              float rt_eps, float lambda, int log_split, int lds_bins, int n_class) {
     const int steps = (tb.n + kSmallBlock - 1) / kSmallBlock;
-    if (steps <= 2) small_level_launch<LPR, BIN16, 2>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
-    else if (steps <= 4) small_level_launch<LPR, BIN16, 4>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
-    else if (steps <= 8) small_level_launch<LPR, BIN16, 8>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
-    else small_level_launch<LPR, BIN16, kSmallSteps>(s, tb, bins, gh, level, rt_eps, lambda, n_class);
+    if (steps <= 2) small_level_launch<LPR, BIN16, 2>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
+    else if (steps <= 4) small_level_launch<LPR, BIN16, 4>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
+    else if (steps <= 8) small_level_launch<LPR, BIN16, 8>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
+    else small_level_launch<LPR, BIN16, kSmallSteps>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
 }
 
 void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
-                        float lambda, int n_class) {
+                        float lambda, const int *part_bins, int n_class) {
     if (level == tb.depth - 1) return;
+    // (up to a workgroup per CU a block's columns are shared out, see kSplitHistGroups)
+    int log_split = 0;
+    while (4 << (log_split + 1) <= bins.W * bins.bin_bytes && ((long)bins.n_blocks * n_class << (level + log_split + 1)) <= kSplitHistGroups) ++log_split;
+    const int lds_bins = part_bins[log_split];
 #define TGBM_SMALL_LEVEL(LPR)                                                                               \
-    if (bins.bin_bytes == 2) small_level_steps<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, n_class); \
-    else small_level_steps<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, n_class);                    \
+    if (bins.bin_bytes == 2) small_level_steps<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class); \
+    else small_level_steps<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);                    \
     break
-    switch (bins.W * bins.bin_bytes) {  // bytes per row of a block
+    switch (bins.W * bins.bin_bytes >> log_split) {  // bytes per row of a part
         case 4: TGBM_SMALL_LEVEL(1);
         case 8: TGBM_SMALL_LEVEL(2);
         case 16: TGBM_SMALL_LEVEL(4);

@@ -177,8 +177,9 @@ class Trainer {
     bool in_boost_ = false;
     bool small_ok_ = false;          // inside boost() the levels go through launch_small_level
     bool small() const { return in_boost_ && small_ok_; }
-    int run_rows_ = 0;               // inside boost() the levels go through launch_partition_hist, runs of so many rows
-    int run() const { return in_boost_ && !small_ok_ ? run_rows_ : 0; }
+    int part_bins_[5] = {0};         // most bins of a part of a feature block in 1, 2, 4, 8, 16 parts
+    SplitHistPlan run_plan_;         // inside boost() the levels go through launch_partition_hist, runs of so many rows
+    int run() const { return in_boost_ && !small_ok_ ? run_plan_.run : 0; }
     bool maps_rows() const { return small() || run() > 0; }  // a tree's rows end in tb.nid: launch_map_end
     int lookup_level_ = -1;          // level whose split nodes have not been partitioned into row lists yet
     bool next_round_ready_ = false;  // d_gh_ and the root statistics already belong to the next round

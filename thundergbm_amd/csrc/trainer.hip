@@ -490,7 +490,7 @@ void Trainer::alloc_tree_buffers() {
     tb.max_level_nodes = max_level_nodes;
     tb.target_hitems = std::min(512, std::max(4, 512 / bins_.n_blocks));  // ~2 resident workgroups per CU
     tb.max_hitems = tb.target_hitems + max_pairs + 1;
-    // The runs of split_hist_run: what they store, packed, in histograms of `partial`'s size.
+    // The runs of split_hist_plan: what they store, packed, in histograms of `partial`'s size.
     const int max_runs = n_ < kSplitHistRows ? n_ / kPartChunk + max_level_nodes / 2 + 2 : 0;
     const size_t run_slots = max_runs == 0 ? 0 : kSplitHistBytes / sizeof(longlong2) / (size_t)n_bins_ + (size_t)max_level_nodes / 4 + 2;
     tb.max_pitems = n_ / kPartChunk + max_level_nodes + 1;
@@ -665,8 +665,17 @@ void Trainer::alloc_tree_buffers() {
         max_block_bins = std::max(max_block_bins, blk_begin[b + 1] - blk_begin[b]);
         for (int j = 0; j < W; ++j) {
             int c = b * W + j;
-            feat_off[(size_t)b * W + j] = c < n_cols ? cbb[c] - blk_begin[b] : 0;
+            feat_off[(size_t)b * W + j] = (c < n_cols ? cbb[c] : blk_begin[b + 1]) - blk_begin[b];
         }
+    }
+    for (int k = 0; k < 5; ++k) {  // (parts of whole dwords of the records)
+        const int cols = W >> k;
+        if (sparse_ || cols * bins_.bin_bytes < 4) break;
+        for (int b = 0; b < nb; ++b)
+            for (int c = 0; c < W; c += cols) {
+                const int end = c + cols < W ? feat_off[(size_t)b * W + c + cols] : blk_begin[b + 1] - blk_begin[b];
+                part_bins_[k] = std::max(part_bins_[k], end - feat_off[(size_t)b * W + c]);
+            }
     }
     TGBM_CHECK(sparse_ || (size_t)max_block_bins * 8 <= 160 * 1024, "feature block histogram exceeds the LDS");
     tb.max_block_bins = max_block_bins;
@@ -682,11 +691,11 @@ void Trainer::alloc_tree_buffers() {
     small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb, bins_) && !(small_env != nullptr && std::string(small_env) == "0");
     const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
     if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
-        run_rows_ = split_hist_run(tb, bins_, n_sets_);
+        run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
     // What target_hitems then plans is the root: a workgroup per CU, each stores a histogram and the atomics of a CU take as long
     // for two (500 k x 28: histogram 15.6 -> 14.6 us, sums of the items 12.6 -> 8.1; 128 items: 19 and 5.8), unless their
     // packed sums would have to be drained.
-    if (run_rows_ > 0 && (long)n_ * n_sets_ <= 256l * kHistFlushRows) tb.target_hitems = std::max(4, tb.target_hitems / 2);
+    if (run_plan_.run > 0 && (long)n_ * n_sets_ <= 256l * kHistFlushRows) tb.target_hitems = std::max(4, tb.target_hitems / 2);
     model_cap_trees_ = std::max(1, param_.n_trees) * param_.tree_per_rounds;
     d_model_ = dalloc<TreeNode>((size_t)model_cap_trees_ * tb.n_nodes);
     d_metric_ = dalloc<float>((size_t)std::max(1, param_.n_trees));
@@ -1088,12 +1097,12 @@ void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level,
     } else if (sparse_)
         launch_partition_csr(stream_, tb, csr_, level, n_class);
     else if (small())
-        launch_small_level(stream_, tb, bins_, gh, level, param_.rt_eps, param_.lambda, n_class);
+        launch_small_level(stream_, tb, bins_, gh, level, param_.rt_eps, param_.lambda, part_bins_, n_class);
     else if (run() > 0) {
         DenseBins b = bins_;
         b.gh_fresh = gh_records_fresh_ && n_class == 1 && gh == d_gh_;
         b.gh_objective = objective_;
-        launch_partition_hist(stream_, tb, b, gh, level, run(), param_.rt_eps, param_.lambda, n_class);
+        launch_partition_hist(stream_, tb, b, gh, level, run_plan_, param_.rt_eps, param_.lambda, n_class);
     } else
         launch_partition_dense(stream_, tb, bins_, level, update_with_partition(level), param_.rt_eps, param_.lambda, n_class);
     mark(PH_PARTITION, level);
