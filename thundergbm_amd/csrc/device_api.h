@@ -104,8 +104,10 @@ constexpr int kRootParts = 512;     // parts of the rows whose sums add up to th
 // 500 k x 2000 regression builds a tree in 1.90 instead of 2.00 ms.
 constexpr int kHistFlushRows = 8192;
 constexpr int kHistFlushRowsInt = 32768;
-// Data of so few rows is trained on by the launches of launch_small_level, trees of so many levels at most.
-constexpr int kSmallRows = 16384;
+// Data of so few rows is trained on by the launches of launch_small_level, trees of so many levels at most. ms a tree with
+// them and with launch_partition_hist, 28 columns and depth 8: 4000 rows 0.142 and 0.152, 8000 0.156 and 0.155, 16 000 0.183 and 0.158;
+// 8 columns and depth 6: 0.099 and 0.105, 0.107 and 0.104, 0.126 and 0.108.
+constexpr int kSmallRows = 8192;
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallDepth = 10;
 constexpr int kRowBlock = 4096;    // rows owned by one workgroup of the row-ordered passes and reductions
@@ -490,7 +492,7 @@ void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins
                            float rt_eps, float lambda, int n_class = 1);
 // Dense layout, few rows: the level's splits, the children's lists and the histograms of the next level's built nodes in one
 // launch. The split search of the next level then derives the siblings (launch_eval_split with derive).
-bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins);
+bool small_levels_fit(const TreeBuffers &tb);
 void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
                         float lambda, const int *part_bins, int n_class = 1);
 // The end of a tree whose rows' nodes are in tb.nid (lookup_level >= 0: split nodes of that level still hold the rows of their

@@ -1003,11 +1003,8 @@ static size_t small_lds(const TreeBuffers &tb, int lds_bins) {
     return (size_t)lds_bins * 8 + ((size_t)(tb.n / 2 + 1) * 2 + 7) / 8 * 8;
 }
 
-// One workgroup adds up to half of the rows to one feature block's histogram (about five bins per clock): beyond 8192 rows x
-// 32 columns that takes longer at the first levels than the launches that are saved.
-bool small_levels_fit(const TreeBuffers &tb, const DenseBins &bins) {
-    return tb.n <= kSmallRows && tb.depth <= kSmallDepth && (long)(tb.n / 2) * std::min(bins.W, bins.n_cols) <= 1l << 18 &&
-           small_lds(tb, tb.max_block_bins) + 4096 <= kLdsBytes;
+bool small_levels_fit(const TreeBuffers &tb) {
+    return tb.n <= kSmallRows && tb.depth <= kSmallDepth && small_lds(tb, tb.max_block_bins) + 4096 <= kLdsBytes;
 }
 
 template <int LPR, bool BIN16, int STEPS>
@@ -1028,7 +1025,6 @@ static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseB
     const int steps = (tb.n + kSmallBlock - 1) / kSmallBlock;
     if (steps <= 2) small_level_launch<LPR, BIN16, 2>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
     else if (steps <= 4) small_level_launch<LPR, BIN16, 4>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
-    else if (steps <= 8) small_level_launch<LPR, BIN16, 8>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
     else small_level_launch<LPR, BIN16, kSmallSteps>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
 }
 

@@ -688,7 +688,7 @@ void Trainer::alloc_tree_buffers() {
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors above go out of scope
 
     const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
-    small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb, bins_) && !(small_env != nullptr && std::string(small_env) == "0");
+    small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb) && !(small_env != nullptr && std::string(small_env) == "0");
     const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
     if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
         run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
