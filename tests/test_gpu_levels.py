@@ -1,5 +1,6 @@
 """The level kernels of the dense layout (thundergbm_amd/csrc/level_kernels.hip): what boost() runs in fewer launches
 against the stages one by one, at the edges of the work items and of the nodes a workgroup looks at together."""
+import ctypes
 import os
 import sys
 
@@ -102,5 +103,35 @@ def test_lists_and_histograms_in_one_launch(n, F, depth, bins, objective, missin
                       objective=objective)
         s.boost(3)
         out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), s.metric_log().tobytes()))
+        s.close()
+    assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("n,depth,bins,objective,rate", [
+    (1_200, 6, 1024, "reg:linear", 1.0), (8_000, 7, 1024, "binary:logistic", 1.0), (8_192, 5, 513, "reg:linear", 0.5),
+    (5_000, 6, 1500, "reg:linear", 1.0), (6_000, 4, 300, "multi:softmax", 1.0)])
+def test_merge_and_search_of_wide_features_in_one_launch(n, depth, bins, objective, rate, monkeypatch):
+    """k_merge_eval_wide (TGBM_SMALL=0) against k_eval_split_wide after k_small_level: columns of 1 .. `bins` values, 0 to 4
+    quarters of 256 bins full or with a remainder, ties between columns, features past the one launch's bins (1500)."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    counts = [c for c in (1, 2, 255, 256, 257, 512, 513, 768, 1023, 1024, 1025, 1500) if c <= bins] + [256]
+    X = np.stack([rng.permutation(np.arange(n) % c) + 1 for c in counts], 1).astype(np.float32)
+    X[:, -1] = X[:, counts.index(256)]
+    X[rng.random(X.shape) < 0.1] = 0
+    z = X[:, 2] / 255 + np.abs(X[:, -2] / counts[-2] - 0.5) + 0.3 * rng.standard_normal(n)
+    y = z if objective == "reg:linear" else (np.digitize(z, [0.7, 1.0]) if objective.startswith("multi") else z > 0.8)
+    val, rp, col = D.dense_to_csr(X)
+    out = []
+    for small in ("1", "0"):
+        monkeypatch.setenv("TGBM_SMALL", small)
+        ctypes.CDLL(None).srand(3)
+        s = T.Session(val, rp, col, np.asarray(y, np.float32), depth=depth, n_trees=3, learning_rate=0.5, max_num_bin=bins,
+                      objective=objective)
+        assert s.info("wide_eval") == 1
+        if rate < 1:
+            s.set_option("column_sampling_rate", rate)
+        s.boost(3)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), np.round(s.metric_log(), 5).tobytes()))
         s.close()
     assert out[0] == out[1]

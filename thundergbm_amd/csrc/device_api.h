@@ -93,6 +93,7 @@ constexpr size_t kSplitHistBytes = 13 << 20;
 constexpr int kSplitHistGroups = 256;
 // Dense layout: up to so many pairs (nodes, where single nodes are built) in a level every workgroup plans for itself.
 constexpr int kUnplannedPairs = 256;
+constexpr int kMergeWideBins = 1024; // bins of a feature that k_merge_eval_wide holds at most
 constexpr int kEvalPackBins = 256; // bins scanned by one wavefront in split finding (4 per lane)
 constexpr int kCsrHeadBins = 4864;  // head slots of the sparse histogram: 2 x 8 bytes each, two workgroups per CU
 constexpr int kRootParts = 512;     // parts of the rows whose sums add up to the root's (the root's work items at most)
@@ -472,6 +473,9 @@ void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mc
 // Split search with one workgroup per (feature, node): any number of bins per feature (n_packs = F candidates per node)
 void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class = 1,
                             bool store_sibling = true, bool derive = false, bool root_of_rows = false);
+// launch_hist_merge and launch_eval_split_wide below the root: one launch where the features' bins and the pairs' items allow it.
+void launch_merge_eval_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run,
+                            int max_feature_bins);
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class = 1);
 // Dense layout: the rows of a level's split nodes move into the children's lists. update: the nodes' best candidates have
 // not been applied to the tree yet (launch_best_update); it happens here.

@@ -612,6 +612,7 @@ void Trainer::alloc_tree_buffers() {
     for (int f = 0; f < F_; ++f) {
         int k = h_cut_row_ptr_[f + 1] - h_cut_row_ptr_[f];
         if (k == 0) continue;
+        max_feature_bins_ = std::max(max_feature_bins_, k);
         TGBM_CHECK(k <= kEvalPackBins || wide_eval_, "feature %d has %d cut points, more than %d", f, k, kEvalPackBins);
         if (cur + k > kEvalPackBins) {
             pack_begin.push_back(h_cut_row_ptr_[f]);
@@ -1035,7 +1036,8 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     if (!sparse_pass_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
         const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0;
-        if (!sparse_ && !derive && !fused) launch_hist_merge(stream_, tb, level, n_class);
+        const bool fused_wide = !sparse_ && !derive && wide_eval_ && hist_cap_level_ < 0 && level > 0;
+        if (!sparse_ && !derive && !fused && !fused_wide) launch_hist_merge(stream_, tb, level, n_class);
         if (level == 0 && !fused && !(wide_eval_ && sum_rows)) launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         mark(PH_MERGE, level);
         // inside boost() nobody looks at the last level's derived histograms (the stage-wise API keeps them); the
@@ -1043,6 +1045,9 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
         if (fused)
             launch_merge_eval(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                               !(in_boost_ && level == param_.depth - 1), run());
+        else if (fused_wide)
+            launch_merge_eval_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
+                                   !(in_boost_ && level == param_.depth - 1), run(), max_feature_bins_);
         else if (wide_eval_)
             launch_eval_split_wide(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                                    !(in_boost_ && level == param_.depth - 1), derive, sum_rows);

@@ -1245,6 +1245,51 @@ __global__ __launch_bounds__(kBlock) void k_eval_split(TreeBuffers tb_all, int l
     search_pack(tb, pm, s_v[w], x_in, pack, active, b_begin, b_end, S, inv_g, inv_h, mcw, lambda);
 }
 
+// The sums of `count` <= kEvalPackBins bins from `first` over the work items it0, it0 + step, .. below ie of a pair, four per lane
+// of a wavefront (past the end: the last one again, so that all loads of an item are issued at once).
+__device__ __forceinline__ void add_items_of_pair(const TreeBuffers &tb, int level, int it0, int ie, int step, int first, int count,
+                                                  long long (&g)[4], long long (&h)[4]) {
+    // every item counted at its own scale (item_shift): shift its sums to the tree's
+    const int2 *__restrict__ shift = tb.hitem_shift;
+    const bool packed = tb.ctl[level].hchunk <= tb.quant->flush_rows;  // 8-byte partials (see k_hist_dense)
+    const int n_bins = tb.n_bins, h_bits = tb.quant->h_bits;
+    const unsigned long long h_mask = (1ull << h_bits) - 1ull;
+    int at[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        at[j] = first + min(j * 64 + lane_id(), count - 1);
+        g[j] = h[j] = 0;
+    }
+    if (packed) {
+        const unsigned long long *__restrict__ from = reinterpret_cast<const unsigned long long *>(tb.partial);
+#pragma unroll 2
+        for (int it = it0; it < ie; it += step) {
+            unsigned long long t[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[j] = from[(size_t)it * n_bins + at[j]];
+            const int2 sh = shift[it];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const unsigned long long lo = t[j] & h_mask;
+                g[j] += ((long long)(t[j] - lo) >> h_bits) << sh.x;
+                h[j] += (long long)lo << sh.y;
+            }
+        }
+    } else {
+        for (int it = it0; it < ie; it += step) {
+            longlong2 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = tb.partial[(size_t)it * n_bins + at[j]];
+            const int2 sh = shift[it];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                g[j] += v[j].x << sh.x;
+                h[j] += v[j].y << sh.y;
+            }
+        }
+    }
+}
+
 // k_hist_merge and k_eval_split of a level in one launch: a workgroup owns a pack of a sibling pair. Its wavefronts share
 // out the pair's work items, the sums meet in LDS, parent - built gives the sibling, one wavefront searches the built node
 // and one its sibling. The histograms are stored for the next level only (not at a tree's last one, which holds half of a
@@ -1277,49 +1322,7 @@ __global__ __launch_bounds__(NW * 64) void k_merge_eval(TreeBuffers tb_all, int 
     GHPair S{0, 0};
     if (!ROOT) S = tb.nodes[w == 0 ? built : sibling].sum_gh_pair;
     const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
-    // every item counted at its own scale (item_shift): shift its sums to the tree's
-    const int2 *__restrict__ shift = tb.hitem_shift;
-    const bool packed = tb.ctl[level].hchunk <= tb.quant->flush_rows;  // 8-byte partials (see k_hist_dense)
-    const int h_bits = tb.quant->h_bits;
-    const unsigned long long h_mask = (1ull << h_bits) - 1ull;
-    // the bins [first, first + count) of all items that are this wavefront's turn, four per lane (past the end: the last
-    // one again, so that all loads of an item are issued at once)
-    auto add_items = [&](int first, int count, long long(&g)[4], long long(&h)[4]) {
-        int at[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            at[j] = first + min(j * 64 + lane, count - 1);
-            g[j] = h[j] = 0;
-        }
-        if (packed) {
-            const unsigned long long *__restrict__ from = reinterpret_cast<const unsigned long long *>(tb.partial);
-#pragma unroll 2
-            for (int it = ib + w; it < ie; it += NW) {
-                unsigned long long t[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) t[j] = from[(size_t)it * n_bins + at[j]];
-                const int2 sh = shift[it];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const unsigned long long lo = t[j] & h_mask;
-                    g[j] += ((long long)(t[j] - lo) >> h_bits) << sh.x;
-                    h[j] += (long long)lo << sh.y;
-                }
-            }
-        } else {
-            for (int it = ib + w; it < ie; it += NW) {
-                longlong2 v[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = tb.partial[(size_t)it * n_bins + at[j]];
-                const int2 sh = shift[it];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    g[j] += v[j].x << sh.x;
-                    h[j] += v[j].y << sh.y;
-                }
-            }
-        }
-    };
+    auto add_items = [&](int first, int count, long long(&g)[4], long long(&h)[4]) { add_items_of_pair(tb, level, ib + w, ie, NW, first, count, g, h); };
     if constexpr (ROOT == kRootOfBins) {
         const int b0 = tb.cut_row_ptr[tb.complete_feature], kf = tb.cut_row_ptr[tb.complete_feature + 1] - b0;
         long long g[4], h[4], G = 0, H = 0;
@@ -1523,6 +1526,143 @@ __global__ __launch_bounds__(kBlock) void k_eval_split_wide(TreeBuffers tb_all, 
         c.bin = best_idx - cb;
         *out = c;
     }
+}
+
+// k_merge_eval for features of more bins than a wavefront holds, up to kMergeWideBins: a workgroup owns a feature and a sibling
+// pair. Quarters of the bins and groups of the work items are shared out over its wavefronts, then one half of them searches
+// the built node and the other one its sibling, consecutive bins per thread, as k_eval_split_wide does (same candidates, gains
+// and tie rule). Bound by its chain of steps where a level has few pairs, by the memory at deep ones (77 777 x 37, level 6: 65 MB
+// of items, parents and stored histograms in 14 us). ms a tree of 1024 bins, two launches -> this one: 20 k x 28, depth 8 0.317 -> 0.217,
+// 500 k x 28 0.496 -> 0.408, 50 k x 200, depth 6 0.332 -> 0.251, 2 M x 28 0.669 -> 0.571.
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void k_merge_eval_wide(TreeBuffers tb_all, int level, float mcw, float lambda, bool store) {
+#pragma clang fp contract(off)
+    constexpr int kHalf = NW / 2, V = kMergeWideBins / (kHalf * 64), C = kMergeWideBins / (NW * 64);
+    __shared__ longlong2 s_sum[NW * kEvalPackBins];
+    __shared__ longlong2 s_tot[NW];
+    __shared__ float s_abs[NW];
+    static_assert(2 * kMergeWideBins <= NW * kEvalPackBins && NW * 64 <= kMergeWideBins, "both nodes' bins");
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int p = blockIdx.y, f = blockIdx.x;
+    const int built = tb.hpair_built[p];
+    if (built < 0) return;  // (nobody reads the candidates of nodes that do not exist)
+    const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
+    const int off = (1 << level) - 1, n_bins = tb.n_bins;
+    const int cb = tb.cut_row_ptr[f], kf = tb.cut_row_ptr[f + 1] - cb;
+    const int sibling = (built & 1) ? built + 1 : built - 1;
+    const int half = w >= kHalf ? 1 : 0, wn = w - half * kHalf, x_in = (half ? sibling : built) - off;
+    if (kf == 0) {
+        if (lane == 0 && wn == 0) tb.cand[(size_t)x_in * tb.n_packs + f].index = 0x7fffffff;  // a feature without bins has no candidate
+        return;
+    }
+    const int ib = tb.hpair_begin[p], ie = tb.hpair_begin[p + 1];
+    longlong2 parent[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        parent[c] = tb.hist(level + 1)[(size_t)p * n_bins + cb + min(c * NW * 64 + (int)threadIdx.x, kf - 1)];
+    const GHPair S = tb.nodes[off + x_in].sum_gh_pair;
+    const double inv_g = tb.quant->inv_g, inv_h = tb.quant->inv_h;
+    const bool ign = tb.ignored != nullptr && tb.ignored[f] != 0;
+    const int parts = (kf + kEvalPackBins - 1) / kEvalPackBins, groups = NW / parts;
+    {
+        const int group = w / parts, part = w - group * parts;
+        if (group < groups) {
+            long long g[4], h[4];
+            add_items_of_pair(tb, level, ib + group, ie, groups, cb + part * kEvalPackBins, min(kEvalPackBins, kf - part * kEvalPackBins), g, h);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s_sum[w * kEvalPackBins + j * 64 + lane] = make_longlong2(g[j], h[j]);
+        }
+    }
+    __syncthreads();
+    longlong2 sum[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int b = c * NW * 64 + (int)threadIdx.x;
+        sum[c] = make_longlong2(0, 0);
+        if (b >= kf) continue;
+        for (int i = 0; i < groups; ++i) {
+            const longlong2 v = s_sum[i * parts * kEvalPackBins + b];
+            sum[c].x += v.x;
+            sum[c].y += v.y;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int b = c * NW * 64 + (int)threadIdx.x;
+        const longlong2 other = make_longlong2(parent[c].x - sum[c].x, parent[c].y - sum[c].y);
+        const bool on = b < kf;
+        s_sum[b] = on ? sum[c] : make_longlong2(0, 0);
+        s_sum[kMergeWideBins + b] = on ? other : make_longlong2(0, 0);
+        if (store && on) {
+            tb.hist(level)[(size_t)(built - off) * n_bins + cb + b] = sum[c];
+            tb.hist(level)[(size_t)(sibling - off) * n_bins + cb + b] = other;
+        }
+    }
+    __syncthreads();
+    const int at = (wn * 64 + lane) * V;  // the thread's bins of its half's node
+    long long exg[V], exh[V], g = 0, h = 0;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const longlong2 v = s_sum[half * kMergeWideBins + at + j];
+        exg[j] = g;
+        exh[j] = h;
+        g += v.x;
+        h += v.y;
+    }
+    long long upg = g, uph = h;
+    wave_scan_pair(upg, uph);
+    if (lane == 63) s_tot[w] = make_longlong2(upg, uph);
+    __syncthreads();
+    long long tg = 0, th = 0, below_g = upg - g, below_h = uph - h;
+#pragma unroll
+    for (int i = 0; i < kHalf; ++i) {
+        const longlong2 v = s_tot[half * kHalf + i];
+        tg += v.x;
+        th += v.y;
+        below_g += i < wn ? v.x : 0;
+        below_h += i < wn ? v.y : 0;
+    }
+    const GHPair m{S.g - scaled_float(tg, inv_g), S.h - scaled_float(th, inv_h)};
+    const float fterm = (S.g * S.g) / (S.h + lambda);
+    float best = -1.f, best_score = 0.f;
+    GHPair best_left{0, 0};
+    int which = 0;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const GHPair l{scaled_float(below_g + exg[j], inv_g), scaled_float(below_h + exh[j], inv_h)};
+        const float gr = split_gain_select(S, fterm, l, mcw, lambda);
+        const float gl = split_gain_select(S, fterm, GHPair{l.g + m.g, l.h + m.h}, mcw, lambda);
+        const float score = ign ? 0.f : (gl > gr ? gl : -gr);  // column sampling: hist_tree_builder_single.cu:304 / :663
+        const float a = at + j < kf ? fabsf(score) : -1.f;
+        const bool better = a > best;
+        which = better ? j : which;
+        best_score = better ? score : best_score;
+        best_left.g = better ? l.g : best_left.g;
+        best_left.h = better ? l.h : best_left.h;
+        best = better ? a : best;
+    }
+    // larger |score| wins, ties go to the smaller bin index (hist_tree_builder_single.cu:330-335): the first wavefront's, the first lane's
+    const float win = wave_max_f(best);
+    if (lane == 0) s_abs[w] = win;
+    __syncthreads();
+    int winner = 0;
+    float top = s_abs[half * kHalf];
+#pragma unroll
+    for (int i = 1; i < kHalf; ++i) {
+        const float a = s_abs[half * kHalf + i];
+        winner = a > top ? i : winner;
+        top = fmaxf(top, a);
+    }
+    if (wn != winner || lane != __ffsll((long long)__ballot(best == win)) - 1) return;
+    SplitCand c;
+    c.score = best_score;
+    c.index = best < 0.f ? 0x7fffffff : cb + at + which;
+    c.miss = m;
+    c.left = best_left;
+    c.feature = f;
+    c.bin = at + which;
+    tb.cand[(size_t)x_in * tb.n_packs + f] = c;
 }
 
 // Per node: reduce the wavefront candidates, fill the split record (hist_tree_builder_single.cu
@@ -2653,12 +2793,17 @@ void launch_eval_split(hipStream_t s, const TreeBuffers &tb, int level, float mc
     else k_eval_split<false><<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, true);
 }
 
+// (as many work items as the level can have, see hist_dense_launch)
+static int items_of_level(const TreeBuffers &tb, int level, int run) {
+    const int n_pairs = tb.n_hpairs(level);
+    if (run > 0 && level > 0) return tb.n / run + n_pairs;
+    return std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
+}
+
 void launch_merge_eval(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run) {
     const int n_pairs = tb.n_hpairs(level);
     const dim3 grid(tb.n_packs, n_pairs, n_class);
-    // (as many items as the level can have, see hist_dense_launch)
-    const int items = run > 0 && level > 0 ? tb.n / run + n_pairs
-                                           : std::min(tb.target_hitems, (level == 0 ? tb.n : tb.n / 2) / kHistMinChunk + n_pairs);
+    const int items = items_of_level(tb, level, run);
     if (level == 0) {
         // One workgroup per pack: with hundreds of items two launches that spread them over the chip are faster (512 items of
         // 28 packs: 12 + 9 instead of 43 us; 245: 8 + 8 and 24; 23 items of 700 packs: 18 instead of 16 + 15).
@@ -2688,6 +2833,18 @@ void launch_eval_split_wide(hipStream_t s, const TreeBuffers &tb, int level, flo
                             bool store_sibling, bool derive, bool root_of_rows) {
     dim3 grid(tb.F, tb.nodes_served(level), n_class);
     k_eval_split_wide<<<grid, kBlock, 0, s>>>(tb, level, mcw, lambda, store_sibling, derive || tb.sparse, root_of_rows);
+}
+
+void launch_merge_eval_wide(hipStream_t s, const TreeBuffers &tb, int level, float mcw, float lambda, int n_class, bool store, int run,
+                            int max_feature_bins) {
+    const int n_pairs = tb.n_hpairs(level), per_pair = items_of_level(tb, level, run) / n_pairs;
+    const dim3 grid(tb.F, n_pairs, n_class);
+    // (many items of few pairs are for launches that spread them over the chip, see launch_merge_eval's root)
+    if (max_feature_bins > kMergeWideBins || per_pair > 64) {
+        launch_hist_merge(s, tb, level, n_class);
+        launch_eval_split_wide(s, tb, level, mcw, lambda, n_class, store, false, false);
+    } else if (per_pair > 8) k_merge_eval_wide<16><<<grid, 1024, 0, s>>>(tb, level, mcw, lambda, store);
+    else k_merge_eval_wide<8><<<grid, 512, 0, s>>>(tb, level, mcw, lambda, store);
 }
 
 void launch_best_update(hipStream_t s, const TreeBuffers &tb, int level, float rt_eps, float lambda, int n_class) {
