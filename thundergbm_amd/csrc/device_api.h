@@ -642,6 +642,9 @@ class UploadSet {
     // an array that another thread is still making: source() waits for it; it is sent last
     void add_late(void *dst, size_t bytes, std::function<const void *()> source);
     void send(hipStream_t s);  // once
+    // The arrays one after the other instead. arrived(j) is called for the j-th one in their order, by one thread at a time, as
+    // soon as what s gets next runs after its copy.
+    void send_in_order(hipStream_t s, const std::function<void(size_t)> &arrived);
 
    private:
     struct Job {
@@ -651,7 +654,7 @@ class UploadSet {
         std::function<void(char *to, size_t offset, size_t length)> fill;  // writes bytes [offset, offset + length) of them
         bool late;
     };
-    friend void send_jobs(hipStream_t s, const std::vector<Job> &jobs, int threads);
+    friend void send_jobs(hipStream_t s, const std::vector<Job> &jobs, int threads, const std::function<void(size_t)> *arrived);
     struct Columns {
         int *dst;
         const int *src;
@@ -659,12 +662,17 @@ class UploadSet {
         int width;  // bytes of the narrow form
         void *narrow;
         std::shared_ptr<std::atomic<bool>> fits;
+        size_t job;
     };
+    static void widen(hipStream_t s, const Columns &c);
+    void release_narrow(hipStream_t s);
     template <typename Narrow>
     bool add_narrow(int *dst, const int *src, size_t count);
     std::vector<Job> jobs_;
     std::vector<Columns> columns_;
 };
+// Device -> pageable host memory after what is queued on s; the bytes are there when the call returns.
+void download_large(hipStream_t s, void *dst, const void *src, size_t bytes);
 // The conversion alone, for arrays that the device reads from host memory.
 void doubles_to_floats(float *to, const double *from, size_t count);
 // A pinned block of kPinnedBytes that the device can read and write directly; kept for later calls.

@@ -139,6 +139,13 @@ std::shared_ptr<const DeviceModel> device_model(hipStream_t s, tgbm_model &model
     return model.on_device;
 }
 
+// Bytes of a slice of rows on their way to the device, see score(). Sparse rows: a walk of k_score_group takes about as long as
+// the slice's values take over PCIe, so an eighth of a call's values is left to walk when the last ones are there (500 k rows
+// of 35 values, 100 trees: 5.4 ms in slices of 64 MB, 4.7 of 32, 4.4 of 16 with every slice a send of its own, 4.3 in one
+// send that has the columns in front). Dense rows: k_score_rows needs many workgroups, slices below 64 MB cost more than they hide
+// (200 k x 28, 200 trees: 203 us in one launch, 147 for 75 k of the rows).
+constexpr size_t kLeastSlice = (size_t)8 << 20, kMostSlice = (size_t)64 << 20;
+
 // The reference takes its shared-memory path - double sums, +inf is missing - when a row's dense vector of as many
 // floats as the data has features fits 128 times into 48 KB (predictor.cu:85); the number of features is the largest
 // column with a stored value + 1.
@@ -318,12 +325,18 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
     ScoreRows rows;
     bool narrow = true;
     int F = 0;
-    // Slices of whole rows go up on a second stream: the traversal of a slice runs while the next one crosses PCIe.
+    // Slices of whole rows go up on a second stream: the traversal of a slice runs while the next ones cross PCIe.
     hipEvent_t up;
     HIP_CHECK(hipEventCreateWithFlags(&up, hipEventDisableTiming));
-    auto slice_ready = [&] {
+    UploadSet slices;
+    std::vector<ScoreRows> rows_of;
+    std::vector<int> first_of;
+    auto score_slice = [&](size_t k) {
         HIP_CHECK(hipEventRecord(up, s_up));
         HIP_CHECK(hipStreamWaitEvent(s, up, 0));
+        if (done)
+            done = launch_score(s, rows_of[k], dm->m, narrow, param.learning_rate, param.base_score, d_out + first_of[k], (size_t)n);
+        HIP_CHECK_LAUNCHES("predict (rows)");  // (a launch's error is its thread's)
     };
     if (!done && ds.is_dense()) {
         rows.columns = ds.dense_columns;
@@ -331,50 +344,52 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         narrow = ds.dense_f64 != nullptr ? !stores_beyond(ds.dense_f64, n, ds.dense_columns, kNarrowFeatures)
                                          : !stores_beyond(ds.dense_f32, n, ds.dense_columns, kNarrowFeatures);
         device_alloc_to(d_x, sizeof(float) * (size_t)n * ds.dense_columns);
-        const int step = usable ? (int)std::max<size_t>(1, ((size_t)64 << 20) / (4 * (size_t)ds.dense_columns)) : n;
+        const size_t row_bytes = 4 * (size_t)ds.dense_columns;
+        const int step = usable ? (int)std::max<size_t>(1, kMostSlice / row_bytes) : n;
         done = usable;
         for (int r0 = 0; r0 < n; r0 += std::min(step, n - r0)) {
-            const int m = std::min(step, n - r0);
-            const size_t off = (size_t)r0 * ds.dense_columns, cells = (size_t)m * ds.dense_columns;
-            if (ds.dense_f64 != nullptr) upload_doubles_as_floats(s_up, d_x + off, ds.dense_f64 + off, cells);
-            else upload_large(s_up, d_x + off, ds.dense_f32 + off, sizeof(float) * cells);
-            slice_ready();
-            rows.n = m;
+            const size_t off = (size_t)r0 * ds.dense_columns;
+            rows.n = std::min(step, n - r0);
             rows.x = d_x + off;
-            if (done)
-                done = launch_score(s, rows, dm->m, narrow, param.learning_rate, param.base_score, d_out + r0, (size_t)n);
+            if (ds.dense_f64 != nullptr) slices.add_doubles(d_x + off, ds.dense_f64 + off, (size_t)rows.n * ds.dense_columns);
+            else slices.add(d_x + off, ds.dense_f32 + off, (size_t)rows.n * row_bytes);
+            rows_of.push_back(rows);
+            first_of.push_back(r0);
         }
+        slices.send_in_order(s_up, score_slice);
     } else if (!done) {
-        // The column indices go up first: the feature count, which selects the traversal, may have to be taken from them.
+        // The column indices go up before the values: the feature count, which selects the traversal, may have to be taken from them.
         F = (int)ds.n_features();
         device_alloc_to(d_val, sizeof(float) * (size_t)std::max(nnz, 1l));
         device_alloc_to(d_col, sizeof(int) * (size_t)std::max(nnz, 1l));
         device_alloc_to(d_row_ptr, sizeof(int) * ((size_t)n + 1));
-        UploadSet first;
-        first.add(d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n + 1));
-        if (nnz) first.add_columns(d_col, ds.col_idx, (size_t)nnz);
-        first.send(s_up);
-        if (!ds.features_counted) F = device_max_int(s_up, d_col, nnz) + 1;
-        narrow = F <= kNarrowFeatures;
+        slices.add(d_row_ptr, ds.row_ptr, sizeof(int) * ((size_t)n + 1));
+        slices.add_columns(d_col, ds.col_idx, (size_t)nnz);
+        constexpr size_t kBefore = 2;  // the values' slices come behind them
         done = usable;
-        const long slice_entries = usable ? 16l << 20 : nnz;
+        const size_t eighth = sizeof(float) * (size_t)nnz / 8 / kPinnedBytes * kPinnedBytes;  // (whole pieces)
+        const long slice_entries = usable ? (long)(std::min(std::max(eighth, kLeastSlice), kMostSlice) / sizeof(float)) : nnz;
+        rows.col = d_col;
+        rows.val = d_val;
         for (int r0 = 0; r0 < n;) {
             const long e0 = ds.row_ptr[r0];
             // last row whose entries still fit the slice (at least one row)
             const int *from = ds.row_ptr + r0 + 1, *last = ds.row_ptr + n + 1;
             int r1 = (int)(std::upper_bound(from, last, (int)std::min<long>(e0 + slice_entries, nnz)) - ds.row_ptr) - 1;
             r1 = std::max(r1, r0 + 1);
-            const long e1 = ds.row_ptr[r1];
-            if (e1 > e0) upload_large(s_up, d_val + e0, ds.val + e0, sizeof(float) * (size_t)(e1 - e0));
-            slice_ready();
             rows.n = r1 - r0;
             rows.row_ptr = d_row_ptr + r0;
-            rows.col = d_col;
-            rows.val = d_val;
-            if (done)
-                done = launch_score(s, rows, dm->m, narrow, param.learning_rate, param.base_score, d_out + r0, (size_t)n);
+            slices.add(d_val + e0, ds.val + e0, sizeof(float) * (size_t)(ds.row_ptr[r1] - e0));
+            rows_of.push_back(rows);
+            first_of.push_back(r0);
             r0 = r1;
         }
+        slices.send_in_order(s_up, [&](size_t j) {
+            if (j >= kBefore) return score_slice(j - kBefore);
+            if (j + 1 < kBefore) return;  // (the columns are on their way as well, the values behind them)
+            if (!ds.features_counted) F = device_max_int(s_up, d_col, nnz) + 1;
+            narrow = F <= kNarrowFeatures;
+        });
     }
     lap("rows");
     TreeNode *d_model = nullptr;
@@ -413,9 +428,8 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         n_ret = transform_scores(s, param, ds, n, n_class, d_out, d_label);
     }
     HIP_CHECK_LAUNCHES("predict (metric, transform)");
-    if (n_ret) HIP_CHECK(hipMemcpyAsync(out, d_out, sizeof(float) * n_ret, hipMemcpyDeviceToHost, s));
+    download_large(s, out, d_out, sizeof(float) * n_ret);
     HIP_CHECK(hipStreamSynchronize(s_up));
-    HIP_CHECK(hipStreamSynchronize(s));
     HIP_CHECK(hipEventDestroy(up));
     lap("traversal, transform and download");
     for (void *p : {(void *)d_val, (void *)d_col, (void *)d_row_ptr, (void *)d_x, (void *)d_model, (void *)d_packed,
