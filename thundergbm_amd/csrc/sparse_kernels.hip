@@ -32,31 +32,32 @@ struct SegResult {
 };
 
 // Best candidate of one (feature, node) segment; one wavefront, lane l looks at ceil(kf / 64) consecutive bins of the
-// feature's kf <= 256 bins. cell(b) = cells[b * stride]. The arithmetic is that of k_eval_split: exact integer prefix sums,
+// feature's kf <= 256 bins. The arithmetic is that of k_eval_split: exact integer prefix sums,
 // missing = node sum - feature total, gain with the missing rows sent right and left
 // (hist_tree_builder_single.cu:300-323), largest |gain| wins, ties go to the smaller bin index (:330-335).
 // `force`: evaluate even when the segment holds no value (the feature owning global bin 0: when no candidate of a
 // node has a positive gain the arg-max of the reference ends on bin 0).
-__device__ SegResult eval_segment(const longlong2 *cells, int stride, int kf, int gbin0, GHPair S, double inv_g,
-                                  double inv_h, float mcw, float lambda, bool ignored, bool force) {
+// A wavefront takes 2.1 ns for an instruction that depends on the one before, so the code has no branches but the ones that
+// all lanes take alike.
+__device__ __forceinline__ SegResult eval_segment(const longlong2 *cells, int kf, int gbin0, GHPair S, double inv_g, double inv_h,
+                                                  float mcw, float lambda, bool ignored, bool force) {
 #pragma clang fp contract(off)
     const int lane = lane_id();
     const int bpl = (kf + 63) >> 6;  // bins per lane: 1 for the usual <= 64 bins, so that every lane has a candidate
-    long long incg[4], inch[4];
-    long long rung = 0, runh = 0;
+    long long exg[4], exh[4], rung = 0, runh = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+        exg[j] = rung;
+        exh[j] = runh;
+        if (j >= bpl) break;
         const int b = lane * bpl + j;
-        if (j < bpl && b < kf) {
-            const longlong2 v = cells[(size_t)b * stride];
-            rung += v.x;
-            runh += v.y;
-        }
-        incg[j] = rung;
-        inch[j] = runh;
+        const longlong2 v = cells[min(b, kf - 1)];
+        rung += b < kf ? v.x : 0;
+        runh += b < kf ? v.y : 0;
     }
-    const long long aggg = wave_scan_ll(rung), aggh = wave_scan_ll(runh);
-    const long long totg = read_lane_ll(aggg, 63), toth = read_lane_ll(aggh, 63);  // the last lane's inclusive sum
+    long long upg = rung, uph = runh;
+    wave_scan_pair(upg, uph);
+    const long long totg = read_lane_ll(upg, 63), toth = read_lane_ll(uph, 63);
     SegResult r;
     r.win = -1.f;
     r.win_idx = 0x7fffffff;
@@ -64,38 +65,33 @@ __device__ SegResult eval_segment(const longlong2 *cells, int stride, int kf, in
     r.score = 0.f;
     r.miss = r.left = GHPair{0, 0};
     if (!force && totg == 0 && toth == 0) return r;
-    const long long carryg = aggg - rung, carryh = aggh - runh;  // exclusive prefix of the lane
-    const GHPair m{S.g - (float)((double)totg * inv_g), S.h - (float)((double)toth * inv_h)};
+    const long long carryg = upg - rung, carryh = uph - runh;  // exclusive prefix of the lane
+    const GHPair m{S.g - scaled_float(totg, inv_g), S.h - scaled_float(toth, inv_h)};
+    const float fterm = (S.g * S.g) / (S.h + lambda);
     float best = -1.f, best_score = 0.f;
-    int best_idx = 0x7fffffff;
+    int which = 0;
     GHPair best_left{0, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         if (j >= bpl) break;
         const int b = lane * bpl + j;
-        if (b < kf) {
-            const long long exg = carryg + (j == 0 ? 0 : incg[j > 0 ? j - 1 : 0]);
-            const long long exh = carryh + (j == 0 ? 0 : inch[j > 0 ? j - 1 : 0]);
-            const GHPair l{(float)((double)exg * inv_g), (float)((double)exh * inv_h)};
-            const float gr = split_gain(S, l, mcw, lambda);
-            const GHPair l2{l.g + m.g, l.h + m.h};
-            const float gl = split_gain(S, l2, mcw, lambda);
-            float score = (gl > gr) ? gl : -gr;
-            if (ignored) score = 0.f;  // column sampling: hist_tree_builder_single.cu:304 / :663
-            const float a = fabsf(score);
-            if (a > best) {
-                best = a;
-                best_score = score;
-                best_idx = gbin0 + b;
-                best_left = l;
-            }
-        }
+        const GHPair l{scaled_float(carryg + exg[j], inv_g), scaled_float(carryh + exh[j], inv_h)};
+        const float gr = split_gain_select(S, fterm, l, mcw, lambda);
+        const float gl = split_gain_select(S, fterm, GHPair{l.g + m.g, l.h + m.h}, mcw, lambda);
+        const float score = ignored ? 0.f : (gl > gr ? gl : -gr);  // column sampling: hist_tree_builder_single.cu:304 / :663
+        const float a = b < kf ? fabsf(score) : -1.f;
+        const bool better = a > best;
+        which = better ? j : which;
+        best_score = better ? score : best_score;
+        best_left.g = better ? l.g : best_left.g;
+        best_left.h = better ? l.h : best_left.h;
+        best = better ? a : best;
     }
     // (lanes hold ascending bins: among equal gains the first lane's is the smallest)
     const float win = wave_max_f(best);
     const int first = __ffsll((long long)__ballot(best == win)) - 1;
     r.win = win;
-    r.win_idx = read_lane(best_idx, first);
+    r.win_idx = win < 0.f ? 0x7fffffff : read_lane(gbin0 + lane * bpl + which, first);
     r.owner = lane == first && best >= 0.f;
     r.score = best_score;
     r.miss = m;
@@ -157,7 +153,7 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
         const int b0 = sh.fbin[fi], kf = sh.fbin[fi + 1] - b0;
         if (kf <= 0) continue;
         const bool ign = tb.ignored != nullptr && tb.ignored[fa + fi] != 0;
-        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, 1, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
+        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
                                          lambda, ign, bin0 + b0 == 0);
         if (r.win >= 0.f && lane == 0) atomicMax(&sh.key[node], cand_key(r.win, r.win_idx));
     }
@@ -176,7 +172,7 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
         }
         const int b0 = sh.fbin[lo], kf = sh.fbin[lo + 1] - b0;
         const bool ign = tb.ignored != nullptr && tb.ignored[fa + lo] != 0;
-        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, 1, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
+        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
                                          lambda, ign, true);
         if (r.owner && r.win_idx == idx) {
             SplitCand c;
