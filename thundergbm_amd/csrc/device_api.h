@@ -274,8 +274,8 @@ struct SparsePass {
     unsigned long long *rare_item = nullptr;  // [n_sets][n_rare] values of a level that may matter, tile by tile
     int *rare_passed = nullptr;               // [n_sets][n_rare_tasks] how many of a tile
     const int *feat_val_begin = nullptr;  // [F + 1] first position of every feature in the bin-major copy
-    // [n_sets][nnz] the gradient pair of every stored value's row, in the order of the bin-major copy, refreshed once
-    // per tree: the level passes then stream it instead of fetching a cache line per value (nullptr: no room, gather)
+    // [n_sets][nnz] the gradient pair of every stored value's row, in the order of the bin-major copy, left there by
+    // the pass of level 0: those below then stream it instead of fetching a cache line per value (nullptr: no room, gather)
     GHPair *csc_gh = nullptr;
     long nnz = 0;
     longlong2 *partial = nullptr;         // [n_sets][n_partial_slots][partial_stride] chunk tables, (bin, node) cells
@@ -519,9 +519,6 @@ void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins
                        unsigned *key);
 // The rows' words of a tree (TreeBuffers::row_word).
 void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class);
-// csc_gh[e] = gh[csc_row[e]] for the values of the table tasks, n_class gradient planes (once per tree)
-void launch_sparse_gh_refresh(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
-                              const GHPair *gh, int n_class = 1);
 // Row-ordered passes over the row lists (one of dbins / cbins by tb.sparse). lookup_level: the level
 // whose split nodes still hold their children's rows (-1: none).
 void launch_nid_rebuild(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbins, const CsrBins *cbins,

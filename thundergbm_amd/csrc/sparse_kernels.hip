@@ -195,6 +195,9 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
 
 // One task = a run of whole features (batched so that their tables fit the LDS) or one chunk of a big feature (its
 // table goes to the partial buffer, k_sparse_big adds the chunks up and searches them).
+// ROOT: level 0, where every row is in the one node; the pairs are looked up there and left in csc_gh for the levels below (a
+// launch of its own before: 130 us and 67 at 1 M rows, together 113).
+template <bool ROOT>
 __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, CsrBins bins, SparsePass sp,
                                                           const GHPair *__restrict__ gh, int level, float mcw,
                                                           float lambda, int dump_hist, int n_cells) {
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
     const unsigned short *__restrict__ nid16 = tb.nid16;
     const int *__restrict__ crp = tb.cut_row_ptr;
     const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
-    const GHPair *__restrict__ csc_gh = sp.csc_gh != nullptr ? sp.csc_gh + (size_t)blockIdx.z * sp.nnz : nullptr;
+    GHPair *__restrict__ csc_gh = sp.csc_gh != nullptr ? sp.csc_gh + (size_t)blockIdx.z * sp.nnz : nullptr;
     sp_begin(tb, sh, level);
     longlong2 *dump = (dump_hist && task.cand_slot >= 0) ? tb.hist(level) : nullptr;
     longlong2 *partial = task.partial_slot >= 0
@@ -263,16 +266,21 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
                     const int e = min(e0 + u * kSpBlock, v1 - 1);
                     gb[u] = __builtin_nontemporal_load(bins.csc_bin + e);
                     row[u] = __builtin_nontemporal_load(bins.csc_row + e);
-                    if (csc_gh != nullptr) {
+                    if (!ROOT && csc_gh != nullptr) {
                         const unsigned long long w = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(csc_gh + e));
                         s[u] = GHPair{__uint_as_float((unsigned)w), __uint_as_float((unsigned)(w >> 32))};
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < U; ++u) x[u] = (int)nid16[row[u]] - off - n0;
-                if (csc_gh == nullptr) {
+                for (int u = 0; u < U; ++u) x[u] = ROOT ? 0 : (int)nid16[row[u]] - off - n0;
+                if (ROOT || csc_gh == nullptr) {
 #pragma unroll
                     for (int u = 0; u < U; ++u) s[u] = gh[row[u]];
+                }
+                if (ROOT && csc_gh != nullptr) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (e0 + u * kSpBlock < v1) csc_gh[e0 + u * kSpBlock] = s[u];
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -909,15 +917,6 @@ __global__ __launch_bounds__(256) void k_sparse_row_words(TreeBuffers tb_all, co
     for (int r = blockIdx.x * 256 + threadIdx.x; r < tb.n; r += gridDim.x * 256) tb.row_word[r] = rare_row_word(0u, gh[r], q);
 }
 
-// csc_gh[e] = gh[csc_row[e]] for the stored values of the table tasks
-__global__ __launch_bounds__(256) void k_sparse_gh_refresh(int n, SparsePass sp, const int *__restrict__ csc_row,
-                                                          const GHPair *__restrict__ gh) {
-    gh += (size_t)blockIdx.z * n;
-    GHPair *__restrict__ out = sp.csc_gh + (size_t)blockIdx.z * sp.nnz;
-    const SparseTask task = sp.tasks[blockIdx.x];
-    for (int e = task.v_begin + threadIdx.x; e < task.v_end; e += 256) out[e] = gh[csc_row[e]];
-}
-
 __global__ __launch_bounds__(256) void k_sparse_cols(long nnz, const int *__restrict__ csc_bin,
                                                     const int *__restrict__ csc_row, const int *__restrict__ cut_fid,
                                                     const int *__restrict__ cut_row_ptr,
@@ -969,12 +968,6 @@ void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair 
     k_sparse_row_words<<<dim3(std::max(1, std::min(1024, (tb.n + 255) / 256)), 1, n_class), 256, 0, s>>>(tb, gh);
 }
 
-void launch_sparse_gh_refresh(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
-                              const GHPair *gh, int n_class) {
-    if (sp.csc_gh == nullptr || sp.n_tasks == 0) return;
-    k_sparse_gh_refresh<<<dim3(sp.n_tasks, 1, n_class), 256, 0, s>>>(tb.n, sp, bins.csc_row, gh);
-}
-
 void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
                          const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class) {
     // LDS table of a table task: room for one feature of 255 bins with every node of the level, at least 2048 and at
@@ -989,10 +982,12 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
                             (size_t)(1 << level) * tb.n_bins * 4);
     }
     static LdsOptIn opt_in;
-    opt_in({reinterpret_cast<const void *>(&k_sparse_level), reinterpret_cast<const void *>(&k_sparse_big)});
-    if (sp.n_tasks > 0)
-        k_sparse_level<<<dim3(sp.n_tasks, 1, n_class), kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda,
-                                                                          dump_hist ? 1 : 0, n_cells);
+    opt_in({reinterpret_cast<const void *>(&k_sparse_level<true>), reinterpret_cast<const void *>(&k_sparse_level<false>), reinterpret_cast<const void *>(&k_sparse_big)});
+    if (sp.n_tasks > 0) {
+        const dim3 tasks(sp.n_tasks, 1, n_class);
+        if (level == 0) k_sparse_level<true><<<tasks, kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+        else k_sparse_level<false><<<tasks, kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+    }
     if (sp.n_big > 0)
         k_sparse_big<<<dim3(sp.n_big, std::min(1 << level, 16), n_class), kSpBlock, lds, s>>>(
             tb, sp, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);

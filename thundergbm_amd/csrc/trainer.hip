@@ -999,7 +999,6 @@ void Trainer::build_sparse_tasks() {
 void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class) {
     if (sparse_pass_ && level == 0) {
         launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
-        launch_sparse_gh_refresh(stream_, tb, csr_, sp_, gh, n_class);
         launch_sparse_row_words(stream_, tb, gh, n_class);
     }
     if (hist_cap_level_ >= 0 && level >= hist_cap_level_) {
