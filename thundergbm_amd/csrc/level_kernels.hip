@@ -499,7 +499,7 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 // columns (1605 x 60, depth 6: 0.105 -> 0.101 ms a tree; 16 k x 30, depth 8: 0.214 -> 0.178). Every workgroup of a node repeats
 // the split, the first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
 // (k_map_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
-// A level of 10 k x 8: 28 -> 14 us with its split search.
+// A level of 1605 x 119: 7.5 us and 7 for its split search.
 // The sums are those of k_hist_dense, whose work items count at a scale that hangs on the node's rows only.
 constexpr int kSmallWaves = kSmallBlock / 64;
 constexpr int kSmallSteps = kSmallRows / kSmallBlock;

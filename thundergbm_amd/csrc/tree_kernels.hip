@@ -2410,10 +2410,9 @@ __global__ __launch_bounds__(BLK) void k_tree_end(TreeBuffers tb_all, DenseBins 
 // levels), and which is small enough for every workgroup to prune it in LDS by itself; the last one has no rows and writes the
 // finished nodes into the model (in place they would change under the other workgroups' eyes). Pruning is a ballot a level in
 // one wavefront and every node's own climb instead of two barriers a level: 11.0 -> 8.0 us at 1605 rows and depth 6, 13.3 -> 11.1 at
-// 500 k and depth 8. One launch instead of k_end_bounds, k_tree_end
-// and the copy: 31 -> 10 us at 10 k rows. At 500 k x 28 the last level's count launch updates the tree and maps the rows (11 us) and
-// the end takes 13.5, where k_best_update, k_end_bounds and k_tree_end took 4.4, 9.7 and 14.7: a tree 0.260 -> 0.255 ms; 100 k rows
-// 0.213 -> 0.204, 300 k x 28 of depth 4 0.131 -> 0.125.
+// 500 k and depth 8. One launch instead of k_end_bounds, k_tree_end and the copy: 31 -> 8 us at 10 k rows. At 500 k x 28 the last
+// level's count launch updates the tree and maps the rows (11 us) and the end takes 11, where k_best_update, k_end_bounds and
+// k_tree_end took 4.4, 9.7 and 14.7.
 template <int MODE>
 __global__ __launch_bounds__(kEndWide) void k_map_end(TreeBuffers tb_all, DenseBins bins, TreeEndArgs a, TreeNode *model) {
     constexpr int kNodes = (2 << kSmallDepth) - 1;
