@@ -135,3 +135,32 @@ def test_merge_and_search_of_wide_features_in_one_launch(n, depth, bins, objecti
         out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), np.round(s.metric_log(), 5).tobytes()))
         s.close()
     assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("n,groups,numbers,depth,objective,rate", [
+    (1_600, (9, 16, 41), 5, 6, "binary:logistic", 1.0), (7_000, (3, 120), 17, 7, "reg:linear", 0.4), (8_192, (40,), 0, 5, "reg:linear", 1.0),
+    (3_000, (6, 7, 8, 9), 30, 6, "multi:softmax", 1.0), (2_500, (), 70, 4, "reg:linear", 1.0), (257, (5,), 2, 10, "reg:logistic", 1.0)])
+def test_search_of_few_rows_with_the_lists(n, groups, numbers, depth, objective, rate, monkeypatch):
+    """k_small_level with the next level's split search in it against the launches of larger data: columns that hold a one-hot
+    group of features, columns without a value, parts of 4, 8 and 16 columns and wider ones, class trees, sampled columns."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    hot = [np.eye(g, dtype=np.float32)[rng.integers(0, g, n)] for g in groups]
+    X = np.concatenate(hot + [rng.standard_normal((n, numbers)).astype(np.float32)], 1)
+    X[:, X.shape[1] // 2] = 0
+    X[rng.random(n) < 0.05] = 0
+    z = X @ rng.standard_normal(X.shape[1]) / 3 + 0.3 * rng.standard_normal(n)
+    y = z if objective == "reg:linear" else (np.digitize(z, [-0.3, 0.3]) if objective.startswith("multi") else z > 0)
+    val, rp, col = D.dense_to_csr(X)
+    out = []
+    for small in ("1", "0"):
+        monkeypatch.setenv("TGBM_SMALL", small)
+        ctypes.CDLL(None).srand(3)
+        s = T.Session(val, rp, col, np.asarray(y, np.float32), depth=depth, n_trees=4, learning_rate=0.5, objective=objective)
+        if rate < 1:
+            s.set_option("column_sampling_rate", rate)
+        s.boost(3)
+        s.boost(1)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), np.round(s.metric_log(), 5).tobytes()))
+        s.close()
+    assert out[0] == out[1]

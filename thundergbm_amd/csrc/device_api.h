@@ -497,8 +497,10 @@ void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins
 // Dense layout, few rows: the level's splits, the children's lists and the histograms of the next level's built nodes in one
 // launch. The split search of the next level then derives the siblings (launch_eval_split with derive).
 bool small_levels_fit(const TreeBuffers &tb);
-void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
-                        float lambda, const int *part_bins, int n_class = 1);
+// next_cand (nullptr: never): room for the next level's candidates, a slot per column of every node. True: they are there, that
+// split search is done.
+bool launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
+                        float lambda, const int *part_bins, int n_class, SplitCand *next_cand, float mcw);
 // The end of a tree whose rows' nodes are in tb.nid (lookup_level >= 0: split nodes of that level still hold the rows of their
 // children): prunes the tree into `model` (n_class trees back to back; tb.nodes
 // stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics.

@@ -499,17 +499,31 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 // columns (1605 x 60, depth 6: 0.105 -> 0.101 ms a tree; 16 k x 30, depth 8: 0.214 -> 0.178). Every workgroup of a node repeats
 // the split, the first one stores it. The children's rows are also marked in the row -> node map, from which the end of the tree is read
 // (k_map_end). Bound by its chain of dependent steps: candidates -> bins of the rows -> lists -> bins and pairs -> LDS.
-// A level of 1605 x 119: 7.5 us and 7 for its split search.
 // The sums are those of k_hist_dense, whose work items count at a scale that hangs on the node's rows only.
 constexpr int kSmallWaves = kSmallBlock / 64;
+constexpr size_t kSmallSearchBytes = sizeof(longlong2) * kEvalPackBins * kSmallWaves;
 constexpr int kSmallSteps = kSmallRows / kSmallBlock;
 static_assert(kSmallRows / 2 <= kHistFlushRows, "the built child's packed sums are never drained");
 static_assert(kSmallRows <= 1 << 16 && kSmallWaves == 16 && kSmallSteps % 4 == 0, "16-bit row ids, the counts of four steps per wavefront");
 
-template <int LPR, bool BIN16, int STEPS>
+// 64-bit words of the histogram and of the built child's row ids (an even number: what follows is read as 16 bytes)
+__host__ __device__ inline int small_words(int n, int lds_bins) { return (lds_bins + ((n / 2 + 1) * 2 + 7) / 8 + 1) / 2 * 2; }
+// SEARCH: the workgroup has the built child's histogram of its columns whole, so it also derives the sibling's and searches both,
+// a column and child per wavefront, into the other one of two candidate arrays (the node's own are still being read). For parts
+// of up to 16 columns, so that a wavefront searches once or twice; wider ones leave it to a launch that spreads it over the chip.
+// A level of 1605 x 119: 12.3 us instead of 7.5 and 7.0 in two launches; ms a tree: 1605 x 60, depth 6 0.0983 -> 0.0845, 4 k x 100
+// 0.1146 -> 0.1012, 8 k x 4, depth 8 0.1326 -> 0.1160, 6 k one-hot of 5 classes 0.1320 -> 0.1183, 2 k x 600 (few levels) 0.1506 -> 0.1475.
+struct SmallSearch {
+    SplitCand *cand = nullptr;  // of the next level, a slot per column
+    int slots = 0;
+    float mcw = 0;
+    bool store = false;  // the children's histograms are parents again
+};
+template <int LPR, bool BIN16, int STEPS, bool SEARCH>
 __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__ gh,
-                                                            int level, float rt_eps, float lambda, int log_split, int lds_bins) {
-    extern __shared__ unsigned long long lds[];  // the block's histogram, then the built child's row ids
+                                                            int level, float rt_eps, float lambda, int log_split, int lds_bins,
+                                                            SmallSearch search) {
+    extern __shared__ __attribute__((aligned(16))) unsigned long long lds[];  // the block's histogram, then the built child's row ids
     __shared__ PickShared s_pick;
     __shared__ int s_left[STEPS * kSmallWaves];  // rows that go left, per step and wavefront
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
@@ -541,6 +555,18 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
             const int pos = min(sg.x + k * kSmallBlock + (int)threadIdx.x, sg.y - 1);
             row[k] = level == 0 ? pos : ridx[pos];
         }
+    }
+    // SEARCH: the wavefront's column and the first child that it searches (0: the built one, 1: its sibling)
+    static_assert(!SEARCH || (COLS <= kSmallWaves && !BIN16), "a column per wavefront");
+    const int my_col = w % COLS, my_child = w / COLS;
+    const int c0 = SEARCH ? col_off[my_col] - off0 : 0;
+    const int c1 = SEARCH ? (part + 1 == 1 << log_split && my_col + 1 == COLS ? nb : col_off[my_col + 1] - off0) : 0;
+    longlong2 parent[4];
+    PackMeta meta;
+    if constexpr (SEARCH) {
+        meta.load(tb, bin0 + c0, bin0 + c1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) parent[j] = tb.hist(level)[(size_t)x_in * tb.n_bins + max(0, bin0 + min(c0 + lane * 4 + j, c1 - 1))];
     }
     for (int i = threadIdx.x; i < nb; i += kSmallBlock) lds[i] = 0ull;
     const Picked best = pick_candidate<kSmallWaves>(tb, x_in, node.is_valid, s_pick, early);
@@ -650,10 +676,44 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     __syncthreads();
     const int built = build_left ? node.lch_index : node.rch_index;
     const unsigned long long h_mask = (1ull << h_bits) - 1ull;
-    longlong2 *out = tb.hist(level + 1) + (size_t)(built - ((2 << level) - 1)) * tb.n_bins + bin0;
-    for (int i = threadIdx.x; i < nb; i += kSmallBlock) {
-        const unsigned long long t = lds[i], low = t & h_mask;
-        out[i] = make_longlong2(((long long)(t - low) >> h_bits) << shift_g, (long long)low << shift_h);
+    auto unpacked = [&](unsigned long long t) {
+        const unsigned long long low = t & h_mask;
+        return make_longlong2(((long long)(t - low) >> h_bits) << shift_g, (long long)low << shift_h);
+    };
+    if constexpr (!SEARCH) {
+        longlong2 *out = tb.hist(level + 1) + (size_t)(built - ((2 << level) - 1)) * tb.n_bins + bin0;
+        for (int i = threadIdx.x; i < nb; i += kSmallBlock) out[i] = unpacked(lds[i]);
+    } else if (const int column = ((fb << log_split) + part) * COLS + my_col; column < search.slots) {
+        // the children's sums as apply_split computes them
+        GHPair ls = best.c.bin != 0 ? best.c.left : GHPair{0, 0};
+        if (!(best.c.score < 0)) {
+            ls.g += best.c.miss.g;
+            ls.h += best.c.miss.h;
+        }
+        const GHPair rs{node.sum_gh_pair.g - ls.g, node.sum_gh_pair.h - ls.h};
+        longlong2 *s_v = reinterpret_cast<longlong2 *>(lds + small_words(tb.n, lds_bins)) + w * kEvalPackBins;
+        TreeBuffers next = tb;
+        next.cand = search.cand + (size_t)blockIdx.z * tb.max_level_nodes * search.slots;
+        next.n_packs = search.slots;
+        for (int child = my_child; child < 2; child += kSmallWaves / COLS) {
+            const bool left = build_left == (child == 0);
+            const int x_child = 2 * x_in + (left ? 0 : 1);
+            longlong2 *out = tb.hist(level + 1) + (size_t)x_child * tb.n_bins + bin0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int b = c0 + lane * 4 + j;
+                longlong2 v = make_longlong2(0, 0);
+                if (b < c1) {
+                    v = unpacked(lds[b]);
+                    if (child == 1) v = make_longlong2(parent[j].x - v.x, parent[j].y - v.y);
+                    if (search.store) out[b] = v;
+                }
+                s_v[lane * 4 + j] = v;
+            }
+            wave_lds_sync();
+            search_pack(next, meta, s_v, x_child, column, true, bin0 + c0, bin0 + c1, left ? ls : rs, quant.inv_g, quant.inv_h, search.mcw, lambda);
+            wave_lds_sync();
+        }
     }
     if (first) {
         tb.node_nleft[x_in] = nleft;
@@ -999,47 +1059,54 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
     if (tb.planned(level + 1)) k_plan_level<<<dim3(1, 1, n_class), kPlanBlock, 0, s>>>(tb, level + 1, tb.n_hpairs(level + 1));
 }
 
-static size_t small_lds(const TreeBuffers &tb, int lds_bins) {
-    return (size_t)lds_bins * 8 + ((size_t)(tb.n / 2 + 1) * 2 + 7) / 8 * 8;
-}
+static size_t small_lds(const TreeBuffers &tb, int lds_bins) { return (size_t)small_words(tb.n, lds_bins) * 8; }
 
 bool small_levels_fit(const TreeBuffers &tb) {
     return tb.n <= kSmallRows && tb.depth <= kSmallDepth && small_lds(tb, tb.max_block_bins) + 4096 <= kLdsBytes;
 }
 
-template <int LPR, bool BIN16, int STEPS>
-static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                               float rt_eps, float lambda, int log_split, int lds_bins, int n_class) {
-    const size_t lds = small_lds(tb, lds_bins);
+struct SmallLaunch {
+    int level, log_split, lds_bins, n_class;
+    float rt_eps, lambda;
+    SmallSearch search;  // cand nullptr: none
+};
+
+template <int LPR, bool BIN16, int STEPS, bool SEARCH>
+static void small_level_launch(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, const SmallLaunch &l) {
+    const size_t lds = small_lds(tb, l.lds_bins) + (SEARCH ? kSmallSearchBytes : 0);
     static LdsOptIn opt_in;
     if (lds > 48 * 1024)  // (with the kernel's own tables more than the default window)
-        opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16, STEPS>)});
-    k_small_level<LPR, BIN16, STEPS><<<dim3(bins.n_blocks << log_split, 1 << level, n_class), kSmallBlock, lds, s>>>(tb, bins, gh, level, rt_eps, lambda,
-                                                                                                                          log_split, lds_bins);
+        opt_in({reinterpret_cast<const void *>(&k_small_level<LPR, BIN16, STEPS, SEARCH>)});
+    k_small_level<LPR, BIN16, STEPS, SEARCH><<<dim3(bins.n_blocks << l.log_split, 1 << l.level, l.n_class), kSmallBlock, lds, s>>>(
+        tb, bins, gh, l.level, l.rt_eps, l.lambda, l.log_split, l.lds_bins, l.search);
 }
 
 // (the code of steps that no node of the data can have is not only skipped but left out, see k_small_level)
-template <int LPR, bool BIN16>
-static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level,
-                              float rt_eps, float lambda, int log_split, int lds_bins, int n_class) {
+template <int LPR, bool BIN16, bool SEARCH>
+static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, const SmallLaunch &l) {
     const int steps = (tb.n + kSmallBlock - 1) / kSmallBlock;
-    if (steps <= 2) small_level_launch<LPR, BIN16, 2>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
-    else if (steps <= 4) small_level_launch<LPR, BIN16, 4>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
-    else small_level_launch<LPR, BIN16, kSmallSteps>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);
+    if (steps <= 2) small_level_launch<LPR, BIN16, 2, SEARCH>(s, tb, bins, gh, l);
+    else if (steps <= 4) small_level_launch<LPR, BIN16, 4, SEARCH>(s, tb, bins, gh, l);
+    else small_level_launch<LPR, BIN16, kSmallSteps, SEARCH>(s, tb, bins, gh, l);
 }
 
-void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
-                        float lambda, const int *part_bins, int n_class) {
-    if (level == tb.depth - 1) return;
+bool launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,
+                        float lambda, const int *part_bins, int n_class, SplitCand *next_cand, float mcw) {
+    if (level == tb.depth - 1) return false;
     // (up to a workgroup per CU a block's columns are shared out, see kSplitHistGroups)
-    int log_split = 0;
-    while (4 << (log_split + 1) <= bins.W * bins.bin_bytes && ((long)bins.n_blocks * n_class << (level + log_split + 1)) <= kSplitHistGroups) ++log_split;
-    const int lds_bins = part_bins[log_split];
-#define TGBM_SMALL_LEVEL(LPR)                                                                               \
-    if (bins.bin_bytes == 2) small_level_steps<LPR, true>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class); \
-    else small_level_steps<LPR, false>(s, tb, bins, gh, level, rt_eps, lambda, log_split, lds_bins, n_class);                    \
+    SmallLaunch l{level, 0, 0, n_class, rt_eps, lambda, {}};
+    while (4 << (l.log_split + 1) <= bins.W * bins.bin_bytes && ((long)bins.n_blocks * n_class << (level + l.log_split + 1)) <= kSplitHistGroups) ++l.log_split;
+    l.lds_bins = part_bins[l.log_split];
+    const int row_bytes = bins.W * bins.bin_bytes >> l.log_split;  // of a part
+    const bool search = next_cand != nullptr && bins.bin_bytes == 1 && row_bytes <= kSmallWaves &&
+                        small_lds(tb, l.lds_bins) + kSmallSearchBytes + 8192 <= kLdsBytes;
+    if (search) l.search = SmallSearch{next_cand, bins.n_cols, mcw, level + 1 < tb.depth - 1};
+#define TGBM_SMALL_LEVEL(LPR)                                                                        \
+    if (bins.bin_bytes == 2) small_level_steps<LPR, true, false>(s, tb, bins, gh, l);                \
+    else if (LPR <= 4 && search) small_level_steps<LPR, false, (LPR <= 4)>(s, tb, bins, gh, l);      \
+    else small_level_steps<LPR, false, false>(s, tb, bins, gh, l);                                   \
     break
-    switch (bins.W * bins.bin_bytes >> log_split) {  // bytes per row of a part
+    switch (row_bytes) {
         case 4: TGBM_SMALL_LEVEL(1);
         case 8: TGBM_SMALL_LEVEL(2);
         case 16: TGBM_SMALL_LEVEL(4);
@@ -1048,6 +1115,7 @@ void launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &b
         default: fatal("unsupported dense block width %d x %d bytes", bins.W, bins.bin_bytes);
     }
 #undef TGBM_SMALL_LEVEL
+    return search;
 }
 
 }  // namespace tgbm

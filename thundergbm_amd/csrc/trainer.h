@@ -177,6 +177,9 @@ class Trainer {
     bool rank_order_fresh_ = false;      // d_yp_ unchanged since the last ranking metric pass
     bool in_boost_ = false;
     bool small_ok_ = false;          // inside boost() the levels go through launch_small_level
+    SplitCand *small_cand_[2] = {nullptr, nullptr};  // candidates by column, of even and odd levels
+    bool searched_ = false;          // the level before has left this one's there
+    TreeBuffers searched_set(const TreeBuffers &tb, int level) const;
     bool small() const { return in_boost_ && small_ok_; }
     int part_bins_[5] = {0};         // most bins of a part of a feature block in 1, 2, 4, 8, 16 parts
     SplitHistPlan run_plan_;         // inside boost() the levels go through launch_partition_hist, runs of so many rows

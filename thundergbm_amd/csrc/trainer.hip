@@ -690,6 +690,9 @@ void Trainer::alloc_tree_buffers() {
 
     const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
     small_ok_ = !sparse_ && hist_cap_level_ < 0 && small_levels_fit(tb) && !(small_env != nullptr && std::string(small_env) == "0");
+    const size_t small_cands = S * (size_t)max_level_nodes * bins_.n_cols;
+    if (small_ok_ && !wide_eval_ && small_cands * sizeof(SplitCand) <= (size_t)64 << 20)
+        for (SplitCand *&c : small_cand_) c = dalloc<SplitCand>(small_cands);
     const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
     if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
         run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
@@ -996,7 +999,17 @@ void Trainer::build_sparse_tasks() {
              sp_.n_rare_tasks, sp_.n_cand_slots);
 }
 
+TreeBuffers Trainer::searched_set(const TreeBuffers &tb, int level) const {
+    TreeBuffers t = tb;
+    if (searched_) {
+        t.cand = small_cand_[level & 1];
+        t.n_packs = bins_.n_cols;
+    }
+    return t;
+}
+
 void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level, int n_class) {
+    if (level == 0) searched_ = false;
     if (sparse_pass_ && level == 0) {
         launch_root_sum(stream_, tb, gh, param_.lambda, n_class);
         launch_sparse_row_words(stream_, tb, gh, n_class);
@@ -1032,7 +1045,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     const bool sum_rows = !sparse_ && level == 0 && hist_cap_level_ != 0 && tb.complete_feature < 0;
     if (!derive && !(run() > 0 && level > 0)) build_level_hist(tb, level, gh, n_class, sum_rows);
     mark(PH_HIST, level);
-    if (!sparse_pass_) {
+    if (!sparse_pass_ && !searched_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
         const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0;
         const bool fused_wide = !sparse_ && !derive && wide_eval_ && hist_cap_level_ < 0 && level > 0;
@@ -1054,7 +1067,7 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
             launch_eval_split(stream_, tb, level, param_.min_child_weight, param_.lambda, n_class,
                               !(in_boost_ && level == param_.depth - 1), derive);
     }
-    if (!update_with_partition(level)) launch_best_update(stream_, tb, level, param_.rt_eps, param_.lambda, n_class);
+    if (!update_with_partition(level)) launch_best_update(stream_, searched_set(tb, level), level, param_.rt_eps, param_.lambda, n_class);
     mark(PH_SPLIT, level);
     lookup_level_ = level;  // until partition(level) moves the rows into the children's lists
     HIP_CHECK_LAUNCHES("find_split");
@@ -1101,7 +1114,8 @@ void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level,
     } else if (sparse_)
         launch_partition_csr(stream_, tb, csr_, level, n_class);
     else if (small())
-        launch_small_level(stream_, tb, bins_, gh, level, param_.rt_eps, param_.lambda, part_bins_, n_class);
+        searched_ = launch_small_level(stream_, searched_set(tb, level), bins_, gh, level, param_.rt_eps, param_.lambda, part_bins_, n_class,
+                                       small_cand_[(level + 1) & 1], param_.min_child_weight);
     else if (run() > 0) {
         DenseBins b = bins_;
         b.gh_fresh = gh_records_fresh_ && n_class == 1 && gh == d_gh_;

@@ -1050,125 +1050,9 @@ __global__ __launch_bounds__(kBlock) void k_part_count_csr(TreeBuffers tb_all, C
 // left = sum of the feature's bins below it, missing = node sum - feature total, gain with missing
 // values sent right and left (hist_tree_builder_single.cu:257-325 / :614-681 of the reference);
 // the wavefront keeps its best candidate: largest |gain|, ties to the smaller bin index (:330-335).
-// What a wavefront has stored in LDS is there for its other lanes (the accesses of a wavefront stay in order).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// What search_pack needs of a lane's four bins, loaded early so that nothing waits for it there.
-struct PackMeta {
-    unsigned meta[4];  // TreeBuffers::bin_meta: one word per bin instead of the chain bin -> feature -> feature's bin range
-    bool ignored[4];
-    __device__ __forceinline__ void load(const TreeBuffers &tb, int b_begin, int b_end) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) meta[j] = tb.bin_meta[max(0, min(b_begin + lane_id() * 4 + j, b_end - 1))];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            ignored[j] = tb.ignored != nullptr && tb.ignored[tb.cut_fid[max(0, min(b_begin + lane_id() * 4 + j, b_end - 1))]] != 0;
-    }
-};
-
 // Where the split search of level 0 takes the node's sums from: a feature stored in every row, whose bins add up to them, or
 // what the histogram launch has added up of the rows.
 enum RootSums { kNoRoot = 0, kRootOfBins, kRootOfRows };
-
-// The search of one pack of one node, by one wavefront: s_v holds the pack's bins (kEvalPackBins entries, overwritten). A lane has
-// four consecutive bins. The sums below a bin within its feature are differences of plain prefix sums, exact in integers. A
-// pack of one feature, the usual one with 255 bins, has them without a detour through LDS, and its missing sum once.
-// A wavefront takes 2.1 ns for an instruction that depends on the one before whatever else the CU does, and deep levels keep
-// the vector ALUs busy, so the code is short before all: no branches, about 650 instructions instead of the
-// 1000 of a segmented scan with them (10 k x 8 0.123 -> 0.119 ms a tree, 500 k x 28 0.254 -> 0.249, 50 k x 700 0.269 -> 0.263).
-__device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMeta &pm, longlong2 *s_v, int x_in, int pack, bool active,
-                                            int b_begin, int b_end, GHPair S, double inv_g, double inv_h, float mcw, float lambda) {
-#pragma clang fp contract(off)
-    const int lane = lane_id(), nb = b_end - b_begin, at = lane * 4;
-    long long exg[4], exh[4];
-    long long g = 0, h = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const longlong2 v = s_v[at + j];
-        exg[j] = g;
-        exh[j] = h;
-        g += at + j < nb ? v.x : 0;
-        h += at + j < nb ? v.y : 0;
-    }
-    long long upg = g, uph = h;
-    wave_scan_pair(upg, uph);
-    const long long allg = read_lane_ll(upg, 63), allh = read_lane_ll(uph, 63);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        exg[j] += upg - g;
-        exh[j] += uph - h;
-    }
-    const float fterm = (S.g * S.g) / (S.h + lambda);
-    auto missing = [&](long long tg, long long th) {
-        return GHPair{S.g - scaled_float(tg, inv_g), S.h - scaled_float(th, inv_h)};
-    };
-    GHPair m[4];
-    const bool one_feature = read_lane((int)(pm.meta[0] & 0xffu), 0) + 1 >= nb;
-    if (one_feature) {
-        m[0] = missing(allg, allh);
-        m[1] = m[2] = m[3] = m[0];
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s_v[at + j] = make_longlong2(exg[j], exh[j]);
-        wave_lds_sync();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            // (past the pack's end the words of its last bin repeat: clamped, nobody looks at the result)
-            const int head = max(0, at + j - (int)(pm.meta[j] >> 8 & 0xffu)), end = min(at + j + (int)(pm.meta[j] & 0xffu) + 1, nb);
-            const longlong2 below = s_v[head], upto = s_v[min(end, kEvalPackBins - 1)];
-            m[j] = missing((end == nb ? allg : upto.x) - below.x, (end == nb ? allh : upto.y) - below.y);
-            exg[j] -= below.x;
-            exh[j] -= below.y;
-        }
-    }
-    float score[4], best = -1.f;
-    GHPair left[4];
-    int which = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        left[j] = GHPair{scaled_float(exg[j], inv_g), scaled_float(exh[j], inv_h)};
-        const float gr = split_gain_select(S, fterm, left[j], mcw, lambda);
-        const float gl = split_gain_select(S, fterm, GHPair{left[j].g + m[j].g, left[j].h + m[j].h}, mcw, lambda);
-        score[j] = gl > gr ? gl : -gr;
-        score[j] = pm.ignored[j] ? 0.f : score[j];  // column sampling: hist_tree_builder_single.cu:304 / :663
-        const float a = at + j < nb ? fabsf(score[j]) : -1.f;
-        which = a > best ? j : which;
-        best = fmaxf(best, a);
-    }
-    // wavefront arg-max: larger |score| wins, ties go to the smaller bin index, which is the first lane's: lanes hold ascending
-    // bins. The lane that holds the winner writes its candidate itself (without any candidate every lane holds the initial
-    // one and the first lane writes the empty record).
-    const unsigned long long owners = __ballot(best == wave_max_f(best));
-    if (active && lane == __ffsll((long long)owners) - 1) {
-        const bool none = best < 0.f;
-        unsigned meta = pm.meta[0];
-        SplitCand c;
-        c.score = score[0];
-        c.left = left[0];
-        c.miss = m[0];
-#pragma unroll
-        for (int j = 1; j < 4; ++j)
-            if (which == j) {
-                c.score = score[j];
-                c.left = left[j];
-                c.miss = m[j];
-                meta = pm.meta[j];
-            }
-        c.index = b_begin + at + which;
-        c.feature = (int)(meta >> 16);
-        c.bin = (int)(meta >> 8 & 0xffu);
-        if (none) {
-            c.score = 0.f;
-            c.index = 0x7fffffff;
-            c.miss = c.left = GHPair{0, 0};
-            c.feature = c.bin = 0;
-        }
-        tb.cand[(size_t)x_in * tb.n_packs + pack] = c;
-    }
-}
 
 // SUB (sparse layout, whose histograms are not merged from work-item partials): the node of a pair that
 // was not built from rows is derived here as parent - built while it is scanned, and stored for the next
