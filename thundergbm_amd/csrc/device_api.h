@@ -106,9 +106,12 @@ constexpr int kRootParts = 512;     // parts of the rows whose sums add up to th
 constexpr int kHistFlushRows = 8192;
 constexpr int kHistFlushRowsInt = 32768;
 // Data of so few rows is trained on by the launches of launch_small_level, trees of so many levels at most. ms a tree with
-// them and with launch_partition_hist, 28 columns and depth 8: 4000 rows 0.142 and 0.152, 8000 0.156 and 0.155, 16 000 0.183 and 0.158;
-// 8 columns and depth 6: 0.099 and 0.105, 0.107 and 0.104, 0.126 and 0.108.
-constexpr int kSmallRows = 8192;
+// them and with launch_partition_hist, 28 columns and depth 8: 4000 rows 0.120 and 0.147, 8000 0.131 and 0.150, 12 000 0.143 and 0.154;
+// depth 6: 0.090 and 0.105, 0.099 and 0.107, 0.109 and 0.109 (14 000 with the code of sixteen steps 0.116 and 0.108). Features of more
+// than 255 bins have their split search in a launch of its own, and the line where it was without it: 28 columns, depth 8, 8000
+// rows 0.156 and 0.155, 16 000 0.183 and 0.158.
+constexpr int kSmallRows = 12288;
+constexpr int kSmallRowsWide = 8192;
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallDepth = 10;
 constexpr int kRowBlock = 4096;    // rows owned by one workgroup of the row-ordered passes and reductions

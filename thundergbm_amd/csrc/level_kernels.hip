@@ -1087,6 +1087,7 @@ static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseB
     const int steps = (tb.n + kSmallBlock - 1) / kSmallBlock;
     if (steps <= 2) small_level_launch<LPR, BIN16, 2, SEARCH>(s, tb, bins, gh, l);
     else if (steps <= 4) small_level_launch<LPR, BIN16, 4, SEARCH>(s, tb, bins, gh, l);
+    else if (steps <= 8) small_level_launch<LPR, BIN16, 8, SEARCH>(s, tb, bins, gh, l);
     else small_level_launch<LPR, BIN16, kSmallSteps, SEARCH>(s, tb, bins, gh, l);
 }
 
