@@ -164,3 +164,43 @@ def test_search_of_few_rows_with_the_lists(n, groups, numbers, depth, objective,
         out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), np.round(s.metric_log(), 5).tobytes()))
         s.close()
     assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("n,objective,bins,empty,descending", [
+    (3_000, "reg:linear", 1024, 8, False), (20_000, "binary:logistic", 1024, 8, False), (70_000, "multi:softmax", 1024, 8, False),
+    (20_000, "reg:linear", 255, 64, True)])
+@pytest.mark.parametrize("route", ["boost", "launches", "stages"])
+def test_first_block_without_bins(n, objective, bins, empty, descending, route, monkeypatch):
+    """The first feature block stores an item's scales and the rows' sums for all of them. Its columns may hold no value at all
+    (16-bit bins and rows whose columns do not ascend are not bundled): the same data with those columns last."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    F = 37 if bins > 255 else 90
+    X = rng.permuted(np.tile(np.arange(n) % 1000 + 1, (F, 1)), axis=1).T.astype(np.float32)
+    X[rng.random((n, F)) < 0.3] = 0  # (no column is stored in every row)
+    X[:, :empty] = 0
+    z = X[:, empty] / 500 + np.abs(X[:, -1] / 500 - 1) + 0.3 * rng.standard_normal(n)
+    K = 3 if objective.startswith("multi") else 1
+    y = z if objective == "reg:linear" else (np.digitize(z, [0.8, 1.4]) if K > 1 else z > 1)
+    if route == "launches":
+        monkeypatch.setenv("TGBM_SPLIT_HIST", "0")
+        monkeypatch.setenv("TGBM_SMALL", "0")
+    out = []
+    for shift in (0, empty):
+        val, rp, col = D.dense_to_csr(np.roll(X, -shift, axis=1))
+        if descending:
+            order = np.lexsort((-col, np.repeat(np.arange(n), np.diff(rp))))
+            val, col = val[order], col[order]
+        s = T.Session(val, rp, col, np.asarray(y, np.float32), depth=6, n_trees=3, learning_rate=0.5, max_num_bin=bins, objective=objective)
+        assert shift > 0 or s.info("dense_W") == empty
+        if route == "stages":
+            one_by_one(s, 3, 6, K)
+        else:
+            s.boost(3)
+        model = s.model()
+        model["split_fid"][model["split_fid"] >= 0] += shift
+        out.append((model.tobytes(), s.y_pred().tobytes(), s.nid().tobytes()))
+        s.close()
+    assert np.any(model["split_fid"] >= empty)
+    same = [a == b for a, b in zip(*out)]  # (a failed comparison of the bytes themselves is printed for minutes)
+    assert all(same), same

@@ -578,7 +578,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     }
     const int bin0 = blk_bin_begin[fb];
     const int nb = blk_bin_begin[fb + 1] - bin0;
-    if (nb == 0) return;
+    if (nb == 0 && fb != 0) return;  // (the first block, with bins or without, stores what an item has once: its scales, its rows' sums)
     if constexpr (!DIRECT) quant = *tb.quant;
     const int h_bits = quant.h_bits;
     const int flush_rows = quant.flush_rows;
