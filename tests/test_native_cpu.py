@@ -39,3 +39,32 @@ def test_kept_device_blocks(run_native):
     """Reuse, the limit, the order in which blocks go, an allocation that fails, and who pays: requests that follow a
     training call free nothing that it has left, and no thread waits for another one's driver call."""
     run_native("device_pool.cpp")
+
+
+def test_scans_keep_the_wait_states(tmp_path):
+    """Hazards inside inline assembly are its author's: gfx950 needs a wait state between a vector instruction that writes vcc
+    and one that takes its carry from there, two before a register is read through DPP, one before a lane is read."""
+    asm = str(tmp_path / "wave_scan.s")
+    subprocess.check_call([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-O3", "-std=c++17", "--offload-arch=gfx950", "-w",
+                           "--offload-device-only", "-S", os.path.join(HERE, "native", "wave_scan.hip"), "-o", asm])
+    age, carries = {}, 0  # wait states since a vector instruction wrote a register
+    for line in open(asm):
+        op, _, rest = line.split(";")[0].strip().partition(" ")
+        if op == "s_nop":
+            age = {r: a + 1 + int(rest) for r, a in age.items()}
+        if not op.startswith("v_"):
+            continue
+        args = [a.split()[0] for a in rest.split(",")]
+        written = args[:2] if "_co_" in op else args[:1]
+        read = args[len(written):]
+        far = lambda r: age.get(r, 99)
+        if "vcc" in read:
+            carries += 1
+            assert far("vcc") >= 1, line
+        if op.endswith("_dpp"):
+            assert far(read[0]) >= 2, line
+        if op.startswith("v_readlane"):
+            assert far(read[0]) >= 1, line
+        age = {r: a + 1 for r, a in age.items()}
+        age.update({r: 0 for r in written})
+    assert carries == 12

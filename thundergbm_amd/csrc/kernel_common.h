@@ -75,16 +75,18 @@ __device__ __forceinline__ long long read_lane_ll(long long v, int lane) {
     return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-// Inclusive sums of two 64-bit integers over a wavefront: four instructions a step, the lane move part of the additions. (A
-// register that a vector instruction has just written may be read through DPP two instructions later: between the four they
-// are, before the first step there is an s_nop.)
+// Inclusive sums of two 64-bit integers over a wavefront: four additions a step, the lane move part of them. The compiler does not
+// look for hazards inside: a carry may be read one wait state after the vector instruction that writes it, a register through
+// DPP two after it was written (between the steps there are more, before the first one there is an s_nop), a lane one after.
 __device__ __forceinline__ void wave_scan_pair(long long &a, long long &b) {
     unsigned al = (unsigned)(unsigned long long)a, ah = (unsigned)((unsigned long long)a >> 32);
     unsigned bl = (unsigned)(unsigned long long)b, bh = (unsigned)((unsigned long long)b >> 32);
 #define TGBM_SCAN_STEP(MOVE)                           \
     "v_add_co_u32_dpp %0, vcc, %0, %0 " MOVE "\n"      \
+    "s_nop 0\n"                                        \
     "v_addc_co_u32_dpp %1, vcc, %1, %1, vcc " MOVE "\n" \
     "v_add_co_u32_dpp %2, vcc, %2, %2 " MOVE "\n"      \
+    "s_nop 0\n"                                        \
     "v_addc_co_u32_dpp %3, vcc, %3, %3, vcc " MOVE "\n"
     asm("s_nop 1\n"
         TGBM_SCAN_STEP("row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0")
@@ -93,6 +95,7 @@ __device__ __forceinline__ void wave_scan_pair(long long &a, long long &b) {
         TGBM_SCAN_STEP("row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0")
         TGBM_SCAN_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf")
         TGBM_SCAN_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+        "s_nop 0\n"
         : "+v"(al), "+v"(ah), "+v"(bl), "+v"(bh) : : "vcc");
 #undef TGBM_SCAN_STEP
     a = (long long)((unsigned long long)ah << 32 | al);
