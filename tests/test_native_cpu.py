@@ -1,6 +1,7 @@
 """Host-side parts of the library compiled with g++ against a runtime that the test itself stands in for: no GPU, no
 HIP runtime."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -68,3 +69,18 @@ def test_scans_keep_the_wait_states(tmp_path):
         age = {r: a + 1 for r, a in age.items()}
         age.update({r: 0 for r in written})
     assert carries == 12
+
+
+def test_all_threads_reach_a_function_with_barriers():
+    """A barrier that some threads of a workgroup never come to is undefined: no device function that has one is called under a
+    condition on the thread's number."""
+    csrc = os.path.join(os.path.dirname(HERE), "thundergbm_amd", "csrc")
+    sources = {f: open(os.path.join(csrc, f)).read() for f in sorted(os.listdir(csrc)) if f.endswith((".hip", ".h"))}
+    with_barrier = set()
+    for text in sources.values():
+        for m in re.finditer(r"^(?:template <[^\n]*>\n)?__device__ [^;{]*?(\w+)\([^;{]*\) \{(?:.*?)^\}", text, re.M | re.S):
+            if "__syncthreads" in m.group(0):
+                with_barrier.add(m.group(1))
+    assert {"tree_init_part", "metric_final", "block_sum"} <= with_barrier
+    calls = re.compile(r"if \([^\n]*threadIdx[^\n]*\) (?:%s)[(<]" % "|".join(sorted(with_barrier)))
+    assert {f: c for f, text in sources.items() if (c := calls.findall(text))} == {}

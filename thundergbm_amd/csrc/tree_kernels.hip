@@ -262,20 +262,22 @@ __device__ __forceinline__ int root_chunk(const TreeBuffers &tb) {
 constexpr int kInitNodes = 1024;
 int init_parts(const TreeBuffers &tb) { return (tb.n_nodes + kInitNodes - 1) / kInitNodes; }
 __device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out);
-__device__ void tree_init_part(const TreeBuffers &tb, float lambda, const TreeLeftovers &left, int part, int parts) {  // kBlock threads
+// (the workgroup's first kBlock threads do it; all of its threads call, there are barriers inside)
+__device__ void tree_init_part(const TreeBuffers &tb, float lambda, const TreeLeftovers &left, int part, int parts) {
     if (part == parts) {
         if (blockIdx.z == 0) metric_final(left.metric_kind, tb.n, left.metric_blocks, left.metric_partial, left.metric_out);
         return;
     }
     __shared__ float sg[kWaves], sh[kWaves], mg[kWaves], mh[kWaves], fh[kWaves];
-    if (left.small && part == 0) {  // every row starts in the root
+    const bool on = threadIdx.x < kBlock;
+    if (left.small && part == 0 && on) {  // every row starts in the root
         for (int i = threadIdx.x; i < tb.n; i += kBlock) tb.nid[i] = 0;
     }
-    if ((left.small || left.run > 0) && part == 0)
+    if ((left.small || left.run > 0) && part == 0 && on)
         for (int i = 1 + threadIdx.x; i < tb.depth; i += kBlock) tb.ctl[i] = LevelCtl{left.run, 0, 0, 0};
     const GradStats *__restrict__ block_sums = tb.root_partial;
     const int nn = tb.n_nodes;
-    for (int i = part * kBlock + threadIdx.x; i < nn; i += parts * kBlock) {
+    for (int i = part * kBlock + threadIdx.x; on && i < nn; i += parts * kBlock) {
         TreeNode nd;
         nd.final_id = i;
         nd.parent_index = i == 0 ? -1 : (i - 1) / 2;
@@ -314,7 +316,7 @@ __device__ void tree_init_part(const TreeBuffers &tb, float lambda, const TreeLe
     }
     if (part != 0) return;
     float g = 0, h = 0, gm = 0, hm = 0, hf = 0;
-    for (int i = threadIdx.x; i < tb.n_grad_blocks; i += kBlock) {
+    for (int i = threadIdx.x; on && i < tb.n_grad_blocks; i += kBlock) {
         g += block_sums[i].g;
         h += block_sums[i].h;
         gm = fmaxf(gm, block_sums[i].gmax);
@@ -329,7 +331,7 @@ __device__ void tree_init_part(const TreeBuffers &tb, float lambda, const TreeLe
         hm = fmaxf(hm, __shfl_xor(hm, d));
         hf = fmaxf(hf, __shfl_xor(hf, d));
     }
-    if (lane_id() == 0) {
+    if (on && lane_id() == 0) {
         sg[wave_id()] = g;
         sh[wave_id()] = h;
         mg[wave_id()] = gm;
@@ -543,8 +545,8 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     const int fb = blockIdx.x;
     QuantCtl quant;
     if constexpr (DIRECT) {
-        if (item < root.init_groups) {  // the tree's set-up, by the first block's workgroups (of kBlock threads)
-            if (fb == 0 && threadIdx.x < kBlock) tree_init_part(tb, root.lambda, root.left, item, root.init_parts);
+        if (item < root.init_groups) {  // the tree's set-up, by the first block's workgroups
+            if (fb == 0) tree_init_part(tb, root.lambda, root.left, item, root.init_parts);
             return;
         }
         item -= root.init_groups;
@@ -2469,13 +2471,15 @@ __global__ __launch_bounds__(kCountBlock) void k_metric_count(int kind, int n, i
     }
 }
 
+// (the first kBlock threads' work, as tree_init_part)
 __device__ void metric_final(int kind, int n, int n_blocks, const double *__restrict__ in, float *__restrict__ out) {
     __shared__ double sd[kWaves];
+    const bool on = threadIdx.x < kBlock;
     double acc = 0;
-    for (int i = threadIdx.x; i < n_blocks; i += kBlock) acc += in[i];
+    for (int i = threadIdx.x; on && i < n_blocks; i += kBlock) acc += in[i];
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d);
-    if (lane_id() == 0) sd[wave_id()] = acc;
+    if (on && lane_id() == 0) sd[wave_id()] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0;
