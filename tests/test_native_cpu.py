@@ -42,6 +42,11 @@ def test_kept_device_blocks(run_native):
     run_native("device_pool.cpp")
 
 
+def test_slices_of_a_scoring_call(run_native):
+    """A slice of fewer rows than the kernel of the whole call is for would go to the other one, which is slower there."""
+    run_native("score_slices.cpp")
+
+
 def test_scans_keep_the_wait_states(tmp_path):
     """Hazards inside inline assembly are its author's: gfx950 needs a wait state between a vector instruction that writes vcc
     and one that takes its carry from there, two before a register is read through DPP, one before a lane is read."""

@@ -743,6 +743,8 @@ struct ScoreRows {
 // false: the rows' keys fit no kernel's LDS and nothing was launched.
 bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &model, bool narrow, float lr, float base_score,
                   float *out, size_t out_stride);
+// k_score_rows has room for the model's keys; it then serves kScoreGroupRows rows and more.
+bool score_rows_fit(const ScoreModel &model);
 // Below this many rows k_score_group takes them (see there).
 constexpr int kScoreGroupRows = 65536;
 void launch_predict_transform(hipStream_t s, int kind, int n, int num_class, const float *label, float *y);

@@ -556,6 +556,14 @@ void launch_pack_model(hipStream_t s, const TreeNode *model, long n_total, int n
     k_pack_model<<<(int)std::min<long>((n_total + 255) / 256, 4096), 256, 0, s>>>(model, n_total, n_nodes, packed);
 }
 
+// k_score_rows: 256 rows per workgroup while their vectors take at most 50 KB, else 128
+static int score_block(const ScoreModel &m) { return (size_t)m.n_slots * 256 * sizeof(float) <= 50 * 1024 ? 256 : 128; }
+
+bool score_rows_fit(const ScoreModel &m) {
+    const size_t dense_bytes = (size_t)m.n_slots * score_block(m) * sizeof(float);
+    return dense_bytes <= 50 * 1024 && dense_bytes + (size_t)m.n_nodes * sizeof(uint2) <= 64 * 1024;
+}
+
 bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, bool narrow, float lr, float base_score,
                   float *out, size_t out_stride) {
     if (rows.n == 0) return true;
@@ -565,10 +573,9 @@ bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, boo
     const char *ce = std::getenv("TGBM_PREDICT_COMPACT"), *te = std::getenv("TGBM_PREDICT_TPS");
     const char *ge = std::getenv("TGBM_PREDICT_GROUP");  // 1 / 0: k_score_group always / never where the other serves
     const int fill = ce != nullptr && atoi(ce) == 2 ? 0 : 1;
-    // k_score_rows: 256 rows per workgroup while their vectors take at most 50 KB, else 128
-    const int B = (size_t)m.n_slots * 256 * sizeof(float) <= 50 * 1024 ? 256 : 128;
+    const int B = score_block(m);
     const size_t dense_bytes = (size_t)m.n_slots * B * sizeof(float), tree_bytes = (size_t)m.n_nodes * sizeof(uint2);
-    const bool rows_fit = dense_bytes <= 50 * 1024 && dense_bytes + tree_bytes <= 64 * 1024;
+    const bool rows_fit = score_rows_fit(m);
     // k_score_group
     const size_t sum_bytes = narrow ? sizeof(double) : sizeof(float);
     auto group_bytes = [&](int G) {

@@ -7,6 +7,7 @@
 #include "host.h"
 #include "model_handle.h"
 #include "rank.h"
+#include "score_slices.h"
 
 namespace tgbm {
 
@@ -142,7 +143,9 @@ std::shared_ptr<const DeviceModel> device_model(hipStream_t s, tgbm_model &model
 // Bytes of a slice of rows on their way to the device, see score(). Sparse rows: a walk of k_score_group takes about as long as
 // the slice's values take over PCIe, so an eighth of a call's values is left to walk when the last ones are there (500 k rows
 // of 35 values, 100 trees: 5.4 ms in slices of 64 MB, 4.7 of 32, 4.4 of 16 with every slice a send of its own, 4.3 in one
-// send that has the columns in front). Dense rows: k_score_rows needs many workgroups, slices below 64 MB cost more than they hide
+// send that has the columns in front). Where k_score_rows serves the call no slice has fewer rows than it is for, or the slice would
+// go to k_score_group, which is slower there (500 k rows of 40 values, 90 columns, 100 trees of depth 8: 4.6 ms in eighths, 3.5
+// with at least kScoreGroupRows rows each, and the same in slices of 24 or 64 MB). Dense rows: k_score_rows needs many workgroups, slices below 64 MB cost more than they hide
 // (200 k x 28, 200 trees: 203 us in one launch, 147 for 75 k of the rows).
 constexpr size_t kLeastSlice = (size_t)8 << 20, kMostSlice = (size_t)64 << 20;
 
@@ -371,18 +374,16 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         const long slice_entries = usable ? (long)(std::min(std::max(eighth, kLeastSlice), kMostSlice) / sizeof(float)) : nnz;
         rows.col = d_col;
         rows.val = d_val;
-        for (int r0 = 0; r0 < n;) {
+        const bool by_rows = usable && n >= kScoreGroupRows && score_rows_fit(dm->m);
+        const std::vector<int> first = score_slices(ds.row_ptr, n, slice_entries, by_rows ? kScoreGroupRows : 1);
+        for (size_t k = 0; k + 1 < first.size(); ++k) {
+            const int r0 = first[k], r1 = first[k + 1];
             const long e0 = ds.row_ptr[r0];
-            // last row whose entries still fit the slice (at least one row)
-            const int *from = ds.row_ptr + r0 + 1, *last = ds.row_ptr + n + 1;
-            int r1 = (int)(std::upper_bound(from, last, (int)std::min<long>(e0 + slice_entries, nnz)) - ds.row_ptr) - 1;
-            r1 = std::max(r1, r0 + 1);
             rows.n = r1 - r0;
             rows.row_ptr = d_row_ptr + r0;
             slices.add(d_val + e0, ds.val + e0, sizeof(float) * (size_t)(ds.row_ptr[r1] - e0));
             rows_of.push_back(rows);
             first_of.push_back(r0);
-            r0 = r1;
         }
         slices.send_in_order(s_up, [&](size_t j) {
             if (j >= kBefore) return score_slice(j - kBefore);
