@@ -47,6 +47,22 @@ def test_slices_of_a_scoring_call(run_native):
     run_native("score_slices.cpp")
 
 
+@pytest.fixture(scope="module")
+def transfers(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("native") / "transfer")
+    subprocess.check_call([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "-std=c++17", "-O1", "-w", "-c",
+                           os.path.join(HERE, "native", "transfer.hip"), "-o", exe + ".o"])
+    subprocess.check_call(["g++", exe + ".o", "-pthread", "-ldl", "-Wl,--unresolved-symbols=ignore-in-object-files", "-no-pie", "-o", exe])
+    return exe
+
+
+def test_a_download_waits_on_the_host(transfers):
+    """The copy streams are the process's: a download that has them wait for its own call's kernels holds up every other call's
+    copies."""
+    out = subprocess.run([transfers], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
 def test_scans_keep_the_wait_states(tmp_path):
     """Hazards inside inline assembly are its author's: gfx950 needs a wait state between a vector instruction that writes vcc
     and one that takes its carry from there, two before a register is read through DPP, one before a lane is read."""

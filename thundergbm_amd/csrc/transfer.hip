@@ -357,7 +357,6 @@ void download_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
     hipEvent_t ready;
     HIP_CHECK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
     HIP_CHECK(hipEventRecord(ready, s));
-    for (hipStream_t c : from) HIP_CHECK(hipStreamWaitEvent(c, ready, 0));
     auto work = [&](int t) {
         if (t > 0) HIP_CHECK(hipSetDevice(dev));
         TwoPieces half;
@@ -365,6 +364,8 @@ void download_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
             p = take_piece();
             if (p.in_flight) HIP_CHECK(hipEventSynchronize(p.sent));
         }
+        // (here and not on the copy streams, which are the whole process's: another call's copies would wait for this one's kernels)
+        HIP_CHECK(hipEventSynchronize(ready));
         auto length = [&](size_t c) { return std::min(kDownChunk, bytes - c * kDownChunk); };
         auto request = [&](size_t c, Piece &p, hipStream_t on) {
             HIP_CHECK(hipMemcpyAsync(p.host, static_cast<const char *>(src) + c * kDownChunk, length(c), hipMemcpyDeviceToHost, on));
