@@ -63,6 +63,12 @@ def test_a_download_waits_on_the_host(transfers):
     assert out.returncode == 0, out.stdout + out.stderr
 
 
+def test_transfers_without_threads(transfers):
+    """A process may have no thread left to start: the copies are the caller's work then, and nothing ends the program."""
+    out = subprocess.run([transfers, "no threads"], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
 def test_scans_keep_the_wait_states(tmp_path):
     """Hazards inside inline assembly are its author's: gfx950 needs a wait state between a vector instruction that writes vcc
     and one that takes its carry from there, two before a register is read through DPP, one before a lane is read."""

@@ -14,6 +14,7 @@
 #include <exception>
 #include <map>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -113,8 +114,14 @@ void on_threads(int n, const Work &work) {
         }
     };
     std::vector<std::thread> pool;
-    for (int t = 1; t < n; ++t) pool.emplace_back(guarded, t);
+    pool.reserve((size_t)n);
+    int on = 1;
+    try {
+        for (; on < n; ++on) pool.emplace_back(guarded, on);
+    } catch (const std::system_error &) {  // (no thread is left: the caller does their work as well)
+    }
     guarded(0);
+    for (int t = on; t < n; ++t) guarded(t);
     for (auto &th : pool) th.join();
     if (failed) std::rethrow_exception(failed);
 }
