@@ -204,3 +204,23 @@ def test_first_block_without_bins(n, objective, bins, empty, descending, route, 
     assert np.any(model["split_fid"] >= empty)
     same = [a == b for a, b in zip(*out)]  # (a failed comparison of the bytes themselves is printed for minutes)
     assert all(same), same
+
+
+@pytest.mark.parametrize("n,F", [(500_001, 28), (60_000, 300)])
+def test_work_items_of_the_stages(n, F):
+    """boost() halves the root's work items where the levels below are built by k_split_hist. Stage by stage they are
+    k_hist_dense's, which wants two workgroups per CU."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, F)).astype(np.float32)
+    y = X[:, 0] + np.abs(X[:, 1])
+    s = T.Session(*D.dense_to_csr(X), y, depth=6, n_trees=2, learning_rate=0.5)
+    target = 512 // s.info("dense_blocks")
+    items = []
+    for step in (lambda: s.boost(1), lambda: one_by_one(s, 1, 6, 1)):
+        step()
+        chunk, count = s.get("ctl", np.int32).reshape(-1, 4)[0][:2]
+        assert count == -(-n // chunk)
+        items.append(count)
+    s.close()
+    assert items[0] <= target // 2 < items[1] <= target

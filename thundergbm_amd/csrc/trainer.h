@@ -183,6 +183,8 @@ class Trainer {
     bool small() const { return in_boost_ && small_ok_; }
     int part_bins_[5] = {0};         // most bins of a part of a feature block in 1, 2, 4, 8, 16 parts
     SplitHistPlan run_plan_;         // inside boost() the levels go through launch_partition_hist, runs of so many rows
+    int boost_hitems_ = 0;           // TreeBuffers::target_hitems inside boost(), 0: the buffers' own
+    int hitems() const { return in_boost_ && boost_hitems_ > 0 ? boost_hitems_ : tb_.target_hitems; }
     int run() const { return in_boost_ && !small_ok_ ? run_plan_.run : 0; }
     bool maps_rows() const { return small() || run() > 0; }  // a tree's rows end in tb.nid: launch_map_end
     int lookup_level_ = -1;          // level whose split nodes have not been partitioned into row lists yet

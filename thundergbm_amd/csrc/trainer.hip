@@ -696,10 +696,10 @@ void Trainer::alloc_tree_buffers() {
     const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
     if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
         run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
-    // What target_hitems then plans is the root: a workgroup per CU, each stores a histogram and the atomics of a CU take as long
-    // for two (500 k x 28: histogram 15.6 -> 14.6 us, sums of the items 12.6 -> 8.1; 128 items: 19 and 5.8), unless their
-    // packed sums would have to be drained.
-    if (run_plan_.run > 0 && (long)n_ * n_sets_ <= 256l * kHistFlushRows) tb.target_hitems = std::max(4, tb.target_hitems / 2);
+    // All that target_hitems plans inside boost() then is the root: a workgroup per CU, each stores a histogram and the atomics of
+    // a CU take as long for two (500 k x 28: histogram 15.6 -> 14.6 us, sums of the items 12.6 -> 8.1; 128 items: 19 and 5.8),
+    // unless their packed sums would have to be drained.
+    if (run_plan_.run > 0 && (long)n_ * n_sets_ <= 256l * kHistFlushRows) boost_hitems_ = std::max(4, tb.target_hitems / 2);
     model_cap_trees_ = std::max(1, param_.n_trees) * param_.tree_per_rounds;
     d_model_ = dalloc<TreeNode>((size_t)model_cap_trees_ * tb.n_nodes);
     d_metric_ = dalloc<float>((size_t)std::max(1, param_.n_trees));
@@ -803,7 +803,11 @@ void Trainer::set_option(const std::string &key, double value) {
 }
 
 // Buffer set of class tree k, and the first set with the item target of a whole round built at once.
-TreeBuffers Trainer::set_of(int k) const { return tb_.for_class(n_sets_ > 1 ? k : 0); }
+TreeBuffers Trainer::set_of(int k) const {
+    TreeBuffers t = tb_.for_class(n_sets_ > 1 ? k : 0);
+    t.target_hitems = hitems();
+    return t;
+}
 
 void Trainer::tree_init(int k) {
     if (!in_boost_) ensure_gh_array();
@@ -1195,7 +1199,7 @@ void Trainer::build_round_together() {
     const int K = param_.tree_per_rounds;
     TreeBuffers tb = tb_;
     // the K classes share the chip: size every class's histogram items for its share of the workgroup slots
-    tb.target_hitems = std::max(4, tb_.target_hitems / K);
+    tb.target_hitems = std::max(4, hitems() / K);
     begin_tree(tb, d_gh_, false, K);
     lookup_level_ = -1;
     nid_materialized_ = false;
