@@ -224,3 +224,27 @@ def test_work_items_of_the_stages(n, F):
         items.append(count)
     s.close()
     assert items[0] <= target // 2 < items[1] <= target
+
+
+@pytest.mark.parametrize("n,F,bins,depth,K,served", [(60_000, 100, 16, 8, 1, True), (60_000, 100, 16, 11, 1, False),
+                                                     (60_000, 400, 255, 6, 8, False), (1_048_576, 70, 8, 5, 1, False)])
+def test_room_for_runs_where_there_are_runs(n, F, bins, depth, K, served, monkeypatch):
+    """The workgroups of k_split_hist store more histograms than the other launches' work items where the features have few bins:
+    room for them is taken where that kernel serves the data, and is enough there."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n + K)
+    X = rng.integers(1, bins, (n, F)).astype(np.float32) if bins < 255 else rng.standard_normal((n, F)).astype(np.float32)
+    z = X[:, 0] + 2 * np.abs(X[:, 1])
+    y = z if K == 1 else np.digitize(z, np.quantile(z, np.arange(1, K) / K))
+    kw = dict(depth=depth, n_trees=1, max_num_bin=bins, objective="reg:linear" if K == 1 else "multi:softmax", num_class=K)
+    room = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("TGBM_SPLIT_HIST", switch)
+        s = T.Session(X.reshape(-1), np.arange(0, n * F + 1, F, dtype=np.int32), np.tile(np.arange(F, dtype=np.int32), n), y.astype(np.float32), **kw)
+        room.append(s.info("partial_histograms"))
+        rows = s.info("split_hist_rows")
+        assert (rows > 0) == (served and switch == "1")
+        if rows:
+            assert 2 * room[0] >= n // rows + 2 ** (depth - 2) + 1
+        s.close()
+    assert served or room[0] == room[1]

@@ -497,6 +497,8 @@ struct SplitHistPlan {
     int run = 0, log_split = 0;
     int lds_bins = 0;  // part_bins[log_split]
 };
+// (split_hist_run: the rows as far as what is stored decides them; the plan's are as many or more)
+int split_hist_run(const TreeBuffers &tb, int n_class);
 SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, const int *part_bins, int n_class);
 void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, const SplitHistPlan &plan,
                            float rt_eps, float lambda, int n_class = 1);

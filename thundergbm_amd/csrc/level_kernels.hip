@@ -960,12 +960,17 @@ static int most_partition_items(const TreeBuffers &tb, int level) {
 
 static size_t split_hist_lds(int lds_bins, int run) { return (size_t)lds_bins * 8 + (size_t)run * 4; }
 
+int split_hist_run(const TreeBuffers &tb, int n_class) {
+    if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return 0;
+    for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2)
+        if ((size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class <= kSplitHistBytes) return run;
+    return 0;
+}
+
 SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, const int *part_bins, int n_class) {
     SplitHistPlan plan;
-    if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return plan;
-    for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2) {
+    for (int run = split_hist_run(tb, n_class); run > 0 && run <= kSplitHistMost * kPartChunk; run *= 2) {
         const long runs = (tb.n + run - 1) / run;
-        if ((size_t)runs * tb.n_bins * 8 * n_class > kSplitHistBytes) continue;
         int parts = 0;  // (log2)
         while (4 << (parts + 1) <= bins.W * bins.bin_bytes && (runs * bins.n_blocks * n_class << (parts + 1)) <= kSplitHistGroups) ++parts;
         if (split_hist_lds(part_bins[parts], run) + 4096 > kLdsBytes) continue;

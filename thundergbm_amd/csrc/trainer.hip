@@ -490,11 +490,16 @@ void Trainer::alloc_tree_buffers() {
     tb.max_level_nodes = max_level_nodes;
     tb.target_hitems = std::min(512, std::max(4, 512 / bins_.n_blocks));  // ~2 resident workgroups per CU
     tb.max_hitems = tb.target_hitems + max_pairs + 1;
-    // The runs of split_hist_plan: what they store, packed, in histograms of `partial`'s size.
-    const int max_runs = n_ < kSplitHistRows ? n_ / kPartChunk + max_level_nodes / 2 + 2 : 0;
-    const size_t run_slots = max_runs == 0 ? 0 : kSplitHistBytes / sizeof(longlong2) / (size_t)n_bins_ + (size_t)max_level_nodes / 4 + 2;
+    // The runs of a level that split_hist_plan has, so many buffer sets side by side; they are stored packed, two to a histogram.
+    const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
+    const bool runs_off = sparse_ || (run_env != nullptr && std::string(run_env) == "0");
+    auto runs_of = [&](int sets) {
+        const int run = runs_off ? 0 : split_hist_run(tb, sets);
+        return run == 0 ? 0 : n_ / run + max_level_nodes / 2 + 2;
+    };
+    const size_t run_slots = ((size_t)runs_of(1) + 1) / 2;
     tb.max_pitems = n_ / kPartChunk + max_level_nodes + 1;
-    tb.n_partial = sparse_ ? 1 : std::max((size_t)tb.max_hitems, run_slots) * n_bins_;
+    tb.n_partial = sparse_ ? 1 : (size_t)tb.max_hitems * n_bins_;
     tb.n_end_bound = ((size_t)row_blocks(n_) + 1) * (((size_t)1 << depth) - 1);
     tb.n_grad_blocks = row_blocks(n_);
     // One set of buffers per class tree of a round when that fits comfortably: the trees of a round are
@@ -546,6 +551,8 @@ void Trainer::alloc_tree_buffers() {
     n_sets_ = (K > 1 && set_bytes * K < free_b / 2 && !(be != nullptr && std::string(be) == "0")) ? K : 1;
     tb.n_sets = n_sets_;
     const size_t S = (size_t)n_sets_;
+    const int max_runs = hist_cap_level_ < 0 ? runs_of(n_sets_) : 0;
+    if (!sparse_) tb.n_partial = std::max(tb.n_partial, ((size_t)max_runs + 1) / 2 * n_bins_);
     tb.nodes = dalloc<TreeNode>(S * tb.n_nodes);
     tb.seg = dalloc<int2>(S * tb.n_nodes);
     tb.nid = dalloc<int>(S * n_);
@@ -693,9 +700,7 @@ void Trainer::alloc_tree_buffers() {
     const size_t small_cands = S * (size_t)max_level_nodes * bins_.n_cols;
     if (small_ok_ && !wide_eval_ && small_cands * sizeof(SplitCand) <= (size_t)64 << 20)
         for (SplitCand *&c : small_cand_) c = dalloc<SplitCand>(small_cands);
-    const char *run_env = std::getenv("TGBM_SPLIT_HIST");  // "0": lists and histograms by launches of their own (tests)
-    if (!sparse_ && hist_cap_level_ < 0 && !(run_env != nullptr && std::string(run_env) == "0"))
-        run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
+    if (max_runs > 0) run_plan_ = split_hist_plan(tb, bins_, part_bins_, n_sets_);
     // All that target_hitems plans inside boost() then is the root: a workgroup per CU, each stores a histogram and the atomics of
     // a CU take as long for two (500 k x 28: histogram 15.6 -> 14.6 us, sums of the items 12.6 -> 8.1; 128 items: 19 and 5.8),
     // unless their packed sums would have to be drained.
@@ -1503,6 +1508,9 @@ int Trainer::info(const std::string &key) const {
     if (key == "depth") return param_.depth;
     if (key == "y_pred_size") return (int)n_yp_;
     if (key == "max_hitems") return tb_.max_hitems;
+    if (key == "partial_histograms") return (int)(tb_.n_partial / (size_t)n_bins_);
+    if (key == "small_levels") return small_ok_ ? 1 : 0;                 // boost() builds the levels by k_small_level,
+    if (key == "split_hist_rows") return small_ok_ ? 0 : run_plan_.run;  // else by k_split_hist, so many rows a workgroup (0: neither)
     fatal("unknown info key %s", key.c_str());
 }
 
