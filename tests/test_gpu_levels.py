@@ -248,3 +248,20 @@ def test_room_for_runs_where_there_are_runs(n, F, bins, depth, K, served, monkey
             assert 2 * room[0] >= n // rows + 2 ** (depth - 2) + 1
         s.close()
     assert served or room[0] == room[1]
+
+
+@pytest.mark.parametrize("n,switch,own", [(5_000, "TGBM_SMALL", False), (40_000, "TGBM_SPLIT_HIST", False), (40_000, "TGBM_SPLIT_HIST", True)])
+def test_profile_counts_histogram_launches(n, switch, own, monkeypatch):
+    """Levels whose histograms are built by the partition's launch have no histogram launch, time or bytes of their own."""
+    import thundergbm_amd as T
+    monkeypatch.setenv(switch, "0" if own else "1")
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 12)).astype(np.float32)
+    s = T.Session(*D.dense_to_csr(X), X[:, 0] + np.abs(X[:, 1]), depth=5, n_trees=3)
+    s.set_profiling(True)
+    s.boost(3)
+    hist = s.phase_profile()["hist"]
+    s.close()
+    assert hist["root"]["launches"] == 3 and hist["root"]["bytes"] == 3 * n * (12 + 8)
+    assert hist["below_root"]["launches"] == (12 if own else 0)
+    assert (hist["below_root"]["bytes"] > 0) == own and (hist["below_root"]["ms"] > 0) == own

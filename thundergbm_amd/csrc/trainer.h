@@ -201,6 +201,7 @@ class Trainer {
     long long prof_rounds_ = 0;
     void mark(int phase, int level = -1);
     std::vector<LevelCtl> ctl_log_;  // per tree, depth + 1 entries (copied at tree end when profiling)
+    std::vector<char> ctl_log_maps_;  // per tree: maps_rows()
     HistProfile prof_;
 };
 

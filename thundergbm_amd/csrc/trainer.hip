@@ -1052,8 +1052,10 @@ void Trainer::find_split_sets(const TreeBuffers &tb, const GHPair *gh, int level
     const bool derive = small() && level > 0;  // the level before has built its histograms
     // the root's sums ride in the launches of its histograms and of its split search (all nodes of the level at once)
     const bool sum_rows = !sparse_ && level == 0 && hist_cap_level_ != 0 && tb.complete_feature < 0;
-    if (!derive && !(run() > 0 && level > 0)) build_level_hist(tb, level, gh, n_class, sum_rows);
-    mark(PH_HIST, level);
+    if (!derive && !(run() > 0 && level > 0)) {
+        build_level_hist(tb, level, gh, n_class, sum_rows);
+        mark(PH_HIST, level);
+    }
     if (!sparse_pass_ && !searched_) {
         // (a capped arena's deeper levels come in batches, and its last level with parents keeps its histograms)
         const bool fused = !sparse_ && !derive && !wide_eval_ && hist_cap_level_ < 0;
@@ -1139,6 +1141,7 @@ void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level,
 void Trainer::log_plan(const TreeBuffers &tb) {
     size_t off = ctl_log_.size();
     ctl_log_.resize(off + param_.depth + 1);
+    ctl_log_maps_.push_back(maps_rows());
     if (sparse_pass_) {
         // rows of the nodes the reference would build from rows: the root, then the smaller child of every pair
         std::vector<int> rows((size_t)tb.n_nodes);
@@ -1470,6 +1473,7 @@ HistProfile Trainer::profile() {
                 b = (long long)((double)c.rows_built * ((double)nnz_ / n_ * 4 + 8 + 8 + (level > 0 ? 4 : 0)));
             else
                 b = (long long)c.rows_built * (F_ * bins_.bin_bytes + 8 + (level > 0 ? 4 : 0));
+            if (level > 0 && ctl_log_maps_[t]) continue;  // (part of the partition's launches: no time of their own either)
             p.hist_bytes += b;
             (level == 0 ? p.root_bytes : p.below_bytes) += b;
         }

@@ -198,7 +198,7 @@ class Session:
 
     def phase_profile(self):
         """Per-stage milliseconds of the rounds boosted with profiling on, and the histogram launches split into the
-        root level and the levels below it."""
+        root level and the levels below it (where those are launches of their own: else they are part of "partition")."""
         out = np.zeros(15, dtype=np.float64)
         self.L.tgbm_trainer_get_phase_profile(self.h, _p(out), 15)
         split = {}
