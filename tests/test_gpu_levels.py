@@ -265,3 +265,34 @@ def test_profile_counts_histogram_launches(n, switch, own, monkeypatch):
     assert hist["root"]["launches"] == 3 and hist["root"]["bytes"] == 3 * n * (12 + 8)
     assert hist["below_root"]["launches"] == (12 if own else 0)
     assert (hist["below_root"]["bytes"] > 0) == own and (hist["below_root"]["ms"] > 0) == own
+
+
+@pytest.mark.parametrize("n,objective", [(60_000, "reg:linear"), (80_001, "binary:logistic")])
+def test_merge_and_search_of_many_items_of_wide_features(n, objective):
+    """k_merge_eval_wide with sixteen wavefronts, for more than eight work items a pair, 1 to 4 quarters of 256 bins (three leave a
+    wavefront without any), against k_hist_merge and k_eval_split_wide: a column of more than kMergeWideBins bins sends all of them
+    there. No split of it leaves enough rows on both sides."""
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    counts = [256, 257, 512, 513, 700, 768, 769, 1023, 1024]
+    X = np.zeros((n, len(counts) + 1), np.float32)
+    for f, c in enumerate(counts):
+        X[:, f] = rng.permutation(np.arange(n) % c) + 1
+    X[rng.random(X.shape) < 0.1] = 0
+    X[:, -1] = 0
+    X[rng.choice(n, 1_500, replace=False), -1] = np.arange(1_500) + 1
+    z = X[:, 4] / 700 + np.abs(X[:, 7] / 1023 - 0.5) + X[:, 0] / 256 * (X[:, 3] > 200) + 0.3 * rng.standard_normal(n)
+    y = (z if objective == "reg:linear" else z > 1).astype(np.float32)
+    out = []
+    for columns in (len(counts), len(counts) + 1):
+        s = T.Session(*D.dense_to_csr(X[:, :columns]), y, depth=5, n_trees=3, learning_rate=0.5, max_num_bin=1_500, objective=objective,
+                      min_child_weight=1_501 if objective == "reg:linear" else 376)
+        bins = np.diff(s.cuts()[1])
+        assert bins[:len(counts)].tolist() == counts and (columns == len(counts) or bins[-1] == 1_500)
+        assert s.info("split_hist_rows") > 0 and n // s.info("split_hist_rows") > 8
+        s.boost(3)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes()))
+        assert len(np.unique(s.model()["split_fid"])) > 3
+        s.close()
+    same = [a == b for a, b in zip(*out)]
+    assert all(same), same
