@@ -503,6 +503,7 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_level(TreeBuffers tb_all, i
 constexpr int kSmallWaves = kSmallBlock / 64;
 constexpr size_t kSmallSearchBytes = sizeof(longlong2) * kEvalPackBins * kSmallWaves;
 constexpr int kSmallSteps = kSmallRows / kSmallBlock;
+static_assert(kSmallRowsWide <= 8 * kSmallBlock, "the steps that 16-bit bins have code for");
 static_assert(kSmallRows / 2 <= kHistFlushRows, "the built child's packed sums are never drained");
 static_assert(kSmallRows <= 1 << 16 && kSmallWaves == 16 && kSmallSteps % 4 == 0, "16-bit row ids, the counts of four steps per wavefront");
 
@@ -658,19 +659,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
         for (int u = 0; u < U; ++u) {
             if (base + u * RPS >= m) break;  // (uniform)
             const unsigned v = base + rsub + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
-            const long long gq = round_to_ll(s[u].g * scale_g), hq = round_to_ll(fmaxf(s[u].h, 0.f) * scale_h);
-            const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
-            if (BIN16) {
-                const unsigned b0 = v & 0xffff, b1 = v >> 16;
-                if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
-            } else {
-                const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
-                if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
-                if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
-                if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
-            }
+            add_row<BIN16>(lds, v, s[u], scale_g, scale_h, h_bits, o0, o1, o2, o3);
         }
     }
     __syncthreads();
@@ -931,19 +920,7 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
             if (base + u * RPS >= m) break;  // (uniform)
             const GHPair sv = GHW ? pair_from_word(bins.gh_objective, __float_as_uint(s[u].g)) : s[u];
             const unsigned v = base + rsub + u * RPS < m && !word_lane ? pk[u] : 0xffffffffu;
-            const long long gq = round_to_ll(sv.g * scale_g), hq = round_to_ll(fmaxf(sv.h, 0.f) * scale_h);
-            const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
-            if (BIN16) {
-                const unsigned b0 = v & 0xffff, b1 = v >> 16;
-                if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
-            } else {
-                const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
-                if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
-                if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
-                if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
-            }
+            add_row<BIN16>(lds, v, sv, scale_g, scale_h, h_bits, o0, o1, o2, o3);
         }
     }
     __syncthreads();
@@ -1093,7 +1070,8 @@ static void small_level_steps(hipStream_t s, const TreeBuffers &tb, const DenseB
     if (steps <= 2) small_level_launch<LPR, BIN16, 2, SEARCH>(s, tb, bins, gh, l);
     else if (steps <= 4) small_level_launch<LPR, BIN16, 4, SEARCH>(s, tb, bins, gh, l);
     else if (steps <= 8) small_level_launch<LPR, BIN16, 8, SEARCH>(s, tb, bins, gh, l);
-    else small_level_launch<LPR, BIN16, kSmallSteps, SEARCH>(s, tb, bins, gh, l);
+    else if constexpr (!BIN16) small_level_launch<LPR, BIN16, kSmallSteps, SEARCH>(s, tb, bins, gh, l);
+    else fatal("%d rows of 16-bit bins", tb.n);
 }
 
 bool launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, const GHPair *gh, int level, float rt_eps,

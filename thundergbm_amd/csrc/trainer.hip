@@ -696,7 +696,7 @@ void Trainer::alloc_tree_buffers() {
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors above go out of scope
 
     const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
-    small_ok_ = !sparse_ && hist_cap_level_ < 0 && n_ <= (wide_eval_ ? kSmallRowsWide : kSmallRows) && small_levels_fit(tb) && !(small_env != nullptr && std::string(small_env) == "0");
+    small_ok_ = !sparse_ && hist_cap_level_ < 0 && n_ <= (bins_.bin_bytes == 2 ? kSmallRowsWide : kSmallRows) && small_levels_fit(tb) && !(small_env != nullptr && std::string(small_env) == "0");
     const size_t small_cands = S * (size_t)max_level_nodes * bins_.n_cols;
     if (small_ok_ && !wide_eval_ && small_cands * sizeof(SplitCand) <= (size_t)64 << 20)
         for (SplitCand *&c : small_cand_) c = dalloc<SplitCand>(small_cands);

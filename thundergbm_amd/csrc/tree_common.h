@@ -217,6 +217,26 @@ __device__ __forceinline__ GHPair pair_from_word(int objective, unsigned w) {
     return o;
 }
 
+// What a lane's columns of a row (v: two bins of 16 bits or four of 8) add to their bins in LDS: exact products (the scales are
+// powers of two), rounded once to the nearest integer, the hessian's in the low h_bits.
+template <bool BIN16>
+__device__ __forceinline__ void add_row(unsigned long long *lds, unsigned v, GHPair p, float scale_g, float scale_h, int h_bits, int o0, int o1,
+                                        int o2, int o3) {
+    const long long gq = round_to_ll(p.g * scale_g), hq = round_to_ll(fmaxf(p.h, 0.f) * scale_h);
+    const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
+    if (BIN16) {
+        const unsigned b0 = v & 0xffff, b1 = v >> 16;
+        if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
+        if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
+    } else {
+        const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
+        if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
+        if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
+        if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
+        if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
+    }
+}
+
 // The value that the last of the LPR lanes of a row holds, in every lane of the row (LPR = 4, 8 or 16 consecutive
 // lanes): a DPP broadcast inside the 16-lane row of the wavefront, no trip through the LDS crossbar.
 template <int LPR>

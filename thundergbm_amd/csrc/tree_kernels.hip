@@ -697,21 +697,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
                 sv = pair_from_word(gh_objective, last_lane_of_row<LPR>(pk[u]));
             }
             if (word_lane) v = 0xffffffffu;  // (that lane's dword holds no bins, whether the word is used or not)
-            // exact products (the scales are powers of two), rounded once to the nearest integer
-            const long long gq = round_to_ll(sv.g * scale_g);
-            const long long hq = round_to_ll(fmaxf(sv.h, 0.f) * scale_h);
-            const unsigned long long add = ((unsigned long long)gq << h_bits) + (unsigned long long)hq;
-            if (BIN16) {
-                const unsigned b0 = v & 0xffff, b1 = v >> 16;
-                if (b0 != kMissingBin16) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin16) atomicAdd(lds + o1 + b1, add);
-            } else {
-                const unsigned b0 = v & 0xff, b1 = (v >> 8) & 0xff, b2 = (v >> 16) & 0xff, b3 = v >> 24;
-                if (b0 != kMissingBin) atomicAdd(lds + o0 + b0, add);
-                if (b1 != kMissingBin) atomicAdd(lds + o1 + b1, add);
-                if (b2 != kMissingBin) atomicAdd(lds + o2 + b2, add);
-                if (b3 != kMissingBin) atomicAdd(lds + o3 + b3, add);
-            }
+            add_row<BIN16>(lds, v, sv, scale_g, scale_h, h_bits, o0, o1, o2, o3);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
