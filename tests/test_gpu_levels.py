@@ -81,11 +81,13 @@ def test_rows_of_nodes_of_many_items(n):
     s.close()
 
 
-@pytest.mark.parametrize("n,F,depth,bins,objective,missing", [
-    (16_385, 4, 8, 255, "binary:logistic", 0.0), (30_000, 3, 10, 16, "reg:linear", 0.3), (20_480, 30, 5, 63, "binary:logistic", 0.1),
-    (70_001, 9, 8, 1000, "reg:linear", 0.1), (100_000, 21, 7, 255, "multi:softmax", 0.1), (240_000, 28, 8, 255, "reg:logistic", 0.0),
-    (500_001, 28, 8, 255, "binary:logistic", 0.05), (50_000, 260, 6, 255, "reg:linear", 0.0), (1_048_575, 16, 7, 255, "reg:linear", 0.0)])
-def test_lists_and_histograms_in_one_launch(n, F, depth, bins, objective, missing, monkeypatch):
+@pytest.mark.parametrize("items,n,F,depth,bins,objective,missing", [
+    (1, 16_385, 4, 8, 255, "binary:logistic", 0.0), (1, 30_000, 3, 10, 16, "reg:linear", 0.3), (1, 20_480, 30, 5, 63, "binary:logistic", 0.1),
+    (1, 65_535, 9, 8, 1000, "reg:linear", 0.1), (2, 65_536, 21, 7, 255, "multi:softmax", 0.1), (2, 240_000, 28, 8, 255, "reg:logistic", 0.0),
+    (2, 70_001, 9, 8, 1000, "reg:linear", 0.1), (2, 500_001, 28, 8, 255, "binary:logistic", 0.05), (2, 50_000, 260, 6, 255, "reg:linear", 0.0),
+    (2, 1_048_575, 16, 7, 255, "reg:linear", 0.0), (4, 1_000_001, 28, 7, 255, "binary:logistic", 0.0), (4, 70_001, 400, 5, 255, "reg:linear", 0.1),
+    (4, 300_001, 28, 6, 1000, "reg:linear", 0.1)])
+def test_lists_and_histograms_in_one_launch(items, n, F, depth, bins, objective, missing, monkeypatch):
     """k_split_hist against the scatter and histogram launches: 1, 2 and 4 partition items a workgroup, records with and
     without gradient words, 16-bit bins, several blocks, class trees, sorted rows (all rows of a child in one workgroup)."""
     import thundergbm_amd as T
@@ -101,10 +103,12 @@ def test_lists_and_histograms_in_one_launch(n, F, depth, bins, objective, missin
         monkeypatch.setenv("TGBM_SPLIT_HIST", switch)
         s = T.Session(val, rp, col, np.asarray(y, np.float32), depth=depth, n_trees=3, learning_rate=0.5, max_num_bin=bins,
                       objective=objective)
+        assert s.info("split_hist_rows") == (2048 * items if switch == "1" else 0)
         s.boost(3)
         out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes(), s.metric_log().tobytes()))
         s.close()
-    assert out[0] == out[1]
+    same = [a == b for a, b in zip(*out)]
+    assert all(same), same
 
 
 @pytest.mark.parametrize("n,depth,bins,objective,rate", [

@@ -79,14 +79,21 @@ constexpr int kPartGroupRows = 1 << 24;
 constexpr int kPartGroup = 64;
 // Dense layout, below so many rows (from there on the rows are re-ordered by leaves: those of a child follow each other, and
 // one workgroup has them all): a level's row lists and the next level's histograms in one launch (launch_partition_hist), by
-// workgroups of 1, 2 or 4 partition items, as few as keep the histograms that they store below kSplitHistBytes. Beyond, storing
-// and reading them back takes longer than more workgroups save, and where four items are not enough the launches for many
-// rows are as fast. ms a tree with 1, 2, 4 items and with launch_hist_dense: 100 k x 28 (3 MB with 1): 0.216, 0.232, 0.269, 0.236;
-// 500 k x 28 (14 MB): 0.270, 0.265, 0.296, 0.281; 900 k x 28 (25 MB): 0.318, 0.298, 0.311, 0.329; 50 k x 700 (36 MB): 0.295, 0.290,
-// 0.275, 0.294; 500 k x 54, 8 classes (41 MB): 0.631, 0.534, 0.515, 0.543; 400 k x 60, 6 classes (144 MB): 0.71, 0.62, 0.556, 0.529.
+// workgroups of 1, 2 or 4 partition items. As long as a block's columns can be shared out instead (kSplitHistGroups) fewer items
+// give as many workgroups and less to store and read back, so it is 2 items; 1 on few rows that store little, where a part of
+// fewer columns would be laid out again by too many workgroups of the deep levels; 4 where 2 store more than kSplitHistBytes. Where
+// 4 do, the launches for many rows are as fast. ms a tree (depth 8, 6 of the wide ones) with launch_hist_dense, 1, 2, 4 items:
+// 20 k x 28 (MB that 1 stores: 0.6) 0.201, 0.154, 0.157; 20 k x 136 (2.8) 0.254, 0.214, 0.234, 0.248; 50 k x 12, 8 classes (4.9) 0.263, 0.234, 0.248;
+// 20 k x 300 (6.1) 0.201, 0.168, 0.167; 60 k x 136 (8.3) 0.281, 0.242, 0.229, 0.253; 34 k x 300 (10.4) 0.209, 0.180, 0.173;
+// 100 k x 28 (2.8) 0.237, 0.198, 0.197, 0.202; 900 k x 4 (3.6) 0.268, 0.262, 0.233, 0.238; 150 k x 28 (4.2) 0.241, 0.205, 0.197, 0.208;
+// 900 k x 10 (9.0) 0.275, 0.291, 0.251, 0.257; 78 k x 37 of 1024 bins (11.5) 0.231, 0.224, 0.203, 0.212; 500 k x 28 (14) 0.274, 0.267, 0.243, 0.253;
+// 200 k x 136 (27) 0.330, 0.310, 0.309, 0.315; 1 M x 28 (28) 0.327, 0.347, 0.304, 0.308; 100 k x 300 (30) 0.245, 0.242, 0.228, 0.218;
+// 300 k x 28 of 1024 bins (34) 0.320, 0.366, 0.332, 0.286; 50 k x 700 (36) 0.276, 0.281, 0.274, 0.256; 400 k x 30, 6 classes (72) 0.520, 0.600, 0.528, 0.538.
 constexpr int kSplitHistRows = 1 << 20;
 constexpr int kSplitHistMost = 4;
 constexpr size_t kSplitHistBytes = 13 << 20;
+constexpr int kSplitHistOneRows = 1 << 16;
+constexpr size_t kSplitHistOneBytes = 6 << 20;
 // A workgroup's LDS adds about 8 pairs a nanosecond, so up to a workgroup per CU a block's columns are shared out as well
 // (each part lays the lists out again): 20 k x 28 0.128 -> 0.111 ms a tree, 100 k x 28 0.198 -> 0.187, 500 k x 28 0.251 -> 0.246; with two per
 // CU 0.111, 0.200 and 0.279.

@@ -939,8 +939,10 @@ static size_t split_hist_lds(int lds_bins, int run) { return (size_t)lds_bins * 
 
 int split_hist_run(const TreeBuffers &tb, int n_class) {
     if (tb.n >= kSplitHistRows || tb.depth > kSmallDepth || tb.planned(tb.depth - 1)) return 0;
-    for (int run = kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2)
-        if ((size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class <= kSplitHistBytes) return run;
+    auto stored = [&](int run) { return (size_t)((tb.n + run - 1) / run) * tb.n_bins * 8 * n_class; };
+    if (tb.n < kSplitHistOneRows && stored(kPartChunk) <= kSplitHistOneBytes) return kPartChunk;
+    for (int run = 2 * kPartChunk; run <= kSplitHistMost * kPartChunk; run *= 2)
+        if (stored(run) <= kSplitHistBytes) return run;
     return 0;
 }
 
