@@ -56,7 +56,7 @@ def transfers(tmp_path_factory):
     return exe
 
 
-def test_a_download_waits_on_the_host(transfers):
+def test_a_download_keeps_off_the_copy_streams(transfers):
     """The copy streams are the process's: a download that has them wait for its own call's kernels holds up every other call's
     copies."""
     out = subprocess.run([transfers], capture_output=True, text=True, timeout=60)

@@ -685,8 +685,9 @@ class UploadSet {
     std::vector<Job> jobs_;
     std::vector<Columns> columns_;
 };
-// Device -> pageable host memory after what is queued on s; the bytes are there when the call returns.
-void download_large(hipStream_t s, void *dst, const void *src, size_t bytes);
+// Device -> pageable host memory after what is queued on s; the bytes are there when the call returns. other: a second stream of
+// the caller's.
+void download_large(hipStream_t s, hipStream_t other, void *dst, const void *src, size_t bytes);
 // The conversion alone, for arrays that the device reads from host memory.
 void doubles_to_floats(float *to, const double *from, size_t count);
 // A pinned block of kPinnedBytes that the device can read and write directly; kept for later calls.

@@ -429,7 +429,7 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         n_ret = transform_scores(s, param, ds, n, n_class, d_out, d_label);
     }
     HIP_CHECK_LAUNCHES("predict (metric, transform)");
-    download_large(s, out, d_out, sizeof(float) * n_ret);
+    download_large(s, s_up, out, d_out, sizeof(float) * n_ret);
     HIP_CHECK(hipStreamSynchronize(s_up));
     HIP_CHECK(hipEventDestroy(up));
     lap("traversal, transform and download");

@@ -350,7 +350,7 @@ void UploadSet::send_in_order(hipStream_t s, const std::function<void(size_t)> &
 constexpr size_t kDownChunk = (size_t)512 << 10;
 constexpr size_t kDownStaged = (size_t)1 << 20;
 
-void download_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
+void download_large(hipStream_t s, hipStream_t other, void *dst, const void *src, size_t bytes) {
     if (bytes < kDownStaged) {
         if (bytes) HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipStreamSynchronize(s));
@@ -360,10 +360,12 @@ void download_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
     const int n_thr = (int)std::min<size_t>(4, (chunks + 1) / 2);
     int dev = 0;
     HIP_CHECK(hipGetDevice(&dev));
-    const std::array<hipStream_t, 2> from = copy_streams(dev);
+    // (the call's own streams: on the copy streams, which are the whole process's, other calls' copies would wait for its kernels)
+    const std::array<hipStream_t, 2> from{s, other};
     hipEvent_t ready;
     HIP_CHECK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
     HIP_CHECK(hipEventRecord(ready, s));
+    HIP_CHECK(hipStreamWaitEvent(other, ready, 0));
     auto work = [&](int t) {
         if (t > 0) HIP_CHECK(hipSetDevice(dev));
         TwoPieces half;
@@ -371,8 +373,6 @@ void download_large(hipStream_t s, void *dst, const void *src, size_t bytes) {
             p = take_piece();
             if (p.in_flight) HIP_CHECK(hipEventSynchronize(p.sent));
         }
-        // (here and not on the copy streams, which are the whole process's: another call's copies would wait for this one's kernels)
-        HIP_CHECK(hipEventSynchronize(ready));
         auto length = [&](size_t c) { return std::min(kDownChunk, bytes - c * kDownChunk); };
         auto request = [&](size_t c, Piece &p, hipStream_t on) {
             HIP_CHECK(hipMemcpyAsync(p.host, static_cast<const char *>(src) + c * kDownChunk, length(c), hipMemcpyDeviceToHost, on));
