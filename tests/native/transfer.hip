@@ -12,6 +12,7 @@
 namespace {
 std::atomic<bool> busy{false};                // the caller's stream has a kernel to run
 std::atomic<int> held_up{0}, too_early{0};    // waits for it on a shared stream, copies of its results that do not wait for it
+std::atomic<int> caller_waits{0};             // of the caller's stream for a copy stream
 std::atomic<bool> no_threads{false};
 std::atomic<size_t> handles{0};
 hipStream_t const kCaller = reinterpret_cast<hipStream_t>((size_t)1 << 40), kOther = reinterpret_cast<hipStream_t>((size_t)2 << 40);
@@ -47,6 +48,7 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    if (s == kCaller) ++caller_waits;
     if (s == kOther) other_waits = other_waits || e == of_caller;
     else if (s != kCaller && e == of_caller && busy) ++held_up;
     return hipSuccess;
@@ -93,7 +95,15 @@ int main(int argc, char **argv) {
     UploadSet set;
     for (size_t j = 0; j < 8; ++j) set.add(to.data() + j * ((size_t)5 << 20), from.data() + j * ((size_t)5 << 20), (size_t)5 << 20);
     set.send_in_order(kCaller, [&](size_t j) { arrived += j == arrived; });
-    CHECK(arrived == 8 && to == from);
+    CHECK(arrived == 8 && to == from && caller_waits <= 2 * 8 + 2 * 3);  // (3: upload_large above, where it is staged)
+    // a small array: the caller's stream waits for the two copy streams once, whoever else does
+    const std::vector<double> x(1000, 0.5);
+    std::vector<float> f(x.size());
+    UploadSet one;
+    one.add_doubles(f.data(), x.data(), x.size());
+    caller_waits = 0;
+    one.send_in_order(kCaller, [&](size_t) { arrived += caller_waits == 2; });
+    CHECK(arrived == 9 && caller_waits == 2 && f.back() == 0.5f);
     std::printf("ok\n");
     return 0;
 }

@@ -58,7 +58,7 @@ def transfers(tmp_path_factory):
 
 def test_a_download_keeps_off_the_copy_streams(transfers):
     """The copy streams are the process's: a download that has them wait for its own call's kernels holds up every other call's
-    copies."""
+    copies. And a small upload pays for one round of waits."""
     out = subprocess.run([transfers], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
 

@@ -167,9 +167,12 @@ void send_jobs(hipStream_t s, const std::vector<UploadSet::Job> &jobs, int threa
     size_t told = 0;  // jobs that `arrived` has been called for
     auto tell = [&] {
         std::lock_guard<std::mutex> lock(arrival);
-        for (; told < jobs.size() && unsent[told] == 0; ++told) {
-            let_wait();  // (all copies of this job are queued - those of the next one may not have been when the last wait was)
-            (*arrived)(told);
+        for (;;) {  // (while the calls below run, other threads may have queued the last copies of the next ones)
+            size_t upto = told;
+            while (upto < jobs.size() && unsent[upto] == 0) ++upto;
+            if (upto == told) return;
+            let_wait();  // (all copies of these jobs are queued - those of the next one may not have been when the last wait was)
+            for (; told < upto; ++told) (*arrived)(told);
         }
     };
     if (arrived != nullptr) tell();  // (jobs without a byte)
@@ -191,7 +194,7 @@ void send_jobs(hipStream_t s, const std::vector<UploadSet::Job> &jobs, int threa
         }
     };
     on_threads(n_thr, work);
-    let_wait();
+    if (arrived == nullptr) let_wait();  // (else it has happened after the last copy)
     for (hipEvent_t e : order) HIP_CHECK(hipEventDestroy(e));
 }
 
