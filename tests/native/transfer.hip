@@ -104,6 +104,12 @@ int main(int argc, char **argv) {
     caller_waits = 0;
     one.send_in_order(kCaller, [&](size_t) { arrived += caller_waits == 2; });
     CHECK(arrived == 9 && caller_waits == 2 && f.back() == 0.5f);
+    // arrays that hipMemcpy takes as fast as the pieces do go without them
+    UploadSet few;
+    for (size_t j = 0; j < 2; ++j) few.add(to.data() + j * ((size_t)7 << 20), from.data(), (size_t)7 << 20);
+    caller_waits = 0;
+    few.send_in_order(kCaller, [&](size_t) { ++arrived; });
+    CHECK(arrived == 11 && caller_waits == 0 && std::memcmp(to.data() + ((size_t)7 << 20), from.data(), (size_t)7 << 20) == 0);
     std::printf("ok\n");
     return 0;
 }
