@@ -300,3 +300,41 @@ def test_merge_and_search_of_many_items_of_wide_features(n, objective):
         s.close()
     same = [a == b for a, b in zip(*out)]
     assert all(same), same
+
+
+@pytest.mark.parametrize("n,F,per_row,objective", [(120_000, 2_823, 20, "binary:logistic"), (540_000, 6, 0, "multi:softmax")])
+def test_root_of_drained_items(n, F, per_row, objective, monkeypatch):
+    """k_merge_eval at the root where the work items have more rows than the LDS adds up packed (few items: many feature blocks or
+    classes) and no feature is stored in every row, against k_hist_merge and k_eval_split (an arena that is too small for the last level)."""
+    import thundergbm_amd as T
+    monkeypatch.setenv("TGBM_LAYOUT", "dense")
+    rng = np.random.default_rng(n)
+    if per_row:
+        col = np.minimum(F * rng.random((n, per_row)) ** 3, F - 1).astype(np.int32)
+        col.sort(axis=1)
+        keep = np.ones(col.shape, bool)
+        keep[:, 1:] = col[:, 1:] != col[:, :-1]
+        rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+        z = 0.3 * (col % 7 == 0).sum(1) - 0.2 * (col < 40).sum(1) + 0.5 * rng.standard_normal(n)
+        col = col[keep]
+        val = np.exp(rng.standard_normal(col.size)).astype(np.float32)
+    else:
+        X = rng.standard_normal((n, F)).astype(np.float32)
+        X[rng.random(X.shape) < 0.1] = 0
+        z = X[:, 0] + np.abs(X[:, 1])
+        val, rp, col = D.dense_to_csr(X)
+    K = 8 if objective.startswith("multi") else 1
+    y = np.digitize(z, np.quantile(z, np.arange(1, K) / K)) if K > 1 else z > np.median(z)
+    out = []
+    for nodes in (None, None, "4"):
+        if nodes:
+            monkeypatch.setenv("TGBM_HIST_ARENA_NODES", nodes)
+        s = T.Session(val, rp, col, y.astype(np.float32), depth=4, n_trees=2, learning_rate=0.3, objective=objective, num_class=K)
+        s.boost(2)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes()))
+        if nodes is None:
+            chunk, items = s.get("ctl", np.int32).reshape(-1, 4)[0][:2]
+            assert chunk > 8192 and items <= 64
+        s.close()
+    same = [[a == b for a, b in zip(o, out[-1])] for o in out[:-1]]
+    assert np.all(same), same
