@@ -154,3 +154,15 @@ def test_no_64_bit_shift_by_the_last_register(tmp_path):
                 if int(m.group(1)) + 1 >= count[kernel]:
                     found.append((kernel, line.strip()))
     assert shifts > 500 and found == []
+
+
+def test_sparse_moves_whatever_thread_is_first(run_native, tmp_path):
+    """k_sparse_partition stores the rows' new nodes while slower threads still load: a thread past the last row that looks the last
+    row's node up may find a child's, which has no entry among the level's."""
+    source = open(os.path.join(os.path.dirname(HERE), "thundergbm_amd", "csrc", "sparse_kernels.hip")).read()
+    begin = source.index("constexpr int kMoveRows")
+    end = source.index("\n}\n", begin) + 3
+    kernel = re.sub(r"__shared__ int (\w+)\[(\w+)\];", r"static Shared<\2> \1;", source[begin:end])
+    assert "k_sparse_partition" in kernel and kernel.count("static Shared<") == 3
+    (tmp_path / "moves.inc").write_text(kernel)
+    run_native("sparse_moves.cpp", "-I" + str(tmp_path))

@@ -876,8 +876,10 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_partition(TreeBuffers tb_al
         }
 #pragma unroll
         for (int k = 0; k < kMoveRows; ++k) {
-            const int r = min(base + k * kSpBlock + (int)threadIdx.x, tb.n - 1);
-            col[k] = node[k] >= off ? s_col[node[k] - off] : (int)STAYS;  // (else in a leaf of an earlier level)
+            const int r = base + k * kSpBlock + (int)threadIdx.x;
+            // (a row past the end stays: the last row's node, which was loaded in its place, is a child's by now if the thread that
+            // has that row was faster. Other rows stay in leaves of earlier levels.)
+            col[k] = r < tb.n && node[k] >= off ? s_col[node[k] - off] : (int)STAYS;
             bin[k] = col[k] >= 0 ? (int)bins.colbin[(size_t)col[k] * bins.col_stride + r] : 0;
         }
 #pragma unroll
