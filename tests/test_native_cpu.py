@@ -166,3 +166,29 @@ def test_sparse_moves_whatever_thread_is_first(run_native, tmp_path):
     assert "k_sparse_partition" in kernel and kernel.count("static Shared<") == 3
     (tmp_path / "moves.inc").write_text(kernel)
     run_native("sparse_moves.cpp", "-I" + str(tmp_path))
+
+
+def test_lanes_are_read_where_all_of_them_are_on():
+    """read_lane takes a register of another lane as it is. Inside a branch that some lanes do not take, the compiler may work the
+    register out for those that do alone."""
+    csrc = os.path.join(os.path.dirname(HERE), "thundergbm_amd", "csrc")
+    per_thread = {"threadIdx", "lane", "lane_id", "i", "r", "valid", "in", "on", "left", "right", "active"}
+    seen = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        blocks = []  # conditions of the blocks that are open
+        for number, line in enumerate(open(os.path.join(csrc, name)), 1):
+            code = line.split("//")[0]
+            if "read_lane" in code and "__forceinline__" not in code:
+                seen += 1
+                own = re.findall(r"\bif \((.*)", code.split("read_lane")[0])
+                names = {w for c in blocks + own for w in re.findall(r"\b[a-zA-Z_]\w*", c)}
+                assert not names & per_thread, (name, number, names & per_thread)
+            for brace in re.findall(r"[{}]", code):
+                if brace == "}":
+                    blocks.pop()
+                else:
+                    found = re.search(r"\bif (?:constexpr )?\((.*)\) \{", code)
+                    blocks.append(found.group(1) if found else "")
+    assert seen > 20

@@ -628,8 +628,9 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
 #pragma unroll
     for (int k = 0; k < STEPS; ++k) {
         const int i = k * kSmallBlock + (int)threadIdx.x;
+        const int before = read_lane(upto[k / 4], k % 4 * kSmallWaves + w);  // (out here: the lane that is read may have no row)
         if (k < steps && i < len) {
-            const int lefts = read_lane(upto[k / 4], k % 4 * kSmallWaves + w) + lanes_below(left_mask[k]);
+            const int lefts = before + lanes_below(left_mask[k]);
             const bool left = (left_mask[k] >> lane & 1ull) != 0;
             const int at = left ? lefts : i - lefts;  // in the child's list
             if (left == build_left) s_rows[at] = (unsigned short)row[k];
