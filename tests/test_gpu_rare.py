@@ -96,3 +96,45 @@ def compare(T, val, rp, col, z, objective, kw, rare_values=None):
     finally:
         del os.environ["TGBM_SPARSE_SORTED"], os.environ["TGBM_LAYOUT"]
     assert runs[0] == runs[1]
+
+
+# Values brought to by blocks of 32 768 rows (TGBM_SPARSE_SPREAD) against values that look their rows up: rows at the edges of blocks,
+# a block without values, a task's last group of places, more than 128 nodes in a level, class trees built together.
+@pytest.mark.parametrize("n,depth", [(300, 4), (32768, 3), (32769, 6), (100003, 10)])
+@pytest.mark.parametrize("objective,kw", [("reg:linear", {}), ("binary:logistic", {"min_child_weight": 0.0}), ("multi:softmax", {"num_class": 3})])
+def test_spread_values_equal_looked_up_ones(T, n, depth, objective, kw):
+    rng = np.random.default_rng(n)
+    counts = np.minimum(n // 2, np.concatenate([[6000] * 3, rng.integers(1, 900, 200), [1] * 2100, [4095, 4096, 2, 3, 4, 5]]))
+    val, rp, col, z = _by_feature([int(k) for k in counts], n, 5)
+    if n > 65536:  # (nothing is stored in the rows of the second block)
+        rp = rp.astype(np.int64)
+        keep = np.ones(len(col), bool)
+        keep[rp[32768]:rp[65536]] = False
+        cut = np.concatenate([[0], np.cumsum(keep)])
+        val, col, rp = val[keep], col[keep], cut[rp].astype(np.int32)
+    y = (z if objective == "reg:linear" else np.digitize(z, [-0.5, 0.5][: 2 if "multi" in objective else 1])).astype(np.float32)
+    runs = []
+    os.environ["TGBM_LAYOUT"] = "sparse"
+    try:
+        for spread in ("1", "0"):
+            os.environ["TGBM_SPARSE_SPREAD"] = spread
+            s = T.Session(val, rp, col, y, objective=objective, depth=depth, n_trees=3, max_num_bin=63, learning_rate=0.5, **kw)
+            assert s.info("sparse_spread_blocks") == (-(-n // 32768) if spread == "1" else 0)
+            s.boost(2)
+            got = [s.model().tobytes(), s.y_pred().tobytes()]
+            if s.tree_per_rounds == 1:  # (stage by stage the levels leave their nodes' histograms too)
+                s.gradient()
+                s.tree_init()
+                for level in range(depth):
+                    s.find_split(level)
+                    if level < 5:
+                        got.append(s.level_hist(level).tobytes())
+                    s.partition(level)
+                s.finish_tree()
+                got.append(s.model().tobytes())
+            runs.append(got)
+            s.close()
+    finally:
+        os.environ.pop("TGBM_SPARSE_SPREAD", None)
+        del os.environ["TGBM_LAYOUT"]
+    assert runs[0] == runs[1]

@@ -251,20 +251,33 @@ struct SparseTask {
 constexpr int kRareBlock = 512;
 constexpr int kRareTile = 4096;       // values per task at most
 constexpr int kRareTileLeast = 512;   // a value per thread: smaller tasks leave threads without one
-constexpr int kRareFeatures = 2048;   // features per task at most
+constexpr int kRareFeatures = 2047;   // features per task at most (one more would meet the mark of an empty place)
 // Features with more than kRareLeast values (at most this many, the most frequent ones) are served through tables too.
 constexpr int kRareExempt = 128;
 constexpr int kRareLeast = 256;
 constexpr int kRareGroupTiles = 16;   // tasks of a search workgroup at most
 constexpr int kRareGroups = 512;      // search workgroups that are resident together (two per CU)
 struct RareTask {
-    int v_begin;     // first position of the task's values in SparsePass::rare_row / rare_key
-    int count;       // stored values of its features
+    int v_begin;     // first place of the task's values in SparsePass::rare_row / rare_key
+    int count;       // stored values of its features (SparsePass::rare_places: places that they take)
     int meta_begin;  // first entry of its features in SparsePass::rare_meta / rare_fid
     int n_feat;      // features of the task
 };
 // key of a stored value: feature (index inside its task) << 20 | sixty-fourth of the feature's values << 8 | local bin
 constexpr int kRareFeatShift = 20;
+// Spread values: the rows are cut into blocks whose nodes fit the LDS beside other workgroups, and a task's values lie in the
+// order of their rows' blocks, four places of one block at a time (kRareEmpty in rare_key: nobody's).
+constexpr int kSpreadLogRows = 15;
+constexpr int kSpreadRows = 1 << kSpreadLogRows;
+constexpr int kSpreadGroup = 4;
+constexpr int kSpreadLevel = 7;       // deepest level with its nodes in a byte (all ones: the row has come to rest above)
+constexpr int kSpreadBlocks = 341;    // (more leave less than three quarters of a tile to values)
+// Stored values from which on the rare ones are spread: a launch more a level, and half the time per value. ms a tree of depth 8,
+// looked up / spread: 0.7 M values 0.424 / 0.465, 1.8 M 0.573 / 0.606, 3.6 M 0.688 / 0.691, 7.2 M 0.837 / 0.754, 18 M 1.27 / 1.06,
+// 72 M (2 M rows, whose words are more than an L2) 5.43 / 3.50.
+constexpr long kSpreadValues = 4000000;
+constexpr unsigned kRareEmpty = ~0u;
+inline int spread_blocks(int n) { return (int)(((long)n + kSpreadRows - 1) >> kSpreadLogRows); }
 struct SparseBig {
     int feature;
     int slot_begin, slot_end;  // partial slots of its chunks
@@ -281,10 +294,22 @@ struct SparsePass {
     int rare_slot = 0;                  // candidate slot of the first group
     const int2 *rare_meta = nullptr;    // per feature of a task: (first global bin, number of bins)
     const int *rare_fid = nullptr;      // its feature id
-    const int *rare_row = nullptr;      // [values of the rare features] rows and keys in the order (feature, bin, row)
+    const int *rare_row = nullptr;      // [n_rare_places] rows and keys of their values
     const unsigned *rare_key = nullptr;
-    long n_rare = 0;
-    unsigned long long *rare_item = nullptr;  // [n_sets][n_rare] values of a level that may matter, tile by tile
+    const int *rare_places = nullptr;   // per task
+    long n_rare = 0;                    // stored values
+    size_t n_rare_places = 0;           // (a multiple of 16)
+    unsigned long long *rare_item = nullptr;  // [n_sets][n_rare_places] values of a level that may matter, tile by tile
+    // Spread values (n_spread > 0: row blocks; else nullptr): a value's group as in its key; groups of places by row block - the
+    // groups of block b in a task from spread_begin[b * n_rare_tasks + task] on -, their rows inside the block and where they lie.
+    // Of the current tree and level: a value's row word with its feature in the node's place, its row's node.
+    int n_spread = 0;
+    const uint8_t *rare_group = nullptr;           // [n_rare_places]
+    const unsigned *spread_begin = nullptr;        // [n_spread * n_rare_tasks + 1]
+    const unsigned short *spread_row = nullptr;    // [groups][kSpreadGroup]
+    const unsigned *spread_place = nullptr;        // [groups] first place / kSpreadGroup
+    unsigned *rare_code = nullptr;                 // [n_sets][n_rare_places]
+    uint8_t *rare_node = nullptr;                  // [n_sets][n_rare_places]
     int *rare_passed = nullptr;               // [n_sets][n_rare_tasks] how many of a tile
     const int *feat_val_begin = nullptr;  // [F + 1] first position of every feature in the bin-major copy
     // [n_sets][nnz] the gradient pair of every stored value's row, in the order of the bin-major copy, left there by
@@ -531,9 +556,11 @@ void launch_sparse_partition(hipStream_t s, const TreeBuffers &tb, const CsrBins
 // Byte columns of the frequent features (CsrBins::colbin, pre-filled with kMissingBin) from the bin-major copy.
 void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *csc_row, const int *cut_fid,
                         const int *cut_row_ptr, const int *col_of_feature, uint8_t *colbin, size_t col_stride);
-// Fills row / key (SparsePass::rare_row / rare_key, sp.n_rare entries) from the bin-major copy.
-void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row,
-                       unsigned *key);
+// Fills what SparsePass points to under the same names from the bin-major copy; the spread_* arrays where sp.n_spread > 0:
+// launch_rare_count leaves the groups of every (block, task) in `count` (their exclusive sums are spread_begin).
+void launch_rare_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count);
+void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
+                       int *places, uint8_t *group, unsigned short *spread_row, unsigned *spread_place);
 // The rows' words of a tree (TreeBuffers::row_word).
 void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class);
 // Row-ordered passes over the row lists (one of dbins / cbins by tb.sparse). lookup_level: the level

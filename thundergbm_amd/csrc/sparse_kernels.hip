@@ -113,14 +113,15 @@ struct SpShared {
     int ctl[8];  // batch: first feature, end feature, first bin, bins, node range begin, nodes in range, first value, end value
 };
 
-// Level-wide state every task starts from: node sums and validity into LDS, keys cleared.
+// Level-wide state every task starts from: node sums and validity into LDS, and the best keys that other tasks have published:
+// a node whose best candidate is another task's by now needs no record of this one's.
 __device__ void sp_begin(const TreeBuffers &tb, SpShared &sh, int level) {
     const int nl = 1 << level, off = nl - 1;
     for (int x = threadIdx.x; x < nl; x += kSpBlock) {
         const TreeNode &nd = tb.nodes[off + x];
         sh.S[x] = nd.sum_gh_pair;
         sh.ok[x] = nd.is_valid ? 1 : 0;
-        sh.key[x] = 0ull;
+        sh.key[x] = __hip_atomic_load(&tb.best_key[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -371,8 +372,12 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_big(TreeBuffers tb_all, Spa
 // that holds a value; the bins in between repeat the previous candidate's gain and lose the tie on the smaller index - so
 // the result is what the scan of a complete (bin, node) table gives.
 //
-// Bound by the row -> word look-ups of every stored value (4 bytes each, the words of 1 M rows fill an L2). The tiles of a
-// group are strided over the features, whose frequencies often fall with their index.
+// Where every value looks its row's word up, that is what bounds it: a request for a 128-byte line of the L2 each, 127 us a level for
+// 18.8 M values of 1 M rows, 361 for twice the values of 2 M rows, whose words are more than an L2. On many values the rows' nodes
+// are therefore brought to them first (k_sparse_spread), 23 us, and the filter takes 47: 30 of them its vector instructions, 25 the
+// LDS. A bound is some 70 instructions: a run's sums alone exclude most runs before their groups are looked at, and at deep levels
+// only runs that weigh enough are looked at, gathered from all threads (67 us without both). The tiles of a group are strided over
+// the features, whose frequencies often fall with their index.
 constexpr int kRareV = kRareTile / kRareBlock;
 constexpr int kRareWaves = kRareBlock / 64;
 constexpr int kRareCells = 3072;  // (with them two workgroups fit a CU)
@@ -389,6 +394,13 @@ __device__ __forceinline__ unsigned rare_row_word(unsigned node, GHPair s, const
 }
 static_assert(kRareTile * 1023 < 1 << 22 && kRareTile < 1 << 13, "fields of a cell");
 
+// No part of `part` that weighs the least leaves the rest of its node as much (rare_hopeless says the same of `part` alone).
+__device__ __forceinline__ bool rare_too_light(RareCell part, float node_h, RareBound u) {
+    const RareCell none{0, 0};
+    const RareRange r = rare_range(none, part, u);
+    return r.h_max + node_h * 0x1p-21f < u.mcw;
+}
+
 // No candidate that splits off all of `whole` and some of the values of `part` reaches the gain `floor`.
 __device__ __forceinline__ bool rare_hopeless(RareCell whole, RareCell part, GHPair S, float P, float floor, RareBound u) {
     const RareRange r = rare_range(whole, part, u);
@@ -403,7 +415,8 @@ __device__ __forceinline__ bool rare_hopeless(RareCell whole, RareCell part, GHP
 }
 
 // The runs of a tile with at least two groups per (feature, node): a thread takes four cells that follow each other, a run
-// is a part of a thread's cells or the cells of up to sixteen neighbouring lanes. open(): the run may hold a winner.
+// is a part of a thread's cells or the cells of up to sixteen neighbouring lanes. open(): the run may hold a winner. The groups
+// are looked at only where some of the wavefront's runs may win by their sums alone.
 template <typename MayWin, typename Open>
 __device__ __forceinline__ void rare_check_cells(const unsigned long long *cell_g, const unsigned *cell_h, int cells,
                                                  int log_groups, const MayWin &may_win, const Open &open) {
@@ -430,6 +443,10 @@ __device__ __forceinline__ void rare_check_cells(const unsigned long long *cell_
                       (unsigned long long)(unsigned)__shfl((int)(total.g >> 32), last) << 32;
             total.h = (unsigned)__shfl((int)total.h, last);
         }
+        const RareCell none{0, 0};
+        bool hope = total.g != 0 && may_win((i0 + V - 1) >> log_groups, none, groups == 2 ? upto[V - 1] : total, none);
+        if (groups == 2) hope = hope || (upto[1].g != 0 && may_win(i0 >> log_groups, none, upto[1], none));
+        if (!__any(hope)) continue;
 #pragma unroll
         for (int j = 0; j < V; ++j) {
             if (groups == 2) total = upto[j | 1];
@@ -535,8 +552,9 @@ __device__ __forceinline__ int rare_bin(unsigned long long item) { return (int)(
 struct RareFilter {
     unsigned long long g[kRareCells];
     unsigned h[kRareCells];
-    unsigned open[kRareCells / 32];  // runs of the tile that may hold a winner
-    int passed;
+    unsigned long long open[kRareCells / 64];  // runs of the tile that may hold a winner
+    unsigned short look[kRareBlock];           // runs of one group that weigh enough
+    int looks, any, passed;
 };
 struct RareShared {
     unsigned long long item[kRareLds];
@@ -697,8 +715,63 @@ __device__ void rare_search(const TreeBuffers &tb, const SparsePass &sp, RareSha
     __syncthreads();
 }
 
+// Brings what the rows of the rare values hold to the values' places: a row block's part in LDS, looked up there. Fetched by
+// the filter itself a look-up is a request for a whole line of the L2, whatever it takes of it.
+// CODES: the rows' words, with the value's feature in the node's place, once per tree; else the rows' nodes of a level. Bound by its
+// traffic: 4 bytes a value (2 the row in its block, 1 the place, 1 the node), 18.8 M values in 23 us, 52 for the words. Blocks of
+// 32 768 rows: their words still fit the LDS, and a tile of 4096 values has some 130 of a block next to each other at 1 M rows.
+template <bool CODES>
+__global__ __launch_bounds__(1024) void k_sparse_spread(TreeBuffers tb_all, SparsePass sp, int level) {
+    extern __shared__ unsigned spread_dyn[];  // [kSpreadRows] words, or as many bytes
+    const TreeBuffers tb = tb_all.for_class(blockIdx.z);
+    const int r0 = (int)blockIdx.y << kSpreadLogRows, rows = min(kSpreadRows, tb.n - r0);
+    const unsigned *__restrict__ begin = sp.spread_begin + (size_t)blockIdx.y * sp.n_rare_tasks;
+    const unsigned g0 = begin[0], g1 = begin[sp.n_rare_tasks];
+    const unsigned per = (g1 - g0 + gridDim.x - 1) / gridDim.x;
+    const unsigned first = g0 + blockIdx.x * per, end = min(g1, first + per);
+    const size_t set = (size_t)blockIdx.z * sp.n_rare_places;
+    if (first >= end) return;
+    if (CODES) {
+        for (int r = threadIdx.x; r < rows; r += 1024) spread_dyn[r] = tb.row_word[r0 + r] & ~kRareNodeMask;
+    } else {
+        const unsigned off = (1u << level) - 1u;
+        const unsigned *__restrict__ pairs = reinterpret_cast<const unsigned *>(tb.nid16 + r0);
+        unsigned short *out = reinterpret_cast<unsigned short *>(spread_dyn);
+        for (int i = threadIdx.x; i < (rows + 1) / 2; i += 1024) {
+            const unsigned v = pairs[i], a = v & 0xffffu, b = v >> 16;
+            out[i] = (unsigned short)((a >= off ? a - off : 0xffu) | (b >= off ? (b - off) & 0xffu : 0xffu) << 8);
+        }
+    }
+    __syncthreads();
+    constexpr int U = CODES ? 2 : 4;
+    for (unsigned i = first + threadIdx.x; i < end; i += 1024 * U) {
+        uint2 row[U];
+        unsigned place[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned g = min(i + u * 1024, end - 1);  // (past the end: the last group once more, with the same result)
+            row[u] = reinterpret_cast<const uint2 *>(sp.spread_row)[g];
+            place[u] = sp.spread_place[g];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned a = row[u].x & 0xffffu, b = row[u].x >> 16, c = row[u].y & 0xffffu, d = row[u].y >> 16;
+            if (CODES) {
+                const uint4 key = reinterpret_cast<const uint4 *>(sp.rare_key)[place[u]];
+                const auto code = [&](unsigned r, unsigned k) { return k == kRareEmpty ? kRareEmpty : spread_dyn[r] | k >> kRareFeatShift; };
+                reinterpret_cast<uint4 *>(sp.rare_code + set)[place[u]] = make_uint4(code(a, key.x), code(b, key.y), code(c, key.z), code(d, key.w));
+            } else {
+                const uint8_t *nodes = reinterpret_cast<const uint8_t *>(spread_dyn);
+                reinterpret_cast<unsigned *>(sp.rare_node + set)[place[u]] =
+                    (unsigned)nodes[a] | (unsigned)nodes[b] << 8 | (unsigned)nodes[c] << 16 | (unsigned)nodes[d] << 24;
+            }
+        }
+    }
+}
+
 // One workgroup per tile: the values of the runs that may hold a winner go to the tile's part of rare_item.
-template <bool DUMP>
+// SPREAD: the rows' words and nodes have been brought to the values (k_sparse_spread), which stream in groups of four places.
+template <bool DUMP, bool SPREAD>
 __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffers tb_all, SparsePass sp,
                                                                      const GHPair *__restrict__ gh, int level, float mcw,
                                                                      float lambda) {
@@ -708,30 +781,68 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
     gh += (size_t)blockIdx.z * tb.n;
     const int nl = 1 << level;
     const RareTask task = sp.rare_tasks[blockIdx.x];
+    const int places = sp.rare_places[blockIdx.x];
     const unsigned *__restrict__ keys = sp.rare_key + task.v_begin;
     const int *__restrict__ rows = sp.rare_row + task.v_begin;
     const unsigned *__restrict__ words = tb.row_word;
-    unsigned key[kRareV], word[kRareV];
-    int row[kRareV];
-    // (positions past the end repeat the last value, so that all loads are issued at once)
+    // k-th place of a thread
+    const auto place = [&](int k) {
+        return SPREAD ? ((k / kSpreadGroup) * kRareBlock + (int)threadIdx.x) * kSpreadGroup + k % kSpreadGroup : k * kRareBlock + (int)threadIdx.x;
+    };
+    // word: of the row, in place of its node the value's feature (below); node: of the level; group: sixty-fourth of the
+    // feature's values. (Places past the end repeat the last ones, so that all loads are issued at once.)
+    unsigned word[kRareV], node_of[kRareV], group_of[kRareV];
+    if (SPREAD) {
+        static_assert(kRareV % kSpreadGroup == 0 && kSpreadGroup == 4, "a thread's places are whole groups");
+        const size_t first = (size_t)blockIdx.z * sp.n_rare_places + task.v_begin;
+        const uint4 *__restrict__ codes = reinterpret_cast<const uint4 *>(sp.rare_code + first);
+        const unsigned *__restrict__ nodes = reinterpret_cast<const unsigned *>(sp.rare_node + first);
+        const unsigned *__restrict__ groups = reinterpret_cast<const unsigned *>(sp.rare_group + task.v_begin);
+        uint4 c[kRareV / 4];
+        unsigned x[kRareV / 4], g[kRareV / 4];
 #pragma unroll
-    for (int k = 0; k < kRareV; ++k) {
-        const int q = min(k * kRareBlock + (int)threadIdx.x, task.count - 1);
-        // (streamed past the caches: the words stay in the L2s)
-        row[k] = __builtin_nontemporal_load(rows + q);
-        key[k] = __builtin_nontemporal_load(keys + q);
+        for (int j = 0; j < kRareV / 4; ++j) {
+            const int q = min(j * kRareBlock + (int)threadIdx.x, places / kSpreadGroup - 1);
+            c[j] = codes[q];
+            x[j] = level > 0 ? nodes[q] : 0u;
+            g[j] = groups[q];
+        }
+#pragma unroll
+        for (int k = 0; k < kRareV; ++k) {
+            word[k] = k % 4 == 0 ? c[k / 4].x : k % 4 == 1 ? c[k / 4].y : k % 4 == 2 ? c[k / 4].z : c[k / 4].w;
+            node_of[k] = x[k / 4] >> 8 * (k % 4) & 0xffu;
+            group_of[k] = g[k / 4] >> 8 * (k % 4) & 0xffu;
+            if (word[k] == kRareEmpty || node_of[k] == 0xffu) node_of[k] = kRareNodeMask;
+        }
+    } else {
+        unsigned key[kRareV];
+        int row[kRareV];
+#pragma unroll
+        for (int k = 0; k < kRareV; ++k) {
+            const int q = min(place(k), places - 1);
+            // (streamed past the caches: the words stay in the L2s)
+            row[k] = __builtin_nontemporal_load(rows + q);
+            key[k] = __builtin_nontemporal_load(keys + q);
+        }
+#pragma unroll
+        for (int k = 0; k < kRareV; ++k) word[k] = words[row[k]];
+#pragma unroll
+        for (int k = 0; k < kRareV; ++k) {
+            node_of[k] = key[k] == kRareEmpty ? kRareNodeMask : word[k] & kRareNodeMask;
+            group_of[k] = key[k] >> 8 & 0x3fu;
+            word[k] = (word[k] & ~kRareNodeMask) | key[k] >> kRareFeatShift;
+        }
     }
-#pragma unroll
-    for (int k = 0; k < kRareV; ++k) word[k] = words[row[k]];
     int log_groups = 0;
     while (2 << log_groups <= kRareMaxGroups && task.n_feat * nl << (log_groups + 1) <= kRareCells) ++log_groups;
-    const int cells = min(kRareCells, task.n_feat * nl << log_groups);
+    const bool folded = task.n_feat * nl > kRareCells;  // (more runs than cells: two runs that meet in one only loosen the bound)
+    const int cells = folded ? kRareCells : task.n_feat * nl << log_groups;
     for (int c = threadIdx.x; c < cells; c += kRareBlock) {
         sh.g[c] = 0ull;
         sh.h[c] = 0u;
     }
-    for (int c = threadIdx.x; c < kRareCells / 32; c += kRareBlock) sh.open[c] = 0u;
-    if (threadIdx.x == 0) sh.passed = 0;
+    if (threadIdx.x < kRareCells / 64) sh.open[threadIdx.x] = 0ull;
+    if (threadIdx.x == 0) sh.looks = sh.any = sh.passed = 0;
     RareNodes node(rare_dyn, nl);
     node.load(tb, nl, lambda);
     const RareBound unit{(float)round_to_ll(tb.quant->gq_max) * tb.quant->inv_g / kRareSteps,
@@ -740,12 +851,12 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
     int cell[kRareV];  // -1: the value takes no part
 #pragma unroll
     for (int k = 0; k < kRareV; ++k) {
-        const unsigned x = word[k] & kRareNodeMask;
-        const int feature = (int)(key[k] >> kRareFeatShift);
-        const bool on = k * kRareBlock + (int)threadIdx.x < task.count && x != kRareNodeMask;
-        // (more runs than cells: two runs that meet in one only loosen the bound)
-        const unsigned group = (key[k] >> 8 & 0x3fu) >> (6 - log_groups);
-        cell[k] = on ? (int)((((unsigned)(feature * nl) + x) << log_groups | group) % kRareCells) : -1;
+        const unsigned x = node_of[k];
+        const int feature = (int)(word[k] & kRareNodeMask);
+        const bool on = place(k) < places && x != kRareNodeMask;
+        unsigned at = (unsigned)feature << (level + log_groups) | x << log_groups | group_of[k] >> (6 - log_groups);
+        if (folded) at %= (unsigned)kRareCells;
+        cell[k] = on ? (int)at : -1;
         if (tb.ignored != nullptr && on && tb.ignored[sp.rare_fid[task.meta_begin + feature]] != 0)
             cell[k] = -1;  // column sampling: all scores are 0 (hist_tree_builder_single.cu:304 / :663)
         if (cell[k] >= 0) {
@@ -754,47 +865,76 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
         }
         if (DUMP && on) {
             // stage-wise inspection: the per-node histograms of the level (zeroed before the launch) get the values
-            const GHPair s = gh[row[k]];
-            const size_t b = (size_t)x * tb.n_bins + sp.rare_meta[task.meta_begin + feature].x + (key[k] & 0xffu);
+            const GHPair s = gh[rows[place(k)]];
+            const size_t b = (size_t)x * tb.n_bins + sp.rare_meta[task.meta_begin + feature].x + (keys[place(k)] & 0xffu);
             unsigned long long *out = reinterpret_cast<unsigned long long *>(tb.hist(level) + b);
             atomicAdd(out, (unsigned long long)round_to_ll(s.g * tb.quant->scale_g));
             atomicAdd(out + 1, (unsigned long long)round_to_ll(s.h * tb.quant->scale_h));
         }
     }
     __syncthreads();
+    const auto hopeless = [&](int x, RareCell whole, RareCell part) {
+        return rare_hopeless(whole, part, node.S[x], node.P[x], node.floor(x), unit);
+    };
+    const auto open = [&](int run) {
+        atomicOr(reinterpret_cast<unsigned *>(sh.open) + (run >> 5), 1u << (run & 31));
+        sh.any = 1;
+    };
+    const auto look_at = [&](int c) {
+        if (!hopeless(c & (nl - 1), RareCell{0, 0}, RareCell{sh.g[c], sh.h[c]})) open(c);
+    };
     if (log_groups > 0) {
         rare_check_cells(
             sh.g, sh.h, cells, log_groups,
             [&](int run, RareCell before, RareCell own, RareCell after) {
                 const int x = run & (nl - 1);
-                const GHPair S = node.S[x];
-                const float P = node.P[x], floor = node.floor(x);
-                return !rare_hopeless(before, own, S, P, floor, unit) || !rare_hopeless(after, own, S, P, floor, unit);
+                return !hopeless(x, before, own) || !hopeless(x, after, own);
             },
-            [&](int run) { atomicOr(&sh.open[run >> 5], 1u << (run & 31)); });
+            open);
+    } else {
+        // A bound takes some 70 instructions and few runs of deep levels weigh enough to split off: those are listed first, one for
+        // every thread (with four workgroups on a CU there is no room for more; what does not fit is looked at at once).
+        static_assert(kRareCells % kSparseMaxLevelNodes == 0 && kRareCells % kRareBlock == 0, "a cell's node");
+#pragma unroll
+        for (int i = 0; i < kRareCells / kRareBlock; ++i) {
+            const int c = i * kRareBlock + (int)threadIdx.x;
+            bool look = c < cells;
+            if (look) {
+                const RareCell cell{sh.g[c], sh.h[c]};
+                look = cell.g != 0 && !rare_too_light(cell, node.S[c & (nl - 1)].h, unit);
+            }
+            const unsigned long long who = __ballot(look);
+            if (who == 0) continue;
+            int at = lane_id() == 0 ? atomicAdd(&sh.looks, __popcll(who)) : 0;
+            at = read_lane(at, 0) + lanes_below(who);
+            if (!look) continue;
+            if (at < kRareBlock) sh.look[at] = (unsigned short)c;
+            else look_at(c);
+        }
         __syncthreads();
+        if ((int)threadIdx.x < sh.looks) look_at(sh.look[threadIdx.x]);
+    }
+    __syncthreads();
+    if (sh.any == 0) {  // (the tile's, after the barrier)
+        if (threadIdx.x == 0) sp.rare_passed[(size_t)blockIdx.z * sp.n_rare_tasks + blockIdx.x] = 0;
+        return;
     }
     unsigned pass = 0;
 #pragma unroll
     for (int k = 0; k < kRareV; ++k) {
         if (cell[k] < 0) continue;
-        const int x = (int)(word[k] & kRareNodeMask);
-        bool on;
-        if (log_groups > 0) {
-            const int run = cell[k] >> log_groups;
-            on = (sh.open[run >> 5] >> (run & 31) & 1u) != 0;
-        } else {
-            on = !rare_hopeless(RareCell{0, 0}, RareCell{sh.g[cell[k]], sh.h[cell[k]]}, node.S[x], node.P[x], node.floor(x), unit);
-        }
-        if (on) pass |= 1u << k;
+        const int run = cell[k] >> log_groups;
+        if (reinterpret_cast<const unsigned *>(sh.open)[run >> 5] >> (run & 31) & 1u) pass |= 1u << k;
     }
     if (__any(pass != 0)) {
         // (few values pass: they are read again)
         int at = pass != 0 ? atomicAdd(&sh.passed, __popc(pass)) : 0;
-        unsigned long long *out = sp.rare_item + (size_t)blockIdx.z * sp.n_rare + task.v_begin;
+        unsigned long long *out = sp.rare_item + (size_t)blockIdx.z * sp.n_rare_places + task.v_begin;
+        const uint8_t *__restrict__ nodes = SPREAD ? sp.rare_node + (size_t)blockIdx.z * sp.n_rare_places + task.v_begin : nullptr;
         for (unsigned left = pass; left != 0; left &= left - 1) {
-            const int q = (__ffs(left) - 1) * kRareBlock + (int)threadIdx.x;
-            out[at++] = rare_item((int)(blockIdx.x / (unsigned)sp.n_rare_groups), keys[q], words[rows[q]] & kRareNodeMask, rows[q]);
+            const int q = place(__ffs(left) - 1);
+            const unsigned x = !SPREAD ? words[rows[q]] & kRareNodeMask : level > 0 ? (unsigned)nodes[q] : 0u;
+            out[at++] = rare_item((int)(blockIdx.x / (unsigned)sp.n_rare_groups), keys[q], x, rows[q]);
         }
     }
     __syncthreads();
@@ -834,7 +974,7 @@ __global__ __launch_bounds__(kRareBlock, 4) void k_sparse_rare_search(TreeBuffer
         }
         if (passed == 0) continue;
         const unsigned long long *__restrict__ in =
-            sp.rare_item + (size_t)blockIdx.z * sp.n_rare + sp.rare_tasks[(int)blockIdx.x + j * (int)gridDim.x].v_begin;
+            sp.rare_item + (size_t)blockIdx.z * sp.n_rare_places + sp.rare_tasks[(int)blockIdx.x + j * (int)gridDim.x].v_begin;
         for (int q = threadIdx.x; q < passed; q += kRareBlock) sh.item[rare_phys(filled + q)] = in[q];
         filled += passed;
         __syncthreads();
@@ -932,21 +1072,78 @@ __global__ __launch_bounds__(256) void k_sparse_cols(long nnz, const int *__rest
     }
 }
 
-// Values of a tile of rare features: its features one after the other, each in the order of the bin-major copy.
-__global__ __launch_bounds__(256) void k_rare_setup(SparsePass sp, CsrBins bins, const int *__restrict__ cut_row_ptr,
-                                                   int *__restrict__ row, unsigned *__restrict__ key) {
+// Groups of four places that the values of a task take in every row block.
+__global__ __launch_bounds__(256) void k_rare_count(SparsePass sp, CsrBins bins, unsigned *__restrict__ count) {
+    __shared__ unsigned values[kSpreadBlocks];
     const RareTask task = sp.rare_tasks[blockIdx.x];
-    int dst = task.v_begin;
+    for (int b = threadIdx.x; b < sp.n_spread; b += 256) values[b] = 0u;
+    __syncthreads();
+    for (int fi = 0; fi < task.n_feat; ++fi) {
+        const int f = sp.rare_fid[task.meta_begin + fi];
+        const int v0 = sp.feat_val_begin[f], v1 = sp.feat_val_begin[f + 1];
+        for (int v = v0 + (int)threadIdx.x; v < v1; v += 256) atomicAdd(&values[bins.csc_row[v] >> kSpreadLogRows], 1u);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < sp.n_spread; b += 256)
+        count[(size_t)b * sp.n_rare_tasks + blockIdx.x] = (values[b] + kSpreadGroup - 1) / kSpreadGroup;
+    if (blockIdx.x == 0 && threadIdx.x == 0) count[(size_t)sp.n_spread * sp.n_rare_tasks] = 0u;
+}
+
+// Places of the values of a task: spread ones by row block (in a block in any order), else its features one after the other, each
+// in the order of the bin-major copy.
+__global__ __launch_bounds__(256) void k_rare_setup(SparsePass sp, CsrBins bins, const int *__restrict__ cut_row_ptr,
+                                                   int *__restrict__ row, unsigned *__restrict__ key, int *__restrict__ places,
+                                                   uint8_t *__restrict__ group, unsigned short *__restrict__ spread_row,
+                                                   unsigned *__restrict__ spread_place) {
+    __shared__ unsigned first[kSpreadBlocks + 1], taken[kSpreadBlocks], from[kSpreadBlocks];
+    const RareTask task = sp.rare_tasks[blockIdx.x];
+    const int blocks = sp.n_spread;
+    for (int b = threadIdx.x; b < blocks; b += 256) {
+        const unsigned *at = sp.spread_begin + (size_t)b * sp.n_rare_tasks + blockIdx.x;
+        from[b] = at[0] * kSpreadGroup;
+        first[b + 1] = (at[1] - at[0]) * kSpreadGroup;
+        taken[b] = 0u;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        first[0] = 0u;
+        for (int b = 0; b < blocks; ++b) first[b + 1] += first[b];
+        places[blockIdx.x] = blocks > 0 ? (int)first[blocks] : task.count;
+    }
+    __syncthreads();
+    int done = 0;
     for (int fi = 0; fi < task.n_feat; ++fi) {
         const int f = sp.rare_fid[task.meta_begin + fi];
         const int v0 = sp.feat_val_begin[f], m = sp.feat_val_begin[f + 1] - v0;
         const int fbegin = cut_row_ptr[f];
         for (int a = threadIdx.x; a < m; a += 256) {
-            row[dst + a] = bins.csc_row[v0 + a];
-            key[dst + a] = ((unsigned)fi << kRareFeatShift) | (unsigned)(a * kRareMaxGroups / m) << 8 |
-                           (unsigned)(bins.csc_bin[v0 + a] - fbegin);
+            const int r = bins.csc_row[v0 + a];
+            const unsigned sixty_fourth = (unsigned)(a * kRareMaxGroups / m);
+            int at = task.v_begin + done + a;
+            if (blocks > 0) {
+                const int b = r >> kSpreadLogRows;
+                const unsigned mine = atomicAdd(&taken[b], 1u);
+                at = task.v_begin + (int)(first[b] + mine);
+                group[at] = (uint8_t)sixty_fourth;
+                spread_row[from[b] + mine] = (unsigned short)(r & (kSpreadRows - 1));
+            }
+            row[at] = r;
+            key[at] = ((unsigned)fi << kRareFeatShift) | sixty_fourth << 8 | (unsigned)(bins.csc_bin[v0 + a] - fbegin);
         }
-        dst += m;
+        done += m;
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < blocks; b += 256) {
+        const unsigned wide = first[b + 1] - first[b];
+        for (unsigned i = taken[b]; i < wide; ++i) {
+            const int at = task.v_begin + (int)(first[b] + i);
+            row[at] = 0;
+            key[at] = kRareEmpty;
+            group[at] = 0;
+            spread_row[from[b] + i] = 0;
+        }
+        for (unsigned i = 0; i < wide; i += kSpreadGroup)
+            spread_place[(from[b] + i) / kSpreadGroup] = (unsigned)(task.v_begin + (int)(first[b] + i)) / kSpreadGroup;
     }
 }
 
@@ -959,10 +1156,14 @@ void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *
     k_sparse_cols<<<grid, 256, 0, s>>>(nnz, csc_bin, csc_row, cut_fid, cut_row_ptr, col_of_feature, colbin, col_stride);
 }
 
-void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row,
-                       unsigned *key) {
+void launch_rare_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count) {
+    k_rare_count<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, count);
+}
+
+void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
+                       int *places, uint8_t *group, unsigned short *spread_row, unsigned *spread_place) {
     if (sp.n_rare_tasks == 0) return;
-    k_rare_setup<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, tb.cut_row_ptr, row, key);
+    k_rare_setup<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, tb.cut_row_ptr, row, key, places, group, spread_row, spread_place);
 }
 
 void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class) {
@@ -984,7 +1185,8 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
                             (size_t)(1 << level) * tb.n_bins * 4);
     }
     static LdsOptIn opt_in;
-    opt_in({reinterpret_cast<const void *>(&k_sparse_level<true>), reinterpret_cast<const void *>(&k_sparse_level<false>), reinterpret_cast<const void *>(&k_sparse_big)});
+    opt_in({reinterpret_cast<const void *>(&k_sparse_level<true>), reinterpret_cast<const void *>(&k_sparse_level<false>), reinterpret_cast<const void *>(&k_sparse_big),
+            reinterpret_cast<const void *>(&k_sparse_spread<true>)});
     if (sp.n_tasks > 0) {
         const dim3 tasks(sp.n_tasks, 1, n_class);
         if (level == 0) k_sparse_level<true><<<tasks, kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
@@ -996,8 +1198,17 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
     if (sp.n_rare_tasks > 0) {
         const size_t nodes_lds = (size_t)(1 << level) * 20;
         const dim3 tiles(sp.n_rare_tasks, 1, n_class);
-        if (dump_hist) k_sparse_rare_filter<true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
-        else k_sparse_rare_filter<false><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        const bool spread = sp.n_spread > 0 && level <= kSpreadLevel;
+        if (spread) {
+            // (a workgroup begins with the block's rows: no more of them than the chip holds at once)
+            const auto grid = [&](int workgroups) { return dim3(std::max(1, workgroups / (sp.n_spread * n_class)), sp.n_spread, n_class); };
+            if (level == 0) k_sparse_spread<true><<<grid(256), 1024, kSpreadRows * sizeof(unsigned), s>>>(tb, sp, level);
+            else k_sparse_spread<false><<<grid(512), 1024, kSpreadRows, s>>>(tb, sp, level);
+        }
+        if (dump_hist && spread) k_sparse_rare_filter<true, true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        else if (dump_hist) k_sparse_rare_filter<true, false><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        else if (spread) k_sparse_rare_filter<false, true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
+        else k_sparse_rare_filter<false, false><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
         k_sparse_rare_search<<<dim3(sp.n_rare_groups, 1, n_class), kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
     }
 }

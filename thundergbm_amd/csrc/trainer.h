@@ -143,6 +143,7 @@ class Trainer {
     int hist_cap_level_ = -1;       // first level with more nodes than the histogram arena holds (-1: none)
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
     long sparse_rare_most_ = 0;  // a feature with more stored values is served through tables
+    long rare_tile_ = 0;         // values per task of the others at most
     bool sparse_feature_in_tables(int f);
     SparsePass sp_;
     void build_sparse_tasks();

@@ -545,7 +545,7 @@ void Trainer::alloc_tree_buffers() {
     const size_t set_bytes =
         sparse_pass_ ? (size_t)n_ * 15 + (size_t)sp_.n_partial_slots * sp_.partial_stride * sizeof(longlong2) +
                            (size_t)max_level_nodes * sp_.n_cand_slots * sizeof(SplitCand) +
-                           (size_t)sp_.n_rare * 8 + (size_t)nnz_ * sizeof(GHPair)
+                           sp_.n_rare_places * (sp_.n_spread > 0 ? 13 : 8) + (size_t)nnz_ * sizeof(GHPair)
                      : fixed_bytes + arena_bytes(hist_nodes);
     const char *be = std::getenv("TGBM_BATCH_CLASSES");  // "0": build the trees of a round one after the other
     n_sets_ = (K > 1 && set_bytes * K < free_b / 2 && !(be != nullptr && std::string(be) == "0")) ? K : 1;
@@ -637,12 +637,37 @@ void Trainer::alloc_tree_buffers() {
         tb.best_key = dalloc<unsigned long long>(S * (size_t)max_level_nodes);
         HIP_CHECK(hipMemsetAsync(tb.best_key, 0, sizeof(unsigned long long) * S * (size_t)max_level_nodes, stream_));
         if (sp_.n_rare_tasks > 0) {
-            int *row = dalloc<int>((size_t)sp_.n_rare);
-            unsigned *key = dalloc<unsigned>((size_t)sp_.n_rare);
-            launch_rare_setup(stream_, tb, csr_, sp_, row, key);
+            int *row = dalloc<int>(sp_.n_rare_places), *places = dalloc<int>((size_t)sp_.n_rare_tasks);
+            unsigned *key = dalloc<unsigned>(sp_.n_rare_places), *spread_place = nullptr;
+            uint8_t *group = nullptr;
+            unsigned short *spread_row = nullptr;
+            if (sp_.n_spread > 0) {
+                const long lists = (long)sp_.n_spread * sp_.n_rare_tasks;
+                unsigned *count = nullptr, *total = nullptr, *begin = dalloc<unsigned>((size_t)lists + 1);
+                device_alloc_to(count, sizeof(unsigned) * ((size_t)lists + 1));
+                device_alloc_to(total, sizeof(unsigned));
+                launch_rare_count(stream_, csr_, sp_, count);
+                ScanScratch scratch;
+                device_exclusive_scan(stream_, count, begin, lists + 1, total, scratch);
+                HIP_CHECK(hipStreamSynchronize(stream_));
+                scratch.release();
+                device_free(count);
+                device_free(total);
+                sp_.spread_begin = begin;
+                group = dalloc<uint8_t>(sp_.n_rare_places);
+                spread_row = dalloc<unsigned short>(sp_.n_rare_places);
+                spread_place = dalloc<unsigned>(sp_.n_rare_places / kSpreadGroup);
+                sp_.rare_code = dalloc<unsigned>(S * sp_.n_rare_places);
+                sp_.rare_node = dalloc<uint8_t>(S * sp_.n_rare_places);
+            }
+            launch_rare_setup(stream_, tb, csr_, sp_, row, key, places, group, spread_row, spread_place);
             sp_.rare_row = row;
             sp_.rare_key = key;
-            sp_.rare_item = dalloc<unsigned long long>(S * (size_t)sp_.n_rare);
+            sp_.rare_places = places;
+            sp_.rare_group = group;
+            sp_.spread_row = spread_row;
+            sp_.spread_place = spread_place;
+            sp_.rare_item = dalloc<unsigned long long>(S * sp_.n_rare_places);
             sp_.rare_passed = dalloc<int>(S * (size_t)sp_.n_rare_tasks);
         }
         sp_.partial = dalloc<longlong2>(S * (size_t)sp_.n_partial_slots * sp_.partial_stride);
@@ -878,8 +903,14 @@ bool Trainer::sparse_feature_in_tables(int f) {
         std::vector<long> count(cuts_.feature_nnz);
         count.resize(std::max<size_t>(count.size(), kRareExempt + 1), 0);
         std::nth_element(count.begin(), count.begin() + kRareExempt, count.end(), std::greater<long>());
+        const char *pe = std::getenv("TGBM_SPARSE_SPREAD");  // "0", "1": never, always where it can be (tests, measurements)
+        const bool wanted = pe != nullptr ? std::string(pe) == "1" : nnz_ >= kSpreadValues;
+        const int blocks = spread_blocks(n_);
+        sp_.n_spread = wanted && blocks <= kSpreadBlocks && nnz_ < (1l << 30) ? blocks : 0;
+        // (a tile with up to three empty places in every row block)
+        rare_tile_ = kRareTile - (kSpreadGroup - 1) * sp_.n_spread;
         sparse_rare_most_ = se != nullptr && std::string(se) == "0"
-                                ? -1 : std::min<long>(kRareTile, std::max<long>(kRareLeast, count[kRareExempt]));
+                                ? -1 : std::min<long>(rare_tile_, std::max<long>(kRareLeast, count[kRareExempt]));
     }
     return cuts_.feature_nnz[f] > sparse_rare_most_ || f == sparse_bin0_owner_;
 }
@@ -952,15 +983,16 @@ void Trainer::build_sparse_tasks() {
     // over as many workgroups, because a level takes as long as its fullest tile: sorting and searching it is one chain.
     long n_rare = 0;
     for (int f : rare_fid) n_rare += cuts_.feature_nnz[f];
-    const long tile_values = std::min<long>(kRareTile, std::max<long>(kRareTileLeast, n_rare / kRareGroups));
-    n_rare = 0;
+    const long tile_values = std::min<long>(rare_tile_, std::max<long>(kRareTileLeast, n_rare / kRareGroups));
+    long places = 0;
     for (size_t i = 0; i < rare_fid.size();) {
         size_t e = i;
         long vals = 0;
         while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && (e == i || vals + cuts_.feature_nnz[rare_fid[e]] <= tile_values))
             vals += cuts_.feature_nnz[rare_fid[e++]];
-        rare_tasks.push_back(RareTask{(int)n_rare, (int)vals, (int)i, (int)(e - i)});
-        n_rare += vals;
+        rare_tasks.push_back(RareTask{(int)places, (int)vals, (int)i, (int)(e - i)});
+        places += vals;
+        if (sp_.n_spread > 0) places = (places + (kSpreadGroup - 1) * std::min<long>(sp_.n_spread, vals) + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
         i = e;
     }
     // as few rounds of resident workgroups as the tasks per workgroup allow
@@ -978,6 +1010,8 @@ void Trainer::build_sparse_tasks() {
     sp_.n_rare_tasks = n_rt;
     sp_.n_rare_groups = n_groups;
     sp_.n_rare = n_rare;
+    sp_.n_rare_places = ((size_t)places + 15) / 16 * 16;
+    if (n_rt == 0) sp_.n_spread = 0;
     sp_.n_cand_slots = std::max(1, next_slot);
     sp_.n_partial_slots = n_partial;
     sp_.partial_stride = (size_t)max_big_bins * (size_t)tb_.max_level_nodes;
@@ -1492,6 +1526,7 @@ int Trainer::info(const std::string &key) const {
     if (key == "sparse") return sparse_ ? 1 : 0;
     if (key == "sparse_pass") return sparse_pass_ ? 1 : 0;
     if (key == "sparse_rare_values") return (int)sp_.n_rare;
+    if (key == "sparse_spread_blocks") return sp_.n_spread;
     if (key == "wide_bins") return wide_bins_ ? 1 : 0;
     if (key == "wide_eval") return wide_eval_ ? 1 : 0;
     if (key == "row_lists") return sparse_pass_ ? 0 : 1;  // the sparse level pass keeps a row -> node map only
