@@ -138,3 +138,27 @@ def test_spread_values_equal_looked_up_ones(T, n, depth, objective, kw):
         os.environ.pop("TGBM_SPARSE_SPREAD", None)
         del os.environ["TGBM_LAYOUT"]
     assert runs[0] == runs[1]
+
+
+# The pass over the tables: bins of a lane (up to 64 bins or up to 255), the pairs as words or as pairs, copied to the values or fetched by
+# row, the nodes brought to the values or looked up; levels whose tables share a CU and levels whose don't; features in chunks.
+@pytest.mark.parametrize("bins", [31, 255])
+@pytest.mark.parametrize("objective", ["reg:linear", "binary:logistic"])
+def test_tables_whatever_form_their_values_have(T, objective, bins):
+    n = 40000
+    counts = [n - 1, 33000, 32769, 9000, 5000, 5001, 5002, 5003] + [300] * 60 + [5] * 40
+    val, rp, col, z = _by_feature(counts, n, 7)
+    y = (z if objective == "reg:linear" else np.digitize(z, [-0.5])).astype(np.float32)
+    runs = []
+    os.environ["TGBM_LAYOUT"] = "sparse"
+    try:
+        for spread, word, copy in [("0", "1", "1"), ("1", "1", "1"), ("0", "0", "1"), ("1", "0", "1"), ("0", "1", "0"), ("1", "1", "0"), ("1", "0", "0")]:
+            os.environ.update(TGBM_SPARSE_SPREAD=spread, TGBM_GH_WORD=word, TGBM_SPARSE_GH_COPY=copy)
+            s = T.Session(val, rp, col, y, objective=objective, depth=7, n_trees=2, max_num_bin=bins, learning_rate=0.5)
+            s.boost(2)
+            runs.append((s.model().tobytes(), s.y_pred().tobytes()))
+            s.close()
+    finally:
+        for key in ("TGBM_LAYOUT", "TGBM_SPARSE_SPREAD", "TGBM_GH_WORD", "TGBM_SPARSE_GH_COPY"):
+            os.environ.pop(key, None)
+    assert all(r == runs[0] for r in runs)

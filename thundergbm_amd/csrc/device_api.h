@@ -241,7 +241,7 @@ constexpr int kSparseTaskValues = 32768;    // stored values per task at most (a
 constexpr int kSparseTasks = 1024;          // smaller tasks where there would be fewer than that
 struct SparseTask {
     int f_begin, f_end;  // features [f_begin, f_end) (a chunk task: one feature)
-    int v_begin, v_end;  // positions of the bin-major copy
+    int v_begin, v_end;  // places of its values (SparsePass::table_bin), multiples of kSpreadGroup
     int cand_slot;       // candidate slot the task fills, -1: a chunk (its feature's slot is filled by k_sparse_big)
     int partial_slot;    // chunk: where its table goes in SparsePass::partial, else -1
 };
@@ -265,18 +265,19 @@ struct RareTask {
 };
 // key of a stored value: feature (index inside its task) << 20 | sixty-fourth of the feature's values << 8 | local bin
 constexpr int kRareFeatShift = 20;
-// Spread values: the rows are cut into blocks whose nodes fit the LDS beside other workgroups, and a task's values lie in the
-// order of their rows' blocks, four places of one block at a time (kRareEmpty in rare_key: nobody's).
+// Spread values: the rows are cut into blocks whose nodes fit the LDS beside other workgroups, and the values of a rare task and of
+// a table feature lie in the order of their rows' blocks, four places of one block at a time (kRareEmpty in rare_key, kTableEmpty
+// in table_bin: nobody's).
 constexpr int kSpreadLogRows = 15;
 constexpr int kSpreadRows = 1 << kSpreadLogRows;
 constexpr int kSpreadGroup = 4;
 constexpr int kSpreadLevel = 7;       // deepest level with its nodes in a byte (all ones: the row has come to rest above)
 constexpr int kSpreadBlocks = 341;    // (more leave less than three quarters of a tile to values)
-// Stored values from which on the rare ones are spread: a launch more a level, and half the time per value. ms a tree of depth 8,
-// looked up / spread: 0.7 M values 0.424 / 0.465, 1.8 M 0.573 / 0.606, 3.6 M 0.688 / 0.691, 7.2 M 0.837 / 0.754, 18 M 1.27 / 1.06,
-// 72 M (2 M rows, whose words are more than an L2) 5.43 / 3.50.
-constexpr long kSpreadValues = 4000000;
+// Stored values from which on they are spread: a launch more a level, and less time per value. ms a tree of depth 8, looked up / spread:
+// 0.7 M values 0.395 / 0.440, 2.2 M 0.647 / 0.648, 3.6 M 0.630 / 0.616, 7.2 M 0.769 / 0.649, 18 M 1.31 / 1.02, 36 M 2.50 / 1.76.
+constexpr long kSpreadValues = 3000000;
 constexpr unsigned kRareEmpty = ~0u;
+constexpr unsigned kTableEmpty = 0xffffu;
 inline int spread_blocks(int n) { return (int)(((long)n + kSpreadRows - 1) >> kSpreadLogRows); }
 struct SparseBig {
     int feature;
@@ -288,6 +289,7 @@ struct SparsePass {
     int n_tasks = 0;
     const SparseBig *big = nullptr;
     int n_big = 0;
+    int max_table_bins = 0;  // most bins of a feature of theirs
     // rare features
     const RareTask *rare_tasks = nullptr;
     int n_rare_tasks = 0, n_rare_groups = 0;
@@ -301,21 +303,31 @@ struct SparsePass {
     size_t n_rare_places = 0;           // (a multiple of 16)
     unsigned long long *rare_item = nullptr;  // [n_sets][n_rare_places] values of a level that may matter, tile by tile
     // Spread values (n_spread > 0: row blocks; else nullptr): a value's group as in its key; groups of places by row block - the
-    // groups of block b in a task from spread_begin[b * n_rare_tasks + task] on -, their rows inside the block and where they lie.
-    // Of the current tree and level: a value's row word with its feature in the node's place, its row's node.
-    int n_spread = 0;
+    // groups of block b in list l (the rare tasks, then the table features) from spread_begin[b * n_lists + l] on -, their rows inside
+    // the block and where they lie, the table values' places after the rare ones'.
+    // Of the current tree and level: a rare value's row word with its feature in the node's place, a value's row's node.
+    int n_spread = 0, n_lists = 0;
     const uint8_t *rare_group = nullptr;           // [n_rare_places]
-    const unsigned *spread_begin = nullptr;        // [n_spread * n_rare_tasks + 1]
+    const unsigned *spread_begin = nullptr;        // [n_spread * n_lists + 1]
     const unsigned short *spread_row = nullptr;    // [groups][kSpreadGroup]
     const unsigned *spread_place = nullptr;        // [groups] first place / kSpreadGroup
     unsigned *rare_code = nullptr;                 // [n_sets][n_rare_places]
-    uint8_t *rare_node = nullptr;                  // [n_sets][n_rare_places]
+    uint8_t *value_node = nullptr;                 // [n_sets][n_rare_places + n_table_places]
     int *rare_passed = nullptr;               // [n_sets][n_rare_tasks] how many of a tile
     const int *feat_val_begin = nullptr;  // [F + 1] first position of every feature in the bin-major copy
-    // [n_sets][nnz] the gradient pair of every stored value's row, in the order of the bin-major copy, left there by
-    // the pass of level 0: those below then stream it instead of fetching a cache line per value (nullptr: no room, gather)
-    GHPair *csc_gh = nullptr;
-    long nnz = 0;
+    // Values of the table features, a feature's in row order
+    const int *table_features = nullptr;  // [n_table_features]
+    int n_table_features = 0;
+    size_t n_table_places = 0;            // (a multiple of 16)
+    const int *table_first = nullptr;     // [F + 1] first place of every feature's values (other features: none)
+    const unsigned short *table_bin = nullptr;  // [n_table_places] bin, counted from the first one of the feature's task
+    const int *table_row = nullptr;             // [n_table_places]
+    // [n_sets][n_table_places] the gradient pair of every value's row, left there by the pass of level 0: those below then stream it
+    // instead of fetching a cache line per value (nullptr: no room, gather). With gh_words (below) the words instead.
+    GHPair *table_gh = nullptr;
+    // the rows' pairs as words (launch_gh_words) and what they are made of, where they match the gradients of the level 0
+    const unsigned *gh_words = nullptr;
+    int gh_objective = 0;
     longlong2 *partial = nullptr;         // [n_sets][n_partial_slots][partial_stride] chunk tables, (bin, node) cells
     size_t partial_stride = 0;            // cells per slot: most bins of a big feature x kSparseMaxLevelNodes at most
     int n_partial_slots = 0;
@@ -552,15 +564,18 @@ void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins,
 // into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q).
 void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp,
                          const GHPair *gh, int level, float mcw, float lambda, bool dump_hist, int n_class = 1);
-void launch_sparse_partition(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class = 1);
+void launch_sparse_partition(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int level, int n_class = 1);
 // Byte columns of the frequent features (CsrBins::colbin, pre-filled with kMissingBin) from the bin-major copy.
 void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *csc_row, const int *cut_fid,
                         const int *cut_row_ptr, const int *col_of_feature, uint8_t *colbin, size_t col_stride);
 // Fills what SparsePass points to under the same names from the bin-major copy; the spread_* arrays where sp.n_spread > 0:
-// launch_rare_count leaves the groups of every (block, task) in `count` (their exclusive sums are spread_begin).
-void launch_rare_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count);
+// launch_spread_count leaves the groups of every (block, list) in `count` (their exclusive sums are spread_begin). task_bin0: [F] first
+// bin of the task that a table feature belongs to.
+void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count);
 void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
                        int *places, uint8_t *group, unsigned short *spread_row, unsigned *spread_place);
+void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,
+                        unsigned short *spread_row, unsigned *spread_place);
 // The rows' words of a tree (TreeBuffers::row_word).
 void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class);
 // Row-ordered passes over the row lists (one of dbins / cbins by tb.sparse). lookup_level: the level

@@ -157,6 +157,22 @@ __device__ __forceinline__ int wave_best(float v, int idx, float *win, int *win_
 }
 
 
+// A row's gradient pair from the word (word_from_row).
+__device__ __forceinline__ GHPair pair_from_word(int objective, unsigned w) {
+    GHPair o;
+    if (objective == OBJ_SQUARE) {
+        o.g = __uint_as_float(w);
+        o.h = 1.f;
+    } else {
+        const float s = __uint_as_float(w & 0x7fffffffu);
+        const float yi = (w >> 31) ? 1.f : 0.f;
+        o.g = s - yi;
+        o.h = fmaxf(s * (1.f - s), 1e-16f);
+    }
+    return o;
+}
+
+
 // Left/right decision of the sparse layout: binary search of the row's bin ids for the one inside
 // the split feature's bin range (absent = missing), hist_tree_builder_single.cu:941-1011.
 // Does the row go right at a split of the feature whose global bins are [cb, ce)? Binary search of the

@@ -31,22 +31,32 @@ struct SegResult {
     bool owner;
 };
 
+// Upper estimate of a gain from the hardware reciprocal (1 ulp) instead of divisions; -1: the weight gate closes
+__device__ __forceinline__ float gain_estimate(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
+    const GHPair r{f.g - l.g, f.h - l.h};
+    if (!(l.h >= mcw && r.h >= mcw)) return -1.f;
+    const float a = l.g * l.g * __builtin_amdgcn_rcpf(l.h + lambda), b = r.g * r.g * __builtin_amdgcn_rcpf(r.h + lambda);
+    return (a + b - fterm) + (a + b + fabsf(fterm)) * 0x1p-18f;  // + 2^-18 of the terms: far above the roundings
+}
+
 // Best candidate of one (feature, node) segment; one wavefront, lane l looks at ceil(kf / 64) consecutive bins of the
 // feature's kf <= 256 bins. The arithmetic is that of k_eval_split: exact integer prefix sums,
 // missing = node sum - feature total, gain with the missing rows sent right and left
 // (hist_tree_builder_single.cu:300-323), largest |gain| wins, ties go to the smaller bin index (:330-335).
 // `force`: evaluate even when the segment holds no value (the feature owning global bin 0: when no candidate of a
 // node has a positive gain the arg-max of the reference ends on bin 0).
+// `floor`: the best gain that the node has seen; a segment none of whose candidates reaches it by their estimates has no result.
 // A wavefront takes 2.1 ns for an instruction that depends on the one before, so the code has no branches but the ones that
-// all lanes take alike.
+// all lanes take alike. BPL: most bins of a lane. TRY: with the estimates.
+template <int BPL, bool TRY>
 __device__ __forceinline__ SegResult eval_segment(const longlong2 *cells, int kf, int gbin0, GHPair S, double inv_g, double inv_h,
-                                                  float mcw, float lambda, bool ignored, bool force) {
+                                                  float mcw, float lambda, bool ignored, bool force, float floor) {
 #pragma clang fp contract(off)
     const int lane = lane_id();
-    const int bpl = (kf + 63) >> 6;  // bins per lane: 1 for the usual <= 64 bins, so that every lane has a candidate
-    long long exg[4], exh[4], rung = 0, runh = 0;
+    const int bpl = BPL == 1 ? 1 : (kf + 63) >> 6;  // bins per lane: 1 for the usual <= 64 bins, so that every lane has a candidate
+    long long exg[BPL], exh[BPL], rung = 0, runh = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < BPL; ++j) {
         exg[j] = rung;
         exh[j] = runh;
         if (j >= bpl) break;
@@ -67,12 +77,24 @@ __device__ __forceinline__ SegResult eval_segment(const longlong2 *cells, int kf
     if (!force && totg == 0 && toth == 0) return r;
     const long long carryg = upg - rung, carryh = uph - runh;  // exclusive prefix of the lane
     const GHPair m{S.g - scaled_float(totg, inv_g), S.h - scaled_float(toth, inv_h)};
+    if (TRY && !force) {
+        const float about = S.g * S.g * __builtin_amdgcn_rcpf(S.h + lambda);
+        float most = -1.f;
+#pragma unroll
+        for (int j = 0; j < BPL; ++j) {
+            if (j >= bpl) break;
+            const GHPair l{scaled_float(carryg + exg[j], inv_g), scaled_float(carryh + exh[j], inv_h)};
+            const float e = fmaxf(gain_estimate(S, about, l, mcw, lambda), gain_estimate(S, about, GHPair{l.g + m.g, l.h + m.h}, mcw, lambda));
+            most = lane * bpl + j < kf ? fmaxf(most, e) : most;
+        }
+        if (!__any(most >= floor)) return r;
+    }
     const float fterm = (S.g * S.g) / (S.h + lambda);
     float best = -1.f, best_score = 0.f;
     int which = 0;
     GHPair best_left{0, 0};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < BPL; ++j) {
         if (j >= bpl) break;
         const int b = lane * bpl + j;
         const GHPair l{scaled_float(carryg + exg[j], inv_g), scaled_float(carryh + exh[j], inv_h)};
@@ -105,7 +127,9 @@ __device__ __forceinline__ unsigned long long cand_key(float abs_gain, int index
 }
 __device__ __forceinline__ int key_index(unsigned long long key) { return (int)(0xffffffffu - (unsigned)key); }
 
+constexpr int kSpKept = 256;  // segments of a batch whose results are kept (what the LDS has left beside the largest tables)
 struct SpShared {
+    float kept[kSpKept][5];  // score, missing and left sums
     GHPair S[kSparseMaxLevelNodes];              // node sums of the level
     unsigned long long key[kSparseMaxLevelNodes];  // best candidate of every node over the task's features so far
     unsigned char ok[kSparseMaxLevelNodes];        // node is valid
@@ -140,7 +164,8 @@ __device__ void sp_publish(const TreeBuffers &tb, SpShared &sh, int level) {
 // Split search over the tables of one batch: features [fa, fa + nf) x nodes [n0, n0 + nn) of the level, cells at
 // (node - n0) * bins + (bin - bin0): the bins of a (feature, node) segment lie next to each other. Phase 1 raises every node's key; after a barrier the wavefronts whose segment holds
 // a node's current best write that candidate's details to the task's slot (a later batch with a better candidate
-// overwrites them). `dump`: also store the cells into the level's per-node histograms.
+// overwrites them), kept from phase 1 or, past kSpKept segments, worked out again. `dump`: also store the cells into the level's per-node histograms.
+template <int BPL, bool DEEP>
 __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longlong2 *cells, int level, int fa, int nf,
                                 int bin0, int n0, int nn, int cand_slot, float mcw, float lambda, longlong2 *dump) {
     const int w = threadIdx.x >> 6, lane = lane_id();
@@ -154,9 +179,16 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
         const int b0 = sh.fbin[fi], kf = sh.fbin[fi + 1] - b0;
         if (kf <= 0) continue;
         const bool ign = tb.ignored != nullptr && tb.ignored[fa + fi] != 0;
-        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
-                                         lambda, ign, bin0 + b0 == 0);
+        const SegResult r = eval_segment<BPL, DEEP>(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw, lambda, ign,
+                                              bin0 + b0 == 0, __uint_as_float((unsigned)(sh.key[node] >> 32)));
         if (r.win >= 0.f && lane == 0) atomicMax(&sh.key[node], cand_key(r.win, r.win_idx));
+        if (DEEP && seg < kSpKept && r.owner) {
+            sh.kept[seg][0] = r.score;
+            sh.kept[seg][1] = r.miss.g;
+            sh.kept[seg][2] = r.miss.h;
+            sh.kept[seg][3] = r.left.g;
+            sh.kept[seg][4] = r.left.h;
+        }
     }
     __syncthreads();
     for (int x = w; x < nn; x += kSpWaves) {
@@ -171,17 +203,24 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
             const int mid = (lo + hi) >> 1;
             if (sh.fbin[mid] <= idx - bin0) lo = mid; else hi = mid;
         }
+        SplitCand c;
+        c.index = idx;
+        c.feature = c.bin = 0;
+        const int seg = lo * nn + x;
+        if (DEEP && seg < kSpKept) {
+            c.score = sh.kept[seg][0];
+            c.miss = GHPair{sh.kept[seg][1], sh.kept[seg][2]};
+            c.left = GHPair{sh.kept[seg][3], sh.kept[seg][4]};
+            if (lane == 0) tb.cand[(size_t)node * tb.n_packs + cand_slot] = c;
+            continue;
+        }
         const int b0 = sh.fbin[lo], kf = sh.fbin[lo + 1] - b0;
         const bool ign = tb.ignored != nullptr && tb.ignored[fa + lo] != 0;
-        const SegResult r = eval_segment(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw,
-                                         lambda, ign, true);
+        const SegResult r = eval_segment<BPL, DEEP>(cells + (size_t)x * bins + b0, kf, bin0 + b0, sh.S[node], inv_g, inv_h, mcw, lambda, ign, true, 0.f);
         if (r.owner && r.win_idx == idx) {
-            SplitCand c;
             c.score = r.score;
-            c.index = idx;
             c.miss = r.miss;
             c.left = r.left;
-            c.feature = c.bin = 0;
             tb.cand[(size_t)node * tb.n_packs + cand_slot] = c;
         }
     }
@@ -196,12 +235,22 @@ __device__ void sp_search_batch(const TreeBuffers &tb, SpShared &sh, const longl
 
 // One task = a run of whole features (batched so that their tables fit the LDS) or one chunk of a big feature (its
 // table goes to the partial buffer, k_sparse_big adds the chunks up and searches them).
-// ROOT: level 0, where every row is in the one node; the pairs are looked up there and left in csc_gh for the levels below (a
-// launch of its own before: 130 us and 67 at 1 M rows, together 113).
-template <bool ROOT>
-__global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, CsrBins bins, SparsePass sp,
-                                                          const GHPair *__restrict__ gh, int level, float mcw,
-                                                          float lambda, int dump_hist, int n_cells) {
+// Added up in 33 us at levels 0 to 3 for the 15 M values of the frequent features of 1 M x 100 k (7 bytes each: the pair's word, the
+// bin, the node), 72 where the nodes are looked up (5 M lines of the L2) and 78 with 8 bytes more a value: waits for loads, the LDS
+// is busy for 14 of them, the vector units for 24. At deep levels the search comes on top, 63 us at level 7: issue of its
+// instructions with a workgroup on a CU. It took 119 us, with winners' segments searched again for their records, without the
+// estimates, and with chunks before the tasks that search.
+// DEEP: one workgroup on a CU, for its registers (more than 64 bins) or its table (from level 4 on); else two, without the estimates and
+// kept records, for which 64 registers are too few (33 -> 45 us at level 1).
+// NODES: kRootNode (level 0): every row is in the one node; the pairs are looked up there and left in table_gh for the levels below (a
+// launch of its own before: 130 us and 67 at 1 M rows, together 113), unless k_sparse_spread has (kRootWords). kSpreadNodes: the rows'
+// nodes have been brought to the values, too. kRowNodes: they are looked up. WORDS: the rows' gradient words instead of their pairs, half the bytes; the
+// pairs that they stand for have the same bits.
+enum { kRootNode, kRootWords, kRowNodes, kSpreadNodes };
+template <int NODES, bool WORDS, int BPL, bool DEEP>
+__global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuffers tb_all, SparsePass sp, const GHPair *__restrict__ gh,
+                                                                            int level, float mcw, float lambda, int dump_hist,
+                                                                            int n_cells) {
     extern __shared__ longlong2 cells[];  // [n_cells]
     __shared__ SpShared sh;
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
@@ -211,7 +260,12 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
     const unsigned short *__restrict__ nid16 = tb.nid16;
     const int *__restrict__ crp = tb.cut_row_ptr;
     const float scale_g = tb.quant->scale_g, scale_h = tb.quant->scale_h;
-    GHPair *__restrict__ csc_gh = sp.csc_gh != nullptr ? sp.csc_gh + (size_t)blockIdx.z * sp.nnz : nullptr;
+    // (in units of a group of places)
+    const size_t set = (size_t)blockIdx.z * (sp.n_table_places / kSpreadGroup);
+    const bool copied = sp.table_gh != nullptr;
+    const unsigned *__restrict__ nodes =
+        reinterpret_cast<const unsigned *>(sp.value_node + (size_t)blockIdx.z * (sp.n_rare_places + sp.n_table_places) + sp.n_rare_places);
+    const int task_bin0 = crp[task.f_begin];
     sp_begin(tb, sh, level);
     longlong2 *dump = (dump_hist && task.cand_slot >= 0) ? tb.hist(level) : nullptr;
     longlong2 *partial = task.partial_slot >= 0
@@ -241,8 +295,8 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
             sh.ctl[2] = crp[f];
             sh.ctl[3] = kf;
             sh.ctl[5] = nn;
-            sh.ctl[6] = max(task.v_begin, sp.feat_val_begin[f]);
-            sh.ctl[7] = min(task.v_end, sp.feat_val_begin[fb]);
+            sh.ctl[6] = max(task.v_begin, sp.table_first[f]);
+            sh.ctl[7] = min(task.v_end, sp.table_first[fb]);
         }
         __syncthreads();
         const int fa = sh.ctl[0], fb = sh.ctl[1], bin0 = sh.ctl[2], nbins = sh.ctl[3], nn_max = sh.ctl[5];
@@ -255,41 +309,85 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
             __syncthreads();
             for (int c = threadIdx.x; c < n_cells; c += kSpBlock) cells[c] = make_longlong2(0, 0);
             __syncthreads();
-            // accumulate: four values in flight per thread (row -> node from the cache-resident map, then the pair)
-            constexpr int U = 8;
-            for (int e0 = v0 + threadIdx.x; e0 < v1; e0 += kSpBlock * U) {
-                // (every load is unconditional - a value index past the end repeats the last value and is skipped
-                // below -, so each stage's eight loads are issued together instead of one after the other)
-                int gb[U], row[U], x[U];
-                GHPair s[U];
+            // accumulate: a thread takes two groups of places at a time (every load is unconditional - past the end the last group
+            // repeats and is skipped below -, so that a stage's loads are issued together instead of one after the other)
+            constexpr int U = DEEP ? 2 : 1, V = kSpreadGroup;
+            static_assert(V == 4, "a group's loads");
+            const int q1 = v1 / V, bin_shift = bin0 - task_bin0;
+            for (int q0 = v0 / V + (int)threadIdx.x; q0 < q1; q0 += kSpBlock * U) {
+                unsigned long long bin4[U];
+                unsigned node4[U];       // (kSpreadNodes)
+                int x[U][V];             // (kRowNodes)
+                float g[U][V], h[U][V];  // (WORDS: g the word)
+                int row[U][V];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int e = min(e0 + u * kSpBlock, v1 - 1);
-                    gb[u] = __builtin_nontemporal_load(bins.csc_bin + e);
-                    row[u] = __builtin_nontemporal_load(bins.csc_row + e);
-                    if (!ROOT && csc_gh != nullptr) {
-                        const unsigned long long w = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(csc_gh + e));
-                        s[u] = GHPair{__uint_as_float((unsigned)w), __uint_as_float((unsigned)(w >> 32))};
+                    const int q = min(q0 + u * kSpBlock, q1 - 1);
+                    bin4[u] = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(sp.table_bin) + q);
+                    if (NODES == kSpreadNodes) node4[u] = __builtin_nontemporal_load(nodes + q);
+                    if ((NODES != kSpreadNodes && NODES != kRootWords) || !copied) {
+                        const int4 r4 = reinterpret_cast<const int4 *>(sp.table_row)[q];
+                        row[u][0] = r4.x, row[u][1] = r4.y, row[u][2] = r4.z, row[u][3] = r4.w;
+                    }
+                    if (NODES != kRootNode && copied) {
+                        if (WORDS) {
+                            const uint4 w4 = reinterpret_cast<const uint4 *>(sp.table_gh)[q];
+                            g[u][0] = __uint_as_float(w4.x), g[u][1] = __uint_as_float(w4.y), g[u][2] = __uint_as_float(w4.z), g[u][3] = __uint_as_float(w4.w);
+                        } else {
+                            const float4 a = reinterpret_cast<const float4 *>(sp.table_gh)[2 * (set + q)], b = reinterpret_cast<const float4 *>(sp.table_gh)[2 * (set + q) + 1];
+                            g[u][0] = a.x, h[u][0] = a.y, g[u][1] = a.z, h[u][1] = a.w;
+                            g[u][2] = b.x, h[u][2] = b.y, g[u][3] = b.z, h[u][3] = b.w;
+                        }
+                    }
+                }
+                if (NODES == kRowNodes) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+#pragma unroll
+                        for (int k = 0; k < V; ++k) x[u][k] = (int)nid16[row[u][k]] - off - n0;
+                    }
+                }
+                if (NODES == kRootNode || !copied) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+#pragma unroll
+                        for (int k = 0; k < V; ++k) {
+                            if (WORDS) {
+                                g[u][k] = __uint_as_float(sp.gh_words[row[u][k]]);
+                            } else {
+                                const GHPair s = gh[row[u][k]];
+                                g[u][k] = s.g;
+                                h[u][k] = s.h;
+                            }
+                        }
+                    }
+                }
+                if (NODES == kRootNode && copied) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int q = q0 + u * kSpBlock;
+                        if (q >= q1) continue;
+                        if (WORDS) {
+                            reinterpret_cast<float4 *>(sp.table_gh)[q] = make_float4(g[u][0], g[u][1], g[u][2], g[u][3]);
+                        } else {
+                            reinterpret_cast<float4 *>(sp.table_gh)[2 * (set + q)] = make_float4(g[u][0], h[u][0], g[u][1], h[u][1]);
+                            reinterpret_cast<float4 *>(sp.table_gh)[2 * (set + q) + 1] = make_float4(g[u][2], h[u][2], g[u][3], h[u][3]);
+                        }
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < U; ++u) x[u] = ROOT ? 0 : (int)nid16[row[u]] - off - n0;
-                if (ROOT || csc_gh == nullptr) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) s[u] = gh[row[u]];
-                }
-                if (ROOT && csc_gh != nullptr) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (e0 + u * kSpBlock < v1) csc_gh[e0 + u * kSpBlock] = s[u];
-                }
-#pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (e0 + u * kSpBlock < v1 && (unsigned)x[u] < (unsigned)nn) {
-                        const long long gq = round_to_ll(s[u].g * scale_g), hq = round_to_ll(s[u].h * scale_h);
-                        unsigned long long *cell = reinterpret_cast<unsigned long long *>(cells + (size_t)x[u] * nbins + (gb[u] - bin0));
-                        atomicAdd(cell, (unsigned long long)gq);
-                        atomicAdd(cell + 1, (unsigned long long)hq);
+#pragma unroll
+                    for (int k = 0; k < V; ++k) {
+                        const int bin = (int)(bin4[u] >> 16 * k & 0xffffu), of = (int)(node4[u] >> 8 * k & 0xffu);
+                        const int at = NODES == kRootNode || NODES == kRootWords ? 0 : NODES == kRowNodes ? x[u][k] : of == 0xff ? -1 : of - n0;
+                        if (q0 + u * kSpBlock < q1 && (unsigned)at < (unsigned)nn && bin != (int)kTableEmpty) {
+                            const GHPair p = WORDS ? pair_from_word(sp.gh_objective, __float_as_uint(g[u][k])) : GHPair{g[u][k], h[u][k]};
+                            const long long gq = round_to_ll(p.g * scale_g), hq = round_to_ll(p.h * scale_h);
+                            unsigned long long *cell = reinterpret_cast<unsigned long long *>(cells + at * nbins + (bin - bin_shift));
+                            atomicAdd(cell, (unsigned long long)gq);
+                            atomicAdd(cell + 1, (unsigned long long)hq);
+                        }
                     }
                 }
             }
@@ -301,7 +399,7 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
                     partial[(size_t)(n0 + xx) * nbins + b] = cells[c];
                 }
             } else {
-                sp_search_batch(tb, sh, cells, level, fa, nf, bin0, n0, nn, task.cand_slot, mcw, lambda, dump);
+                sp_search_batch<BPL, DEEP>(tb, sh, cells, level, fa, nf, bin0, n0, nn, task.cand_slot, mcw, lambda, dump);
             }
         }
         f = fb;
@@ -310,6 +408,7 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_level(TreeBuffers tb_all, C
 }
 
 // A big feature: the tables of its chunks are added up (node range by node range) and searched.
+template <int BPL>
 __global__ __launch_bounds__(kSpBlock) void k_sparse_big(TreeBuffers tb_all, SparsePass sp, int level, float mcw,
                                                         float lambda, int dump_hist, int n_cells) {
     extern __shared__ longlong2 cells[];
@@ -335,18 +434,30 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_big(TreeBuffers tb_all, Spa
         const int nn = min(nn_max, ny1 - n0);
         const int n_cells = kf * nn;
         __syncthreads();
-        for (int c = threadIdx.x; c < n_cells; c += kSpBlock) {
+        // (few cells: the chunks are shared out over the threads that are left, whose sums meet in the cells)
+        const int parts = max(1, min(kSpBlock / n_cells, (big.slot_end - big.slot_begin) / 4));
+        if (parts > 1) {
+            for (int c = threadIdx.x; c < n_cells; c += kSpBlock) cells[c] = make_longlong2(0, 0);
+            __syncthreads();
+        }
+        for (int i = threadIdx.x; i < n_cells * parts; i += kSpBlock) {
+            const int part = i / n_cells, c = i - part * n_cells;
             long long g = 0, h = 0;
-#pragma unroll 4
-            for (int slot = big.slot_begin; slot < big.slot_end; ++slot) {
+#pragma unroll 8
+            for (int slot = big.slot_begin + part; slot < big.slot_end; slot += parts) {
                 const longlong2 v = base[(size_t)slot * sp.partial_stride + (size_t)n0 * kf + c];
                 g += v.x;
                 h += v.y;
             }
-            cells[c] = make_longlong2(g, h);
+            if (parts == 1) {
+                cells[c] = make_longlong2(g, h);
+            } else {
+                atomicAdd(reinterpret_cast<unsigned long long *>(cells + c), (unsigned long long)g);
+                atomicAdd(reinterpret_cast<unsigned long long *>(cells + c) + 1, (unsigned long long)h);
+            }
         }
         __syncthreads();
-        sp_search_batch(tb, sh, cells, level, f, 1, bin0, n0, nn, big.cand_slot, mcw, lambda, dump);
+        sp_search_batch<BPL, true>(tb, sh, cells, level, f, 1, bin0, n0, nn, big.cand_slot, mcw, lambda, dump);
     }
     sp_publish(tb, sh, level);
 }
@@ -374,7 +485,7 @@ __global__ __launch_bounds__(kSpBlock) void k_sparse_big(TreeBuffers tb_all, Spa
 //
 // Where every value looks its row's word up, that is what bounds it: a request for a 128-byte line of the L2 each, 127 us a level for
 // 18.8 M values of 1 M rows, 361 for twice the values of 2 M rows, whose words are more than an L2. On many values the rows' nodes
-// are therefore brought to them first (k_sparse_spread), 23 us, and the filter takes 47: 30 of them its vector instructions, 25 the
+// are therefore brought to them first (k_sparse_spread), and the filter takes 47: 30 of them its vector instructions, 25 the
 // LDS. A bound is some 70 instructions: a run's sums alone exclude most runs before their groups are looked at, and at deep levels
 // only runs that weigh enough are looked at, gathered from all threads (67 us without both). The tiles of a group are strided over
 // the features, whose frequencies often fall with their index.
@@ -519,21 +630,13 @@ __device__ __forceinline__ float rare_gain(GHPair f, float fterm, GHPair l, floa
     return fmaxf(0.f, gain);
 }
 
-// Upper estimate of rare_gain from the hardware reciprocal (1 ulp) instead of divisions; -1: the weight gate closes
-__device__ __forceinline__ float rare_gain_estimate(GHPair f, float fterm, GHPair l, float mcw, float lambda) {
-    const GHPair r{f.g - l.g, f.h - l.h};
-    if (!(l.h >= mcw && r.h >= mcw)) return -1.f;
-    const float a = l.g * l.g * __builtin_amdgcn_rcpf(l.h + lambda), b = r.g * r.g * __builtin_amdgcn_rcpf(r.h + lambda);
-    return (a + b - fterm) + (a + b + fabsf(fterm)) * 0x1p-18f;  // + 2^-18 of the terms: far above the roundings
-}
-
 // Signed score of a candidate (> 0: missing values go left), hist_tree_builder_single.cu:300-323. `floor`: the
 // largest |score| the candidate's node has seen so far; a candidate whose estimate stays below it cannot become the
 // node's best and is not evaluated (0 = no candidate).
 __device__ __forceinline__ float rare_score(GHPair S, float fterm, GHPair m, GHPair l, float mcw, float lambda, float floor) {
 #pragma clang fp contract(off)
     const GHPair l2{l.g + m.g, l.h + m.h};
-    const float er = rare_gain_estimate(S, fterm, l, mcw, lambda), el = rare_gain_estimate(S, fterm, l2, mcw, lambda);
+    const float er = gain_estimate(S, fterm, l, mcw, lambda), el = gain_estimate(S, fterm, l2, mcw, lambda);
     if (fmaxf(er, el) < floor) return 0.f;
     const float gr = rare_gain(S, fterm, l, mcw, lambda);
     const float gl = rare_gain(S, fterm, l2, mcw, lambda);
@@ -715,54 +818,78 @@ __device__ void rare_search(const TreeBuffers &tb, const SparsePass &sp, RareSha
     __syncthreads();
 }
 
-// Brings what the rows of the rare values hold to the values' places: a row block's part in LDS, looked up there. Fetched by
+// Brings what the rows of the values hold to the values' places: a row block's part in LDS, looked up there. Fetched by
 // the filter itself a look-up is a request for a whole line of the L2, whatever it takes of it.
-// CODES: the rows' words, with the value's feature in the node's place, once per tree; else the rows' nodes of a level. Bound by its
-// traffic: 4 bytes a value (2 the row in its block, 1 the place, 1 the node), 18.8 M values in 23 us, 52 for the words. Blocks of
-// 32 768 rows: their words still fit the LDS, and a tile of 4096 values has some 130 of a block next to each other at 1 M rows.
-template <bool CODES>
+// kBringCodes: the rows' words, with the value's feature in the node's place, to the rare values, once per tree; kBringPairs: the rows'
+// gradient words to the table values, once per tree; kBringNodes: the rows' nodes of a level to all of them. Bound by its traffic: 4
+// bytes a node (2 the row in its block, 1 the place, 1 the node), 36 M values in 33.5 us, 4.3 TB/s (37 with the groups of a step
+// fetched when it begins). Blocks of 32 768 rows: their words still fit the LDS, and a tile of
+// 4096 values has some 130 of a block next to each other at 1 M rows.
+enum { kBringCodes, kBringPairs, kBringNodes };
+template <int WHAT>
 __global__ __launch_bounds__(1024) void k_sparse_spread(TreeBuffers tb_all, SparsePass sp, int level) {
     extern __shared__ unsigned spread_dyn[];  // [kSpreadRows] words, or as many bytes
     const TreeBuffers tb = tb_all.for_class(blockIdx.z);
     const int r0 = (int)blockIdx.y << kSpreadLogRows, rows = min(kSpreadRows, tb.n - r0);
-    const unsigned *__restrict__ begin = sp.spread_begin + (size_t)blockIdx.y * sp.n_rare_tasks;
-    const unsigned g0 = begin[0], g1 = begin[sp.n_rare_tasks];
+    const unsigned *__restrict__ begin = sp.spread_begin + (size_t)blockIdx.y * sp.n_lists;
+    const unsigned g0 = begin[WHAT == kBringPairs ? sp.n_rare_tasks : 0], g1 = begin[WHAT == kBringCodes ? sp.n_rare_tasks : sp.n_lists];
     const unsigned per = (g1 - g0 + gridDim.x - 1) / gridDim.x;
     const unsigned first = g0 + blockIdx.x * per, end = min(g1, first + per);
-    const size_t set = (size_t)blockIdx.z * sp.n_rare_places;
     if (first >= end) return;
-    if (CODES) {
-        for (int r = threadIdx.x; r < rows; r += 1024) spread_dyn[r] = tb.row_word[r0 + r] & ~kRareNodeMask;
-    } else {
+    constexpr int U = WHAT == kBringNodes ? 4 : 2;
+    // (the groups of the next step are on their way while this one's are looked up; past the end the last group once more, with the
+    // same result)
+    uint2 next_row[U];
+    unsigned next_place[U];
+    const auto fetch = [&](unsigned i) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned g = min(i + u * 1024, end - 1);
+            next_row[u] = reinterpret_cast<const uint2 *>(sp.spread_row)[g];
+            next_place[u] = sp.spread_place[g];
+        }
+    };
+    fetch(first + threadIdx.x);
+    if (WHAT == kBringNodes) {
         const unsigned off = (1u << level) - 1u;
         const unsigned *__restrict__ pairs = reinterpret_cast<const unsigned *>(tb.nid16 + r0);
         unsigned short *out = reinterpret_cast<unsigned short *>(spread_dyn);
-        for (int i = threadIdx.x; i < (rows + 1) / 2; i += 1024) {
-            const unsigned v = pairs[i], a = v & 0xffffu, b = v >> 16;
-            out[i] = (unsigned short)((a >= off ? a - off : 0xffu) | (b >= off ? (b - off) & 0xffu : 0xffu) << 8);
+        const int n_pairs = (rows + 1) / 2;
+        constexpr int L = kSpreadRows / 2 / 1024;
+        unsigned v[L];
+#pragma unroll
+        for (int l = 0; l < L; ++l) v[l] = pairs[min(l * 1024 + (int)threadIdx.x, n_pairs - 1)];
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            const unsigned a = v[l] & 0xffffu, b = v[l] >> 16;
+            out[l * 1024 + threadIdx.x] = (unsigned short)((a >= off ? a - off : 0xffu) | (b >= off ? (b - off) & 0xffu : 0xffu) << 8);
         }
+    } else {
+        const unsigned *__restrict__ words = WHAT == kBringCodes ? tb.row_word : sp.gh_words;
+#pragma unroll 8
+        for (int r = threadIdx.x; r < rows; r += 1024) spread_dyn[r] = WHAT == kBringCodes ? words[r0 + r] & ~kRareNodeMask : words[r0 + r];
     }
     __syncthreads();
-    constexpr int U = CODES ? 2 : 4;
     for (unsigned i = first + threadIdx.x; i < end; i += 1024 * U) {
         uint2 row[U];
         unsigned place[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const unsigned g = min(i + u * 1024, end - 1);  // (past the end: the last group once more, with the same result)
-            row[u] = reinterpret_cast<const uint2 *>(sp.spread_row)[g];
-            place[u] = sp.spread_place[g];
-        }
+        for (int u = 0; u < U; ++u) row[u] = next_row[u], place[u] = next_place[u];
+        fetch(i + 1024 * U);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const unsigned a = row[u].x & 0xffffu, b = row[u].x >> 16, c = row[u].y & 0xffffu, d = row[u].y >> 16;
-            if (CODES) {
+            if (WHAT == kBringCodes) {
                 const uint4 key = reinterpret_cast<const uint4 *>(sp.rare_key)[place[u]];
                 const auto code = [&](unsigned r, unsigned k) { return k == kRareEmpty ? kRareEmpty : spread_dyn[r] | k >> kRareFeatShift; };
-                reinterpret_cast<uint4 *>(sp.rare_code + set)[place[u]] = make_uint4(code(a, key.x), code(b, key.y), code(c, key.z), code(d, key.w));
+                reinterpret_cast<uint4 *>(sp.rare_code + (size_t)blockIdx.z * sp.n_rare_places)[place[u]] =
+                    make_uint4(code(a, key.x), code(b, key.y), code(c, key.z), code(d, key.w));
+            } else if (WHAT == kBringPairs) {
+                reinterpret_cast<uint4 *>(sp.table_gh)[place[u] - (unsigned)(sp.n_rare_places / kSpreadGroup)] =
+                    make_uint4(spread_dyn[a], spread_dyn[b], spread_dyn[c], spread_dyn[d]);
             } else {
                 const uint8_t *nodes = reinterpret_cast<const uint8_t *>(spread_dyn);
-                reinterpret_cast<unsigned *>(sp.rare_node + set)[place[u]] =
+                reinterpret_cast<unsigned *>(sp.value_node + (size_t)blockIdx.z * (sp.n_rare_places + sp.n_table_places))[place[u]] =
                     (unsigned)nodes[a] | (unsigned)nodes[b] << 8 | (unsigned)nodes[c] << 16 | (unsigned)nodes[d] << 24;
             }
         }
@@ -795,8 +922,9 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
     if (SPREAD) {
         static_assert(kRareV % kSpreadGroup == 0 && kSpreadGroup == 4, "a thread's places are whole groups");
         const size_t first = (size_t)blockIdx.z * sp.n_rare_places + task.v_begin;
+        const size_t first_node = (size_t)blockIdx.z * (sp.n_rare_places + sp.n_table_places) + task.v_begin;
         const uint4 *__restrict__ codes = reinterpret_cast<const uint4 *>(sp.rare_code + first);
-        const unsigned *__restrict__ nodes = reinterpret_cast<const unsigned *>(sp.rare_node + first);
+        const unsigned *__restrict__ nodes = reinterpret_cast<const unsigned *>(sp.value_node + first_node);
         const unsigned *__restrict__ groups = reinterpret_cast<const unsigned *>(sp.rare_group + task.v_begin);
         uint4 c[kRareV / 4];
         unsigned x[kRareV / 4], g[kRareV / 4];
@@ -930,7 +1058,8 @@ __global__ __launch_bounds__(kRareBlock, 8) void k_sparse_rare_filter(TreeBuffer
         // (few values pass: they are read again)
         int at = pass != 0 ? atomicAdd(&sh.passed, __popc(pass)) : 0;
         unsigned long long *out = sp.rare_item + (size_t)blockIdx.z * sp.n_rare_places + task.v_begin;
-        const uint8_t *__restrict__ nodes = SPREAD ? sp.rare_node + (size_t)blockIdx.z * sp.n_rare_places + task.v_begin : nullptr;
+        const uint8_t *__restrict__ nodes =
+            SPREAD ? sp.value_node + (size_t)blockIdx.z * (sp.n_rare_places + sp.n_table_places) + task.v_begin : nullptr;
         for (unsigned left = pass; left != 0; left &= left - 1) {
             const int q = place(__ffs(left) - 1);
             const unsigned x = !SPREAD ? words[rows[q]] & kRareNodeMask : level > 0 ? (unsigned)nodes[q] : 0u;
@@ -1072,6 +1201,56 @@ __global__ __launch_bounds__(256) void k_sparse_cols(long nnz, const int *__rest
     }
 }
 
+// First value of a table feature (positions [v0, v1) of the bin-major copy, rows ascend) whose row is not before `row`.
+__device__ __forceinline__ int first_value_of(const int *__restrict__ rows, int v0, int v1, long row) {
+    while (v0 < v1) {
+        const int mid = v0 + (v1 - v0) / 2;
+        if (rows[mid] < row) v0 = mid + 1;
+        else v1 = mid;
+    }
+    return v0;
+}
+
+__global__ __launch_bounds__(256) void k_table_count(SparsePass sp, CsrBins bins, unsigned *__restrict__ count) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= sp.n_table_features) return;
+    const int f = sp.table_features[i], v0 = sp.feat_val_begin[f], v1 = sp.feat_val_begin[f + 1];
+    const long r0 = (long)blockIdx.y << kSpreadLogRows;
+    const int m = first_value_of(bins.csc_row, v0, v1, r0 + kSpreadRows) - first_value_of(bins.csc_row, v0, v1, r0);
+    count[(size_t)blockIdx.y * sp.n_lists + sp.n_rare_tasks + i] = (unsigned)(m + kSpreadGroup - 1) / kSpreadGroup;
+}
+
+// Places of the values of a table feature, blockIdx.y its row block (not spread: the one block is all rows). What is left of
+// its places after the last block's is nobody's.
+__global__ __launch_bounds__(256) void k_table_setup(SparsePass sp, CsrBins bins, const int *__restrict__ task_bin0, int *__restrict__ row,
+                                                    unsigned short *__restrict__ table_bin, unsigned short *__restrict__ spread_row,
+                                                    unsigned *__restrict__ spread_place) {
+    const int i = blockIdx.x, f = sp.table_features[i], b = blockIdx.y;
+    const bool spread = sp.n_spread > 0;
+    int v0 = sp.feat_val_begin[f], v1 = sp.feat_val_begin[f + 1], at = sp.table_first[f];
+    unsigned list = 0;
+    if (spread) {
+        const unsigned *begin = sp.spread_begin + sp.n_rare_tasks + i;
+        for (int a = 0; a < b; ++a) at += (int)(begin[(size_t)a * sp.n_lists + 1] - begin[(size_t)a * sp.n_lists]) * kSpreadGroup;
+        list = begin[(size_t)b * sp.n_lists];
+        const long r0 = (long)b << kSpreadLogRows;
+        const int end = v1;
+        v1 = first_value_of(bins.csc_row, v0, end, r0 + kSpreadRows);
+        v0 = first_value_of(bins.csc_row, v0, end, r0);
+    }
+    const int m = v1 - v0, wide = (m + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
+    const int stop = b + 1 == (int)gridDim.y ? sp.table_first[f + 1] - at : wide;
+    for (int a = threadIdx.x; a < stop; a += 256) {
+        const int r = a < m ? bins.csc_row[v0 + a] : 0;
+        row[at + a] = r;
+        table_bin[at + a] = a < m ? (unsigned short)(bins.csc_bin[v0 + a] - task_bin0[f]) : (unsigned short)kTableEmpty;
+        if (spread && a < wide) {
+            spread_row[(size_t)list * kSpreadGroup + a] = (unsigned short)(r & (kSpreadRows - 1));
+            if (a % kSpreadGroup == 0) spread_place[list + a / kSpreadGroup] = (unsigned)((sp.n_rare_places + at + a) / kSpreadGroup);
+        }
+    }
+}
+
 // Groups of four places that the values of a task take in every row block.
 __global__ __launch_bounds__(256) void k_rare_count(SparsePass sp, CsrBins bins, unsigned *__restrict__ count) {
     __shared__ unsigned values[kSpreadBlocks];
@@ -1085,8 +1264,7 @@ __global__ __launch_bounds__(256) void k_rare_count(SparsePass sp, CsrBins bins,
     }
     __syncthreads();
     for (int b = threadIdx.x; b < sp.n_spread; b += 256)
-        count[(size_t)b * sp.n_rare_tasks + blockIdx.x] = (values[b] + kSpreadGroup - 1) / kSpreadGroup;
-    if (blockIdx.x == 0 && threadIdx.x == 0) count[(size_t)sp.n_spread * sp.n_rare_tasks] = 0u;
+        count[(size_t)b * sp.n_lists + blockIdx.x] = (values[b] + kSpreadGroup - 1) / kSpreadGroup;
 }
 
 // Places of the values of a task: spread ones by row block (in a block in any order), else its features one after the other, each
@@ -1099,7 +1277,7 @@ __global__ __launch_bounds__(256) void k_rare_setup(SparsePass sp, CsrBins bins,
     const RareTask task = sp.rare_tasks[blockIdx.x];
     const int blocks = sp.n_spread;
     for (int b = threadIdx.x; b < blocks; b += 256) {
-        const unsigned *at = sp.spread_begin + (size_t)b * sp.n_rare_tasks + blockIdx.x;
+        const unsigned *at = sp.spread_begin + (size_t)b * sp.n_lists + blockIdx.x;
         from[b] = at[0] * kSpreadGroup;
         first[b + 1] = (at[1] - at[0]) * kSpreadGroup;
         taken[b] = 0u;
@@ -1156,8 +1334,17 @@ void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *
     k_sparse_cols<<<grid, 256, 0, s>>>(nnz, csc_bin, csc_row, cut_fid, cut_row_ptr, col_of_feature, colbin, col_stride);
 }
 
-void launch_rare_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count) {
-    k_rare_count<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, count);
+void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count) {
+    if (sp.n_rare_tasks > 0) k_rare_count<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, count);
+    if (sp.n_table_features > 0)
+        k_table_count<<<dim3((sp.n_table_features + 255) / 256, sp.n_spread), 256, 0, s>>>(sp, bins, count);
+}
+
+void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,
+                        unsigned short *spread_row, unsigned *spread_place) {
+    if (sp.n_table_features > 0)
+        k_table_setup<<<dim3(sp.n_table_features, std::max(1, sp.n_spread)), 256, 0, s>>>(sp, bins, task_bin0, row, table_bin, spread_row,
+                                                                                         spread_place);
 }
 
 void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
@@ -1184,27 +1371,53 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
             launch_fill_f32(s, reinterpret_cast<float *>(tb.for_class(k).hist(level)), 0.f,
                             (size_t)(1 << level) * tb.n_bins * 4);
     }
+#define TGBM_SPARSE_LEVEL(NODES, WORDS, BPL, DEEP)                                                                            \
+    {                                                                                                                       \
+        static LdsOptIn opt_in;                                                                                             \
+        opt_in({reinterpret_cast<const void *>(&k_sparse_level<NODES, WORDS, BPL, DEEP>)});                                  \
+        k_sparse_level<NODES, WORDS, BPL, DEEP><<<tasks, kSpBlock, lds, s>>>(tb, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells); \
+    }
+#define TGBM_SPARSE_LEVEL_OF(WORDS, BPL, ROOT_DEEP)                                                                          \
+    {                                                                                                                       \
+        if (level == 0 && spread && WORDS && sp.table_gh != nullptr) TGBM_SPARSE_LEVEL(kRootWords, true, BPL, ROOT_DEEP)      \
+        else if (level == 0) TGBM_SPARSE_LEVEL(kRootNode, WORDS, BPL, ROOT_DEEP)                                             \
+        else if (spread && (ROOT_DEEP || level > 3)) TGBM_SPARSE_LEVEL(kSpreadNodes, WORDS, BPL, true)                        \
+        else if (spread) TGBM_SPARSE_LEVEL(kSpreadNodes, WORDS, BPL, ROOT_DEEP)                                              \
+        else if (ROOT_DEEP || level > 3) TGBM_SPARSE_LEVEL(kRowNodes, WORDS, BPL, true)                                      \
+        else TGBM_SPARSE_LEVEL(kRowNodes, WORDS, BPL, ROOT_DEEP)                                                             \
+    }
     static LdsOptIn opt_in;
-    opt_in({reinterpret_cast<const void *>(&k_sparse_level<true>), reinterpret_cast<const void *>(&k_sparse_level<false>), reinterpret_cast<const void *>(&k_sparse_big),
-            reinterpret_cast<const void *>(&k_sparse_spread<true>)});
+    opt_in({reinterpret_cast<const void *>(&k_sparse_big<1>), reinterpret_cast<const void *>(&k_sparse_big<4>),
+            reinterpret_cast<const void *>(&k_sparse_spread<kBringCodes>), reinterpret_cast<const void *>(&k_sparse_spread<kBringPairs>)});
+    const bool spread = sp.n_spread > 0 && level <= kSpreadLevel;
+    if (spread) {
+        // (a workgroup begins with the block's rows: no more of them than the chip holds at once)
+        const auto grid = [&](int workgroups) { return dim3(std::max(1, workgroups / (sp.n_spread * n_class)), sp.n_spread, n_class); };
+        if (level > 0) k_sparse_spread<kBringNodes><<<grid(512), 1024, kSpreadRows, s>>>(tb, sp, level);
+        if (level == 0 && sp.n_rare_tasks > 0) k_sparse_spread<kBringCodes><<<grid(256), 1024, kSpreadRows * sizeof(unsigned), s>>>(tb, sp, level);
+        if (level == 0 && sp.gh_words != nullptr && sp.table_gh != nullptr)
+            k_sparse_spread<kBringPairs><<<grid(256), 1024, kSpreadRows * sizeof(unsigned), s>>>(tb, sp, level);
+    }
     if (sp.n_tasks > 0) {
         const dim3 tasks(sp.n_tasks, 1, n_class);
-        if (level == 0) k_sparse_level<true><<<tasks, kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
-        else k_sparse_level<false><<<tasks, kSpBlock, lds, s>>>(tb, bins, sp, gh, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+        if (sp.gh_words != nullptr && sp.max_table_bins <= 64) TGBM_SPARSE_LEVEL_OF(true, 1, false)
+        else if (sp.gh_words != nullptr) TGBM_SPARSE_LEVEL_OF(true, 4, true)
+        else if (sp.max_table_bins <= 64) TGBM_SPARSE_LEVEL_OF(false, 1, false)
+        else TGBM_SPARSE_LEVEL_OF(false, 4, true)
     }
-    if (sp.n_big > 0)
-        k_sparse_big<<<dim3(sp.n_big, std::min(1 << level, 16), n_class), kSpBlock, lds, s>>>(
-            tb, sp, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+#undef TGBM_SPARSE_LEVEL_OF
+#undef TGBM_SPARSE_LEVEL
+    if (sp.n_big > 0) {
+        // (as many workgroups as the chip holds at once: each is a chain of some ten dependent steps, whatever its nodes are)
+        const dim3 grid(sp.n_big, std::min(1 << level, std::max(1, std::min(16, 512 / (sp.n_big * n_class)))), n_class);
+        n_cells = std::min(n_cells, sp.max_table_bins * (((1 << level) + (int)grid.y - 1) / (int)grid.y));
+        const size_t lds = sizeof(longlong2) * (size_t)n_cells;
+        if (sp.max_table_bins <= 64) k_sparse_big<1><<<grid, kSpBlock, lds, s>>>(tb, sp, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+        else k_sparse_big<4><<<grid, kSpBlock, lds, s>>>(tb, sp, level, mcw, lambda, dump_hist ? 1 : 0, n_cells);
+    }
     if (sp.n_rare_tasks > 0) {
         const size_t nodes_lds = (size_t)(1 << level) * 20;
         const dim3 tiles(sp.n_rare_tasks, 1, n_class);
-        const bool spread = sp.n_spread > 0 && level <= kSpreadLevel;
-        if (spread) {
-            // (a workgroup begins with the block's rows: no more of them than the chip holds at once)
-            const auto grid = [&](int workgroups) { return dim3(std::max(1, workgroups / (sp.n_spread * n_class)), sp.n_spread, n_class); };
-            if (level == 0) k_sparse_spread<true><<<grid(256), 1024, kSpreadRows * sizeof(unsigned), s>>>(tb, sp, level);
-            else k_sparse_spread<false><<<grid(512), 1024, kSpreadRows, s>>>(tb, sp, level);
-        }
         if (dump_hist && spread) k_sparse_rare_filter<true, true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
         else if (dump_hist) k_sparse_rare_filter<true, false><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
         else if (spread) k_sparse_rare_filter<false, true><<<tiles, kRareBlock, nodes_lds, s>>>(tb, sp, gh, level, mcw, lambda);
@@ -1213,7 +1426,10 @@ void launch_sparse_level(hipStream_t s, const TreeBuffers &tb, const CsrBins &bi
     }
 }
 
-void launch_sparse_partition(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, int level, int n_class) {
+void launch_sparse_partition(hipStream_t s, const TreeBuffers &all, const CsrBins &bins, const SparsePass &sp, int level, int n_class) {
+    // (spread values: nobody asks a row's word for its node but the levels past kSpreadLevel)
+    TreeBuffers tb = all;
+    if (sp.n_spread > 0 && (level < kSpreadLevel || level + 1 >= tb.depth)) tb.row_word = nullptr;
     const int grid = std::max(1, std::min(1024, (tb.n + kSpBlock * kMoveRows - 1) / (kSpBlock * kMoveRows)));
     k_sparse_partition<<<dim3(grid, 1, n_class), kSpBlock, 0, s>>>(tb, bins, level);
 }

@@ -108,13 +108,14 @@ class Trainer {
     int n_ = 0, F_ = 0, n_bins_ = 0;
     long nnz_ = 0;
     int objective_ = OBJ_SQUARE, metric_kind_ = 0;
-    // Dense layout with a spare dword at the end of every row's record, one tree per round, squared or binary logistic
-    // loss: the rows' gradient pairs also travel as one word in that dword (DenseBins::gh_lane), written by whatever
+    // Sparse level pass: the rows' pairs also as words, which it copies to the values. Dense layout with a spare dword at the end of
+    // every row's record, one tree per round, squared or binary logistic loss: the rows' gradient pairs also travel as one word in that dword (DenseBins::gh_lane), written by whatever
     // computes the round's gradients (into an array of their own; the root level's histogram launch moves them).
     int gh_word_lane_ = -1;
     bool gh_words_fresh_ = false;   // d_gh_words_ matches d_gh_
     bool gh_records_fresh_ = false;  // and the root level's histogram launch of this tree has copied it into the records
     unsigned *d_gh_words_ = nullptr;  // [n]
+    bool sparse_words_ = false;       // the level pass of this tree goes by them
     // Inside boost() the fused end of a round leaves the next gradients as words only when nothing of the next tree
     // reads the pair array (the histogram kernels take the words, the root's sums come from a complete feature's
     // bins, the tree's scales from the pass's own statistics); whoever wants the array then - the stage-wise API, a
@@ -143,8 +144,10 @@ class Trainer {
     int hist_cap_level_ = -1;       // first level with more nodes than the histogram arena holds (-1: none)
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
     long sparse_rare_most_ = 0;  // a feature with more stored values is served through tables
+    int *d_task_bin0_ = nullptr;  // [F] sparse level pass: first bin of the table task that a feature belongs to
     long rare_tile_ = 0;         // values per task of the others at most
     bool sparse_feature_in_tables(int f);
+    bool gradient_words_wanted() const;
     SparsePass sp_;
     void build_sparse_tasks();
     void ensure_hist_arena();  // per-node histograms for stage-wise inspection (the level pass itself keeps none)

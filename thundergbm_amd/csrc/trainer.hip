@@ -291,6 +291,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
                          (double)(n_cols * col_stride) * 1e-6);
             }
         }
+        if (sparse_pass_ && gradient_words_wanted()) d_gh_words_ = dalloc<unsigned>((size_t)n_);
         bins_.W = 4;
         bins_.n_blocks = 1;
         HIP_CHECK(hipStreamSynchronize(stream_));
@@ -420,11 +421,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         bins_.col_stride = col_stride;
         bins_.data = d_binmat_;
         {
-            // (TGBM_GH_WORD=0: the histogram kernels always gather the pairs from the gradient array; tests)
-            const char *ge = std::getenv("TGBM_GH_WORD");
-            const bool off = ge != nullptr && std::string(ge) == "0";
-            const bool loss_ok = param.objective == "reg:linear" || param.objective == "binary:logistic";  // (labels 0 / 1)
-            if (!off && loss_ok && param.tree_per_rounds == 1 && bin_bytes == 1 && n_blocks == 1 && W >= 16 && P <= W - 4) {
+            if (gradient_words_wanted() && bin_bytes == 1 && n_blocks == 1 && W >= 16 && P <= W - 4) {
                 gh_word_lane_ = W / 4 - 1;
                 bins_.gh_lane = gh_word_lane_;
                 d_gh_words_ = dalloc<unsigned>((size_t)n_);
@@ -545,7 +542,7 @@ void Trainer::alloc_tree_buffers() {
     const size_t set_bytes =
         sparse_pass_ ? (size_t)n_ * 15 + (size_t)sp_.n_partial_slots * sp_.partial_stride * sizeof(longlong2) +
                            (size_t)max_level_nodes * sp_.n_cand_slots * sizeof(SplitCand) +
-                           sp_.n_rare_places * (sp_.n_spread > 0 ? 13 : 8) + (size_t)nnz_ * sizeof(GHPair)
+                           sp_.n_rare_places * (sp_.n_spread > 0 ? 13 : 8) + sp_.n_table_places * (sizeof(GHPair) + (sp_.n_spread > 0 ? 1 : 0))
                      : fixed_bytes + arena_bytes(hist_nodes);
     const char *be = std::getenv("TGBM_BATCH_CLASSES");  // "0": build the trees of a round one after the other
     n_sets_ = (K > 1 && set_bytes * K < free_b / 2 && !(be != nullptr && std::string(be) == "0")) ? K : 1;
@@ -636,47 +633,56 @@ void Trainer::alloc_tree_buffers() {
     if (sparse_pass_) {
         tb.best_key = dalloc<unsigned long long>(S * (size_t)max_level_nodes);
         HIP_CHECK(hipMemsetAsync(tb.best_key, 0, sizeof(unsigned long long) * S * (size_t)max_level_nodes, stream_));
+        unsigned *spread_place = nullptr;
+        unsigned short *spread_row = nullptr;
+        if (sp_.n_spread > 0) {
+            const long lists = (long)sp_.n_spread * sp_.n_lists;
+            unsigned *count = nullptr, *total = nullptr, *begin = dalloc<unsigned>((size_t)lists + 1);
+            device_alloc_to(count, sizeof(unsigned) * ((size_t)lists + 1));
+            device_alloc_to(total, sizeof(unsigned));
+            HIP_CHECK(hipMemsetAsync(count + lists, 0, sizeof(unsigned), stream_));
+            launch_spread_count(stream_, csr_, sp_, count);
+            ScanScratch scratch;
+            device_exclusive_scan(stream_, count, begin, lists + 1, total, scratch);
+            HIP_CHECK(hipStreamSynchronize(stream_));
+            scratch.release();
+            device_free(count);
+            device_free(total);
+            sp_.spread_begin = begin;
+            const size_t places = sp_.n_rare_places + sp_.n_table_places;
+            spread_row = dalloc<unsigned short>(places);
+            spread_place = dalloc<unsigned>(places / kSpreadGroup);
+            sp_.value_node = dalloc<uint8_t>(S * places);
+        }
         if (sp_.n_rare_tasks > 0) {
             int *row = dalloc<int>(sp_.n_rare_places), *places = dalloc<int>((size_t)sp_.n_rare_tasks);
-            unsigned *key = dalloc<unsigned>(sp_.n_rare_places), *spread_place = nullptr;
+            unsigned *key = dalloc<unsigned>(sp_.n_rare_places);
             uint8_t *group = nullptr;
-            unsigned short *spread_row = nullptr;
             if (sp_.n_spread > 0) {
-                const long lists = (long)sp_.n_spread * sp_.n_rare_tasks;
-                unsigned *count = nullptr, *total = nullptr, *begin = dalloc<unsigned>((size_t)lists + 1);
-                device_alloc_to(count, sizeof(unsigned) * ((size_t)lists + 1));
-                device_alloc_to(total, sizeof(unsigned));
-                launch_rare_count(stream_, csr_, sp_, count);
-                ScanScratch scratch;
-                device_exclusive_scan(stream_, count, begin, lists + 1, total, scratch);
-                HIP_CHECK(hipStreamSynchronize(stream_));
-                scratch.release();
-                device_free(count);
-                device_free(total);
-                sp_.spread_begin = begin;
                 group = dalloc<uint8_t>(sp_.n_rare_places);
-                spread_row = dalloc<unsigned short>(sp_.n_rare_places);
-                spread_place = dalloc<unsigned>(sp_.n_rare_places / kSpreadGroup);
                 sp_.rare_code = dalloc<unsigned>(S * sp_.n_rare_places);
-                sp_.rare_node = dalloc<uint8_t>(S * sp_.n_rare_places);
             }
             launch_rare_setup(stream_, tb, csr_, sp_, row, key, places, group, spread_row, spread_place);
             sp_.rare_row = row;
             sp_.rare_key = key;
             sp_.rare_places = places;
             sp_.rare_group = group;
-            sp_.spread_row = spread_row;
-            sp_.spread_place = spread_place;
             sp_.rare_item = dalloc<unsigned long long>(S * sp_.n_rare_places);
             sp_.rare_passed = dalloc<int>(S * (size_t)sp_.n_rare_tasks);
         }
+        int *table_row = dalloc<int>(sp_.n_table_places);
+        unsigned short *table_bin = dalloc<unsigned short>(sp_.n_table_places);
+        launch_table_setup(stream_, csr_, sp_, d_task_bin0_, table_row, table_bin, spread_row, spread_place);
+        sp_.table_row = table_row;
+        sp_.table_bin = table_bin;
+        sp_.spread_row = spread_row;
+        sp_.spread_place = spread_place;
         sp_.partial = dalloc<longlong2>(S * (size_t)sp_.n_partial_slots * sp_.partial_stride);
-        // per-value gradient pairs in the order of the bin-major copy, when they fit comfortably
-        sp_.nnz = nnz_;
+        // the pairs of the table features' values, when they fit comfortably
         device_mem_info(&free_b, &total_b);
         const char *ge = std::getenv("TGBM_SPARSE_GH_COPY");  // "0": gather the pairs per value instead (tests)
-        if (S * (size_t)nnz_ * sizeof(GHPair) < free_b / 4 && !(ge != nullptr && std::string(ge) == "0"))
-            sp_.csc_gh = dalloc<GHPair>(S * (size_t)nnz_);
+        if (S * sp_.n_table_places * sizeof(GHPair) < free_b / 4 && !(ge != nullptr && std::string(ge) == "0"))
+            sp_.table_gh = dalloc<GHPair>(S * sp_.n_table_places);
     }
     int *d_pack = dalloc<int>(pack_begin.size());
     upload(stream_, d_pack, pack_begin.data(), pack_begin.size());
@@ -771,7 +777,7 @@ void Trainer::compute_gradient() {
         launch_gradient(stream_, objective_, n_, param_.num_class, d_y_, d_yp_, d_gh_, nullptr, 0);
     }
     gh_words_fresh_ = gh_records_fresh_ = false;
-    if (gh_word_lane_ >= 0 && !param_.bagging) {  // (bagging multiplies the pairs by draw counts)
+    if (d_gh_words_ != nullptr && !param_.bagging) {  // (bagging multiplies the pairs by draw counts)
         launch_gh_words(stream_, objective_, n_, d_y_, d_yp_, d_gh_words_);
         gh_words_fresh_ = true;
     }
@@ -886,6 +892,14 @@ void Trainer::ensure_hist_arena() {
     tb_.hist_nodes = tb_.max_level_nodes;
 }
 
+// A row's gradient pair also as one word (word_from_row): squared loss, or logistic loss on labels of 0 and 1, one tree a round.
+// (TGBM_GH_WORD=0: the pairs only; tests)
+bool Trainer::gradient_words_wanted() const {
+    const char *ge = std::getenv("TGBM_GH_WORD");
+    return !(ge != nullptr && std::string(ge) == "0") && (param_.objective == "reg:linear" || param_.objective == "binary:logistic") &&
+           param_.tree_per_rounds == 1;
+}
+
 // Which features the sparse level pass serves through (bin, node) tables: those with more values than a tile of rare
 // features holds, the most frequent ones of the others, and the feature that owns global bin 0 (its table is searched
 // for every node even without values: the arg-max of a node without any positive gain ends there).
@@ -920,9 +934,25 @@ bool Trainer::sparse_feature_in_tables(int f) {
 // task_values values, a feature with more than kSparseTaskValues cut into chunks (tasks of their own) whose tables
 // k_sparse_big adds up.
 void Trainer::build_sparse_tasks() {
-    std::vector<int> fvb(F_ + 1, 0);
-    for (int f = 0; f < F_; ++f) fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
+    std::vector<int> fvb(F_ + 1, 0), first(F_ + 1, 0), task_bin0(F_, 0), table_features;
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
+    (void)is_table(0);  // (decides whether values are spread)
+    // places of a feature or task: its values, and up to three nobody's in every row block
+    const auto places_of = [&](long values) {
+        const long blocks = std::min<long>(std::max(1, sp_.n_spread), values);
+        return (values + (kSpreadGroup - 1) * blocks + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
+    };
+    long table_places = 0;
+    for (int f = 0; f < F_; ++f) {
+        fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
+        first[f] = (int)table_places;
+        if (is_table(f)) {
+            table_features.push_back(f);
+            table_places += places_of(cuts_.feature_nnz[f]);
+        }
+    }
+    first[F_] = (int)table_places;
+    TGBM_CHECK(table_places < (1l << 31) - 16, "%ld places for the values of the frequent features", table_places);
     // A task serves its features one after the other, about 12 us each at 128 nodes: where all tasks together do not fill the
     // chip they are smaller (200 k x 100 k, depth 8, 67 tasks of 32768 values: 1.48 ms a tree, a thousandth of the values
     // each: 1.05; 1 M rows: 2.63 -> 2.43).
@@ -936,6 +966,9 @@ void Trainer::build_sparse_tasks() {
     std::vector<int2> rare_meta;
     std::vector<int> feat_slot(F_, -1);
     int n_small = 0, n_partial = 0, max_big_bins = 0;
+    sp_.max_table_bins = 0;
+    for (int q = 0; q < F_; ++q)
+        if (is_table(q)) sp_.max_table_bins = std::max(sp_.max_table_bins, h_cut_row_ptr_[q + 1] - h_cut_row_ptr_[q]);
     int f = 0;
     while (f < F_) {
         const long m = cuts_.feature_nnz[f];
@@ -951,10 +984,11 @@ void Trainer::build_sparse_tasks() {
             SparseBig b;
             b.feature = f;
             b.slot_begin = n_partial;
-            for (long v = 0; v < m; v += kSparseTaskValues) {
-                SparseTask t{f, f + 1, fvb[f] + (int)v, fvb[f] + (int)std::min(m, v + kSparseTaskValues), -1, n_partial++};
+            for (int v = first[f]; v < first[f + 1]; v += kSparseTaskValues) {
+                SparseTask t{f, f + 1, v, std::min(first[f + 1], v + kSparseTaskValues), -1, n_partial++};
                 tasks.push_back(t);
             }
+            task_bin0[f] = h_cut_row_ptr_[f];
             b.slot_end = n_partial;
             b.cand_slot = -1;  // numbered below
             big.push_back(b);
@@ -965,12 +999,12 @@ void Trainer::build_sparse_tasks() {
         int fe = f;
         long vals = 0;
         while (fe < F_ && is_table(fe) && cuts_.feature_nnz[fe] <= kSparseTaskValues &&
-               (fe == f || vals + cuts_.feature_nnz[fe] <= task_values)) {
+               (fe == f || (vals + cuts_.feature_nnz[fe] <= task_values && h_cut_row_ptr_[fe + 1] - h_cut_row_ptr_[f] <= 65535))) {
             vals += cuts_.feature_nnz[fe];
             ++fe;
         }
-        for (int q = f; q < fe; ++q) feat_slot[q] = n_small;
-        SparseTask t{f, fe, fvb[f], fvb[fe], n_small++, -1};
+        for (int q = f; q < fe; ++q) feat_slot[q] = n_small, task_bin0[q] = h_cut_row_ptr_[f];
+        SparseTask t{f, fe, first[f], first[fe], n_small++, -1};
         tasks.push_back(t);
         f = fe;
     }
@@ -991,8 +1025,7 @@ void Trainer::build_sparse_tasks() {
         while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && (e == i || vals + cuts_.feature_nnz[rare_fid[e]] <= tile_values))
             vals += cuts_.feature_nnz[rare_fid[e++]];
         rare_tasks.push_back(RareTask{(int)places, (int)vals, (int)i, (int)(e - i)});
-        places += vals;
-        if (sp_.n_spread > 0) places = (places + (kSpreadGroup - 1) * std::min<long>(sp_.n_spread, vals) + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
+        places += sp_.n_spread > 0 ? places_of(vals) : vals;
         i = e;
     }
     // as few rounds of resident workgroups as the tasks per workgroup allow
@@ -1002,16 +1035,19 @@ void Trainer::build_sparse_tasks() {
     for (int t = 0; t < n_rt; ++t)
         for (int q = 0; q < rare_tasks[t].n_feat; ++q) feat_slot[rare_fid[rare_tasks[t].meta_begin + q]] = next_slot + t % n_groups;
     next_slot += n_groups;
-    // the biggest tasks first: they decide when the level is done
-    std::stable_sort(tasks.begin(), tasks.end(),
-                     [](const SparseTask &a, const SparseTask &b) { return a.v_end - a.v_begin > b.v_end - b.v_begin; });
+    // the longest tasks first: they decide when the level is done. A feature's search at deep levels takes about as long as adding up
+    // 16 000 values (a chunk has none).
+    const auto length = [](const SparseTask &t) { return t.v_end - t.v_begin + (t.cand_slot >= 0 ? 16000 * (long)(t.f_end - t.f_begin) : 0); };
+    std::stable_sort(tasks.begin(), tasks.end(), [&](const SparseTask &a, const SparseTask &b) { return length(a) > length(b); });
     sp_.n_tasks = (int)tasks.size();
     sp_.n_big = (int)big.size();
     sp_.n_rare_tasks = n_rt;
     sp_.n_rare_groups = n_groups;
     sp_.n_rare = n_rare;
     sp_.n_rare_places = ((size_t)places + 15) / 16 * 16;
-    if (n_rt == 0) sp_.n_spread = 0;
+    sp_.n_table_features = (int)table_features.size();
+    sp_.n_table_places = ((size_t)table_places + 15) / 16 * 16;
+    sp_.n_lists = n_rt + sp_.n_table_features;
     sp_.n_cand_slots = std::max(1, next_slot);
     sp_.n_partial_slots = n_partial;
     sp_.partial_stride = (size_t)max_big_bins * (size_t)tb_.max_level_nodes;
@@ -1021,7 +1057,8 @@ void Trainer::build_sparse_tasks() {
     int *d_rare_fid = dalloc<int>(rare_fid.size());
     int2 *d_rare_meta = dalloc<int2>(rare_meta.size());
     int *d_feat_slot = dalloc<int>(feat_slot.size());
-    int *d_fvb = dalloc<int>(fvb.size());
+    int *d_fvb = dalloc<int>(fvb.size()), *d_first = dalloc<int>(first.size()), *d_table = dalloc<int>(table_features.size());
+    d_task_bin0_ = dalloc<int>(task_bin0.size());
     upload(stream_, d_tasks, tasks.data(), tasks.size());
     upload(stream_, d_big, big.data(), big.size());
     upload(stream_, d_rare, rare_tasks.data(), rare_tasks.size());
@@ -1029,6 +1066,9 @@ void Trainer::build_sparse_tasks() {
     upload(stream_, d_rare_meta, rare_meta.data(), rare_meta.size());
     upload(stream_, d_feat_slot, feat_slot.data(), feat_slot.size());
     upload(stream_, d_fvb, fvb.data(), fvb.size());
+    upload(stream_, d_first, first.data(), first.size());
+    upload(stream_, d_table, table_features.data(), table_features.size());
+    upload(stream_, d_task_bin0_, task_bin0.data(), task_bin0.size());
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
     sp_.tasks = d_tasks;
     sp_.big = d_big;
@@ -1036,6 +1076,8 @@ void Trainer::build_sparse_tasks() {
     sp_.rare_fid = d_rare_fid;
     sp_.rare_meta = d_rare_meta;
     sp_.feat_val_begin = d_fvb;
+    sp_.table_first = d_first;
+    sp_.table_features = d_table;
     tb_.feat_slot = d_feat_slot;
     log_info("sparse level pass: %d table tasks, %d features in chunks (%d chunks), %zu features (%ld values) in %d "
              "rare tasks, %d candidate slots per node", sp_.n_tasks, sp_.n_big, n_partial, rare_fid.size(), n_rare,
@@ -1130,8 +1172,13 @@ bool Trainer::update_with_partition(int level) const {
 
 void Trainer::build_level_hist(const TreeBuffers &tb, int level, const GHPair *gh, int n_class, bool sum_rows) {
     if (sparse_pass_) {
+        // (the words of level 0 are the tree's: the levels below read the copy that it leaves)
+        if (level == 0) sparse_words_ = gh_words_fresh_ && n_class == 1 && gh == d_gh_;
+        SparsePass sp = sp_;
+        sp.gh_words = sparse_words_ ? d_gh_words_ : nullptr;
+        sp.gh_objective = objective_;
         // histogram and split search of the level in one pass; stage-wise driving also gets the per-node histograms
-        launch_sparse_level(stream_, tb, csr_, sp_, gh, level, param_.min_child_weight, param_.lambda,
+        launch_sparse_level(stream_, tb, csr_, sp, gh, level, param_.min_child_weight, param_.lambda,
                             !in_boost_ && tb_.hist_q[0] != nullptr, n_class);
     } else if (sparse_)
         launch_hist_csr(stream_, tb, csr_, gh, level, n_class);
@@ -1154,7 +1201,7 @@ void Trainer::partition_sets(const TreeBuffers &tb, const GHPair *gh, int level,
     // the last level is not partitioned: its split nodes keep their rows until the tree's final pass
     if (level < param_.depth - 1) lookup_level_ = -1;
     if (sparse_pass_) {
-        launch_sparse_partition(stream_, tb, csr_, level, n_class);  // every level: the map is the only row state
+        launch_sparse_partition(stream_, tb, csr_, sp_, level, n_class);  // every level: the map is the only row state
         lookup_level_ = -1;
     } else if (sparse_)
         launch_partition_csr(stream_, tb, csr_, level, n_class);

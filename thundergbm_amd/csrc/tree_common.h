@@ -202,21 +202,6 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
     return out;
 }
 
-// A row's gradient pair from the word that travels in its record (word_from_row).
-__device__ __forceinline__ GHPair pair_from_word(int objective, unsigned w) {
-    GHPair o;
-    if (objective == OBJ_SQUARE) {
-        o.g = __uint_as_float(w);
-        o.h = 1.f;
-    } else {
-        const float s = __uint_as_float(w & 0x7fffffffu);
-        const float yi = (w >> 31) ? 1.f : 0.f;
-        o.g = s - yi;
-        o.h = fmaxf(s * (1.f - s), 1e-16f);
-    }
-    return o;
-}
-
 // What a lane's columns of a row (v: two bins of 16 bits or four of 8) add to their bins in LDS: exact products (the scales are
 // powers of two), rounded once to the nearest integer, the hessian's in the low h_bits.
 template <bool BIN16>

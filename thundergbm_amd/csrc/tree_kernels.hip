@@ -60,7 +60,7 @@ __global__ void k_gradient_pointwise(int objective, int n, const float *__restri
 // (launch_gh_words, k_tree_end); the root level's histogram launch, which streams every record anyway, reads them
 // there and writes the records back with the word in place - whole records, so that memory sees full-sector writes
 // (4 bytes of every 32 written by themselves cost a read-modify-write per sector: 90 us per tree on 10 M rows). Squared loss: the gradient itself (the hessian is 1). Logistic loss with 0/1 labels: the
-// sigmoid s (never negative) with the label in the sign bit; pair_from_word (tree_common.h) repeats pointwise_gradient's operations on
+// sigmoid s (never negative) with the label in the sign bit; pair_from_word (kernel_common.h) repeats pointwise_gradient's operations on
 // s, so both give the same bits.
 __device__ __forceinline__ unsigned word_from_row(int objective, float yi, float p) {
     if (objective == OBJ_SQUARE) return __float_as_uint(p - yi);
