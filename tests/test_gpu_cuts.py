@@ -53,3 +53,28 @@ def test_cut_points(n, F, filled, max_bin, dense):
     per = [np.clip(np.searchsorted(want[ptr[f]:ptr[f + 1]], X[:, f], side="right"), 0, max(ptr[f + 1] - ptr[f] - 1, 0)) + ptr[f] for f in range(F)]
     assert np.array_equal(ids, np.stack(per, 1)[r, c])
     s.close()
+
+
+# Dense cells of which some hold no value, sorted along with the values or not (at most a quarter of them on wide data, a 32nd else; 1024
+# rows), and bins by runs of features (16 384 cut points a run), against the same values as CSR.
+@pytest.mark.parametrize("n,F,filled,max_bin", [
+    (1023, 257, 0.99, 31), (1024, 257, 0.99, 31), (4096, 300, 0.76, 63), (4097, 300, 0.74, 63), (5000, 40, 0.98, 255), (5000, 40, 0.95, 255),
+    (3000, 130, 0.97, 255), (4100, 260, 0.9, 300), (2049, 64, 1.0, 255)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_cells_without_values(n, F, filled, max_bin, dtype):
+    import scipy.sparse as sp
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n + F)
+    X = rng.standard_normal((n, F)).astype(dtype)
+    X[:, ::3] = np.round(X[:, ::3] * 4) / 4
+    X[rng.random((n, F)) >= filled] = 0
+    X[:, F // 2] = 0
+    X[5, 3], X[6, 3], X[7, 4] = np.inf, -np.inf, -0.0
+    if dtype == np.float64:
+        X[8, 5] = 1e-60  # (stored, and zero as a float)
+    y = (X[:, 0] + np.abs(X[:, 1]) - X[:, F - 1]).astype(np.float32)
+    runs = []
+    for data in (X, sp.csr_matrix(X)):
+        m = T.TGBMRegressor(depth=4, n_trees=3, max_num_bin=max_bin, verbose=0).fit(data, y)
+        runs.append([{k: v.tobytes() for k, v in t.items()} for t in m.get_trees()] + [m.predict(data).tobytes()])
+    assert runs[0] == runs[1]

@@ -36,13 +36,14 @@ __device__ __forceinline__ float key_float(unsigned k) {
 // The tiles of all segments, numbered segment by segment.
 struct Segments {
     const unsigned *start;    // [F + 1] first value
+    const unsigned *end;      // [F] behind the last one
     const int *tile_begin;    // [F + 1] first tile
     int F, n_tiles;
 };
 struct Tile {
     int feature, index, of;  // the index-th of `of` tiles of its feature
     unsigned base;
-    int count;
+    int count;               // (0: behind the feature's last value, see k_transpose_cells)
 };
 __device__ __forceinline__ Tile find_tile(const Segments &sg, int tile) {
     int lo = 0, hi = sg.F;  // the last feature whose first tile is not behind (features without values have no tile)
@@ -55,7 +56,7 @@ __device__ __forceinline__ Tile find_tile(const Segments &sg, int tile) {
     t.index = tile - sg.tile_begin[lo];
     t.of = sg.tile_begin[lo + 1] - sg.tile_begin[lo];
     t.base = sg.start[lo] + (unsigned)t.index * kTile;
-    t.count = (int)min((unsigned)kTile, sg.start[lo + 1] - t.base);
+    t.count = (int)min((unsigned)kTile, max(sg.end[lo], t.base) - t.base);
     return t;
 }
 
@@ -72,6 +73,39 @@ __global__ __launch_bounds__(kBlock) void k_transpose_keys(int n, int C, const f
 #pragma unroll 4
     for (int c = w; c < 64; c += kWaves)
         if (r0 + lane < n && c0 + c < C) keys[(size_t)(c0 + c) * n + r0 + lane] = s[lane][c];
+}
+
+// The same for cells of which some hold no value (is_stored of dense_to_csr): their keys are the largest there are, which sorts them
+// behind the values. stored[f] += values of the feature.
+constexpr int kCellRows = 256;  // rows per workgroup
+constexpr unsigned kNoValue = ~0u;
+__global__ __launch_bounds__(kBlock) void k_transpose_cells(DenseCells cells, int F, unsigned *__restrict__ keys, unsigned *__restrict__ stored) {
+    __shared__ unsigned s[64][65];
+    __shared__ unsigned s_cnt[kWaves][64];
+    const int c0 = blockIdx.y * 64, lane = lane_id(), w = wave_id();
+    unsigned count = 0;
+    for (int r0 = blockIdx.x * kCellRows; r0 < min(cells.n, ((int)blockIdx.x + 1) * kCellRows); r0 += 64) {
+#pragma unroll 4
+        for (int r = w; r < 64; r += kWaves)
+            if (r0 + r < cells.n && c0 + lane < F) {
+                const float v = cells.x[(size_t)(r0 + r) * cells.columns + c0 + lane];
+                const bool in = v != 0.f || (cells.minus_zero_is_stored && __float_as_uint(v) != 0u);
+                count += in ? 1u : 0u;
+                s[r][lane] = in ? float_key(v) : kNoValue;
+            }
+        __syncthreads();
+#pragma unroll 4
+        for (int c = w; c < 64; c += kWaves)
+            if (r0 + lane < cells.n && c0 + c < F) keys[(size_t)(c0 + c) * cells.n + r0 + lane] = s[lane][c];
+        __syncthreads();
+    }
+    s_cnt[w][lane] = count;
+    __syncthreads();
+    if (w == 0 && c0 + lane < F) {
+#pragma unroll
+        for (int i = 1; i < kWaves; ++i) count += s_cnt[i][lane];
+        atomicAdd(&stored[c0 + lane], count);
+    }
 }
 
 // counts[feature * tiles + tile]: entries of the tile (a run of kTile CSR entries) in the feature's column.
@@ -262,6 +296,10 @@ __device__ __forceinline__ unsigned first_of_value(const Tile &t, const unsigned
 __global__ __launch_bounds__(kBlock) void k_distinct_count(Segments sg, const unsigned *__restrict__ keys, unsigned *__restrict__ counts) {
     __shared__ unsigned s[kWaves];
     const Tile t = find_tile(sg, blockIdx.x);
+    if (t.count == 0) {
+        if (threadIdx.x == 0) counts[blockIdx.x] = 0u;
+        return;
+    }
     unsigned k[kRounds];
     unsigned long long first[kRounds];
     const unsigned c = first_of_value(t, keys, k, first);
@@ -277,6 +315,7 @@ __global__ __launch_bounds__(kBlock) void k_distinct_emit(Segments sg, const uns
                                                          int max_bin, float *__restrict__ cut_val, int *__restrict__ cut_fid) {
     __shared__ unsigned s[kWaves];
     const Tile t = find_tile(sg, blockIdx.x);
+    if (t.count == 0) return;
     unsigned k[kRounds];
     unsigned long long first[kRounds];
     const unsigned c = first_of_value(t, keys, k, first);
@@ -303,16 +342,29 @@ __global__ __launch_bounds__(kBlock) void k_distinct_emit(Segments sg, const uns
 }  // namespace
 
 DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, bool full_rows,
-                                       int max_num_bin) {
+                                       int max_num_bin, const DenseCells *cells) {
     DeviceCuts out;
     const unsigned feature_grid = (unsigned)((F + kBlock) / kBlock);
     ScanScratch scratch;
     unsigned *keys[2] = {nullptr, nullptr}, *d_start = nullptr, *d_total = nullptr;
-    for (unsigned *&k : keys) device_alloc_to(k, sizeof(unsigned) * (size_t)nnz);
+    const size_t n_keys = cells != nullptr ? (size_t)cells->n * F : (size_t)nnz;
+    for (unsigned *&k : keys) device_alloc_to(k, sizeof(unsigned) * n_keys);
     device_alloc_to(d_start, sizeof(unsigned) * ((size_t)F + 1));
     device_alloc_to(d_total, sizeof(unsigned));
     std::vector<unsigned> start((size_t)F + 1);
-    if (full_rows) {
+    unsigned *d_stored = nullptr;  // behind the features' last values
+    std::vector<unsigned> stored;
+    if (cells != nullptr) {
+        device_alloc_to(d_stored, sizeof(unsigned) * (size_t)F);
+        HIP_CHECK(hipMemsetAsync(d_stored, 0, sizeof(unsigned) * (size_t)F, s));
+        for (int f = 0; f <= F; ++f) start[(size_t)f] = (unsigned)((long)f * cells->n);
+        k_transpose_cells<<<dim3((unsigned)((cells->n + kCellRows - 1) / kCellRows), (unsigned)((F + 63) / 64)), kBlock, 0, s>>>(*cells, F, keys[0],
+                                                                                                                       d_stored);
+        HIP_CHECK(hipMemcpyAsync(d_start, start.data(), sizeof(unsigned) * start.size(), hipMemcpyHostToDevice, s));
+        stored.resize((size_t)F);
+        HIP_CHECK(hipMemcpyAsync(stored.data(), d_stored, sizeof(unsigned) * stored.size(), hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipStreamSynchronize(s));
+    } else if (full_rows) {
         const long n = nnz / F;
         for (int f = 0; f <= F; ++f) start[(size_t)f] = (unsigned)(f * n);
         k_transpose_keys<<<dim3((unsigned)((n + 63) / 64), (unsigned)((F + 63) / 64)), kBlock, 0, s>>>((int)n, F, d_val, keys[0]);
@@ -334,8 +386,9 @@ DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const flo
     out.feature_nnz.resize((size_t)F);
     std::vector<int> tile_begin((size_t)F + 1, 0);
     for (int f = 0; f < F; ++f) {
-        out.feature_nnz[(size_t)f] = (long)(start[(size_t)f + 1] - start[(size_t)f]);
-        tile_begin[(size_t)f + 1] = tile_begin[(size_t)f] + (int)((out.feature_nnz[(size_t)f] + kTile - 1) / kTile);
+        const long keys_of = (long)(start[(size_t)f + 1] - start[(size_t)f]);
+        out.feature_nnz[(size_t)f] = cells != nullptr ? (long)stored[(size_t)f] : keys_of;
+        tile_begin[(size_t)f + 1] = tile_begin[(size_t)f] + (int)((keys_of + kTile - 1) / kTile);
     }
     const int n_tiles = tile_begin[(size_t)F];
     int *d_tile_begin = nullptr;
@@ -344,17 +397,22 @@ DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const flo
     device_alloc_to(counts, sizeof(unsigned) * 256 * (size_t)n_tiles);
     device_alloc_to(offsets, sizeof(unsigned) * 256 * (size_t)n_tiles);
     HIP_CHECK(hipMemcpyAsync(d_tile_begin, tile_begin.data(), sizeof(int) * tile_begin.size(), hipMemcpyHostToDevice, s));
-    const Segments sg{d_start, d_tile_begin, F, n_tiles};
+    Segments sg{d_start, d_start + 1, d_tile_begin, F, n_tiles};
     int cur = 0;
     for (int shift = 0; shift < 32; shift += 8, cur ^= 1) {
         k_segment_count<<<(unsigned)n_tiles, kBlock, 0, s>>>(sg, keys[cur], shift, counts);
         device_exclusive_scan(s, counts, offsets, 256l * n_tiles, d_total, scratch);
         k_segment_scatter<<<(unsigned)n_tiles, kBlock, 0, s>>>(sg, keys[cur], keys[cur ^ 1], shift, offsets);
     }
+    if (cells != nullptr) {  // (the empty cells lie behind the values now)
+        for (int f = 0; f < F; ++f) stored[(size_t)f] += start[(size_t)f];
+        HIP_CHECK(hipMemcpyAsync(d_stored, stored.data(), sizeof(unsigned) * stored.size(), hipMemcpyHostToDevice, s));
+        sg.end = d_stored;
+    }
     k_distinct_count<<<(unsigned)n_tiles, kBlock, 0, s>>>(sg, keys[cur], counts);
     device_exclusive_scan(s, counts, offsets, n_tiles, d_total, scratch);
     unsigned *d_ustart = keys[cur ^ 1];  // (free by now, and at least one value long)
-    if ((long)F + 1 > nnz) device_alloc_to(d_ustart, sizeof(unsigned) * ((size_t)F + 1));
+    if ((size_t)F + 1 > n_keys) device_alloc_to(d_ustart, sizeof(unsigned) * ((size_t)F + 1));
     k_pick_starts<<<feature_grid, kBlock, 0, s>>>(F, offsets, 0, d_tile_begin, n_tiles, d_total, d_ustart);
     std::vector<unsigned> ustart((size_t)F + 1);
     HIP_CHECK(hipMemcpyAsync(ustart.data(), d_ustart, sizeof(unsigned) * ustart.size(), hipMemcpyDeviceToHost, s));
@@ -377,6 +435,7 @@ DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const flo
     if (d_ustart != keys[cur ^ 1]) device_free(d_ustart);
     for (unsigned *k : keys) device_free(k);
     device_free(d_start);
+    if (d_stored != nullptr) device_free(d_stored);
     device_free(d_total);
     device_free(d_tile_begin);
     device_free(counts);

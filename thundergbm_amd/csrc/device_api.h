@@ -605,7 +605,11 @@ void launch_fill_u8(hipStream_t s, uint8_t *p, uint8_t v, size_t n);
 void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, const float *val, const float *cut_val,
                       const int *cut_row_ptr, uint8_t *binmat, int W, size_t block_stride, uint8_t *colmat,
                       size_t col_stride, int bin_bytes, int F, const int *feat_col,
-                      const uint8_t *feat_lo, bool rows_ascend, int n_features, int n_bins);
+                      const uint8_t *feat_lo, bool rows_ascend, int n_features, int n_bins, const int *group_first = nullptr,
+                      int n_groups = 0);
+// Runs of features whose cut points a workgroup of launch_bin_dense has room for: the first one of each, and the end (group_first, on the
+// device, and the number of runs); empty: a feature has too many.
+std::vector<int> bin_groups(const std::vector<int> &cut_row_ptr);
 // false when some row holds a column index below its predecessor's
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col);
 // min_next[c] (pre-filled with INT_MAX) = smallest column index that follows column c in a row (equal neighbours, a
@@ -622,12 +626,18 @@ struct DeviceCuts {
     int n_bins = 0;
     std::vector<long> feature_nnz;  // host: stored values per feature
 };
-// full_rows: every row stores every column, in order (d_val is a row-major matrix)
+// full_rows: every row stores every column, in order (d_val is a row-major matrix). cells: the matrix that the values come from, if it
+// is still there
+struct DenseCells {
+    const float *x;
+    int n, columns;
+    bool minus_zero_is_stored;
+};
 DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin,
-                            bool full_rows = false);
-// (at most 256 features, or full rows)
+                            bool full_rows = false, const DenseCells *cells = nullptr);
+// (at most 256 features, full rows, or the cells)
 DeviceCuts build_cut_points_by_feature(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, bool full_rows,
-                                       int max_num_bin);
+                                       int max_num_bin, const DenseCells *cells = nullptr);
 
 // Tile sums of the device-wide exclusive scan, one pair of arrays per recursion level (grown on demand).
 struct ScanScratch {
@@ -746,9 +756,11 @@ struct DeviceCsr {
     int *row_ptr = nullptr;
     long nnz = 0;
     int n_features = 1;  // largest column with a stored value + 1, at least 1
+    float *cells = nullptr;  // see dense_to_csr
 };
-// Takes `x` over (it becomes the value array when every cell is stored, and is freed otherwise). Synchronises.
-DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored);
+// Takes `x` over: it becomes the value array when every cell is stored, else it is freed, or (keep) handed back as `cells`.
+// Synchronises.
+DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored, bool keep = false);
 
 // Prediction of the n rows that row_ptr addresses (entry offsets into col / val); out[t * out_stride + i] for
 // class tree t and row i, out_stride = 0 means n (a slice of a larger row set passes the whole set's size); adds to out.

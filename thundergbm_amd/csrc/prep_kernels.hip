@@ -380,6 +380,55 @@ __global__ __launch_bounds__(kBinBlock) void k_bin_dense_lds(int n, int F, const
     }
 }
 
+// The same for more cut points than the LDS holds: a workgroup bins the features [first[g], first[g + 1]) of its rows, whose cut points
+// fit it. Sixteen lanes look for the first of them in the row, sixteen places a step. 27 M values of 136 features 542 -> 197 us, 35 M of
+// 700 825 -> 260, where every step of a value's search was a trip to a cache.
+template <typename BinT>
+__global__ __launch_bounds__(kBinBlock) void k_bin_dense_groups(int n, const int *__restrict__ first, const int *__restrict__ row_ptr,
+                                                               const int *__restrict__ col, const float *__restrict__ val,
+                                                               const float *__restrict__ cut_val, const int *__restrict__ cut_row_ptr,
+                                                               BinT *__restrict__ binmat, int W, size_t block_stride,
+                                                               const int *__restrict__ feat_col, const uint8_t *__restrict__ feat_lo) {
+    extern __shared__ float s_cut[];  // the cut points, then the features' ranges
+    const int f0 = first[blockIdx.y], f1 = first[blockIdx.y + 1];
+    const int base = cut_row_ptr[f0], n_bins = cut_row_ptr[f1] - base;
+    int *s_ptr = reinterpret_cast<int *>(s_cut + n_bins);
+    for (int i = threadIdx.x; i < n_bins; i += kBinBlock) s_cut[i] = cut_val[base + i];
+    for (int i = threadIdx.x; i <= f1 - f0; i += kBinBlock) s_ptr[i] = cut_row_ptr[f0 + i] - base;
+    __syncthreads();
+    constexpr int kLanes = 16;
+    const int sub = threadIdx.x % kLanes, group = (threadIdx.x & 63) / kLanes * kLanes;
+    // (all lanes of a wavefront go through the same rounds: the search asks them all)
+    for (int i0 = blockIdx.x * (kBinBlock / kLanes); i0 < n; i0 += gridDim.x * (kBinBlock / kLanes)) {
+        const int i = min(i0 + (int)threadIdx.x / kLanes, n - 1);
+        const int e1 = row_ptr[i + 1];
+        int lo = row_ptr[i], hi = e1;  // the first entry of the features from f0 on
+        while (__any(lo < hi)) {
+            const int step = (hi - lo + kLanes - 1) / kLanes, at = lo + sub * step;
+            const bool below = at < hi && col[at] < f0;
+            const int c = __popc((unsigned)(__ballot(below) >> group) & 0xffffu);
+            if (lo < hi) {
+                hi = min(hi, lo + c * step);
+                lo = c == 0 ? lo : lo + (c - 1) * step + 1;
+            }
+        }
+        if (i0 + (int)threadIdx.x / kLanes >= n) continue;
+        for (int e = lo + sub; e < e1; e += kLanes) {
+            const int f = col[e];
+            if (f >= f1) break;
+            const float v = val[e];
+            if (e + 1 < e1 && col[e + 1] == f) continue;
+            const int cb = s_ptr[f - f0];
+            int c = f, b = local_bin(s_cut + cb, s_ptr[f - f0 + 1] - cb, v);
+            if (feat_col != nullptr) {
+                c = feat_col[f];
+                b += feat_lo[f];
+            }
+            binmat[(size_t)(c / W) * block_stride + (size_t)i * W + (c % W)] = (BinT)b;
+        }
+    }
+}
+
 // The same for data with rows whose columns do not ascend (nothing the reference's wrappers produce: they sort the
 // indices of every row, thundergbm.py:103): a row may then store a column twice with other entries in between, and
 // sixteen lanes writing one cell would leave whichever bin arrived last. One thread walks its row front to back, so
@@ -529,7 +578,13 @@ int grid_for(size_t n, int cap = 8192) {
 // Sorted by feature (cut_kernels.hip) where one radix step of 8 bits, or a transposition, makes the features' segments and the
 // segments fill a quarter of their tiles; the rest by (feature, value) pairs.
 DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin,
-                            bool full_rows) {
+                            bool full_rows, const DenseCells *cells) {
+    // Sorting the cells that hold no value along costs less than grouping the values: on wide data, where they would be sorted as
+    // 64-bit pairs, up to a quarter of the cells, else up to a 32nd (all passes: 35 M cells of 700 features 1.9 -> 0.95 ms).
+    if (cells != nullptr && nnz > 0 && cells->n >= 1024) {
+        const long all = (long)cells->n * F, empty = all - nnz;
+        if (empty <= all / (F > 256 ? 4 : 32)) return build_cut_points_by_feature(s, F, nnz, d_val, d_col, full_rows, max_num_bin, cells);
+    }
     if (nnz > 0 && (F <= 256 || (full_rows && nnz / F >= 1024))) return build_cut_points_by_feature(s, F, nnz, d_val, d_col, full_rows, max_num_bin);
     DeviceCuts out;
     device_alloc_to(out.cut_row_ptr, sizeof(int) * (size_t)(F + 1));
@@ -651,13 +706,15 @@ int device_max_int(hipStream_t s, const int *d_v, long n) {
 // ---- dense input -----------------------------------------------------------------------------------
 // Streaming passes over the matrix, sixteen lanes per row as in the binning kernels (a row of 28 floats is two
 // lines): 140 MB take 60 us to count and 130 us to rewrite, next to 2.4 ms for their way over PCIe.
-__device__ __forceinline__ bool is_stored(float v, bool minus_zero_is_stored) {
+__device__ __forceinline__ bool is_stored(float v, bool minus_zero_is_stored) {  // (cut_kernels.hip has it too)
     return v != 0.f || (minus_zero_is_stored && __float_as_uint(v) != 0u);
 }
 
 // Stored values per row, and the last column that holds one.
+// (one atomic per workgroup, and 1024 of them: all to one word, a wavefront's each took 200 us whatever the rows)
 __global__ __launch_bounds__(kBlock) void k_dense_count(int n, int C, const float *__restrict__ x, bool mz,
                                                        unsigned *__restrict__ count, int *__restrict__ last_col) {
+    __shared__ int s_last[kWaves];
     constexpr int kLanes = 16;
     const int sub = threadIdx.x % kLanes;
     int last = 0;
@@ -675,7 +732,12 @@ __global__ __launch_bounds__(kBlock) void k_dense_count(int n, int C, const floa
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) last = max(last, __shfl_xor(last, d));
-    if ((threadIdx.x & 63) == 0 && last > *last_col) atomicMax(last_col, last);  // (the plain read spares most atomics)
+    if ((threadIdx.x & 63) == 0) s_last[threadIdx.x / 64] = last;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) last = max(last, s_last[w]);
+    if (last > *last_col) atomicMax(last_col, last);  // (the plain read spares most atomics)
 }
 
 __global__ __launch_bounds__(kBlock) void k_dense_compact(int n, int C, const float *__restrict__ x, bool mz,
@@ -709,7 +771,7 @@ __global__ __launch_bounds__(kBlock) void k_full_csr(int n, int C, int *__restri
     for (int i = blockIdx.x * kBlock + threadIdx.x; i <= n; i += gridDim.x * kBlock) row_ptr[i] = i * C;
 }
 
-DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz) {
+DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz, bool keep) {
     DeviceCsr out;
     const size_t cells = (size_t)n * C;
     TGBM_CHECK(n > 0 && C > 0 && cells < ((size_t)1 << 32), "dense input of %d x %d", n, C);
@@ -719,7 +781,7 @@ DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz) {
     device_alloc_to(out.row_ptr, sizeof(int) * ((size_t)n + 1));
     HIP_CHECK(hipMemsetAsync(result, 0, 2 * sizeof(unsigned), s));
     const int grid = grid_for((size_t)n * 16, 8192);
-    k_dense_count<<<grid, kBlock, 0, s>>>(n, C, x, mz, count, reinterpret_cast<int *>(result + 1));
+    k_dense_count<<<std::min(grid, 1024), kBlock, 0, s>>>(n, C, x, mz, count, reinterpret_cast<int *>(result + 1));
     ScanScratch scratch;
     exclusive_scan<false>(s, count, reinterpret_cast<unsigned *>(out.row_ptr), n, result, scratch);
     HIP_CHECK(hipMemcpyAsync(out.row_ptr + n, result, sizeof(unsigned), hipMemcpyDeviceToDevice, s));
@@ -739,8 +801,12 @@ DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz) {
     } else {
         device_alloc_to(out.val, sizeof(float) * (size_t)std::max(out.nnz, 1l));
         k_dense_compact<<<grid, kBlock, 0, s>>>(n, C, x, mz, out.row_ptr, out.val, out.col);
-        HIP_CHECK(hipStreamSynchronize(s));
-        device_free(x);
+        if (keep) {
+            out.cells = x;
+        } else {
+            HIP_CHECK(hipStreamSynchronize(s));
+            device_free(x);
+        }
     }
     return out;
 }
@@ -898,7 +964,7 @@ int sort_pairs(hipStream_t s, PairSorter &ps, long n, int key_bits) {
 void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, const float *val, const float *cut_val,
                       const int *cut_row_ptr, uint8_t *binmat, int W, size_t block_stride, uint8_t *colmat,
                       size_t col_stride, int bin_bytes, int F, const int *feat_col, const uint8_t *feat_lo,
-                      bool rows_ascend, int n_features, int n_bins) {
+                      bool rows_ascend, int n_features, int n_bins, const int *group_first, int n_groups) {
     const int grid = grid_for((size_t)n * 16, 1 << 20);
     const size_t lds = sizeof(float) * (size_t)n_bins + sizeof(int) * ((size_t)n_features + 1);
     const int lds_grid = (int)std::min<long>(512, ((long)n * 16 + kBinBlock - 1) / kBinBlock);
@@ -917,6 +983,16 @@ void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, 
         else
             k_bin_dense_lds<uint8_t><<<lds_grid, kBinBlock, lds, s>>>(n, n_features, row_ptr, col, val, cut_val, cut_row_ptr, binmat,
                                                                    W, block_stride, feat_col, feat_lo);
+    } else if (n_groups > 0) {
+        const int rows = (int)std::min<long>(std::max(1, 512 / n_groups), ((long)n * 16 + kBinBlock - 1) / kBinBlock);
+        const dim3 groups((unsigned)rows, (unsigned)n_groups);
+        if (bin_bytes == 2)
+            k_bin_dense_groups<uint16_t><<<groups, kBinBlock, sizeof(float) * kBinLds, s>>>(n, group_first, row_ptr, col, val, cut_val, cut_row_ptr,
+                                                                                  reinterpret_cast<uint16_t *>(binmat), W,
+                                                                                  block_stride / 2, nullptr, nullptr);
+        else
+            k_bin_dense_groups<uint8_t><<<groups, kBinBlock, sizeof(float) * kBinLds, s>>>(n, group_first, row_ptr, col, val, cut_val, cut_row_ptr,
+                                                                                 binmat, W, block_stride, feat_col, feat_lo);
     } else if (bin_bytes == 2)
         k_bin_dense<uint16_t><<<grid, kBlock, 0, s>>>(n, row_ptr, col, val, cut_val, cut_row_ptr,
                                                      reinterpret_cast<uint16_t *>(binmat), W, block_stride / 2, nullptr,
@@ -925,6 +1001,18 @@ void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, 
         k_bin_dense<uint8_t><<<grid, kBlock, 0, s>>>(n, row_ptr, col, val, cut_val, cut_row_ptr, binmat, W, block_stride,
                                                     feat_col, feat_lo);
     launch_cols_from_rows(s, n, W, F, (F + W - 1) / W, binmat, block_stride, colmat, col_stride, bin_bytes);
+}
+
+std::vector<int> bin_groups(const std::vector<int> &cut_row_ptr) {
+    std::vector<int> first{0};
+    const int F = (int)cut_row_ptr.size() - 1;
+    for (int f = 0; f < F; ++f) {
+        const int cuts = cut_row_ptr[(size_t)f + 1] - cut_row_ptr[(size_t)first.back()];
+        if (f > first.back() && cuts + (f + 1 - first.back()) + 1 > kBinLds) first.push_back(f);
+        if (cut_row_ptr[(size_t)f + 1] - cut_row_ptr[(size_t)f] + 2 > kBinLds) return {};
+    }
+    first.push_back(F);
+    return first;
 }
 
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col) {

@@ -46,17 +46,19 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     int *d_col = nullptr, *d_row_ptr = nullptr;
     auto t_up = std::chrono::steady_clock::now();
     bool rows_ascend = true, ascend_known = false;
+    DenseCells cells{nullptr, n_, 0, false};
     UploadSet up;  // the labels last: the host threads that group them start with the upload
     d_y_ = dalloc<float>(n_);
     up.add_late(d_y_, sizeof(float) * (size_t)n_, [&ds] { return ds.labels_when_ready(); });
     if (ds.is_dense()) {
-        const size_t cells = (size_t)n_ * ds.dense_columns;
+        const size_t n_cells = (size_t)n_ * ds.dense_columns;
         float *d_x = nullptr;
-        device_alloc_to(d_x, sizeof(float) * cells);
-        if (ds.dense_f64 != nullptr) up.add_doubles(d_x, ds.dense_f64, cells);
-        else up.add(d_x, ds.dense_f32, sizeof(float) * cells);
+        device_alloc_to(d_x, sizeof(float) * n_cells);
+        if (ds.dense_f64 != nullptr) up.add_doubles(d_x, ds.dense_f64, n_cells);
+        else up.add(d_x, ds.dense_f32, sizeof(float) * n_cells);
         up.send(stream_);
-        const DeviceCsr csr = dense_to_csr(stream_, n_, ds.dense_columns, d_x, ds.dense_f64 != nullptr);
+        const DeviceCsr csr = dense_to_csr(stream_, n_, ds.dense_columns, d_x, ds.dense_f64 != nullptr, true);
+        cells = DenseCells{csr.cells, n_, ds.dense_columns, ds.dense_f64 != nullptr};
         d_val = csr.val;
         d_col = csr.col;
         d_row_ptr = csr.row_ptr;
@@ -120,7 +122,9 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     }
     log_info("Fast getting cut points...");
     auto t_cut = std::chrono::steady_clock::now();
-    cuts_ = build_cut_points(stream_, F_, nnz_, d_val, d_col, param_.max_num_bin, ds.is_dense() && nnz_ == (long)n_ * ds.dense_columns);
+    cuts_ = build_cut_points(stream_, F_, nnz_, d_val, d_col, param_.max_num_bin, ds.is_dense() && nnz_ == (long)n_ * ds.dense_columns,
+                             cells.x != nullptr ? &cells : nullptr);
+    if (cells.x != nullptr) device_free(const_cast<float *>(cells.x));
     log_debug("cut points: %.3f s", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_cut).count());
     auto t_bin = std::chrono::steady_clock::now();
     n_bins_ = cuts_.n_bins;
@@ -415,8 +419,15 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         // (rows that store every feature cannot hold a column twice)
         if (!ascend_known && nnz_ != (long)n_ * F_) rows_ascend = device_rows_ascend(stream_, n_, d_row_ptr, d_col);
         if (!rows_ascend) log_info("rows with descending column indices: the dense bins are filled row by row");
+        const std::vector<int> groups = bin_groups(h_cut_row_ptr_);
+        int *d_groups = nullptr;
+        if (!groups.empty()) {
+            device_alloc_to(d_groups, sizeof(int) * groups.size());
+            upload(stream_, d_groups, groups.data(), groups.size());
+        }
         launch_bin_dense(stream_, n_, d_row_ptr, d_col, d_val, cuts_.cut_val, cuts_.cut_row_ptr, d_binmat_, W,
-                         bins_.block_stride, d_colmat, col_stride, bin_bytes, P, bins_.feat_col, bins_.feat_lo, rows_ascend, F_, n_bins_);
+                         bins_.block_stride, d_colmat, col_stride, bin_bytes, P, bins_.feat_col, bins_.feat_lo, rows_ascend, F_, n_bins_,
+                         d_groups, (int)groups.size() - 1);
         bins_.col = d_colmat;
         bins_.col_stride = col_stride;
         bins_.data = d_binmat_;
@@ -430,6 +441,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             }
         }
         HIP_CHECK(hipStreamSynchronize(stream_));
+        if (d_groups != nullptr) device_free(d_groups);
         device_free(d_val);
         device_free(d_col);
         device_free(d_row_ptr);
