@@ -145,6 +145,33 @@ def test_rank_full_size_parity(T, sort, monkeypatch):
         s.close()
 
 
+# The tables of short groups (one workgroup each: wavefronts of 64 positions, 2048 rows at most) against those that the host
+# makes for long ones: the same sums and metrics, bit for bit. "steps": many runs of one row, where every other one draws.
+@pytest.mark.parametrize("objective", ["rank:pairwise", "rank:ndcg"])
+@pytest.mark.parametrize("labels", ["few", "steps", "zeros"])
+@pytest.mark.parametrize("groups", [[2048], [1, 0, 63, 64, 65, 2, 0], [127, 128, 129, 1, 1, 257], [0, 1], [3] * 700])
+def test_rank_tables_of_short_groups(T, objective, labels, groups, monkeypatch):
+    rng = np.random.default_rng(len(groups) + len(labels))
+    n = sum(groups)
+    y = (rng.integers(0, 5, n) if labels == "few" else rng.permutation(n) % 31 if labels == "steps" else np.zeros(n)).astype(np.float32)
+    if objective == "rank:pairwise" and labels == "steps":
+        y = rng.permutation(n).astype(np.float32) - n // 2  # (all different, some negative)
+    y[y == 0] = np.where(rng.random((y == 0).sum()) < 0.5, -0.0, 0.0)
+    val, rp, col = D.dense_to_csr(rng.normal(size=(n, 2)).astype(np.float32))
+    score = np.round(rng.normal(size=n), 1).astype(np.float32)
+    got = []
+    for sort in ("radix", "counting"):
+        monkeypatch.setenv("TGBM_RANK_SORT", sort)
+        s = T.Session(val, rp, col, y, depth=2, n_trees=1, objective=objective, groups=groups)
+        s.set("y_pred", score)
+        _round_seed(5)
+        s.gradient()
+        got.append((s.gh(), s.get("rank_order", np.int32), s.metric()))
+        s.close()
+    assert np.array_equal(got[0][1], got[1][1])
+    assert np.array_equal(got[0][0], got[1][0]) and got[0][2] == got[1][2]
+
+
 def test_rank_gradient_is_bit_reproducible(T):
     (val, rp, col), y, groups = _ranking_case("many_groups")
     s = T.Session(val, rp, col, y, depth=4, n_trees=2, objective="rank:ndcg", groups=groups)

@@ -171,7 +171,7 @@ void log_the_metric(hipStream_t s, const GBMParam &param, const DataSet &ds, int
         for (int g : ds.group) covered += g;
         if (!ds.group.empty() && covered == (long)n && (int)ds.y.size() == n) {
             const bool ndcg = param.objective == "rank:ndcg";
-            RankContext rc(s, ds.y, ds.group, ndcg);
+            RankContext rc(s, ds.y, nullptr, ds.group, ndcg);
             float *d_m = nullptr;
             device_alloc_to(d_m, sizeof(float));
             rc.metric(ndcg ? RANK_METRIC_NDCG : RANK_METRIC_MAP, d_out, d_m);

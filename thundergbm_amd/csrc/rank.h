@@ -32,8 +32,9 @@ struct RankRun {
 
 class RankContext {
    public:
-    // y: labels of all rows; group: sizes of the query groups (consecutive rows), their sum must be y.size()
-    RankContext(hipStream_t s, const LabelVector &y, const std::vector<int> &group, bool ndcg);
+    // y: labels of all rows, d_y: the same on the device, where they outlive this object, or none; group: sizes of the query
+    // groups (consecutive rows), their sum must be y.size()
+    RankContext(hipStream_t s, const LabelVector &y, const float *d_y, const std::vector<int> &group, bool ndcg);
     ~RankContext();
     RankContext(const RankContext &) = delete;
     RankContext &operator=(const RankContext &) = delete;
@@ -52,15 +53,18 @@ class RankContext {
    private:
     template <typename T>
     T *dalloc(size_t count);
+    void upload(void *dst, const void *src, size_t bytes);
+    void setup_short_groups(int longest);
+    void setup_groups(const LabelVector &y, const std::vector<int> &gptr);
     hipStream_t stream_;
-    int n_ = 0, n_groups_ = 0, n_runs_ = 0;
+    int n_ = 0, n_groups_ = 0;
     bool ndcg_ = false;
     int run_bits_ = 0, group_bits_ = 0;
     int zero_hit_groups_ = 0;   // groups without a non-zero label: MAP = 1 by definition
     int ndcg_one_groups_ = 0;   // groups with IDCG == 0: NDCG = 1 by definition
     bool idcg_valid_ = false;   // all labels in 0..30
     std::vector<void *> allocs_;
-    float *d_y_ = nullptr;
+    const float *d_y_ = nullptr;
     int *d_static_row_ = nullptr;  // rows of every group by label descending (ties: row ascending)
     int *d_run_of_ = nullptr;      // run of a position of that order
     int *d_run_of_row_ = nullptr;  // run of a row

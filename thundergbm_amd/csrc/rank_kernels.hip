@@ -4,7 +4,7 @@
 // (src/thundergbm/objective/ranking_obj.cpp:20-96, src/thundergbm/metric/rank_metric.cpp:9-104). Here a
 // round is a handful of data-parallel passes over all rows:
 //   * labels never change, so the label-descending order of every group, its runs of equal labels and the
-//     part of each run that draws partners are tables built once on the host;
+//     part of each run that draws partners are tables built once (k_rank_setup; on the host where groups are long);
 //   * per round one stable radix sort of (run, descending score) keys orders the rows inside their runs,
 //     which reproduces "sort by score, then stably by label";
 //   * one thread per position draws its partner, evaluates the pair and adds the lambdas to both rows with
@@ -51,6 +51,105 @@ __device__ __forceinline__ float discounted_gain(int label, int rank) {
 // bits of the fixed-point fraction for a group of `len` rows: a row collects at most len + 1 lambdas of
 // magnitude <= 2, so sums stay below 2^62
 __device__ __forceinline__ int acc_bits(int len) { return 59 - (32 - __clz(max(len, 1))); }
+
+// The tables of a group whose rows one workgroup orders by counting: its rows by label descending, the runs of equal labels
+// (numbered by the position of the group's first row + the run's number in the group: ascending, with gaps), the positions that
+// draw partners, IDCG and the number of rows with a label. NaNs are ordered as their bits are, each a run of its own.
+// log2_of[i] = log2(i + 2) as the host has it: the terms of IDCG and their sum are its own, bit for bit.
+// Bound by the counting (len^2 steps of LDS a group). 200 003 rows in 1667 groups: 22 us, where eight threads of the host, the
+// copies of their tables and the look at the labels took 1.7 ms (a call of 40 rounds 20.5 -> 19.4 ms).
+constexpr int kSetupBlock = 128;
+__global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restrict__ y, const int *__restrict__ gptr,
+                                                            const float *__restrict__ log2_of, int longest, int *__restrict__ static_row,
+                                                            int *__restrict__ run_of, int *__restrict__ run_of_row,
+                                                            int *__restrict__ group_of, RankRun *__restrict__ runs,
+                                                            float *__restrict__ idcg, int *__restrict__ hits, int *__restrict__ counts) {
+    extern __shared__ unsigned s_mem[];
+    __shared__ int s_hits, s_bad, s_runs;
+    unsigned *s_key = s_mem;                                          // keys by row, then IDCG's terms by position
+    float *s_sorted = reinterpret_cast<float *>(s_key + longest);    // labels by position
+    unsigned short *s_at = reinterpret_cast<unsigned short *>(s_sorted + longest);  // position of a row
+    unsigned short *s_run = s_at + longest;                          // run of a position, within the group
+    unsigned short *s_first = s_run + longest;                       // first position of a run; the top bit: it draws no partner
+    const int g = blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
+    if (threadIdx.x == 0) s_hits = s_bad = s_runs = 0;
+    __syncthreads();
+    int nonzero = 0, bad = 0;
+    for (int i = threadIdx.x; i < len; i += kSetupBlock) {
+        const float v = y[b + i];
+        s_key[i] = float_key(v);
+        group_of[b + i] = g;
+        nonzero += v != 0.f ? 1 : 0;
+        bad |= v >= 0.f && v < 31.f ? 0 : 1;
+    }
+    if (nonzero) atomicAdd(&s_hits, nonzero);
+    if (bad) s_bad = 1;
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += kSetupBlock) {
+        const unsigned key = s_key[i];
+        int before = 0;
+        for (int j = 0; j < len; ++j) before += s_key[j] > key || (s_key[j] == key && j < i) ? 1 : 0;
+        s_at[i] = (unsigned short)before;
+        s_sorted[before] = y[b + i];
+        static_row[b + before] = b + i;
+    }
+    __syncthreads();
+    bad = s_bad;
+    for (int i = threadIdx.x; i < len; i += kSetupBlock) {
+        const float term = bad ? 0.f : (float)((1 << (int)s_sorted[i]) - 1) / log2_of[i];
+        s_key[i] = __float_as_uint(term);
+    }
+    if (threadIdx.x < 64) {  // the runs, by one wavefront
+        const int lane = threadIdx.x;
+        int n_runs = 0;
+        for (int base = 0; base < len; base += 64) {
+            const int i = base + lane;
+            const bool first = i < len && (i == 0 || s_sorted[i] != s_sorted[i - 1]);
+            const unsigned long long firsts = __ballot(first);
+            const int k = n_runs + __popcll(firsts & (~0ull >> (63 - lane))) - 1;
+            if (i < len) s_run[i] = (unsigned short)k;
+            if (first) s_first[k] = (unsigned short)i;
+            n_runs += __popcll(firsts);
+        }
+        if (lane == 0) s_runs = n_runs;
+    }
+    __syncthreads();
+    const int n_runs = s_runs;
+    if (threadIdx.x == 0) {  // a processed run makes the loop step over the next run's first position
+        bool skip = false;
+        int first = 0;
+        for (int k = 0; k < n_runs; ++k) {
+            const int end = k + 1 < n_runs ? s_first[k + 1] : len;
+            if (skip) s_first[k] = (unsigned short)(first | 0x8000);
+            skip = first + (skip ? 1 : 0) < end;
+            first = end;
+        }
+    }
+    if (threadIdx.x == 64) {
+        float z = 0.f;
+        for (int i = 0; i < len; ++i) z += __uint_as_float(s_key[i]);
+        idcg[g] = z;
+        hits[g] = s_hits;
+        if (s_bad) atomicOr(&counts[0], 1);
+        if (z == 0.f) atomicAdd(&counts[1], 1);
+        if (s_hits == 0) atomicAdd(&counts[2], 1);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < n_runs; k += kSetupBlock) {
+        RankRun r;
+        r.group_begin = b;
+        r.group_end = b + len;
+        r.begin = b + (s_first[k] & 0x7fff);
+        r.end = b + (k + 1 < n_runs ? s_first[k + 1] & 0x7fff : len);
+        r.first_l = min(r.end, r.begin + (s_first[k] >> 15));
+        r.group = g;
+        runs[b + k] = r;
+    }
+    for (int i = threadIdx.x; i < len; i += kSetupBlock) {
+        run_of[b + i] = b + s_run[i];
+        run_of_row[b + i] = b + s_run[s_at[i]];
+    }
+}
 
 int grid_for(size_t n) {
     size_t b = (n + kBlock - 1) / kBlock;
@@ -283,8 +382,8 @@ T *RankContext::dalloc(size_t count) {
     return static_cast<T *>(p);
 }
 
-RankContext::RankContext(hipStream_t s, const LabelVector &y, const std::vector<int> &group, bool ndcg)
-    : stream_(s), ndcg_(ndcg) {
+RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, const std::vector<int> &group, bool ndcg)
+    : stream_(s), ndcg_(ndcg), d_y_(d_y) {
     n_ = (int)y.size();
     n_groups_ = (int)group.size();
     TGBM_CHECK(n_groups_ > 0, "ranking needs query groups (a .group file or the group argument)");
@@ -296,10 +395,74 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const std::vector<
     }
     TGBM_CHECK(gptr.back() == n_, "query groups cover %d instances, the dataset has %d", gptr.back(), n_);
 
-    bool labels_ok = true;  // NDCG takes labels as small non-negative integers (1 << label)
-    for (float v : y) labels_ok = labels_ok && v >= 0.f && v < 31.f;
-    TGBM_CHECK(!ndcg || labels_ok, "rank:ndcg needs labels in 0..30");
+    // ordering by counting costs sum(len^2) steps (measured: 50 us for a million rows in groups of 120, where the radix
+    // sort takes 220 us): taken while the average row sits in a group of at most kRankCountSortMean rows
+    int longest = 0;
+    double steps = 0;
+    for (int g : group) {
+        longest = std::max(longest, g);
+        steps += (double)g * (double)g;
+    }
+    const char *sort_env = std::getenv("TGBM_RANK_SORT");  // "radix": the radix sort whatever the group sizes (tests)
+    short_groups_ = longest <= kRankCountSortMax && steps <= (double)kRankCountSortMean * (double)std::max(n_, 1) &&
+                    !(sort_env != nullptr && std::string(sort_env) == "radix");
+    group_bits_ = bits_for(n_groups_);
+    if (d_y_ == nullptr) {
+        float *own = dalloc<float>(n_);
+        upload(own, y.data(), sizeof(float) * (size_t)n_);
+        d_y_ = own;
+    }
+    d_static_row_ = dalloc<int>(n_);
+    d_run_of_ = dalloc<int>(n_);
+    d_run_of_row_ = dalloc<int>(n_);
+    d_group_of_ = dalloc<int>(n_);
+    d_gptr_ = dalloc<int>(gptr.size());
+    d_idcg_ = dalloc<float>(n_groups_);
+    d_group_hits_ = dalloc<int>(n_groups_);
+    d_acc_ = dalloc<long long>(2 * (size_t)n_);
+    d_flags_ = dalloc<unsigned>(n_);
+    d_hits_before_ = dalloc<unsigned>((size_t)n_ + 1);
+    n_partial_ = grid_for(n_);
+    d_partial_ = dalloc<double>(n_partial_);
+    upload(d_gptr_, gptr.data(), sizeof(int) * gptr.size());
+    HIP_CHECK(hipMemsetAsync(d_acc_, 0, sizeof(long long) * 2 * (size_t)std::max(n_, 1), stream_));
+    sorter_.alloc(n_);
+    if (short_groups_) setup_short_groups(longest);
+    else setup_groups(y, gptr);
+    TGBM_CHECK(!ndcg || idcg_valid_, "rank:ndcg needs labels in 0..30");  // (small non-negative integers: 1 << label)
+}
 
+void RankContext::upload(void *dst, const void *src, size_t bytes) {
+    if (bytes) HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream_));
+}
+
+void RankContext::setup_short_groups(int longest) {
+    d_runs_ = dalloc<RankRun>(n_);
+    run_bits_ = bits_for(n_);
+    std::vector<float> log2_of((size_t)longest);
+    for (int i = 0; i < longest; ++i) log2_of[i] = log2f((float)(i + 2));
+    float *d_log2 = dalloc<float>((size_t)longest);
+    upload(d_log2, log2_of.data(), sizeof(float) * (size_t)longest);
+    int *d_counts = dalloc<int>(3);
+    HIP_CHECK(hipMemsetAsync(d_counts, 0, sizeof(int) * 3, stream_));
+    static_assert(kRankCountSortMax <= 1 << 15, "positions of a group in 15 bits");
+    const size_t lds = (size_t)longest * (2 * sizeof(unsigned) + 3 * sizeof(unsigned short));
+    static_assert(kRankCountSortMax * 14 <= 48 << 10, "no opt-in for the LDS");
+    k_rank_setup<<<n_groups_, kSetupBlock, lds, stream_>>>(d_y_, d_gptr_, d_log2, longest, d_static_row_, d_run_of_, d_run_of_row_, d_group_of_,
+                                                           d_runs_, d_idcg_, d_group_hits_, d_counts);
+    HIP_CHECK(hipGetLastError());
+    int counts[3];
+    HIP_CHECK(hipMemcpyAsync(counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, stream_));
+    HIP_CHECK(hipStreamSynchronize(stream_));  // (and the host's arrays have been read)
+    idcg_valid_ = counts[0] == 0;
+    ndcg_one_groups_ = idcg_valid_ ? counts[1] : n_groups_;
+    zero_hit_groups_ = counts[2];
+}
+
+// Groups that the counting sort does not take are ordered on the host.
+void RankContext::setup_groups(const LabelVector &y, const std::vector<int> &gptr) {
+    bool labels_ok = true;
+    for (float v : y) labels_ok = labels_ok && v >= 0.f && v < 31.f;
     // The groups are independent: the threads take contiguous ranges of about equally many rows (one thread: 6.8 ms for
     // 200 k rows in groups of 120). Runs are numbered inside a range first, then moved behind the earlier ranges' runs.
     std::vector<int> static_row(n_), run_of(n_), run_of_row(n_), group_of(n_), hits(n_groups_, 0);
@@ -367,49 +530,15 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const std::vector<
         zero_hit_groups_ += range.zero_hit;
     }
     idcg_valid_ = labels_ok;
-    n_runs_ = (int)runs.size();
-    // ordering by counting costs sum(len^2) steps (measured: 50 us for a million rows in groups of 120, where the radix
-    // sort takes 220 us): taken while the average row sits in a group of at most kRankCountSortMean rows
-    int longest = 0;
-    double steps = 0;
-    for (int g : group) {
-        longest = std::max(longest, g);
-        steps += (double)g * (double)g;
-    }
-    const char *sort_env = std::getenv("TGBM_RANK_SORT");  // "radix": the radix sort whatever the group sizes (tests)
-    short_groups_ = longest <= kRankCountSortMax && steps <= (double)kRankCountSortMean * (double)std::max(n_, 1) &&
-                    !(sort_env != nullptr && std::string(sort_env) == "radix");
-    run_bits_ = bits_for(n_runs_);
-    group_bits_ = bits_for(n_groups_);
-
-    d_y_ = dalloc<float>(n_);
-    d_static_row_ = dalloc<int>(n_);
-    d_run_of_ = dalloc<int>(n_);
-    d_run_of_row_ = dalloc<int>(n_);
-    d_group_of_ = dalloc<int>(n_);
+    run_bits_ = bits_for((long)runs.size());
     d_runs_ = dalloc<RankRun>(runs.size());
-    d_gptr_ = dalloc<int>(gptr.size());
-    d_idcg_ = dalloc<float>(n_groups_);
-    d_group_hits_ = dalloc<int>(n_groups_);
-    d_acc_ = dalloc<long long>(2 * (size_t)n_);
-    d_flags_ = dalloc<unsigned>(n_);
-    d_hits_before_ = dalloc<unsigned>((size_t)n_ + 1);
-    n_partial_ = grid_for(n_);
-    d_partial_ = dalloc<double>(n_partial_);
-    auto up = [&](void *dst, const void *src, size_t bytes) {
-        if (bytes) HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream_));
-    };
-    up(d_y_, y.data(), sizeof(float) * (size_t)n_);
-    up(d_static_row_, static_row.data(), sizeof(int) * (size_t)n_);
-    up(d_run_of_, run_of.data(), sizeof(int) * (size_t)n_);
-    up(d_run_of_row_, run_of_row.data(), sizeof(int) * (size_t)n_);
-    up(d_group_of_, group_of.data(), sizeof(int) * (size_t)n_);
-    up(d_runs_, runs.data(), sizeof(RankRun) * runs.size());
-    up(d_gptr_, gptr.data(), sizeof(int) * gptr.size());
-    up(d_idcg_, idcg.data(), sizeof(float) * (size_t)n_groups_);
-    up(d_group_hits_, hits.data(), sizeof(int) * (size_t)n_groups_);
-    HIP_CHECK(hipMemsetAsync(d_acc_, 0, sizeof(long long) * 2 * (size_t)std::max(n_, 1), stream_));
-    sorter_.alloc(n_);
+    upload(d_static_row_, static_row.data(), sizeof(int) * (size_t)n_);
+    upload(d_run_of_, run_of.data(), sizeof(int) * (size_t)n_);
+    upload(d_run_of_row_, run_of_row.data(), sizeof(int) * (size_t)n_);
+    upload(d_group_of_, group_of.data(), sizeof(int) * (size_t)n_);
+    upload(d_runs_, runs.data(), sizeof(RankRun) * runs.size());
+    upload(d_idcg_, idcg.data(), sizeof(float) * (size_t)n_groups_);
+    upload(d_group_hits_, hits.data(), sizeof(int) * (size_t)n_groups_);
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
 }
 

@@ -458,7 +458,7 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
     launch_fill_f32(stream_, reinterpret_cast<float *>(d_gh_), 0.f, (size_t)param_.num_class * n_ * 2);
     alloc_tree_buffers();
 
-    if (objective_ == OBJ_RANK) rank_.reset(new RankContext(stream_, ds.y, ds.group, param_.objective == "rank:ndcg"));
+    if (objective_ == OBJ_RANK) rank_.reset(new RankContext(stream_, ds.y, d_y_, ds.group, param_.objective == "rank:ndcg"));
 
     // base score (regression_obj.h:35-53, :95-114; only for squared / logistic objectives)
     if (objective_ != OBJ_SOFTMAX && objective_ != OBJ_RANK) {
