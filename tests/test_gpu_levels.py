@@ -338,3 +338,27 @@ def test_root_of_drained_items(n, F, per_row, objective, monkeypatch):
         s.close()
     same = [[a == b for a, b in zip(o, out[-1])] for o in out[:-1]]
     assert np.all(same), same
+
+
+# Pairs that fill the fields of a packed bin (every row at the largest gradient of one sign, every hessian at the largest, all in one
+# bin), at the ends of what an item adds before it is drained (8192 rows with float hessians, 32 768 with whole ones), and one row.
+@pytest.mark.parametrize("n", [1, 2, 8191, 8192, 8193, 32769])
+@pytest.mark.parametrize("g,h", [(-0.7366291, 0.19483), (1.0, 0.2499999), (3.1e8, 1.0), (-1e-12, 1e-16), (5.0, 3.0)])
+def test_pairs_that_fill_their_fields(n, g, h):
+    import parity as P
+    import thundergbm_amd as T
+    X = np.ones((n, 2), np.float32)
+    X[:, 1] = np.arange(n) % 3 + 1
+    val, rp, col = D.dense_to_csr(X)
+    s = T.Session(val, rp, col, np.arange(n).astype(np.float32), depth=2, n_trees=1, objective="reg:linear")
+    gh = np.empty((n, 2), np.float32)
+    gh[:] = g, h
+    s.set("gh", gh)
+    s.tree_init(0)
+    s.find_split(0)
+    q = P.node_quantum(s.quant(), n, False)
+    got = s.level_hist(0)[0]
+    one = np.rint(gh[0].astype(np.float64) / q) * q
+    want = np.bincount(s.global_bin_ids(rp, col)[0], minlength=s.n_bins)[:, None] * one
+    assert np.array_equal(got, want)  # (the steps are powers of two and the sums integers below 2^53 of them)
+    s.close()

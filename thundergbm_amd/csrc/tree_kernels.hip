@@ -617,6 +617,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     // (a block is smaller than 4 GiB and has fewer than 2^29 rows - checked when the layout is chosen -, so a lane
     // addresses its dword, its gradient pair and its row id with an unsigned 32-bit offset from a uniform base)
     const uint8_t *blk = bins.data + (size_t)fb * bins.block_stride;
+    const char *words = reinterpret_cast<const char *>(bins.gh_words);
     const unsigned qoff = q * 4;
     long long accg[SLOTS], acch[SLOTS];
 #pragma unroll
@@ -642,7 +643,7 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
             opk[u] = *reinterpret_cast<const unsigned *>(blk + ((unsigned)r[u] * (unsigned)ROWB + qoff));
             if (!GHW) os[u] = *reinterpret_cast<const GHPair *>(reinterpret_cast<const char *>(gh) + (unsigned)r[u] * 8u);
             if (GHW && DIRECT)  // (the word travels in the pair's first slot)
-                os[u].g = __uint_as_float(*reinterpret_cast<const unsigned *>(reinterpret_cast<const char *>(bins.gh_words) + (unsigned)r[u] * 4u));
+                os[u].g = __uint_as_float(*reinterpret_cast<const unsigned *>(words + (unsigned)r[u] * 4u));
         }
     };
     constexpr int STEP = RPS * U;
@@ -690,9 +691,9 @@ void k_hist_dense(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
                 const unsigned w = __float_as_uint(s[u].g);
                 sv = pair_from_word(gh_objective, w);
                 // the record goes back with the word in its last dword (whole records: full-sector writes)
-                const int pos = base + rsub + u * RPS;
-                if (pos < end)
-                    *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(blk) + ((unsigned)pos * (unsigned)ROWB + qoff)) = word_lane ? w : pk[u];
+                // (positions past the end write the last row's again, as it is)
+                const int pos = min(base + rsub + u * RPS, end - 1);
+                *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(blk) + ((unsigned)pos * (unsigned)ROWB + qoff)) = word_lane ? w : pk[u];
             } else if constexpr (GHW) {
                 // the row's last lane holds the word: every lane of the row takes it from there
                 sv = pair_from_word(gh_objective, last_lane_of_row<LPR>(pk[u]));
