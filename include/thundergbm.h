@@ -89,6 +89,10 @@ void get_a_tree(tgbm_model **model, int tree_id, int n_nodes, int *children_left
                 int *children_default, int *features, float *thresholds, float *values,
                 float *node_sample_weights);
 
+/* The first n_trees trees like that, one behind the other in every array (get_n_nodes tells how long each is). */
+void tgbm_get_trees(tgbm_model **model, int n_trees, int *children_left, int *children_right, int *children_default, int *features,
+                    float *thresholds, float *values, float *node_sample_weights);
+
 /* scikit_tgbm.cpp:250-254. */
 void model_free(tgbm_model **model);
 

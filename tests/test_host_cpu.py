@@ -111,6 +111,14 @@ def test_model_file_round_trip(lib, tmp_path):
     assert arr["f"].tolist() == [0, 1, 2, -1, -1, -1, -1]
     np.testing.assert_allclose(val, [0, 0, 0, 0.3, 0.4, 0.5, 0.6], rtol=1e-6)
     np.testing.assert_allclose(w, 10 + np.arange(7))
+    for k in (3, 2, 0):  # all trees, the first of them, none
+        every = [np.full(7 * 3, 99, t) for t in [np.int32] * 4 + [np.float32] * 3]
+        lib.tgbm_get_trees(vp(C.byref(model)), k, *map(p, every))
+        for t in range(k):
+            one = [np.zeros(7, a.dtype) for a in every]
+            lib.get_a_tree(vp(C.byref(model)), t, 7, *map(p, one))
+            assert all(np.array_equal(a[7 * t:7 * t + 7], b) for a, b in zip(every, one))
+        assert all((a[7 * k:] == 99).all() for a in every)
     dst = tmp_path / "out.model"
     lab = np.array([-1.0, 1.0], np.float32)
     lib.save(str(dst).encode(), b"binary:logistic", 0.25, 2, 3, 1, vp(C.byref(model)), p(lab))

@@ -26,6 +26,7 @@ SIGNATURES = {
     "load_config": (None, [C.c_char_p, _P]),
     "get_n_nodes": (None, [_P, _P, C.c_int, C.c_int]),
     "get_a_tree": (None, [_P, C.c_int, C.c_int, _P, _P, _P, _P, _P, _P, _P]),
+    "tgbm_get_trees": (None, [_P, C.c_int, _P, _P, _P, _P, _P, _P, _P]),
     "model_free": (None, [_P]),
     "train_R": (None, [_P] * 18),
     "predict_R": (None, [_P] * 3),

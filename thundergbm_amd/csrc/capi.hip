@@ -134,6 +134,25 @@ int count_distinct(const float *v, int n) {
 
 }  // namespace
 
+// A tree as parallel arrays in heap order (scikit_tgbm.cpp:208-248).
+struct TreeArrays {
+    int *children_left, *children_right, *children_default, *features;
+    float *thresholds, *values, *node_sample_weights;
+};
+static void copy_tree(const Tree &tree, const TreeArrays &to) {
+    for (size_t i = 0; i < tree.nodes.size(); ++i) {
+        const TreeNode &nd = tree.nodes[i];
+        const int lch = nd.is_leaf ? -1 : nd.lch_index, rch = nd.is_leaf ? -1 : nd.rch_index;
+        to.children_left[i] = lch;
+        to.children_right[i] = rch;
+        to.children_default[i] = nd.default_right ? rch : lch;
+        to.values[i] = nd.is_leaf ? nd.base_weight : 0;
+        to.features[i] = nd.split_feature_id;
+        to.thresholds[i] = nd.split_value;
+        to.node_sample_weights[i] = nd.sum_gh_pair.h;
+    }
+}
+
 extern "C" {
 
 void set_logger(int verbose) { g_verbose = verbose; }
@@ -249,20 +268,20 @@ void get_a_tree(tgbm_model **model, int tree_id, int n_nodes, int *children_left
     TGBM_CHECK(tree_id >= 0 && (size_t)tree_id < m->trees.size(), "tree id %d out of range", tree_id);
     const Tree &tree = m->trees[(size_t)tree_id];
     TGBM_CHECK(n_nodes == (int)tree.nodes.size(), "n_nodes %d != %zu", n_nodes, tree.nodes.size());
-    for (int i = 0; i < n_nodes; ++i) {
-        const TreeNode &nd = tree.nodes[(size_t)i];
-        children_left[i] = nd.lch_index;
-        children_right[i] = nd.rch_index;
-        children_default[i] = nd.default_right ? nd.rch_index : nd.lch_index;
-        if (nd.is_leaf) {
-            children_left[i] = children_right[i] = children_default[i] = -1;
-            values[i] = nd.base_weight;
-        } else {
-            values[i] = 0;
-        }
-        features[i] = nd.split_feature_id;
-        thresholds[i] = nd.split_value;
-        node_sample_weights[i] = nd.sum_gh_pair.h;
+    copy_tree(tree, TreeArrays{children_left, children_right, children_default, features, thresholds, values, node_sample_weights});
+}
+
+void tgbm_get_trees(tgbm_model **model, int n_trees, int *children_left, int *children_right, int *children_default, int *features,
+                    float *thresholds, float *values, float *node_sample_weights) {
+    TGBM_CHECK(model != nullptr && *model != nullptr, "model is null!");
+    const tgbm_model *m = *model;
+    TGBM_CHECK(n_trees >= 0 && (size_t)n_trees <= m->trees.size(), "model holds %zu trees", m->trees.size());
+    size_t at = 0;
+    for (int t = 0; t < n_trees; ++t) {
+        const Tree &tree = m->trees[(size_t)t];
+        copy_tree(tree, TreeArrays{children_left + at, children_right + at, children_default + at, features + at, thresholds + at, values + at,
+                                   node_sample_weights + at});
+        at += tree.nodes.size();
     }
 }
 
