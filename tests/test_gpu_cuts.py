@@ -55,6 +55,16 @@ def test_cut_points(n, F, filled, max_bin, dense):
     s.close()
 
 
+# Segments that one workgroup sorts: 2, 4, 8 and 16 keys a thread, and the first ones that are too long for it; features that
+# share a value or none.
+@pytest.mark.parametrize("n,F,filled,max_bin", [
+    (2048, 3, 1.0, 255), (2049, 9, 1.0, 255), (2500, 119, 0.1, 255), (8192, 2, 1.0, 1024), (8193, 33, 0.99, 255), (16384, 5, 1.0, 63),
+    (16385, 5, 1.0, 63), (16500, 300, 0.98, 255), (64, 256, 0.4, 2), (65, 1, 1.0, 255)])
+@pytest.mark.parametrize("dense", [False, True])
+def test_cut_points_of_short_segments(n, F, filled, max_bin, dense):
+    test_cut_points(n, F, filled, max_bin, dense)
+
+
 # Dense cells of which some hold no value, sorted along with the values or not (at most a quarter of them on wide data, a 32nd else; 1024
 # rows), and bins by runs of features (16 384 cut points a run), against the same values as CSR.
 @pytest.mark.parametrize("n,F,filled,max_bin", [
