@@ -268,6 +268,14 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
                                             int b_begin, int b_end, GHPair S, double inv_g, double inv_h, float mcw, float lambda) {
 #pragma clang fp contract(off)
     const int lane = lane_id(), nb = b_end - b_begin, at = lane * 4;
+    // (read here, all of them: read where one of four is picked below, the record would be looked up by its index, in scratch memory)
+    unsigned word[4];
+    bool ignored[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        word[j] = pm.meta[j];
+        ignored[j] = pm.ignored[j];
+    }
     long long exg[4], exh[4];
     long long g = 0, h = 0;
 #pragma unroll
@@ -291,7 +299,7 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
         return GHPair{S.g - scaled_float(tg, inv_g), S.h - scaled_float(th, inv_h)};
     };
     GHPair m[4];
-    const bool one_feature = read_lane((int)(pm.meta[0] & 0xffu), 0) + 1 >= nb;
+    const bool one_feature = read_lane((int)(word[0] & 0xffu), 0) + 1 >= nb;
     if (one_feature) {
         m[0] = missing(allg, allh);
         m[1] = m[2] = m[3] = m[0];
@@ -302,7 +310,7 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             // (past the pack's end the words of its last bin repeat: clamped, nobody looks at the result)
-            const int head = max(0, at + j - (int)(pm.meta[j] >> 8 & 0xffu)), end = min(at + j + (int)(pm.meta[j] & 0xffu) + 1, nb);
+            const int head = max(0, at + j - (int)(word[j] >> 8 & 0xffu)), end = min(at + j + (int)(word[j] & 0xffu) + 1, nb);
             const longlong2 below = s_v[head], upto = s_v[min(end, kEvalPackBins - 1)];
             m[j] = missing((end == nb ? allg : upto.x) - below.x, (end == nb ? allh : upto.y) - below.y);
             exg[j] -= below.x;
@@ -318,7 +326,7 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
         const float gr = split_gain_select(S, fterm, left[j], mcw, lambda);
         const float gl = split_gain_select(S, fterm, GHPair{left[j].g + m[j].g, left[j].h + m[j].h}, mcw, lambda);
         score[j] = gl > gr ? gl : -gr;
-        score[j] = pm.ignored[j] ? 0.f : score[j];  // column sampling: hist_tree_builder_single.cu:304 / :663
+        score[j] = ignored[j] ? 0.f : score[j];  // column sampling: hist_tree_builder_single.cu:304 / :663
         const float a = at + j < nb ? fabsf(score[j]) : -1.f;
         which = a > best ? j : which;
         best = fmaxf(best, a);
@@ -329,7 +337,7 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
     const unsigned long long owners = __ballot(best == wave_max_f(best));
     if (active && lane == __ffsll((long long)owners) - 1) {
         const bool none = best < 0.f;
-        unsigned meta = pm.meta[0];
+        unsigned meta = word[0];
         SplitCand c;
         c.score = score[0];
         c.left = left[0];
@@ -340,7 +348,7 @@ __device__ __forceinline__ void search_pack(const TreeBuffers &tb, const PackMet
                 c.score = score[j];
                 c.left = left[j];
                 c.miss = m[j];
-                meta = pm.meta[j];
+                meta = word[j];
             }
         c.index = b_begin + at + which;
         c.feature = (int)(meta >> 16);
