@@ -219,12 +219,14 @@ __global__ __launch_bounds__(kBlock) void k_split_count(TreeBuffers tb_all, Dens
         const int pos = max(min(pb + k * kBlock + (int)threadIdx.x, pe - 1), 0);
         row[k] = DIRECT ? pos : ridx[pos];
     }
-    const TreeNode node = tb.nodes[x];
+    SplitCand early;
+    if (UPDATE) early = early_candidate(tb, x_in);
+    const TreeNode node = node_of_wave(tb, x);
     Picked best{};
     bool splits, dr = false;
     int f = 0, sbid = 0;
     if (UPDATE) {
-        best = pick_candidate<kWaves>(tb, x_in, node.is_valid, s_pick, early_candidate(tb, x_in));
+        best = pick_candidate<kWaves>(tb, x_in, node.is_valid, s_pick, early);
         splits = best.found && fabsf(best.c.score) > rt_eps;
         if (splits) {
             f = best.c.feature;
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(kBlock) void k_split_scatter(TreeBuffers tb_all, in
     const int pb = sg.x + mine * kPartChunk;
     const int pe = min(sg.y, pb + kPartChunk);
     const int lane = lane_id(), w = wave_id();
-    const TreeNode &nd = tb.nodes[x];
+    const TreeNode nd = node_of_wave(tb, x);
     const bool splits = node_splits(nd);
     const int lch = nd.lch_index, rch = nd.rch_index;
     // all loads of the item first (unconditional, clamped positions), then one barrier for the sums of the node's counts
@@ -535,7 +537,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_level(TreeBuffers tb_all,
     // (all that follows from the node alone is requested at once)
     const SplitCand early = early_candidate(tb, x_in);
     const int2 sg = level == 0 ? make_int2(0, tb.n) : tb.seg[x];
-    const TreeNode node = tb.nodes[x];
+    const TreeNode node = node_of_wave(tb, x);
     const QuantCtl quant = *tb.quant;
     constexpr int RPS = kSmallBlock / LPR, FPL = BIN16 ? 2 : 4, COLS = LPR * FPL, U = 8;
     const int q = threadIdx.x % LPR, rsub = threadIdx.x / LPR;
@@ -808,7 +810,7 @@ void k_split_hist(TreeBuffers tb_all, DenseBins bins, const GHPair *__restrict__
     const int pe = min(sg.y, pb + S * kPartChunk);
     const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     const int *__restrict__ ridx = tb.list(level);
-    const TreeNode &nd = tb.nodes[x];
+    const TreeNode nd = node_of_wave(tb, x);
     const bool splits = node_splits(nd);
     const int lch = nd.lch_index, rch = nd.rch_index;
     int row[R];
