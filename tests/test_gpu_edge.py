@@ -369,6 +369,30 @@ def test_column_sampling_matches_oracle(T, objective, kind, rate):
     s.close()
 
 
+@pytest.mark.parametrize("F", [1, 63, 64, 65, 4095, 4097, 65_536, 65_537])
+def test_sampled_columns_reach_the_device(T, F):
+    """The flags of a round's ignored columns against the same shuffle here, at the ends of a word, a launch and the columns whose
+    flags are copied."""
+    import ctypes
+    libc = ctypes.CDLL(None)
+    val, col = np.arange(1, F + 1, dtype=np.float32), np.arange(F, dtype=np.int32)
+    rp = np.array([0, F // 2, F], np.int32)
+    s = T.Session(val, rp, col, np.array([1, 2], np.float32), depth=1, n_trees=3, objective="reg:linear", max_num_bin=4)
+    s.set_option("column_sampling_rate", 0.3)
+    for seed in (7, 8, 9):
+        libc.srand(seed)
+        s.boost(1)
+        libc.srand(seed)
+        idx = list(range(F))
+        for i in range(1, F):
+            j = libc.rand() % (i + 1)
+            idx[i], idx[j] = idx[j], idx[i]
+        want = np.zeros(F, np.uint8)
+        want[idx[:max(1, int(np.float32(F) * np.float32(0.3)))]] = 1
+        assert np.array_equal(s.get("ignored", np.uint8), want)
+    s.close()
+
+
 @pytest.mark.parametrize("objective,kind,reorder", [("reg:linear", "reg", False), ("binary:logistic", "bin", False),
                                                     ("multi:softmax", "multi", False), ("reg:linear", "reg", True),
                                                     ("binary:logistic", "bin", True), ("multi:softmax", "multi", True)])

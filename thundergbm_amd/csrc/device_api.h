@@ -478,6 +478,12 @@ enum Objective { OBJ_SQUARE = 0, OBJ_LOGISTIC = 1, OBJ_SOFTMAX = 2, OBJ_RANK = 3
 
 void launch_gradient(hipStream_t s, int objective, int n, int num_class, const float *y, const float *yp, GHPair *gh,
                      GHPair *block_sums, int n_blocks);
+// flags[f] = the f-th bit of the caller's, which travel with the launches' arguments: nothing is copied and nobody waits.
+constexpr int kColumnFlagWords = 64;  // of a launch
+struct ColumnFlags {
+    unsigned long long bits[kColumnFlagWords];
+};
+void launch_column_flags(hipStream_t s, const std::vector<unsigned long long> &bits, int F, uint8_t *flags);
 // RowSampler::do_bagging over the N gradient pairs; `count` holds N zeroed ints and is left zeroed. perm (may
 // be null): original row of each of the n_rows physical positions; the N entries are planes of n_rows rows
 void launch_bagging(hipStream_t s, int N, unsigned seed, int *count, GHPair *gh, const int *perm = nullptr,

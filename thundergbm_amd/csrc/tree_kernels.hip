@@ -94,6 +94,14 @@ __global__ void k_gradient_softmax(int n, int K, const float *__restrict__ y, co
     }
 }
 
+// A wavefront per word of the flags.
+__global__ __launch_bounds__(kBlock) void k_column_flags(ColumnFlags in, int count, uint8_t *__restrict__ flags) {
+    const int word = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kWaves + wave_id());
+    if (word >= kColumnFlagWords) return;
+    const int f = word * 64 + lane_id();
+    if (f < count) flags[f] = (uint8_t)(in.bits[word] >> lane_id() & 1ull);
+}
+
 // Bagging, RowSampler::do_bagging (src/thundergbm/row_sampler.cu:9-38): entry i of the gradient array draws
 // idx_i from thrust::default_random_engine(seed) after discard(i) through
 // thrust::uniform_int_distribution<int>(0, N - 1); every gradient pair is multiplied by the number of draws
@@ -2556,6 +2564,17 @@ void launch_gradient(hipStream_t s, int objective, int n, int num_class, const f
 void launch_bagging(hipStream_t s, int N, unsigned seed, int *count, GHPair *gh, const int *perm, int n_rows) {
     k_bagging_draw<<<grid_for(N), kBlock, 0, s>>>(N, seed, count);
     k_bagging_apply<<<grid_for(N), kBlock, 0, s>>>(N, count, gh, perm, n_rows);
+}
+
+void launch_column_flags(hipStream_t s, const std::vector<unsigned long long> &bits, int F, uint8_t *flags) {
+    constexpr int kOf = kColumnFlagWords * 64;
+    for (int f0 = 0; f0 < F; f0 += kOf) {
+        const int count = std::min(kOf, F - f0), words = (count + 63) / 64;
+        ColumnFlags in;
+        for (int w = 0; w < words; ++w) in.bits[w] = bits[(size_t)(f0 / 64 + w)];
+        for (int w = words; w < kColumnFlagWords; ++w) in.bits[w] = 0;
+        k_column_flags<<<(unsigned)((words + kWaves - 1) / kWaves), kBlock, 0, s>>>(in, count, flags + f0);
+    }
 }
 
 // Launchers: `tb` is the first buffer set to use, `n_class` consecutive sets (class trees of one round)
