@@ -62,3 +62,20 @@ def test_sparse_rows_in_slices(n, F, far):
     assert np.allclose(whole, part, rtol=2e-6, atol=2e-6)
     if F > 96:
         assert whole.tobytes() == part.tobytes()
+
+
+# Several classes: the ends of k_score_group's range (65 536 rows through the classes), of the launches that share the classes out
+# (2048 workgroups of 256 rows) and of one slice (1024 workgroups through the classes), against k_score_group, which gives the same bits.
+@pytest.mark.parametrize("classes,n", [
+    (3, 21_845), (3, 21_846), (5, 13_108), (7, 9_363), (3, 174_762), (3, 174_763), (5, 209_716), (8, 66_000), (3, 262_144), (3, 524_289)])
+def test_classes_are_shared_out(classes, n, monkeypatch):
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 3)).astype(np.float32)
+    X[rng.random((n, 3)) < 0.1] = 0
+    y = rng.integers(0, classes, 2000)
+    m = T.TGBMClassifier(depth=4, n_trees=3, verbose=0, objective="multi:softprob").fit(X[:2000], y)
+    assert m.num_class == classes
+    got = np.asarray(m.predict(X))
+    monkeypatch.setenv("TGBM_PREDICT_GROUP", "1")
+    assert got.tobytes() == np.asarray(m.predict(X)).tobytes()

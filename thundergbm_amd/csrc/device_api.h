@@ -816,9 +816,13 @@ struct ScoreRows {
 // false: the rows' keys fit no kernel's LDS and nothing was launched.
 bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &model, bool narrow, float lr, float base_score,
                   float *out, size_t out_stride);
-// k_score_rows has room for the model's keys; it then serves kScoreGroupRows rows and more.
+int score_slice_rows(const ScoreModel &m);  // rows that fill the chip once, in a launch of their own
+int score_least_rows(const ScoreModel &m);  // the fewest that k_score_rows serves
+// k_score_rows has room for the model's keys; it then serves score_least_rows rows and more.
 bool score_rows_fit(const ScoreModel &model);
-// Below this many rows k_score_group takes them (see there).
+// Below this many rows k_score_group takes them (see there); with several classes, which k_score_rows shares out, below their part of
+// it: the same number of walks of one class. Whole calls with k_score_group and k_score_rows, us: 22 k x 28, 3 x 33 trees of depth 8
+// 225, 177; 13 200 rows, 5 x 20 169, 143; 30 k 299, 212; 8200 rows, 8 x 12 123, 113; 30 k one-hot rows, 6 x 15 310, 278.
 constexpr int kScoreGroupRows = 65536;
 void launch_predict_transform(hipStream_t s, int kind, int n, int num_class, const float *label, float *y);
 

@@ -229,10 +229,11 @@ __device__ __forceinline__ float add_leaf(float sum, float lr, float w) { return
 template <int B, int ILP, int kFetch, bool NARROW>
 __global__ __launch_bounds__(B) void k_score_rows(ScoreRows rows_in, ScoreModel m, float lr, float base_score,
                                                   float *__restrict__ out, size_t out_stride, int trees_per_stage,
-                                                  int coalesced_fill) {
+                                                  int coalesced_fill, int classes) {
     using Sum = typename std::conditional<NARROW, double, float>::type;
     extern __shared__ unsigned smem_u[];
-    const int n = rows_in.n, slots = m.n_slots, n_nodes = m.n_nodes, n_iter = m.n_iter, n_class_trees = m.n_class;
+    const int n = rows_in.n, slots = m.n_slots, n_nodes = m.n_nodes, n_iter = m.n_iter;
+    const int class0 = blockIdx.y * classes, class1 = min(m.n_class, class0 + classes);  // (one at least)
     unsigned *dense = smem_u;                                        // [slots][B] keys
     uint2 *nodes = reinterpret_cast<uint2 *>(smem_u + slots * B);    // [trees_per_stage][n_nodes]
     const int row0 = blockIdx.x * B;
@@ -334,8 +335,8 @@ __global__ __launch_bounds__(B) void k_score_rows(ScoreRows rows_in, ScoreModel 
 #pragma unroll
         for (int q = 0; q < kFetch; ++q) fetched[q] = src[min((int)threadIdx.x + q * B, count - 1)];
     };
-    if (prefetch) fetch(0, 0);
-    for (int t = 0; t < n_class_trees; ++t) {
+    if (prefetch) fetch(class0, 0);
+    for (int t = class0; t < class1; ++t) {
         Sum sum = base_score;
         for (int it0 = 0; it0 < n_iter; it0 += trees_per_stage) {
             const int staged = min(trees_per_stage, n_iter - it0);
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(B) void k_score_rows(ScoreRows rows_in, ScoreModel 
                 }
                 // the next stage: of this class, or the first of the next class
                 if (it0 + trees_per_stage < n_iter) fetch(t, it0 + trees_per_stage);
-                else if (t + 1 < n_class_trees) fetch(t + 1, 0);
+                else if (t + 1 < class1) fetch(t + 1, 0);
             } else {
                 const uint2 *src = m.records + ((size_t)t * n_iter + it0) * n_nodes;
                 for (int idx = threadIdx.x; idx < staged * n_nodes; idx += B) nodes[idx] = src[idx];
@@ -559,6 +560,14 @@ void launch_pack_model(hipStream_t s, const TreeNode *model, long n_total, int n
 // k_score_rows: 256 rows per workgroup while their vectors take at most 50 KB, else 128
 static int score_block(const ScoreModel &m) { return (size_t)m.n_slots * 256 * sizeof(float) <= 50 * 1024 ? 256 : 128; }
 
+constexpr int kScoreChip = 1024;  // workgroups of k_score_rows that the chip holds at a time
+
+int score_least_rows(const ScoreModel &m) { return (kScoreGroupRows + m.n_class - 1) / m.n_class; }
+
+int score_slice_rows(const ScoreModel &m) {
+    return (kScoreChip * score_block(m) + m.n_class - 1) / m.n_class;
+}
+
 bool score_rows_fit(const ScoreModel &m) {
     const size_t dense_bytes = (size_t)m.n_slots * score_block(m) * sizeof(float);
     return dense_bytes <= 50 * 1024 && dense_bytes + (size_t)m.n_nodes * sizeof(uint2) <= 64 * 1024;
@@ -585,7 +594,7 @@ bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, boo
     // few to fill the chip otherwise, and for wider ones.
     const int G = rows.n > 1024 && group_bytes(64) <= 40 * 1024 ? 64 : 256;
     const bool group_fits = group_bytes(G) <= 150 * 1024;
-    bool group = rows.n < kScoreGroupRows;
+    bool group = rows.n < score_least_rows(m);
     if (te != nullptr && atoi(te) > 0) group = false;
     if (ge != nullptr) group = atoi(ge) != 0;
     if (group_fits && (group || !rows_fit)) {
@@ -610,10 +619,14 @@ bool launch_score(hipStream_t s, const ScoreRows &rows, const ScoreModel &m, boo
     const size_t fit = (64 * 1024 - dense_bytes) / tree_bytes;  // (>= 1)
     const int tps = (int)std::max<size_t>(1, std::min<size_t>(te != nullptr && atoi(te) == 1 ? 1 : 2, fit));
     const size_t lds = dense_bytes + (size_t)tps * tree_bytes;
-    const int g = (rows.n + B - 1) / B;
+    // Classes are shared out as well where the rows alone make fewer workgroups than twice the chip's (each spreads
+    // its rows' keys again): 200 k x 28, 5 x 40 trees, in four launches side by side with the upload instead of one behind it.
+    const int row_groups = (rows.n + B - 1) / B, parts = std::min(m.n_class, (2 * kScoreChip + row_groups - 1) / row_groups);
+    const int classes = (m.n_class + parts - 1) / parts;
+    const dim3 g((unsigned)row_groups, (unsigned)((m.n_class + classes - 1) / classes));
     const int per_thread = (tps * m.n_nodes + B - 1) / B;  // records of a stage
 #define TGBM_SCORE_ROWS(BLK, ILP, FETCH, NN) \
-    k_score_rows<BLK, ILP, FETCH, NN><<<g, BLK, lds, s>>>(rows, m, lr, base_score, out, out_stride, tps, fill)
+    k_score_rows<BLK, ILP, FETCH, NN><<<g, BLK, lds, s>>>(rows, m, lr, base_score, out, out_stride, tps, fill, classes)
 #define TGBM_SCORE_FETCH(BLK, ILP, NN)                          \
     if (per_thread <= 2) TGBM_SCORE_ROWS(BLK, ILP, 2, NN);      \
     else if (per_thread <= 4) TGBM_SCORE_ROWS(BLK, ILP, 4, NN); \

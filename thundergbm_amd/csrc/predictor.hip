@@ -145,8 +145,10 @@ std::shared_ptr<const DeviceModel> device_model(hipStream_t s, tgbm_model &model
 // of 35 values, 100 trees: 5.4 ms in slices of 64 MB, 4.7 of 32, 4.4 of 16 with every slice a send of its own, 4.3 in one
 // send that has the columns in front). Where k_score_rows serves the call no slice has fewer rows than it is for, or the slice would
 // go to k_score_group, which is slower there (500 k rows of 40 values, 90 columns, 100 trees of depth 8: 4.6 ms in eighths, 3.5
-// with at least kScoreGroupRows rows each, and the same in slices of 24 or 64 MB). Dense rows: k_score_rows needs many workgroups, slices below 64 MB cost more than they hide
-// (200 k x 28, 200 trees: 203 us in one launch, 147 for 75 k of the rows).
+// with at least kScoreGroupRows rows each, and the same in slices of 24 or 64 MB). Dense rows: up to
+// kDenseSlices slices that fill the chip once each (200 k x 28, 5 x 40
+// trees of depth 8: 1.19 -> 1.08 ms; 600 k x 28, 100 trees of depth 6: 1.99 -> 1.95).
+constexpr int kDenseSlices = 4;
 constexpr size_t kLeastSlice = (size_t)8 << 20, kMostSlice = (size_t)64 << 20;
 
 // The reference takes its shared-memory path - double sums, +inf is missing - when a row's dense vector of as many
@@ -348,7 +350,11 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
                                          : !stores_beyond(ds.dense_f32, n, ds.dense_columns, kNarrowFeatures);
         device_alloc_to(d_x, sizeof(float) * (size_t)n * ds.dense_columns);
         const size_t row_bytes = 4 * (size_t)ds.dense_columns;
-        const int step = usable ? (int)std::max<size_t>(1, kMostSlice / row_bytes) : n;
+        int step = n;
+        if (usable) {
+            if (score_rows_fit(dm->m)) step = (n - 1) / std::max(1, std::min(kDenseSlices, n / score_slice_rows(dm->m))) + 1;
+            step = (int)std::max<size_t>(1, std::min((size_t)step, kMostSlice / row_bytes));
+        }
         done = usable;
         for (int r0 = 0; r0 < n; r0 += std::min(step, n - r0)) {
             const size_t off = (size_t)r0 * ds.dense_columns;
@@ -374,7 +380,7 @@ void score(const GBMParam &param, tgbm_model &model, int n_iter, int n_class, co
         const long slice_entries = usable ? (long)(std::min(std::max(eighth, kLeastSlice), kMostSlice) / sizeof(float)) : nnz;
         rows.col = d_col;
         rows.val = d_val;
-        const bool by_rows = usable && n >= kScoreGroupRows && score_rows_fit(dm->m);
+        const bool by_rows = usable && n >= score_least_rows(dm->m) && score_rows_fit(dm->m);
         const std::vector<int> first = score_slices(ds.row_ptr, n, slice_entries, by_rows ? kScoreGroupRows : 1);
         for (size_t k = 0; k + 1 < first.size(); ++k) {
             const int r0 = first[k], r1 = first[k + 1];
