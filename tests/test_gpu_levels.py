@@ -362,3 +362,32 @@ def test_pairs_that_fill_their_fields(n, g, h):
     want = np.bincount(s.global_bin_ids(rp, col)[0], minlength=s.n_bins)[:, None] * one
     assert np.array_equal(got, want)  # (the steps are powers of two and the sums integers below 2^53 of them)
     s.close()
+
+
+# Class trees whose rows walk them at the end (655 360 rows of all trees on) against the launches that keep row lists, byte for byte: records
+# of 4, 8, 16 and 32 bytes, features that share a column, missing values, trees that stop early, an odd number of rows.
+@pytest.mark.parametrize("n,F,K,depth,hot", [
+    (163_840, 3, 4, 8, 0), (163_839, 3, 4, 8, 0), (218_455, 7, 3, 6, 0), (131_073, 13, 5, 4, 0), (93_623, 31, 7, 8, 0), (131_072, 6, 5, 1, 0),
+    (120_001, 8, 6, 7, 60), (220_000, 2, 3, 10, 30)])
+def test_class_trees_are_walked(n, F, K, depth, hot, monkeypatch):
+    import thundergbm_amd as T
+    rng = np.random.default_rng(n + F)
+    X = np.zeros((n, F + hot), np.float32)
+    X[:, :F] = rng.standard_normal((n, F)).astype(np.float32)
+    X[:, :F][rng.random((n, F)) < 0.15] = 0
+    group = rng.integers(0, hot + 1, n)
+    if hot:
+        X[np.arange(n)[group < hot], F + group[group < hot]] = 1
+    z = X[:, 0] + np.abs(X[:, F - 1]) + 0.2 * (group % 5) + 0.3 * rng.standard_normal(n)
+    y = np.digitize(z, np.quantile(z, np.arange(1, K) / K)).astype(np.float32)
+    val, rp, col = D.dense_to_csr(X)
+    out = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("TGBM_SPLIT_HIST", switch)
+        s = T.Session(val, rp, col, y, depth=depth, n_trees=2, learning_rate=0.4, objective="multi:softmax", num_class=K, gamma=2.0)
+        assert (s.info("split_hist_rows") > 0) == (switch == "1")
+        s.boost(2)
+        out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes()))
+        s.close()
+    same = [a == b for a, b in zip(*out)]
+    assert all(same), same

@@ -546,7 +546,12 @@ void launch_partition_dense(hipStream_t s, const TreeBuffers &tb, const DenseBin
 struct SplitHistPlan {
     int run = 0, log_split = 0;
     int lds_bins = 0;  // part_bins[log_split]
+    // Class trees whose rows have all of their bins, of a byte each, in one record: launch_map_end walks the trees with them, and
+    // tb.nid is left alone until then. From so many rows of all trees on: calls of 10 rounds, depth 8, without and with, ms: 8 x 60 k one-hot rows
+    // 3.53, 3.52; 3 x 250 k 4.28, 4.16; 4 x 200 k x 28 4.51, 4.39; 4 x 500 k 6.69, 6.62; 20 rounds of 8 x 500 k 12.9, 12.55.
+    bool walk = false;
 };
+constexpr int kWalkRows = 5 << 17;
 // (split_hist_run: the rows as far as what is stored decides them; the plan's are as many or more)
 int split_hist_run(const TreeBuffers &tb, int n_class);
 SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, const int *part_bins, int n_class);
@@ -561,10 +566,11 @@ bool launch_small_level(hipStream_t s, const TreeBuffers &tb, const DenseBins &b
                         float lambda, const int *part_bins, int n_class, SplitCand *next_cand, float mcw);
 // The end of a tree whose rows' nodes are in tb.nid (lookup_level >= 0: split nodes of that level still hold the rows of their
 // children): prunes the tree into `model` (n_class trees back to back; tb.nodes
-// stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics.
+// stays as it is) and updates the predictions; y: also the metric partials, the next gradients and their statistics. walk (not with y):
+// SplitHistPlan::walk.
 void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int lookup_level, TreeNode *model, float gamma, float *yp,
                       float lr, int n_class = 1, const float *y = nullptr, int objective = 0, int metric_kind = 0,
-                      GHPair *gh = nullptr, double *metric_scratch = nullptr, unsigned *gh_words = nullptr);
+                      GHPair *gh = nullptr, double *metric_scratch = nullptr, unsigned *gh_words = nullptr, bool walk = false);
 // Sparse level pass (tb.nid16 set): split search of a level (candidates into tb.cand, one slot per task / big
 // feature; launch_best_update follows) and the row -> node update. dump_hist: also store the (node, bin) tables
 // into tb.hist(level) (stage-wise driving and tests; needs tb.hist_q).

@@ -959,6 +959,7 @@ SplitHistPlan split_hist_plan(const TreeBuffers &tb, const DenseBins &bins, cons
         plan.run = run;
         plan.log_split = parts;
         plan.lds_bins = part_bins[parts];
+        plan.walk = n_class > 1 && (long)tb.n * n_class >= kWalkRows && bins.n_blocks == 1 && bins.bin_bytes == 1 && bins.W <= 32 && tb.split_bin == nullptr;
         return plan;
     }
     return plan;
@@ -988,12 +989,17 @@ void launch_partition_hist(hipStream_t s, const TreeBuffers &tb, const DenseBins
                            float rt_eps, float lambda, int n_class) {
     const dim3 items(most_partition_items(tb, level), 1, n_class);
     const bool last = level == tb.depth - 1;
+    if (plan.walk) {  // (bytes)
+        if (last) return launch_best_update(s, tb, level, rt_eps, lambda, n_class);
+        if (level == 0) k_split_count<true, uint8_t, true, false><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);
+        else k_split_count<false, uint8_t, true, false><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);
+    }
 #define TGBM_SPLIT_MAP(T)                                                                                                          \
     if (last && level == 0) k_split_count<true, T, true, false, 2><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);       \
     else if (last) k_split_count<false, T, true, false, 2><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);               \
     else if (level == 0) k_split_count<true, T, true, false, 1><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda);          \
     else k_split_count<false, T, true, false, 1><<<items, kBlock, 0, s>>>(tb, bins, level, rt_eps, lambda)
-    if (bins.bin_bytes == 2) { TGBM_SPLIT_MAP(uint16_t); }
+    else if (bins.bin_bytes == 2) { TGBM_SPLIT_MAP(uint16_t); }
     else { TGBM_SPLIT_MAP(uint8_t); }
 #undef TGBM_SPLIT_MAP
     if (last) return;

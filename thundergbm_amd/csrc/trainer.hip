@@ -1318,7 +1318,8 @@ void Trainer::build_round_together() {
         partition_sets(tb, d_gh_, level, K);
     }
     if (maps_rows())
-        launch_map_end(stream_, tb, bins_, small() ? param_.depth - 1 : -1, d_model_ + (size_t)trees_built_ * tb.n_nodes, param_.gamma, d_yp_, param_.learning_rate, K);
+        launch_map_end(stream_, tb, bins_, small() ? param_.depth - 1 : -1, d_model_ + (size_t)trees_built_ * tb.n_nodes, param_.gamma, d_yp_, param_.learning_rate, K,
+                       nullptr, objective_, metric_kind_, nullptr, nullptr, nullptr, run() > 0 && run_plan_.walk);
     else
         launch_predict_in_training(stream_, tb, &bins_, &csr_, lookup_level_, d_yp_, param_.learning_rate, K, &param_.gamma);
     TGBM_CHECK(trees_built_ + K <= model_cap_trees_, "more trees built than n_trees * tree_per_rounds");

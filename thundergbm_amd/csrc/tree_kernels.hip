@@ -2332,7 +2332,39 @@ __global__ __launch_bounds__(BLK) void k_tree_end(TreeBuffers tb_all, DenseBins 
 // 500 k and depth 8. One launch instead of k_end_bounds, k_tree_end and the copy: 31 -> 8 us at 10 k rows. At 500 k x 28 the last
 // level's count launch updates the tree and maps the rows (11 us) and the end takes 11, where k_best_update, k_end_bounds and
 // k_tree_end took 4.4, 9.7 and 14.7.
-template <int MODE>
+// RW: 0, or the dwords of a row's record, where a row has all of its bins in one: then the rows' nodes are not in the map, but every row
+// walks the tree here, its record in registers and a word of every node in LDS, and leaves its node there. What the count launches
+// stored row by row, 4 bytes to a line of its own each, is what this saves; the last level's update of the tree is a launch of its own again.
+// Bound by the walk's vector instructions. Eight trees of 500 k rows of 12 columns, last count and end: 43 and 15.5 us -> 4.9 (the update)
+// and 32.7; one tree of 500 k x 28 10.7 and 11.1 -> 4.2 and 18.6, which is why only class trees built together walk.
+// (by value: a choice between two places of an array is a choice of addresses to the compiler, and the array goes to scratch memory)
+__device__ __forceinline__ unsigned either(bool second, unsigned a, unsigned b) { return second ? b : a; }
+template <int RW>
+struct RowRecord {
+    uint4 v[RW / 4];
+    __device__ __forceinline__ void load(const uint8_t *from) {
+#pragma unroll
+        for (int i = 0; i < RW / 4; ++i) v[i] = reinterpret_cast<const uint4 *>(from)[i];
+    }
+    __device__ __forceinline__ unsigned dword(unsigned d) const {
+        uint4 q = v[0];
+        if constexpr (RW == 8) q = make_uint4(either(d & 4u, v[0].x, v[1].x), either(d & 4u, v[0].y, v[1].y), either(d & 4u, v[0].z, v[1].z), either(d & 4u, v[0].w, v[1].w));
+        return either(d & 2u, either(d & 1u, q.x, q.y), either(d & 1u, q.z, q.w));
+    }
+};
+template <>
+struct RowRecord<2> {
+    uint2 v;
+    __device__ __forceinline__ void load(const uint8_t *from) { v = *reinterpret_cast<const uint2 *>(from); }
+    __device__ __forceinline__ unsigned dword(unsigned d) const { return either(d & 1u, v.x, v.y); }
+};
+template <>
+struct RowRecord<1> {
+    unsigned v;
+    __device__ __forceinline__ void load(const uint8_t *from) { v = *reinterpret_cast<const unsigned *>(from); }
+    __device__ __forceinline__ unsigned dword(unsigned) const { return v; }
+};
+template <int MODE, int RW>
 __global__ __launch_bounds__(kEndWide) void k_map_end(TreeBuffers tb_all, DenseBins bins, TreeEndArgs a, TreeNode *model) {
     constexpr int kNodes = (2 << kSmallDepth) - 1;
     __shared__ short s_leaf[kRowBlock];
@@ -2348,19 +2380,61 @@ __global__ __launch_bounds__(kEndWide) void k_map_end(TreeBuffers tb_all, DenseB
     const int r0 = blockIdx.x * kRowBlock, r1 = min(tb.n, r0 + kRowBlock);  // (none for the last workgroup)
     constexpr int V = kRowBlock / kEndWide;
     int at[V];
+    __shared__ uint2 s_step[RW > 0 ? kNodes : 1];  // x: first bin, bins, split bin, a bit for the default and for a split; y: shift and dword
+    RowRecord<(RW > 0 ? RW : 1)> record[V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) at[v] = tb.nid[min(r0 + v * kEndWide + (int)threadIdx.x, tb.n - 1)];
+    for (int v = 0; v < V; ++v) {
+        const int row = min(r0 + v * kEndWide + (int)threadIdx.x, tb.n - 1);
+        if constexpr (RW == 0) {
+            at[v] = tb.nid[row];
+        } else {
+            record[v].load(bins.data + (size_t)row * (RW * 4));
+        }
+    }
     for (int i = threadIdx.x; i < tb.n_nodes; i += kEndWide) {
         const TreeNode nd = tb.nodes[i];
+        if constexpr (RW > 0) {
+            uint2 step = make_uint2(0u, 0u);
+            if (node_splits(nd)) {  // (see k_split_count)
+                unsigned c = (unsigned)nd.split_feature_id, lo = 0, span = kMissingBin;
+                if (bins.feat_col != nullptr) {
+                    lo = bins.feat_lo[c];
+                    span = (unsigned)(tb.cut_row_ptr[c + 1] - tb.cut_row_ptr[c]);
+                    c = (unsigned)bins.feat_col[c];
+                }
+                step = make_uint2(lo | span << 8 | (unsigned)nd.split_bid << 16 | (nd.default_right ? 1u << 24 : 0u) | 1u << 25, (c & 3u) * 8u | (c >> 2) << 8);
+            }
+            s_step[i] = step;
+        }
         s_flag[i] = (unsigned char)((nd.is_valid ? VALID : 0) | (nd.is_leaf ? LEAF : 0) | (nd.gain < a.gamma ? BELOW : 0));
         s_value[i] = nd.base_weight;
+    }
+    if constexpr (RW > 0) {
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < V; ++v) at[v] = 0;
+        for (int level = 0; level < tb.depth; ++level) {
+            uint2 step[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) step[v] = s_step[at[v]];
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const unsigned bin = record[v].dword(step[v].y >> 8) >> (step[v].y & 31u) & 0xffu;
+                const int t = (int)bin - (int)(step[v].x & 0xffu);
+                const bool right = (unsigned)t >= (step[v].x >> 8 & 0xffu) ? (step[v].x >> 24 & 1u) != 0 : t >= (int)(step[v].x >> 16 & 0xffu);
+                at[v] = step[v].x >> 25 ? 2 * at[v] + (right ? 2 : 1) : at[v];  // (heap order)
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (r0 + v * kEndWide + (int)threadIdx.x < r1) tb.nid[r0 + v * kEndWide + (int)threadIdx.x] = at[v];
     }
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         const int i = v * kEndWide + (int)threadIdx.x;
         if (r0 + i >= r1) continue;
         int leaf = at[v];
-        if (a.lookup_level >= 0) {  // (that level's split nodes still hold their rows)
+        if (RW == 0 && a.lookup_level >= 0) {  // (that level's split nodes still hold their rows)
             const TreeNode &nd = tb.nodes[leaf];
             if (nd.split_feature_id >= 0 && leaf >= (1 << a.lookup_level) - 1) leaf = end_child_of<false>(tb, bins, CsrBins{}, nd, r0 + i);
         }
@@ -2893,7 +2967,7 @@ void launch_round_end(hipStream_t s, const TreeBuffers &tb, const DenseBins *dbi
 
 void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins, int lookup_level, TreeNode *model, float gamma, float *yp,
                       float lr, int n_class, const float *y, int objective, int metric_kind, GHPair *gh,
-                      double *metric_scratch, unsigned *gh_words) {
+                      double *metric_scratch, unsigned *gh_words, bool walk) {
     TreeEndArgs a{};
     a.lookup_level = lookup_level;
     a.gamma = gamma;
@@ -2907,8 +2981,15 @@ void launch_map_end(hipStream_t s, const TreeBuffers &tb, const DenseBins &bins,
     a.metric_partial = metric_scratch;
     a.gh_words = gh_words;
     const dim3 grid(row_blocks(tb.n) + 1, 1, n_class);  // (the last one writes the model)
-    if (y != nullptr) k_map_end<2><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
-    else k_map_end<1><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+    if (y != nullptr) return k_map_end<2, 0><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+    switch (walk ? bins.W : 0) {  // (bytes of a record: split_hist_plan)
+        case 0: return k_map_end<1, 0><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+        case 4: return k_map_end<1, 1><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+        case 8: return k_map_end<1, 2><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+        case 16: return k_map_end<1, 4><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+        case 32: return k_map_end<1, 8><<<grid, kEndWide, 0, s>>>(tb, bins, a, model);
+        default: fatal("a walk over records of %d bytes", bins.W);
+    }
 }
 
 void launch_metric_final(hipStream_t s, int n, const TreeLeftovers &left) {
