@@ -13,7 +13,7 @@ namespace tgbm {
 enum RankMetric { RANK_METRIC_MAP = 3, RANK_METRIC_NDCG = 4 };
 
 // Groups of at most this many rows are ordered by counting (every row counts the rows of its segment that go before
-// it: one launch, quadratic in the segment length); data with a longer group takes the radix sort.
+// it, in the LDS of a workgroup: quadratic in the segment length); data with a longer group takes the radix sort.
 constexpr int kRankCountSortMax = 2048;
 constexpr int kRankCountSortMean = 384;  // ... and only while sum(len^2) / rows stays below this
 
@@ -67,19 +67,20 @@ class RankContext {
     const float *d_y_ = nullptr;
     int *d_static_row_ = nullptr;  // rows of every group by label descending (ties: row ascending)
     int *d_run_of_ = nullptr;      // run of a position of that order
-    int *d_run_of_row_ = nullptr;  // run of a row
+    int *d_run_of_row_ = nullptr;  // run of a row (long groups)
     RankRun *d_runs_ = nullptr;
     int *d_group_of_ = nullptr;    // group of a row
     int *d_gptr_ = nullptr;
     float *d_idcg_ = nullptr;
     int *d_group_hits_ = nullptr;  // rows with a non-zero label per group
-    long long *d_acc_ = nullptr;   // [2n] fixed-point gradient / hessian sums
+    long long *d_acc_ = nullptr;   // [2n] fixed-point gradient / hessian sums (long groups)
     unsigned *d_flags_ = nullptr, *d_hits_before_ = nullptr;
     double *d_partial_ = nullptr;
     int n_partial_ = 0;
     PairSorter sorter_;
     int last_cur_ = 0;
     bool have_metric_order_ = false;  // sorter_.vals[last_cur_] is the (group, score) order of a metric() call
+    int longest_ = 0;                 // group
     bool short_groups_ = false;       // groups short enough to be ordered by counting (kRankCountSortMax / Mean)
 };
 

@@ -5,8 +5,8 @@
 // round is a handful of data-parallel passes over all rows:
 //   * labels never change, so the label-descending order of every group, its runs of equal labels and the
 //     part of each run that draws partners are tables built once (k_rank_setup; on the host where groups are long);
-//   * per round one stable radix sort of (run, descending score) keys orders the rows inside their runs,
-//     which reproduces "sort by score, then stably by label";
+//   * per round a workgroup per group (k_rank_gradient_group), or one stable radix sort of (run, descending score) keys
+//     where groups are long, orders the rows inside their runs, which reproduces "sort by score, then stably by label";
 //   * one thread per position draws its partner, evaluates the pair and adds the lambdas to both rows with
 //     64-bit fixed-point atomics (exact integer sums: the result does not depend on the order of the adds).
 // Two things differ from the reference by necessity, because there they are not reproducible: ties between
@@ -59,17 +59,18 @@ __device__ __forceinline__ int acc_bits(int len) { return 59 - (32 - __clz(max(l
 // Bound by the counting (len^2 steps of LDS a group). 200 003 rows in 1667 groups: 22 us, where eight threads of the host, the
 // copies of their tables and the look at the labels took 1.7 ms (a call of 40 rounds 20.5 -> 19.4 ms).
 constexpr int kSetupBlock = 128;
+// threads of the rounds' kernels, where no group is longer than 64 or 256 rows, and where one is
+constexpr int kShortGroup = 64, kMiddleGroup = 256, kLongGroupBlock = 512;
+constexpr size_t kRankGroupBytes = 2 * sizeof(unsigned long long) + 2 * sizeof(int) + sizeof(float);  // LDS of k_rank_gradient_group per row
 __global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restrict__ y, const int *__restrict__ gptr,
                                                             const float *__restrict__ log2_of, int longest, int *__restrict__ static_row,
-                                                            int *__restrict__ run_of, int *__restrict__ run_of_row,
-                                                            int *__restrict__ group_of, RankRun *__restrict__ runs,
+                                                            int *__restrict__ run_of, int *__restrict__ group_of, RankRun *__restrict__ runs,
                                                             float *__restrict__ idcg, int *__restrict__ hits, int *__restrict__ counts) {
     extern __shared__ unsigned s_mem[];
     __shared__ int s_hits, s_bad, s_runs;
     unsigned *s_key = s_mem;                                          // keys by row, then IDCG's terms by position
     float *s_sorted = reinterpret_cast<float *>(s_key + longest);    // labels by position
-    unsigned short *s_at = reinterpret_cast<unsigned short *>(s_sorted + longest);  // position of a row
-    unsigned short *s_run = s_at + longest;                          // run of a position, within the group
+    unsigned short *s_run = reinterpret_cast<unsigned short *>(s_sorted + longest);  // run of a position, within the group
     unsigned short *s_first = s_run + longest;                       // first position of a run; the top bit: it draws no partner
     const int g = blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
     if (threadIdx.x == 0) s_hits = s_bad = s_runs = 0;
@@ -89,7 +90,6 @@ __global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restr
         const unsigned key = s_key[i];
         int before = 0;
         for (int j = 0; j < len; ++j) before += s_key[j] > key || (s_key[j] == key && j < i) ? 1 : 0;
-        s_at[i] = (unsigned short)before;
         s_sorted[before] = y[b + i];
         static_row[b + before] = b + i;
     }
@@ -145,10 +145,7 @@ __global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restr
         r.group = g;
         runs[b + k] = r;
     }
-    for (int i = threadIdx.x; i < len; i += kSetupBlock) {
-        run_of[b + i] = b + s_run[i];
-        run_of_row[b + i] = b + s_run[s_at[i]];
-    }
+    for (int i = threadIdx.x; i < len; i += kSetupBlock) run_of[b + i] = b + s_run[i];
 }
 
 int grid_for(size_t n) {
@@ -187,56 +184,114 @@ __global__ __launch_bounds__(kBlock) void k_rank_metric_keys(int n, const int *_
     vals[row] = row;
 }
 
-// Stable order by descending score inside every segment through counting: the place of an element is the number of
-// elements of its segment with a smaller key (the radix sort's key: ~float_key(score)) or with the same key and an
-// earlier position - the order the stable radix sort of (segment, key) pairs gives, in one launch. Segments are short
-// (kRankCountSortMax at most) and the threads of a wavefront mostly walk the same one, so the loads of the walk are
-// shared. RUNS: segments are the runs of equal labels in the label-descending order (positions -> rows through
-// static_row); otherwise the query groups in row order.
-// (the keys of all elements in segment order first, so that the walk loads them from consecutive addresses)
-__global__ __launch_bounds__(kBlock) void k_rank_sort_keys(int n, const float *__restrict__ score,
-                                                          const int *__restrict__ static_row, unsigned *__restrict__ key) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p < n) key[p] = ~float_key(score[static_row != nullptr ? static_row[p] : p]);
+// The body of the inner loop of LambdaRank::get_gradient (ranking_obj.cpp:63-90) for position p of the (label descending, score
+// descending) order of its group: its partner, and what the pair adds to the row nearer the top of the label order (the other
+// one gets the gradient's opposite). idcg: of the group, nullptr: rank:pairwise.
+struct RankPair {
+    int high, low;  // positions inside the group
+    long long ql;
+    unsigned long long qh;
+};
+__device__ __forceinline__ bool draw_partner(const RankRun &r, int p, unsigned seed, RankPair &pair) {
+    if (p < r.first_l) return false;
+    const int nleft = r.first_l - r.group_begin;
+    const int nright = r.group_end - r.end;
+    if (nleft + nright == 0) return false;
+    const int m = (int)rank_draw(seed, (unsigned)p, (unsigned)(nleft + nright));
+    const int l = p - r.group_begin;
+    const bool left = m < nleft;
+    pair.high = left ? m : l;
+    pair.low = left ? l : m - nleft + (r.end - r.group_begin);
+    return true;
 }
-
-template <bool RUNS>
-__global__ __launch_bounds__(kBlock) void k_rank_count_sort(int n, const unsigned *__restrict__ keys,
-                                                           const int *__restrict__ static_row,
-                                                           const int *__restrict__ run_of,
-                                                           const RankRun *__restrict__ runs,
-                                                           const int *__restrict__ group_of,
-                                                           const int *__restrict__ gptr, int *__restrict__ sorted) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= n) return;
-    int sb, se;
-    if (RUNS) {
-        const RankRun r = runs[run_of[p]];
-        sb = r.begin;
-        se = r.end;
-    } else {
-        const int g = group_of[p];
-        sb = gptr[g];
-        se = gptr[g + 1];
-    }
-    const unsigned key = keys[p];
-    int before = 0;
-    constexpr int kAhead = 8;
-    for (int j0 = sb; j0 < se; j0 += kAhead) {
-        unsigned kj[kAhead];
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) kj[u] = keys[min(j0 + u, se - 1)];
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const int j = j0 + u;
-            before += (j < se && (kj[u] < key || (kj[u] == key && j < p))) ? 1 : 0;
+__device__ __forceinline__ void weigh_pair(RankPair &pair, const float *idcg, float label_high, float label_low, float score_high,
+                                           float score_low, int group_rows) {
+    float dz = 1.f;  // LambdaRank::get_delta_z
+    if (idcg != nullptr) {  // LambdaRankNDCG::get_delta_z (ranking_obj.cpp:105-113)
+        const float z = *idcg;
+        if (z == 0.f) {
+            dz = 0.f;
+        } else {
+            const int li = (int)label_high, lj = (int)label_low;
+            dz = (discounted_gain(li, pair.high) + discounted_gain(lj, pair.low) - discounted_gain(li, pair.low) -
+                  discounted_gain(lj, pair.high)) / z;
         }
     }
-    sorted[sb + before] = RUNS ? static_row[p] : p;
+    const float adz = fabsf(dz);
+    const float rho = 1.f / (1.f + expf(score_high - score_low));
+    const float lambda = -adz * rho;
+    const float hess = 2.f * fmaxf(adz * rho * (1.f - rho), 1e-16f);
+    const int sb = acc_bits(group_rows);
+    pair.ql = __double2ll_rn(ldexp((double)lambda, sb));
+    pair.qh = (unsigned long long)__double2ll_rn(ldexp((double)hess, sb));
+}
+__device__ __forceinline__ GHPair pair_of_sums(long long g, long long h, int group_rows) {
+    const int sb = acc_bits(group_rows);
+    return GHPair{(float)ldexp((double)g, -sb), (float)ldexp((double)h, -sb)};
 }
 
-// One thread per position of the (label descending, score descending) order of its group; the body is the
-// inner loop of LambdaRank::get_gradient (ranking_obj.cpp:63-90) for l = that position.
+// Groups of at most kRankCountSortMax rows: a workgroup has a group to itself, orders it by counting in LDS and adds the lambdas up
+// there. Bound by the counting, len^2 steps of LDS a group. 200 003 rows in 1667 groups of about 120: the order by score 15 us (keys and
+// counting through the L1: 4.6 and 16.3), the gradients 20 (keys, counting, pairs with four 64-bit atomics a row, sums: 4.9, 11, 28, 5.2).
+// Keys read four at a time, or eight ahead: 15, 27 us.
+__device__ __forceinline__ int rows_before(const unsigned *s_key, int from, int to, unsigned key, int at) {
+    int before = 0;
+    for (int j = from; j < to; ++j) {
+        const unsigned k = s_key[j];
+        before += k < key || (k == key && j < at) ? 1 : 0;
+    }
+    return before;
+}
+
+// sorted: the rows of every group by score descending, ties by row.
+template <int BLK>
+__global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict__ gptr, const float *__restrict__ score, int *__restrict__ sorted) {
+    extern __shared__ unsigned s_key[];
+    const int b = gptr[blockIdx.x], len = gptr[blockIdx.x + 1] - b;
+    for (int i = threadIdx.x; i < len; i += BLK) s_key[i] = ~float_key(score[b + i]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += BLK) sorted[b + rows_before(s_key, 0, len, s_key[i], i)] = b + i;
+}
+
+// Rows inside their runs of equal labels by score descending, ties by row (static_row ascends inside a run), then every position's pair.
+template <int BLK>
+__global__ __launch_bounds__(BLK) void k_rank_gradient_group(const int *__restrict__ gptr, const float *__restrict__ score, const float *__restrict__ y,
+                                                             const int *__restrict__ static_row, const int *__restrict__ run_of,
+                                                             const RankRun *__restrict__ runs, const float *__restrict__ idcg, unsigned seed,
+                                                             int longest, int *__restrict__ sorted, GHPair *__restrict__ gh) {
+    extern __shared__ unsigned long long s_acc[];  // [2 longest] by row
+    unsigned *s_key = reinterpret_cast<unsigned *>(s_acc + 2 * longest);  // by position of static_row
+    int *s_row = reinterpret_cast<int *>(s_key + longest);                // by position of the order, within the group
+    float *s_score = reinterpret_cast<float *>(s_row + longest);
+    const int g = blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
+    for (int i = threadIdx.x; i < len; i += BLK) {
+        s_key[i] = ~float_key(score[static_row[b + i]]);
+        s_acc[2 * i] = s_acc[2 * i + 1] = 0ull;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += BLK) {
+        const RankRun r = runs[run_of[b + i]];
+        const int row = static_row[b + i], at = r.begin - b + rows_before(s_key, r.begin - b, r.end - b, s_key[i], i);
+        s_row[at] = row - b;
+        s_score[at] = score[row];
+        sorted[b + at] = row;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += BLK) {
+        RankPair pair;
+        if (!draw_partner(runs[run_of[b + i]], b + i, seed, pair)) continue;
+        const int high = s_row[pair.high], low = s_row[pair.low];
+        weigh_pair(pair, idcg != nullptr ? idcg + g : nullptr, y[b + high], y[b + low], s_score[pair.high], s_score[pair.low], len);
+        atomicAdd(&s_acc[2 * high], (unsigned long long)pair.ql);
+        atomicAdd(&s_acc[2 * high + 1], pair.qh);
+        atomicAdd(&s_acc[2 * low], (unsigned long long)(-pair.ql));
+        atomicAdd(&s_acc[2 * low + 1], pair.qh);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < len; i += BLK) gh[b + i] = pair_of_sums((long long)s_acc[2 * i], (long long)s_acc[2 * i + 1], len);
+}
+
+// One thread per position, for groups of any length.
 __global__ __launch_bounds__(kBlock) void k_rank_pairs(int n, const RankRun *__restrict__ runs,
                                                       const int *__restrict__ run_of, const int *__restrict__ sorted_row,
                                                       const float *__restrict__ score, const float *__restrict__ y,
@@ -245,44 +300,14 @@ __global__ __launch_bounds__(kBlock) void k_rank_pairs(int n, const RankRun *__r
     const int p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= n) return;
     const RankRun r = runs[run_of[p]];
-    if (p < r.first_l) return;
-    const int nleft = r.first_l - r.group_begin;
-    const int nright = r.group_end - r.end;
-    if (nleft + nright == 0) return;
-    const int m = (int)rank_draw(seed, (unsigned)p, (unsigned)(nleft + nright));
-    const int l = p - r.group_begin;
-    int high, low;  // positions inside the group; `high` is the one nearer the top of the label order
-    if (m < nleft) {
-        high = m;
-        low = l;
-    } else {
-        high = l;
-        low = m - nleft + (r.end - r.group_begin);
-    }
-    const int high_row = sorted_row[r.group_begin + high];
-    const int low_row = sorted_row[r.group_begin + low];
-    float dz = 1.f;  // LambdaRank::get_delta_z
-    if (idcg != nullptr) {  // LambdaRankNDCG::get_delta_z (ranking_obj.cpp:105-113)
-        const float z = idcg[r.group];
-        if (z == 0.f) {
-            dz = 0.f;
-        } else {
-            const int li = (int)y[high_row], lj = (int)y[low_row];
-            dz = (discounted_gain(li, high) + discounted_gain(lj, low) - discounted_gain(li, low) -
-                  discounted_gain(lj, high)) / z;
-        }
-    }
-    const float adz = fabsf(dz);
-    const float rho = 1.f / (1.f + expf(score[high_row] - score[low_row]));
-    const float lambda = -adz * rho;
-    const float hess = 2.f * fmaxf(adz * rho * (1.f - rho), 1e-16f);
-    const int sb = acc_bits(r.group_end - r.group_begin);
-    const long long ql = __double2ll_rn(ldexp((double)lambda, sb));
-    const unsigned long long qh = (unsigned long long)__double2ll_rn(ldexp((double)hess, sb));
-    atomicAdd(acc + 2 * (size_t)high_row, (unsigned long long)ql);
-    atomicAdd(acc + 2 * (size_t)high_row + 1, qh);
-    atomicAdd(acc + 2 * (size_t)low_row, (unsigned long long)(-ql));
-    atomicAdd(acc + 2 * (size_t)low_row + 1, qh);
+    RankPair pair;
+    if (!draw_partner(r, p, seed, pair)) return;
+    const int high_row = sorted_row[r.group_begin + pair.high], low_row = sorted_row[r.group_begin + pair.low];
+    weigh_pair(pair, idcg != nullptr ? idcg + r.group : nullptr, y[high_row], y[low_row], score[high_row], score[low_row], r.group_end - r.group_begin);
+    atomicAdd(acc + 2 * (size_t)high_row, (unsigned long long)pair.ql);
+    atomicAdd(acc + 2 * (size_t)high_row + 1, pair.qh);
+    atomicAdd(acc + 2 * (size_t)low_row, (unsigned long long)(-pair.ql));
+    atomicAdd(acc + 2 * (size_t)low_row + 1, pair.qh);
 }
 
 // fixed point -> GHPair, and the accumulators are cleared for the next round
@@ -292,11 +317,9 @@ __global__ __launch_bounds__(kBlock) void k_rank_finish(int n, const int *__rest
     const int row = blockIdx.x * kBlock + threadIdx.x;
     if (row >= n) return;
     const int g = group_of[row];
-    const int sb = acc_bits(gptr[g + 1] - gptr[g]);
-    const long long ag = acc[2 * (size_t)row], ah = acc[2 * (size_t)row + 1];
+    gh[row] = pair_of_sums(acc[2 * (size_t)row], acc[2 * (size_t)row + 1], gptr[g + 1] - gptr[g]);
     acc[2 * (size_t)row] = 0;
     acc[2 * (size_t)row + 1] = 0;
-    gh[row] = GHPair{(float)ldexp((double)ag, -sb), (float)ldexp((double)ah, -sb)};
 }
 
 // Sum of a block's per-thread doubles in thread order (the same bits on every run).
@@ -395,7 +418,7 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, 
     }
     TGBM_CHECK(gptr.back() == n_, "query groups cover %d instances, the dataset has %d", gptr.back(), n_);
 
-    // ordering by counting costs sum(len^2) steps (measured: 50 us for a million rows in groups of 120, where the radix
+    // ordering by counting costs sum(len^2) steps (a launch per pass: 50 us for a million rows in groups of 120, where the radix
     // sort takes 220 us): taken while the average row sits in a group of at most kRankCountSortMean rows
     int longest = 0;
     double steps = 0;
@@ -414,19 +437,17 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, 
     }
     d_static_row_ = dalloc<int>(n_);
     d_run_of_ = dalloc<int>(n_);
-    d_run_of_row_ = dalloc<int>(n_);
     d_group_of_ = dalloc<int>(n_);
     d_gptr_ = dalloc<int>(gptr.size());
     d_idcg_ = dalloc<float>(n_groups_);
     d_group_hits_ = dalloc<int>(n_groups_);
-    d_acc_ = dalloc<long long>(2 * (size_t)n_);
     d_flags_ = dalloc<unsigned>(n_);
     d_hits_before_ = dalloc<unsigned>((size_t)n_ + 1);
     n_partial_ = grid_for(n_);
     d_partial_ = dalloc<double>(n_partial_);
     upload(d_gptr_, gptr.data(), sizeof(int) * gptr.size());
-    HIP_CHECK(hipMemsetAsync(d_acc_, 0, sizeof(long long) * 2 * (size_t)std::max(n_, 1), stream_));
     sorter_.alloc(n_);
+    longest_ = longest;
     if (short_groups_) setup_short_groups(longest);
     else setup_groups(y, gptr);
     TGBM_CHECK(!ndcg || idcg_valid_, "rank:ndcg needs labels in 0..30");  // (small non-negative integers: 1 << label)
@@ -446,10 +467,9 @@ void RankContext::setup_short_groups(int longest) {
     int *d_counts = dalloc<int>(3);
     HIP_CHECK(hipMemsetAsync(d_counts, 0, sizeof(int) * 3, stream_));
     static_assert(kRankCountSortMax <= 1 << 15, "positions of a group in 15 bits");
-    const size_t lds = (size_t)longest * (2 * sizeof(unsigned) + 3 * sizeof(unsigned short));
-    static_assert(kRankCountSortMax * 14 <= 48 << 10, "no opt-in for the LDS");
-    k_rank_setup<<<n_groups_, kSetupBlock, lds, stream_>>>(d_y_, d_gptr_, d_log2, longest, d_static_row_, d_run_of_, d_run_of_row_, d_group_of_,
-                                                           d_runs_, d_idcg_, d_group_hits_, d_counts);
+    const size_t lds = (size_t)longest * (2 * sizeof(unsigned) + 2 * sizeof(unsigned short));
+    static_assert(kRankCountSortMax * 12 <= 48 << 10, "no opt-in for the LDS");
+    k_rank_setup<<<n_groups_, kSetupBlock, lds, stream_>>>(d_y_, d_gptr_, d_log2, longest, d_static_row_, d_run_of_, d_group_of_, d_runs_, d_idcg_, d_group_hits_, d_counts);
     HIP_CHECK(hipGetLastError());
     int counts[3];
     HIP_CHECK(hipMemcpyAsync(counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, stream_));
@@ -532,6 +552,9 @@ void RankContext::setup_groups(const LabelVector &y, const std::vector<int> &gpt
     idcg_valid_ = labels_ok;
     run_bits_ = bits_for((long)runs.size());
     d_runs_ = dalloc<RankRun>(runs.size());
+    d_run_of_row_ = dalloc<int>(n_);
+    d_acc_ = dalloc<long long>(2 * (size_t)n_);
+    HIP_CHECK(hipMemsetAsync(d_acc_, 0, sizeof(long long) * 2 * (size_t)std::max(n_, 1), stream_));
     upload(d_static_row_, static_row.data(), sizeof(int) * (size_t)n_);
     upload(d_run_of_, run_of.data(), sizeof(int) * (size_t)n_);
     upload(d_run_of_row_, run_of_row.data(), sizeof(int) * (size_t)n_);
@@ -552,11 +575,21 @@ void RankContext::gradient(const float *d_score, GHPair *d_gh, unsigned seed, bo
     const int grid = grid_for(n_);
     if (short_groups_) {
         last_cur_ = 0;
-        unsigned *keys = reinterpret_cast<unsigned *>(sorter_.keys[0]);
-        k_rank_sort_keys<<<grid, kBlock, 0, stream_>>>(n_, d_score, d_static_row_, keys);
-        k_rank_count_sort<true><<<grid, kBlock, 0, stream_>>>(n_, keys, d_static_row_, d_run_of_, d_runs_, nullptr, nullptr,
-                                                             sorter_.vals[0]);
-    } else if (order_is_fresh && have_metric_order_) {
+        have_metric_order_ = false;
+        static LdsOptIn opt_in;
+        const size_t lds = (size_t)longest_ * kRankGroupBytes;
+        const float *idcg = ndcg_ ? d_idcg_ : nullptr;
+        if (lds > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_rank_gradient_group<kLongGroupBlock>)});
+#define TGBM_RANK_GRADIENT(BLK)                                                                                                        \
+    k_rank_gradient_group<BLK><<<n_groups_, BLK, lds, stream_>>>(d_gptr_, d_score, d_y_, d_static_row_, d_run_of_, d_runs_, idcg, seed, \
+                                                                 longest_, sorter_.vals[0], d_gh)
+        if (longest_ <= kShortGroup) TGBM_RANK_GRADIENT(kShortGroup);
+        else if (longest_ <= kMiddleGroup) TGBM_RANK_GRADIENT(kSetupBlock);
+        else TGBM_RANK_GRADIENT(kLongGroupBlock);
+#undef TGBM_RANK_GRADIENT
+        return;
+    }
+    if (order_is_fresh && have_metric_order_) {
         // rows already ordered by (group, score descending, row): a stable sort by run id yields
         // (run, score descending, row), the same order as the full sort below
         k_rank_run_keys<<<grid, kBlock, 0, stream_>>>(n_, d_run_of_row_, sorter_.vals[last_cur_], sorter_.keys[0],
@@ -579,10 +612,12 @@ void RankContext::metric(int kind, const float *d_score, float *d_out) {
     const int grid = grid_for(n_);
     int cur = 0;
     if (short_groups_) {
-        unsigned *keys = reinterpret_cast<unsigned *>(sorter_.keys[0]);
-        k_rank_sort_keys<<<grid, kBlock, 0, stream_>>>(n_, d_score, nullptr, keys);
-        k_rank_count_sort<false><<<grid, kBlock, 0, stream_>>>(n_, keys, nullptr, nullptr, nullptr, d_group_of_, d_gptr_,
-                                                              sorter_.vals[0]);
+        const size_t lds = (size_t)longest_ * sizeof(unsigned);
+#define TGBM_RANK_ORDER(BLK) k_rank_order_group<BLK><<<n_groups_, BLK, lds, stream_>>>(d_gptr_, d_score, sorter_.vals[0])
+        if (longest_ <= kShortGroup) TGBM_RANK_ORDER(kShortGroup);
+        else if (longest_ <= kMiddleGroup) TGBM_RANK_ORDER(kSetupBlock);
+        else TGBM_RANK_ORDER(kLongGroupBlock);
+#undef TGBM_RANK_ORDER
     } else {
         k_rank_metric_keys<<<grid, kBlock, 0, stream_>>>(n_, d_group_of_, d_score, sorter_.keys[0], sorter_.vals[0]);
         cur = sort_pairs(stream_, sorter_, n_, 32 + group_bits_);
