@@ -149,7 +149,7 @@ def test_rank_full_size_parity(T, sort, monkeypatch):
 # makes for long ones: the same sums and metrics, bit for bit. "steps": many runs of one row, where every other one draws.
 @pytest.mark.parametrize("objective", ["rank:pairwise", "rank:ndcg"])
 @pytest.mark.parametrize("labels", ["few", "steps", "zeros"])
-@pytest.mark.parametrize("groups", [[2048], [1, 0, 63, 64, 65, 2, 0], [127, 128, 129, 1, 1, 257], [0, 1], [3] * 700])
+@pytest.mark.parametrize("groups", [[2048], [1, 0, 63, 64, 65, 2, 0], [127, 128, 129, 1, 1, 257], [256, 2048, 2, 300, 0, 64], [0, 1], [3] * 700])
 def test_rank_tables_of_short_groups(T, objective, labels, groups, monkeypatch):
     rng = np.random.default_rng(len(groups) + len(labels))
     n = sum(groups)

@@ -81,6 +81,8 @@ class RankContext {
     int last_cur_ = 0;
     bool have_metric_order_ = false;  // sorter_.vals[last_cur_] is the (group, score) order of a metric() call
     int longest_ = 0;                 // group
+    int *d_wide_ = nullptr;           // groups that take the widest workgroups
+    int n_wide_ = 0;
     bool short_groups_ = false;       // groups short enough to be ordered by counting (kRankCountSortMax / Mean)
 };
 

@@ -59,7 +59,9 @@ __device__ __forceinline__ int acc_bits(int len) { return 59 - (32 - __clz(max(l
 // Bound by the counting (len^2 steps of LDS a group). 200 003 rows in 1667 groups: 22 us, where eight threads of the host, the
 // copies of their tables and the look at the labels took 1.7 ms (a call of 40 rounds 20.5 -> 19.4 ms).
 constexpr int kSetupBlock = 128;
-// threads of the rounds' kernels, where no group is longer than 64 or 256 rows, and where one is
+// Threads of the rounds' kernels: 64 where no group is longer than 64 rows, 128 for groups of up to 256, 512 for longer ones. Those have a
+// launch of their own, so that the others don't ask for LDS for the longest group, and sort in LDS: counting 2000 rows is 2000 steps for
+// each of four rows a thread, 95 us a round for one such group among 19 800 of ten rows (200 k x 20, 20 rounds: 12.5 -> 7.1 ms).
 constexpr int kShortGroup = 64, kMiddleGroup = 256, kLongGroupBlock = 512;
 constexpr size_t kRankGroupBytes = 2 * sizeof(unsigned long long) + 2 * sizeof(int) + sizeof(float);  // LDS of k_rank_gradient_group per row
 __global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restrict__ y, const int *__restrict__ gptr,
@@ -243,11 +245,45 @@ __device__ __forceinline__ int rows_before(const unsigned *s_key, int from, int 
     return before;
 }
 
-// sorted: the rows of every group by score descending, ties by row.
+// Ascending order of count (a power of two) keys of the workgroup, by a bitonic network; the caller has waited for them.
 template <int BLK>
-__global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict__ gptr, const float *__restrict__ score, int *__restrict__ sorted) {
-    extern __shared__ unsigned s_key[];
-    const int b = gptr[blockIdx.x], len = gptr[blockIdx.x + 1] - b;
+__device__ __forceinline__ void sort_keys(unsigned long long *s, int count) {
+    for (int k = 2; k <= count; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int p = threadIdx.x; p < count / 2; p += BLK) {
+                const int a = 2 * p - (p & (j - 1));
+                const unsigned long long x = s[a], z = s[a + j];
+                if ((x > z) == ((a & k) == 0)) {
+                    s[a] = z;
+                    s[a + j] = x;
+                }
+            }
+            __syncthreads();
+        }
+}
+__host__ __device__ inline int keys_to_sort(int len) {  // fewer than 2 len
+    int count = 1;
+    while (count < len) count <<= 1;
+    return count;
+}
+
+// sorted: the rows of every group by score descending, ties by row. which: the groups of the launch (nullptr: all of at most `most` rows).
+template <int BLK>
+__global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict__ which, int most, const int *__restrict__ gptr,
+                                                          const float *__restrict__ score, int *__restrict__ sorted) {
+    extern __shared__ unsigned long long s_order[];  // [keys_to_sort(most)], as unsigned [most] where they are counted
+    const int g = which != nullptr ? which[blockIdx.x] : (int)blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
+    if (len > most) return;
+    if (BLK == kLongGroupBlock) {
+        const int count = keys_to_sort(len);
+        for (int i = threadIdx.x; i < count; i += BLK)
+            s_order[i] = i < len ? (unsigned long long)~float_key(score[b + i]) << 32 | (unsigned)i : ~0ull;
+        __syncthreads();
+        sort_keys<BLK>(s_order, count);
+        for (int i = threadIdx.x; i < len; i += BLK) sorted[b + i] = b + (int)(unsigned)s_order[i];
+        return;
+    }
+    unsigned *s_key = reinterpret_cast<unsigned *>(s_order);
     for (int i = threadIdx.x; i < len; i += BLK) s_key[i] = ~float_key(score[b + i]);
     __syncthreads();
     for (int i = threadIdx.x; i < len; i += BLK) sorted[b + rows_before(s_key, 0, len, s_key[i], i)] = b + i;
@@ -255,26 +291,45 @@ __global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict_
 
 // Rows inside their runs of equal labels by score descending, ties by row (static_row ascends inside a run), then every position's pair.
 template <int BLK>
-__global__ __launch_bounds__(BLK) void k_rank_gradient_group(const int *__restrict__ gptr, const float *__restrict__ score, const float *__restrict__ y,
+__global__ __launch_bounds__(BLK) void k_rank_gradient_group(const int *__restrict__ which, int most, const int *__restrict__ gptr,
+                                                             const float *__restrict__ score, const float *__restrict__ y,
                                                              const int *__restrict__ static_row, const int *__restrict__ run_of,
                                                              const RankRun *__restrict__ runs, const float *__restrict__ idcg, unsigned seed,
-                                                             int longest, int *__restrict__ sorted, GHPair *__restrict__ gh) {
-    extern __shared__ unsigned long long s_acc[];  // [2 longest] by row
-    unsigned *s_key = reinterpret_cast<unsigned *>(s_acc + 2 * longest);  // by position of static_row
-    int *s_row = reinterpret_cast<int *>(s_key + longest);                // by position of the order, within the group
-    float *s_score = reinterpret_cast<float *>(s_row + longest);
-    const int g = blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
-    for (int i = threadIdx.x; i < len; i += BLK) {
-        s_key[i] = ~float_key(score[static_row[b + i]]);
-        s_acc[2 * i] = s_acc[2 * i + 1] = 0ull;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < len; i += BLK) {
-        const RankRun r = runs[run_of[b + i]];
-        const int row = static_row[b + i], at = r.begin - b + rows_before(s_key, r.begin - b, r.end - b, s_key[i], i);
-        s_row[at] = row - b;
-        s_score[at] = score[row];
-        sorted[b + at] = row;
+                                                             int *__restrict__ sorted, GHPair *__restrict__ gh) {
+    extern __shared__ unsigned long long s_acc[];  // [2 most] by row
+    unsigned *s_key = reinterpret_cast<unsigned *>(s_acc + 2 * most);  // by position of static_row
+    int *s_row = reinterpret_cast<int *>(s_key + most);                // by position of the order, within the group
+    float *s_score = reinterpret_cast<float *>(s_row + most);
+    const int g = which != nullptr ? which[blockIdx.x] : (int)blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
+    if (len > most) return;
+    if (BLK == kLongGroupBlock) {  // (run, key, position) where the sums will be
+        static_assert(kRankCountSortMax <= 1 << 12, "positions of a group in 12 bits");
+        const int count = keys_to_sort(len);
+        for (int i = threadIdx.x; i < count; i += BLK)
+            s_acc[i] = i < len ? (unsigned long long)(run_of[b + i] - b) << 44 | (unsigned long long)~float_key(score[static_row[b + i]]) << 12 | (unsigned)i : ~0ull;
+        __syncthreads();
+        sort_keys<BLK>(s_acc, count);
+        for (int at = threadIdx.x; at < len; at += BLK) {
+            const int row = static_row[b + (int)(s_acc[at] & 4095u)];
+            s_row[at] = row - b;
+            s_score[at] = score[row];
+            sorted[b + at] = row;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < len; i += BLK) s_acc[2 * i] = s_acc[2 * i + 1] = 0ull;
+    } else {
+        for (int i = threadIdx.x; i < len; i += BLK) {
+            s_key[i] = ~float_key(score[static_row[b + i]]);
+            s_acc[2 * i] = s_acc[2 * i + 1] = 0ull;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < len; i += BLK) {
+            const RankRun r = runs[run_of[b + i]];
+            const int row = static_row[b + i], at = r.begin - b + rows_before(s_key, r.begin - b, r.end - b, s_key[i], i);
+            s_row[at] = row - b;
+            s_score[at] = score[row];
+            sorted[b + at] = row;
+        }
     }
     __syncthreads();
     for (int i = threadIdx.x; i < len; i += BLK) {
@@ -448,7 +503,15 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, 
     upload(d_gptr_, gptr.data(), sizeof(int) * gptr.size());
     sorter_.alloc(n_);
     longest_ = longest;
-    if (short_groups_) setup_short_groups(longest);
+    std::vector<int> wide;  // (read by the copy until the set-up has waited)
+    if (short_groups_) {
+        for (int g = 0; g < n_groups_; ++g)
+            if (group[g] > kMiddleGroup) wide.push_back(g);
+        n_wide_ = (int)wide.size();
+        d_wide_ = dalloc<int>(wide.size());
+        upload(d_wide_, wide.data(), sizeof(int) * wide.size());
+        setup_short_groups(longest);
+    }
     else setup_groups(y, gptr);
     TGBM_CHECK(!ndcg || idcg_valid_, "rank:ndcg needs labels in 0..30");  // (small non-negative integers: 1 << label)
 }
@@ -577,15 +640,14 @@ void RankContext::gradient(const float *d_score, GHPair *d_gh, unsigned seed, bo
         last_cur_ = 0;
         have_metric_order_ = false;
         static LdsOptIn opt_in;
-        const size_t lds = (size_t)longest_ * kRankGroupBytes;
         const float *idcg = ndcg_ ? d_idcg_ : nullptr;
-        if (lds > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_rank_gradient_group<kLongGroupBlock>)});
-#define TGBM_RANK_GRADIENT(BLK)                                                                                                        \
-    k_rank_gradient_group<BLK><<<n_groups_, BLK, lds, stream_>>>(d_gptr_, d_score, d_y_, d_static_row_, d_run_of_, d_runs_, idcg, seed, \
-                                                                 longest_, sorter_.vals[0], d_gh)
-        if (longest_ <= kShortGroup) TGBM_RANK_GRADIENT(kShortGroup);
-        else if (longest_ <= kMiddleGroup) TGBM_RANK_GRADIENT(kSetupBlock);
-        else TGBM_RANK_GRADIENT(kLongGroupBlock);
+        if (longest_ * kRankGroupBytes > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_rank_gradient_group<kLongGroupBlock>)});
+#define TGBM_RANK_GRADIENT(BLK, GROUPS, WHICH, MOST)                                                                                \
+    k_rank_gradient_group<BLK><<<GROUPS, BLK, (MOST) * kRankGroupBytes, stream_>>>(WHICH, MOST, d_gptr_, d_score, d_y_, d_static_row_, \
+                                                                                  d_run_of_, d_runs_, idcg, seed, sorter_.vals[0], d_gh)
+        if (longest_ <= kShortGroup) TGBM_RANK_GRADIENT(kShortGroup, n_groups_, nullptr, longest_);
+        else if (n_wide_ < n_groups_) TGBM_RANK_GRADIENT(kSetupBlock, n_groups_, nullptr, std::min(longest_, kMiddleGroup));
+        if (n_wide_ > 0) TGBM_RANK_GRADIENT(kLongGroupBlock, n_wide_, d_wide_, longest_);
 #undef TGBM_RANK_GRADIENT
         return;
     }
@@ -612,11 +674,11 @@ void RankContext::metric(int kind, const float *d_score, float *d_out) {
     const int grid = grid_for(n_);
     int cur = 0;
     if (short_groups_) {
-        const size_t lds = (size_t)longest_ * sizeof(unsigned);
-#define TGBM_RANK_ORDER(BLK) k_rank_order_group<BLK><<<n_groups_, BLK, lds, stream_>>>(d_gptr_, d_score, sorter_.vals[0])
-        if (longest_ <= kShortGroup) TGBM_RANK_ORDER(kShortGroup);
-        else if (longest_ <= kMiddleGroup) TGBM_RANK_ORDER(kSetupBlock);
-        else TGBM_RANK_ORDER(kLongGroupBlock);
+#define TGBM_RANK_ORDER(BLK, GROUPS, WHICH, MOST) \
+    k_rank_order_group<BLK><<<GROUPS, BLK, keys_to_sort(MOST) * sizeof(unsigned long long), stream_>>>(WHICH, MOST, d_gptr_, d_score, sorter_.vals[0])
+        if (longest_ <= kShortGroup) TGBM_RANK_ORDER(kShortGroup, n_groups_, nullptr, longest_);
+        else if (n_wide_ < n_groups_) TGBM_RANK_ORDER(kSetupBlock, n_groups_, nullptr, std::min(longest_, kMiddleGroup));
+        if (n_wide_ > 0) TGBM_RANK_ORDER(kLongGroupBlock, n_wide_, d_wide_, longest_);
 #undef TGBM_RANK_ORDER
     } else {
         k_rank_metric_keys<<<grid, kBlock, 0, stream_>>>(n_, d_group_of_, d_score, sorter_.keys[0], sorter_.vals[0]);
