@@ -1243,12 +1243,22 @@ __global__ __launch_bounds__(256) void k_table_setup(SparsePass sp, CsrBins bins
     for (int a = threadIdx.x; a < stop; a += 256) {
         const int r = a < m ? bins.csc_row[v0 + a] : 0;
         row[at + a] = r;
-        table_bin[at + a] = a < m ? (unsigned short)(bins.csc_bin[v0 + a] - task_bin0[f]) : (unsigned short)kTableEmpty;
+        table_bin[at + a] = a < m ? (unsigned short)(bins.csc_bin[v0 + a] - task_bin0[i]) : (unsigned short)kTableEmpty;
         if (spread && a < wide) {
             spread_row[(size_t)list * kSpreadGroup + a] = (unsigned short)(r & (kSpreadRows - 1));
             if (a % kSpreadGroup == 0) spread_place[list + a / kSpreadGroup] = (unsigned)((sp.n_rare_places + at + a) / kSpreadGroup);
         }
     }
+}
+
+// table_first from the table features' places. The others' are not read, and the host does not make them: 2 M features of three values
+// 57.7 ms a call with one tree while it did, 43.0 without (49.3 before their values were spread).
+__global__ __launch_bounds__(256) void k_table_first(int n_table, const int *__restrict__ table_features, const int *__restrict__ place,
+                                                     int *__restrict__ table_first) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_table) return;
+    table_first[table_features[i]] = place[i];
+    table_first[table_features[i] + 1] = place[i + 1];  // (a table feature's own, if it is one)
 }
 
 // Groups of four places that the values of a task take in every row block.
@@ -1338,6 +1348,10 @@ void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &s
     if (sp.n_rare_tasks > 0) k_rare_count<<<sp.n_rare_tasks, 256, 0, s>>>(sp, bins, count);
     if (sp.n_table_features > 0)
         k_table_count<<<dim3((sp.n_table_features + 255) / 256, sp.n_spread), 256, 0, s>>>(sp, bins, count);
+}
+
+void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *place, int *table_first) {
+    if (n_table > 0) k_table_first<<<(n_table + 255) / 256, 256, 0, s>>>(n_table, table_features, place, table_first);
 }
 
 void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,

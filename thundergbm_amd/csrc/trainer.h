@@ -144,7 +144,7 @@ class Trainer {
     int hist_cap_level_ = -1;       // first level with more nodes than the histogram arena holds (-1: none)
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
     long sparse_rare_most_ = 0;  // a feature with more stored values is served through tables
-    int *d_task_bin0_ = nullptr;  // [F] sparse level pass: first bin of the table task that a feature belongs to
+    int *d_task_bin0_ = nullptr;  // [n_table_features] sparse level pass: first bin of the feature's table task
     long rare_tile_ = 0;         // values per task of the others at most
     bool sparse_feature_in_tables(int f);
     bool gradient_words_wanted() const;

@@ -955,7 +955,7 @@ bool Trainer::sparse_feature_in_tables(int f) {
 // task_values values, a feature with more than kSparseTaskValues cut into chunks (tasks of their own) whose tables
 // k_sparse_big adds up.
 void Trainer::build_sparse_tasks() {
-    std::vector<int> fvb(F_ + 1, 0), first(F_ + 1, 0), task_bin0(F_, 0), table_features;
+    std::vector<int> fvb(F_ + 1, 0), table_features, first, task_bin0;  // (the last three by table feature: of 2 M features few are)
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
     (void)is_table(0);  // (decides whether values are spread)
     // places of a feature or task: its values, and up to three nobody's in every row block
@@ -963,22 +963,23 @@ void Trainer::build_sparse_tasks() {
         const long blocks = std::min<long>(std::max(1, sp_.n_spread), values);
         return (values + (kSpreadGroup - 1) * blocks + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
     };
-    long table_places = 0;
+    long table_places = 0, table_values = 0;
+    sp_.max_table_bins = 0;
     for (int f = 0; f < F_; ++f) {
         fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
-        first[f] = (int)table_places;
         if (is_table(f)) {
             table_features.push_back(f);
+            first.push_back((int)table_places);
             table_places += places_of(cuts_.feature_nnz[f]);
+            table_values += cuts_.feature_nnz[f];
+            sp_.max_table_bins = std::max(sp_.max_table_bins, h_cut_row_ptr_[f + 1] - h_cut_row_ptr_[f]);
         }
     }
-    first[F_] = (int)table_places;
+    first.push_back((int)table_places);
     TGBM_CHECK(table_places < (1l << 31) - 16, "%ld places for the values of the frequent features", table_places);
     // A task serves its features one after the other, about 12 us each at 128 nodes: where all tasks together do not fill the
     // chip they are smaller (200 k x 100 k, depth 8, 67 tasks of 32768 values: 1.48 ms a tree, a thousandth of the values
     // each: 1.05; 1 M rows: 2.63 -> 2.43).
-    long table_values = 0;
-    for (int f = 0; f < F_; ++f) table_values += is_table(f) ? cuts_.feature_nnz[f] : 0;
     const long task_values = std::min<long>(kSparseTaskValues, std::max<long>(kRareLeast, table_values / kSparseTasks));
     std::vector<SparseTask> tasks;
     std::vector<SparseBig> big;
@@ -987,9 +988,6 @@ void Trainer::build_sparse_tasks() {
     std::vector<int2> rare_meta;
     std::vector<int> feat_slot(F_, -1);
     int n_small = 0, n_partial = 0, max_big_bins = 0;
-    sp_.max_table_bins = 0;
-    for (int q = 0; q < F_; ++q)
-        if (is_table(q)) sp_.max_table_bins = std::max(sp_.max_table_bins, h_cut_row_ptr_[q + 1] - h_cut_row_ptr_[q]);
     int f = 0;
     while (f < F_) {
         const long m = cuts_.feature_nnz[f];
@@ -1005,11 +1003,12 @@ void Trainer::build_sparse_tasks() {
             SparseBig b;
             b.feature = f;
             b.slot_begin = n_partial;
-            for (int v = first[f]; v < first[f + 1]; v += kSparseTaskValues) {
-                SparseTask t{f, f + 1, v, std::min(first[f + 1], v + kSparseTaskValues), -1, n_partial++};
+            const int end = first[task_bin0.size() + 1];
+            for (int v = first[task_bin0.size()]; v < end; v += kSparseTaskValues) {
+                SparseTask t{f, f + 1, v, std::min(end, v + kSparseTaskValues), -1, n_partial++};
                 tasks.push_back(t);
             }
-            task_bin0[f] = h_cut_row_ptr_[f];
+            task_bin0.push_back(h_cut_row_ptr_[f]);
             b.slot_end = n_partial;
             b.cand_slot = -1;  // numbered below
             big.push_back(b);
@@ -1024,8 +1023,10 @@ void Trainer::build_sparse_tasks() {
             vals += cuts_.feature_nnz[fe];
             ++fe;
         }
-        for (int q = f; q < fe; ++q) feat_slot[q] = n_small, task_bin0[q] = h_cut_row_ptr_[f];
-        SparseTask t{f, fe, first[f], first[fe], n_small++, -1};
+        const int begin = first[task_bin0.size()];
+        for (int q = f; q < fe; ++q) feat_slot[q] = n_small;
+        task_bin0.insert(task_bin0.end(), (size_t)(fe - f), h_cut_row_ptr_[f]);
+        SparseTask t{f, fe, begin, first[task_bin0.size()], n_small++, -1};
         tasks.push_back(t);
         f = fe;
     }
@@ -1078,7 +1079,7 @@ void Trainer::build_sparse_tasks() {
     int *d_rare_fid = dalloc<int>(rare_fid.size());
     int2 *d_rare_meta = dalloc<int2>(rare_meta.size());
     int *d_feat_slot = dalloc<int>(feat_slot.size());
-    int *d_fvb = dalloc<int>(fvb.size()), *d_first = dalloc<int>(first.size()), *d_table = dalloc<int>(table_features.size());
+    int *d_fvb = dalloc<int>(fvb.size()), *d_first = dalloc<int>((size_t)F_ + 1), *d_place = nullptr, *d_table = dalloc<int>(table_features.size());
     d_task_bin0_ = dalloc<int>(task_bin0.size());
     upload(stream_, d_tasks, tasks.data(), tasks.size());
     upload(stream_, d_big, big.data(), big.size());
@@ -1087,10 +1088,13 @@ void Trainer::build_sparse_tasks() {
     upload(stream_, d_rare_meta, rare_meta.data(), rare_meta.size());
     upload(stream_, d_feat_slot, feat_slot.data(), feat_slot.size());
     upload(stream_, d_fvb, fvb.data(), fvb.size());
-    upload(stream_, d_first, first.data(), first.size());
+    device_alloc_to(d_place, sizeof(int) * first.size());
+    upload(stream_, d_place, first.data(), first.size());
     upload(stream_, d_table, table_features.data(), table_features.size());
     upload(stream_, d_task_bin0_, task_bin0.data(), task_bin0.size());
+    launch_table_first(stream_, (int)table_features.size(), d_table, d_place, d_first);
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
+    device_free(d_place);
     sp_.tasks = d_tasks;
     sp_.big = d_big;
     sp_.rare_tasks = d_rare;
