@@ -48,6 +48,11 @@ def test_slices_of_a_scoring_call(run_native):
     run_native("score_slices.cpp")
 
 
+def test_places_of_frequent_features(run_native):
+    """Sparse data with close to 2^31 values has more places than an int counts; what counts them must not overflow."""
+    run_native("table_places.cpp")
+
+
 @pytest.fixture(scope="module")
 def transfers(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("native") / "transfer")

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "common.h"
+#include "table_places.h"
 
 #define HIP_CHECK(expr)                                                                              \
     do {                                                                                             \
@@ -237,11 +238,10 @@ struct CsrBins {
 constexpr int kSparseCells = 8192;      // (node, bin) cells of 16 bytes an LDS table holds
 constexpr int kSparseMaxLevelNodes = 1024;  // deepest level the pass serves (depth <= 11)
 constexpr int kSparseBatchFeatures = 2047;  // features whose tables share one LDS batch at most
-constexpr int kSparseTaskValues = 32768;    // stored values per task at most (and per chunk of a big feature)
 constexpr int kSparseTasks = 1024;          // smaller tasks where there would be fewer than that
 struct SparseTask {
     int f_begin, f_end;  // features [f_begin, f_end) (a chunk task: one feature)
-    int v_begin, v_end;  // places of its values (SparsePass::table_bin), multiples of kSpreadGroup
+    int g_begin, g_end;  // groups of kSpreadGroup places of its values (SparsePass::table_bin)
     int cand_slot;       // candidate slot the task fills, -1: a chunk (its feature's slot is filled by k_sparse_big)
     int partial_slot;    // chunk: where its table goes in SparsePass::partial, else -1
 };
@@ -270,7 +270,6 @@ constexpr int kRareFeatShift = 20;
 // in table_bin: nobody's).
 constexpr int kSpreadLogRows = 15;
 constexpr int kSpreadRows = 1 << kSpreadLogRows;
-constexpr int kSpreadGroup = 4;
 constexpr int kSpreadLevel = 7;       // deepest level with its nodes in a byte (all ones: the row has come to rest above)
 constexpr int kSpreadBlocks = 341;    // (more leave less than three quarters of a tile to values)
 // Stored values from which on they are spread: a launch more a level, and less time per value. ms a tree of depth 8, looked up / spread:
@@ -319,7 +318,7 @@ struct SparsePass {
     const int *table_features = nullptr;  // [n_table_features]
     int n_table_features = 0;
     size_t n_table_places = 0;            // (a multiple of 16)
-    const int *table_first = nullptr;     // [F + 1] first place of every feature's values (other features: none)
+    const int *table_first = nullptr;     // [F + 1] first group of places of every feature's values (other features: none)
     const unsigned short *table_bin = nullptr;  // [n_table_places] bin, counted from the first one of the feature's task
     const int *table_row = nullptr;             // [n_table_places]
     // [n_sets][n_table_places] the gradient pair of every value's row, left there by the pass of level 0: those below then stream it
@@ -586,7 +585,7 @@ void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *
 void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count);
 void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
                        int *places, uint8_t *group, unsigned short *spread_row, unsigned *spread_place);
-void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *place /* [n_table + 1] */, int *table_first);
+void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *first /* [n_table + 1] */, int *table_first);
 void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,
                         unsigned short *spread_row, unsigned *spread_place);
 // The rows' words of a tree (TreeBuffers::row_word).

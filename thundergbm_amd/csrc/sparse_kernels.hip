@@ -134,7 +134,7 @@ struct SpShared {
     unsigned long long key[kSparseMaxLevelNodes];  // best candidate of every node over the task's features so far
     unsigned char ok[kSparseMaxLevelNodes];        // node is valid
     int fbin[kSparseBatchFeatures + 2];            // first bin (relative to the batch) of every feature of the batch
-    int ctl[8];  // batch: first feature, end feature, first bin, bins, node range begin, nodes in range, first value, end value
+    int ctl[8];  // batch: first feature, end feature, first bin, bins, node range begin, nodes in range, first group, end group
 };
 
 // Level-wide state every task starts from: node sums and validity into LDS, and the best keys that other tasks have published:
@@ -295,12 +295,12 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
             sh.ctl[2] = crp[f];
             sh.ctl[3] = kf;
             sh.ctl[5] = nn;
-            sh.ctl[6] = max(task.v_begin, sp.table_first[f]);
-            sh.ctl[7] = min(task.v_end, sp.table_first[fb]);
+            sh.ctl[6] = max(task.g_begin, sp.table_first[f]);
+            sh.ctl[7] = min(task.g_end, sp.table_first[fb]);
         }
         __syncthreads();
         const int fa = sh.ctl[0], fb = sh.ctl[1], bin0 = sh.ctl[2], nbins = sh.ctl[3], nn_max = sh.ctl[5];
-        const int v0 = sh.ctl[6], v1 = sh.ctl[7];
+        const int g0 = sh.ctl[6], g1 = sh.ctl[7];
         const int nf = fb - fa;
         for (int i = threadIdx.x; i <= nf; i += kSpBlock) sh.fbin[i] = crp[fa + i] - bin0;
         for (int n0 = 0; n0 < nl; n0 += nn_max) {
@@ -313,8 +313,8 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
             // repeats and is skipped below -, so that a stage's loads are issued together instead of one after the other)
             constexpr int U = DEEP ? 2 : 1, V = kSpreadGroup;
             static_assert(V == 4, "a group's loads");
-            const int q1 = v1 / V, bin_shift = bin0 - task_bin0;
-            for (int q0 = v0 / V + (int)threadIdx.x; q0 < q1; q0 += kSpBlock * U) {
+            const int bin_shift = bin0 - task_bin0;
+            for (int q0 = g0 + (int)threadIdx.x; q0 < g1; q0 += kSpBlock * U) {
                 unsigned long long bin4[U];
                 unsigned node4[U];       // (kSpreadNodes)
                 int x[U][V];             // (kRowNodes)
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
                 int row[U][V];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int q = min(q0 + u * kSpBlock, q1 - 1);
+                    const int q = min(q0 + u * kSpBlock, g1 - 1);
                     bin4[u] = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(sp.table_bin) + q);
                     if (NODES == kSpreadNodes) node4[u] = __builtin_nontemporal_load(nodes + q);
                     if ((NODES != kSpreadNodes && NODES != kRootWords) || !copied) {
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         const int q = q0 + u * kSpBlock;
-                        if (q >= q1) continue;
+                        if (q >= g1) continue;
                         if (WORDS) {
                             reinterpret_cast<float4 *>(sp.table_gh)[q] = make_float4(g[u][0], g[u][1], g[u][2], g[u][3]);
                         } else {
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
                     for (int k = 0; k < V; ++k) {
                         const int bin = (int)(bin4[u] >> 16 * k & 0xffffu), of = (int)(node4[u] >> 8 * k & 0xffu);
                         const int at = NODES == kRootNode || NODES == kRootWords ? 0 : NODES == kRowNodes ? x[u][k] : of == 0xff ? -1 : of - n0;
-                        if (q0 + u * kSpBlock < q1 && (unsigned)at < (unsigned)nn && bin != (int)kTableEmpty) {
+                        if (q0 + u * kSpBlock < g1 && (unsigned)at < (unsigned)nn && bin != (int)kTableEmpty) {
                             const GHPair p = WORDS ? pair_from_word(sp.gh_objective, __float_as_uint(g[u][k])) : GHPair{g[u][k], h[u][k]};
                             const long long gq = round_to_ll(p.g * scale_g), hq = round_to_ll(p.h * scale_h);
                             unsigned long long *cell = reinterpret_cast<unsigned long long *>(cells + at * nbins + (bin - bin_shift));
@@ -1227,20 +1227,21 @@ __global__ __launch_bounds__(256) void k_table_setup(SparsePass sp, CsrBins bins
                                                     unsigned *__restrict__ spread_place) {
     const int i = blockIdx.x, f = sp.table_features[i], b = blockIdx.y;
     const bool spread = sp.n_spread > 0;
-    int v0 = sp.feat_val_begin[f], v1 = sp.feat_val_begin[f + 1], at = sp.table_first[f];
+    int v0 = sp.feat_val_begin[f], v1 = sp.feat_val_begin[f + 1], group = sp.table_first[f];
     unsigned list = 0;
     if (spread) {
         const unsigned *begin = sp.spread_begin + sp.n_rare_tasks + i;
-        for (int a = 0; a < b; ++a) at += (int)(begin[(size_t)a * sp.n_lists + 1] - begin[(size_t)a * sp.n_lists]) * kSpreadGroup;
+        for (int a = 0; a < b; ++a) group += (int)(begin[(size_t)a * sp.n_lists + 1] - begin[(size_t)a * sp.n_lists]);
         list = begin[(size_t)b * sp.n_lists];
         const long r0 = (long)b << kSpreadLogRows;
         const int end = v1;
         v1 = first_value_of(bins.csc_row, v0, end, r0 + kSpreadRows);
         v0 = first_value_of(bins.csc_row, v0, end, r0);
     }
-    const int m = v1 - v0, wide = (m + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
-    const int stop = b + 1 == (int)gridDim.y ? sp.table_first[f + 1] - at : wide;
-    for (int a = threadIdx.x; a < stop; a += 256) {
+    const size_t at = (size_t)group * kSpreadGroup;
+    const long m = v1 - v0, wide = (m + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
+    const long stop = b + 1 == (int)gridDim.y ? (long)(sp.table_first[f + 1] - group) * kSpreadGroup : wide;
+    for (long a = threadIdx.x; a < stop; a += 256) {
         const int r = a < m ? bins.csc_row[v0 + a] : 0;
         row[at + a] = r;
         table_bin[at + a] = a < m ? (unsigned short)(bins.csc_bin[v0 + a] - task_bin0[i]) : (unsigned short)kTableEmpty;
@@ -1251,14 +1252,14 @@ __global__ __launch_bounds__(256) void k_table_setup(SparsePass sp, CsrBins bins
     }
 }
 
-// table_first from the table features' places. The others' are not read, and the host does not make them: 2 M features of three values
+// table_first from the table features' groups. The others' are not read, and the host does not make them: 2 M features of three values
 // 57.7 ms a call with one tree while it did, 43.0 without (49.3 before their values were spread).
-__global__ __launch_bounds__(256) void k_table_first(int n_table, const int *__restrict__ table_features, const int *__restrict__ place,
+__global__ __launch_bounds__(256) void k_table_first(int n_table, const int *__restrict__ table_features, const int *__restrict__ first,
                                                      int *__restrict__ table_first) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n_table) return;
-    table_first[table_features[i]] = place[i];
-    table_first[table_features[i] + 1] = place[i + 1];  // (a table feature's own, if it is one)
+    table_first[table_features[i]] = first[i];
+    table_first[table_features[i] + 1] = first[i + 1];  // (a table feature's own, if it is one)
 }
 
 // Groups of four places that the values of a task take in every row block.
@@ -1350,8 +1351,8 @@ void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &s
         k_table_count<<<dim3((sp.n_table_features + 255) / 256, sp.n_spread), 256, 0, s>>>(sp, bins, count);
 }
 
-void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *place, int *table_first) {
-    if (n_table > 0) k_table_first<<<(n_table + 255) / 256, 256, 0, s>>>(n_table, table_features, place, table_first);
+void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *first, int *table_first) {
+    if (n_table > 0) k_table_first<<<(n_table + 255) / 256, 256, 0, s>>>(n_table, table_features, first, table_first);
 }
 
 void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,

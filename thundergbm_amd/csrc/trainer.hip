@@ -958,25 +958,20 @@ void Trainer::build_sparse_tasks() {
     std::vector<int> fvb(F_ + 1, 0), table_features, first, task_bin0;  // (the last three by table feature: of 2 M features few are)
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
     (void)is_table(0);  // (decides whether values are spread)
-    // places of a feature or task: its values, and up to three nobody's in every row block
-    const auto places_of = [&](long values) {
-        const long blocks = std::min<long>(std::max(1, sp_.n_spread), values);
-        return (values + (kSpreadGroup - 1) * blocks + kSpreadGroup - 1) / kSpreadGroup * kSpreadGroup;
-    };
-    long table_places = 0, table_values = 0;
+    long table_groups = 0, table_values = 0;
     sp_.max_table_bins = 0;
     for (int f = 0; f < F_; ++f) {
         fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
         if (is_table(f)) {
             table_features.push_back(f);
-            first.push_back((int)table_places);
-            table_places += places_of(cuts_.feature_nnz[f]);
+            first.push_back((int)table_groups);
+            table_groups += groups_of(cuts_.feature_nnz[f], sp_.n_spread);
             table_values += cuts_.feature_nnz[f];
             sp_.max_table_bins = std::max(sp_.max_table_bins, h_cut_row_ptr_[f + 1] - h_cut_row_ptr_[f]);
         }
     }
-    first.push_back((int)table_places);
-    TGBM_CHECK(table_places < (1l << 31) - 16, "%ld places for the values of the frequent features", table_places);
+    first.push_back((int)table_groups);
+    TGBM_CHECK(table_groups < 1l << 31, "%ld groups of values of the frequent features", table_groups);
     // A task serves its features one after the other, about 12 us each at 128 nodes: where all tasks together do not fill the
     // chip they are smaller (200 k x 100 k, depth 8, 67 tasks of 32768 values: 1.48 ms a tree, a thousandth of the values
     // each: 1.05; 1 M rows: 2.63 -> 2.43).
@@ -1003,10 +998,11 @@ void Trainer::build_sparse_tasks() {
             SparseBig b;
             b.feature = f;
             b.slot_begin = n_partial;
-            const int end = first[task_bin0.size() + 1];
-            for (int v = first[task_bin0.size()]; v < end; v += kSparseTaskValues) {
-                SparseTask t{f, f + 1, v, std::min(end, v + kSparseTaskValues), -1, n_partial++};
+            int begin = first[task_bin0.size()];
+            for (int end : chunk_ends(begin, first[task_bin0.size() + 1])) {
+                SparseTask t{f, f + 1, begin, end, -1, n_partial++};
                 tasks.push_back(t);
+                begin = end;
             }
             task_bin0.push_back(h_cut_row_ptr_[f]);
             b.slot_end = n_partial;
@@ -1047,7 +1043,7 @@ void Trainer::build_sparse_tasks() {
         while (e < rare_fid.size() && e - i < (size_t)kRareFeatures && (e == i || vals + cuts_.feature_nnz[rare_fid[e]] <= tile_values))
             vals += cuts_.feature_nnz[rare_fid[e++]];
         rare_tasks.push_back(RareTask{(int)places, (int)vals, (int)i, (int)(e - i)});
-        places += sp_.n_spread > 0 ? places_of(vals) : vals;
+        places += sp_.n_spread > 0 ? groups_of(vals, sp_.n_spread) * kSpreadGroup : vals;
         i = e;
     }
     // as few rounds of resident workgroups as the tasks per workgroup allow
@@ -1059,7 +1055,7 @@ void Trainer::build_sparse_tasks() {
     next_slot += n_groups;
     // the longest tasks first: they decide when the level is done. A feature's search at deep levels takes about as long as adding up
     // 16 000 values (a chunk has none).
-    const auto length = [](const SparseTask &t) { return t.v_end - t.v_begin + (t.cand_slot >= 0 ? 16000 * (long)(t.f_end - t.f_begin) : 0); };
+    const auto length = [](const SparseTask &t) { return (long)(t.g_end - t.g_begin) * kSpreadGroup + (t.cand_slot >= 0 ? 16000 * (long)(t.f_end - t.f_begin) : 0); };
     std::stable_sort(tasks.begin(), tasks.end(), [&](const SparseTask &a, const SparseTask &b) { return length(a) > length(b); });
     sp_.n_tasks = (int)tasks.size();
     sp_.n_big = (int)big.size();
@@ -1068,7 +1064,7 @@ void Trainer::build_sparse_tasks() {
     sp_.n_rare = n_rare;
     sp_.n_rare_places = ((size_t)places + 15) / 16 * 16;
     sp_.n_table_features = (int)table_features.size();
-    sp_.n_table_places = ((size_t)table_places + 15) / 16 * 16;
+    sp_.n_table_places = ((size_t)table_groups * kSpreadGroup + 15) / 16 * 16;
     sp_.n_lists = n_rt + sp_.n_table_features;
     sp_.n_cand_slots = std::max(1, next_slot);
     sp_.n_partial_slots = n_partial;
@@ -1079,7 +1075,7 @@ void Trainer::build_sparse_tasks() {
     int *d_rare_fid = dalloc<int>(rare_fid.size());
     int2 *d_rare_meta = dalloc<int2>(rare_meta.size());
     int *d_feat_slot = dalloc<int>(feat_slot.size());
-    int *d_fvb = dalloc<int>(fvb.size()), *d_first = dalloc<int>((size_t)F_ + 1), *d_place = nullptr, *d_table = dalloc<int>(table_features.size());
+    int *d_fvb = dalloc<int>(fvb.size()), *d_first = dalloc<int>((size_t)F_ + 1), *d_groups = nullptr, *d_table = dalloc<int>(table_features.size());
     d_task_bin0_ = dalloc<int>(task_bin0.size());
     upload(stream_, d_tasks, tasks.data(), tasks.size());
     upload(stream_, d_big, big.data(), big.size());
@@ -1088,13 +1084,13 @@ void Trainer::build_sparse_tasks() {
     upload(stream_, d_rare_meta, rare_meta.data(), rare_meta.size());
     upload(stream_, d_feat_slot, feat_slot.data(), feat_slot.size());
     upload(stream_, d_fvb, fvb.data(), fvb.size());
-    device_alloc_to(d_place, sizeof(int) * first.size());
-    upload(stream_, d_place, first.data(), first.size());
+    device_alloc_to(d_groups, sizeof(int) * first.size());
+    upload(stream_, d_groups, first.data(), first.size());
     upload(stream_, d_table, table_features.data(), table_features.size());
     upload(stream_, d_task_bin0_, task_bin0.data(), task_bin0.size());
-    launch_table_first(stream_, (int)table_features.size(), d_table, d_place, d_first);
+    launch_table_first(stream_, (int)table_features.size(), d_table, d_groups, d_first);
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
-    device_free(d_place);
+    device_free(d_groups);
     sp_.tasks = d_tasks;
     sp_.big = d_big;
     sp_.rare_tasks = d_rare;
