@@ -75,3 +75,35 @@ def test_an_idle_process_holds_little_and_can_give_it_back():
     assert 0 < kept <= total // 32
     T.release_memory()
     assert free - memory()[0] < kept // 4
+
+
+@pytest.mark.parametrize("filled,more", [(0.9, 0.5), (0.99, 1.5)])
+def test_a_dense_matrix_goes_once_its_values_are_grouped(filled, more):
+    """Beside what the same data takes as CSR a dense call needs its matrix: with empty cells past a 32nd (of up to 256 columns) until the
+    values are grouped, when its block becomes one of the sort's, else until the cells are sorted."""
+    import ctypes as C
+    import scipy.sparse as sp
+    import thundergbm_amd as T
+    D.warm_up(T)
+    hip = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    rng = np.random.default_rng(3)
+    X = rng.standard_normal((400_000, 40)).astype(np.float32)
+    X[rng.random(X.shape) >= filled] = 0
+    y = X[:, 0] + X[:, 1] ** 2
+
+    def kept(data):  # (the blocks of a call are kept until they are given back: the most that it held at a time, by size)
+        T.release_memory()
+        before = free()
+        T.TGBMRegressor(depth=3, n_trees=1).fit(data, y)
+        return before - free()
+
+    as_csr = sp.csr_matrix(X)
+    kept(as_csr)
+    extra = kept(X) - kept(as_csr)
+    assert extra < more * X.nbytes, extra

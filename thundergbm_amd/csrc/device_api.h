@@ -638,13 +638,20 @@ struct DeviceCuts {
     int n_bins = 0;
     std::vector<long> feature_nnz;  // host: stored values per feature
 };
-// full_rows: every row stores every column, in order (d_val is a row-major matrix). cells: the matrix that the values come from, if it
-// is still there
+// full_rows: every row stores every column, in order (d_val is a row-major matrix). cells: the matrix that the values come from, where
+// its cells are sorted along
 struct DenseCells {
     const float *x;
     int n, columns;
     bool minus_zero_is_stored;
 };
+// Are the cells that hold no value sorted along with the others (build_cut_points)? That costs less than grouping the values: on wide
+// data, where they would be sorted as 64-bit pairs, up to a quarter of the cells, else up to a 32nd (all passes: 35 M cells of 700
+// features 1.9 -> 0.95 ms).
+inline bool sorts_cells_along(int n, int F, long nnz) {
+    const long all = (long)n * F;
+    return nnz > 0 && n >= 1024 && all - nnz <= all / (F > 256 ? 4 : 32);
+}
 DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin,
                             bool full_rows = false, const DenseCells *cells = nullptr);
 // (at most 256 features, full rows, or the cells)
@@ -770,9 +777,9 @@ struct DeviceCsr {
     int n_features = 1;  // largest column with a stored value + 1, at least 1
     float *cells = nullptr;  // see dense_to_csr
 };
-// Takes `x` over: it becomes the value array when every cell is stored, else it is freed, or (keep) handed back as `cells`.
-// Synchronises.
-DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored, bool keep = false);
+// Takes `x` over: it becomes the value array when every cell is stored, is handed back as `cells` where cut points are made of them
+// (for_cuts, sorts_cells_along), else it is freed. Synchronises.
+DeviceCsr dense_to_csr(hipStream_t s, int n, int columns, float *x, bool minus_zero_is_stored, bool for_cuts = false);
 
 // Prediction of the n rows that row_ptr addresses (entry offsets into col / val); out[t * out_stride + i] for
 // class tree t and row i, out_stride = 0 means n (a slice of a larger row set passes the whole set's size); adds to out.

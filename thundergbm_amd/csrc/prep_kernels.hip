@@ -579,12 +579,7 @@ int grid_for(size_t n, int cap = 8192) {
 // segments fill a quarter of their tiles; the rest by (feature, value) pairs.
 DeviceCuts build_cut_points(hipStream_t s, int F, long nnz, const float *d_val, const int *d_col, int max_num_bin,
                             bool full_rows, const DenseCells *cells) {
-    // Sorting the cells that hold no value along costs less than grouping the values: on wide data, where they would be sorted as
-    // 64-bit pairs, up to a quarter of the cells, else up to a 32nd (all passes: 35 M cells of 700 features 1.9 -> 0.95 ms).
-    if (cells != nullptr && nnz > 0 && cells->n >= 1024) {
-        const long all = (long)cells->n * F, empty = all - nnz;
-        if (empty <= all / (F > 256 ? 4 : 32)) return build_cut_points_by_feature(s, F, nnz, d_val, d_col, full_rows, max_num_bin, cells);
-    }
+    if (cells != nullptr) return build_cut_points_by_feature(s, F, nnz, d_val, d_col, full_rows, max_num_bin, cells);
     if (nnz > 0 && (F <= 256 || (full_rows && nnz / F >= 1024))) return build_cut_points_by_feature(s, F, nnz, d_val, d_col, full_rows, max_num_bin);
     DeviceCuts out;
     device_alloc_to(out.cut_row_ptr, sizeof(int) * (size_t)(F + 1));
@@ -771,7 +766,7 @@ __global__ __launch_bounds__(kBlock) void k_full_csr(int n, int C, int *__restri
     for (int i = blockIdx.x * kBlock + threadIdx.x; i <= n; i += gridDim.x * kBlock) row_ptr[i] = i * C;
 }
 
-DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz, bool keep) {
+DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz, bool for_cuts) {
     DeviceCsr out;
     const size_t cells = (size_t)n * C;
     TGBM_CHECK(n > 0 && C > 0 && cells < ((size_t)1 << 32), "dense input of %d x %d", n, C);
@@ -801,9 +796,9 @@ DeviceCsr dense_to_csr(hipStream_t s, int n, int C, float *x, bool mz, bool keep
     } else {
         device_alloc_to(out.val, sizeof(float) * (size_t)std::max(out.nnz, 1l));
         k_dense_compact<<<grid, kBlock, 0, s>>>(n, C, x, mz, out.row_ptr, out.val, out.col);
-        if (keep) {
+        if (for_cuts && sorts_cells_along(n, out.n_features, out.nnz)) {
             out.cells = x;
-        } else {
+        } else {  // (nothing else reads it: it would lie beside the sort's keys)
             HIP_CHECK(hipStreamSynchronize(s));
             device_free(x);
         }
