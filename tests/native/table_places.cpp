@@ -31,6 +31,20 @@ int main() {
                     groups = next;
                 }
             }
+    // Parts of the set-up: every value has one, and there are no more of them than features and values call for, however many row blocks
+    // there are (an ordinary feature of 10 M rows has a few values in each of 300, one that most rows store has them all in the one
+    // "block" of values that are not spread).
+    for (long all : {0l, 1l, 8191l, 8192l, 8193l, 12000000l, (1l << 31) - 1})
+        for (int features : {1, 7, 15000}) {
+            std::vector<TablePart> parts;
+            for (int f = 0; f < features; ++f) add_table_parts(parts, f, all / features + (f < all % features ? 1 : 0));
+            CHECK((long)parts.size() <= std::min<long>(features, all) + all / kTableSetupValues);
+            size_t at = 0;
+            for (int f = 0; f < features; ++f)
+                for (long v = 0, values = all / features + (f < all % features ? 1 : 0); v < values; v += kTableSetupValues, ++at)
+                    CHECK(at < parts.size() && parts[at].feature == f && parts[at].begin == v);
+            CHECK(at == parts.size());
+        }
     std::printf("ok\n");
     return 0;
 }

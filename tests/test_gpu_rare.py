@@ -162,3 +162,40 @@ def test_tables_whatever_form_their_values_have(T, objective, bins):
         for key in ("TGBM_LAYOUT", "TGBM_SPARSE_SPREAD", "TGBM_GH_WORD", "TGBM_SPARSE_GH_COPY"):
             os.environ.pop(key, None)
     assert all(r == runs[0] for r in runs)
+
+
+# Values of frequent features that several workgroups of the set-up give their places: a part's edge inside a group of four places, at a row
+# block's edge and next to a block without values; the levels' histograms against the bins themselves.
+@pytest.mark.parametrize("n", [40001, 100003])
+def test_frequent_features_in_parts(T, n):
+    counts = [min(k, n - 1) for k in (8191, 8192, 8193, 16384, 16390, 33000, n - 1, 70000)] + [900] * 130 + [20] * 10
+    val, rp, col, z = _by_feature(counts, n, 11)
+    if n > 65536:  # (nothing is stored in the rows of the second block)
+        keep = np.ones(len(col), bool)
+        keep[rp[32768]:rp[65536]] = False
+        rp = np.concatenate([[0], np.cumsum(keep)])[rp].astype(np.int32)
+        val, col = val[keep], col[keep]
+    runs = []
+    os.environ["TGBM_LAYOUT"] = "sparse"
+    try:
+        for spread in ("1", "0"):
+            os.environ["TGBM_SPARSE_SPREAD"] = spread
+            s = T.Session(val, rp, col, z.astype(np.float32), depth=5, n_trees=3, max_num_bin=63, learning_rate=0.5)
+            bins = s.global_bin_ids(rp, col)[0]
+            gh = np.ones((n, 2), np.float32)
+            gh[:, 0] = np.arange(n) % 7 - 3  # (whole numbers: the histograms are exact)
+            s.set("gh", gh)
+            s.tree_init(0)
+            s.find_split(0)
+            row = np.repeat(np.arange(n), np.diff(rp))
+            want = np.stack([np.bincount(bins, gh[row, k], minlength=s.n_bins) for k in (0, 1)], 1)
+            assert np.array_equal(s.level_hist(0)[0], want)
+            s.close()
+            s = T.Session(val, rp, col, z.astype(np.float32), depth=5, n_trees=3, max_num_bin=63, learning_rate=0.5)
+            s.boost(3)
+            runs.append((s.model().tobytes(), s.y_pred().tobytes()))
+            s.close()
+    finally:
+        os.environ.pop("TGBM_SPARSE_SPREAD", None)
+        del os.environ["TGBM_LAYOUT"]
+    assert runs[0] == runs[1]

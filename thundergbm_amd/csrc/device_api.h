@@ -581,13 +581,13 @@ void launch_sparse_cols(hipStream_t s, long nnz, const int *csc_bin, const int *
                         const int *cut_row_ptr, const int *col_of_feature, uint8_t *colbin, size_t col_stride);
 // Fills what SparsePass points to under the same names from the bin-major copy; the spread_* arrays where sp.n_spread > 0:
 // launch_spread_count leaves the groups of every (block, list) in `count` (their exclusive sums are spread_begin). task_bin0: [n_table_features] first
-// bin of the task that a table feature belongs to.
+// bin of the task that a table feature belongs to; parts: of their values (add_table_parts).
 void launch_spread_count(hipStream_t s, const CsrBins &bins, const SparsePass &sp, unsigned *count);
 void launch_rare_setup(hipStream_t s, const TreeBuffers &tb, const CsrBins &bins, const SparsePass &sp, int *row, unsigned *key,
                        int *places, uint8_t *group, unsigned short *spread_row, unsigned *spread_place);
 void launch_table_first(hipStream_t s, int n_table, const int *table_features, const int *first /* [n_table + 1] */, int *table_first);
-void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, const int *task_bin0, int *row, unsigned short *table_bin,
-                        unsigned short *spread_row, unsigned *spread_place);
+void launch_table_setup(hipStream_t s, const CsrBins &bins, const SparsePass &sp, int n_parts, const TablePart *parts, const int *task_bin0,
+                        int *row, unsigned short *table_bin, unsigned short *spread_row, unsigned *spread_place);
 // The rows' words of a tree (TreeBuffers::row_word).
 void launch_sparse_row_words(hipStream_t s, const TreeBuffers &tb, const GHPair *gh, int n_class);
 // Row-ordered passes over the row lists (one of dbins / cbins by tb.sparse). lookup_level: the level

@@ -23,4 +23,15 @@ inline std::vector<int> chunk_ends(int begin, int end) {
     return ends;
 }
 
+// What a workgroup of the set-up gives their places: up to so many values of a frequent feature, from the begin-th on. (Counted in values
+// and not in row blocks: a feature of 10 000 values has some in each of 300 blocks, one of 10 M may have them all in one.)
+constexpr int kTableSetupValues = 8192;
+struct TablePart {
+    int feature;  // among the frequent ones
+    int begin;
+};
+inline void add_table_parts(std::vector<TablePart> &parts, int feature, long values) {
+    for (long v = 0; v < values; v += kTableSetupValues) parts.push_back(TablePart{feature, (int)v});
+}
+
 }  // namespace tgbm

@@ -145,6 +145,8 @@ class Trainer {
     int sparse_bin0_owner_ = -2;    // -2: not looked up yet
     long sparse_rare_most_ = 0;  // a feature with more stored values is served through tables
     int *d_task_bin0_ = nullptr;  // [n_table_features] sparse level pass: first bin of the feature's table task
+    TablePart *d_table_parts_ = nullptr;  // [n_table_parts_] of their values, for the set-up
+    int n_table_parts_ = 0;
     long rare_tile_ = 0;         // values per task of the others at most
     bool sparse_feature_in_tables(int f);
     bool gradient_words_wanted() const;

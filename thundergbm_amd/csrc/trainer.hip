@@ -684,7 +684,7 @@ void Trainer::alloc_tree_buffers() {
         }
         int *table_row = dalloc<int>(sp_.n_table_places);
         unsigned short *table_bin = dalloc<unsigned short>(sp_.n_table_places);
-        launch_table_setup(stream_, csr_, sp_, d_task_bin0_, table_row, table_bin, spread_row, spread_place);
+        launch_table_setup(stream_, csr_, sp_, n_table_parts_, d_table_parts_, d_task_bin0_, table_row, table_bin, spread_row, spread_place);
         sp_.table_row = table_row;
         sp_.table_bin = table_bin;
         sp_.spread_row = spread_row;
@@ -958,11 +958,13 @@ void Trainer::build_sparse_tasks() {
     std::vector<int> fvb(F_ + 1, 0), table_features, first, task_bin0;  // (the last three by table feature: of 2 M features few are)
     auto is_table = [&](int f) { return sparse_feature_in_tables(f); };
     (void)is_table(0);  // (decides whether values are spread)
+    std::vector<TablePart> table_parts;
     long table_groups = 0, table_values = 0;
     sp_.max_table_bins = 0;
     for (int f = 0; f < F_; ++f) {
         fvb[f + 1] = fvb[f] + (int)cuts_.feature_nnz[f];
         if (is_table(f)) {
+            add_table_parts(table_parts, (int)table_features.size(), cuts_.feature_nnz[f]);
             table_features.push_back(f);
             first.push_back((int)table_groups);
             table_groups += groups_of(cuts_.feature_nnz[f], sp_.n_spread);
@@ -1088,6 +1090,9 @@ void Trainer::build_sparse_tasks() {
     upload(stream_, d_groups, first.data(), first.size());
     upload(stream_, d_table, table_features.data(), table_features.size());
     upload(stream_, d_task_bin0_, task_bin0.data(), task_bin0.size());
+    n_table_parts_ = (int)table_parts.size();
+    d_table_parts_ = dalloc<TablePart>(table_parts.size());
+    upload(stream_, d_table_parts_, table_parts.data(), table_parts.size());
     launch_table_first(stream_, (int)table_features.size(), d_table, d_groups, d_first);
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors go out of scope
     device_free(d_groups);
