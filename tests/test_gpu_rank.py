@@ -172,6 +172,13 @@ def test_rank_tables_of_short_groups(T, objective, labels, groups, monkeypatch):
     assert np.array_equal(got[0][0], got[1][0]) and got[0][2] == got[1][2]
 
 
+# The same where neighbours share a workgroup: many groups of one row, groups without rows first, last and between, packs that are full.
+@pytest.mark.parametrize("objective", ["rank:pairwise", "rank:ndcg"])
+@pytest.mark.parametrize("groups", [[1] * 1000, [0, 0, 5, 0, 123, 0, 1, 0], [128, 1, 127, 2, 129, 256, 3, 257, 1, 1], [40] * 30 + [0] + [7, 2] * 50, [64, 65] * 9])
+def test_rank_groups_that_share_a_workgroup(T, objective, groups, monkeypatch):
+    test_rank_tables_of_short_groups(T, objective, "few", groups, monkeypatch)
+
+
 def test_rank_gradient_is_bit_reproducible(T):
     (val, rp, col), y, groups = _ranking_case("many_groups")
     s = T.Session(val, rp, col, y, depth=4, n_trees=2, objective="rank:ndcg", groups=groups)

@@ -48,6 +48,11 @@ def test_slices_of_a_scoring_call(run_native):
     run_native("score_slices.cpp")
 
 
+def test_query_groups_of_a_workgroup(run_native):
+    """Short query groups share a workgroup: one each makes a million workgroups of a million groups of one or two rows."""
+    run_native("rank_packs.cpp")
+
+
 def test_places_of_frequent_features(run_native):
     """Sparse data with close to 2^31 values has more places than an int counts; what counts them must not overflow."""
     run_native("table_places.cpp")

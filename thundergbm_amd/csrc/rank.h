@@ -7,6 +7,7 @@
 
 #include "device_api.h"
 #include "host.h"
+#include "rank_packs.h"
 
 namespace tgbm {
 
@@ -81,8 +82,9 @@ class RankContext {
     int last_cur_ = 0;
     bool have_metric_order_ = false;  // sorter_.vals[last_cur_] is the (group, score) order of a metric() call
     int longest_ = 0;                 // group
-    int *d_wide_ = nullptr;           // groups that take the widest workgroups
-    int n_wide_ = 0;
+    RankPack *d_packs_ = nullptr, *d_wide_ = nullptr;  // RankPacks
+    int n_packs_ = 0, n_wide_ = 0, pack_rows_ = 0;
+    bool shared_ = false;
     bool short_groups_ = false;       // groups short enough to be ordered by counting (kRankCountSortMax / Mean)
 };
 

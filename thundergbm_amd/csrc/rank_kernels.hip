@@ -59,10 +59,10 @@ __device__ __forceinline__ int acc_bits(int len) { return 59 - (32 - __clz(max(l
 // Bound by the counting (len^2 steps of LDS a group). 200 003 rows in 1667 groups: 22 us, where eight threads of the host, the
 // copies of their tables and the look at the labels took 1.7 ms (a call of 40 rounds 20.5 -> 19.4 ms).
 constexpr int kSetupBlock = 128;
-// Threads of the rounds' kernels: 64 where no group is longer than 64 rows, 128 for groups of up to 256, 512 for longer ones. Those have a
-// launch of their own, so that the others don't ask for LDS for the longest group, and sort in LDS: counting 2000 rows is 2000 steps for
-// each of four rows a thread, 95 us a round for one such group among 19 800 of ten rows (200 k x 20, 20 rounds: 12.5 -> 7.1 ms).
-constexpr int kShortGroup = 64, kMiddleGroup = 256, kLongGroupBlock = 512;
+// Threads of the rounds' kernels: 64 where no group is longer than 64 rows, 128 for groups of up to 256 and where they share workgroups, 512
+// for longer ones. Those have a launch of their own, so that the others don't ask for LDS for the longest group, and sort in LDS: counting 2000 rows is
+// 2000 steps for each of four rows a thread, 95 us a round for one such group among 19 800 of ten rows (200 k x 20, 20 rounds: 12.5 -> 7.1 ms).
+constexpr int kPackBlock = 128, kLongGroupBlock = 512;
 constexpr size_t kRankGroupBytes = 2 * sizeof(unsigned long long) + 2 * sizeof(int) + sizeof(float);  // LDS of k_rank_gradient_group per row
 __global__ __launch_bounds__(kSetupBlock) void k_rank_setup(const float *__restrict__ y, const int *__restrict__ gptr,
                                                             const float *__restrict__ log2_of, int longest, int *__restrict__ static_row,
@@ -267,13 +267,14 @@ __host__ __device__ inline int keys_to_sort(int len) {  // fewer than 2 len
     return count;
 }
 
-// sorted: the rows of every group by score descending, ties by row. which: the groups of the launch (nullptr: all of at most `most` rows).
-template <int BLK>
-__global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict__ which, int most, const int *__restrict__ gptr,
-                                                          const float *__restrict__ score, int *__restrict__ sorted) {
-    extern __shared__ unsigned long long s_order[];  // [keys_to_sort(most)], as unsigned [most] where they are counted
-    const int g = which != nullptr ? which[blockIdx.x] : (int)blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
-    if (len > most) return;
+// sorted: the rows of every group by score descending, ties by row. SHARED: some packs are of several groups.
+template <int BLK, bool SHARED>
+__global__ __launch_bounds__(BLK) void k_rank_order_group(const RankPack *__restrict__ packs, const int *__restrict__ gptr,
+                                                          const int *__restrict__ group_of, const float *__restrict__ score,
+                                                          int *__restrict__ sorted) {
+    extern __shared__ unsigned long long s_order[];  // [keys_to_sort(rows)], as unsigned [rows] where they are counted
+    const RankPack pack = packs[blockIdx.x];
+    const int b = pack.begin, len = pack.end - b;
     if (BLK == kLongGroupBlock) {
         const int count = keys_to_sort(len);
         for (int i = threadIdx.x; i < count; i += BLK)
@@ -286,22 +287,30 @@ __global__ __launch_bounds__(BLK) void k_rank_order_group(const int *__restrict_
     unsigned *s_key = reinterpret_cast<unsigned *>(s_order);
     for (int i = threadIdx.x; i < len; i += BLK) s_key[i] = ~float_key(score[b + i]);
     __syncthreads();
-    for (int i = threadIdx.x; i < len; i += BLK) sorted[b + rows_before(s_key, 0, len, s_key[i], i)] = b + i;
+    for (int i = threadIdx.x; i < len; i += BLK) {
+        int from = 0, to = len;
+        if (SHARED) {
+            const int g = group_of[b + i];
+            from = gptr[g] - b;
+            to = gptr[g + 1] - b;
+        }
+        sorted[b + from + rows_before(s_key, from, to, s_key[i], i)] = b + i;
+    }
 }
 
 // Rows inside their runs of equal labels by score descending, ties by row (static_row ascends inside a run), then every position's pair.
-template <int BLK>
-__global__ __launch_bounds__(BLK) void k_rank_gradient_group(const int *__restrict__ which, int most, const int *__restrict__ gptr,
-                                                             const float *__restrict__ score, const float *__restrict__ y,
+template <int BLK, bool SHARED>
+__global__ __launch_bounds__(BLK) void k_rank_gradient_group(const RankPack *__restrict__ packs, int most, const float *__restrict__ score,
+                                                             const float *__restrict__ y,
                                                              const int *__restrict__ static_row, const int *__restrict__ run_of,
                                                              const RankRun *__restrict__ runs, const float *__restrict__ idcg, unsigned seed,
                                                              int *__restrict__ sorted, GHPair *__restrict__ gh) {
-    extern __shared__ unsigned long long s_acc[];  // [2 most] by row
+    extern __shared__ unsigned long long s_acc[];  // [2 most] by row (most: rows of a workgroup of the launch)
     unsigned *s_key = reinterpret_cast<unsigned *>(s_acc + 2 * most);  // by position of static_row
-    int *s_row = reinterpret_cast<int *>(s_key + most);                // by position of the order, within the group
+    int *s_row = reinterpret_cast<int *>(s_key + most);                // by position of the order, within the workgroup
     float *s_score = reinterpret_cast<float *>(s_row + most);
-    const int g = which != nullptr ? which[blockIdx.x] : (int)blockIdx.x, b = gptr[g], len = gptr[g + 1] - b;
-    if (len > most) return;
+    const RankPack pack = packs[blockIdx.x];
+    const int b = pack.begin, len = pack.end - b;
     if (BLK == kLongGroupBlock) {  // (run, key, position) where the sums will be
         static_assert(kRankCountSortMax <= 1 << 12, "positions of a group in 12 bits");
         const int count = keys_to_sort(len);
@@ -333,17 +342,26 @@ __global__ __launch_bounds__(BLK) void k_rank_gradient_group(const int *__restri
     }
     __syncthreads();
     for (int i = threadIdx.x; i < len; i += BLK) {
+        const RankRun r = runs[run_of[b + i]];
         RankPair pair;
-        if (!draw_partner(runs[run_of[b + i]], b + i, seed, pair)) continue;
-        const int high = s_row[pair.high], low = s_row[pair.low];
-        weigh_pair(pair, idcg != nullptr ? idcg + g : nullptr, y[b + high], y[b + low], s_score[pair.high], s_score[pair.low], len);
+        if (!draw_partner(r, b + i, seed, pair)) continue;
+        const int at = SHARED ? r.group_begin - b : 0, high = s_row[at + pair.high], low = s_row[at + pair.low];
+        weigh_pair(pair, idcg != nullptr ? idcg + (SHARED ? r.group : pack.group) : nullptr, y[b + high], y[b + low],
+                   s_score[at + pair.high], s_score[at + pair.low], SHARED ? r.group_end - r.group_begin : len);
         atomicAdd(&s_acc[2 * high], (unsigned long long)pair.ql);
         atomicAdd(&s_acc[2 * high + 1], pair.qh);
         atomicAdd(&s_acc[2 * low], (unsigned long long)(-pair.ql));
         atomicAdd(&s_acc[2 * low + 1], pair.qh);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < len; i += BLK) gh[b + i] = pair_of_sums((long long)s_acc[2 * i], (long long)s_acc[2 * i + 1], len);
+    for (int i = threadIdx.x; i < len; i += BLK) {
+        int rows = len;
+        if (SHARED) {  // (the run at a row's place: of the row's group)
+            const RankRun r = runs[run_of[b + i]];
+            rows = r.group_end - r.group_begin;
+        }
+        gh[b + i] = pair_of_sums((long long)s_acc[2 * i], (long long)s_acc[2 * i + 1], rows);
+    }
 }
 
 // One thread per position, for groups of any length.
@@ -503,13 +521,17 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, 
     upload(d_gptr_, gptr.data(), sizeof(int) * gptr.size());
     sorter_.alloc(n_);
     longest_ = longest;
-    std::vector<int> wide;  // (read by the copy until the set-up has waited)
+    RankPacks packs;  // (read by the copies until the set-up has waited)
     if (short_groups_) {
-        for (int g = 0; g < n_groups_; ++g)
-            if (group[g] > kMiddleGroup) wide.push_back(g);
-        n_wide_ = (int)wide.size();
-        d_wide_ = dalloc<int>(wide.size());
-        upload(d_wide_, wide.data(), sizeof(int) * wide.size());
+        packs = rank_packs(group);
+        n_packs_ = (int)packs.packs.size();
+        n_wide_ = (int)packs.wide.size();
+        pack_rows_ = packs.most;
+        shared_ = packs.shared;
+        d_packs_ = dalloc<RankPack>(packs.packs.size());
+        d_wide_ = dalloc<RankPack>(packs.wide.size());
+        upload(d_packs_, packs.packs.data(), sizeof(RankPack) * packs.packs.size());
+        upload(d_wide_, packs.wide.data(), sizeof(RankPack) * packs.wide.size());
         setup_short_groups(longest);
     }
     else setup_groups(y, gptr);
@@ -641,13 +663,14 @@ void RankContext::gradient(const float *d_score, GHPair *d_gh, unsigned seed, bo
         have_metric_order_ = false;
         static LdsOptIn opt_in;
         const float *idcg = ndcg_ ? d_idcg_ : nullptr;
-        if (longest_ * kRankGroupBytes > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_rank_gradient_group<kLongGroupBlock>)});
-#define TGBM_RANK_GRADIENT(BLK, GROUPS, WHICH, MOST)                                                                                \
-    k_rank_gradient_group<BLK><<<GROUPS, BLK, (MOST) * kRankGroupBytes, stream_>>>(WHICH, MOST, d_gptr_, d_score, d_y_, d_static_row_, \
+        if (longest_ * kRankGroupBytes > 48 * 1024) opt_in({reinterpret_cast<const void *>(&k_rank_gradient_group<kLongGroupBlock, false>)});
+#define TGBM_RANK_GRADIENT(BLK, SHARED, GROUPS, WHICH, MOST)                                                                                \
+    k_rank_gradient_group<BLK, SHARED><<<GROUPS, BLK, (MOST) * kRankGroupBytes, stream_>>>(WHICH, MOST, d_score, d_y_, d_static_row_, \
                                                                                   d_run_of_, d_runs_, idcg, seed, sorter_.vals[0], d_gh)
-        if (longest_ <= kShortGroup) TGBM_RANK_GRADIENT(kShortGroup, n_groups_, nullptr, longest_);
-        else if (n_wide_ < n_groups_) TGBM_RANK_GRADIENT(kSetupBlock, n_groups_, nullptr, std::min(longest_, kMiddleGroup));
-        if (n_wide_ > 0) TGBM_RANK_GRADIENT(kLongGroupBlock, n_wide_, d_wide_, longest_);
+        if (n_packs_ > 0 && shared_) TGBM_RANK_GRADIENT(kPackBlock, true, n_packs_, d_packs_, pack_rows_);
+        else if (n_packs_ > 0 && pack_rows_ <= 64) TGBM_RANK_GRADIENT(64, false, n_packs_, d_packs_, pack_rows_);
+        else if (n_packs_ > 0) TGBM_RANK_GRADIENT(kPackBlock, false, n_packs_, d_packs_, pack_rows_);
+        if (n_wide_ > 0) TGBM_RANK_GRADIENT(kLongGroupBlock, false, n_wide_, d_wide_, longest_);
 #undef TGBM_RANK_GRADIENT
         return;
     }
@@ -674,11 +697,12 @@ void RankContext::metric(int kind, const float *d_score, float *d_out) {
     const int grid = grid_for(n_);
     int cur = 0;
     if (short_groups_) {
-#define TGBM_RANK_ORDER(BLK, GROUPS, WHICH, MOST) \
-    k_rank_order_group<BLK><<<GROUPS, BLK, keys_to_sort(MOST) * sizeof(unsigned long long), stream_>>>(WHICH, MOST, d_gptr_, d_score, sorter_.vals[0])
-        if (longest_ <= kShortGroup) TGBM_RANK_ORDER(kShortGroup, n_groups_, nullptr, longest_);
-        else if (n_wide_ < n_groups_) TGBM_RANK_ORDER(kSetupBlock, n_groups_, nullptr, std::min(longest_, kMiddleGroup));
-        if (n_wide_ > 0) TGBM_RANK_ORDER(kLongGroupBlock, n_wide_, d_wide_, longest_);
+#define TGBM_RANK_ORDER(BLK, SHARED, GROUPS, WHICH, LDS) \
+    k_rank_order_group<BLK, SHARED><<<GROUPS, BLK, LDS, stream_>>>(WHICH, d_gptr_, d_group_of_, d_score, sorter_.vals[0])
+        if (n_packs_ > 0 && shared_) TGBM_RANK_ORDER(kPackBlock, true, n_packs_, d_packs_, pack_rows_ * sizeof(unsigned));
+        else if (n_packs_ > 0 && pack_rows_ <= 64) TGBM_RANK_ORDER(64, false, n_packs_, d_packs_, pack_rows_ * sizeof(unsigned));
+        else if (n_packs_ > 0) TGBM_RANK_ORDER(kPackBlock, false, n_packs_, d_packs_, pack_rows_ * sizeof(unsigned));
+        if (n_wide_ > 0) TGBM_RANK_ORDER(kLongGroupBlock, false, n_wide_, d_wide_, keys_to_sort(longest_) * sizeof(unsigned long long));
 #undef TGBM_RANK_ORDER
     } else {
         k_rank_metric_keys<<<grid, kBlock, 0, stream_>>>(n_, d_group_of_, d_score, sorter_.keys[0], sorter_.vals[0]);
