@@ -366,10 +366,11 @@ def test_pairs_that_fill_their_fields(n, g, h):
 
 # Class trees whose rows walk them at the end (655 360 rows of all trees on) against the launches that keep row lists, byte for byte: records
 # of 4, 8, 16 and 32 bytes, features that share a column, missing values, trees that stop early, an odd number of rows.
-@pytest.mark.parametrize("n,F,K,depth,hot", [
-    (163_840, 3, 4, 8, 0), (163_839, 3, 4, 8, 0), (218_455, 7, 3, 6, 0), (131_073, 13, 5, 4, 0), (93_623, 31, 7, 8, 0), (131_072, 6, 5, 1, 0),
-    (120_001, 8, 6, 7, 60), (220_000, 2, 3, 10, 30)])
-def test_class_trees_are_walked(n, F, K, depth, hot, monkeypatch):
+# (width: of the records, 0 where the rows are one or two too few)
+@pytest.mark.parametrize("n,F,K,depth,hot,width", [
+    (163_840, 3, 4, 8, 0, 4), (163_839, 3, 4, 8, 0, 0), (218_455, 7, 3, 6, 0, 8), (131_073, 13, 5, 4, 0, 16), (93_623, 31, 7, 8, 0, 32),
+    (131_072, 6, 5, 1, 0, 8), (120_001, 8, 6, 7, 60, 16), (220_000, 2, 3, 10, 30, 4)])
+def test_class_trees_are_walked(n, F, K, depth, hot, width, monkeypatch):
     import thundergbm_amd as T
     rng = np.random.default_rng(n + F)
     X = np.zeros((n, F + hot), np.float32)
@@ -386,6 +387,7 @@ def test_class_trees_are_walked(n, F, K, depth, hot, monkeypatch):
         monkeypatch.setenv("TGBM_SPLIT_HIST", switch)
         s = T.Session(val, rp, col, y, depth=depth, n_trees=2, learning_rate=0.4, objective="multi:softmax", num_class=K, gamma=2.0)
         assert (s.info("split_hist_rows") > 0) == (switch == "1")
+        assert s.info("class_walk") == (width if switch == "1" else 0)
         s.boost(2)
         out.append((s.model().tobytes(), s.nid().tobytes(), s.y_pred().tobytes()))
         s.close()

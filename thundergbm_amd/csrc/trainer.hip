@@ -1624,6 +1624,7 @@ int Trainer::info(const std::string &key) const {
     if (key == "partial_histograms") return (int)(tb_.n_partial / (size_t)n_bins_);
     if (key == "small_levels") return small_ok_ ? 1 : 0;                 // boost() builds the levels by k_small_level,
     if (key == "split_hist_rows") return small_ok_ ? 0 : run_plan_.run;  // else by k_split_hist, so many rows a workgroup (0: neither)
+    if (key == "class_walk") return !small_ok_ && run_plan_.walk ? bins_.W : 0;  // class trees are walked over records of so many bytes, 0: not
     fatal("unknown info key %s", key.c_str());
 }
 
