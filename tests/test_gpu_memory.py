@@ -107,3 +107,35 @@ def test_a_dense_matrix_goes_once_its_values_are_grouped(filled, more):
     kept(as_csr)
     extra = kept(X) - kept(as_csr)
     assert extra < more * X.nbytes, extra
+
+
+@pytest.mark.parametrize("spread", ["1", "0"])
+def test_sparse_sessions_hold_a_value_once(spread, monkeypatch):
+    """A session of the sparse level pass: its values have places of their own, and the copy that those are made of goes. A value of a
+    frequent feature takes 4 bytes as a bin, 18 in its place (14 looked up) and 1/0.6 in a byte column here, the copy 8."""
+    import ctypes as C
+    import thundergbm_amd as T
+    D.warm_up(T)
+    hip = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+    def free():
+        T.release_memory()
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    monkeypatch.setenv("TGBM_LAYOUT", "sparse")
+    monkeypatch.setenv("TGBM_SPARSE_SPREAD", spread)
+    rng = np.random.default_rng(1)
+    n, F = 300_000, 40
+    X = np.exp(rng.standard_normal((n, F))).astype(np.float32)
+    X[rng.random(X.shape) >= 0.6] = 0
+    val, rp, col = D.dense_to_csr(X)
+    before = free()
+    s = T.Session(val, rp, col, X[:, 0] + X[:, 1], depth=3, n_trees=2, max_num_bin=15)
+    assert s.info("sparse_pass") == 1 and s.info("sparse_spread_blocks") == (10 if spread == "1" else 0)
+    held = (before - free()) / len(val)
+    s.boost(2)
+    s.close()
+    rows = 40 * n / len(val)  # (what a row takes itself: labels, predictions, pairs, nodes, words)
+    assert held < 4 + (18 if spread == "1" else 14) + 1 / 0.6 + rows + 4, held

@@ -221,7 +221,7 @@ struct CsrBins {
     int head_bins = 0;
     // The same stored values sorted by global bin id (rows ascending inside a bin): the root histogram, where
     // every row takes part, is a segmented sum over this copy instead of atomics to random bins. nullptr: none.
-    const int *csc_bin = nullptr;  // [nnz]
+    const int *csc_bin = nullptr;  // [nnz] (with the level pass until its values have places of their own)
     const int *csc_row = nullptr;  // [nnz]
     long nnz = 0;
     // Sparse level pass: byte columns of the frequent features (local bin id of the row, kMissingBin = no stored

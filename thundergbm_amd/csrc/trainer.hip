@@ -254,7 +254,10 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
             int bits = 1;
             while (bits < 31 && (1l << bits) < (long)n_bins_) ++bits;
             const int cur = sort_pairs(stream_, ps, nnz_, bits);
-            int *d_cbin = dalloc<int>((size_t)nnz_), *d_crow = dalloc<int>((size_t)nnz_);
+            int *d_cbin = nullptr, *d_crow = nullptr;
+            device_alloc_to(d_cbin, sizeof(int) * (size_t)nnz_);
+            device_alloc_to(d_crow, sizeof(int) * (size_t)nnz_);
+            if (!sparse_pass_) allocs_.insert(allocs_.end(), {d_cbin, d_crow});  // (the level pass goes by copies of its own: alloc_tree_buffers)
             launch_csc_unpack(stream_, nnz_, ps.keys[cur], ps.vals[cur], d_cbin, d_crow);
             HIP_CHECK(hipStreamSynchronize(stream_));
             ps.release();
@@ -737,6 +740,11 @@ void Trainer::alloc_tree_buffers() {
     tb.blk_bin_begin = d_blk;
     tb.feat_lds_off = d_off;
     HIP_CHECK(hipStreamSynchronize(stream_));  // the host vectors above go out of scope
+    if (sparse_pass_) {  // the values' places have been made of it
+        device_free(const_cast<int *>(csr_.csc_bin));
+        device_free(const_cast<int *>(csr_.csc_row));
+        csr_.csc_bin = csr_.csc_row = nullptr;
+    }
 
     const char *small_env = std::getenv("TGBM_SMALL");  // "0": the launches of larger data (tests)
     small_ok_ = !sparse_ && hist_cap_level_ < 0 && n_ <= (bins_.bin_bytes == 2 ? kSmallRowsWide : kSmallRows) && small_levels_fit(tb) && !(small_env != nullptr && std::string(small_env) == "0");
