@@ -136,6 +136,8 @@ struct SpShared {
     int fbin[kSparseBatchFeatures + 2];            // first bin (relative to the batch) of every feature of the batch
     int ctl[8];  // batch: first feature, end feature, first bin, bins, node range begin, nodes in range, first group, end group
 };
+// (a launch asks for n_cells <= kSparseCells of LDS beside these)
+static_assert(sizeof(SpShared) + kSparseCells * sizeof(longlong2) <= kLdsBytes, "the largest tables' LDS");
 
 // Level-wide state every task starts from: node sums and validity into LDS, and the best keys that other tasks have published:
 // a node whose best candidate is another task's by now needs no record of this one's.
@@ -309,8 +311,9 @@ __global__ __launch_bounds__(kSpBlock, DEEP ? 4 : 8) void k_sparse_level(TreeBuf
             __syncthreads();
             for (int c = threadIdx.x; c < n_cells; c += kSpBlock) cells[c] = make_longlong2(0, 0);
             __syncthreads();
-            // accumulate: a thread takes two groups of places at a time (every load is unconditional - past the end the last group
-            // repeats and is skipped below -, so that a stage's loads are issued together instead of one after the other)
+            // accumulate: a thread takes two groups of places at a time, one where 64 registers have to do (every load is unconditional -
+            // past the end the last group repeats and is skipped below -, so that a stage's loads are issued together instead of one after
+            // the other)
             constexpr int U = DEEP ? 2 : 1, V = kSpreadGroup;
             static_assert(V == 4, "a group's loads");
             const int bin_shift = bin0 - task_bin0;
