@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kBlock) void k_transpose_keys(int n, int C, const f
         if (r0 + lane < n && c0 + c < C) keys[(size_t)(c0 + c) * n + r0 + lane] = s[lane][c];
 }
 
-// The same for cells of which some hold no value (is_stored of dense_to_csr): their keys are the largest there are, which sorts them
+// The same for cells of which some hold no value (is_stored): their keys are the largest there are, which sorts them
 // behind the values. stored[f] += values of the feature.
 constexpr int kCellRows = 256;  // rows per workgroup
 constexpr unsigned kNoValue = ~0u;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kBlock) void k_transpose_cells(DenseCells cells, in
         for (int r = w; r < 64; r += kWaves)
             if (r0 + r < cells.n && c0 + lane < F) {
                 const float v = cells.x[(size_t)(r0 + r) * cells.columns + c0 + lane];
-                const bool in = v != 0.f || (cells.minus_zero_is_stored && __float_as_uint(v) != 0u);
+                const bool in = is_stored(v, cells.minus_zero_is_stored);
                 count += in ? 1u : 0u;
                 s[r][lane] = in ? float_key(v) : kNoValue;
             }

@@ -207,7 +207,7 @@ __device__ __forceinline__ unsigned stored_key(float v) {
 }
 template <bool NARROW>
 __device__ __forceinline__ unsigned dense_key(float v, bool minus_zero_is_stored) {
-    const bool stored = v != 0.f || (minus_zero_is_stored && __float_as_uint(v) != 0u);
+    const bool stored = is_stored(v, minus_zero_is_stored);
     return stored ? stored_key<NARROW>(v) : kMissingKey;
 }
 // Sums: double where the reference's shared-memory path is (predictor.cu:85-160), else float with the product and the

@@ -701,9 +701,6 @@ int device_max_int(hipStream_t s, const int *d_v, long n) {
 // ---- dense input -----------------------------------------------------------------------------------
 // Streaming passes over the matrix, sixteen lanes per row as in the binning kernels (a row of 28 floats is two
 // lines): 140 MB take 60 us to count and 130 us to rewrite, next to 2.4 ms for their way over PCIe.
-__device__ __forceinline__ bool is_stored(float v, bool minus_zero_is_stored) {  // (cut_kernels.hip has it too)
-    return v != 0.f || (minus_zero_is_stored && __float_as_uint(v) != 0u);
-}
 
 // Stored values per row, and the last column that holds one.
 // (one atomic per workgroup, and 1024 of them: all to one word, a wavefront's each took 200 us whatever the rows)
