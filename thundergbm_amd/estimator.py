@@ -218,7 +218,8 @@ class TGBMModel(BaseEstimator):
         self.group_label = [labels[i] for i in range(self.num_class)]
 
     def get_trees(self):
-        """Every tree as parallel heap-ordered arrays (the dictionaries the reference hands to shap)."""
+        """Every tree as parallel heap-ordered arrays (the dictionaries the reference hands to shap). The trees' arrays are disjoint parts
+        of seven that all of them share: copy those of a tree that is kept without the others."""
         if not self.model:
             raise ValueError("Please train the model first or load model from file!")
         lib = _lib.load()
