@@ -199,3 +199,33 @@ def test_frequent_features_in_parts(T, n):
         os.environ.pop("TGBM_SPARSE_SPREAD", None)
         del os.environ["TGBM_LAYOUT"]
     assert runs[0] == runs[1]
+
+
+# Spread values where columns are sampled (their segments and values take no part, in tables with kept records and in the filter) and rows are
+# resampled (pairs instead of words), against looked-up values and against tables for every feature; 31 and 255 bins (one bin of a lane, four).
+@pytest.mark.parametrize("bagging", [0, 1])
+@pytest.mark.parametrize("objective,kw", [("reg:linear", {}), ("binary:logistic", {"min_child_weight": 0.0}), ("multi:softmax", {"num_class": 3})])
+@pytest.mark.parametrize("bins", [31, 255])
+def test_spread_values_of_sampled_columns(T, bins, objective, kw, bagging):
+    n = 40000
+    counts = [n - 1, 33000, 32769, 9000, 5000] + [700] * 130 + [300] * 60 + [4, 5, 1] * 20
+    val, rp, col, z = _by_feature(counts, n, 3)
+    y = (z if objective == "reg:linear" else np.digitize(z, [-0.5, 0.5][: 2 if "multi" in objective else 1])).astype(np.float32)
+    runs = []
+    os.environ["TGBM_LAYOUT"] = "sparse"
+    try:
+        for spread, rare in (("1", "1"), ("0", "1"), ("1", "0")):
+            os.environ.update(TGBM_SPARSE_SPREAD=spread, TGBM_SPARSE_SORTED=rare)
+            ctypes.CDLL(None).srand(7)
+            s = T.Session(val, rp, col, y, objective=objective, depth=7, n_trees=3, max_num_bin=bins, learning_rate=0.5, **kw)
+            assert s.info("sparse_spread_blocks") == (2 if spread == "1" else 0)
+            assert (s.info("sparse_rare_values") > 0) == (rare == "1")
+            s.set_option("bagging", bagging)
+            s.set_option("column_sampling_rate", 0.5)
+            s.boost(3)
+            runs.append((s.model().tobytes(), s.y_pred().tobytes()))
+            s.close()
+    finally:
+        for key in ("TGBM_LAYOUT", "TGBM_SPARSE_SPREAD", "TGBM_SPARSE_SORTED"):
+            os.environ.pop(key, None)
+    assert runs[0] == runs[1] and runs[0] == runs[2]
