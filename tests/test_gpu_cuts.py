@@ -88,3 +88,10 @@ def test_cells_without_values(n, F, filled, max_bin, dtype):
         m = T.TGBMRegressor(depth=4, n_trees=3, max_num_bin=max_bin, verbose=0).fit(data, y)
         runs.append([{k: v.tobytes() for k, v in t.items()} for t in m.get_trees()] + [m.predict(data).tobytes()])
     assert runs[0] == runs[1]
+
+
+# Bins by runs of features (two here) and by each value's own search: rows with fewer and with more than four values a run.
+@pytest.mark.parametrize("filled", [0.035, 0.045])
+def test_bins_of_rows_with_few_values(filled, monkeypatch):
+    monkeypatch.setenv("TGBM_LAYOUT", "dense")
+    test_cut_points(6000, 200, filled, 200, False)

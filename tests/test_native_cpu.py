@@ -48,6 +48,11 @@ def test_slices_of_a_scoring_call(run_native):
     run_native("score_slices.cpp")
 
 
+def test_runs_of_features_for_bins(run_native):
+    """Bins looked for by runs of features: rows with few values in a run take the other way."""
+    run_native("bin_groups.cpp")
+
+
 def test_query_groups_of_a_workgroup(run_native):
     """Short query groups share a workgroup: one each makes a million workgroups of a million groups of one or two rows."""
     run_native("rank_packs.cpp")

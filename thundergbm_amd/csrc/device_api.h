@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "common.h"
+#include "bin_groups.h"
 #include "table_places.h"
 
 #define HIP_CHECK(expr)                                                                              \
@@ -613,15 +614,12 @@ void launch_fill_f32(hipStream_t s, float *p, float v, size_t n);
 void launch_fill_u8(hipStream_t s, uint8_t *p, uint8_t v, size_t n);
 
 // data preparation
-// F: columns of the matrix; feat_col / feat_lo: DenseBins' bundle tables or nullptr
+// F: columns of the matrix; feat_col / feat_lo: DenseBins' bundle tables or nullptr; group_first: bin_groups on the device, n_groups runs
 void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, const float *val, const float *cut_val,
                       const int *cut_row_ptr, uint8_t *binmat, int W, size_t block_stride, uint8_t *colmat,
                       size_t col_stride, int bin_bytes, int F, const int *feat_col,
                       const uint8_t *feat_lo, bool rows_ascend, int n_features, int n_bins, const int *group_first = nullptr,
                       int n_groups = 0);
-// Runs of features whose cut points a workgroup of launch_bin_dense has room for: the first one of each, and the end (group_first, on the
-// device, and the number of runs); empty: a feature has too many.
-std::vector<int> bin_groups(const std::vector<int> &cut_row_ptr);
 // false when some row holds a column index below its predecessor's
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col);
 // min_next[c] (pre-filled with INT_MAX) = smallest column index that follows column c in a row (equal neighbours, a

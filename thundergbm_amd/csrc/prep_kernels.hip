@@ -347,7 +347,6 @@ __global__ __launch_bounds__(kBlock) void k_bin_dense(int n, const int *__restri
 
 // The same with all cut points in LDS (kBinLds of them at most), where the eight steps of a value's search take a few
 // cycles each instead of a trip to a cache: 280 M values 3.9 -> 1.24 ms.
-constexpr int kBinLds = 16384;
 constexpr int kBinBlock = 1024;
 template <typename BinT>
 __global__ __launch_bounds__(kBinBlock) void k_bin_dense_lds(int n, int F, const int *__restrict__ row_ptr, const int *__restrict__ col,
@@ -993,18 +992,6 @@ void launch_bin_dense(hipStream_t s, int n, const int *row_ptr, const int *col, 
         k_bin_dense<uint8_t><<<grid, kBlock, 0, s>>>(n, row_ptr, col, val, cut_val, cut_row_ptr, binmat, W, block_stride,
                                                     feat_col, feat_lo);
     launch_cols_from_rows(s, n, W, F, (F + W - 1) / W, binmat, block_stride, colmat, col_stride, bin_bytes);
-}
-
-std::vector<int> bin_groups(const std::vector<int> &cut_row_ptr) {
-    std::vector<int> first{0};
-    const int F = (int)cut_row_ptr.size() - 1;
-    for (int f = 0; f < F; ++f) {
-        const int cuts = cut_row_ptr[(size_t)f + 1] - cut_row_ptr[(size_t)first.back()];
-        if (f > first.back() && cuts + (f + 1 - first.back()) + 1 > kBinLds) first.push_back(f);
-        if (cut_row_ptr[(size_t)f + 1] - cut_row_ptr[(size_t)f] + 2 > kBinLds) return {};
-    }
-    first.push_back(F);
-    return first;
 }
 
 bool device_rows_ascend(hipStream_t s, int n, const int *row_ptr, const int *col) {

@@ -422,7 +422,8 @@ Trainer::Trainer(const DataSet &ds, GBMParam &param) {
         // (rows that store every feature cannot hold a column twice)
         if (!ascend_known && nnz_ != (long)n_ * F_) rows_ascend = device_rows_ascend(stream_, n_, d_row_ptr, d_col);
         if (!rows_ascend) log_info("rows with descending column indices: the dense bins are filled row by row");
-        const std::vector<int> groups = bin_groups(h_cut_row_ptr_);
+        std::vector<int> groups = bin_groups(h_cut_row_ptr_);
+        if (!groups.empty() && !bins_by_groups(nnz_, n_, (int)groups.size() - 1)) groups.clear();
         int *d_groups = nullptr;
         if (!groups.empty()) {
             device_alloc_to(d_groups, sizeof(int) * groups.size());
