@@ -644,8 +644,8 @@ struct DenseCells {
     bool minus_zero_is_stored;
 };
 // Does a cell hold a value? A zero does not; -0 does in double-precision matrices (minus_zero_is_stored, upload_doubles_as_floats).
-__device__ __forceinline__ bool is_stored(float v, bool minus_zero_is_stored) {
-    return v != 0.f || (minus_zero_is_stored && __float_as_uint(v) != 0u);
+__host__ __device__ inline bool is_stored(float v, bool minus_zero_is_stored) {
+    return v != 0.f || (minus_zero_is_stored && __builtin_signbit(v) != 0);
 }
 // Are the cells that hold no value sorted along with the others (build_cut_points)? That costs less than grouping the values: on wide
 // data, where they would be sorted as 64-bit pairs, up to a quarter of the cells, else up to a 32nd (all passes: 35 M cells of 700
