@@ -13,10 +13,14 @@ namespace tgbm {
 
 enum RankMetric { RANK_METRIC_MAP = 3, RANK_METRIC_NDCG = 4 };
 
-// Groups of at most this many rows are ordered by counting (every row counts the rows of its segment that go before
-// it, in the LDS of a workgroup: quadratic in the segment length); data with a longer group takes the radix sort.
+// Data whose groups have at most kRankCountSortMax rows, and whose average row is in a group of at most kRankCountSortMean
+// (sum(len^2) / rows), is ordered in the LDS of workgroups (k_rank_order_group, k_rank_gradient_group); other data takes the radix sort.
+// The mean is from an order by counting throughout, quadratic in a group's rows. Groups of more than 256 rows are sorted by now, for
+// which it is too low: 20 rounds of 200 k x 8, depth 4, in groups of 300, 500, 1000, 2000 rows take 3.1, 2.5, 2.7, 3.1 ms in LDS (set-up,
+// which counts still, 1.1, 1.1, 1.3, 1.9) and 8.7, 8.9, 8.3, 8.4 by the radix sort (set-up 2.4); of 1 M rows in groups of 1000 3.9 (2.3)
+// and 13.0 (8.1).
 constexpr int kRankCountSortMax = 2048;
-constexpr int kRankCountSortMean = 384;  // ... and only while sum(len^2) / rows stays below this
+constexpr int kRankCountSortMean = 384;
 
 constexpr int kRankSetupRows = 1 << 14;  // the groups of fewer rows are ordered by one thread (about 0.5 ms)
 
@@ -85,7 +89,7 @@ class RankContext {
     RankPack *d_packs_ = nullptr, *d_wide_ = nullptr;  // RankPacks
     int n_packs_ = 0, n_wide_ = 0, pack_rows_ = 0;
     bool shared_ = false;
-    bool short_groups_ = false;       // groups short enough to be ordered by counting (kRankCountSortMax / Mean)
+    bool short_groups_ = false;       // groups short enough to be ordered in LDS (kRankCountSortMax / Mean)
 };
 
 }  // namespace tgbm

@@ -232,9 +232,10 @@ __device__ __forceinline__ GHPair pair_of_sums(long long g, long long h, int gro
     return GHPair{(float)ldexp((double)g, -sb), (float)ldexp((double)h, -sb)};
 }
 
-// Groups of at most kRankCountSortMax rows: a workgroup has a group to itself, orders it by counting in LDS and adds the lambdas up
-// there. Bound by the counting, len^2 steps of LDS a group. 200 003 rows in 1667 groups of about 120: the order by score 15 us (keys and
-// counting through the L1: 4.6 and 16.3), the gradients 20 (keys, counting, pairs with four 64-bit atomics a row, sums: 4.9, 11, 28, 5.2).
+// Groups of at most kRankCountSortMax rows: a workgroup has a group to itself, or several short ones (rank_packs.h), orders it in LDS, by
+// counting up to 256 rows, and adds the lambdas up there. Bound by the counting, len^2 steps of LDS a group. 200 003 rows in 1667 groups of
+// about 120: the order by score 15 us (keys and counting through the L1: 4.6 and 16.3), the gradients 13 (keys, counting, pairs with four
+// 64-bit atomics a row, sums: 4.9, 11, 28, 5.2).
 // Keys read four at a time, or eight ahead: 15, 27 us.
 __device__ __forceinline__ int rows_before(const unsigned *s_key, int from, int to, unsigned key, int at) {
     int before = 0;
@@ -491,8 +492,6 @@ RankContext::RankContext(hipStream_t s, const LabelVector &y, const float *d_y, 
     }
     TGBM_CHECK(gptr.back() == n_, "query groups cover %d instances, the dataset has %d", gptr.back(), n_);
 
-    // ordering by counting costs sum(len^2) steps (a launch per pass: 50 us for a million rows in groups of 120, where the radix
-    // sort takes 220 us): taken while the average row sits in a group of at most kRankCountSortMean rows
     int longest = 0;
     double steps = 0;
     for (int g : group) {

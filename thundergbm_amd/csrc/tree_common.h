@@ -233,7 +233,7 @@ __device__ __forceinline__ HistPlan plan_hist_item(const TreeBuffers &tb, int n_
 // powers of two), rounded once to the nearest integer, the hessian's in the low h_bits. Its integer is below 2^32, and the
 // gradient's below 2^31 where the hessian has 32 bits (item_shift: rows * the largest fit the field), so these are converted
 // in 32 bits and lie side by side; only whole-number hessians leave the gradient more. With both through doubles and 64-bit
-// shifts the root launch of 10 M x 28 was bound by vector instructions: 153 -> 141 us, which is its bytes at the rate of a copy
+// shifts the root launch of 10 M x 28 was bound by vector instructions: 150 -> 141 us, which is its bytes at the rate of a copy
 // (320 MB read, 320 written, 40 of words).
 template <bool BIN16>
 __device__ __forceinline__ void add_row(unsigned long long *lds, unsigned v, GHPair p, float scale_g, float scale_h, int h_bits, int o0, int o1,
